@@ -327,6 +327,9 @@ int saga_hip_axpby(const SagaTensorView *src, const SagaTensorView *dst, float a
                    saga_stream_t stream);
 /* dst = (float)src * scale : convert kernels (src/cuda/cuda_kernels.cu:102-151). */
 int saga_hip_convert(const SagaTensorView *src, const SagaTensorView *dst, float scale, saga_stream_t stream);
+/* dst = src bit for bit, same shape and type, any strides; either side may be pinned host memory.  Host access to a
+ * device tensor (managed memory in the reference, src/cuda/cuda_tensor.cpp:283-330). */
+int saga_hip_copy(const SagaTensorView *src, const SagaTensorView *dst, saga_stream_t stream);
 /* softmax over C at every (n,h,w): cudnnSoftmaxForward ACCURATE / MODE_CHANNEL (src/cuda/cuda_dnn.cpp:1937-1945). */
 int saga_hip_softmax(const SagaTensorView *x, const SagaTensorView *y, saga_stream_t stream);
 

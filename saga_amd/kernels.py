@@ -84,6 +84,7 @@ SIGNATURES = {
     "saga_hip_add": (_I, [_TV, _TV, _TV, _VP]),
     "saga_hip_axpby": (_I, [_TV, _TV, _F, _F, _VP]),
     "saga_hip_convert": (_I, [_TV, _TV, _F, _VP]),
+    "saga_hip_copy": (_I, [_TV, _TV, _VP]),
     "saga_hip_maxpool_fwd_codes": (_I, [_TV, _TV, _VP, _I, _I, _I, _VP]),
     "saga_hip_maxpool_bwd_codes": (_I, [_VP, _TV, _TV, _I, _I, _I, _F, _VP]),
     "saga_hip_maxpool_fwd_codes_bn": (_I, [_TV, _TV, _VP, _I, _I, _I, _VP, _I, _VP]),

@@ -104,11 +104,18 @@ static int transfer(saga_tensor_t tb, void *buf, size_t bytes, bool write)
 {
     return guard([&] {
         auto &t = ((TensorBox *)tb)->t;
+        const size_t es = Tensor::DataTypeSize(t->m_data_type);
+        const size_t n = t->m_dims.elements();
+        if(auto ht = dynamic_cast<HipTensor *>(t.get()); ht && ht->hostCopies() && bytes == n * es) {
+            if(write)
+                ht->writeHost(buf);
+            else
+                ht->readHost(buf);
+            return;
+        }
         auto ta = t->access();
         if(!ta)
             throw std::runtime_error("tensor has no storage: " + t->info());
-        const size_t es = Tensor::DataTypeSize(t->m_data_type);
-        const size_t n = t->m_dims.elements();
         if(bytes != n * es)
             throw std::runtime_error(fmt("payload is %zd bytes, tensor %s needs %zd", bytes, t->info().c_str(), n * es));
         const size_t rank = t->m_dims.size();

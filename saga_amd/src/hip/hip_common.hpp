@@ -9,8 +9,10 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <atomic>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <set>
 #include <string>
 #include <vector>
@@ -47,7 +49,7 @@ struct HipOperation;
 
 // A device allocation (possibly shared by several storages, e.g. the optimizer arena).
 struct HipMemory {
-    explicit HipMemory(size_t bytes);
+    explicit HipMemory(size_t bytes, bool clear = true);
     ~HipMemory();
     void *m_ptr = nullptr;
     size_t m_bytes = 0;
@@ -107,11 +109,15 @@ public:
     void *deviceMem() const override { return m_dev[m_index]; }
     bool doubleBuffered() const override { return true; }
     void *hostBack() const { return m_host[m_index ^ 1]; }
-    void uploadBack(hipStream_t st);    // host[back] -> device[back]
+    // host[back] -> device[back]; false (nothing enqueued) when the device already holds what the host does
+    bool uploadBack(hipStream_t st);
     void downloadFront(hipStream_t st); // device[front] -> host[front]
     void flip() { m_index ^= 1; }
     void *m_dev[2] = {nullptr, nullptr};
     void *m_host[2] = {nullptr, nullptr};
+    // host[i] was handed out for writing, or filled by a download, since it last went to the device
+    bool m_host_touched[2] = {false, false};
+    bool m_written_by_ops = false; // the device side changes too: every upload counts
     int m_index = 0;
 };
 
@@ -150,6 +156,12 @@ public:
     // host -> device copy of a front-end tensor (any type / layout); values are converted
     void copyFromHost(Tensor &src);
 
+    // all elements in logical row-major order, in the tensor's own type, from / to host memory.  A write is complete
+    // when the context's stream reaches it; the source may be reused at once.
+    bool hostCopies() const { return m_dims.size() <= 4 && m_dims.elements() > 0 && (m_storage->m_ctx || m_storage->doubleBuffered()); }
+    void writeHost(const void *src);
+    void readHost(void *dst);
+
     std::shared_ptr<HipStorage> m_storage;
     std::vector<int64_t> m_strides;
     int64_t m_offset = 0;
@@ -157,6 +169,10 @@ public:
 };
 
 std::vector<int64_t> hip_strides(const Dims &dims, HipLayout layout);
+
+// Host copy of an array of `ext` elements of `es` bytes between two layouts (strides in elements).
+void hip_permute(void *dst, std::vector<int64_t> dst_strides, const void *src, std::vector<int64_t> src_strides,
+                 std::vector<int64_t> ext, size_t es);
 
 using HipOp = std::shared_ptr<HipOperation>;
 using HipOps = std::vector<HipOp>;
@@ -227,7 +243,8 @@ public:
     void sync()
     {
         chkHip(hipStreamSynchronize(m_stream));
-        chkHip(hipStreamSynchronize(m_copy_stream));
+        if(m_copies_pending.exchange(false))
+            chkHip(hipStreamSynchronize(m_copy_stream));
     }
 
     const std::shared_ptr<UI> m_ui;
@@ -235,6 +252,16 @@ public:
     hipStream_t m_stream = nullptr;
     // uploads of the batched tensors' BACK buffers: they run beside the step that computes on the front buffers
     hipStream_t m_copy_stream = nullptr;
+    std::atomic<bool> m_copies_pending{false}; // something was enqueued on m_copy_stream since the last sync()
+
+    // Pinned memory that host reads and writes of small tensors go through (HipTensor::writeHost / readHost), and the
+    // event after which its last user on the stream is done with it.  At most STAGE_BYTES, owned by the context.
+    static constexpr size_t STAGE_BYTES = 1 << 20;
+    void *stage(size_t bytes); // caller holds m_stage_mutex
+    std::mutex m_stage_mutex;
+    void *m_stage = nullptr;
+    size_t m_stage_bytes = 0;
+    hipEvent_t m_stage_event = nullptr;
     int m_num_cu = 0;
     int m_storage_id_gen = 0;
     int m_program_index_gen = 0;
@@ -294,7 +321,7 @@ public:
     void runOps(const HipOps &ops);
     void addBatchedTensors(const ProgramSource &ps);
     void runCallbacks(const TensorBatchCallback &cb, long batch, Phase phase);
-    void flip(Phase upload_phase);
+    void flip(Phase upload_phase, hipStream_t st);
     void eliminateDeadOps();
     void checkAnomaly(HipOperation &op, const HipOpArgs &tensors, const char *what);
     HipOps createOptimizers();

@@ -150,8 +150,33 @@ HipContext::HipContext(const std::shared_ptr<UI> &ui, int device) : m_ui(ui), m_
     m_workspace.request(4096);
 }
 
+// The staging memory, free of earlier users, with room for `bytes` (at most STAGE_BYTES).
+void *HipContext::stage(size_t bytes)
+{
+    if(m_stage_event)
+        chkHip(hipEventSynchronize(m_stage_event));
+    else
+        chkHip(hipEventCreateWithFlags(&m_stage_event, hipEventDisableTiming));
+    if(m_stage_bytes < bytes) {
+        if(m_stage)
+            chkHip(hipHostFree(m_stage));
+        size_t n = 64 << 10;
+        while(n < bytes)
+            n *= 2;
+        chkHip(hipHostMalloc(&m_stage, n, hipHostMallocDefault));
+        m_stage_bytes = n;
+    }
+    return m_stage;
+}
+
 HipContext::~HipContext()
 {
+    if(m_stage_event) {
+        (void)hipEventSynchronize(m_stage_event);
+        (void)hipEventDestroy(m_stage_event);
+    }
+    if(m_stage)
+        (void)hipHostFree(m_stage);
     if(m_stream) {
         (void)hipStreamSynchronize(m_stream);
         (void)hipStreamDestroy(m_stream);
@@ -599,6 +624,11 @@ void HipProgram::finalize()
         fuse_bn_pooling(*this, m_ops);
     }
 
+    for(auto &op : m_ops)
+        for(auto &o : op->getOutputs())
+            if(o.second->m_storage->doubleBuffered())
+                static_cast<HipDoubleBuffer *>(o.second->m_storage.get())->m_written_by_ops = true;
+
     m_ctx->m_workspace.alloc();
     m_ctx->m_programs.push_back(this);
     m_ctx->planMemory();
@@ -623,14 +653,15 @@ void HipProgram::runCallbacks(const TensorBatchCallback &cb, long batch, Phase p
 }
 
 // Upload what the host wrote into the back buffers, then swap front and back.  The uploads go to the
-// copy stream: the operations of the step in flight only touch the front buffers, so the transfer
-// overlaps them; every caller synchronises both streams (HipContext::sync) before the next step is
-// enqueued, which is when the swapped buffers are first read.
-void HipProgram::flip(Phase upload_phase)
+// copy stream while a step is in flight: its operations only touch the front buffers, so the transfer overlaps
+// them, and step() synchronises both streams (HipContext::sync) before the next step, which reads the swapped
+// buffers, is enqueued.  Before the first step they go to the program's own stream, in front of it.
+void HipProgram::flip(Phase upload_phase, hipStream_t st)
 {
     for(auto &bt : m_batched) {
         if(!!(bt.second.second & upload_phase))
-            bt.second.first->uploadBack(m_ctx->m_copy_stream);
+            if(bt.second.first->uploadBack(st) && st == m_ctx->m_copy_stream)
+                m_ctx->m_copies_pending = true;
         bt.second.first->flip();
     }
 }
@@ -874,8 +905,7 @@ void HipProgram::prep(long, long batch_offset)
 {
     finalize();
     runCallbacks(m_pc.pre_ops, 0 + batch_offset, Phase::PRE);
-    flip(Phase::PRE);
-    m_ctx->sync();
+    flip(Phase::PRE, m_ctx->m_stream);
     m_total_samples = 0;
     m_epoch_start = now();
 }
@@ -893,7 +923,7 @@ void HipProgram::step(long batch, long batches, long batch_offset)
         runCallbacks(m_pc.post_ops, batch - 1 + batch_offset, Phase::POST);
     if(batch < batches - 1)
         runCallbacks(m_pc.pre_ops, batch + 1 + batch_offset, Phase::PRE);
-    flip(Phase::PRE);
+    flip(Phase::PRE, m_ctx->m_copy_stream);
 
     for(const auto &u : m_units)
         m_total_samples += u.m_batch_size;

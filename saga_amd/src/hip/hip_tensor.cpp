@@ -6,6 +6,7 @@
 #include <math.h>
 #include <string.h>
 
+#include <algorithm>
 #include <sstream>
 
 #include "hip_common.hpp"
@@ -14,10 +15,11 @@ namespace saga {
 
 // ---------------------------------------------------------------- memory
 
-HipMemory::HipMemory(size_t bytes) : m_bytes(bytes)
+HipMemory::HipMemory(size_t bytes, bool clear) : m_bytes(bytes)
 {
     chkHip(hipMalloc(&m_ptr, std::max<size_t>(bytes, 256)));
-    chkHip(hipMemset(m_ptr, 0, std::max<size_t>(bytes, 256)));
+    if(clear)
+        chkHip(hipMemset(m_ptr, 0, std::max<size_t>(bytes, 256)));
 }
 
 HipMemory::~HipMemory()
@@ -76,14 +78,19 @@ HipDoubleBuffer::~HipDoubleBuffer()
     }
 }
 
-void HipDoubleBuffer::uploadBack(hipStream_t st)
+bool HipDoubleBuffer::uploadBack(hipStream_t st)
 {
     const int b = m_index ^ 1;
+    if(!m_host_touched[b] && !m_written_by_ops)
+        return false;
+    m_host_touched[b] = false;
     chkHip(hipMemcpyAsync(m_dev[b], m_host[b], m_elements * m_element_size, hipMemcpyHostToDevice, st));
+    return true;
 }
 
 void HipDoubleBuffer::downloadFront(hipStream_t st)
 {
+    m_host_touched[m_index] = true;
     chkHip(hipMemcpyAsync(m_host[m_index], m_dev[m_index], m_elements * m_element_size, hipMemcpyDeviceToHost, st));
 }
 
@@ -296,7 +303,8 @@ private:
 // Host window onto the back buffer of a batched tensor: no copies, the program moves the data.
 class HipBatchAccess : public TensorAccess {
 public:
-    HipBatchAccess(HipTensor &t, std::shared_ptr<HipDoubleBuffer> db) : m_t(t), m_db(db) {}
+    HipBatchAccess(HipTensor &t, std::shared_ptr<HipDoubleBuffer> db) : m_t(t), m_db(db), m_back(db->m_index ^ 1) {}
+    ~HipBatchAccess() { m_db->m_host_touched[m_back] = true; } // writes may have come after an upload
     Dims strides() override
     {
         Dims d;
@@ -304,7 +312,7 @@ public:
             d.push_back(s);
         return d;
     }
-    void *data() override { return (char *)m_db->hostBack() + m_t.m_offset * (int64_t)m_db->m_element_size; }
+    void *data() override { return (char *)back() + m_t.m_offset * (int64_t)m_db->m_element_size; }
     size_t index(const Dims &e) const
     {
         int64_t o = m_t.m_offset;
@@ -313,13 +321,20 @@ public:
         return (size_t)o;
     }
     double get(const Dims &e) override { return host_load(m_db->hostBack(), m_db->m_data_type, index(e)); }
-    void set(const Dims &e, double v) override { host_store(m_db->hostBack(), m_db->m_data_type, index(e), v); }
-    void *getAddr(const Dims &e) override { return (char *)m_db->hostBack() + index(e) * m_db->m_element_size; }
+    void set(const Dims &e, double v) override { host_store(back(), m_db->m_data_type, index(e), v); }
+    void *getAddr(const Dims &e) override { return (char *)back() + index(e) * m_db->m_element_size; }
     void copyBytesFrom(const Dims &e, const void *src, size_t size) override { memcpy(getAddr(e), src, size); }
 
 private:
+    void *back() // for writing
+    {
+        m_back = m_db->m_index ^ 1;
+        m_db->m_host_touched[m_back] = true;
+        return m_db->hostBack();
+    }
     HipTensor &m_t;
     std::shared_ptr<HipDoubleBuffer> m_db;
+    int m_back;
 };
 
 std::unique_ptr<TensorAccess> HipTensor::access()
@@ -339,6 +354,215 @@ std::shared_ptr<Tensor> HipTensor::slice(const Dims &offset, const Dims &size)
 
 Tensor::Stats HipTensor::stats() { return Tensor::stats(); }
 
+// ---------------------------------------------------------------- host copies
+
+// Planes to pixels: dst[p * C + c] = src[c * plane + p].  The fixed channel count lets the compiler build whole
+// vectors of the interleaved stream (three bytes' or halves' planes of an image: 1.7 ns per element with the general
+// loop over every element that this replaces, 0.2 ns here).
+template <typename T, int C>
+__attribute__((optimize("O3"))) static void interleave(T *__restrict__ dst, const T *__restrict__ src, int64_t plane, int64_t n)
+{
+    for(int64_t p = 0; p < n; p++)
+        for(int c = 0; c < C; c++)
+            dst[p * C + c] = src[c * plane + p];
+}
+
+template <typename T, int C>
+__attribute__((optimize("O3"))) static void deinterleave(T *__restrict__ dst, const T *__restrict__ src, int64_t plane, int64_t n)
+{
+    for(int64_t p = 0; p < n; p++)
+        for(int c = 0; c < C; c++)
+            dst[c * plane + p] = src[p * C + c];
+}
+
+// dst[i * db + j] = src[i + j * sa] for i < n, j < m: blocks of 16 x 16, so that a block's lines stay in the cache
+template <typename T>
+static void transpose(T *__restrict__ dst, int64_t db, const T *__restrict__ src, int64_t sa, int64_t n, int64_t m)
+{
+    if(db == m && m <= 4) {
+        switch(m) {
+        case 2: return interleave<T, 2>(dst, src, sa, n);
+        case 3: return interleave<T, 3>(dst, src, sa, n);
+        case 4: return interleave<T, 4>(dst, src, sa, n);
+        }
+    }
+    if(sa == n && n <= 4) {
+        switch(n) {
+        case 2: return deinterleave<T, 2>(dst, src, db, m);
+        case 3: return deinterleave<T, 3>(dst, src, db, m);
+        case 4: return deinterleave<T, 4>(dst, src, db, m);
+        }
+    }
+    for(int64_t i0 = 0; i0 < n; i0 += 16)
+        for(int64_t j0 = 0; j0 < m; j0 += 16)
+            for(int64_t i = i0; i < std::min(n, i0 + 16); i++)
+                for(int64_t j = j0; j < std::min(m, j0 + 16); j++)
+                    dst[i * db + j] = src[i + j * sa];
+}
+
+template <typename T>
+static void permute(T *dst, const std::vector<int64_t> &ds, const T *src, const std::vector<int64_t> &ss,
+                    const std::vector<int64_t> &ext)
+{
+    const int rank = (int)ext.size();
+    // the axes along which each side is contiguous
+    int a = -1, b = -1;
+    for(int j = 0; j < rank; j++) {
+        if(ss[j] == 1)
+            a = j;
+        if(ds[j] == 1)
+            b = j;
+    }
+    const bool runs = a >= 0 && a == b, swaps = a >= 0 && b >= 0 && a != b;
+    std::vector<int> outer;
+    for(int j = 0; j < rank; j++)
+        if(!(runs && j == a) && !(swaps && (j == a || j == b)))
+            outer.push_back(j);
+    std::vector<int64_t> c(rank, 0);
+    for(;;) {
+        int64_t so = 0, d = 0;
+        for(int j : outer) {
+            so += c[j] * ss[j];
+            d += c[j] * ds[j];
+        }
+        if(runs)
+            memcpy(dst + d, src + so, ext[a] * sizeof(T));
+        else if(swaps)
+            transpose(dst + d, ds[a], src + so, ss[b], ext[a], ext[b]);
+        else
+            dst[d] = src[so];
+        int k = (int)outer.size() - 1;
+        for(; k >= 0; k--) {
+            if(++c[outer[k]] < ext[outer[k]])
+                break;
+            c[outer[k]] = 0;
+        }
+        if(k < 0)
+            return;
+    }
+}
+
+void hip_permute(void *dst, std::vector<int64_t> ds, const void *src, std::vector<int64_t> ss, std::vector<int64_t> ext,
+                 size_t es)
+{
+    // axes of one element say nothing; neighbours that are one run on both sides are one axis
+    for(size_t j = ext.size(); j-- > 0;) {
+        const bool merge = j + 1 < ext.size() && ss[j] == ext[j + 1] * ss[j + 1] && ds[j] == ext[j + 1] * ds[j + 1];
+        if(ext[j] != 1 && !merge)
+            continue;
+        if(ext[j] != 1)
+            ext[j + 1] *= ext[j];
+        ext.erase(ext.begin() + j);
+        ss.erase(ss.begin() + j);
+        ds.erase(ds.begin() + j);
+    }
+    switch(es) {
+    case 1: return permute((uint8_t *)dst, ds, (const uint8_t *)src, ss, ext);
+    case 2: return permute((uint16_t *)dst, ds, (const uint16_t *)src, ss, ext);
+    case 4: return permute((uint32_t *)dst, ds, (const uint32_t *)src, ss, ext);
+    default: return permute((uint64_t *)dst, ds, (const uint64_t *)src, ss, ext);
+    }
+}
+
+// row-major strides of the extents of a view
+static void row_major(SagaTensorView &v)
+{
+    int64_t acc = 1;
+    for(int j = 3; j >= 0; j--) {
+        v.strides[j] = acc;
+        acc *= v.dims[j];
+    }
+}
+
+// Up to STAGE_BYTES a tensor goes through pinned memory that a kernel reads or writes over PCIe itself, in the tensor's
+// own layout: one copy of the host's and one launch.  Larger ones are cheaper to hand to the runtime's copy (27 GB/s
+// from pageable memory, more than one core copies), sample by sample through device memory where the layout changes.
+void HipTensor::writeHost(const void *src)
+{
+    const size_t es = m_storage->m_element_size, bytes = m_dims.elements() * es;
+    if(m_storage->doubleBuffered()) {
+        auto ta = access();
+        const std::vector<int64_t> ext = m_dims.i64();
+        std::vector<int64_t> ss(ext.size(), 1);
+        for(ssize_t j = (ssize_t)ext.size() - 2; j >= 0; j--)
+            ss[j] = ss[j + 1] * ext[j + 1];
+        hip_permute(ta->data(), m_strides, src, ss, ext, es);
+        return;
+    }
+    HipContext &ctx = *m_storage->m_ctx;
+    hipStream_t st = ctx.m_stream;
+    SagaTensorView dv = view(), hv = dv;
+    row_major(hv);
+    if(bytes <= HipContext::STAGE_BYTES) {
+        std::lock_guard<std::mutex> lock(ctx.m_stage_mutex);
+        hv.ptr = ctx.stage(bytes);
+        memcpy(hv.ptr, src, bytes);
+        chkSaga(saga_hip_copy(&hv, &dv, (saga_stream_t)st));
+        chkHip(hipEventRecord(ctx.m_stage_event, st));
+        return;
+    }
+    ctx.sync();
+    if(rowMajor()) {
+        chkHip(hipMemcpy(dv.ptr, src, bytes, hipMemcpyHostToDevice));
+        return;
+    }
+    const size_t sample = bytes / dv.dims[0];
+    const int per = (int)std::max<size_t>(1, std::min<size_t>(dv.dims[0], (16 << 20) / sample));
+    HipMemory scratch(per * sample, false);
+    for(int n = 0; n < dv.dims[0]; n += per) {
+        SagaTensorView a = hv, b = dv;
+        a.dims[0] = b.dims[0] = std::min(per, dv.dims[0] - n);
+        a.ptr = scratch.m_ptr;
+        b.ptr = (char *)dv.ptr + n * dv.strides[0] * (int64_t)es;
+        chkHip(hipMemcpy(a.ptr, (const char *)src + n * sample, a.dims[0] * sample, hipMemcpyHostToDevice));
+        chkSaga(saga_hip_copy(&a, &b, (saga_stream_t)st));
+        chkHip(hipStreamSynchronize(st));
+    }
+}
+
+void HipTensor::readHost(void *dst)
+{
+    const size_t es = m_storage->m_element_size, bytes = m_dims.elements() * es;
+    if(m_storage->doubleBuffered()) {
+        const char *back = (const char *)std::static_pointer_cast<HipDoubleBuffer>(m_storage)->hostBack();
+        const std::vector<int64_t> ext = m_dims.i64();
+        std::vector<int64_t> ds(ext.size(), 1);
+        for(ssize_t j = (ssize_t)ext.size() - 2; j >= 0; j--)
+            ds[j] = ds[j + 1] * ext[j + 1];
+        hip_permute(dst, ds, back + m_offset * (int64_t)es, m_strides, ext, es);
+        return;
+    }
+    HipContext &ctx = *m_storage->m_ctx;
+    hipStream_t st = ctx.m_stream;
+    SagaTensorView dv = view(), hv = dv;
+    row_major(hv);
+    if(bytes <= HipContext::STAGE_BYTES) {
+        std::lock_guard<std::mutex> lock(ctx.m_stage_mutex);
+        hv.ptr = ctx.stage(bytes);
+        chkSaga(saga_hip_copy(&dv, &hv, (saga_stream_t)st));
+        ctx.sync();
+        memcpy(dst, hv.ptr, bytes);
+        return;
+    }
+    ctx.sync();
+    if(rowMajor()) {
+        chkHip(hipMemcpy(dst, dv.ptr, bytes, hipMemcpyDeviceToHost));
+        return;
+    }
+    const size_t sample = bytes / dv.dims[0];
+    const int per = (int)std::max<size_t>(1, std::min<size_t>(dv.dims[0], (16 << 20) / sample));
+    HipMemory scratch(per * sample, false);
+    for(int n = 0; n < dv.dims[0]; n += per) {
+        SagaTensorView a = hv, b = dv;
+        a.dims[0] = b.dims[0] = std::min(per, dv.dims[0] - n);
+        a.ptr = scratch.m_ptr;
+        b.ptr = (char *)dv.ptr + n * dv.strides[0] * (int64_t)es;
+        chkSaga(saga_hip_copy(&b, &a, (saga_stream_t)st));
+        chkHip(hipStreamSynchronize(st));
+        chkHip(hipMemcpy((char *)dst + n * sample, a.ptr, a.dims[0] * sample, hipMemcpyDeviceToHost));
+    }
+}
+
 // Fills this tensor from a front-end tensor: a straight memcpy when type and strides agree,
 // else element by element with conversion (also serves generated tensors, whose access
 // object produces a fresh random value per read).
@@ -350,27 +574,45 @@ void HipTensor::copyFromHost(Tensor &src)
     m_auto_initialized = ta->data() == nullptr;
     const size_t n = m_storage->m_elements;
     const size_t es = m_storage->m_element_size;
-    std::vector<uint8_t> host(std::max<size_t>(n * es, 16));
-    if(m_storage->m_ctx)
-        m_storage->m_ctx->sync();
-    chkHip(hipMemcpy(host.data(), m_storage->deviceMem(), n * es, hipMemcpyDeviceToHost));
-
     const size_t rank = m_dims.size(), srank = src.m_dims.size();
     if(src.m_dims.elements() != m_dims.elements())
         throw std::runtime_error("copyFromHost: element count mismatch " + src.info() + " -> " + info());
     const std::vector<int64_t> ext = m_dims.i64();
     const std::vector<int64_t> sext = src.m_dims.i64();
+    std::unique_ptr<uint8_t[]> owned(new uint8_t[std::max<size_t>(n * es, 16)]);
+    uint8_t *const host = owned.get();
+    if(m_storage->m_ctx)
+        m_storage->m_ctx->sync();
+    if(m_dims.elements() != n) // part of a storage: the rest stays
+        chkHip(hipMemcpy(host, m_storage->deviceMem(), n * es, hipMemcpyDeviceToHost));
     const Dims sstr = ta->strides();
     const void *sdata = ta->data();
     const bool fast = sdata != nullptr && src.m_data_type == m_data_type && sstr.size() == srank;
     std::vector<int64_t> sstr64;
     if(fast)
         sstr64 = sstr.i64();
+    // same type, and extents that differ in ones at most: a copy between two layouts
+    auto no_ones = [](std::vector<int64_t> v) {
+        v.erase(std::remove(v.begin(), v.end(), 1), v.end());
+        return v;
+    };
+    const bool layouts = fast && no_ones(ext) == no_ones(sext);
+    if(layouts) {
+        auto strides_of = [](const std::vector<int64_t> &e, const std::vector<int64_t> &st) {
+            std::vector<int64_t> v;
+            for(size_t j = 0; j < e.size(); j++)
+                if(e[j] != 1)
+                    v.push_back(st[j]);
+            return v;
+        };
+        hip_permute(host + m_offset * (int64_t)es, strides_of(ext, m_strides), sdata, strides_of(sext, sstr64),
+                    no_ones(ext), es);
+    }
     // iterate this tensor's logical coordinates; the source is walked in row-major order of
     // ITS OWN dims (ranks may differ, e.g. {C} params lowered to {1,C})
     std::vector<int64_t> c(rank, 0), sc(srank, 0);
     Dims se(srank, (int64_t)0);
-    for(size_t i = 0; i < n; i++) {
+    for(size_t i = 0; i < m_dims.elements() && !layouts; i++) {
         int64_t o = m_offset;
         for(size_t j = 0; j < rank; j++)
             o += c[j] * m_strides[j];
@@ -378,11 +620,11 @@ void HipTensor::copyFromHost(Tensor &src)
             int64_t so = 0;
             for(size_t j = 0; j < srank; j++)
                 so += sc[j] * sstr64[j];
-            memcpy(host.data() + o * es, (const char *)sdata + so * es, es);
+            memcpy(host + o * es, (const char *)sdata + so * es, es);
         } else {
             for(size_t j = 0; j < srank; j++)
                 se[j] = sc[j];
-            host_store(host.data(), m_data_type, (size_t)o, ta->get(se));
+            host_store(host, m_data_type, (size_t)o, ta->get(se));
         }
         for(ssize_t j = (ssize_t)rank - 1; j >= 0; j--) {
             if(++c[j] == ext[j])
@@ -400,11 +642,11 @@ void HipTensor::copyFromHost(Tensor &src)
     if(m_storage->doubleBuffered()) {
         auto db = std::static_pointer_cast<HipDoubleBuffer>(m_storage);
         for(int i = 0; i < 2; i++) {
-            memcpy(db->m_host[i], host.data(), n * es);
-            chkHip(hipMemcpy(db->m_dev[i], host.data(), n * es, hipMemcpyHostToDevice));
+            memcpy(db->m_host[i], host, n * es);
+            chkHip(hipMemcpy(db->m_dev[i], host, n * es, hipMemcpyHostToDevice));
         }
     } else {
-        chkHip(hipMemcpy(m_storage->deviceMem(), host.data(), n * es, hipMemcpyHostToDevice));
+        chkHip(hipMemcpy(m_storage->deviceMem(), host, n * es, hipMemcpyHostToDevice));
     }
 }
 
