@@ -13,7 +13,9 @@
 // element.  fp32 matrix instructions run at 1/16 of the fp16 rate, so plain register-staged tiles
 // (global -> registers -> LDS, one barrier per slice, the next slice's loads in flight during the
 // MFMAs) keep them busy; none of the fp16 path's load-to-LDS pipelining is needed here.
-#include "conv.hpp"
+#include "stream_f32.hpp"
+
+#include <algorithm>
 
 namespace {
 
@@ -826,13 +828,14 @@ size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorVie
 {
     if(!f32_ok(x, w, y, g))
         return 0;
+    const size_t stream = kind == SAGA_CONV_BWD_FILTER ? 0 : stream_f32_conv_workspace(kind == SAGA_CONV_BWD_DATA, g) + 256;
     if(kind == SAGA_CONV_FWD) {
         const size_t a = tab_bytes(g.C * g.R * g.S), b = plan_uniform(g.C * g.R * g.S, g.K).bytes;
-        return (a > b ? a : b) + 256;
+        return std::max(stream, (a > b ? a : b) + 256);
     }
     if(kind == SAGA_CONV_BWD_DATA) {
         const size_t a = tab_bytes(g.K * g.R * g.S), b = plan_uniform(g.K * g.R * g.S, g.C).bytes;
-        return (a > b ? a : b) + 256;
+        return std::max(stream, (a > b ? a : b) + 256);
     }
     const FilterSplit p = plan_filter_f32(g), pu = plan_filter_uniform(g);
     const int splits = p.splits > pu.splits ? p.splits : pu.splits;
@@ -845,6 +848,17 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
     // forward: a = x (N,C,H,W), out = y (N,K,P,Q); backward data: a = dy (N,K,P,Q), out = dx (N,C,H,W)
     const int red_ch = bwd ? g.K : g.C;
     const int Kred = red_ch * g.R * g.S;
+    // Operands shared through LDS pay once there are several rounds of full tiles: 537 against 562 us on 3x3 64->64 at
+    // 256x56x56, 478 against 500 us on 3x3 32->464 at 36x70x70 (1x1 64->256 at 8x56x56, one round: equal).  Reduction channels
+    // in other numbers than eights go through a table in both kernels, and the stream kernel's is read by every lane: 42
+    // against 53 us on 7x7 3->64 at 8x224x224.
+    const int cols = out->dims[1], bn = cols > 64 ? 128 : 64;
+    const long long tiles = ((long long)out->dims[0] * out->dims[2] * out->dims[3] + FBM - 1) / FBM * ((cols + bn - 1) / bn);
+    if(!(tiles >= (red_ch % 8 ? 512 : 2048) && cols > 48 && uniform_ok(bwd, a, g))) {
+        const int r = stream_f32_conv(bwd, a, w, out, g, alpha, beta, StreamEpilogue(), ws, ws_bytes, st);
+        if(r != SAGA_HIP_EUNSUPPORTED)
+            return r;
+    }
     if(!ws || ws_bytes < tab_bytes(Kred) || !aligned16(ws))
         return SAGA_HIP_EWORKSPACE;
     if(uniform_ok(bwd, a, g)) {

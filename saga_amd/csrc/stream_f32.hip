@@ -1,0 +1,618 @@
+// fp32 matrix products on v_mfma_f32_32x32x2_f32 straight from global memory.
+//
+// An fp32 matrix instruction keeps the matrix unit busy for 64 cycles with 256 bytes of each operand, so a wavefront
+// that loads its own operands from the caches into registers needs 8 - 16 bytes per cycle and SIMD's share of the L1:
+// there is nothing for LDS tiles to save, and without them there are no barriers, no LDS traffic and no block-wide
+// steps.  A wavefront owns a tile of 32*TM lanes-side elements (pixels of the image written, or columns of the row-major
+// GEMM result) x 32*TN others (output channels, or GEMM rows) and a range of the reduction; it loads eight reduction
+// indices at a time, DEPTH - 1 steps ahead of the multiplications (the loads of a step are independent, so the compiler's
+// counted waits leave the later ones in flight).  The reduction order inside a step is free as long as both operands
+// agree: lanes 0 - 31 take indices 0 - 3, lanes 32 - 63 indices 4 - 7, so that an operand whose reduction index is
+// contiguous in memory is one 16-byte load.
+//
+// Small problems fill the chip by splitting the reduction over the KS wavefronts of a block, which add up through LDS
+// at the end: one launch, no partial results in memory, a fixed order of additions.
+//
+// Measured against the LDS-tiled kernels that did all of this before (us; graph replays, launch included): fc 64x3136 ->
+// 1024 306 -> 21 (12.8 MB of weights, 0.6 TB/s), its backward data 95 -> 14; 4096^3 2433 -> 1038 (132 TFLOP/s); 3x3
+// 512->512 at 8x7x7 499 -> 50, 256->256 at 8x14x14 249 -> 44, at 32x14x14 250 -> 96 (77 TFLOP/s); stride-2 backward data
+// of 3x3 128->128 at 8x56x56 292 -> 55.  A fp32 ResNet-50 batch of 8 7.5 -> 2.1 ms.  What bounds the small ones now is
+// the launch, the first trip to memory and, under filters larger than 1x1, the copy of the filter in front.
+#include "stream_f32.hpp"
+
+#include <string.h>
+#include <algorithm>
+
+namespace {
+
+// The lanes-side operand P: PTAP: addressed by tap and channel, the channel count a multiple of eight (also a matrix
+// with the lanes' index contiguous); PTAB: by a table of all reduction indices; PROW: reduction index contiguous.
+// The other operand Q: QROW: reduction index contiguous; QCOL: row index contiguous; QTAB: by the same table.
+enum { PTAP, PTAB, PROW };
+enum { QROW, QCOL, QTAB };
+
+constexpr int MAX_CLASSES = 16;
+constexpr int MAX_TABLE = 4096; // reduction indices of a table
+
+// Output pixels whose taps sit at the same distances.  Forward: one class, all pixels.  Backward data at stride s: pixels
+// (y, x) with the same y mod s and x mod s; inside a class consecutive taps are a fixed distance apart.
+struct Class {
+    int oy, ox;   // output pixel = class pixel * ostep + (oy, ox)
+    int OH, OW;   // the class's grid
+    int r0, s0;   // first tap
+    int Tr, Ts;   // taps
+    int iy0, ix0; // input position of class pixel (0, 0) under its first tap
+    int M;        // class pixels over all samples
+    int block0;   // first block
+    long long q0; // first element of the class's rows in a packed filter
+};
+
+template <int CLASSES> struct ArgsOf {
+    const float *p, *q;
+    float *out;
+    unsigned p_bytes, q_bytes;
+    int N, C; // rows of Q; reduction channels per tap
+    int IH, IW, OH, OW;
+    int istep, ostep;      // input pixels per class pixel, output pixels per class pixel
+    int tstep;             // input pixels per tap (negative: backward)
+    int rstep;             // filter rows per tap row
+    long long p_sn, p_sc, p_sh, p_sw;
+    long long o_sn, o_sc, o_sh, o_sw;
+    long long q_sn, q_sc, q_sr, q_ss;
+    float alpha, beta;
+    const float *bias, *bn_s, *bn_b, *bn_m, *bn_v, *z;
+    float bn_eps;
+    int relu;
+    long long z_sn, z_sc, z_sh, z_sw;
+    int nclasses, nblk_q, blocks, KS;
+    Class cls[CLASSES];
+};
+typedef ArgsOf<MAX_CLASSES> Args;
+typedef ArgsOf<1> Args1; // a kilobyte less to fetch before anything else can start
+
+constexpr unsigned OOB = 0x7fffff00u; // beyond every buffer: the load returns zero
+
+__device__ __forceinline__ float load1(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s)
+{
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, v, s, 0));
+}
+__device__ __forceinline__ float4_t load4(__amdgpu_buffer_rsrc_t r, unsigned v, unsigned s)
+{
+    return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
+}
+
+__device__ __forceinline__ int xcd_order(int b, int n)
+{
+    const int per = n >> 3, rem = n & 7, xcd = b & 7, slot = b >> 3;
+    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + slot;
+}
+
+template <int PM, int QM, int TM, int TN, int DEPTH, int MAXW, typename A>
+__global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
+{
+    extern __shared__ __attribute__((aligned(16))) float smem[];
+    const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, fk = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int KS = g.KS, WM = (int)(blockDim.x >> 6) / KS;
+    const int wm = wave / KS, ks = wave - wm * KS;
+    int b = xcd_order(blockIdx.x, g.blocks), ci = 0;
+    while(sizeof(A) > sizeof(Args1) && ci + 1 < g.nclasses && b >= g.cls[ci + 1].block0)
+        ci++;
+    const Class &c = g.cls[ci];
+    b -= c.block0;
+    const int bm = b / g.nblk_q, bq = b - bm * g.nblk_q;
+    const int m0 = (bm * WM + wm) * (32 * TM), n0 = bq * (32 * TN);
+    const int T = c.Tr * c.Ts;
+    const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)g.p, 0, (int)g.p_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)g.q, 0, (int)g.q_bytes, 0x00020000);
+
+    // this lane's pixels: byte offset of the first tap (negative outside the image: only valid taps are read) and one
+    // bit per tap that falls inside
+    int base[TM];
+    unsigned long long mask[TM];
+    bool ok[TM];
+#pragma unroll
+    for(int i = 0; i < TM; i++) {
+        const int m = m0 + 32 * i + fr;
+        ok[i] = m < c.M;
+        const int mm = ok[i] ? m : 0;
+        const int ox = mm % c.OW, t = mm / c.OW;
+        const int oy = t % c.OH, n = t / c.OH;
+        const int iy = oy * g.istep + c.iy0, ix = ox * g.istep + c.ix0;
+        base[i] = (int)((n * g.p_sn + iy * g.p_sh + ix * g.p_sw + (PM == PTAP ? 4 * fk * g.p_sc : PM == PROW ? 4 * fk : 0)) * 4);
+        mask[i] = 0;
+        if(PM == PROW || !ok[i])
+            mask[i] = ok[i] ? 1 : 0;
+        else
+            for(int a = 0; a < c.Tr; a++) {
+                const int yy = iy + a * g.tstep;
+                if(yy < 0 || yy >= g.IH)
+                    continue;
+                for(int e = 0; e < c.Ts; e++) {
+                    const int xx = ix + e * g.tstep;
+                    if(xx >= 0 && xx < g.IW)
+                        mask[i] |= 1ull << (a * c.Ts + e);
+                }
+            }
+    }
+    const int kred = T * g.C;
+    unsigned qoff[TN];
+    bool nok[TN];
+#pragma unroll
+    for(int t = 0; t < TN; t++) {
+        const int n = n0 + 32 * t + fr;
+        nok[t] = n < g.N;
+        const long long o = QM == QROW ? c.q0 + (long long)n * (g.q_sn ? g.q_sn : kred) + 4 * fk : QM == QCOL ? c.q0 + n + 4 * fk * g.q_sc : n * g.q_sn;
+        qoff[t] = nok[t] ? (unsigned)(o * 4) : OOB;
+    }
+
+    // table: byte offsets of both operands and the tap of every reduction index, eight dead entries behind the last
+    int4 *tab = (int4 *)smem;
+    const int S8 = PM == PTAB ? (kred + 7) / 8 : g.C / 8; // steps per tap; of the whole reduction with a table
+    const int total = PM == PTAB ? S8 : S8 * T;
+    if constexpr(PM == PTAB) {
+        for(int k = tid; k < total * 8 + 8; k += blockDim.x) {
+            int4 e = {0, 63, (int)OOB, 0};
+            if(k < kred) {
+                const int ch = k / T, tap = k - ch * T, a = tap / c.Ts, s = tap - a * c.Ts;
+                e.x = (int)((ch * g.p_sc + a * g.tstep * g.p_sh + s * g.tstep * g.p_sw) * 4);
+                e.y = tap;
+                e.z = (int)((ch * g.q_sc + (c.r0 + a * g.rstep) * g.q_sr + (c.s0 + s * g.rstep) * g.q_ss) * 4);
+            }
+            tab[k] = e;
+        }
+        __syncthreads();
+    }
+    const int s_begin = (int)((long long)ks * total / KS), s_end = (int)((long long)(ks + 1) * total / KS);
+
+    // next step to be loaded: channels 8 * c8 ... of tap (ta, te)
+    int s_next = s_begin, tap = PM == PTAB || !total ? 0 : s_begin / S8, c8 = PM == PTAB ? 0 : s_begin - tap * S8;
+    int ta = c.Ts ? tap / c.Ts : 0, te = tap - ta * c.Ts;
+    unsigned pv[TM];
+    const int dh = (int)(g.tstep * g.p_sh * 4), dw = (int)(g.tstep * g.p_sw * 4);
+    auto tap_setup = [&]() {
+        const int d = PM == PTAP ? ta * dh + te * dw : 0;
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+            pv[i] = (mask[i] >> tap) & 1 ? (unsigned)(base[i] + d) : OOB;
+    };
+    if(PM != PTAB)
+        tap_setup();
+    const unsigned psc4 = (unsigned)(g.p_sc * 4), qsc4 = (unsigned)(g.q_sc * 4);
+
+    float pr[DEPTH][TM][4];
+    float4_t qr[DEPTH][TN];
+    auto load_step = [&](int u) {
+        const bool live = s_next < s_end;
+        if constexpr(PM == PTAB) {
+            const int4 *e = tab + (live ? s_next : total) * 8 + 4 * fk;
+#pragma unroll
+            for(int j = 0; j < 4; j++) {
+                const int4 w = e[j];
+#pragma unroll
+                for(int i = 0; i < TM; i++)
+                    pr[u][i][j] = load1(rp, (mask[i] >> w.y) & 1 ? (unsigned)(base[i] + w.x) : OOB, 0);
+#pragma unroll
+                for(int t = 0; t < TN; t++)
+                    qr[u][t][j] = load1(rq, nok[t] && w.y < 63 ? qoff[t] + (unsigned)w.z : OOB, 0);
+            }
+        } else {
+#pragma unroll
+            for(int i = 0; i < TM; i++) {
+                const unsigned v = live ? pv[i] : OOB;
+                if constexpr(PM == PROW) {
+                    const float4_t f = load4(rp, v, (unsigned)(c8 * 32));
+#pragma unroll
+                    for(int j = 0; j < 4; j++)
+                        pr[u][i][j] = f[j];
+                } else {
+#pragma unroll
+                    for(int j = 0; j < 4; j++)
+                        pr[u][i][j] = load1(rp, v, (unsigned)(c8 * 8 + j) * psc4);
+                }
+            }
+#pragma unroll
+            for(int t = 0; t < TN; t++) {
+                const unsigned v = live ? qoff[t] : OOB;
+                if constexpr(QM == QROW) {
+                    qr[u][t] = load4(rq, v, (unsigned)(s_next * 32));
+                } else {
+#pragma unroll
+                    for(int j = 0; j < 4; j++)
+                        qr[u][t][j] = load1(rq, v, (unsigned)(s_next * 8 + j) * qsc4);
+                }
+            }
+            if(++c8 == S8) {
+                c8 = 0;
+                tap++;
+                if(++te == c.Ts) {
+                    te = 0;
+                    ta++;
+                }
+                if(s_next + 1 < s_end)
+                    tap_setup();
+            }
+        }
+        s_next++;
+    };
+
+    float16_t acc[TM][TN];
+#pragma unroll
+    for(int i = 0; i < TM; i++)
+#pragma unroll
+        for(int t = 0; t < TN; t++)
+#pragma unroll
+            for(int v = 0; v < 16; v++)
+                acc[i][t][v] = 0.0f;
+    auto multiply = [&](const float(&a)[TM][4], const float4_t(&b)[TN]) {
+#pragma unroll
+        for(int j = 0; j < 4; j++)
+#pragma unroll
+            for(int i = 0; i < TM; i++)
+#pragma unroll
+                for(int t = 0; t < TN; t++)
+                    acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[t][j], a[i][j], acc[i][t], 0, 0, 0);
+    };
+    // a matrix whose reduction length is no multiple of eight: the last, partial step, each index tested; requested
+    // first, so that a short reduction pays one trip to memory
+    float tp[TM][4];
+    float4_t tq[TN];
+    const bool tail = PM != PTAB && g.C % 8 && ks == KS - 1;
+    if(tail) {
+#pragma unroll
+        for(int j = 0; j < 4; j++) {
+            const int k = S8 * 8 + 4 * fk + j;
+#pragma unroll
+            for(int i = 0; i < TM; i++)
+                tp[i][j] = load1(rp, ok[i] && k < g.C ? (unsigned)(base[i] + (PM == PROW ? (S8 * 8 + j) * 4 : (int)((S8 * 8 + j) * psc4))) : OOB, 0);
+#pragma unroll
+            for(int t = 0; t < TN; t++)
+                tq[t][j] = load1(rq, nok[t] && k < g.C ? qoff[t] + (QM == QROW ? (unsigned)((S8 * 8 + j) * 4) : (unsigned)(S8 * 8 + j) * qsc4) : OOB, 0);
+        }
+    }
+#pragma unroll
+    for(int u = 0; u < DEPTH - 1; u++)
+        load_step(u);
+    for(int s = s_begin; s < s_end; s += DEPTH) {
+#pragma unroll
+        for(int u = 0; u < DEPTH; u++) {
+            load_step((u + DEPTH - 1) % DEPTH);
+            if(s + u < s_end)
+                multiply(pr[u], qr[u]);
+        }
+    }
+    if(tail)
+        multiply(tp, tq);
+
+    // acc[i][t][v]: pixel m0 + 32*i + lane%32, channel n0 + 32*t + 8*(v/4) + 4*(lane/32) + v%4
+    long long opos[TM], zpos[TM];
+#pragma unroll
+    for(int i = 0; i < TM; i++) {
+        const int mm = ok[i] ? m0 + 32 * i + fr : 0;
+        const int ox = mm % c.OW, t = mm / c.OW;
+        const int oy = t % c.OH, n = t / c.OH;
+        const int y = oy * g.ostep + c.oy, x = ox * g.ostep + c.ox;
+        opos[i] = n * g.o_sn + y * g.o_sh + x * g.o_sw;
+        zpos[i] = n * g.z_sn + y * g.z_sh + x * g.z_sw;
+    }
+    auto store = [&](bool pok, long long op, long long zp, int t, int v, float val) {
+        const int n = n0 + 32 * t + 8 * (v >> 2) + 4 * fk + (v & 3);
+        if(!pok || n >= g.N)
+            return;
+        val *= g.alpha;
+        float *o = g.out + op + n * g.o_sc;
+        if(g.beta != 0.0f)
+            val += g.beta * *o;
+        if(g.bias)
+            val += g.bias[n];
+        if(g.bn_s) {
+            const float sc = g.bn_s[n] * rsqrtf(g.bn_v[n] + g.bn_eps);
+            val = __builtin_fmaf(val, sc, g.bn_b[n] - g.bn_m[n] * sc);
+        }
+        if(g.z)
+            val += g.z[zp + n * g.z_sc];
+        if(g.relu)
+            val = val != val ? val : fmaxf(val, 0.0f);
+        *o = val;
+    };
+    constexpr int NV = TM * TN * 16;
+    if(KS == 1) {
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+#pragma unroll
+            for(int t = 0; t < TN; t++)
+#pragma unroll
+                for(int v = 0; v < 16; v++)
+                    store(ok[i], opos[i], zpos[i], t, v, acc[i][t][v]);
+        return;
+    }
+    if(PM == PTAB)
+        __syncthreads(); // the table's memory is reused
+#pragma unroll
+    for(int i = 0; i < TM; i++)
+#pragma unroll
+        for(int t = 0; t < TN; t++)
+#pragma unroll
+            for(int v = 0; v < 16; v++)
+                smem[(wave * NV + (i * TN + t) * 16 + v) * 64 + lane] = acc[i][t][v];
+    __syncthreads();
+    const int per = NV / KS; // KS divides 16
+    for(int e = ks * per; e < (ks + 1) * per; e++) {
+        float sum = 0.0f;
+        for(int k = 0; k < KS; k++)
+            sum += smem[((wm * KS + k) * NV + e) * 64 + lane];
+        const int i = e / (16 * TN), t = (e >> 4) % TN;
+        const bool hi = TM > 1 && i;
+        store(hi ? ok[TM - 1] : ok[0], hi ? opos[TM - 1] : opos[0], hi ? zpos[TM - 1] : zpos[0], t, e & 15, sum);
+    }
+}
+
+// The filter in the order of the reduction, tap by tap: forward rows [n][tap][channel] for QROW, backward data
+// [class][tap][channel][n] for QCOL.  Consecutive lanes write consecutive elements and leave the gathering to the caches
+// (turning 64-channel pieces through LDS was 9 us slower on 512 -> 512 channels: too little in flight per block).
+__global__ void __launch_bounds__(256) stream_pack(Args g, const float *__restrict__ w, float *__restrict__ out, int cols)
+{
+    const Class &c = g.cls[blockIdx.y];
+    const int T = c.Tr * c.Ts;
+    const long long total = (long long)T * g.C * g.N;
+    for(long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
+        const int inner = cols ? g.N : g.C, e = (int)(i % inner), o = (int)(i / inner);
+        const int n = cols ? e : o / T, tap = cols ? o / g.C : o - n * T, ch = cols ? o - tap * g.C : e;
+        const int a = tap / c.Ts, s = tap - a * c.Ts;
+        out[c.q0 + i] = w[n * g.q_sn + ch * g.q_sc + (c.r0 + a * g.rstep) * g.q_sr + (c.s0 + s * g.rstep) * g.q_ss];
+    }
+}
+
+struct Config {
+    int tm, tn, ks, wm;
+};
+
+// Tile (32*tm x 32*tn per wavefront), wavefronts of a block along the reduction (ks) and along the pixels (wm) for
+// `pixels` x N results with `steps` reduction steps of eight.  Large tiles reuse what they load, small ones and splits
+// fill 1024 SIMDs: the limits are where the measured times cross (us, tm,tn,ks,wm; launches of 4 - 10 us included):
+//   3x3 256->256, 32x14x14   2,2,4,1  93   2,1,4,1 101   1,1,4,1 115   2,2,1,4 199
+//   3x3 256->256,  8x14x14   2,1,4,1  41   1,1,8,1  42   1,1,16,1 48   2,2,4,1  62
+//   3x3 512->512,  8x7x7     1,1,8,1  50   2,1,4,1  69   2,2,4,1 111
+//   1x1 1024->256, 8x14x14   1,1,4,1  18   2,1,4,1  20   1,1,1,4  33
+//   1x1 64->256,   8x56x56   2,1,1,4  22   1,1,1,4  23   1,1,4,1  37
+//   fc 64x3136 -> 1024       1,1,8,1  21   1,1,4,1  26   2,1,4,1  44   2,2,1,4 244
+Config choose(long long pixels, int N, long long steps)
+{
+    auto tiles = [&](int tm, int tn) { return ((pixels + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
+    const int tn = N > 32 ? 2 : 1;
+    if(tiles(2, tn) >= 2048)
+        return {2, tn, 1, 4};
+    if(tiles(2, tn) >= 384 && steps >= 128)
+        return {2, tn, 4, 1};
+    if(tiles(2, 1) >= 256 && steps >= 48)
+        return {2, 1, 4, 1};
+    if(tiles(2, 1) >= 1536)
+        return {2, 1, 1, 4};
+    int ks = 1;
+    while(ks < 16 && tiles(1, 1) * ks < 2048 && steps >= 16 * ks)
+        ks *= 2;
+    return {1, 1, ks, ks >= 4 ? 1 : 4 / ks};
+}
+
+template <int PM, int QM, typename A> int launch_as(const A &k, const Config &cf, int threads, size_t lds, hipStream_t st)
+{
+#define GO(TM, TN, DEPTH, MAXW)                                                                                        \
+    do {                                                                                                               \
+        auto kern = stream_f32_k<PM, QM, TM, TN, DEPTH, MAXW, A>;                                                      \
+        static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, \
+                                                           (MAX_TABLE + 8) * 16);                                      \
+        if(attr != hipSuccess)                                                                                         \
+            return (int)attr;                                                                                          \
+        kern<<<k.blocks, threads, lds, st>>>(k);                                                                       \
+    } while(0)
+    if(cf.tm == 2 && cf.tn == 2)
+        GO(2, 2, 3, 4);
+    else if(cf.tm == 2)
+        GO(2, 1, 4, 4);
+    else
+        GO(1, 1, 6, 16);
+#undef GO
+    SAGA_CHECK_LAUNCH();
+    return 0;
+}
+
+template <int PM, int QM> int launch(Args &g, hipStream_t st, long long pixels, long long steps)
+{
+    const Config cf = choose(pixels, g.N, steps);
+    g.KS = cf.ks;
+    g.nblk_q = (g.N + 32 * cf.tn - 1) / (32 * cf.tn);
+    long long blocks = 0;
+    for(int i = 0; i < g.nclasses; i++) {
+        g.cls[i].block0 = (int)blocks;
+        blocks += ((g.cls[i].M + 32ll * cf.tm * cf.wm - 1) / (32 * cf.tm * cf.wm)) * g.nblk_q;
+    }
+    if(blocks > 0x7fffffff)
+        return SAGA_HIP_EUNSUPPORTED;
+    g.blocks = (int)blocks;
+    const int threads = 64 * cf.ks * cf.wm;
+    size_t lds = cf.ks > 1 ? (size_t)cf.ks * cf.wm * cf.tm * cf.tn * 16 * 256 : 0;
+    if(PM == PTAB) {
+        int T = 0;
+        for(int i = 0; i < g.nclasses; i++)
+            T = std::max(T, g.cls[i].Tr * g.cls[i].Ts);
+        lds = std::max(lds, (size_t)((T * g.C + 7) / 8 * 8 + 8) * 16);
+    }
+    if(g.nclasses > 1)
+        return launch_as<PM, QM, Args>(g, cf, threads, lds, st);
+    Args1 one;
+    memcpy(&one, &g, sizeof(one)); // the same members up to the first class
+    return launch_as<PM, QM, Args1>(one, cf, threads, lds, st);
+}
+
+long long extent(const SagaTensorView *v)
+{
+    long long e = 1;
+    for(int i = 0; i < 4; i++) {
+        if(v->strides[i] < 0)
+            return -1;
+        e += (long long)(v->dims[i] - 1) * v->strides[i];
+    }
+    return e * 4;
+}
+
+int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }
+
+// the classes of a convolution and how its taps step; false if there are too many
+bool classes(bool bwd, const ConvGeom &g, Args &a)
+{
+    const int s = bwd ? g.stride : 1;
+    if(s * s > MAX_CLASSES)
+        return false;
+    a.nclasses = s * s;
+    a.istep = bwd ? 1 : g.stride;
+    a.ostep = s;
+    const int q = gcd(s, g.dil);
+    a.rstep = s / q;
+    a.tstep = bwd ? -g.dil / q : g.dil;
+    const int OH = bwd ? g.H : g.P, OW = bwd ? g.W : g.Q;
+    long long at = 0;
+    for(int i = 0; i < a.nclasses; i++) {
+        Class &c = a.cls[i];
+        c.oy = i / s;
+        c.ox = i % s;
+        c.OH = (OH - c.oy + s - 1) / s;
+        c.OW = (OW - c.ox + s - 1) / s;
+        auto axis = [&](int o, int taps, int &first, int &n, int &pos) {
+            for(first = 0; first < a.rstep && (o + g.pad - first * g.dil) % s; first++)
+                ;
+            if(!bwd) {
+                n = taps;
+                pos = -g.pad;
+                return;
+            }
+            n = first < a.rstep && first < taps ? (taps - first + a.rstep - 1) / a.rstep : 0;
+            pos = n ? (o + g.pad - first * g.dil) / s : 0; // divides
+        };
+        axis(c.oy, g.R, c.r0, c.Tr, c.iy0);
+        axis(c.ox, g.S, c.s0, c.Ts, c.ix0);
+        if(!c.Tr || !c.Ts)
+            c.Tr = c.Ts = 0;
+        const long long M = (long long)g.N * c.OH * c.OW;
+        if(M >= 1ll << 31)
+            return false;
+        c.M = (int)M;
+        c.q0 = at;
+        at += (long long)c.Tr * c.Ts * g.C * g.K;
+    }
+    return true;
+}
+
+// the filter has to be copied into the order of the reduction
+bool packs(bool bwd, const ConvGeom &g) { return (bwd ? g.K : g.C) % 8 == 0 && !(g.R == 1 && g.S == 1 && g.stride == 1); }
+
+} // namespace
+
+size_t stream_f32_conv_workspace(bool bwd, const ConvGeom &g)
+{
+    return packs(bwd, g) ? (size_t)g.K * g.C * g.R * g.S * sizeof(float) : 0;
+}
+
+int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g,
+                    float alpha, float beta, const StreamEpilogue &e, void *ws, size_t ws_bytes, hipStream_t st)
+{
+    Args k = {};
+    const long long pe = extent(a), qe = extent(w);
+    const long long limit = 0x7ffffe00ll;
+    const long long wlen = (long long)g.K * g.C * g.R * g.S * 4;
+    // (a pixel outside the image starts at an offset below the tensor; the sum with a valid tap's offset is inside again)
+    if(g.group != 1 || pe < 0 || qe < 0 || pe > limit || qe > limit || wlen > limit || !classes(bwd, g, k))
+        return SAGA_HIP_EUNSUPPORTED;
+    k.p = (const float *)a->ptr;
+    k.q = (const float *)w->ptr;
+    k.out = (float *)out->ptr;
+    k.p_bytes = (unsigned)pe;
+    k.q_bytes = (unsigned)qe;
+    k.N = out->dims[1];
+    k.C = a->dims[1];
+    k.IH = a->dims[2];
+    k.IW = a->dims[3];
+    k.p_sn = a->strides[0]; k.p_sc = a->strides[1]; k.p_sh = a->strides[2]; k.p_sw = a->strides[3];
+    k.o_sn = out->strides[0]; k.o_sc = out->strides[1]; k.o_sh = out->strides[2]; k.o_sw = out->strides[3];
+    k.q_sn = bwd ? w->strides[1] : w->strides[0];
+    k.q_sc = bwd ? w->strides[0] : w->strides[1];
+    k.q_sr = w->strides[2];
+    k.q_ss = w->strides[3];
+    k.alpha = alpha;
+    k.beta = beta;
+    k.bias = e.bias;
+    k.bn_s = e.bn_s; k.bn_b = e.bn_b; k.bn_m = e.bn_m; k.bn_v = e.bn_v;
+    k.bn_eps = e.bn_eps;
+    k.relu = e.relu;
+    if(e.z) {
+        k.z = (const float *)e.z->ptr;
+        k.z_sn = e.z->strides[0]; k.z_sc = e.z->strides[1]; k.z_sh = e.z->strides[2]; k.z_sw = e.z->strides[3];
+    }
+    const long long pixels = (long long)out->dims[0] * out->dims[2] * out->dims[3];
+    const long long steps = ((long long)k.C * g.R * g.S / k.nclasses + 7) / 8;
+    int taps = 0;
+    for(int i = 0; i < k.nclasses; i++)
+        taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
+    if(k.C % 8 == 0 && taps <= 64) {
+        if(packs(bwd, g)) {
+            if(!ws || ws_bytes < (size_t)wlen || !aligned16(ws))
+                return SAGA_HIP_EWORKSPACE;
+            const dim3 grid(grid_for(wlen / 4 / k.nclasses, 256, 4096), k.nclasses);
+            stream_pack<<<grid, 256, 0, st>>>(k, k.q, (float *)ws, bwd);
+            k.q = (const float *)ws;
+            k.q_bytes = (unsigned)wlen;
+            k.q_sn = 0; // rows as long as the class's reduction
+            k.q_sc = k.N;
+            return bwd ? launch<PTAP, QCOL>(k, st, pixels, steps) : launch<PTAP, QROW>(k, st, pixels, steps);
+        }
+        // 1x1: the filter as it is, if its rows are dense
+        if(!bwd && k.q_sc == 1)
+            return launch<PTAP, QROW>(k, st, pixels, steps);
+        if(bwd && k.q_sn == 1)
+            return launch<PTAP, QCOL>(k, st, pixels, steps);
+    }
+    if(taps <= 63 && (long long)taps * k.C <= MAX_TABLE - 8)
+        return launch<PTAB, QTAB>(k, st, pixels, steps);
+    return SAGA_HIP_EUNSUPPORTED;
+}
+
+int stream_f32_gemm(int tA, int tB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
+                    float beta, float *C, int ldc, const float *bias, int relu, hipStream_t st)
+{
+    Args k = {};
+    const long long ae = ((long long)(tA ? K - 1 : M - 1) * lda + (tA ? M : K)) * 4;
+    const long long be = ((long long)(tB ? N - 1 : K - 1) * ldb + (tB ? K : N)) * 4;
+    if(ae > 0x7ffffe00ll || be > 0x7ffffe00ll)
+        return SAGA_HIP_EUNSUPPORTED;
+    k.p = B;
+    k.q = A;
+    k.out = C;
+    k.p_bytes = (unsigned)be;
+    k.q_bytes = (unsigned)ae;
+    k.N = M;
+    k.C = K;
+    k.IH = k.IW = 1;
+    k.istep = k.ostep = 1;
+    k.nclasses = 1;
+    Class &c = k.cls[0];
+    c.OH = 1;
+    c.OW = 1; // "sample" n is column n
+    c.Tr = c.Ts = 1;
+    c.M = N;
+    k.p_sn = tB ? ldb : 1;
+    k.p_sc = tB ? 1 : ldb;
+    k.o_sn = 1;
+    k.o_sc = ldc;
+    k.q_sn = tA ? 1 : lda;
+    k.q_sc = tA ? lda : 1;
+    k.alpha = alpha;
+    k.beta = beta;
+    k.relu = relu;
+    if(bias) { // per column: read like a residual with no row stride
+        k.z = bias;
+        k.z_sn = 1;
+    }
+    const long long steps = (K + 7) / 8;
+    if(tB)
+        return tA ? launch<PROW, QCOL>(k, st, N, steps) : launch<PROW, QROW>(k, st, N, steps);
+    return tA ? launch<PTAP, QCOL>(k, st, N, steps) : launch<PTAP, QROW>(k, st, N, steps);
+}

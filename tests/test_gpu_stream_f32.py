@@ -1,0 +1,63 @@
+"""The fp32 matrix products that read their operands straight from memory (csrc/stream_f32.hip): one case per tile and per
+split of the reduction that the launch rule can choose, at sizes with remainders on every axis, forward and backward data
+against the oracle, and the GEMM's four operand orders with partial last steps."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ref
+from saga_amd import kernels as K
+from tests.gpu_util import assert_close, dev, host, rnd
+
+pytestmark = pytest.mark.gpu
+F32 = torch.float32
+
+# N, C, H, W, K, R, stride, pad
+CONVS = [
+    (2, 8, 255, 257, 65, 1, 1, 0),    # 64x64 tiles, four along the pixels
+    (1, 128, 150, 161, 64, 3, 1, 1),  # 64x64 tiles, the reduction over four wavefronts
+    (1, 48, 127, 131, 30, 3, 1, 1),   # 64x32 tiles, the reduction over four
+    (1, 16, 311, 317, 7, 1, 1, 0),    # 64x32 tiles, four along the pixels
+    (1, 512, 3, 5, 33, 3, 1, 1),      # 32x32, sixteen wavefronts along the reduction
+    (3, 64, 9, 7, 31, 1, 1, 0),       # 32x32, few steps per wavefront
+    (2, 24, 11, 13, 40, 3, 2, 1),     # residue classes backward, tap-major copy
+    (2, 16, 10, 9, 24, 2, 3, 0),      # stride beyond the filter: classes no tap reaches
+    (2, 13, 12, 11, 9, 5, 2, 2),      # table: channels in other numbers than eights
+    (1, 3, 23, 29, 16, 7, 2, 3),
+    (2, 8, 9, 9, 8, 3, 4, 1),
+]
+
+
+@pytest.mark.parametrize("shape", CONVS)
+@pytest.mark.parametrize("layout", ["nchw", "nhwc"])
+def test_conv(shape, layout):
+    N, Cc, H, W, Kk, R, stride, pad = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rnd(rng, N, Cc, H, W, dtype=F32)
+    w = rnd(rng, Kk, Cc, R, R, dtype=F32, scale=(2.0 / (Cc * R * R)) ** 0.5)
+    y_ref = ref.conv2d_fwd(x, w, pad, stride)
+    dy = rnd(rng, *y_ref.shape, dtype=F32)
+    xd, wd, dyd = dev(x, F32, layout), dev(w, F32, layout), dev(dy, F32, layout)
+    yd = dev(np.full(y_ref.shape, 7.0, np.float32), F32, layout)
+    K.conv2d(K.CONV_FWD, xd, wd, yd, pad, stride)
+    assert_close(host(yd), y_ref, F32, "y")
+    K.conv2d(K.CONV_FWD, xd, wd, yd, pad, stride, alpha=0.5, beta=1.0)
+    assert_close(host(yd), 1.5 * y_ref, F32, "accumulated y")
+    dxd = dev(np.full(x.shape, 7.0, np.float32), F32, layout)
+    K.conv2d(K.CONV_BWD_DATA, dyd, wd, dxd, pad, stride)
+    assert_close(host(dxd), ref.conv2d_bwd_data(dy, w, x.shape, pad, stride), F32, "dx")
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("size", [(64, 1030, 400), (33, 31, 17), (1, 1, 24), (5, 70, 1027), (130, 300, 65), (640, 2048, 20)])
+def test_gemm(tA, tB, size):
+    M, N, Kd = size
+    rng = np.random.default_rng(M + N + Kd)
+    A, B = rnd(rng, M, Kd, dtype=F32), rnd(rng, Kd, N, dtype=F32)
+    want = A.astype(np.float64) @ B.astype(np.float64)
+    Ad, Bd = dev(A.T if tA else A, F32), dev(B.T if tB else B, F32)
+    Cd = dev(np.ones((M, N), np.float32), F32)
+    stream = K.stream_ptr()
+    K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 2.0, K.ptr(Ad), Ad.shape[1], K.ptr(Bd), Bd.shape[1], 3.0, K.ptr(Cd), N,
+                                  K.FLOAT, stream))
+    assert_close(host(Cd), 2 * want + 3, F32, "C")
