@@ -18,6 +18,7 @@
 // fragment reads of a wavefront spread over the banks.
 // Blocks are renumbered so that consecutive tiles land on the same XCD and share its L2.
 #include "conv.hpp"
+#include "stream_f16.hpp"
 
 #include <stdlib.h>
 #include <algorithm>
@@ -71,6 +72,11 @@ struct GatherArgs {
     float *bq_partial;  // null: no link
     int no_stage;      // the epilogue stores straight from registers (experiment switch SAGA_HIP_NO_STAGED_STORES)
     int b_krsc;        // conv_rows64_wide<.., FLIP>: b is the filter as the forward pass has it (K,R,S,C), not transposed
+    // kernels instantiated with SPLIT: the reduction of a tile is shared by ksplit blocks, which leave their fp32 sums in
+    // part (see split_reduce)
+    int ksplit;
+    float4_t *part;
+    size_t part_bytes; // room behind part
     unsigned out_bytes; // extent of out, for the epilogue variant that stores through a range-checked buffer (BUFST)
     float *stats;      // forward only, optional: per block row and output channel, sum and sum of
                        // squares of the stored outputs, [ceil(M / BM)][Ngemm][2]
@@ -862,7 +868,7 @@ __device__ __forceinline__ void gather_epilogue_bnbwd(const GatherArgs &g, float
     }
 }
 
-template <int BM, int BN, int WGM, int WGN, int STAGES, int BKT, bool BWD, int PROD = 0, bool BQ = false>
+template <int BM, int BN, int WGM, int WGN, int STAGES, int BKT, bool BWD, int PROD = 0, bool BQ = false, bool SPLIT = false>
 __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PROD == 8) ? 4 : PROD ? (WGM * WGN + PROD + 3) / 4 : 1)
     conv_gather_gemm_dma(GatherArgs g)
 {
@@ -886,7 +892,11 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PR
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    int bid = xcd_remap(blockIdx.x, g.nblocks);
+    int bid = xcd_remap(blockIdx.x, SPLIT ? g.nblocks * g.ksplit : g.nblocks);
+    const int split = SPLIT ? bid / g.nblocks : 0;
+    if(SPLIT)
+        bid -= split * g.nblocks;
+    const int tile_id = bid;
     int py = 0, px = 0, r0 = 0, s0 = 0, nr = g.R, ns = g.S, rstep = 1;
     int PH = g.OH, PW = g.OW; // pixel grid this block's rows are numbered over
     int srow0 = 0;            // first row of this block's class in the per-row sums
@@ -961,9 +971,19 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PR
     };
     const int ktot = g.R * g.S * g.Cred;
     const int csteps = (g.Cred + BKT - 1) / BKT;
-    const int KT = nr * ns * csteps;
+    int KT = nr * ns * csteps;
     const bool ragged = g.Cred % BKT != 0;
     int ri = 0, si = 0, c0 = 0; // tap counters and channel offset of the NEXT slice to be issued
+    if constexpr(SPLIT) { // this block's slices
+        const int k0 = (int)((int64_t)split * KT / g.ksplit), k1 = (int)((int64_t)(split + 1) * KT / g.ksplit);
+        if(KT) {
+            const int tap = k0 / csteps;
+            c0 = (k0 - tap * csteps) * BKT;
+            ri = tap / ns;
+            si = tap - ri * ns;
+        }
+        KT = k1 - k0;
+    }
 
     // With PROD > 0 the block has PROD extra wavefronts that do nothing but issue the loads:
     // a load-to-LDS instruction holds its wavefront at issue until the memory pipeline takes
@@ -1059,7 +1079,7 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PR
                         produce((u + STAGES - 1) % STAGES);
                 }
             }
-            if constexpr(!BQ) {
+            if constexpr(!BQ && !SPLIT) {
                 if(!BWD && g.bn_s) { // the two barriers around the folded batch norm's parameter table
                     __syncthreads();
                     __syncthreads();
@@ -1263,6 +1283,18 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PR
         }
     }
 
+    if constexpr(SPLIT) {
+        // every wavefront's sums in the order it holds them: a store is a kilobyte in one piece
+        float4_t *part = g.part + ((int64_t)(split * g.nblocks + tile_id) * NW + wave) * (TM * TN * 4) * 64 + lane;
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+#pragma unroll
+            for(int j = 0; j < TN; j++)
+#pragma unroll
+                for(int q = 0; q < 4; q++)
+                    part[((i * TN + j) * 4 + q) * 64] = float4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+        return;
+    }
     if constexpr(BQ && PROD == 0)
         bnbwd_prefetch<TM, TN, 0, TM * TN>(g, lane, wn, n0, bq_ok, bq_pix, bq_x);
     if constexpr(BQ)
@@ -1270,6 +1302,150 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PR
                                                     bq_x, bq_tab);
     else
         gather_epilogue<TM, TN, WGM, WGN, BN, BWD, false>(g, acc, smem, tid, lane, wave, wm, wn, n0, bm, rowpix);
+}
+
+// ---------------------------------------------------------------- few tiles, long reductions
+//
+// A layer of few output pixels has too few 256-row tiles for the chip, and each of its blocks walks the whole reduction
+// alone (3x3 512->512 at 42x42 pixels of one image: 28 blocks, 144 slices, 50 us at 6 % of the matrix rate).  There the
+// reduction of a tile is shared by ksplit blocks (conv_gather_gemm_dma with SPLIT) and this kernel adds their fp32 sums, in
+// a fixed order, and does what the tile's own epilogue would have done: alpha, beta, the folded norm, the statistics, or
+// the link to a batch norm's backward.
+//
+// A block owns 128 pixels x 32 channels.  Thread t: pixel t % 32 of four 32-pixel groups (t / 128 and t / 128 + 2), channels
+// 8 * ((t / 32) % 4) .. + 7, which two lanes of the wavefront that computed them held: both reads of a wavefront are whole
+// half-kilobytes.
+template <int WGN, bool BWD, bool BQ> __global__ void __launch_bounds__(256) split_reduce(GatherArgs g)
+{
+    constexpr int WGM = 4, NW = WGM * WGN, BN = WGN * 64;
+    __shared__ float red[16][256 + 4];
+    const int t = threadIdx.x, p = t & 31, q = (t >> 5) & 3;
+    const int ncg = (g.Ngemm + 31) / 32;
+    int b = blockIdx.x;
+    const int cg = b % ncg;
+    b /= ncg;
+    const int rgs = (g.Mc + 127) / 128, ci = b / rgs, rg = b - ci * rgs; // class, 128-pixel group of it
+    int py = 0, px = 0;
+    if(BWD && g.classes > 1) {
+        py = g.cls_ids[ci] >> g.sshift;
+        px = g.cls_ids[ci] & (g.stride - 1);
+    }
+    const int bn = cg * 32 / BN, wx = cg * 32 / 64 % WGN, j = cg & 1;
+    // (classes of one tile position are neighbours in block order, see conv_gather_gemm_dma)
+    const int tile = ((rg >> 1) * g.nblk_n + bn) * (BWD && g.classes > 1 ? g.nactive : 1) + (BWD && g.classes > 1 ? ci : 0);
+    const int n = cg * 32 + 8 * q;
+    float sc[8], sh[8], mean[8];
+#pragma unroll
+    for(int e = 0; e < 8; e++) {
+        sc[e] = sh[e] = mean[e] = 0.0f;
+        if(n + e >= g.Ngemm)
+            continue;
+        if(BQ) {
+            mean[e] = g.bq_mean[n + e];
+            if(g.bq_relu) {
+                sc[e] = g.bq_s[n + e] * g.bq_invstd[n + e];
+                sh[e] = __builtin_fmaf(-mean[e], sc[e], g.bq_b[n + e]); // the forward's own expression
+            }
+        } else if(!BWD && g.bn_s) {
+            sc[e] = g.bn_s[n + e] * rsqrtf(g.bn_v[n + e] + g.bn_eps);
+            sh[e] = g.bn_b[n + e] - g.bn_m[n + e] * sc[e];
+        }
+    }
+    float s1[8], s2[8];
+#pragma unroll
+    for(int e = 0; e < 8; e++)
+        s1[e] = s2[e] = 0.0f;
+    const int64_t step = (int64_t)g.nblocks * NW * 16 * 64;
+#pragma unroll
+    for(int it = 0; it < 2; it++) {
+        const int grp = (t >> 7) + 2 * it; // 32-pixel group of the 128
+        const int wy = (rg & 1) * 2 + (grp >> 1), i = grp & 1;
+        const int m = rg * 128 + grp * 32 + p;
+        const float4_t *src = g.part + ((int64_t)tile * NW + wy * WGN + wx) * 16 * 64 + ((i * 2 + j) * 4 + q) * 64 + p;
+        float4_t lo = src[0], hi = src[32];
+        int k = 1;
+        for(; k + 3 < g.ksplit; k += 4) { // eight loads in flight
+            float4_t a[4], c[4];
+#pragma unroll
+            for(int u = 0; u < 4; u++) {
+                a[u] = src[(k + u) * step];
+                c[u] = src[(k + u) * step + 32];
+            }
+#pragma unroll
+            for(int u = 0; u < 4; u++) {
+                lo += a[u];
+                hi += c[u];
+            }
+        }
+        for(; k < g.ksplit; k++) {
+            lo += src[k * step];
+            hi += src[k * step + 32];
+        }
+        bool ok = m < g.Mc;
+        int64_t pix = m;
+        if(BWD && g.classes > 1) {
+            const int mm = ok ? m : 0, ox = mm % g.OWc, tt = mm / g.OWc, oy = tt % g.OHc, im = tt / g.OHc;
+            const int y = oy * g.stride + py, x = ox * g.stride + px;
+            ok = ok && y < g.OH && x < g.OW;
+            pix = ((int64_t)im * g.OH + y) * g.OW + x;
+        }
+        if(!ok || n >= g.Ngemm)
+            continue;
+        half8_t old = {}, z = {}, xx = {}, r;
+        half_t *o = g.out + pix * g.ldo + n;
+        if(g.beta != 0.0f)
+            old = *(const half8_t *)o;
+        if(!BWD && g.bn_s && (g.bn_flags & SAGA_BN_ADD))
+            z = *(const half8_t *)(g.z + pix * g.ldz + n);
+        if(BQ)
+            xx = *(const half8_t *)(g.bq_x + pix * g.bq_ldx + n);
+#pragma unroll
+        for(int e = 0; e < 8; e++) {
+            float f = g.alpha * (e < 4 ? lo[e & 3] : hi[e & 3]);
+            if(g.beta != 0.0f)
+                f += g.beta * (float)old[e];
+            if(!BWD && g.bn_s) {
+                f = __builtin_fmaf(f, sc[e], sh[e]);
+                if(g.bn_flags & SAGA_BN_ADD)
+                    f += (float)z[e];
+                if(g.bn_flags & SAGA_BN_RELU)
+                    f = (f != f) ? f : fmaxf(f, 0.0f);
+            }
+            r[e] = (half_t)f;
+            if(BQ) {
+                const float xf = (float)xx[e];
+                if(g.bq_relu && !((float)(half_t)__builtin_fmaf(xf, sc[e], sh[e]) > 0.0f))
+                    r[e] = (half_t)0;
+                s1[e] += (float)r[e];
+                s2[e] += (float)r[e] * (xf - mean[e]);
+            } else if(!BWD) {
+                s1[e] += (float)r[e];
+                s2[e] += (float)r[e] * (float)r[e];
+            }
+        }
+        *(half8_t *)o = r;
+    }
+    float *sums = BQ ? g.bq_partial : BWD ? nullptr : g.stats;
+    if(!sums)
+        return;
+#pragma unroll
+    for(int e = 0; e < 8; e++) {
+        red[e][t] = s1[e];
+        red[8 + e][t] = s2[e];
+    }
+    __syncthreads();
+    // channel 8 * q + e and quantity: the 64 threads with that q, in a fixed order, four partial sums each
+    const int v = t >> 2, part = t & 3, vq = v >> 4, ve = v & 15; // v = q * 16 + (quantity * 8 + e)
+    float sum = 0.0f;
+    for(int l = 0; l < 16; l++) {
+        const int idx = part * 16 + l; // of the 64: pixel idx % 32 of half idx / 32
+        sum += red[ve][(idx >> 5) * 128 + vq * 32 + (idx & 31)];
+    }
+    sum += __shfl_xor(sum, 1, 64);
+    sum += __shfl_xor(sum, 2, 64);
+    const int ch = cg * 32 + vq * 8 + (ve & 7);
+    if(part == 0 && ch < g.Ngemm)
+        sums[((int64_t)(ci * rgs + rg) * g.Ngemm + ch) * 2 + (ve >> 3)] = sum;
 }
 
 // Many filters in one launch: job j owns the blocks first_block[j] .. first_block[j+1]-1, one block per
@@ -3490,6 +3666,84 @@ static int tile_override()
     return v;
 }
 
+// How many blocks share the reduction of a tile (1: none), by the number of tiles and slices of 32.  Fitted to measured
+// times: a slice takes a block 0.36 us, a shared launch and its second kernel cost 9 us more than a plain one, and writing
+// and reading the sums of a 256x128 tile 33 ns; more blocks than CUs only add sums.  (us, alone -> shared by k:
+// 3x3 1024->1024 at 21x21 90 -> 28 k=10; 3x3 1024->512 at 42x42 96 -> 35 k=8; 3x3 512->512 at 64x7x7 50 -> 34 k=4;
+// at 128x7x7 52 -> 47 k=2; 1x1 2048->512 at 23x7x7 23 -> 18 k=3; 3x3 256->256 at 64x14x14 31 -> 35 k=2, not taken.)
+static int split_rule(int64_t tiles, int bn, int slices)
+{
+    double best = 0.93 * (4 + 0.36 * slices);
+    int k = 1;
+    for(int c = 2; c <= 16 && tiles * c <= 256 && c * 4 <= slices; c++) {
+        const double t = 13 + 0.36 * ((slices + c - 1) / c) + 0.033 * bn / 128 * (double)(tiles * c);
+        if(t < best) {
+            best = t;
+            k = c;
+        }
+    }
+    return k;
+}
+
+template <bool BWD> static int split_of(const GatherArgs &g, int64_t tiles, int active)
+{
+    const bool vec_ok = (g.ldo & 7) == 0 && (g.Ngemm & 7) == 0 && ((uintptr_t)g.out & 15) == 0;
+    if(!vec_ok || !g.part)
+        return 1;
+    const int sdiv = BWD ? g.stride : 1;
+    const int slices = ((g.R + sdiv - 1) / sdiv) * ((g.S + sdiv - 1) / sdiv) * ((g.Cred + 31) / 32);
+    const int bn = g.Ngemm <= 64 ? 64 : 128, k = split_rule(tiles, bn, slices);
+    const int64_t tile_bytes = 256ll * bn * 4;
+    return k > 1 && (int64_t)g.part_bytes >= tiles * k * tile_bytes ? k : 1;
+}
+
+// small grids: stream_f16.hip; false if it is not for that kernel
+template <bool BWD> static bool launch_stream(GatherArgs &g, hipStream_t st, int *rc)
+{
+    if(!g.a_bytes || !g.b_bytes)
+        return false;
+    StreamF16 s = {};
+    s.a = g.a; s.b = g.b; s.out = g.out;
+    s.a_bytes = g.a_bytes; s.b_bytes = g.b_bytes;
+    s.batch = g.M / (g.OH * g.OW);
+    s.N = g.Ngemm; s.C = g.Cred;
+    s.IH = g.IH; s.IW = g.IW; s.OH = g.OH; s.OW = g.OW;
+    s.R = g.R; s.S = g.S; s.pad = g.pad; s.stride = g.stride; s.dil = g.dil;
+    s.lda = g.lda; s.ldo = g.ldo;
+    s.bwd = BWD;
+    s.alpha = g.alpha; s.beta = g.beta;
+    if(!BWD && g.bn_s) {
+        s.bn_s = g.bn_s; s.bn_b = g.bn_b; s.bn_m = g.bn_m; s.bn_v = g.bn_v;
+        s.bn_eps = g.bn_eps;
+        s.bn_flags = g.bn_flags;
+        s.z = g.z; s.ldz = g.ldz;
+    }
+    if(!BWD)
+        s.sums = g.stats;
+    if(BWD && g.bq_partial) {
+        s.sums = g.bq_partial;
+        s.bq_x = g.bq_x; s.bq_ldx = g.bq_ldx; s.bq_relu = g.bq_relu;
+        s.bq_mean = g.bq_mean; s.bq_s = g.bq_s; s.bq_invstd = g.bq_invstd; s.bq_b = g.bq_b;
+    }
+    if(!stream_f16_wanted(s))
+        return false;
+    *rc = stream_f16_launch(s, st, &g.stats_rows);
+    return *rc != SAGA_HIP_EUNSUPPORTED;
+}
+
+static int stream_rows(bool bwd, const ConvGeom &g)
+{
+    StreamF16 s = {};
+    s.batch = g.N;
+    s.N = bwd ? g.C : g.K;
+    s.C = bwd ? g.K : g.C;
+    s.OH = bwd ? g.H : g.P;
+    s.OW = bwd ? g.W : g.Q;
+    s.R = g.R; s.S = g.S; s.stride = g.stride;
+    s.bwd = bwd;
+    return stream_f16_sum_rows(s);
+}
+
 template <bool BWD> static int launch_gather(GatherArgs &g, hipStream_t st)
 {
     static const int no_stage = getenv("SAGA_HIP_NO_STAGED_STORES") ? 1 : 0;
@@ -3541,6 +3795,42 @@ template <bool BWD> static int launch_gather(GatherArgs &g, hipStream_t st)
             // 5-15 % faster on the 7x7-pixel layers of ResNet-50, slower once CUs hold two blocks)
             if(tile == 5 && (int64_t)((g.Mc + 255) / 256) * ((g.Ngemm + 127) / 128) * active <= 256)
                 tile = 12;
+        }
+        // few tiles: the reduction of each shared by several blocks
+        const int bn_tile = g.Ngemm <= 64 ? 64 : 128;
+        const int64_t tiles = (int64_t)((g.Mc + 255) / 256) * ((g.Ngemm + bn_tile - 1) / bn_tile) * active;
+        const int ksplit = split_of<BWD>(g, tiles, active);
+        if(ksplit > 1) {
+            g.ksplit = ksplit;
+            g.nblk_n = (g.Ngemm + bn_tile - 1) / bn_tile;
+            g.blocks_per_class = ((g.Mc + 255) / 256) * g.nblk_n;
+            g.nblocks = (int)tiles;
+            g.nactive = active;
+            g.stats_rows = ((g.Mc + 127) / 128) * active;
+            const unsigned rblocks = (unsigned)(g.stats_rows * ((g.Ngemm + 31) / 32));
+#define SPLIT_GO(BN, WGN)                                                                                                   \
+    do {                                                                                                                    \
+        auto kern = conv_gather_gemm_dma<256, BN, 4, WGN, ST, 32, BWD, 4, false, true>;                                     \
+        constexpr int lds = ST * (256 + BN) * 64;                                                                           \
+        static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+        if(attr != hipSuccess)                                                                                              \
+            return (int)attr;                                                                                               \
+        kern<<<(unsigned)tiles * ksplit, 64 * (4 * WGN + 4), lds, st>>>(g);                                                 \
+        if constexpr(BWD) {                                                                                                 \
+            if(g.bq_partial) {                                                                                              \
+                split_reduce<WGN, BWD, true><<<rblocks, 256, 0, st>>>(g);                                                   \
+                break;                                                                                                      \
+            }                                                                                                               \
+        }                                                                                                                   \
+        split_reduce<WGN, BWD, false><<<rblocks, 256, 0, st>>>(g);                                                          \
+    } while(0)
+            if(bn_tile == 64)
+                SPLIT_GO(64, 1);
+            else
+                SPLIT_GO(128, 2);
+#undef SPLIT_GO
+            SAGA_CHECK_LAUNCH();
+            return 0;
         }
         // linked to a batch norm's backward: only the 256-row tiles carry the link
         if(g.bq_partial && tile != 5 && tile != 12 && tile != 13)
@@ -3603,6 +3893,15 @@ template <bool BWD> static int launch_gather(GatherArgs &g, hipStream_t st)
     return 0;
 }
 
+// the workspace behind its first `used` bytes for partial sums
+static void set_part(GatherArgs &g, void *ws, size_t ws_bytes, size_t used)
+{
+    used = (used + 255) & ~(size_t)255;
+    const bool room = ws && aligned16(ws) && ws_bytes > used;
+    g.part = room ? (float4_t *)((char *)ws + used) : nullptr;
+    g.part_bytes = room ? ws_bytes - used : 0;
+}
+
 static int round8(int v) { return (v + 7) & ~7; }
 
 // *pad is set when the gathered tensor cannot be loaded in 16-byte channel vectors as it is
@@ -3657,18 +3956,31 @@ static bool set_bn(GatherArgs &a, const ConvBnFold *bn, const SagaTensorView *y,
 
 } // namespace
 
-// floats a linked backward-data launch may write: per residue class of the stride, one row per 128 pixels
+// floats a linked backward-data launch may write: per residue class of the stride, one row per 128 pixels (or as many
+// as the kernel for small grids leaves)
 size_t conv_mfma_bnbwd_floats(const ConvGeom &g)
 {
     const int64_t Mc = (int64_t)g.N * ((g.H + g.stride - 1) / g.stride) * ((g.W + g.stride - 1) / g.stride);
-    return (size_t)((Mc + 127) / 128) * g.stride * g.stride * g.C * 2;
+    return std::max((size_t)((Mc + 127) / 128) * g.stride * g.stride, (size_t)stream_rows(true, g)) * g.C * 2;
 }
 
-// floats a forward launch may write into its statistics buffer: the smallest M tile is 128 rows
+// floats a forward launch may write into its statistics buffer: the smallest M tile of the tiled kernels is 128 rows
 size_t conv_mfma_stats_floats(const ConvGeom &g)
 {
     const int64_t M = (int64_t)g.N * g.P * g.Q;
-    return (size_t)((M + 127) / 128) * g.K * 2;
+    return std::max((size_t)((M + 127) / 128), (size_t)stream_rows(false, g)) * g.K * 2;
+}
+
+// partial sums of a launch whose tiles share their reductions
+static size_t split_bytes(bool bwd, const ConvGeom &g)
+{
+    const int s = bwd ? g.stride : 1, n = bwd ? g.C : g.K, red = bwd ? g.K : g.C;
+    const int64_t Mc = (int64_t)g.N * (bwd ? (g.H + s - 1) / s : g.P) * (bwd ? (g.W + s - 1) / s : g.Q);
+    const int bn = n <= 64 ? 64 : 128;
+    const int64_t tiles = ((Mc + 255) / 256) * ((n + bn - 1) / bn) * s * s;
+    const int slices = ((g.R + s - 1) / s) * ((g.S + s - 1) / s) * ((red + 31) / 32);
+    const int k = split_rule(tiles, bn, slices);
+    return k > 1 ? (size_t)(tiles * k * 256 * bn * 4) : 0;
 }
 
 size_t conv_mfma_workspace(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
@@ -3684,9 +3996,9 @@ size_t conv_mfma_workspace(int kind, const SagaTensorView *x, const SagaTensorVi
     ThinGeom tg;
     const bool thin = thin_ok(g, &tg);
     if(kind == SAGA_CONV_FWD)
-        return std::max(xpad + wpad, thin ? tg.x4_bytes + tg.wv_bytes : 0) + 256;
+        return std::max(xpad + wpad, thin ? tg.x4_bytes + tg.wv_bytes : 0) + 512 + split_bytes(false, g);
     if(kind == SAGA_CONV_BWD_DATA)
-        return (size_t)g.K * g.C * g.R * g.S * sizeof(half_t) + 256;
+        return (size_t)g.K * g.C * g.R * g.S * sizeof(half_t) + 512 + split_bytes(true, g);
     if(kind == SAGA_CONV_BWD_FILTER) {
         ConvGeom gp = g;
         gp.C = (int)Cp;
@@ -3742,6 +4054,7 @@ int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
         a.b_bytes = (unsigned)(wn * 2);
         a.stats = stats;
         a.bq_partial = nullptr;
+        a.part = nullptr;
         if(!set_bn(a, bn, y, ly))
             return SAGA_HIP_EUNSUPPORTED;
         // whole rows in LDS (conv_thin_rows): 7-row filters into at most 64 channels, output rows of at most 256 pixels
@@ -3839,9 +4152,15 @@ int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
     }
     a.stats = stats;
     a.bq_partial = nullptr;
+    set_part(a, ws, ws_bytes, pad ? (size_t)((char *)a.b - (char *)ws) + (size_t)g.K * g.R * g.S * a.Cred * sizeof(half_t) : 0);
     if(!set_bn(a, bn, y, ly))
         return SAGA_HIP_EUNSUPPORTED;
     int rc = 0;
+    if(launch_stream<false>(a, st, &rc)) {
+        if(stats_rows)
+            *stats_rows = a.stats_rows;
+        return rc;
+    }
     if(!(dma_stages() >= 2 && !pad && (launch_rows64<false>(a, ly, st, stats_floats, &rc) || launch_c64_wide(a, ly, st, stats_floats, &rc))))
         rc = launch_gather<false>(a, st);
     if(stats_rows)
@@ -3942,6 +4261,7 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
     a.stats = nullptr;
     a.bn_s = nullptr;
     a.bq_partial = nullptr;
+    set_part(a, ws, ws_bytes, (size_t)g.K * g.C * g.R * g.S * sizeof(half_t));
     if(link) {
         a.bq_x = (const half_t *)link->x->ptr;
         a.bq_ldx = (int)lbx.pitch;
@@ -3962,6 +4282,11 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
                                                                         g.R * g.S);
         a.b = (const half_t *)ws;
         a.b_krsc = 0;
+    }
+    if(launch_stream<true>(a, st, &rc)) {
+        if(link && link->partial_rows)
+            *link->partial_rows = a.stats_rows;
+        return rc;
     }
     if(!(dma_stages() >= 2 && !link && launch_rows64<true>(a, ldx, st, 0, &rc)))
         rc = launch_gather<true>(a, st);
