@@ -1,8 +1,9 @@
 // Row-major GEMM used by the fully-connected node: C = alpha*op(A)*op(B) + beta*C, either
 // operand may be stored transposed.
-//  * fp16: gemm_mfma_f16, 64x64x32 block tiles on v_mfma_f32_32x32x16_f16 (one 32x32 tile per
+//  * fp16: gemm_mfma_f16, 64x64x128 block tiles on v_mfma_f32_32x32x16_f16 (one 32x32 tile per
 //    wave), operands staged through LDS with the reduction index contiguous; an operand
-//    stored with the other index contiguous is transposed on its way into LDS.
+//    stored with the other index contiguous is transposed on its way into LDS; gemm_split_f16,
+//    32x32 tiles whose reduction is split over a block, for grids that leave compute units idle.
 //  * fp32: stream_f32_gemm (stream_f32.hip); gemm_mfma_f32, 64x64x16 LDS tiles on v_mfma_f32_32x32x2_f32, for reductions
 //    of up to 16 and operands beyond 2 GB.
 #include "stream_f32.hpp"
@@ -205,6 +206,110 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// The same for grids that leave compute units idle (few rows, or few outputs): a 32x32 tile per block of 8 wavefronts that
+// split the reduction, every eighth slice of 64 steps each, and add their tiles through LDS in a fixed order.  What bounds
+// such a product is the chain of trips to memory of one block: with 64x64 tiles fc 2048 -> 1000 ran in 16 blocks of 16
+// dependent slices (1 sample: 34 -> 5 us, 256 samples: 31 -> 6 us).
+// A slice is one cache line per row.  A wavefront fetches it in the order of memory (8 lanes per line), turns it through an
+// LDS area of its own into operand order, and has the next slice in flight meanwhile; nothing is shared before the sum, so
+// the loop holds no barrier.
+constexpr int GS_K = 64, GS_LD = GS_K + 8, GS_WAVES = 8;
+
+template <bool tA, bool tB, bool VEC>
+__global__ void __launch_bounds__(64 * GS_WAVES)
+    gemm_split_f16(int M, int N, int K, float alpha, const half_t *__restrict__ A, int lda,
+                   const half_t *__restrict__ B, int ldb, float beta, half_t *__restrict__ C, int ldc)
+{
+    __shared__ __attribute__((aligned(16))) half_t st[GS_WAVES][2][32][GS_LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
+    float16_t acc;
+#pragma unroll
+    for(int v = 0; v < 16; v++)
+        acc[v] = 0.0f;
+    // 8 consecutive elements in memory order: along the reduction (kcontig), or along the rows
+    auto fetch = [&](half8_t(&d)[4], const half_t *__restrict__ base, int ld, bool kcontig, int row0, int rows, int k0) {
+#pragma unroll
+        for(int j = 0; j < 4; j++) {
+            const int r = row0 + (kcontig ? (lane >> 3) + 8 * j : (lane & 3) * 8), k = k0 + (kcontig ? (lane & 7) * 8 : (lane >> 2) + 16 * j);
+            if constexpr(VEC) { // runs are either whole or outside: no branch around the load
+                const bool ok = r < rows && k < K;
+                d[j] = *(const half8_t *)(base + (ok ? kcontig ? (int64_t)r * ld + k : (int64_t)k * ld + r : 0));
+            } else {
+#pragma unroll
+                for(int e = 0; e < 8; e++) {
+                    const int re = kcontig ? r : r + e, ke = kcontig ? k + e : k;
+                    const bool ok = re < rows && ke < K;
+                    const half_t v = base[ok ? kcontig ? (int64_t)re * ld + ke : (int64_t)ke * ld + re : 0];
+                    d[j][e] = ok ? v : (half_t)0;
+                }
+            }
+        }
+    };
+    // (steps beyond the reduction become zeros here, not where they are loaded: that would wait for the load; rows beyond
+    // the operand feed outputs that are not stored)
+    auto put = [&](half_t(*d)[GS_LD], half8_t(&v)[4], bool kcontig, int k0) {
+#pragma unroll
+        for(int j = 0; j < 4; j++) {
+            if(k0 + (kcontig ? (lane & 7) * 8 : (lane >> 2) + 16 * j) >= K)
+                v[j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+            if(kcontig) {
+                *(half8_t *)&d[(lane >> 3) + 8 * j][(lane & 7) * 8] = v[j];
+            } else {
+#pragma unroll
+                for(int e = 0; e < 8; e++)
+                    d[(lane & 3) * 8 + e][(lane >> 2) + 16 * j] = v[j][e];
+            }
+        }
+    };
+    const int slices = (K + GS_K - 1) / GS_K;
+    const int fr = lane & 31, fk = (lane >> 5) * 8;
+    half8_t va[4], vb[4];
+    auto load = [&](int s) {
+        fetch(va, A, lda, !tA, m0, M, s * GS_K);
+        fetch(vb, B, ldb, tB, n0, N, s * GS_K);
+    };
+    if(wave < slices)
+        load(wave);
+    for(int s = wave; s < slices; s += GS_WAVES) {
+        put(st[wave][0], va, !tA, s * GS_K);
+        put(st[wave][1], vb, tB, s * GS_K);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if(s + GS_WAVES < slices)
+            load(s + GS_WAVES);
+#pragma unroll
+        for(int kk = 0; kk < GS_K / 16; kk++) {
+            const half8_t fa = *(const half8_t *)&st[wave][0][fr][kk * 16 + fk];
+            const half8_t fb = *(const half8_t *)&st[wave][1][fr][kk * 16 + fk];
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(fa, fb, acc, 0, 0, 0);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    }
+    __syncthreads();
+    float(*red)[32][33] = (float(*)[32][33]) & st[0][0][0][0];
+    static_assert(sizeof(st) >= GS_WAVES * 32 * 33 * sizeof(float), "the tiles of the sum fit the staging area");
+#pragma unroll
+    for(int v = 0; v < 16; v++)
+        red[wave][(v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)][lane & 31] = acc[v];
+    __syncthreads();
+    const int n = n0 + (tid & 31);
+#pragma unroll
+    for(int h = 0; h < 2; h++) {
+        const int ml = (tid >> 5) + 16 * h, m = m0 + ml;
+        float r = 0;
+#pragma unroll
+        for(int w = 0; w < GS_WAVES; w++)
+            r += red[w][ml][tid & 31];
+        if(m < M && n < N) {
+            half_t *o = C + (int64_t)m * ldc + n;
+            r *= alpha;
+            *o = (half_t)(beta != 0.0f ? r + beta * (float)*o : r);
+        }
+    }
+}
+
 } // namespace
 
 extern "C" int saga_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda,
@@ -218,6 +323,22 @@ extern "C" int saga_hip_gemm(int transA, int transB, int M, int N, int K, float 
     hipStream_t st = as_stream(stream);
     if(dtype == SAGA_HALF) {
         const int a_vec = lda % 8 == 0 && ((uintptr_t)A & 15) == 0, b_vec = ldb % 8 == 0 && ((uintptr_t)B & 15) == 0;
+        // Below one 64x64 tile per compute unit the reduction is split, unless it is shorter than there are tiles: then a tile's
+        // chain is short beside the work of the others (1024x1024: K = 1024 19 -> 14 us, 256 equal, 64 5.0 -> 5.4 us;
+        // 1000x2048, 512 tiles, K = 256: 12 -> 14 us).  A reduction of up to 16 is one slice in both.
+        const int64_t tiles = (int64_t)grid.x * grid.y;
+        if(tiles <= 256 && K > 16 && (tiles <= 64 || K > tiles)) {
+            // (a run of 8 that is only partly in range goes element by element)
+            const bool vec = a_vec && (transA ? M : K) % 8 == 0 && b_vec && (transB ? K : N) % 8 == 0;
+            auto kern = transA ? transB ? vec ? gemm_split_f16<true, true, true> : gemm_split_f16<true, true, false>
+                                        : vec ? gemm_split_f16<true, false, true> : gemm_split_f16<true, false, false>
+                               : transB ? vec ? gemm_split_f16<false, true, true> : gemm_split_f16<false, true, false>
+                                        : vec ? gemm_split_f16<false, false, true> : gemm_split_f16<false, false, false>;
+            kern<<<dim3((N + 31) / 32, (M + 31) / 32), 64 * GS_WAVES, 0, st>>>(M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
+                                                                             ldb, beta, (half_t *)C, ldc);
+            SAGA_CHECK_LAUNCH();
+            return 0;
+        }
         gemm_mfma_f16<<<grid, 256, 0, st>>>(transA, transB, M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
                                             ldb, beta, (half_t *)C, ldc, a_vec, b_vec);
     } else if(dtype == SAGA_FLOAT) {
