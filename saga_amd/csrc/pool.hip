@@ -155,46 +155,60 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Average pooling over windows of 1024 positions or more (global pooling of a large image): one
-// block per output vector, the window positions striped over its 256 threads, then a tree sum in LDS.
-template <typename T, int VN>
-__global__ void __launch_bounds__(256) avgpool_fwd_wide_k(DView x, DView y, int k, int pad, int stride)
+// Average pooling over windows of 16 positions or more: G lanes of a block share an output vector, each taking every
+// G-th position of its window, and LDS adds their sums in a fixed order.  One lane per output vector left the chip idle
+// where there are few of them and paid a trip to memory per position: global pooling of one 7x7x2048 sample ran in a
+// single block (12 -> 5 us), of 128 8x8x64 samples in four (15 -> 4 us).
+// Lanes that sit next to each other read what is contiguous: channel vectors (VN > 1) or the positions of a row (VN == 1).
+// Wide windows take a block of 1024 lanes per vector; the blocks of one sample, which share its cache lines, go to the
+// same XCD (its blocks are every eighth): 256x256x64 at 16 samples 146 -> 67 us.
+template <typename T, int VN, int NT>
+__global__ void __launch_bounds__(NT) avgpool_fwd_split_k(DView x, DView y, int k, int pad, int stride, int G, int64_t total)
 {
-    __shared__ float part[256][VN];
+    __shared__ float part[VN][NT];
     const int C = y.d[1], P = y.d[2], Q = y.d[3], H = x.d[2], W = x.d[3];
-    int n, c, p, q;
-    decode<VN>(blockIdx.x, C, P, Q, n, c, p, q);
+    const int tid = threadIdx.x, per = NT / G;
+    const int g = VN > 1 ? tid / per : tid % G, v = VN > 1 ? tid % per : tid / G;
+    const int64_t blk = gridDim.x % 8 == 0 ? (int64_t)(blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
+    const int64_t o = blk * per + v;
+    int n = 0, c = 0, p = 0, q = 0;
     float acc[VN];
 #pragma unroll
     for(int j = 0; j < VN; j++)
         acc[j] = 0.0f;
-    for(int t = threadIdx.x; t < k * k; t += 256) {
-        const int h = p * stride - pad + t / k, w = q * stride - pad + t % k;
-        if(h < 0 || h >= H || w < 0 || w >= W)
-            continue;
-        float v[VN];
-        PV<T, VN>::load((const T *)x.ptr + off4(x, n, c, h, w), v);
+    if(o < total) {
+        decode<VN>(o, C, P, Q, n, c, p, q);
+        const T *base = (const T *)x.ptr + n * x.s[0] + c * x.s[1];
+        const int h0 = p * stride - pad, w0 = q * stride - pad;
+#pragma unroll 4
+        for(int t = g; t < k * k; t += G) {
+            const int h = h0 + t / k, w = w0 + t % k;
+            const bool in = h >= 0 && h < H && w >= 0 && w < W;
+            float e[VN];
+            PV<T, VN>::load(base + (in ? h * x.s[2] + w * x.s[3] : 0), e); // (position 0 exists: no branch around a load)
 #pragma unroll
-        for(int j = 0; j < VN; j++)
-            acc[j] += v[j];
+            for(int j = 0; j < VN; j++)
+                acc[j] += in ? e[j] : 0.0f;
+        }
     }
 #pragma unroll
     for(int j = 0; j < VN; j++)
-        part[threadIdx.x][j] = acc[j];
+        part[j][tid] = acc[j];
     __syncthreads();
-    for(int w = 128; w > 0; w >>= 1) {
-        if((int)threadIdx.x < w) {
+    const int step = VN > 1 ? per : 1;
+    for(int w = G / 2; w > 0; w >>= 1) {
+        if(g < w) {
 #pragma unroll
             for(int j = 0; j < VN; j++)
-                part[threadIdx.x][j] += part[threadIdx.x + w][j];
+                part[j][tid] += part[j][tid + w * step];
         }
         __syncthreads();
     }
-    if(threadIdx.x == 0) {
+    if(g == 0 && o < total) {
         const float inv = 1.0f / (float)(k * k);
 #pragma unroll
         for(int j = 0; j < VN; j++)
-            acc[j] = part[0][j] * inv;
+            acc[j] = part[j][tid] * inv;
         PV<T, VN>::store((T *)y.ptr + off4(y, n, c, p, q), acc);
     }
 }
@@ -283,6 +297,45 @@ __global__ void __launch_bounds__(256)
                 acc[j] += beta * old[j];
         }
         PV<T, VN>::store(o, acc);
+    }
+}
+
+// Max-pool backward where the windows tile the input (stride == size, no padding) and w is the innermost dimension: one
+// lane per window, which finds the FIRST position that holds the maximum and writes all of its K*K gradients.  pool_bwd_k
+// reads x, y and dy once per input position and walks the window again for the tie-break, each step waiting for the one
+// before: 64x20x24x24 fp32, 2x2: 13 -> 4 us.  Positions beyond the last full window (a remainder of H or W) get a zero
+// gradient from the partial windows of the last row and column.
+template <typename T, int K>
+__global__ void __launch_bounds__(256)
+    maxpool_bwd_tiles_k(DView x, DView y, DView dy, DView dx, float beta, int PW, int QW, int64_t total)
+{
+    const int C = dx.d[1], H = dx.d[2], W = dx.d[3], P = dy.d[2], Q = dy.d[3];
+    for(int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256) {
+        int n, c, p, q;
+        decode<1>(i, C, PW, QW, n, c, p, q);
+        const bool full = p < P && q < Q;
+        float g = 0.0f, yv = 0.0f, xv[K * K], old[K * K];
+        const T *xs = (const T *)x.ptr + off4(x, n, c, p * K, q * K);
+        T *ds = (T *)dx.ptr + off4(dx, n, c, p * K, q * K);
+        if(full) {
+            g = (float)((const T *)dy.ptr)[off4(dy, n, c, p, q)];
+            yv = (float)((const T *)y.ptr)[off4(y, n, c, p, q)];
+        }
+#pragma unroll
+        for(int e = 0; e < K * K; e++) {
+            const bool in = p * K + e / K < H && q * K + e % K < W;
+            xv[e] = full ? (float)xs[(e / K) * x.s[2] + (e % K) * x.s[3]] : 0.0f;
+            old[e] = beta != 0.0f && in ? (float)ds[(e / K) * dx.s[2] + (e % K) * dx.s[3]] : 0.0f;
+        }
+        bool open = full;
+#pragma unroll
+        for(int e = 0; e < K * K; e++) {
+            const bool hit = open && same(xv[e], yv);
+            open = open && !hit;
+            const float v = hit ? g : 0.0f;
+            if(p * K + e / K < H && q * K + e % K < W)
+                ds[(e / K) * dx.s[2] + (e % K) * dx.s[3]] = (T)(beta != 0.0f ? v + beta * old[e] : v);
+        }
     }
 }
 
@@ -1050,14 +1103,23 @@ int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y
         SAGA_CHECK_LAUNCH();
         return 0;
     }
+    // lanes that share an average (0: one lane each): a few positions per lane, and only while single lanes would be
+    // few for the length of their chains (4x4 windows of 64x64x56x56, 100352 vectors: 9 us by single lanes, 14 shared; 7x7 of
+    // 256x2048x7x7, 65536 vectors: 20 and 16)
+    int lanes = 0;
+    if(size >= 4 && total <= (int64_t)size * size * 2048 && total < (1 << 22))
+        lanes = size < 16 ? 16 : size < 90 ? 256 : 1024;
     DView dvx = dview(x), dvy = dview(y), dvi = idx ? dview(idx) : dview(y);
 #define GO(T, VN)                                                                                        \
     do {                                                                                                 \
         if(mode == SAGA_POOL_MAX)                                                                        \
             pool_fwd_k<T, VN, SAGA_POOL_MAX><<<g, 256, 0, st>>>(dvx, dvy, dvi, idx != nullptr, size, pad, \
                                                                 stride, total);                          \
-        else if(size >= 32 && total < ((int64_t)1 << 30))                                                \
-            avgpool_fwd_wide_k<T, VN><<<(int)total, 256, 0, st>>>(dvx, dvy, size, pad, stride);           \
+        else if(lanes == 1024)                                                                           \
+            avgpool_fwd_split_k<T, VN, 1024><<<(int)total, 1024, 0, st>>>(dvx, dvy, size, pad, stride, 1024, total); \
+        else if(lanes)                                                                                   \
+            avgpool_fwd_split_k<T, VN, 256><<<(int)((total * lanes + 255) / 256), 256, 0, st>>>(dvx, dvy, size, pad, stride, \
+                                                                                                lanes, total); \
         else                                                                                             \
             pool_fwd_k<T, VN, SAGA_POOL_AVG><<<g, 256, 0, st>>>(dvx, dvy, dvi, 0, size, pad, stride, total); \
     } while(0)
@@ -1107,6 +1169,23 @@ int saga_hip_pool_bwd(int mode, const SagaTensorView *x, const SagaTensorView *y
             SAGA_CHECK_LAUNCH();
             return 0;
         }
+    }
+    // (lanes run along w: with the channels innermost they would touch a cache line each)
+    if(mx && vn == 1 && pad == 0 && size == stride && (size == 2 || size == 3) && dx->strides[3] == 1 && x->strides[3] == 1) {
+        const int PW = (dx->dims[2] + size - 1) / size, QW = (dx->dims[3] + size - 1) / size;
+        const int64_t nw = (int64_t)dx->dims[0] * dx->dims[1] * PW * QW;
+        const int gw = grid_for(nw, 256, 256 * 32);
+#define GOW(T)                                                                                          \
+    do {                                                                                                \
+        if(size == 2)                                                                                   \
+            maxpool_bwd_tiles_k<T, 2><<<gw, 256, 0, st>>>(dvx, dvy, dvdy, dvdx, beta, PW, QW, nw);      \
+        else                                                                                            \
+            maxpool_bwd_tiles_k<T, 3><<<gw, 256, 0, st>>>(dvx, dvy, dvdy, dvdx, beta, PW, QW, nw);      \
+    } while(0)
+        if(dt == SAGA_HALF) GOW(half_t); else GOW(float);
+#undef GOW
+        SAGA_CHECK_LAUNCH();
+        return 0;
     }
 #define GO(T, VN)                                                                                              \
     do {                                                                                                       \
