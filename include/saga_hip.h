@@ -148,8 +148,8 @@ int saga_hip_conv2d_fwd_bnstats(const SagaTensorView *x, const SagaTensorView *w
  *      The reference runs cudnnConvolutionForward (src/cuda/cuda_dnn.cpp:207-221) and
  *      cudnnBatchNormalizationForwardInference (:1641-1651) as two passes over the tensor; here the
  *      convolution's output never reaches memory un-normalised (and is not rounded to fp16 in
- *      between).  Returns SAGA_HIP_EUNSUPPORTED, with nothing written, outside the fp16
- *      channels-last MFMA path: run saga_hip_conv2d_fwd and saga_hip_bn_infer instead. */
+ *      between).  Returns SAGA_HIP_EUNSUPPORTED, with nothing written, outside the MFMA
+ *      paths (fp16 channels-last, fp32): run saga_hip_conv2d_fwd and saga_hip_bn_infer instead. */
 int saga_hip_conv2d_fwd_bn_infer(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                                  const SagaTensorView *z, const SagaConvParams *p, const float *s, const float *b,
                                  const float *m, const float *v, float eps, int flags, void *workspace,

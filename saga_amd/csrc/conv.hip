@@ -3,6 +3,7 @@
 #include "conv.hpp"
 
 #include <stdlib.h>
+#include <string.h>
 
 namespace {
 
@@ -116,6 +117,16 @@ int saga_hip_conv2d_fwd_bn_infer(const SagaTensorView *x, const SagaTensorView *
         return SAGA_HIP_EINVAL;
     if(force_direct())
         return SAGA_HIP_EUNSUPPORTED;
+    if(x->dtype == SAGA_FLOAT) {
+        if(z && (z->dtype != SAGA_FLOAT || !valid_view(z) || memcmp(z->dims, y->dims, sizeof(z->dims))))
+            return SAGA_HIP_EUNSUPPORTED;
+        StreamEpilogue e;
+        e.bn_s = s, e.bn_b = b, e.bn_m = m, e.bn_v = v;
+        e.bn_eps = eps;
+        e.z = flags & SAGA_BN_ADD ? z : nullptr;
+        e.relu = flags & SAGA_BN_RELU ? 1 : 0;
+        return conv_f32_fwd(x, w, y, g, 1.0f, 0.0f, workspace, ws_bytes, as_stream(stream), e);
+    }
     const ConvBnFold bn = {s, b, m, v, eps, flags, z};
     return conv_mfma_fwd(x, w, y, g, 1.0f, 0.0f, workspace, ws_bytes, as_stream(stream), nullptr, 0, nullptr, &bn);
 }

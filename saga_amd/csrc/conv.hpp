@@ -60,8 +60,16 @@ int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, cons
 // fp32 MFMA implicit-GEMM kernels (any strides, groups == 1); SAGA_HIP_EUNSUPPORTED otherwise.
 size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                           const ConvGeom &g);
+// Per output channel and element, after alpha and beta: out = act(v * scale + shift + z).
+struct StreamEpilogue {
+    const float *bias = nullptr;                                                    // shift
+    const float *bn_s = nullptr, *bn_b = nullptr, *bn_m = nullptr, *bn_v = nullptr; // scale = s*rsqrt(v+eps), shift = b - m*scale
+    float bn_eps = 0;
+    const SagaTensorView *z = nullptr;
+    int relu = 0;
+};
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,
-                 float beta, void *ws, size_t ws_bytes, hipStream_t st);
+                 float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue());
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
                       float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st);
 int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g,

@@ -69,6 +69,7 @@ struct GatherF32 {
     long long b_sn; // filter stride of the GEMM column (fwd: k, bwd-data: c)
     int stride, pad, dil, R, S;
     float alpha, beta;
+    EpilogueF32 e;
 };
 
 typedef float float16_t __attribute__((ext_vector_type(16)));
@@ -76,9 +77,12 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
 constexpr int FBM = 128, FBK = 16, FPAD = 8;
 
 // acc[i][j][v]: pixel wm + 32*i + lane%32, channel wn + 32*j + 8*(v/4) + 4*(lane/32) + v%4
-template <int TN>
+// scale, shift: of the block's channels (see EpilogueF32).  EX: there is something to add to the values or to apply to them;
+// those loads are requested eight at a time (all 64 of a wavefront at once would take the registers of two thirds of its
+// neighbours: 3x3 32->464 at 36x70x70 478 -> 762 us).
+template <int TN, bool EX>
 __device__ __forceinline__ void f32_store_tile(const GatherF32 &g, const float16_t (&acc)[2][TN], int m0, int n0, int wm,
-                                               int wn, int fr, int fk)
+                                               int wn, int fr, int fk, const float *scale, const float *shift)
 {
 #pragma unroll
     for(int i = 0; i < 2; i++) {
@@ -88,21 +92,57 @@ __device__ __forceinline__ void f32_store_tile(const GatherF32 &g, const float16
         const int ow = mo % g.OW, t = mo / g.OW;
         const int oh = t % g.OH, n = t / g.OH;
         float *op = g.out + n * g.o_sn + oh * g.o_sh + ow * g.o_sw;
+        const float *zp = EX && g.e.z ? g.e.z + n * g.e.z_sn + oh * g.e.z_sh + ow * g.e.z_sw : nullptr;
 #pragma unroll
-        for(int j = 0; j < TN; j++)
+        for(int e0 = 0; e0 < TN * 16; e0 += 8) {
+            auto channel = [&](int e) { return n0 + wn + (e >> 4) * 32 + 8 * ((e >> 2) & 3) + 4 * fk + (e & 3); };
+            float before[8] = {}, res[8] = {};
+            if constexpr(EX) {
+                if(g.beta != 0.0f)
 #pragma unroll
-            for(int v = 0; v < 16; v++) {
-                const int c = n0 + wn + j * 32 + 8 * (v >> 2) + 4 * fk + (v & 3);
+                    for(int j = 0; j < 8; j++)
+                        before[j] = op[(channel(e0 + j) < g.Ngemm ? channel(e0 + j) : 0) * g.o_sc];
+                if(zp)
+#pragma unroll
+                    for(int j = 0; j < 8; j++)
+                        res[j] = zp[(channel(e0 + j) < g.Ngemm ? channel(e0 + j) : 0) * g.e.z_sc];
+            }
+#pragma unroll
+            for(int j = 0; j < 8; j++) {
+                const int e = e0 + j, c = channel(e);
                 if(c >= g.Ngemm)
                     continue;
-                float val = g.alpha * acc[i][j][v];
-                if(g.beta != 0.0f)
-                    val += g.beta * op[c * g.o_sc];
+                float val = g.alpha * acc[i][e >> 4][e & 15];
+                if constexpr(EX) {
+                    if(g.beta != 0.0f)
+                        val += g.beta * before[j];
+                    val = g.e.apply(val, scale[c - n0], shift[c - n0], res[j]);
+                }
                 op[c * g.o_sc] = val;
             }
+        }
     }
 }
 
+// one channel per thread, before the main loop and (whole block) after it
+template <int BN, bool EX> __device__ __forceinline__ EpilogueF32::Raw f32_fetch(const GatherF32 &g, int n0, int tid)
+{
+    EpilogueF32::Raw r;
+    if(EX && g.e.affine() && tid < BN)
+        r = g.e.fetch(n0 + tid < g.Ngemm ? n0 + tid : g.Ngemm - 1);
+    return r;
+}
+template <int BN, bool EX>
+__device__ __forceinline__ void f32_leave(const GatherF32 &g, const EpilogueF32::Raw &r, float (&chan)[2][EX ? BN : 1], int tid)
+{
+    if(!EX || !g.e.affine())
+        return;
+    if(tid < BN)
+        g.e.leave(r, chan[0][tid], chan[1][tid]);
+    __syncthreads();
+}
+
+static bool f32_extras(float beta, const StreamEpilogue &e) { return beta != 0.0f || e.bias || e.bn_s || e.z || e.relu; }
 
 // 256 threads = 4 wavefronts (2 x 2), each a 64 x (BN/2) part of the 128 x BN tile.  The filter is
 // the MFMA's first operand, so a lane ends up with 16 channels of ONE pixel and consecutive lanes
@@ -110,7 +150,7 @@ __device__ __forceinline__ void f32_store_tile(const GatherF32 &g, const float16
 // LIN (stride 1 backward, any forward, at most 64 taps): the address of a tap is linear in the
 // tap's displacement, so the table holds the finished offset, and whether a tap of this thread's
 // pixel lies inside the image is one bit of a mask computed once.
-template <int BN, bool BWD, bool LIN>
+template <int BN, bool BWD, bool LIN, bool EX>
 __global__ void __launch_bounds__(256) conv_f32_gather(GatherF32 g)
 {
     constexpr int TN = BN / 64;        // 32-wide column tiles per wavefront
@@ -123,6 +163,9 @@ __global__ void __launch_bounds__(256) conv_f32_gather(GatherF32 g)
     const int bm = blockIdx.x / nblk_n, bn = blockIdx.x - bm * nblk_n;
     const int m0 = bm * FBM, n0 = bn * BN;
     const int wm = (wave >> 1) * 64, wn = (wave & 1) * (BN / 2);
+
+    __shared__ float chan[2][EX ? BN : 1];
+    const EpilogueF32::Raw raw = f32_fetch<BN, EX>(g, n0, tid);
 
     // this thread's pixel of the A tile (fixed for the whole kernel) and its two reduction rows
     const int am = tid & (FBM - 1), ak0 = tid >> 7;
@@ -255,7 +298,8 @@ __global__ void __launch_bounds__(256) conv_f32_gather(GatherF32 g)
         __syncthreads();
     }
 
-    f32_store_tile<TN>(g, acc, m0, n0, wm, wn, fr, fk);
+    f32_leave<BN, EX>(g, raw, chan, tid);
+    f32_store_tile<TN, EX>(g, acc, m0, n0, wm, wn, fr, fk, chan[0], chan[1]);
 }
 
 // ---------------------------------------------------------------- gather kernel, wave-uniform addressing
@@ -324,7 +368,7 @@ constexpr int UBK = F32_UBK; // reduction indices per slice of the wave-uniform 
 // returns zero without touching memory.
 constexpr unsigned U_RANGE = 0x80000000u;
 
-template <int BM, int BN, bool BWD, bool TAPU>
+template <int BM, int BN, bool BWD, bool TAPU, bool EX>
 __global__ void __launch_bounds__(256) conv_f32_gather_uniform(GatherU32 u)
 {
     const GatherF32 &g = u.g;
@@ -347,6 +391,9 @@ __global__ void __launch_bounds__(256) conv_f32_gather_uniform(GatherU32 u)
     const __amdgpu_buffer_rsrc_t rsa =
         __builtin_amdgcn_make_buffer_rsrc((void *)((const char *)g.a + u.minoff), 0, (int)U_RANGE, 0x00020000);
     const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc((void *)u.wt, 0, (int)U_RANGE, 0x00020000);
+
+    __shared__ float chan[2][EX ? BN : 1];
+    const EpilogueF32::Raw raw = f32_fetch<BN, EX>(g, n0, tid);
 
     // A tile: this thread's pixel, reduction rows ak0, ak0 + AKS, ... (ak0 is the same for a whole wavefront)
     const int am = tid & (BM - 1), ak0 = BM == 256 ? 0 : wave >> 1;
@@ -446,7 +493,8 @@ __global__ void __launch_bounds__(256) conv_f32_gather_uniform(GatherU32 u)
         __syncthreads();
     }
 
-    f32_store_tile<TN>(g, acc, m0, n0, wm, wn, fr, fk);
+    f32_leave<BN, EX>(g, raw, chan, tid);
+    f32_store_tile<TN, EX>(g, acc, m0, n0, wm, wn, fr, fk, chan[0], chan[1]);
 }
 
 // ---------------------------------------------------------------- backward filter
@@ -886,7 +934,7 @@ size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorVie
 }
 
 static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out,
-                         const ConvGeom &g, float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st)
+                         const ConvGeom &g, float alpha, float beta, const StreamEpilogue &e, void *ws, size_t ws_bytes, hipStream_t st)
 {
     // forward: a = x (N,C,H,W), out = y (N,K,P,Q); backward data: a = dy (N,K,P,Q), out = dx (N,C,H,W)
     const int red_ch = bwd ? g.K : g.C;
@@ -898,7 +946,7 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
     const int cols = out->dims[1], bn = cols > 64 ? 128 : 64;
     const long long tiles = ((long long)out->dims[0] * out->dims[2] * out->dims[3] + FBM - 1) / FBM * ((cols + bn - 1) / bn);
     if(!(tiles >= (red_ch % 8 ? 512 : 2048) && cols > 48 && uniform_ok(bwd, a, g))) {
-        const int r = stream_f32_conv(bwd, a, w, out, g, alpha, beta, StreamEpilogue(), ws, ws_bytes, st);
+        const int r = stream_f32_conv(bwd, a, w, out, g, alpha, beta, e, ws, ws_bytes, st);
         if(r != SAGA_HIP_EUNSUPPORTED)
             return r;
     }
@@ -961,18 +1009,24 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
         k.g.S = g.S;
         k.g.alpha = alpha;
         k.g.beta = beta;
+        k.g.e = epilogue_f32(e);
         k.tu = t.tu;
         k.wt = t.wt;
         k.npad = up.npad;
         k.bias = bias;
         k.minoff = minoff * 4;
+        const bool ex = f32_extras(beta, e);
         const int blocks = ((k.g.M + up.bm - 1) / up.bm) * (up.npad / up.bn);
-#define GOU(BM, BN, TAPU)                                                              \
-    do {                                                                           \
-        if(bwd)                                                                    \
-            conv_f32_gather_uniform<BM, BN, true, TAPU><<<blocks, 256, 0, st>>>(k);    \
-        else                                                                       \
-            conv_f32_gather_uniform<BM, BN, false, TAPU><<<blocks, 256, 0, st>>>(k);   \
+#define GOU(BM, BN, TAPU)                                                                  \
+    do {                                                                                   \
+        if(bwd && ex)                                                                      \
+            conv_f32_gather_uniform<BM, BN, true, TAPU, true><<<blocks, 256, 0, st>>>(k);  \
+        else if(bwd)                                                                       \
+            conv_f32_gather_uniform<BM, BN, true, TAPU, false><<<blocks, 256, 0, st>>>(k); \
+        else if(ex)                                                                        \
+            conv_f32_gather_uniform<BM, BN, false, TAPU, true><<<blocks, 256, 0, st>>>(k); \
+        else                                                                               \
+            conv_f32_gather_uniform<BM, BN, false, TAPU, false><<<blocks, 256, 0, st>>>(k); \
     } while(0)
         if(up.bn == 128) {
             if(t.tap_major) GOU(128, 128, true); else GOU(128, 128, false);
@@ -1029,17 +1083,18 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
     k.S = g.S;
     k.alpha = alpha;
     k.beta = beta;
+    k.e = epilogue_f32(e);
     const int bm = (k.M + FBM - 1) / FBM;
-#define GO(BN, BLOCKS)                                                                  \
-    do {                                                                                \
-        if(bwd && lin)                                                                  \
-            conv_f32_gather<BN, true, true><<<BLOCKS, 256, 0, st>>>(k);                 \
-        else if(bwd)                                                                    \
-            conv_f32_gather<BN, true, false><<<BLOCKS, 256, 0, st>>>(k);                \
-        else if(lin)                                                                    \
-            conv_f32_gather<BN, false, true><<<BLOCKS, 256, 0, st>>>(k);                \
-        else                                                                            \
-            conv_f32_gather<BN, false, false><<<BLOCKS, 256, 0, st>>>(k);               \
+#define GO(BN, BLOCKS)                                                       \
+    do {                                                                     \
+        if(bwd && lin)                                                       \
+            conv_f32_gather<BN, true, true, true><<<BLOCKS, 256, 0, st>>>(k);   \
+        else if(bwd)                                                         \
+            conv_f32_gather<BN, true, false, true><<<BLOCKS, 256, 0, st>>>(k);  \
+        else if(lin)                                                         \
+            conv_f32_gather<BN, false, true, true><<<BLOCKS, 256, 0, st>>>(k);  \
+        else                                                                 \
+            conv_f32_gather<BN, false, false, true><<<BLOCKS, 256, 0, st>>>(k); \
     } while(0)
     if(k.Ngemm > 64)
         GO(128, bm * ((k.Ngemm + 127) / 128));
@@ -1051,11 +1106,11 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
 }
 
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,
-                 float beta, void *ws, size_t ws_bytes, hipStream_t st)
+                 float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e)
 {
     if(!f32_ok(x, w, y, g))
         return SAGA_HIP_EUNSUPPORTED;
-    return gather_launch(false, x, w, y, g, alpha, beta, ws, ws_bytes, st);
+    return gather_launch(false, x, w, y, g, alpha, beta, e, ws, ws_bytes, st);
 }
 
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
@@ -1063,7 +1118,7 @@ int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const S
 {
     if(!f32_ok(dy, w, dx, g))
         return SAGA_HIP_EUNSUPPORTED;
-    return gather_launch(true, dy, w, dx, g, alpha, beta, ws, ws_bytes, st);
+    return gather_launch(true, dy, w, dx, g, alpha, beta, StreamEpilogue(), ws, ws_bytes, st);
 }
 
 int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g,

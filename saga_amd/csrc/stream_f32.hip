@@ -60,10 +60,7 @@ template <int CLASSES> struct ArgsOf {
     long long o_sn, o_sc, o_sh, o_sw;
     long long q_sn, q_sc, q_sr, q_ss;
     float alpha, beta;
-    const float *bias, *bn_s, *bn_b, *bn_m, *bn_v, *z;
-    float bn_eps;
-    int relu;
-    long long z_sn, z_sc, z_sh, z_sw;
+    EpilogueF32 e;
     int nclasses, nblk_q, blocks, KS;
     Class cls[CLASSES];
 };
@@ -87,10 +84,11 @@ __device__ __forceinline__ int xcd_order(int b, int n)
     return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + slot;
 }
 
-template <int PM, int QM, int TM, int TN, int DEPTH, int MAXW, typename A>
+template <int PM, int QM, int TM, int TN, int DEPTH, int MAXW, bool EX, typename A>
 __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
 {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    __shared__ __attribute__((aligned(16))) float chan[2][EX ? 32 * TN : 1]; // scale and shift of the block's channels
     const int tid = threadIdx.x, lane = tid & 63, fr = lane & 31, fk = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KS = g.KS, WM = (int)(blockDim.x >> 6) / KS;
@@ -105,6 +103,10 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
     const int T = c.Tr * c.Ts;
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)g.p, 0, (int)g.p_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)g.q, 0, (int)g.q_bytes, 0x00020000);
+
+    EpilogueF32::Raw raw;
+    if(EX && g.e.affine() && tid < 32 * TN)
+        raw = g.e.fetch(n0 + tid < g.N ? n0 + tid : g.N - 1);
 
     // this lane's pixels: byte offset of the first tap (negative outside the image: only valid taps are read) and one
     // bit per tap that falls inside
@@ -293,37 +295,47 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
         const int oy = t % c.OH, n = t / c.OH;
         const int y = oy * g.ostep + c.oy, x = ox * g.ostep + c.ox;
         opos[i] = n * g.o_sn + y * g.o_sh + x * g.o_sw;
-        zpos[i] = n * g.z_sn + y * g.z_sh + x * g.z_sw;
+        zpos[i] = n * g.e.z_sn + y * g.e.z_sh + x * g.e.z_sw;
     }
-    auto store = [&](bool pok, long long op, long long zp, int t, int v, float val) {
-        const int n = n0 + 32 * t + 8 * (v >> 2) + 4 * fk + (v & 3);
+    if(EX && g.e.affine() && tid < 32 * TN)
+        g.e.leave(raw, chan[0][tid], chan[1][tid]);
+    // what is added to the values is requested for many of them before the first is needed
+    auto channel = [&](int t, int v) { return n0 + 32 * t + 8 * (v >> 2) + 4 * fk + (v & 3); };
+    auto old = [&](long long op, int t, int v) { const int n = channel(t, v); return g.out[op + (n < g.N ? n : 0) * g.o_sc]; };
+    auto residual = [&](long long zp, int t, int v) { const int n = channel(t, v); return g.e.z[zp + (n < g.N ? n : 0) * g.e.z_sc]; };
+    auto store = [&](bool pok, long long op, int t, int v, float val, float before, float res) {
+        const int n = channel(t, v);
         if(!pok || n >= g.N)
             return;
         val *= g.alpha;
-        float *o = g.out + op + n * g.o_sc;
-        if(g.beta != 0.0f)
-            val += g.beta * *o;
-        if(g.bias)
-            val += g.bias[n];
-        if(g.bn_s) {
-            const float sc = g.bn_s[n] * rsqrtf(g.bn_v[n] + g.bn_eps);
-            val = __builtin_fmaf(val, sc, g.bn_b[n] - g.bn_m[n] * sc);
+        if constexpr(EX) {
+            if(g.beta != 0.0f)
+                val += g.beta * before;
+            val = g.e.apply(val, chan[0][n - n0], chan[1][n - n0], res);
         }
-        if(g.z)
-            val += g.z[zp + n * g.z_sc];
-        if(g.relu)
-            val = val != val ? val : fmaxf(val, 0.0f);
-        *o = val;
+        g.out[op + n * g.o_sc] = val;
     };
     constexpr int NV = TM * TN * 16;
     if(KS == 1) {
+        if(EX && g.e.affine())
+            __syncthreads();
 #pragma unroll
         for(int i = 0; i < TM; i++)
 #pragma unroll
-            for(int t = 0; t < TN; t++)
+            for(int e0 = 0; e0 < TN * 16; e0 += 8) {
+                float before[8] = {}, res[8] = {};
+                if(EX && g.beta != 0.0f)
 #pragma unroll
-                for(int v = 0; v < 16; v++)
-                    store(ok[i], opos[i], zpos[i], t, v, acc[i][t][v]);
+                    for(int j = 0; j < 8; j++)
+                        before[j] = old(opos[i], (e0 + j) >> 4, (e0 + j) & 15);
+                if(EX && g.e.z)
+#pragma unroll
+                    for(int j = 0; j < 8; j++)
+                        res[j] = residual(zpos[i], (e0 + j) >> 4, (e0 + j) & 15);
+#pragma unroll
+                for(int j = 0; j < 8; j++)
+                    store(ok[i], opos[i], (e0 + j) >> 4, (e0 + j) & 15, acc[i][e0 >> 4][(e0 + j) & 15], before[j], res[j]);
+            }
         return;
     }
     if(PM == PTAB)
@@ -335,15 +347,41 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
 #pragma unroll
             for(int v = 0; v < 16; v++)
                 smem[(wave * NV + (i * TN + t) * 16 + v) * 64 + lane] = acc[i][t][v];
-    __syncthreads();
     const int per = NV / KS; // KS divides 16
-    for(int e = ks * per; e < (ks + 1) * per; e++) {
-        float sum = 0.0f;
-        for(int k = 0; k < KS; k++)
-            sum += smem[((wm * KS + k) * NV + e) * 64 + lane];
-        const int i = e / (16 * TN), t = (e >> 4) % TN;
-        const bool hi = TM > 1 && i;
-        store(hi ? ok[TM - 1] : ok[0], hi ? opos[TM - 1] : opos[0], hi ? zpos[TM - 1] : zpos[0], t, e & 15, sum);
+    auto place = [&](int j, int &t, int &v) {
+        const int e = ks * per + j;
+        t = (e >> 4) % TN;
+        v = e & 15;
+        return TM > 1 && e / (16 * TN);
+    };
+    auto gather = [&](int j0, float(&before)[4], float(&res)[4]) {
+#pragma unroll
+        for(int j = 0; j < 4; j++) {
+            int t, v;
+            const bool hi = place(j0 + (j0 + j < per ? j : 0), t, v);
+            if(EX && g.beta != 0.0f)
+                before[j] = old(hi ? opos[TM - 1] : opos[0], t, v);
+            if(EX && g.e.z)
+                res[j] = residual(hi ? zpos[TM - 1] : zpos[0], t, v);
+        }
+    };
+    float before[4] = {}, res[4] = {};
+    gather(0, before, res);
+    __syncthreads();
+    for(int j0 = 0; j0 < per; j0 += 4) {
+        if(j0)
+            gather(j0, before, res);
+#pragma unroll
+        for(int j = 0; j < 4; j++) {
+            if(j0 + j >= per)
+                break;
+            int t, v;
+            const bool hi = place(j0 + j, t, v);
+            float sum = 0.0f;
+            for(int k = 0; k < KS; k++)
+                sum += smem[((wm * KS + k) * NV + ks * per + j0 + j) * 64 + lane];
+            store(hi ? ok[TM - 1] : ok[0], hi ? opos[TM - 1] : opos[0], t, v, sum, before[j], res[j]);
+        }
     }
 }
 
@@ -394,11 +432,11 @@ Config choose(long long pixels, int N, long long steps)
     return {1, 1, ks, ks >= 4 ? 1 : 4 / ks};
 }
 
-template <int PM, int QM, typename A> int launch_as(const A &k, const Config &cf, int threads, size_t lds, hipStream_t st)
+template <int PM, int QM, bool EX, typename A> int launch_as(const A &k, const Config &cf, int threads, size_t lds, hipStream_t st)
 {
 #define GO(TM, TN, DEPTH, MAXW)                                                                                        \
     do {                                                                                                               \
-        auto kern = stream_f32_k<PM, QM, TM, TN, DEPTH, MAXW, A>;                                                      \
+        auto kern = stream_f32_k<PM, QM, TM, TN, DEPTH, MAXW, EX, A>;                                                      \
         static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, \
                                                            (MAX_TABLE + 8) * 16);                                      \
         if(attr != hipSuccess)                                                                                         \
@@ -429,6 +467,7 @@ template <int PM, int QM> int launch(Args &g, hipStream_t st, long long pixels, 
     if(blocks > 0x7fffffff)
         return SAGA_HIP_EUNSUPPORTED;
     g.blocks = (int)blocks;
+    const bool ex = g.beta != 0.0f || g.e.bias || g.e.bn_s || g.e.z || g.e.relu;
     const int threads = 64 * cf.ks * cf.wm;
     size_t lds = cf.ks > 1 ? (size_t)cf.ks * cf.wm * cf.tm * cf.tn * 16 * 256 : 0;
     if(PM == PTAB) {
@@ -438,10 +477,10 @@ template <int PM, int QM> int launch(Args &g, hipStream_t st, long long pixels, 
         lds = std::max(lds, (size_t)((T * g.C + 7) / 8 * 8 + 8) * 16);
     }
     if(g.nclasses > 1)
-        return launch_as<PM, QM, Args>(g, cf, threads, lds, st);
+        return ex ? launch_as<PM, QM, true, Args>(g, cf, threads, lds, st) : launch_as<PM, QM, false, Args>(g, cf, threads, lds, st);
     Args1 one;
     memcpy(&one, &g, sizeof(one)); // the same members up to the first class
-    return launch_as<PM, QM, Args1>(one, cf, threads, lds, st);
+    return ex ? launch_as<PM, QM, true, Args1>(one, cf, threads, lds, st) : launch_as<PM, QM, false, Args1>(one, cf, threads, lds, st);
 }
 
 long long extent(const SagaTensorView *v)
@@ -539,14 +578,7 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
     k.q_ss = w->strides[3];
     k.alpha = alpha;
     k.beta = beta;
-    k.bias = e.bias;
-    k.bn_s = e.bn_s; k.bn_b = e.bn_b; k.bn_m = e.bn_m; k.bn_v = e.bn_v;
-    k.bn_eps = e.bn_eps;
-    k.relu = e.relu;
-    if(e.z) {
-        k.z = (const float *)e.z->ptr;
-        k.z_sn = e.z->strides[0]; k.z_sc = e.z->strides[1]; k.z_sh = e.z->strides[2]; k.z_sw = e.z->strides[3];
-    }
+    k.e = epilogue_f32(e);
     const long long pixels = (long long)out->dims[0] * out->dims[2] * out->dims[3];
     const long long steps = ((long long)k.C * g.R * g.S / k.nclasses + 7) / 8;
     int taps = 0;
@@ -606,10 +638,10 @@ int stream_f32_gemm(int tA, int tB, int M, int N, int K, float alpha, const floa
     k.q_sc = tA ? lda : 1;
     k.alpha = alpha;
     k.beta = beta;
-    k.relu = relu;
+    k.e.relu = relu;
     if(bias) { // per column: read like a residual with no row stride
-        k.z = bias;
-        k.z_sn = 1;
+        k.e.z = bias;
+        k.e.z_sn = 1;
     }
     const long long steps = (K + 7) / 8;
     if(tB)

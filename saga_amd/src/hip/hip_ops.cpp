@@ -72,7 +72,7 @@ struct ConvFwd : public HipOperation {
     }
     bool foldBn(T s, T b, T m, T v, T z, T y, float eps, int flags)
     {
-        if(stats_ || bn_y_ || x_->m_data_type != Tensor::DataType::HALF)
+        if(stats_ || bn_y_)
             return false;
         bn_s_ = s; bn_b_ = b; bn_m_ = m; bn_v_ = v; bn_z_ = z; bn_y_ = y;
         bn_eps_ = eps;

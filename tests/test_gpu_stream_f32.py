@@ -1,6 +1,8 @@
 """The fp32 matrix products that read their operands straight from memory (csrc/stream_f32.hip): one case per tile and per
 split of the reduction that the launch rule can choose, at sizes with remainders on every axis, forward and backward data
 against the oracle, and the GEMM's four operand orders with partial last steps."""
+import ctypes as C
+
 import numpy as np
 import pytest
 import torch
@@ -61,3 +63,33 @@ def test_gemm(tA, tB, size):
     K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 2.0, K.ptr(Ad), Ad.shape[1], K.ptr(Bd), Bd.shape[1], 3.0, K.ptr(Cd), N,
                                   K.FLOAT, stream))
     assert_close(host(Cd), 2 * want + 3, F32, "C")
+
+
+@pytest.mark.parametrize("flags", [0, K.BN_RELU, K.BN_ADD | K.BN_RELU])
+@pytest.mark.parametrize("shape", CONVS + [(8, 8, 190, 191, 80, 1, 1, 0), (2, 3, 186, 184, 64, 3, 1, 1)])  # the last: tiles in LDS
+def test_folded_norm(shape, flags):
+    N, Cc, H, W, Kk, R, stride, pad = shape
+    rng = np.random.default_rng(sum(shape) + flags)
+    x = rnd(rng, N, Cc, H, W, dtype=F32)
+    w = rnd(rng, Kk, Cc, R, R, dtype=F32, scale=(2.0 / (Cc * R * R)) ** 0.5)
+    f = lambda a: np.asarray(a, np.float32)
+    s, b = f(1 + 0.3 * rng.standard_normal(Kk)), f(0.2 * rng.standard_normal(Kk))
+    m, v = f(0.1 * rng.standard_normal(Kk)), f(rng.uniform(0.5, 1.5, Kk))
+    y = ref.conv2d_fwd(x, w, pad, stride)
+    z = rnd(rng, *y.shape, dtype=F32)
+    col = lambda a: a[None, :, None, None]
+    want = (y - col(m)) * col(s / np.sqrt(v + 1e-3)) + col(b)
+    if flags & K.BN_ADD:
+        want = want + z
+    if flags & K.BN_RELU:
+        want = np.maximum(want, 0)
+    xd, wd, zd = dev(x, F32), dev(w, F32), dev(z, F32, "nhwc")
+    yd = dev(np.full(y.shape, np.nan, np.float32), F32)
+    L, p = K.lib(), K.ConvParams(pad, stride, 1, 1)
+    vx, vw, vy, vz = (K.view(t) for t in (xd, wd, yd, zd))
+    n = L.saga_hip_conv2d_workspace_size(K.CONV_FWD, C.byref(vx), C.byref(vw), C.byref(vy), C.byref(p))
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device="cuda")
+    prm = [dev(a, F32) for a in (s, b, m, v)]
+    K.check(L.saga_hip_conv2d_fwd_bn_infer(C.byref(vx), C.byref(vw), C.byref(vy), C.byref(vz) if flags & K.BN_ADD else None,
+                                           C.byref(p), *(K.ptr(t) for t in prm), 1e-3, flags, K.ptr(ws), n, K.stream_ptr()))
+    assert_close(host(yd), want, F32, "folded norm")
