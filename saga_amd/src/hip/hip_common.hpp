@@ -197,6 +197,9 @@ struct HipOperation {
     // false for an operation whose launches take host values that change from step to step
     // (loss scale, Adam's bias corrections): it is never recorded into a HIP graph
     virtual bool graphSafe() const { return true; }
+    // true for an operation that may run on the context's side stream (see HipProgram::planSide): everything it reads
+    // and writes is in its lists, and it launches on p.stream() with p.workspace()
+    virtual bool sideSafe() const { return false; }
 
     // inputs plus the outputs that are accumulated into
     HipOpArgs getInputs();
@@ -252,6 +255,9 @@ public:
     hipStream_t m_stream = nullptr;
     // uploads of the batched tensors' BACK buffers: they run beside the step that computes on the front buffers
     hipStream_t m_copy_stream = nullptr;
+    // operations that nothing soon depends on run here, beside the rest of the step (HipProgram::planSide)
+    hipStream_t m_side_stream = nullptr;
+    HipScratch m_side_workspace;
     std::atomic<bool> m_copies_pending{false}; // something was enqueued on m_copy_stream since the last sync()
 
     // Pinned memory that host reads and writes of small tensors go through (HipTensor::writeHost / readHost), and the
@@ -378,6 +384,24 @@ public:
     bool graphsEnabled() const;
     void dropGraphs();
     void runOpsGraphed();
+
+    // ---- the side stream.  Per operation: where it runs, the first operation on the program's own stream that needs its
+    // results (or overwrites what it reads), and the events between the two streams (see planSide)
+    struct Side {
+        bool on = false;
+        int join = 0;
+        hipEvent_t fork = nullptr;      // the side stream waits for this one before the operation
+        hipEvent_t done = nullptr;      // recorded behind it, if an operation of the main stream waits
+        hipEvent_t reached = nullptr;   // main stream: recorded behind the operation, for forks
+        hipEvent_t needs = nullptr;     // main stream: waited for in front of the operation
+    };
+    std::vector<Side> m_side; // indexed like m_ops; empty: all on the program's stream
+    hipEvent_t m_side_start = nullptr, m_side_end = nullptr; // fork from the step's start, join behind its last operation
+    std::vector<hipEvent_t> m_side_events;
+    bool m_on_side = false;
+    void planSide();
+    hipStream_t stream() const { return m_on_side ? m_ctx->m_side_stream : m_ctx->m_stream; }
+    HipScratch &workspace() const { return m_on_side ? m_ctx->m_side_workspace : m_ctx->m_workspace; }
 
     // the operation that transposes the filters of all backward-data convolutions in one launch (hip_ops.cpp)
     std::shared_ptr<HipOperation> m_transpose_batch;

@@ -11,7 +11,7 @@ namespace {
 
 using T = std::shared_ptr<HipTensor>;
 
-saga_stream_t S(HipProgram &p) { return (saga_stream_t)p.m_ctx->m_stream; }
+saga_stream_t S(HipProgram &p) { return (saga_stream_t)p.stream(); }
 
 double nbytes(const T &t) { return (double)t->m_dims.elements() * Tensor::DataTypeSize(t->m_data_type); }
 
@@ -89,15 +89,15 @@ struct ConvFwd : public HipOperation {
         const float *s = (const float *)bn_s_->deviceMem(), *b = (const float *)bn_b_->deviceMem();
         const float *m = (const float *)bn_m_->deviceMem(), *v = (const float *)bn_v_->deviceMem();
         const int r = saga_hip_conv2d_fwd_bn_infer(&vx, &vw, &vo, bn_z_ ? &vz : nullptr, &cp_, s, b, m, v, bn_eps_, bn_flags_,
-                                                   p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(), S(p));
+                                                   p.workspace().ptr(), p.workspace().size(), S(p));
         if(r == 0)
             return;
         if(r != SAGA_HIP_EUNSUPPORTED)
             chkSaga(r);
         // two passes through the convolution's own output tensor
         const SagaTensorView vy = y_->view();
-        chkSaga(saga_hip_conv2d_fwd(&vx, &vw, &vy, &cp_, 1.0f, 0.0f, p.m_ctx->m_workspace.ptr(),
-                                    p.m_ctx->m_workspace.size(), S(p)));
+        chkSaga(saga_hip_conv2d_fwd(&vx, &vw, &vy, &cp_, 1.0f, 0.0f, p.workspace().ptr(),
+                                    p.workspace().size(), S(p)));
         chkSaga(saga_hip_bn_infer(&vy, bn_z_ ? &vz : nullptr, &vo, s, b, m, v, bn_eps_, bn_flags_, S(p)));
     }
     void exec(HipProgram &p) override
@@ -108,8 +108,8 @@ struct ConvFwd : public HipOperation {
         if(stats_) {
             stats_->valid = false;
             if(beta_ == 0.0f) {
-                const int r = saga_hip_conv2d_fwd_bnstats(&vx, &vw, &vy, &cp_, 1.0f, p.m_ctx->m_workspace.ptr(),
-                                                          p.m_ctx->m_workspace.size(), (float *)stats_->partial->m_ptr,
+                const int r = saga_hip_conv2d_fwd_bnstats(&vx, &vw, &vy, &cp_, 1.0f, p.workspace().ptr(),
+                                                          p.workspace().size(), (float *)stats_->partial->m_ptr,
                                                           stats_->partial->m_bytes, &stats_->rows, S(p));
                 if(r == 0) {
                     stats_->valid = true;
@@ -119,8 +119,8 @@ struct ConvFwd : public HipOperation {
                     chkSaga(r);
             }
         }
-        chkSaga(saga_hip_conv2d_fwd(&vx, &vw, &vy, &cp_, 1.0f, beta_, p.m_ctx->m_workspace.ptr(),
-                                    p.m_ctx->m_workspace.size(), S(p)));
+        chkSaga(saga_hip_conv2d_fwd(&vx, &vw, &vy, &cp_, 1.0f, beta_, p.workspace().ptr(),
+                                    p.workspace().size(), S(p)));
     }
     HipOpArgs listInputs() const override
     {
@@ -184,7 +184,7 @@ struct FilterTransposeBatch : public HipOperation {
             if(!jobs_dev_ || jobs_dev_->m_bytes < bytes)
                 jobs_dev_ = std::make_unique<HipMemory>(bytes);
             // synchronous copy of a few kilobytes, only when the table changed; jobs_ stays valid meanwhile
-            chkHip(hipStreamSynchronize(p.m_ctx->m_stream));
+            chkHip(hipStreamSynchronize(p.stream()));
             chkHip(hipMemcpy(jobs_dev_->m_ptr, jobs_.data(), bytes, hipMemcpyHostToDevice));
             epoch_ = p.m_ctx->m_mem_epoch;
             dirty_ = false;
@@ -192,6 +192,7 @@ struct FilterTransposeBatch : public HipOperation {
         chkSaga(saga_hip_filter_transpose_batched((const SagaFilterTransposeJob *)jobs_dev_->m_ptr, (int)jobs_.size(),
                                                   total_blocks_, S(p)));
     }
+    bool sideSafe() const override { return true; }
     HipOpArgs listInputs() const override
     {
         HipOpArgs r;
@@ -302,7 +303,7 @@ struct ConvBwdData : public HipOperation {
                                (float *)link_->partial->m_ptr,
                                link_->partial->m_bytes};
             const int r = saga_hip_conv2d_bwd_data_bnbwd(&vdy, &vw, wt_ ? wt_->deviceMem() : nullptr, &vdx, &cp_, 1.0f, beta_,
-                                                         p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(), &l, S(p));
+                                                         p.workspace().ptr(), p.workspace().size(), &l, S(p));
             if(r == 0) {
                 link_->rows = l.partial_rows;
                 link_->valid = true;
@@ -313,7 +314,7 @@ struct ConvBwdData : public HipOperation {
             link_->refused = true;
         }
         chkSaga(saga_hip_conv2d_bwd_data_wt(&vdy, &vw, wt_ ? wt_->deviceMem() : nullptr, &vdx, &cp_, 1.0f, beta_,
-                                            p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(), S(p)));
+                                            p.workspace().ptr(), p.workspace().size(), S(p)));
     }
     HipOpArgs listInputs() const override
     {
@@ -346,9 +347,10 @@ struct ConvBwdFilter : public HipOperation {
     void exec(HipProgram &p) override
     {
         const SagaTensorView vx = x_->view(), vdy = dy_->view(), vdw = dw_->view();
-        chkSaga(saga_hip_conv2d_bwd_filter(&vx, &vdy, &vdw, &cp_, 1.0f, beta_, p.m_ctx->m_workspace.ptr(),
-                                           p.m_ctx->m_workspace.size(), S(p)));
+        chkSaga(saga_hip_conv2d_bwd_filter(&vx, &vdy, &vdw, &cp_, 1.0f, beta_, p.workspace().ptr(),
+                                           p.workspace().size(), S(p)));
     }
+    bool sideSafe() const override { return true; }
     HipOpArgs listInputs() const override { return {{"x", x_}, {"dy", dy_}}; }
     HipOpArgs listOutputs() const override { return {{"dw", dw_}}; }
     float *getBeta(const T &t) override { return t == dw_ ? &beta_ : nullptr; }
@@ -384,8 +386,9 @@ struct BiasBwd : public HipOperation {
     void exec(HipProgram &p) override
     {
         const SagaTensorView vdy = dy_->view(), vdb = db_->view();
-        chkSaga(saga_hip_bias_bwd(&vdy, &vdb, beta_, p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(), S(p)));
+        chkSaga(saga_hip_bias_bwd(&vdy, &vdb, beta_, p.workspace().ptr(), p.workspace().size(), S(p)));
     }
+    bool sideSafe() const override { return true; }
     HipOpArgs listInputs() const override { return {{"dy", dy_}}; }
     HipOpArgs listOutputs() const override { return {{"db", db_}}; }
     double bytes() const override { return nbytes(dy_); }
@@ -539,6 +542,7 @@ struct Gemm : public HipOperation {
         chkSaga(saga_hip_gemm(ta_, tb_, m_, n_, k_, 1.0f, a_->deviceMem(), lda_, b_->deviceMem(), ldb_, beta_,
                               c_->deviceMem(), ldc_, (int)a_->m_data_type, S(p)));
     }
+    bool sideSafe() const override { return true; }
     HipOpArgs listInputs() const override { return {{"a", a_}, {"b", b_}}; }
     HipOpArgs listOutputs() const override { return {{"c", c_}}; }
     float *getBeta(const T &t) override { return t == c_ ? &beta_ : nullptr; }
@@ -812,7 +816,7 @@ struct BnTrain : public HipOperation {
                 &vx, z_ ? &vz : nullptr, &vy, (const float *)s_->deviceMem(), (const float *)b_->deviceMem(),
                 (float *)m_->deviceMem(), (float *)v_->deviceMem(), (float *)sm_->deviceMem(), (float *)sv_->deviceMem(),
                 eps_, expavg_, flags_, (const float *)stats_->partial->m_ptr, stats_->rows,
-                mask_ ? (uint8_t *)mask_->deviceMem() : nullptr, p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(),
+                mask_ ? (uint8_t *)mask_->deviceMem() : nullptr, p.workspace().ptr(), p.workspace().size(),
                 S(p));
             if(r == 0) {
                 expavg_ = p.m_pc.bn_expavg;
@@ -825,7 +829,7 @@ struct BnTrain : public HipOperation {
         chkSaga(saga_hip_bn_train_fwd(&vx, z_ ? &vz : nullptr, &vy, (const float *)s_->deviceMem(),
                                       (const float *)b_->deviceMem(), (float *)m_->deviceMem(),
                                       (float *)v_->deviceMem(), (float *)sm_->deviceMem(), (float *)sv_->deviceMem(),
-                                      eps_, expavg_, flags_, p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(),
+                                      eps_, expavg_, flags_, p.workspace().ptr(), p.workspace().size(),
                                       S(p)));
         expavg_ = p.m_pc.bn_expavg;
     }
@@ -886,8 +890,8 @@ struct BnBwd : public HipOperation {
             chkSaga(saga_hip_bn_bwd_linked(&vx, &vdy, &vdx, (const float *)fwd_->s_->deviceMem(),
                                            (const float *)fwd_->sm_->deviceMem(), (const float *)fwd_->sv_->deviceMem(),
                                            (float *)ds_->deviceMem(), (float *)db_->deviceMem(), dx_beta_, ds_beta_,
-                                           (const float *)link_->partial->m_ptr, link_->rows, p.m_ctx->m_workspace.ptr(),
-                                           p.m_ctx->m_workspace.size(), S(p)));
+                                           (const float *)link_->partial->m_ptr, link_->rows, p.workspace().ptr(),
+                                           p.workspace().size(), S(p)));
             return;
         }
         // the bias lets the kernels rebuild the relu mask from x when there is no residual
@@ -898,7 +902,7 @@ struct BnBwd : public HipOperation {
                                 (const float *)fwd_->sv_->deviceMem(), (float *)ds_->deviceMem(),
                                 (float *)db_->deviceMem(), dx_beta_, dz_beta_, ds_beta_, flags_,
                                 fwd_->mask_valid_ ? (const uint8_t *)fwd_->mask_->deviceMem() : nullptr,
-                                p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(), S(p)));
+                                p.workspace().ptr(), p.workspace().size(), S(p)));
     }
     HipOpArgs listInputs() const override
     {
@@ -1337,7 +1341,7 @@ struct BnBwdPooled : public HipOperation {
                                        (const float *)fwd_->s_->deviceMem(), (const float *)fwd_->b_->deviceMem(),
                                        (const float *)fwd_->sm_->deviceMem(), (const float *)fwd_->sv_->deviceMem(),
                                        (float *)ds_->deviceMem(), (float *)db_->deviceMem(), dx_beta_, ds_beta_, flags_, size_,
-                                       pad_, stride_, p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(), S(p)));
+                                       pad_, stride_, p.workspace().ptr(), p.workspace().size(), S(p)));
     }
     HipOpArgs listInputs() const override
     {
@@ -1625,7 +1629,7 @@ struct Stats : public HipOperation {
     void exec(HipProgram &p) override
     {
         const SagaTensorView vx = x_->view();
-        chkSaga(saga_hip_tensor_stats(&vx, (float *)y_->deviceMem(), p.m_ctx->m_workspace.ptr(), p.m_ctx->m_workspace.size(),
+        chkSaga(saga_hip_tensor_stats(&vx, (float *)y_->deviceMem(), p.workspace().ptr(), p.workspace().size(),
                                       S(p)));
     }
     HipOpArgs listInputs() const override { return {{"x", x_}}; }
