@@ -137,6 +137,16 @@ int saga_hip_conv2d_bwd_data_wt(const SagaTensorView *dy, const SagaTensorView *
  *      SAGA_HIP_EUNSUPPORTED (nothing written to y) when the fp16 channels-last MFMA path does
  *      not cover the problem: run saga_hip_conv2d_fwd and saga_hip_bn_train_fwd instead.
  *      _size: bytes `partial` must hold (0: never supported for these operands). */
+/* y = act(conv(x, w) + beta * y + bias), bias broadcast over the channels (any view of K elements), act a relu if `relu`:
+ * in the convolution's epilogue where its kernel has one, otherwise in passes of their own.  The backward-data form is the
+ * forward pass of a transposed convolution with a bias; wt as in saga_hip_conv2d_bwd_data_wt (may be null). */
+int saga_hip_conv2d_fwd_bias(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *bias,
+                             const SagaTensorView *y, const SagaConvParams *p, float beta, int relu, void *workspace,
+                             size_t ws_bytes, saga_stream_t stream);
+int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView *w, const void *wt,
+                                  const SagaTensorView *bias, const SagaTensorView *dx, const SagaConvParams *p, float beta,
+                                  void *workspace, size_t ws_bytes, saga_stream_t stream);
+
 size_t saga_hip_conv2d_fwd_bnstats_size(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                                         const SagaConvParams *p);
 int saga_hip_conv2d_fwd_bnstats(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
@@ -212,6 +222,10 @@ int saga_hip_bias_bwd_noalloc(const SagaTensorView *dy, const SagaTensorView *db
  *      fp16 operands accumulate in fp32. */
 int saga_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B,
                   int ldb, float beta, void *C, int ldc, int dtype, saga_stream_t stream);
+/* the same with a bias per column (may be null; fp32, or fp16 for an fp16 product) and a relu in the epilogue */
+int saga_hip_gemm_bias(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B,
+                       int ldb, float beta, void *C, int ldc, int dtype, const void *bias, int bias_dtype, int relu,
+                       saga_stream_t stream);
 
 /* ---- batch normalisation (spatial, per channel; s,b,m,v and saved statistics are fp32 [C]).
  *      infer: cudnnBatchNormalizationForwardInference (src/cuda/cuda_dnn.cpp:1641-1651);
@@ -280,6 +294,9 @@ int saga_hip_act_bwd(int mode, float alpha, const SagaTensorView *x, const SagaT
  *      flat h*W+w position of each window's maximum, first maximum in scan order. */
 int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *idx,
                       int size, int pad, int stride, saga_stream_t stream);
+/* the same with a relu of the result, without idx; SAGA_HIP_EUNSUPPORTED (nothing enqueued) where no kernel has one */
+int saga_hip_pool_fwd_relu(int mode, const SagaTensorView *x, const SagaTensorView *y, int size, int pad, int stride,
+                           saga_stream_t stream);
 int saga_hip_pool_bwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *dy,
                       const SagaTensorView *dx, int size, int pad, int stride, float beta, saga_stream_t stream);
 /* Max pooling for training that remembers where each maximum came from.  No single counterpart in the

@@ -79,6 +79,84 @@ int saga_hip_conv2d_fwd(const SagaTensorView *x, const SagaTensorView *w, const 
     return conv_direct_fwd(x, w, y, g, alpha, beta, as_stream(stream));
 }
 
+// the bias of a convolution into `out`, where no kernel takes it along
+static int add_bias(const SagaTensorView *bias, const SagaTensorView *out, int relu, saga_stream_t stream)
+{
+    const int r = saga_hip_bias_add(out, bias, stream);
+    return r || !relu ? r : saga_hip_act_fwd(SAGA_ACT_RELU, 0, out, out, 0.0f, stream);
+}
+
+static bool bias_ok(const SagaTensorView *bias, const SagaTensorView *out)
+{
+    return valid_view(bias) && view_elements(bias) == out->dims[1];
+}
+
+int saga_hip_conv2d_fwd_bias(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *bias,
+                             const SagaTensorView *y, const SagaConvParams *p, float beta, int relu, void *workspace,
+                             size_t ws_bytes, saga_stream_t stream)
+{
+    ConvGeom g;
+    int r = geometry(x, w, y, p, &g);
+    if(r)
+        return r;
+    if(!bias_ok(bias, y))
+        return SAGA_HIP_ESHAPE;
+    hipStream_t st = as_stream(stream);
+    bool done = false;
+    r = SAGA_HIP_EUNSUPPORTED;
+    if(!force_direct()) {
+        r = conv_mfma_fwd(x, w, y, g, 1.0f, beta, workspace, ws_bytes, st, nullptr, 0, nullptr, nullptr,
+                          bias->dtype == SAGA_HALF && !relu ? bias->ptr : nullptr, &done);
+        if(r == SAGA_HIP_EUNSUPPORTED) {
+            StreamEpilogue e;
+            done = bias->dtype == SAGA_FLOAT;
+            if(done) {
+                e.bias = (const float *)bias->ptr;
+                e.relu = relu;
+            }
+            r = conv_f32_fwd(x, w, y, g, 1.0f, beta, workspace, ws_bytes, st, e);
+        }
+    }
+    if(r == SAGA_HIP_EUNSUPPORTED) {
+        done = false;
+        r = conv_direct_fwd(x, w, y, g, 1.0f, beta, st);
+    }
+    return r || done ? r : add_bias(bias, y, relu, stream);
+}
+
+int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView *w, const void *wt, const SagaTensorView *bias,
+                                  const SagaTensorView *dx, const SagaConvParams *p, float beta, void *workspace, size_t ws_bytes,
+                                  saga_stream_t stream)
+{
+    ConvGeom g;
+    int r = geometry(dx, w, dy, p, &g);
+    if(r)
+        return r;
+    if(!bias_ok(bias, dx))
+        return SAGA_HIP_ESHAPE;
+    if(wt && (force_direct() || !conv_mfma_bwd_data_ok(dy, w, dx, g)))
+        return SAGA_HIP_EUNSUPPORTED;
+    hipStream_t st = as_stream(stream);
+    bool done = false;
+    r = SAGA_HIP_EUNSUPPORTED;
+    if(!force_direct()) {
+        r = conv_mfma_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, wt, nullptr,
+                               bias->dtype == SAGA_HALF ? bias->ptr : nullptr, &done);
+        if(r == SAGA_HIP_EUNSUPPORTED) {
+            StreamEpilogue e;
+            done = bias->dtype == SAGA_FLOAT;
+            if(done)
+                e.bias = (const float *)bias->ptr;
+            r = conv_f32_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, e);
+        }
+    }
+    if(r == SAGA_HIP_EUNSUPPORTED) {
+        done = false;
+        r = conv_direct_bwd_data(dy, w, dx, g, 1.0f, beta, st);
+    }
+    return r || done ? r : add_bias(bias, dx, 0, stream);
+}
+
 size_t saga_hip_conv2d_fwd_bnstats_size(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                                         const SagaConvParams *p)
 {

@@ -24,6 +24,7 @@ size_t conv_mfma_workspace(int kind, const SagaTensorView *x, const SagaTensorVi
 // stats (optional): receives per block row and output channel the sum and the sum of squares of
 // the stored outputs, [*stats_rows][K][2] floats; needs beta == 0 and conv_mfma_stats_floats(g) floats
 size_t conv_mfma_stats_floats(const ConvGeom &g);
+// bias (optional, fp16, alpha == 1): *bias_done says whether the launch added it
 // batch-norm inference (+ residual + relu) folded into the forward epilogue
 struct ConvBnFold {
     const float *s, *b, *m, *v;
@@ -33,7 +34,8 @@ struct ConvBnFold {
 };
 int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g,
                   float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, float *stats = nullptr,
-                  size_t stats_floats = 0, int *stats_rows = nullptr, const ConvBnFold *bn = nullptr);
+                  size_t stats_floats = 0, int *stats_rows = nullptr, const ConvBnFold *bn = nullptr, const void *bias = nullptr,
+                  bool *bias_done = nullptr);
 // backward data whose result dx is the gradient of a batch norm's (+ relu) output, with that norm's first
 // backward pass done in the epilogue: dx is stored masked by the relu and partial[*partial_rows][C][2]
 // receives sum(dx) and sum(dx * (x - mean)) per block row and channel.  EUNSUPPORTED (nothing written)
@@ -49,7 +51,8 @@ struct ConvBnBwdLink {
 size_t conv_mfma_bnbwd_floats(const ConvGeom &g);
 int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx,
                        const ConvGeom &g, float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st,
-                       const void *wt_ready = nullptr, const ConvBnBwdLink *link = nullptr);
+                       const void *wt_ready = nullptr, const ConvBnBwdLink *link = nullptr, const void *bias = nullptr,
+                       bool *bias_done = nullptr);
 bool conv_mfma_bwd_data_ok(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g);
 bool conv_mfma_bnbwd_link_ok(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g);
 int conv_mfma_transpose_blocks(int K, int C, int RS);
@@ -71,6 +74,6 @@ struct StreamEpilogue {
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,
                  float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue());
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
-                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st);
+                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue());
 int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g,
                         float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st);

@@ -1114,11 +1114,11 @@ int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTen
 }
 
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
-                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st)
+                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e)
 {
     if(!f32_ok(dy, w, dx, g))
         return SAGA_HIP_EUNSUPPORTED;
-    return gather_launch(true, dy, w, dx, g, alpha, beta, StreamEpilogue(), ws, ws_bytes, st);
+    return gather_launch(true, dy, w, dx, g, alpha, beta, e, ws, ws_bytes, st);
 }
 
 int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g,

@@ -78,6 +78,11 @@ struct GatherArgs {
     float4_t *part;
     size_t part_bytes; // room behind part
     unsigned out_bytes; // extent of out, for the epilogue variant that stores through a range-checked buffer (BUFST)
+    // optional, alpha == 1: one value per output channel, which the accumulators start from (conv_gather_gemm_dma and
+    // stream_f16; bias_done says that the launch took one of them).  Starting from it costs no register and no store path of
+    // its own; a pass over the output took 14 - 92 us per up-convolution of a U-Net at 16 x 256x256, 3 % of its step.
+    const half_t *bias = nullptr;
+    bool bias_done = false;
     float *stats;      // forward only, optional: per block row and output channel, sum and sum of
                        // squares of the stored outputs, [ceil(M / BM)][Ngemm][2]
     int stats_rows;    // out: block rows the launch wrote
@@ -1181,6 +1186,18 @@ __global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PR
                 acc[i][j][v] = 0.0f;
 
     const int wm = (wave / WGN) * WTM, wn = (wave % WGN) * WTN;
+    if(g.bias && split == 0) {
+#pragma unroll
+        for(int j = 0; j < TN; j++)
+#pragma unroll
+            for(int v = 0; v < 16; v++) {
+                const int n = n0 + wn + j * 32 + 8 * (v >> 2) + 4 * (lane >> 5) + (v & 3);
+                const float b = n < g.Ngemm ? (float)g.bias[n] : 0.0f;
+#pragma unroll
+                for(int i = 0; i < TM; i++)
+                    acc[i][j][v] = b;
+            }
+    }
     auto rowpix = [&](int mrow, bool &ok, int64_t &pix) {
         const int m = m0 + mrow;
         ok = m < Mloc;
@@ -3703,6 +3720,7 @@ template <bool BWD> static bool launch_stream(GatherArgs &g, hipStream_t st, int
     s.lda = g.lda; s.ldo = g.ldo;
     s.bwd = BWD;
     s.alpha = g.alpha; s.beta = g.beta;
+    s.bias = g.bias;
     if(!BWD && g.bn_s) {
         s.bn_s = g.bn_s; s.bn_b = g.bn_b; s.bn_m = g.bn_m; s.bn_v = g.bn_v;
         s.bn_eps = g.bn_eps;
@@ -3751,6 +3769,7 @@ template <bool BWD> static int launch_gather(GatherArgs &g, hipStream_t st)
     if(dma_stages() >= 2 && g.a_bytes && g.b_bytes && fits) {
         constexpr int ST = 3;
         int active = 1;
+        g.bias_done = g.bias != nullptr;
         if(BWD && g.stride > 1 && g.stride <= 4 && g.dil == 1) {
             g.classes = g.stride * g.stride;
             g.OHc = (g.OH + g.stride - 1) / g.stride;
@@ -3760,7 +3779,7 @@ template <bool BWD> static int launch_gather(GatherArgs &g, hipStream_t st)
             // coalesced fill for beta == 0 (a vectorisable output; otherwise they keep their blocks)
             const bool can_fill = (g.ldo & 7) == 0 && (g.Ngemm & 7) == 0 && ((uintptr_t)g.out & 15) == 0;
             // (linked to a batch norm's backward, every pixel's old value counts in the sums: beta == 1 keeps all classes)
-            const bool drop = (g.beta == 1.0f && !g.bq_partial) || (g.beta == 0.0f && can_fill);
+            const bool drop = !g.bias && ((g.beta == 1.0f && !g.bq_partial) || (g.beta == 0.0f && can_fill));
             active = 0;
             for(int c = 0; c < g.classes; c++) {
                 const int r0 = ((c >> g.sshift) + g.pad) & (g.stride - 1), s0 = ((c & (g.stride - 1)) + g.pad) & (g.stride - 1);
@@ -4010,7 +4029,7 @@ size_t conv_mfma_workspace(int kind, const SagaTensorView *x, const SagaTensorVi
 
 int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g,
                   float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, float *stats, size_t stats_floats,
-                  int *stats_rows, const ConvBnFold *bn)
+                  int *stats_rows, const ConvBnFold *bn, const void *bias, bool *bias_done)
 {
     if(bn && (stats || beta != 0.0f))
         return SAGA_HIP_EINVAL;
@@ -4146,16 +4165,21 @@ int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
     set_part(a, ws, ws_bytes, pad ? (size_t)((char *)a.b - (char *)ws) + (size_t)g.K * g.R * g.S * a.Cred * sizeof(half_t) : 0);
     if(!set_bn(a, bn, y, ly))
         return SAGA_HIP_EUNSUPPORTED;
+    a.bias = (const half_t *)bias;
     int rc = 0;
     if(launch_stream<false>(a, st, &rc)) {
         if(stats_rows)
             *stats_rows = a.stats_rows;
+        if(bias_done)
+            *bias_done = bias != nullptr;
         return rc;
     }
     if(!(dma_stages() >= 2 && !pad && (launch_rows64<false>(a, ly, st, stats_floats, &rc) || launch_c64_wide(a, ly, st, stats_floats, &rc))))
         rc = launch_gather<false>(a, st);
     if(stats_rows)
         *stats_rows = a.stats_rows;
+    if(bias_done)
+        *bias_done = a.bias_done;
     return rc;
 }
 
@@ -4193,7 +4217,7 @@ bool conv_mfma_bnbwd_link_ok(const SagaTensorView *dy, const SagaTensorView *w, 
 // otherwise it is transposed into the workspace first
 int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx,
                        const ConvGeom &g, float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st,
-                       const void *wt_ready, const ConvBnBwdLink *link)
+                       const void *wt_ready, const ConvBnBwdLink *link, const void *bias, bool *bias_done)
 {
     CLInfo ldy, ldx, lbx;
     if(!common_ok(dy, w, dx, g, &ldy, &ldx))
@@ -4274,13 +4298,18 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
         a.b = (const half_t *)ws;
         a.b_krsc = 0;
     }
+    a.bias = (const half_t *)bias;
     if(launch_stream<true>(a, st, &rc)) {
         if(link && link->partial_rows)
             *link->partial_rows = a.stats_rows;
+        if(bias_done)
+            *bias_done = bias != nullptr;
         return rc;
     }
     if(!(dma_stages() >= 2 && !link && launch_rows64<true>(a, ldx, st, 0, &rc)))
         rc = launch_gather<true>(a, st);
+    if(bias_done)
+        *bias_done = a.bias_done;
     if(link && link->partial_rows)
         *link->partial_rows = a.stats_rows;
     return rc;

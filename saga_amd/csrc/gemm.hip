@@ -14,7 +14,8 @@ namespace {
 // n = lane%32, rows 8*(v/4) + 4*(lane/32) + v%4 of the tile.
 __global__ void __launch_bounds__(256)
     gemm_mfma_f32(int tA, int tB, int M, int N, int K, float alpha, const float *__restrict__ A, int lda,
-                  const float *__restrict__ B, int ldb, float beta, float *__restrict__ C, int ldc)
+                  const float *__restrict__ B, int ldb, float beta, float *__restrict__ C, int ldc,
+                  const float *__restrict__ bias, int relu)
 {
     typedef float float16_t __attribute__((ext_vector_type(16)));
     constexpr int BM = 64, BN = 64, BK = 16;
@@ -62,10 +63,29 @@ __global__ void __launch_bounds__(256)
         if(gm >= M)
             continue;
         float *o = C + (int64_t)gm * ldc + gn;
-        const float r = alpha * acc[v];
-        *o = beta != 0.0f ? r + beta * *o : r;
+        float r = alpha * acc[v];
+        if(beta != 0.0f)
+            r += beta * *o;
+        if(bias)
+            r += bias[gn];
+        *o = relu && r == r ? fmaxf(r, 0.0f) : r;
     }
 }
+
+// what follows a product: a bias per column, in the product's type or fp32, and a relu
+struct ColumnBias {
+    const half_t *h;
+    const float *f;
+    int relu;
+    __device__ __forceinline__ float apply(float v, int n) const
+    {
+        if(h)
+            v += (float)h[n];
+        if(f)
+            v += f[n];
+        return relu && v == v ? fmaxf(v, 0.0f) : v;
+    }
+};
 
 // One operand tile (64 rows x 32 reduction steps) from global memory into LDS rows of LDK
 // halves.  kcontig: element (row, k) is at base[row*ld + k], else at base[k*ld + row].
@@ -113,7 +133,7 @@ __device__ __forceinline__ void gemm_stage(half_t (*dst)[GLDK], const half_t *__
 __global__ void __launch_bounds__(256)
     gemm_mfma_f16(int tA, int tB, int M, int N, int K, float alpha, const half_t *__restrict__ A, int lda,
                   const half_t *__restrict__ B, int ldb, float beta, half_t *__restrict__ C, int ldc, int a_vec,
-                  int b_vec)
+                  int b_vec, ColumnBias cb)
 {
     __shared__ __attribute__((aligned(16))) half_t As[2][64][GLDK];
     __shared__ __attribute__((aligned(16))) half_t Bs[2][64][GLDK];
@@ -202,7 +222,7 @@ __global__ void __launch_bounds__(256)
             continue;
         half_t *o = C + (int64_t)m * ldc + n;
         const float r = alpha * acc[v];
-        *o = (half_t)(beta != 0.0f ? r + beta * (float)*o : r);
+        *o = (half_t)cb.apply(beta != 0.0f ? r + beta * (float)*o : r, n);
     }
 }
 
@@ -218,7 +238,7 @@ constexpr int GS_K = 64, GS_LD = GS_K + 8, GS_WAVES = 8;
 template <bool tA, bool tB, bool VEC>
 __global__ void __launch_bounds__(64 * GS_WAVES)
     gemm_split_f16(int M, int N, int K, float alpha, const half_t *__restrict__ A, int lda,
-                   const half_t *__restrict__ B, int ldb, float beta, half_t *__restrict__ C, int ldc)
+                   const half_t *__restrict__ B, int ldb, float beta, half_t *__restrict__ C, int ldc, ColumnBias cb)
 {
     __shared__ __attribute__((aligned(16))) half_t st[GS_WAVES][2][32][GS_LD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -305,15 +325,15 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
         if(m < M && n < N) {
             half_t *o = C + (int64_t)m * ldc + n;
             r *= alpha;
-            *o = (half_t)(beta != 0.0f ? r + beta * (float)*o : r);
+            *o = (half_t)cb.apply(beta != 0.0f ? r + beta * (float)*o : r, n);
         }
     }
 }
 
 } // namespace
 
-extern "C" int saga_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda,
-                             const void *B, int ldb, float beta, void *C, int ldc, int dtype, saga_stream_t stream)
+static int gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B, int ldb,
+                float beta, void *C, int ldc, int dtype, const ColumnBias &cb, saga_stream_t stream)
 {
     if(!A || !B || !C || M < 1 || N < 1 || K < 1)
         return SAGA_HIP_EINVAL;
@@ -335,24 +355,41 @@ extern "C" int saga_hip_gemm(int transA, int transB, int M, int N, int K, float 
                                : transB ? vec ? gemm_split_f16<false, true, true> : gemm_split_f16<false, true, false>
                                         : vec ? gemm_split_f16<false, false, true> : gemm_split_f16<false, false, false>;
             kern<<<dim3((N + 31) / 32, (M + 31) / 32), 64 * GS_WAVES, 0, st>>>(M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
-                                                                             ldb, beta, (half_t *)C, ldc);
+                                                                             ldb, beta, (half_t *)C, ldc, cb);
             SAGA_CHECK_LAUNCH();
             return 0;
         }
         gemm_mfma_f16<<<grid, 256, 0, st>>>(transA, transB, M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
-                                            ldb, beta, (half_t *)C, ldc, a_vec, b_vec);
+                                            ldb, beta, (half_t *)C, ldc, a_vec, b_vec, cb);
     } else if(dtype == SAGA_FLOAT) {
         // (one slice of the LDS tiles holds such a reduction: 3.5 against 5.8 us on 31x17x9)
         if(K > 16) {
             const int r = stream_f32_gemm(transA, transB, M, N, K, alpha, (const float *)A, lda, (const float *)B, ldb, beta,
-                                          (float *)C, ldc, nullptr, 0, st);
+                                          (float *)C, ldc, cb.f, cb.relu, st);
             if(r != SAGA_HIP_EUNSUPPORTED)
                 return r;
         }
         gemm_mfma_f32<<<grid, 256, 0, st>>>(transA, transB, M, N, K, alpha, (const float *)A, lda, (const float *)B, ldb,
-                                            beta, (float *)C, ldc);
+                                            beta, (float *)C, ldc, cb.f, cb.relu);
     } else
         return SAGA_HIP_EUNSUPPORTED;
     SAGA_CHECK_LAUNCH();
     return 0;
+}
+
+extern "C" int saga_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda,
+                             const void *B, int ldb, float beta, void *C, int ldc, int dtype, saga_stream_t stream)
+{
+    return gemm(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, dtype, ColumnBias{nullptr, nullptr, 0}, stream);
+}
+
+extern "C" int saga_hip_gemm_bias(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda,
+                                  const void *B, int ldb, float beta, void *C, int ldc, int dtype, const void *bias, int bias_dtype,
+                                  int relu, saga_stream_t stream)
+{
+    if(bias && bias_dtype != SAGA_FLOAT && !(bias_dtype == SAGA_HALF && dtype == SAGA_HALF))
+        return SAGA_HIP_EUNSUPPORTED;
+    const ColumnBias cb = {bias_dtype == SAGA_HALF ? (const half_t *)bias : nullptr, bias_dtype == SAGA_FLOAT ? (const float *)bias : nullptr,
+                           relu};
+    return gemm(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, dtype, cb, stream);
 }

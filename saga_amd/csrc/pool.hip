@@ -102,7 +102,7 @@ __device__ __forceinline__ bool same(float a, float b) { return a == b || (a != 
 
 template <typename T, int VN, int MODE>
 __global__ void __launch_bounds__(256)
-    pool_fwd_k(DView x, DView y, DView idx, int has_idx, int k, int pad, int stride, int64_t total)
+    pool_fwd_k(DView x, DView y, DView idx, int has_idx, int k, int pad, int stride, int relu, int64_t total)
 {
     const int C = y.d[1], P = y.d[2], Q = y.d[3], H = x.d[2], W = x.d[3];
     const float inv = 1.0f / (float)(k * k);
@@ -145,6 +145,11 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
             for(int j = 0; j < VN; j++)
                 acc[j] *= inv;
+        }
+        if(relu) {
+#pragma unroll
+            for(int j = 0; j < VN; j++)
+                acc[j] = acc[j] != acc[j] ? acc[j] : fmaxf(acc[j], 0.0f);
         }
         PV<T, VN>::store((T *)y.ptr + off4(y, n, c, p, q), acc);
         if(MODE == SAGA_POOL_MAX && has_idx) {
@@ -1077,10 +1082,8 @@ static bool codes_ok(const SagaTensorView *a, const SagaTensorView *b, int size,
 static void launch_maxpool_codes(const SagaTensorView *x, const SagaTensorView *y, uint8_t *codes, int size, int pad,
                                  int stride, hipStream_t st, const float *ss = nullptr, int relu = 0);
 
-extern "C" {
-
-int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *idx,
-                      int size, int pad, int stride, saga_stream_t stream)
+static int pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *idx, int size, int pad,
+                    int stride, int relu, saga_stream_t stream)
 {
     if(!valid_view(x) || !valid_view(y) || size < 1 || stride < 1 || pad < 0 || (idx && !valid_view(idx)))
         return SAGA_HIP_EINVAL;
@@ -1099,6 +1102,8 @@ int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y
     // variant, which has all loads of a window in flight at once (no division in the work mapping), without its
     // position codes (the 112x112 stem output of ResNet-50 b256: 150 -> 110 us)
     if(mode == SAGA_POOL_MAX && !idx && codes_ok(x, y, size, pad, stride)) {
+        if(relu)
+            return SAGA_HIP_EUNSUPPORTED;
         launch_maxpool_codes(x, y, nullptr, size, pad, stride, st);
         SAGA_CHECK_LAUNCH();
         return 0;
@@ -1109,19 +1114,21 @@ int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y
     int lanes = 0;
     if(size >= 4 && total <= (int64_t)size * size * 2048 && total < (1 << 22))
         lanes = size < 16 ? 16 : size < 90 ? 256 : 1024;
+    if(relu && mode == SAGA_POOL_AVG && lanes)
+        return SAGA_HIP_EUNSUPPORTED;
     DView dvx = dview(x), dvy = dview(y), dvi = idx ? dview(idx) : dview(y);
 #define GO(T, VN)                                                                                        \
     do {                                                                                                 \
         if(mode == SAGA_POOL_MAX)                                                                        \
             pool_fwd_k<T, VN, SAGA_POOL_MAX><<<g, 256, 0, st>>>(dvx, dvy, dvi, idx != nullptr, size, pad, \
-                                                                stride, total);                          \
+                                                                stride, relu, total);                    \
         else if(lanes == 1024)                                                                           \
             avgpool_fwd_split_k<T, VN, 1024><<<(int)total, 1024, 0, st>>>(dvx, dvy, size, pad, stride, 1024, total); \
         else if(lanes)                                                                                   \
             avgpool_fwd_split_k<T, VN, 256><<<(int)((total * lanes + 255) / 256), 256, 0, st>>>(dvx, dvy, size, pad, stride, \
                                                                                                 lanes, total); \
         else                                                                                             \
-            pool_fwd_k<T, VN, SAGA_POOL_AVG><<<g, 256, 0, st>>>(dvx, dvy, dvi, 0, size, pad, stride, total); \
+            pool_fwd_k<T, VN, SAGA_POOL_AVG><<<g, 256, 0, st>>>(dvx, dvy, dvi, 0, size, pad, stride, relu, total); \
     } while(0)
     if(x->dtype == SAGA_HALF) {
         if(vn == 8) GO(half_t, 8); else GO(half_t, 1);
@@ -1131,6 +1138,20 @@ int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y
 #undef GO
     SAGA_CHECK_LAUNCH();
     return 0;
+}
+
+extern "C" {
+
+int saga_hip_pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *idx,
+                      int size, int pad, int stride, saga_stream_t stream)
+{
+    return pool_fwd(mode, x, y, idx, size, pad, stride, 0, stream);
+}
+
+int saga_hip_pool_fwd_relu(int mode, const SagaTensorView *x, const SagaTensorView *y, int size, int pad, int stride,
+                           saga_stream_t stream)
+{
+    return pool_fwd(mode, x, y, nullptr, size, pad, stride, 1, stream);
 }
 
 int saga_hip_pool_bwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *dy,

@@ -205,6 +205,17 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
 #pragma unroll
         for(int t = 0; t < TN; t++)
             acc[i][t] = float4_t{0, 0, 0, 0};
+    if(g.bias && ks == 0) // one of the wavefronts that share the reduction starts from it
+#pragma unroll
+        for(int t = 0; t < TN; t++)
+#pragma unroll
+            for(int v = 0; v < 4; v++) {
+                const int n = n0 + 16 * t + 4 * kq + v;
+                const float b = n < g.N ? (float)g.bias[n] : 0.0f;
+#pragma unroll
+                for(int i = 0; i < TM; i++)
+                    acc[i][t][v] = b;
+            }
 #pragma unroll
     for(int u = 0; u < DEPTH - 1; u++)
         load_step(u);

@@ -12,6 +12,7 @@ struct StreamF16 {
     int IH, IW, OH, OW, R, S, pad, stride, dil, lda, ldo;
     int bwd;         // backward data: stride and dilation act on the output side
     float alpha, beta;
+    const half_t *bias; // optional, alpha == 1: per output channel, added to the product
     // forward, optional: y = act(v * sc + sh (+ z)), sc = s*rsqrt(v+eps), sh = b - m*sc
     const float *bn_s, *bn_b, *bn_m, *bn_v;
     float bn_eps;

@@ -189,6 +189,8 @@ struct HipOperation {
     virtual float *getBeta(const std::shared_ptr<HipTensor> &t) { return nullptr; }
     // drop an output nobody reads; false if the op cannot do without it
     virtual bool killOutput(const std::shared_ptr<HipStorage> &s) { return false; }
+    // inference: write relu(output) to y instead of the output; false if the operation cannot
+    virtual bool foldRelu(const std::shared_ptr<HipTensor> &y) { return false; }
     virtual std::string info() const { return ""; }
     // algorithmic work of one execution: floating point operations (matrix ops) and bytes that
     // must cross HBM (memory-bound ops); used for roofline accounting only

@@ -52,7 +52,11 @@ struct ConvFwd : public HipOperation {
     T bn_s_, bn_b_, bn_m_, bn_v_, bn_z_, bn_y_;
     float bn_eps_ = 0;
     int bn_flags_ = 0;
-    ConvFwd(HipProgram &p, T x, T w, T y, SagaConvParams cp) : HipOperation("convfwd"), x_(x), w_(w), y_(y), cp_(cp)
+    // the layer's bias, and (inference) the tensor of a relu behind it
+    const T b_;
+    T relu_y_;
+    ConvFwd(HipProgram &p, T x, T w, T y, SagaConvParams cp, T b = nullptr)
+      : HipOperation("convfwd"), x_(x), w_(w), y_(y), cp_(cp), b_(b)
     {
         const SagaTensorView vx = x->shapeView(), vw = w->shapeView(), vy = y->shapeView();
         p.m_ctx->m_workspace.request(saga_hip_conv2d_workspace_size(SAGA_CONV_FWD, &vx, &vw, &vy, &cp_));
@@ -62,6 +66,8 @@ struct ConvFwd : public HipOperation {
     {
         if(stats_)
             return stats_;
+        if(b_)
+            return nullptr;
         const SagaTensorView vx = x_->shapeView(), vw = w_->shapeView(), vy = y_->shapeView();
         const size_t bytes = saga_hip_conv2d_fwd_bnstats_size(&vx, &vw, &vy, &cp_);
         if(!bytes)
@@ -72,12 +78,20 @@ struct ConvFwd : public HipOperation {
     }
     bool foldBn(T s, T b, T m, T v, T z, T y, float eps, int flags)
     {
-        if(stats_ || bn_y_)
+        if(stats_ || bn_y_ || b_)
             return false;
         bn_s_ = s; bn_b_ = b; bn_m_ = m; bn_v_ = v; bn_z_ = z; bn_y_ = y;
         bn_eps_ = eps;
         bn_flags_ = flags;
         m_kind = "convfwd.bn";
+        return true;
+    }
+    // (a kernel takes both only together, and only in fp32)
+    bool foldRelu(const T &y) override
+    {
+        if(!b_ || relu_y_ || x_->m_data_type != Tensor::DataType::FLOAT)
+            return false;
+        relu_y_ = y;
         return true;
     }
     void execFolded(HipProgram &p)
@@ -104,7 +118,13 @@ struct ConvFwd : public HipOperation {
     {
         if(bn_y_)
             return execFolded(p);
-        const SagaTensorView vx = x_->view(), vw = w_->view(), vy = y_->view();
+        const SagaTensorView vx = x_->view(), vw = w_->view(), vy = relu_y_ ? relu_y_->view() : y_->view();
+        if(b_) {
+            const SagaTensorView vb = b_->view();
+            chkSaga(saga_hip_conv2d_fwd_bias(&vx, &vw, &vb, &vy, &cp_, beta_, relu_y_ ? 1 : 0, p.workspace().ptr(),
+                                             p.workspace().size(), S(p)));
+            return;
+        }
         if(stats_) {
             stats_->valid = false;
             if(beta_ == 0.0f) {
@@ -125,6 +145,8 @@ struct ConvFwd : public HipOperation {
     HipOpArgs listInputs() const override
     {
         HipOpArgs r{{"x", x_}, {"w", w_}};
+        if(b_)
+            r.push_back({"b", b_});
         if(bn_y_) {
             r.insert(r.end(), {{"s", bn_s_}, {"b", bn_b_}, {"m", bn_m_}, {"v", bn_v_}});
             if(bn_z_)
@@ -132,8 +154,8 @@ struct ConvFwd : public HipOperation {
         }
         return r;
     }
-    HipOpArgs listOutputs() const override { return {{"y", bn_y_ ? bn_y_ : y_}}; }
-    float *getBeta(const T &t) override { return !bn_y_ && t == y_ ? &beta_ : nullptr; }
+    HipOpArgs listOutputs() const override { return {{"y", bn_y_ ? bn_y_ : relu_y_ ? relu_y_ : y_}}; }
+    float *getBeta(const T &t) override { return !bn_y_ && !relu_y_ && t == y_ ? &beta_ : nullptr; }
     double flops() const override { return conv_flops(x_, w_, y_, cp_.group); }
     double bytes() const override
     {
@@ -251,7 +273,7 @@ struct ConvBwdData : public HipOperation {
     int bn_flags_ = 0;
     std::shared_ptr<BnBwdLinkState> linkBnBwd(T x, T s, T b, T sm, T sv, int flags)
     {
-        if(link_)
+        if(link_ || b_)
             return nullptr;
         // The epilogue's extra work (one more tensor to read, the mask and the sums) costs the convolution
         // more than the norm's first pass saves where the convolution has little arithmetic per output to
@@ -271,8 +293,9 @@ struct ConvBwdData : public HipOperation {
         m_kind = "convbwddata.bn";
         return link_;
     }
-    ConvBwdData(HipProgram &p, HipProgramUnit &pu, T w, T dy, T dx, SagaConvParams cp)
-      : HipOperation("convbwddata"), w_(w), dy_(dy), dx_(dx), cp_(cp)
+    const T b_; // the bias of a transposed convolution
+    ConvBwdData(HipProgram &p, HipProgramUnit &pu, T w, T dy, T dx, SagaConvParams cp, T b = nullptr)
+      : HipOperation("convbwddata"), w_(w), dy_(dy), dx_(dx), cp_(cp), b_(b)
     {
         const SagaTensorView vx = dx->shapeView(), vw = w->shapeView(), vy = dy->shapeView();
         p.m_ctx->m_workspace.request(saga_hip_conv2d_workspace_size(SAGA_CONV_BWD_DATA, &vx, &vw, &vy, &cp_));
@@ -290,6 +313,12 @@ struct ConvBwdData : public HipOperation {
     void exec(HipProgram &p) override
     {
         const SagaTensorView vdy = dy_->view(), vw = w_->view(), vdx = dx_->view();
+        if(b_) {
+            const SagaTensorView vb = b_->view();
+            chkSaga(saga_hip_conv2d_bwd_data_bias(&vdy, &vw, wt_ ? wt_->deviceMem() : nullptr, &vb, &vdx, &cp_, beta_,
+                                                  p.workspace().ptr(), p.workspace().size(), S(p)));
+            return;
+        }
         if(link_ && !link_->refused) {
             link_->valid = false;
             const SagaTensorView vx = bn_x_->view();
@@ -321,6 +350,8 @@ struct ConvBwdData : public HipOperation {
         HipOpArgs r{{"w", w_}, {"dy", dy_}};
         if(wt_)
             r.push_back({"wt", wt_});
+        if(b_)
+            r.push_back({"b", b_});
         if(link_)
             r.insert(r.end(), {{"bn.x", bn_x_}, {"bn.s", bn_s_}, {"bn.b", bn_b_}, {"bn.sm", bn_sm_}, {"bn.sv", bn_sv_}});
         return r;
@@ -409,10 +440,11 @@ void conv_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
     cp.group = n.m_attributes.get("group", 1);
     const bool transpose = n.m_attributes.get("transpose", false);
     const bool training = p.m_pt == ProgramType::TRAINING;
+    const T fused_b = p.m_pc.disable_op_fusing ? nullptr : b; // the bias goes along in the epilogue
 
     if(!transpose) {
-        pu.fwd(std::make_shared<ConvFwd>(p, x, w, y, cp));
-        if(b)
+        pu.fwd(std::make_shared<ConvFwd>(p, x, w, y, cp, fused_b));
+        if(b && !fused_b)
             pu.fwd(std::make_shared<BiasAdd>(b, y));
         if(!training)
             return;
@@ -429,8 +461,8 @@ void conv_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
             pu.bwd(std::make_shared<ConvBwdData>(p, pu, w, dy, dx, cp));
     } else {
         // transposed convolution: the three kernels with x and y exchanged (:542-574)
-        pu.fwd(std::make_shared<ConvBwdData>(p, pu, w, x, y, cp));
-        if(b)
+        pu.fwd(std::make_shared<ConvBwdData>(p, pu, w, x, y, cp, fused_b));
+        if(b && !fused_b)
             pu.fwd(std::make_shared<BiasAdd>(b, y));
         if(!training)
             return;
@@ -494,10 +526,30 @@ struct ActBwd : public HipOperation {
     double bytes() const override { return (beta_ != 0 ? 4 : 3) * nbytes(dx_); }
 };
 
+bool single_consumer(const Nodes &nodes, const std::shared_ptr<Tensor> &t);
+
 void activation_setup(HipProgram &p, HipProgramUnit &pu, const Node &n, int mode, float alpha)
 {
     auto x = p.lower(pu, n.m_inputs["x"]);
     auto y = p.lowerLike(pu, n.m_outputs["y"], *x);
+    if(p.m_pt == ProgramType::INFERENCE && mode == SAGA_ACT_RELU && !p.m_pc.disable_op_fusing) {
+        // the one operation that writes x writes y instead, if nobody else looks at x
+        std::shared_ptr<HipOperation> producer;
+        int touching = 0;
+        for(const auto &op : pu.m_fwd)
+            for(const auto &list : {op->listInputs(), op->listOutputs()})
+                for(const auto &o : list)
+                    if(o.second->m_storage == x->m_storage) {
+                        touching++;
+                        producer = op;
+                    }
+        const auto &ex = p.m_ctx->m_exported;
+        const bool held = std::any_of(ex.begin(), ex.end(), [&](const auto &e) { return e == x->m_storage; });
+        const auto outs = producer ? producer->listOutputs() : HipOpArgs();
+        if(touching == 1 && !held && outs.size() == 1 && outs[0].second == x && single_consumer(pu.m_transformed, n.m_inputs["x"]) &&
+           producer->foldRelu(y))
+            return;
+    }
     pu.fwd(std::make_shared<ActFwd>(x, y, mode, alpha));
     if(p.m_pt == ProgramType::INFERENCE)
         return;
@@ -528,9 +580,11 @@ struct Gemm : public HipOperation {
     const int ta_, tb_, m_, n_, k_;
     const T a_, b_, c_;
     const int lda_, ldb_, ldc_;
+    const T bias_; // per column
+    T relu_c_;     // inference: the tensor of a relu behind it
     float beta_ = 0;
-    Gemm(int ta, int tb, int m, int n, int k, T a, int lda, T b, int ldb, T c, int ldc, const char *name)
-      : HipOperation(name), ta_(ta), tb_(tb), m_(m), n_(n), k_(k), a_(a), b_(b), c_(c), lda_(lda), ldb_(ldb), ldc_(ldc)
+    Gemm(int ta, int tb, int m, int n, int k, T a, int lda, T b, int ldb, T c, int ldc, const char *name, T bias = nullptr)
+      : HipOperation(name), ta_(ta), tb_(tb), m_(m), n_(n), k_(k), a_(a), b_(b), c_(c), lda_(lda), ldb_(ldb), ldc_(ldc), bias_(bias)
     {
         if(a->m_data_type != b->m_data_type || a->m_data_type != c->m_data_type)
             throw std::runtime_error("fc: operand data types differ");
@@ -539,13 +593,28 @@ struct Gemm : public HipOperation {
     }
     void exec(HipProgram &p) override
     {
-        chkSaga(saga_hip_gemm(ta_, tb_, m_, n_, k_, 1.0f, a_->deviceMem(), lda_, b_->deviceMem(), ldb_, beta_,
-                              c_->deviceMem(), ldc_, (int)a_->m_data_type, S(p)));
+        chkSaga(saga_hip_gemm_bias(ta_, tb_, m_, n_, k_, 1.0f, a_->deviceMem(), lda_, b_->deviceMem(), ldb_, beta_,
+                                   (relu_c_ ? relu_c_ : c_)->deviceMem(), ldc_, (int)a_->m_data_type,
+                                   bias_ ? bias_->deviceMem() : nullptr, bias_ ? (int)bias_->m_data_type : SAGA_FLOAT,
+                                   relu_c_ ? 1 : 0, S(p)));
+    }
+    bool foldRelu(const T &y) override
+    {
+        if(relu_c_ || !y->rowMajor())
+            return false;
+        relu_c_ = y;
+        return true;
     }
     bool sideSafe() const override { return true; }
-    HipOpArgs listInputs() const override { return {{"a", a_}, {"b", b_}}; }
-    HipOpArgs listOutputs() const override { return {{"c", c_}}; }
-    float *getBeta(const T &t) override { return t == c_ ? &beta_ : nullptr; }
+    HipOpArgs listInputs() const override
+    {
+        HipOpArgs r{{"a", a_}, {"b", b_}};
+        if(bias_)
+            r.push_back({"bias", bias_});
+        return r;
+    }
+    HipOpArgs listOutputs() const override { return {{"c", relu_c_ ? relu_c_ : c_}}; }
+    float *getBeta(const T &t) override { return !relu_c_ && t == c_ ? &beta_ : nullptr; }
     double flops() const override { return 2.0 * m_ * n_ * k_; }
     double bytes() const override { return nbytes(a_) + nbytes(b_) + nbytes(c_); }
 };
@@ -559,10 +628,12 @@ void fc_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
     const bool transW = n.m_attributes.get("transW", false);
     const int in = x->m_dims[1], out = y->m_dims[1], batch = x->m_dims[0];
 
+    const bool takes = b && (b->m_data_type == Tensor::DataType::FLOAT || b->m_data_type == x->m_data_type);
+    const T fused_b = takes && !p.m_pc.disable_op_fusing ? b : nullptr; // the bias goes along in the epilogue
     // y[batch,out] = x[batch,in] * W ; W stored [in,out], or [out,in] when transW
     pu.fwd(std::make_shared<Gemm>(0, transW ? 1 : 0, batch, out, in, x, in, w, transW ? in : out, y, out,
-                                  transW ? "fc.fwd.t" : "fc.fwd.n"));
-    if(b)
+                                  transW ? "fc.fwd.t" : "fc.fwd.n", fused_b));
+    if(b && !fused_b)
         pu.fwd(std::make_shared<BiasAdd>(b, y));
     if(p.m_pt == ProgramType::INFERENCE)
         return;
@@ -1059,8 +1130,6 @@ void link_bn_backward(HipProgram &p, HipOps &ops)
 
 namespace {
 
-bool single_consumer(const Nodes &nodes, const std::shared_ptr<Tensor> &t);
-
 // x0 = normalised input, x1 = residual (optional); flags from the "relu" attribute
 void batchnorm_lower(HipProgram &p, HipProgramUnit &pu, const Node &n, std::shared_ptr<Tensor> xh,
                      std::shared_ptr<Tensor> zh, int flags)
@@ -1219,10 +1288,29 @@ struct PoolFwd : public HipOperation {
     void exec(HipProgram &p) override
     {
         const SagaTensorView vx = x_->view(), vy = y_->view();
-        chkSaga(saga_hip_pool_fwd(mode_, &vx, &vy, nullptr, size_, pad_, stride_, S(p)));
+        if(!relu_y_) {
+            chkSaga(saga_hip_pool_fwd(mode_, &vx, &vy, nullptr, size_, pad_, stride_, S(p)));
+            return;
+        }
+        const SagaTensorView vr = relu_y_->view();
+        const int r = saga_hip_pool_fwd_relu(mode_, &vx, &vr, size_, pad_, stride_, S(p));
+        if(r != SAGA_HIP_EUNSUPPORTED) {
+            chkSaga(r);
+            return;
+        }
+        chkSaga(saga_hip_pool_fwd(mode_, &vx, &vr, nullptr, size_, pad_, stride_, S(p)));
+        chkSaga(saga_hip_act_fwd(SAGA_ACT_RELU, 0, &vr, &vr, 0.0f, S(p)));
+    }
+    T relu_y_; // inference: the tensor of a relu behind it
+    bool foldRelu(const T &y) override
+    {
+        if(relu_y_)
+            return false;
+        relu_y_ = y;
+        return true;
     }
     HipOpArgs listInputs() const override { return {{"x", x_}}; }
-    HipOpArgs listOutputs() const override { return {{"y", y_}}; }
+    HipOpArgs listOutputs() const override { return {{"y", relu_y_ ? relu_y_ : y_}}; }
     std::string info() const override { return mode_ == SAGA_POOL_MAX ? "max" : "avg"; }
     double bytes() const override { return nbytes(x_) + nbytes(y_); }
 };
