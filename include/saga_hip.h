@@ -137,12 +137,42 @@ int saga_hip_conv2d_bwd_data_wt(const SagaTensorView *dy, const SagaTensorView *
  *      SAGA_HIP_EUNSUPPORTED (nothing written to y) when the fp16 channels-last MFMA path does
  *      not cover the problem: run saga_hip_conv2d_fwd and saga_hip_bn_train_fwd instead.
  *      _size: bytes `partial` must hold (0: never supported for these operands). */
-/* y = act(conv(x, w) + beta * y + bias), bias broadcast over the channels (any view of K elements), act a relu if `relu`:
- * in the convolution's epilogue where its kernel has one, otherwise in passes of their own.  The backward-data form is the
- * forward pass of a transposed convolution with a bias; wt as in saga_hip_conv2d_bwd_data_wt (may be null). */
-int saga_hip_conv2d_fwd_bias(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *bias,
-                             const SagaTensorView *y, const SagaConvParams *p, float beta, int relu, void *workspace,
-                             size_t ws_bytes, saga_stream_t stream);
+/* fp32 filters in the order in which the convolution kernel loads them.  A program that runs a layer many times packs its
+ * filter once per change of the weights, all filters in one launch:
+ *   pack_bytes: size of the packed copy, 0 where no kernel reads one; `kind` FWD or BWD_DATA;
+ *   pack_jobs:  describes the copying of one filter (w->ptr and `packed` are device addresses) in up to
+ *               SAGA_CONV_PACK_JOBS jobs, whose number it returns; first_block is the caller's: running sum of `blocks`;
+ *   filter_pack_batched: runs the jobs (an array in device memory).
+ * The copy goes to saga_hip_conv2d_fwd_ex (packed) or to the wt of saga_hip_conv2d_bwd_data_wt / _bias. */
+#define SAGA_CONV_PACK_JOBS 16
+typedef struct SagaFilterPackJob {
+    const void *w;
+    void *packed;
+    int64_t w_sn, w_sc, w_sr, w_ss;
+    int32_t N, C, T, Ts, r0, s0, rstep;
+    int32_t first_block, blocks;
+} SagaFilterPackJob;
+size_t saga_hip_conv2d_pack_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
+                                  const SagaConvParams *p);
+int saga_hip_conv2d_pack_jobs(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
+                              const SagaConvParams *p, void *packed, SagaFilterPackJob *jobs);
+int saga_hip_filter_pack_batched(const SagaFilterPackJob *jobs_device, int njobs, int total_blocks, saga_stream_t stream);
+
+/* y = act(norm(conv(x, w) + beta * y + bias) + z): what a network puts behind a convolution, in its epilogue where its
+ * kernel has one and otherwise in passes of their own.  bias: any view of K elements; norm: as in
+ * saga_hip_conv2d_fwd_bn_infer, without bias and beta, and SAGA_HIP_EUNSUPPORTED as there; z only with a norm; all optional.
+ * The backward-data form is the forward pass of a transposed convolution with a bias (may be null); wt as in
+ * saga_hip_conv2d_bwd_data_wt (may be null), or a packed fp32 filter. */
+typedef struct SagaConvExtras {
+    const void *packed;
+    const SagaTensorView *bias;
+    const float *s, *b, *m, *v;
+    float eps;
+    const SagaTensorView *z;
+    int relu;
+} SagaConvExtras;
+int saga_hip_conv2d_fwd_ex(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
+                           float beta, const SagaConvExtras *e, void *workspace, size_t ws_bytes, saga_stream_t stream);
 int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView *w, const void *wt,
                                   const SagaTensorView *bias, const SagaTensorView *dx, const SagaConvParams *p, float beta,
                                   void *workspace, size_t ws_bytes, saga_stream_t stream);

@@ -1,9 +1,8 @@
 // Convolution entry points: argument checking, geometry, and the choice between the MFMA
 // implicit-GEMM kernels and the direct fallback.
-#include "conv.hpp"
+#include "stream_f32.hpp"
 
 #include <stdlib.h>
-#include <string.h>
 
 namespace {
 
@@ -60,6 +59,33 @@ size_t saga_hip_conv2d_workspace_size(int kind, const SagaTensorView *x, const S
     return std::max(conv_mfma_workspace(kind, x, w, y, g), conv_f32_workspace(kind, x, w, y, g));
 }
 
+// forward with the norm of `e` (+ residual + relu) in the epilogue
+static int fwd_norm(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g,
+                    const SagaConvExtras &e, void *workspace, size_t ws_bytes, hipStream_t st)
+{
+    if(force_direct())
+        return SAGA_HIP_EUNSUPPORTED;
+    if(x->dtype == SAGA_FLOAT) {
+        if(e.z && (e.z->dtype != SAGA_FLOAT || !valid_view(e.z) || !same_dims(e.z, y)))
+            return SAGA_HIP_EUNSUPPORTED;
+        StreamEpilogue se;
+        se.bn_s = e.s, se.bn_b = e.b, se.bn_m = e.m, se.bn_v = e.v;
+        se.bn_eps = e.eps;
+        se.z = e.z;
+        se.relu = e.relu;
+        return conv_f32_fwd(x, w, y, g, 1.0f, 0.0f, workspace, ws_bytes, st, se, e.packed);
+    }
+    const ConvBnFold bn = {e.s, e.b, e.m, e.v, e.eps, (e.z ? SAGA_BN_ADD : 0) | (e.relu ? SAGA_BN_RELU : 0), e.z};
+    return conv_mfma_fwd(x, w, y, g, 1.0f, 0.0f, workspace, ws_bytes, st, nullptr, 0, nullptr, &bn);
+}
+
+// whether backward data reads a filter that was transposed (fp16) or packed (fp32) beforehand
+static bool takes_wt(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g)
+{
+    return !force_direct() && (dx->dtype == SAGA_FLOAT ? conv_f32_packed_bytes(SAGA_CONV_BWD_DATA, dx, w, dy, g) > 0
+                                                       : conv_mfma_bwd_data_ok(dy, w, dx, g));
+}
+
 int saga_hip_conv2d_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                         const SagaConvParams *p, float alpha, float beta, void *workspace, size_t ws_bytes,
                         saga_stream_t stream)
@@ -91,37 +117,71 @@ static bool bias_ok(const SagaTensorView *bias, const SagaTensorView *out)
     return valid_view(bias) && view_elements(bias) == out->dims[1];
 }
 
-int saga_hip_conv2d_fwd_bias(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *bias,
-                             const SagaTensorView *y, const SagaConvParams *p, float beta, int relu, void *workspace,
-                             size_t ws_bytes, saga_stream_t stream)
+int saga_hip_conv2d_fwd_ex(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
+                           float beta, const SagaConvExtras *e, void *workspace, size_t ws_bytes, saga_stream_t stream)
 {
     ConvGeom g;
     int r = geometry(x, w, y, p, &g);
     if(r)
         return r;
-    if(!bias_ok(bias, y))
-        return SAGA_HIP_ESHAPE;
+    if(!e)
+        return SAGA_HIP_EINVAL;
     hipStream_t st = as_stream(stream);
+    if(e->s) {
+        if(!e->b || !e->m || !e->v || e->bias || beta != 0.0f)
+            return SAGA_HIP_EINVAL;
+        return fwd_norm(x, w, y, g, *e, workspace, ws_bytes, st);
+    }
+    if(e->z || (e->relu && !e->bias))
+        return SAGA_HIP_EUNSUPPORTED;
+    const SagaTensorView *bias = e->bias;
+    if(bias && !bias_ok(bias, y))
+        return SAGA_HIP_ESHAPE;
     bool done = false;
     r = SAGA_HIP_EUNSUPPORTED;
     if(!force_direct()) {
         r = conv_mfma_fwd(x, w, y, g, 1.0f, beta, workspace, ws_bytes, st, nullptr, 0, nullptr, nullptr,
-                          bias->dtype == SAGA_HALF && !relu ? bias->ptr : nullptr, &done);
+                          bias && bias->dtype == SAGA_HALF && !e->relu ? bias->ptr : nullptr, &done);
         if(r == SAGA_HIP_EUNSUPPORTED) {
-            StreamEpilogue e;
-            done = bias->dtype == SAGA_FLOAT;
+            StreamEpilogue se;
+            done = bias && bias->dtype == SAGA_FLOAT;
             if(done) {
-                e.bias = (const float *)bias->ptr;
-                e.relu = relu;
+                se.bias = (const float *)bias->ptr;
+                se.relu = e->relu;
             }
-            r = conv_f32_fwd(x, w, y, g, 1.0f, beta, workspace, ws_bytes, st, e);
+            r = conv_f32_fwd(x, w, y, g, 1.0f, beta, workspace, ws_bytes, st, se, e->packed);
         }
     }
     if(r == SAGA_HIP_EUNSUPPORTED) {
         done = false;
         r = conv_direct_fwd(x, w, y, g, 1.0f, beta, st);
     }
-    return r || done ? r : add_bias(bias, y, relu, stream);
+    return r || done || !bias ? r : add_bias(bias, y, e->relu, stream);
+}
+
+size_t saga_hip_conv2d_pack_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
+                                  const SagaConvParams *p)
+{
+    ConvGeom g;
+    if(geometry(x, w, y, p, &g) || force_direct() || (kind != SAGA_CONV_FWD && kind != SAGA_CONV_BWD_DATA))
+        return 0;
+    return conv_f32_packed_bytes(kind, x, w, y, g);
+}
+
+int saga_hip_conv2d_pack_jobs(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
+                              const SagaConvParams *p, void *packed, SagaFilterPackJob *jobs)
+{
+    ConvGeom g;
+    if(!packed || !jobs || !aligned16(packed) || !saga_hip_conv2d_pack_bytes(kind, x, w, y, p) || geometry(x, w, y, p, &g))
+        return 0;
+    return stream_f32_pack_jobs(kind == SAGA_CONV_BWD_DATA, w, g, packed, jobs);
+}
+
+int saga_hip_filter_pack_batched(const SagaFilterPackJob *jobs_device, int njobs, int total_blocks, saga_stream_t stream)
+{
+    if(!jobs_device || njobs < 1 || total_blocks < 1)
+        return SAGA_HIP_EINVAL;
+    return stream_f32_pack(jobs_device, njobs, total_blocks, as_stream(stream));
 }
 
 int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView *w, const void *wt, const SagaTensorView *bias,
@@ -132,29 +192,29 @@ int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView
     int r = geometry(dx, w, dy, p, &g);
     if(r)
         return r;
-    if(!bias_ok(bias, dx))
+    if(bias && !bias_ok(bias, dx))
         return SAGA_HIP_ESHAPE;
-    if(wt && (force_direct() || !conv_mfma_bwd_data_ok(dy, w, dx, g)))
+    if(wt && !takes_wt(dy, w, dx, g))
         return SAGA_HIP_EUNSUPPORTED;
     hipStream_t st = as_stream(stream);
     bool done = false;
     r = SAGA_HIP_EUNSUPPORTED;
     if(!force_direct()) {
         r = conv_mfma_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, wt, nullptr,
-                               bias->dtype == SAGA_HALF ? bias->ptr : nullptr, &done);
+                               bias && bias->dtype == SAGA_HALF ? bias->ptr : nullptr, &done);
         if(r == SAGA_HIP_EUNSUPPORTED) {
             StreamEpilogue e;
-            done = bias->dtype == SAGA_FLOAT;
+            done = bias && bias->dtype == SAGA_FLOAT;
             if(done)
                 e.bias = (const float *)bias->ptr;
-            r = conv_f32_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, e);
+            r = conv_f32_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, e, wt);
         }
     }
     if(r == SAGA_HIP_EUNSUPPORTED) {
         done = false;
         r = conv_direct_bwd_data(dy, w, dx, g, 1.0f, beta, st);
     }
-    return r || done ? r : add_bias(bias, dx, 0, stream);
+    return r || done || !bias ? r : add_bias(bias, dx, 0, stream);
 }
 
 size_t saga_hip_conv2d_fwd_bnstats_size(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
@@ -193,20 +253,8 @@ int saga_hip_conv2d_fwd_bn_infer(const SagaTensorView *x, const SagaTensorView *
         return r;
     if(!s || !b || !m || !v || ((flags & SAGA_BN_ADD) && !z))
         return SAGA_HIP_EINVAL;
-    if(force_direct())
-        return SAGA_HIP_EUNSUPPORTED;
-    if(x->dtype == SAGA_FLOAT) {
-        if(z && (z->dtype != SAGA_FLOAT || !valid_view(z) || memcmp(z->dims, y->dims, sizeof(z->dims))))
-            return SAGA_HIP_EUNSUPPORTED;
-        StreamEpilogue e;
-        e.bn_s = s, e.bn_b = b, e.bn_m = m, e.bn_v = v;
-        e.bn_eps = eps;
-        e.z = flags & SAGA_BN_ADD ? z : nullptr;
-        e.relu = flags & SAGA_BN_RELU ? 1 : 0;
-        return conv_f32_fwd(x, w, y, g, 1.0f, 0.0f, workspace, ws_bytes, as_stream(stream), e);
-    }
-    const ConvBnFold bn = {s, b, m, v, eps, flags, z};
-    return conv_mfma_fwd(x, w, y, g, 1.0f, 0.0f, workspace, ws_bytes, as_stream(stream), nullptr, 0, nullptr, &bn);
+    const SagaConvExtras e = {nullptr, nullptr, s, b, m, v, eps, flags & SAGA_BN_ADD ? z : nullptr, flags & SAGA_BN_RELU ? 1 : 0};
+    return fwd_norm(x, w, y, g, e, workspace, ws_bytes, as_stream(stream));
 }
 
 int saga_hip_conv2d_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx,
@@ -262,8 +310,10 @@ int saga_hip_conv2d_bwd_data_wt(const SagaTensorView *dy, const SagaTensorView *
     int r = geometry(dx, w, dy, p, &g);
     if(r)
         return r;
-    if(force_direct() || !conv_mfma_bwd_data_ok(dy, w, dx, g))
-        return SAGA_HIP_EUNSUPPORTED; // only the path saga_hip_conv2d_bwd_data_wt_bytes answered for takes wt
+    if(!takes_wt(dy, w, dx, g))
+        return SAGA_HIP_EUNSUPPORTED;
+    if(dx->dtype == SAGA_FLOAT)
+        return conv_f32_bwd_data(dy, w, dx, g, alpha, beta, workspace, ws_bytes, as_stream(stream), StreamEpilogue(), wt);
     return conv_mfma_bwd_data(dy, w, dx, g, alpha, beta, workspace, ws_bytes, as_stream(stream), wt);
 }
 

@@ -72,8 +72,12 @@ struct StreamEpilogue {
     int relu = 0;
 };
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,
-                 float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue());
+                 float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue(),
+                 const void *packed = nullptr);
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
-                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue());
+                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue(),
+                      const void *packed = nullptr);
+// bytes of the packed filter that a launch on these tensors reads (see stream_f32.hip); 0: none
+size_t conv_f32_packed_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g);
 int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g,
                         float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st);

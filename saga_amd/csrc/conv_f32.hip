@@ -933,20 +933,26 @@ size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorVie
     return tab_bytes(g.C * g.R * g.S) + (size_t)splits * g.K * g.C * g.R * g.S * sizeof(float) + 256;
 }
 
+// Operands shared through LDS pay once there are several rounds of full tiles: 537 against 562 us on 3x3 64->64 at
+// 256x56x56, 478 against 500 us on 3x3 32->464 at 36x70x70 (1x1 64->256 at 8x56x56, one round: equal).  Reduction channels
+// in other numbers than eights go through a table in both kernels, and the stream kernel's is read by every lane: 42
+// against 53 us on 7x7 3->64 at 8x224x224.
+static bool tiles_in_lds(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g)
+{
+    const int cols = out->dims[1], bn = cols > 64 ? 128 : 64;
+    const long long tiles = ((long long)out->dims[0] * out->dims[2] * out->dims[3] + FBM - 1) / FBM * ((cols + bn - 1) / bn);
+    return tiles >= ((bwd ? g.K : g.C) % 8 ? 512 : 2048) && cols > 48 && uniform_ok(bwd, a, g);
+}
+
 static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out,
-                         const ConvGeom &g, float alpha, float beta, const StreamEpilogue &e, void *ws, size_t ws_bytes, hipStream_t st)
+                         const ConvGeom &g, float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes,
+                         hipStream_t st)
 {
     // forward: a = x (N,C,H,W), out = y (N,K,P,Q); backward data: a = dy (N,K,P,Q), out = dx (N,C,H,W)
     const int red_ch = bwd ? g.K : g.C;
     const int Kred = red_ch * g.R * g.S;
-    // Operands shared through LDS pay once there are several rounds of full tiles: 537 against 562 us on 3x3 64->64 at
-    // 256x56x56, 478 against 500 us on 3x3 32->464 at 36x70x70 (1x1 64->256 at 8x56x56, one round: equal).  Reduction channels
-    // in other numbers than eights go through a table in both kernels, and the stream kernel's is read by every lane: 42
-    // against 53 us on 7x7 3->64 at 8x224x224.
-    const int cols = out->dims[1], bn = cols > 64 ? 128 : 64;
-    const long long tiles = ((long long)out->dims[0] * out->dims[2] * out->dims[3] + FBM - 1) / FBM * ((cols + bn - 1) / bn);
-    if(!(tiles >= (red_ch % 8 ? 512 : 2048) && cols > 48 && uniform_ok(bwd, a, g))) {
-        const int r = stream_f32_conv(bwd, a, w, out, g, alpha, beta, e, ws, ws_bytes, st);
+    if(!tiles_in_lds(bwd, a, out, g)) {
+        const int r = stream_f32_conv(bwd, a, w, out, g, alpha, beta, e, packed, ws, ws_bytes, st);
         if(r != SAGA_HIP_EUNSUPPORTED)
             return r;
     }
@@ -1105,20 +1111,26 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
     return 0;
 }
 
+size_t conv_f32_packed_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g)
+{
+    const bool bwd = kind == SAGA_CONV_BWD_DATA;
+    return f32_ok(x, w, y, g) && !tiles_in_lds(bwd, bwd ? y : x, bwd ? x : y, g) ? stream_f32_packed_bytes(bwd, g) : 0;
+}
+
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,
-                 float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e)
+                 float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e, const void *packed)
 {
     if(!f32_ok(x, w, y, g))
         return SAGA_HIP_EUNSUPPORTED;
-    return gather_launch(false, x, w, y, g, alpha, beta, e, ws, ws_bytes, st);
+    return gather_launch(false, x, w, y, g, alpha, beta, e, packed, ws, ws_bytes, st);
 }
 
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
-                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e)
+                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e, const void *packed)
 {
     if(!f32_ok(dy, w, dx, g))
         return SAGA_HIP_EUNSUPPORTED;
-    return gather_launch(true, dy, w, dx, g, alpha, beta, e, ws, ws_bytes, st);
+    return gather_launch(true, dy, w, dx, g, alpha, beta, e, packed, ws, ws_bytes, st);
 }
 
 int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g,

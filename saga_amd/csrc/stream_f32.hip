@@ -14,10 +14,10 @@
 // at the end: one launch, no partial results in memory, a fixed order of additions.
 //
 // Measured against the LDS-tiled kernels that did all of this before (us; graph replays, launch included): fc 64x3136 ->
-// 1024 306 -> 21 (12.8 MB of weights, 0.6 TB/s), its backward data 95 -> 14; 4096^3 2433 -> 1038 (132 TFLOP/s); 3x3
-// 512->512 at 8x7x7 499 -> 50, 256->256 at 8x14x14 249 -> 44, at 32x14x14 250 -> 96 (77 TFLOP/s); stride-2 backward data
-// of 3x3 128->128 at 8x56x56 292 -> 55.  A fp32 ResNet-50 batch of 8 7.5 -> 2.1 ms.  What bounds the small ones now is
-// the launch, the first trip to memory and, under filters larger than 1x1, the copy of the filter in front.
+// 1024 306 -> 21, its backward data 95 -> 14; 4096^3 2433 -> 1038 (132 TFLOP/s); 3x3 512->512 at 8x7x7 499 -> 28 with a
+// packed filter, 256->256 at 8x14x14 249 -> 27, at 32x14x14 250 -> 79 (94 TFLOP/s); stride-2 backward data of 3x3 128->128
+// at 8x56x56 292 -> 45.  A fp32 ResNet-50 batch of 8 7.5 -> 1.5 ms.  What bounds the small ones now is the launch, the first
+// trip to memory, and the last round of tiles.
 #include "stream_f32.hpp"
 
 #include <string.h>
@@ -27,9 +27,10 @@ namespace {
 
 // The lanes-side operand P: PTAP: addressed by tap and channel, the channel count a multiple of eight (also a matrix
 // with the lanes' index contiguous); PTAB: by a table of all reduction indices; PROW: reduction index contiguous.
-// The other operand Q: QROW: reduction index contiguous; QCOL: row index contiguous; QTAB: by the same table.
+// The other operand Q: QLANE: packed, 1 KB per step of 32 rows in the order of the lanes (stream_pack); QROW: reduction
+// index contiguous; QCOL: row index contiguous; QTAB: by the same table.
 enum { PTAP, PTAB, PROW };
-enum { QROW, QCOL, QTAB };
+enum { QROW, QCOL, QTAB, QLANE };
 
 constexpr int MAX_CLASSES = 16;
 constexpr int MAX_TABLE = 4096; // reduction indices of a table
@@ -144,7 +145,10 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
     for(int t = 0; t < TN; t++) {
         const int n = n0 + 32 * t + fr;
         nok[t] = n < g.N;
-        const long long o = QM == QROW ? c.q0 + (long long)n * (g.q_sn ? g.q_sn : kred) + 4 * fk : QM == QCOL ? c.q0 + n + 4 * fk * g.q_sc : n * g.q_sn;
+        const long long o = QM == QLANE  ? c.q0 + (long long)(n0 / 32 + t) * (kred / 8) * 256 + lane * 4
+                            : QM == QROW ? (long long)n * g.q_sn + 4 * fk
+                            : QM == QCOL ? n + 4 * fk * g.q_sc
+                                         : n * g.q_sn;
         qoff[t] = nok[t] ? (unsigned)(o * 4) : OOB;
     }
 
@@ -216,8 +220,8 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
 #pragma unroll
             for(int t = 0; t < TN; t++) {
                 const unsigned v = live ? qoff[t] : OOB;
-                if constexpr(QM == QROW) {
-                    qr[u][t] = load4(rq, v, (unsigned)(s_next * 32));
+                if constexpr(QM == QLANE || QM == QROW) {
+                    qr[u][t] = load4(rq, v, (unsigned)(s_next * (QM == QLANE ? 1024 : 32)));
                 } else {
 #pragma unroll
                     for(int j = 0; j < 4; j++)
@@ -385,20 +389,61 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
     }
 }
 
-// The filter in the order of the reduction, tap by tap: forward rows [n][tap][channel] for QROW, backward data
-// [class][tap][channel][n] for QCOL.  Consecutive lanes write consecutive elements and leave the gathering to the caches
-// (turning 64-channel pieces through LDS was 9 us slower on 512 -> 512 channels: too little in flight per block).
-__global__ void __launch_bounds__(256) stream_pack(Args g, const float *__restrict__ w, float *__restrict__ out, int cols)
+// The filter in the order that the kernel's lanes load it: [class][32 rows][step of eight][lane][4].  A 16-byte load whose
+// neighbouring lanes are rows of the filter apart takes the address unit four times as long as one of consecutive addresses
+// (73 and 16 cycles for a kilobyte), and that unit, not the matrix unit, bounded 32x32 tiles: 3x3 256->256 at 8x14x14 44 ->
+// 34 us, 512->512 at 8x7x7 51 -> 40, this copy included.
+__device__ __forceinline__ void pack_chunk(const SagaFilterPackJob &g, long long i)
 {
-    const Class &c = g.cls[blockIdx.y];
-    const int T = c.Tr * c.Ts;
-    const long long total = (long long)T * g.C * g.N;
-    for(long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256) {
-        const int inner = cols ? g.N : g.C, e = (int)(i % inner), o = (int)(i / inner);
-        const int n = cols ? e : o / T, tap = cols ? o / g.C : o - n * T, ch = cols ? o - tap * g.C : e;
-        const int a = tap / c.Ts, s = tap - a * c.Ts;
-        out[c.q0 + i] = w[n * g.q_sn + ch * g.q_sc + (c.r0 + a * g.rstep) * g.q_sr + (c.s0 + s * g.rstep) * g.q_ss];
+    const int S8 = g.C / 8, steps = g.T * S8;
+    const int lane = (int)(i & 63);
+    const long long q = i >> 6;
+    const int tile = (int)(q / steps), step = (int)(q - (long long)tile * steps);
+    const int n = tile * 32 + (lane & 31), tap = step / S8, ch = (step - tap * S8) * 8 + 4 * (lane >> 5);
+    const int a = tap / g.Ts, s = tap - a * g.Ts;
+    const float *src = (const float *)g.w + n * g.w_sn + ch * g.w_sc + (g.r0 + a * g.rstep) * g.w_sr + (g.s0 + s * g.rstep) * g.w_ss;
+    float4_t v = {0, 0, 0, 0};
+    if(n < g.N) {
+#pragma unroll
+        for(int j = 0; j < 4; j++)
+            v[j] = src[j * g.w_sc];
     }
+    *(float4_t *)((float *)g.packed + i * 4) = v;
+}
+
+constexpr int PACK_CHUNKS = 1024; // of 16 bytes, per block
+
+__global__ void __launch_bounds__(256) stream_pack(const SagaFilterPackJob *__restrict__ jobs, int njobs)
+{
+    int lo = 0, hi = njobs - 1;
+    while(lo < hi) {
+        const int mid = (lo + hi + 1) / 2;
+        if(jobs[mid].first_block <= (int)blockIdx.x)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    const SagaFilterPackJob g = jobs[lo];
+    const long long total = (long long)g.T * (g.C / 8) * 64 * ((g.N + 31) / 32);
+#pragma unroll
+    for(int k = 0; k < PACK_CHUNKS / 256; k++) {
+        const long long i = (long long)((int)blockIdx.x - g.first_block) * PACK_CHUNKS + k * 256 + threadIdx.x;
+        if(i < total)
+            pack_chunk(g, i);
+    }
+}
+
+// one call's filter, the jobs (one per class) as an argument
+struct PackArgs {
+    int n;
+    SagaFilterPackJob job[MAX_CLASSES];
+};
+__global__ void __launch_bounds__(256) stream_pack_call(PackArgs a)
+{
+    const SagaFilterPackJob &g = a.job[blockIdx.y];
+    const long long total = (long long)g.T * (g.C / 8) * 64 * ((g.N + 31) / 32);
+    for(long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256)
+        pack_chunk(g, i);
 }
 
 struct Config {
@@ -406,18 +451,34 @@ struct Config {
 };
 
 // Tile (32*tm x 32*tn per wavefront), wavefronts of a block along the reduction (ks) and along the pixels (wm) for
-// `pixels` x N results with `steps` reduction steps of eight.  Large tiles reuse what they load, small ones and splits
-// fill 1024 SIMDs: the limits are where the measured times cross (us, tm,tn,ks,wm; launches of 4 - 10 us included):
-//   3x3 256->256, 32x14x14   2,2,4,1  93   2,1,4,1 101   1,1,4,1 115   2,2,1,4 199
-//   3x3 256->256,  8x14x14   2,1,4,1  41   1,1,8,1  42   1,1,16,1 48   2,2,4,1  62
-//   3x3 512->512,  8x7x7     1,1,8,1  50   2,1,4,1  69   2,2,4,1 111
-//   1x1 1024->256, 8x14x14   1,1,4,1  18   2,1,4,1  20   1,1,1,4  33
-//   1x1 64->256,   8x56x56   2,1,1,4  22   1,1,1,4  23   1,1,4,1  37
-//   fc 64x3136 -> 1024       1,1,8,1  21   1,1,4,1  26   2,1,4,1  44   2,2,1,4 244
-Config choose(long long pixels, int N, long long steps)
+// `pixels` x N results with `steps` reduction steps of eight.  Splits fill 1024 SIMDs; the limits are where the measured
+// times cross (us, tm,tn,ks,wm; launches included).
+// Packed filters: the address unit has room, so the smallest tile balances best, four wavefronts to one tile (blocks of
+// one tile spread more evenly than blocks of four), unless the reduction is so short that writing the result dominates:
+//   3x3   64->64,  8x56x56   1,1,4,1  27.5   1,1,1,4  27.8   2,1,4,1  30.7   1,1,2,2  28.7
+//   3x3  256->256, 32x14x14  1,1,4,1  79.1   2,2,4,1  84.3   1,1,2,2  87.9
+//   3x3  256->256, 8x14x14   1,1,8,1  26.8   1,1,4,1  28.5   2,1,4,1  32.3
+//   3x3  512->512, 8x7x7     1,1,8,1  28.1   1,1,16,1 28.3   1,1,4,1  34.9
+//   1x1  256->64,  8x56x56   1,1,1,4  15.6   1,1,2,2  17.1   1,1,4,1  17.9   2,1,1,4  17.6
+//   1x1   64->256, 8x56x56   2,2,1,4  18.2   1,1,1,4  20.3
+//   3x3   64->64,  32x56x56  1,1,1,4  80.0   2,2,1,4  82.8
+// Filters and matrices read in place or through a table: large tiles reuse what they load.
+//   1x1 1024->256, 8x14x14   1,1,4,1  18     2,1,4,1  20     1,1,1,4  33
+//   1x1 64->256,   8x56x56   2,1,1,4  22     1,1,1,4  23     1,1,4,1  37
+//   fc 64x3136 -> 1024       1,1,8,1  21     1,1,4,1  26     2,1,4,1  44     2,2,1,4 244
+Config choose(bool packed, long long pixels, int N, long long steps)
 {
     auto tiles = [&](int tm, int tn) { return ((pixels + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
     const int tn = N > 32 ? 2 : 1;
+    const long long t = tiles(1, 1);
+    if(packed) {
+        if(t >= 3072 && steps <= 32)
+            return {2, tn, 1, 4};
+        int ks = t < 4096 && steps >= 64 ? 4 : 1;
+        while(ks < 16 && t * ks < (steps >= 64 ? 2048 : 1536) && steps >= 16 * ks)
+            ks *= 2;
+        return {1, 1, ks, ks >= 4 ? 1 : 4 / ks};
+    }
     if(tiles(2, tn) >= 2048)
         return {2, tn, 1, 4};
     if(tiles(2, tn) >= 384 && steps >= 128)
@@ -427,7 +488,7 @@ Config choose(long long pixels, int N, long long steps)
     if(tiles(2, 1) >= 1536)
         return {2, 1, 1, 4};
     int ks = 1;
-    while(ks < 16 && tiles(1, 1) * ks < 2048 && steps >= 16 * ks)
+    while(ks < 16 && t * ks < 2048 && steps >= 16 * ks)
         ks *= 2;
     return {1, 1, ks, ks >= 4 ? 1 : 4 / ks};
 }
@@ -456,7 +517,7 @@ template <int PM, int QM, bool EX, typename A> int launch_as(const A &k, const C
 
 template <int PM, int QM> int launch(Args &g, hipStream_t st, long long pixels, long long steps)
 {
-    const Config cf = choose(pixels, g.N, steps);
+    const Config cf = choose(QM == QLANE, pixels, g.N, steps);
     g.KS = cf.ks;
     g.nblk_q = (g.N + 32 * cf.tn - 1) / (32 * cf.tn);
     long long blocks = 0;
@@ -495,6 +556,9 @@ long long extent(const SagaTensorView *v)
 }
 
 int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }
+
+// packed size of a class with that many taps
+long long packed_floats(bool bwd, const ConvGeom &g, int taps) { return (long long)taps * (bwd ? g.K : g.C) * (((bwd ? g.C : g.K) + 31) / 32 * 32); }
 
 // the classes of a convolution and how its taps step; false if there are too many
 bool classes(bool bwd, const ConvGeom &g, Args &a)
@@ -536,30 +600,90 @@ bool classes(bool bwd, const ConvGeom &g, Args &a)
             return false;
         c.M = (int)M;
         c.q0 = at;
-        at += (long long)c.Tr * c.Ts * g.C * g.K;
+        at += packed_floats(bwd, g, c.Tr * c.Ts);
     }
     return true;
 }
 
-// the filter has to be copied into the order of the reduction
-bool packs(bool bwd, const ConvGeom &g) { return (bwd ? g.K : g.C) % 8 == 0 && !(g.R == 1 && g.S == 1 && g.stride == 1); }
+// the filter has to be packed: it cannot be read in place
+bool packs(bool bwd, const ConvGeom &g) { return (bwd ? g.K : g.C) % 8 == 0 && !(g.R == 1 && g.S == 1 && (!bwd || g.stride == 1)); }
+
+void describe(bool bwd, const SagaTensorView *w, Args &k)
+{
+    k.q_sn = bwd ? w->strides[1] : w->strides[0];
+    k.q_sc = bwd ? w->strides[0] : w->strides[1];
+    k.q_sr = w->strides[2];
+    k.q_ss = w->strides[3];
+}
+
+int pack_jobs(const Args &k, const void *w, float *packed, SagaFilterPackJob *jobs)
+{
+    int n = 0;
+    for(int i = 0; i < k.nclasses; i++) {
+        const Class &c = k.cls[i];
+        if(!c.Tr || !c.Ts)
+            continue;
+        SagaFilterPackJob &j = jobs[n++];
+        j.w = w;
+        j.packed = packed + c.q0;
+        j.w_sn = k.q_sn; j.w_sc = k.q_sc; j.w_sr = k.q_sr; j.w_ss = k.q_ss;
+        j.N = k.N;
+        j.C = k.C;
+        j.T = c.Tr * c.Ts;
+        j.Ts = c.Ts;
+        j.r0 = c.r0;
+        j.s0 = c.s0;
+        j.rstep = k.rstep;
+        j.first_block = 0;
+        j.blocks = (int)(((long long)j.T * (j.C / 8) * 64 * ((j.N + 31) / 32) + PACK_CHUNKS - 1) / PACK_CHUNKS);
+    }
+    return n;
+}
 
 } // namespace
 
-size_t stream_f32_conv_workspace(bool bwd, const ConvGeom &g)
+size_t stream_f32_packed_bytes(bool bwd, const ConvGeom &g)
 {
-    return packs(bwd, g) ? (size_t)g.K * g.C * g.R * g.S * sizeof(float) : 0;
+    Args k = {};
+    if((bwd ? g.K : g.C) % 8 || g.group != 1 || !classes(bwd, g, k))
+        return 0;
+    long long n = 0;
+    int taps = 0;
+    for(int i = 0; i < k.nclasses; i++) {
+        n += packed_floats(bwd, g, k.cls[i].Tr * k.cls[i].Ts);
+        taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
+    }
+    return taps <= 64 && n * 4 <= 0x7ffffe00ll ? (size_t)n * 4 : 0;
 }
 
+int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob *jobs)
+{
+    Args k = {};
+    if(!classes(bwd, g, k))
+        return 0;
+    k.N = bwd ? g.C : g.K;
+    k.C = bwd ? g.K : g.C;
+    describe(bwd, w, k);
+    return pack_jobs(k, w->ptr, (float *)packed, jobs);
+}
+
+int stream_f32_pack(const SagaFilterPackJob *jobs, int njobs, int blocks, hipStream_t st)
+{
+    stream_pack<<<blocks, 256, 0, st>>>(jobs, njobs);
+    SAGA_CHECK_LAUNCH();
+    return 0;
+}
+
+size_t stream_f32_conv_workspace(bool bwd, const ConvGeom &g) { return packs(bwd, g) ? stream_f32_packed_bytes(bwd, g) : 0; }
+
 int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g,
-                    float alpha, float beta, const StreamEpilogue &e, void *ws, size_t ws_bytes, hipStream_t st)
+                    float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st)
 {
     Args k = {};
     const long long pe = extent(a), qe = extent(w);
     const long long limit = 0x7ffffe00ll;
-    const long long wlen = (long long)g.K * g.C * g.R * g.S * 4;
     // (a pixel outside the image starts at an offset below the tensor; the sum with a valid tap's offset is inside again)
-    if(g.group != 1 || pe < 0 || qe < 0 || pe > limit || qe > limit || wlen > limit || !classes(bwd, g, k))
+    if(g.group != 1 || pe < 0 || qe < 0 || pe > limit || qe > limit || !classes(bwd, g, k))
         return SAGA_HIP_EUNSUPPORTED;
     k.p = (const float *)a->ptr;
     k.q = (const float *)w->ptr;
@@ -572,10 +696,7 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
     k.IW = a->dims[3];
     k.p_sn = a->strides[0]; k.p_sc = a->strides[1]; k.p_sh = a->strides[2]; k.p_sw = a->strides[3];
     k.o_sn = out->strides[0]; k.o_sc = out->strides[1]; k.o_sh = out->strides[2]; k.o_sw = out->strides[3];
-    k.q_sn = bwd ? w->strides[1] : w->strides[0];
-    k.q_sc = bwd ? w->strides[0] : w->strides[1];
-    k.q_sr = w->strides[2];
-    k.q_ss = w->strides[3];
+    describe(bwd, w, k);
     k.alpha = alpha;
     k.beta = beta;
     k.e = epilogue_f32(e);
@@ -585,16 +706,20 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
     for(int i = 0; i < k.nclasses; i++)
         taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
     if(k.C % 8 == 0 && taps <= 64) {
-        if(packs(bwd, g)) {
-            if(!ws || ws_bytes < (size_t)wlen || !aligned16(ws))
-                return SAGA_HIP_EWORKSPACE;
-            const dim3 grid(grid_for(wlen / 4 / k.nclasses, 256, 4096), k.nclasses);
-            stream_pack<<<grid, 256, 0, st>>>(k, k.q, (float *)ws, bwd);
-            k.q = (const float *)ws;
-            k.q_bytes = (unsigned)wlen;
-            k.q_sn = 0; // rows as long as the class's reduction
-            k.q_sc = k.N;
-            return bwd ? launch<PTAP, QCOL>(k, st, pixels, steps) : launch<PTAP, QROW>(k, st, pixels, steps);
+        const size_t bytes = packed || packs(bwd, g) ? stream_f32_packed_bytes(bwd, g) : 0;
+        if(bytes) {
+            if(!packed) {
+                if(!ws || ws_bytes < bytes || !aligned16(ws))
+                    return SAGA_HIP_EWORKSPACE;
+                PackArgs pa;
+                pa.n = pack_jobs(k, w->ptr, (float *)ws, pa.job);
+                const dim3 grid(grid_for((long long)bytes / 16 / k.nclasses, 256, 4096), pa.n);
+                stream_pack_call<<<grid, 256, 0, st>>>(pa);
+                packed = ws;
+            }
+            k.q = (const float *)packed;
+            k.q_bytes = (unsigned)bytes;
+            return launch<PTAP, QLANE>(k, st, pixels, steps);
         }
         // 1x1: the filter as it is, if its rows are dense
         if(!bwd && k.q_sc == 1)

@@ -52,9 +52,13 @@ inline EpilogueF32 epilogue_f32(const StreamEpilogue &e)
 
 // bytes of workspace for a convolution; 0 when it needs none
 size_t stream_f32_conv_workspace(bool bwd, const ConvGeom &g);
-// a: x or dy, out: y or dx.  SAGA_HIP_EUNSUPPORTED (nothing enqueued) outside what the kernel covers.
+// a: x or dy, out: y or dx; packed (may be null): what stream_f32_pack left, otherwise packed into ws where needed.  SAGA_HIP_EUNSUPPORTED (nothing enqueued) outside what the kernel covers.
 int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g,
-                    float alpha, float beta, const StreamEpilogue &e, void *ws, size_t ws_bytes, hipStream_t st);
+                    float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st);
+// the filter in the order that the kernel loads it: bytes (0: not for this convolution), jobs (at most 16), launch
+size_t stream_f32_packed_bytes(bool bwd, const ConvGeom &g);
+int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob *jobs);
+int stream_f32_pack(const SagaFilterPackJob *jobs, int njobs, int blocks, hipStream_t st);
 // row-major C[M][N] = alpha * op(A) * op(B) + beta * C, bias per column of C
 int stream_f32_gemm(int tA, int tB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb,
                     float beta, float *C, int ldc, const float *bias, int relu, hipStream_t st);

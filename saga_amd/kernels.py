@@ -29,6 +29,17 @@ class FilterTransposeJob(C.Structure):
                 ("first_block", C.c_int32)]
 
 
+class FilterPackJob(C.Structure):
+    _fields_ = [("w", C.c_void_p), ("packed", C.c_void_p), ("strides", C.c_int64 * 4), ("N", C.c_int32), ("C", C.c_int32),
+                ("T", C.c_int32), ("Ts", C.c_int32), ("r0", C.c_int32), ("s0", C.c_int32), ("rstep", C.c_int32),
+                ("first_block", C.c_int32), ("blocks", C.c_int32)]
+
+
+class ConvExtras(C.Structure):
+    _fields_ = [("packed", C.c_void_p), ("bias", C.POINTER(TensorView)), ("s", C.c_void_p), ("b", C.c_void_p), ("m", C.c_void_p),
+                ("v", C.c_void_p), ("eps", C.c_float), ("z", C.POINTER(TensorView)), ("relu", C.c_int32)]
+
+
 class BnBwdLink(C.Structure):
     _fields_ = [("x", C.POINTER(TensorView)), ("s", C.c_void_p), ("b", C.c_void_p), ("save_mean", C.c_void_p),
                 ("save_invstd", C.c_void_p), ("flags", C.c_int32), ("partial_rows", C.c_int32), ("partial", C.c_void_p),
@@ -49,7 +60,10 @@ SIGNATURES = {
     "saga_hip_init": (_I, [_I, C.POINTER(C.c_int)]),
     "saga_hip_conv2d_workspace_size": (_SZ, [_I, _TV, _TV, _TV, C.POINTER(ConvParams)]),
     "saga_hip_conv2d_fwd": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), _F, _F, _VP, _SZ, _VP]),
-    "saga_hip_conv2d_fwd_bias": (_I, [_TV, _TV, _TV, _TV, C.POINTER(ConvParams), _F, _I, _VP, _SZ, _VP]),
+    "saga_hip_conv2d_fwd_ex": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), _F, C.POINTER(ConvExtras), _VP, _SZ, _VP]),
+    "saga_hip_conv2d_pack_bytes": (_SZ, [_I, _TV, _TV, _TV, C.POINTER(ConvParams)]),
+    "saga_hip_conv2d_pack_jobs": (_I, [_I, _TV, _TV, _TV, C.POINTER(ConvParams), _VP, C.POINTER(FilterPackJob)]),
+    "saga_hip_filter_pack_batched": (_I, [_VP, _I, _I, _VP]),
     "saga_hip_conv2d_bwd_data_bias": (_I, [_TV, _TV, _VP, _TV, _TV, C.POINTER(ConvParams), _F, _VP, _SZ, _VP]),
     "saga_hip_conv2d_fwd_bnstats_size": (_SZ, [_TV, _TV, _TV, C.POINTER(ConvParams)]),
     "saga_hip_conv2d_fwd_bnstats": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), _F, _VP, _SZ, _VP, _SZ,

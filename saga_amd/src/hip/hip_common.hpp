@@ -95,6 +95,8 @@ public:
     const int m_id;
     std::shared_ptr<HipMemory> m_memory;
     void *m_data = nullptr;
+    // counts what may have changed the contents: host writes, and the steps of programs whose operations write it
+    std::atomic<uint64_t> m_version{1};
     bool m_in_arena = false; // m_data points into the context's arena (contents do not survive a step)
     bool m_nonfinite_is_valid = false;
 };
@@ -191,6 +193,8 @@ struct HipOperation {
     virtual bool killOutput(const std::shared_ptr<HipStorage> &s) { return false; }
     // inference: write relu(output) to y instead of the output; false if the operation cannot
     virtual bool foldRelu(const std::shared_ptr<HipTensor> &y) { return false; }
+    // do without an optional input
+    virtual void forget(const std::shared_ptr<HipTensor> &t) {}
     virtual std::string info() const { return ""; }
     // algorithmic work of one execution: floating point operations (matrix ops) and bytes that
     // must cross HBM (memory-bound ops); used for roofline accounting only
@@ -218,6 +222,7 @@ struct HipProgram;
 void link_bn_backward(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 // hip_ops.cpp: a strided 1x1 backward data that writes a fan-in gradient first is moved behind the last writer
 void reorder_sparse_first_writers(std::vector<std::shared_ptr<HipOperation>> &ops);
+void drop_small_packs(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 void fuse_bn_pooling(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 
 struct HipProgramUnit {
@@ -405,8 +410,10 @@ public:
     hipStream_t stream() const { return m_on_side ? m_ctx->m_side_stream : m_ctx->m_stream; }
     HipScratch &workspace() const { return m_on_side ? m_ctx->m_side_workspace : m_ctx->m_workspace; }
 
-    // the operation that transposes the filters of all backward-data convolutions in one launch (hip_ops.cpp)
-    std::shared_ptr<HipOperation> m_transpose_batch;
+    // the operations that transpose the filters of all fp16 backward-data convolutions, and pack those of the fp32
+    // convolutions of the forward and of the backward pass, in one launch each (hip_ops.cpp)
+    std::shared_ptr<HipOperation> m_transpose_batch, m_pack_batch[2];
+    std::vector<HipStorage *> m_written; // by m_ops
 
     SagaAux *m_aux = nullptr; // pinned host memory the optimizer kernels write their flags to
     float m_mp_scaling = 1.0f;

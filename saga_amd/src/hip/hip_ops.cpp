@@ -42,6 +42,173 @@ struct ConvStatsLink {
     bool valid = false; // set by every ConvFwd::exec, consumed by the BnTrain::exec that follows
 };
 
+// A copy of filters in another layout, all of a program's in one launch: made again when one of the filters may have
+// changed (HipStorage::m_version), so in training once per step and in inference once.  The copies have memory of their own.
+struct FilterCopies : public HipOperation {
+    struct Item {
+        T w, copy;
+    };
+    std::vector<Item> items_;
+    std::unique_ptr<HipMemory> jobs_dev_;
+    uint64_t epoch_ = ~(uint64_t)0;
+    int jobs_ = 0, total_blocks_ = 0;
+    bool dirty_ = true;
+    std::vector<uint64_t> versions_;
+    FilterCopies(const char *name) : HipOperation(name) {}
+    virtual std::vector<char> table() = 0; // the jobs, with jobs_ and total_blocks_
+    virtual int launch(HipProgram &p) = 0;
+    void exec(HipProgram &p) override
+    {
+        if(items_.empty())
+            return;
+        if(dirty_ || epoch_ != p.m_ctx->m_mem_epoch) { // a storage moved: the job table holds addresses
+            const std::vector<char> t = table();
+            if(!jobs_dev_ || jobs_dev_->m_bytes < t.size())
+                jobs_dev_ = std::make_unique<HipMemory>(t.size());
+            // synchronous copy of a few kilobytes, only when the table changed
+            chkHip(hipStreamSynchronize(p.stream()));
+            chkHip(hipMemcpy(jobs_dev_->m_ptr, t.data(), t.size(), hipMemcpyHostToDevice));
+            epoch_ = p.m_ctx->m_mem_epoch;
+            dirty_ = false;
+            versions_.clear();
+        }
+        bool changed = versions_.size() != items_.size();
+        versions_.resize(items_.size());
+        for(size_t i = 0; i < items_.size(); i++) {
+            const uint64_t v = items_[i].w->m_storage->m_version;
+            changed |= versions_[i] != v;
+            versions_[i] = v;
+        }
+        if(changed)
+            chkSaga(launch(p));
+    }
+    bool sideSafe() const override { return true; }
+    HipOpArgs listInputs() const override
+    {
+        HipOpArgs r;
+        for(auto &it : items_)
+            r.push_back({"w", it.w});
+        return r;
+    }
+    HipOpArgs listOutputs() const override
+    {
+        HipOpArgs r;
+        for(auto &it : items_)
+            r.push_back({"copy", it.copy});
+        return r;
+    }
+    bool killOutput(const std::shared_ptr<HipStorage> &s) override
+    {
+        for(size_t i = 0; i < items_.size(); i++)
+            if(items_[i].copy->m_storage == s) {
+                items_.erase(items_.begin() + i);
+                dropped(i);
+                dirty_ = true;
+                return true;
+            }
+        return false;
+    }
+    virtual void dropped(size_t) {}
+    // the table upload synchronises, and whether there is a launch is decided per step: not for recorded graphs
+    bool graphSafe() const override { return false; }
+    double bytes() const override
+    {
+        double b = 0;
+        for(auto &it : items_)
+            b += 2.0 * nbytes(it.w);
+        return b;
+    }
+};
+
+// The fp16 channels-last backward-data kernel reads the filter as C,R,S,K.  Instead of one small transpose
+// launch per layer and step, every backward-data operation of a program registers its filter here, and this
+// one operation - placed in the forward list, i.e. after the previous step's optimizer and before any
+// backward operation - transposes them all in a single launch into per-layer tensors.
+struct FilterTransposeBatch : public FilterCopies {
+    FilterTransposeBatch() : FilterCopies("filtertranspose") {}
+    void add(T w, T wt) { items_.push_back({w, wt}); }
+    std::vector<char> table() override
+    {
+        std::vector<char> t(items_.size() * sizeof(SagaFilterTransposeJob));
+        auto *j = (SagaFilterTransposeJob *)t.data();
+        total_blocks_ = 0;
+        jobs_ = (int)items_.size();
+        for(auto &it : items_) {
+            const SagaTensorView vw = it.w->view();
+            j->w = it.w->deviceMem();
+            j->wt = it.copy->deviceMem();
+            j->K = vw.dims[0];
+            j->C = vw.dims[1];
+            j->RS = vw.dims[2] * vw.dims[3];
+            j->first_block = total_blocks_;
+            total_blocks_ += saga_hip_filter_transpose_blocks(&vw);
+            j++;
+        }
+        return t;
+    }
+    int launch(HipProgram &p) override
+    {
+        return saga_hip_filter_transpose_batched((const SagaFilterTransposeJob *)jobs_dev_->m_ptr, jobs_, total_blocks_, S(p));
+    }
+};
+
+// The same for the fp32 kernels, forward and backward data, which load a packed filter (saga_hip_conv2d_pack_bytes).
+struct FilterPackBatch : public FilterCopies {
+    struct Shape {
+        int kind;
+        T x, y;
+        SagaConvParams cp;
+    };
+    std::vector<Shape> shapes_;
+    FilterPackBatch() : FilterCopies("filterpack") {}
+    void dropped(size_t i) override { shapes_.erase(shapes_.begin() + i); }
+    // (the first layers of a forward pass are soon waiting for theirs)
+    bool sideSafe() const override { return shapes_.size() && shapes_[0].kind == SAGA_CONV_BWD_DATA; }
+    std::vector<char> table() override
+    {
+        std::vector<SagaFilterPackJob> jobs(items_.size() * SAGA_CONV_PACK_JOBS);
+        jobs_ = total_blocks_ = 0;
+        for(size_t i = 0; i < items_.size(); i++) {
+            const SagaTensorView vx = shapes_[i].x->shapeView(), vw = items_[i].w->view(), vy = shapes_[i].y->shapeView();
+            const int n = saga_hip_conv2d_pack_jobs(shapes_[i].kind, &vx, &vw, &vy, &shapes_[i].cp, items_[i].copy->deviceMem(),
+                                                    jobs.data() + jobs_);
+            for(int k = 0; k < n; k++, jobs_++) {
+                jobs[jobs_].first_block = total_blocks_;
+                total_blocks_ += jobs[jobs_].blocks;
+            }
+        }
+        const char *p = (const char *)jobs.data();
+        return std::vector<char>(p, p + jobs_ * sizeof(SagaFilterPackJob));
+    }
+    int launch(HipProgram &p) override
+    {
+        return saga_hip_filter_pack_batched((const SagaFilterPackJob *)jobs_dev_->m_ptr, jobs_, total_blocks_, S(p));
+    }
+    // the packed filter of a convolution, or null where none is read
+    static T request(HipProgram &p, HipProgramUnit &pu, int kind, const T &x, const T &w, const T &y, const SagaConvParams &cp)
+    {
+        // (a 1x1 filter can be read in place: copying it in every training step costs what it saves)
+        if(p.m_pt == ProgramType::TRAINING && (int)w->m_dims[2] * (int)w->m_dims[3] == 1)
+            return nullptr;
+        const SagaTensorView vx = x->shapeView(), vw = w->shapeView(), vy = y->shapeView();
+        const size_t bytes = saga_hip_conv2d_pack_bytes(kind, &vx, &vw, &vy, &cp);
+        if(!bytes)
+            return nullptr;
+        auto t = std::make_shared<HipTensor>(Tensor::DataType::FLOAT, Dims{(int64_t)(bytes / 4)}, HipLayout::NCHW, p.m_ctx.get(),
+                                             w->namePostfix("packed"));
+        t->deviceMem(); // not a slot of the arena: it outlives the step
+        auto &batch = p.m_pack_batch[kind == SAGA_CONV_BWD_DATA];
+        if(!batch) {
+            batch = std::make_shared<FilterPackBatch>();
+            pu.fwd(batch);
+        }
+        auto *b = static_cast<FilterPackBatch *>(batch.get());
+        b->items_.push_back({w, t});
+        b->shapes_.push_back({kind, x, y, cp});
+        return t;
+    }
+};
+
 struct ConvFwd : public HipOperation {
     const T x_, w_, y_;
     const SagaConvParams cp_;
@@ -55,8 +222,15 @@ struct ConvFwd : public HipOperation {
     // the layer's bias, and (inference) the tensor of a relu behind it
     const T b_;
     T relu_y_;
-    ConvFwd(HipProgram &p, T x, T w, T y, SagaConvParams cp, T b = nullptr)
-      : HipOperation("convfwd"), x_(x), w_(w), y_(y), cp_(cp), b_(b)
+    T packed_; // the fp32 filter as the kernel loads it
+    ConvFwd(HipProgram &p, HipProgramUnit &pu, T x, T w, T y, SagaConvParams cp, T b = nullptr)
+      : HipOperation("convfwd")
+      , x_(x)
+      , w_(w)
+      , y_(y)
+      , cp_(cp)
+      , b_(b)
+      , packed_(FilterPackBatch::request(p, pu, SAGA_CONV_FWD, x, w, y, cp))
     {
         const SagaTensorView vx = x->shapeView(), vw = w->shapeView(), vy = y->shapeView();
         p.m_ctx->m_workspace.request(saga_hip_conv2d_workspace_size(SAGA_CONV_FWD, &vx, &vw, &vy, &cp_));
@@ -102,8 +276,9 @@ struct ConvFwd : public HipOperation {
             vz = bn_z_->view();
         const float *s = (const float *)bn_s_->deviceMem(), *b = (const float *)bn_b_->deviceMem();
         const float *m = (const float *)bn_m_->deviceMem(), *v = (const float *)bn_v_->deviceMem();
-        const int r = saga_hip_conv2d_fwd_bn_infer(&vx, &vw, &vo, bn_z_ ? &vz : nullptr, &cp_, s, b, m, v, bn_eps_, bn_flags_,
-                                                   p.workspace().ptr(), p.workspace().size(), S(p));
+        const SagaConvExtras e = {packed_ ? packed_->deviceMem() : nullptr, nullptr, s, b, m, v, bn_eps_,
+                                  bn_flags_ & SAGA_BN_ADD ? &vz : nullptr, bn_flags_ & SAGA_BN_RELU ? 1 : 0};
+        const int r = saga_hip_conv2d_fwd_ex(&vx, &vw, &vo, &cp_, 0.0f, &e, p.workspace().ptr(), p.workspace().size(), S(p));
         if(r == 0)
             return;
         if(r != SAGA_HIP_EUNSUPPORTED)
@@ -119,10 +294,13 @@ struct ConvFwd : public HipOperation {
         if(bn_y_)
             return execFolded(p);
         const SagaTensorView vx = x_->view(), vw = w_->view(), vy = relu_y_ ? relu_y_->view() : y_->view();
-        if(b_) {
-            const SagaTensorView vb = b_->view();
-            chkSaga(saga_hip_conv2d_fwd_bias(&vx, &vw, &vb, &vy, &cp_, beta_, relu_y_ ? 1 : 0, p.workspace().ptr(),
-                                             p.workspace().size(), S(p)));
+        if(b_ || packed_) {
+            SagaTensorView vb;
+            if(b_)
+                vb = b_->view();
+            const SagaConvExtras e = {packed_ ? packed_->deviceMem() : nullptr, b_ ? &vb : nullptr, nullptr, nullptr, nullptr,
+                                      nullptr, 0.0f, nullptr, relu_y_ ? 1 : 0};
+            chkSaga(saga_hip_conv2d_fwd_ex(&vx, &vw, &vy, &cp_, beta_, &e, p.workspace().ptr(), p.workspace().size(), S(p)));
             return;
         }
         if(stats_) {
@@ -147,12 +325,19 @@ struct ConvFwd : public HipOperation {
         HipOpArgs r{{"x", x_}, {"w", w_}};
         if(b_)
             r.push_back({"b", b_});
+        if(packed_)
+            r.push_back({"packed", packed_});
         if(bn_y_) {
             r.insert(r.end(), {{"s", bn_s_}, {"b", bn_b_}, {"m", bn_m_}, {"v", bn_v_}});
             if(bn_z_)
                 r.push_back({"z", bn_z_});
         }
         return r;
+    }
+    void forget(const T &t) override
+    {
+        if(packed_ == t)
+            packed_ = nullptr;
     }
     HipOpArgs listOutputs() const override { return {{"y", bn_y_ ? bn_y_ : relu_y_ ? relu_y_ : y_}}; }
     float *getBeta(const T &t) override { return !bn_y_ && !relu_y_ && t == y_ ? &beta_ : nullptr; }
@@ -163,92 +348,27 @@ struct ConvFwd : public HipOperation {
     }
 };
 
-// The fp16 channels-last backward-data kernel reads the filter as C,R,S,K.  Instead of one small transpose
-// launch per layer and step, every backward-data operation of a program registers its filter here, and this
-// one operation - placed in the forward list, i.e. after the previous step's optimizer and before any
-// backward operation - transposes them all in a single launch into per-layer tensors.
-struct FilterTransposeBatch : public HipOperation {
-    struct Item {
-        T w, wt;
-    };
-    std::vector<Item> items_;
-    std::unique_ptr<HipMemory> jobs_dev_;
-    std::vector<SagaFilterTransposeJob> jobs_;
-    uint64_t epoch_ = ~(uint64_t)0;
-    int total_blocks_ = 0;
-    bool dirty_ = true;
-    FilterTransposeBatch() : HipOperation("filtertranspose") {}
-    void add(T w, T wt)
-    {
-        items_.push_back({w, wt});
-        dirty_ = true;
+} // namespace
+
+// In training every step packs: a launch for fewer than four filters costs more than the convolutions' own copies in
+// front of their products (LeNet, one filter each way: 379 against 389 us per step).
+void drop_small_packs(HipProgram &p, HipOps &ops)
+{
+    if(p.m_pt != ProgramType::TRAINING)
+        return;
+    for(auto &batch : p.m_pack_batch) {
+        auto *b = static_cast<FilterPackBatch *>(batch.get());
+        if(!b || b->items_.size() >= 4)
+            continue;
+        for(auto &op : ops)
+            for(const auto &it : b->items_)
+                op->forget(it.copy);
+        ops.erase(std::find(ops.begin(), ops.end(), batch));
+        batch.reset();
     }
-    void exec(HipProgram &p) override
-    {
-        if(items_.empty())
-            return;
-        if(dirty_ || epoch_ != p.m_ctx->m_mem_epoch) { // a storage moved: the job table holds addresses
-            jobs_.clear();
-            total_blocks_ = 0;
-            for(auto &it : items_) {
-                const SagaTensorView vw = it.w->view();
-                SagaFilterTransposeJob j;
-                j.w = it.w->deviceMem();
-                j.wt = it.wt->deviceMem();
-                j.K = vw.dims[0];
-                j.C = vw.dims[1];
-                j.RS = vw.dims[2] * vw.dims[3];
-                j.first_block = total_blocks_;
-                total_blocks_ += saga_hip_filter_transpose_blocks(&vw);
-                jobs_.push_back(j);
-            }
-            const size_t bytes = jobs_.size() * sizeof(SagaFilterTransposeJob);
-            if(!jobs_dev_ || jobs_dev_->m_bytes < bytes)
-                jobs_dev_ = std::make_unique<HipMemory>(bytes);
-            // synchronous copy of a few kilobytes, only when the table changed; jobs_ stays valid meanwhile
-            chkHip(hipStreamSynchronize(p.stream()));
-            chkHip(hipMemcpy(jobs_dev_->m_ptr, jobs_.data(), bytes, hipMemcpyHostToDevice));
-            epoch_ = p.m_ctx->m_mem_epoch;
-            dirty_ = false;
-        }
-        chkSaga(saga_hip_filter_transpose_batched((const SagaFilterTransposeJob *)jobs_dev_->m_ptr, (int)jobs_.size(),
-                                                  total_blocks_, S(p)));
-    }
-    bool sideSafe() const override { return true; }
-    HipOpArgs listInputs() const override
-    {
-        HipOpArgs r;
-        for(auto &it : items_)
-            r.push_back({"w", it.w});
-        return r;
-    }
-    HipOpArgs listOutputs() const override
-    {
-        HipOpArgs r;
-        for(auto &it : items_)
-            r.push_back({"wt", it.wt});
-        return r;
-    }
-    bool killOutput(const std::shared_ptr<HipStorage> &s) override
-    {
-        for(size_t i = 0; i < items_.size(); i++)
-            if(items_[i].wt->m_storage == s) {
-                items_.erase(items_.begin() + i);
-                dirty_ = true;
-                return true;
-            }
-        return false;
-    }
-    // the table upload synchronises; keep the operation out of recorded graphs
-    bool graphSafe() const override { return false; }
-    double bytes() const override
-    {
-        double b = 0;
-        for(auto &it : items_)
-            b += 2.0 * nbytes(it.w);
-        return b;
-    }
-};
+}
+
+namespace {
 
 // Per-channel sums of a relu-masked gradient, handed from the ConvBwdData that is the last writer of a
 // batch norm's output gradient to that norm's BnBwd, which then skips its own first pass over the tensor.
@@ -263,7 +383,7 @@ struct BnBwdLinkState {
 
 struct ConvBwdData : public HipOperation {
     const T w_, dy_, dx_;
-    T wt_; // the filter as C,R,S,K, written by the program's FilterTransposeBatch (null: transposed per call)
+    T wt_; // the filter as C,R,S,K (fp16) or packed (fp32), written by the program's batch (null: per call)
     const SagaConvParams cp_;
     float beta_ = 0;
     // dx is the gradient of a batch norm's (+ relu) output and this is its last writer: the epilogue masks it
@@ -300,9 +420,12 @@ struct ConvBwdData : public HipOperation {
         const SagaTensorView vx = dx->shapeView(), vw = w->shapeView(), vy = dy->shapeView();
         p.m_ctx->m_workspace.request(saga_hip_conv2d_workspace_size(SAGA_CONV_BWD_DATA, &vx, &vw, &vy, &cp_));
         const size_t wt_bytes = saga_hip_conv2d_bwd_data_wt_bytes(&vy, &vw, &vx, &cp_);
-        if(wt_bytes && !getenv("SAGA_HIP_NO_BATCHED_TRANSPOSE")) {
+        wt_ = FilterPackBatch::request(p, pu, SAGA_CONV_BWD_DATA, dx, w, dy, cp);
+        if(wt_bytes && !wt_ && !getenv("SAGA_HIP_NO_BATCHED_TRANSPOSE")) {
             wt_ = std::make_shared<HipTensor>(Tensor::DataType::HALF, Dims{(int64_t)(wt_bytes / 2)}, HipLayout::NCHW,
                                               p.m_ctx.get(), w->namePostfix("transposed"));
+            if(p.m_pt == ProgramType::INFERENCE)
+                wt_->deviceMem(); // transposed once: not a slot of the arena
             if(!p.m_transpose_batch) {
                 p.m_transpose_batch = std::make_shared<FilterTransposeBatch>();
                 pu.fwd(p.m_transpose_batch);
@@ -344,6 +467,11 @@ struct ConvBwdData : public HipOperation {
         }
         chkSaga(saga_hip_conv2d_bwd_data_wt(&vdy, &vw, wt_ ? wt_->deviceMem() : nullptr, &vdx, &cp_, 1.0f, beta_,
                                             p.workspace().ptr(), p.workspace().size(), S(p)));
+    }
+    void forget(const T &t) override
+    {
+        if(wt_ == t)
+            wt_ = nullptr;
     }
     HipOpArgs listInputs() const override
     {
@@ -443,7 +571,7 @@ void conv_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
     const T fused_b = p.m_pc.disable_op_fusing ? nullptr : b; // the bias goes along in the epilogue
 
     if(!transpose) {
-        pu.fwd(std::make_shared<ConvFwd>(p, x, w, y, cp, fused_b));
+        pu.fwd(std::make_shared<ConvFwd>(p, pu, x, w, y, cp, fused_b));
         if(b && !fused_b)
             pu.fwd(std::make_shared<BiasAdd>(b, y));
         if(!training)
@@ -476,7 +604,7 @@ void conv_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
         pu.bwd(std::make_shared<ConvBwdFilter>(p, dy, x, dw, cp));
         p.upd(n.m_inputs["w"], w, dw);
         if(auto dx = p.lowerGrad(pu, n.m_inputs["x"]))
-            pu.bwd(std::make_shared<ConvFwd>(p, dy, w, dx, cp));
+            pu.bwd(std::make_shared<ConvFwd>(p, pu, dy, w, dx, cp));
     }
 }
 REGISTER_HIP_OP("conv", conv_setup);

@@ -613,6 +613,7 @@ void HipProgram::finalize()
     // are added inside the convolution / GEMM epilogue (reference: src/cuda/cuda_program.cpp:429-453).
     // An accumulating writer reads its output, so the dead-op pass below keeps the first writer
     // whenever it keeps a later one.
+    drop_small_packs(*this, m_ops);
     if(m_pt == ProgramType::TRAINING)
         reorder_sparse_first_writers(m_ops);
     std::set<HipTensor *> written;
@@ -638,10 +639,14 @@ void HipProgram::finalize()
         fuse_bn_pooling(*this, m_ops);
     }
 
+    std::set<HipStorage *> outputs;
     for(auto &op : m_ops)
-        for(auto &o : op->getOutputs())
+        for(auto &o : op->getOutputs()) {
+            outputs.insert(o.second->m_storage.get());
             if(o.second->m_storage->doubleBuffered())
                 static_cast<HipDoubleBuffer *>(o.second->m_storage.get())->m_written_by_ops = true;
+        }
+    m_written.assign(outputs.begin(), outputs.end());
 
     m_ctx->m_workspace.alloc();
     planSide();
@@ -973,6 +978,8 @@ void HipProgram::planSide()
 void HipProgram::runOps(const HipOps &ops)
 {
     if(&ops == &m_ops) {
+        for(HipStorage *s : m_written)
+            s->m_version.fetch_add(1, std::memory_order_relaxed);
         if(graphsEnabled()) {
             runOpsGraphed();
             m_steps_run++;

@@ -257,6 +257,7 @@ public:
     {
         if(m_dirty) {
             chkHip(hipMemcpy(m_storage->deviceMem(), m_host, m_bytes, hipMemcpyHostToDevice));
+            m_storage->m_version++;
         }
         free(m_host);
     }
@@ -489,6 +490,7 @@ void HipTensor::writeHost(const void *src)
         hip_permute(ta->data(), m_strides, src, ss, ext, es);
         return;
     }
+    m_storage->m_version++;
     HipContext &ctx = *m_storage->m_ctx;
     hipStream_t st = ctx.m_stream;
     SagaTensorView dv = view(), hv = dv;
@@ -647,6 +649,7 @@ void HipTensor::copyFromHost(Tensor &src)
         }
     } else {
         chkHip(hipMemcpy(m_storage->deviceMem(), host, n * es, hipMemcpyHostToDevice));
+        m_storage->m_version++;
     }
 }
 

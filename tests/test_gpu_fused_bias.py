@@ -52,8 +52,9 @@ def test_convolution(name):
     yd = dev(np.full(want.shape, np.nan, np.float32), dtype, lay)
     vx, vw, vb, vy, p = K.view(xd), K.view(wd), K.view(bd.view(1, Kk, 1, 1)), K.view(yd), K.ConvParams(pad, stride, 1, 1)
     ws, n = workspace(K.CONV_FWD, vx, vw, vy, p)
-    K.check(K.lib().saga_hip_conv2d_fwd_bias(C.byref(vx), C.byref(vw), C.byref(vb), C.byref(vy), C.byref(p), 0.0, relu, K.ptr(ws), n,
-                                             K.stream_ptr()))
+    e = K.ConvExtras(bias=C.pointer(vb), relu=relu)
+    K.check(K.lib().saga_hip_conv2d_fwd_ex(C.byref(vx), C.byref(vw), C.byref(vy), C.byref(p), 0.0, C.byref(e), K.ptr(ws), n,
+                                           K.stream_ptr()))
     assert_close(host(yd), want, dtype, name, tol=2e-3 if dtype == HALF else None)
 
 

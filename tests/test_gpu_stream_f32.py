@@ -93,3 +93,40 @@ def test_folded_norm(shape, flags):
     K.check(L.saga_hip_conv2d_fwd_bn_infer(C.byref(vx), C.byref(vw), C.byref(vy), C.byref(vz) if flags & K.BN_ADD else None,
                                            C.byref(p), *(K.ptr(t) for t in prm), 1e-3, flags, K.ptr(ws), n, K.stream_ptr()))
     assert_close(host(yd), want, F32, "folded norm")
+
+
+@pytest.mark.parametrize("shape", CONVS + [(3, 64, 150, 161, 64, 1, 1, 0)])
+def test_packed_filter(shape):
+    """Forward and backward data from a filter that was packed beforehand: the same results as packing per call gives."""
+    N, Cc, H, W, Kk, R, stride, pad = shape
+    rng = np.random.default_rng(sum(shape))
+    x = rnd(rng, N, Cc, H, W, dtype=F32)
+    w = rnd(rng, Kk, Cc, R, R, dtype=F32, scale=(2.0 / (Cc * R * R)) ** 0.5)
+    y = ref.conv2d_fwd(x, w, pad, stride)
+    dy = rnd(rng, *y.shape, dtype=F32)
+    L, p, stream = K.lib(), K.ConvParams(pad, stride, 1, 1), K.stream_ptr()
+    xd, wd, dyd = dev(x, F32), dev(w, F32), dev(dy, F32)
+    for kind, want in ((K.CONV_FWD, y), (K.CONV_BWD_DATA, ref.conv2d_bwd_data(dy, w, x.shape, pad, stride))):
+        out = dev(np.full(want.shape, np.nan, np.float32), F32)
+        vx, vw, vy = (K.view(t) for t in ((xd, wd, out) if kind == K.CONV_FWD else (out, wd, dyd)))
+        args = (kind, C.byref(vx), C.byref(vw), C.byref(vy), C.byref(p))
+        n = L.saga_hip_conv2d_pack_bytes(*args)
+        assert (n > 0) == ((Cc if kind == K.CONV_FWD else Kk) % 8 == 0)
+        if not n:
+            continue
+        packed = torch.full((n // 4,), np.nan, device="cuda")
+        jobs = (K.FilterPackJob * 16)()
+        count = L.saga_hip_conv2d_pack_jobs(*args, K.ptr(packed), jobs)
+        blocks = 0
+        for j in jobs[:count]:
+            j.first_block = blocks
+            blocks += j.blocks
+        table = torch.frombuffer(bytearray(C.string_at(jobs, C.sizeof(K.FilterPackJob) * count)), dtype=torch.uint8).cuda()
+        K.check(L.saga_hip_filter_pack_batched(K.ptr(table), count, blocks, stream))
+        if kind == K.CONV_FWD:
+            e = K.ConvExtras(packed=packed.data_ptr())
+            K.check(L.saga_hip_conv2d_fwd_ex(C.byref(vx), C.byref(vw), C.byref(vy), C.byref(p), 0.0, C.byref(e), None, 0, stream))
+        else:
+            K.check(L.saga_hip_conv2d_bwd_data_wt(C.byref(vy), C.byref(vw), K.ptr(packed), C.byref(vx), C.byref(p), 1.0, 0.0, None, 0,
+                                                  stream))
+        assert_close(host(out), want, F32, "packed")
