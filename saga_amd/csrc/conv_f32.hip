@@ -809,7 +809,9 @@ static FilterSplit plan_filter_f32(const ConvGeom &g)
     p.tiles_c = (CRS + WBN - 1) / WBN;
     const int tiles = p.tiles_k * p.tiles_c;
     long long want = (2048 + tiles - 1) / tiles; // a few blocks per CU
-    const long long maxs = (M + 511) / 512;      // at least 512 pixels per split
+    // At least four slices per block: its chain of trips to memory is what the small ones wait for (at least 512 pixels: 5x5
+    // 1->32 at 64x28x28 37 us, this 19; 3x3 16->16 at 128x32x32 the same 63).
+    const long long maxs = (M + 127) / 128;
     if(want > maxs)
         want = maxs;
     if(want < 1)
@@ -829,8 +831,13 @@ static FilterSplit plan_filter_uniform(const ConvGeom &g)
     p.tiles_k = (g.K + UW_K - 1) / UW_K;
     p.tiles_c = (CRS + UW_C - 1) / UW_C;
     const int tiles = p.tiles_k * p.tiles_c;
-    long long want = (768 + tiles - 1) / tiles; // three blocks per CU
-    const long long maxs = (M + 1023) / 1024;   // at least 1024 pixels per split
+    // Three blocks per CU where each has enough to do, otherwise two, as every block's partial is written and added up; at
+    // least two slices per block (at least 1024 pixels, us: 5x5 32->64 at 64x14x14 60 and this 34, 3x3 64->64 at 8x56x56 55 and
+    // 36, 64->64 at 16x8x8 57 and 13, 1x1 1024->256 at 32x14x14 51 and 52).
+    long long want = 768 / tiles;
+    if(M < want * 512)
+        want = std::min(want, std::max(512ll / tiles, M / 512));
+    const long long maxs = (M + 127) / 128;
     if(want > maxs)
         want = maxs;
     if(want < 1)
