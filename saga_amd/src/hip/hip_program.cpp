@@ -197,6 +197,7 @@ void HipContext::reset()
     m_exported.clear();
     m_tensors.clear();
     m_deferred_copy.clear();
+    m_layout_scratch.reset();
     m_storage_id_gen = 0;
     m_program_index_gen = 0;
 }

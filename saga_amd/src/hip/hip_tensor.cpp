@@ -510,11 +510,12 @@ void HipTensor::writeHost(const void *src)
     }
     const size_t sample = bytes / dv.dims[0];
     const int per = (int)std::max<size_t>(1, std::min<size_t>(dv.dims[0], (16 << 20) / sample));
-    HipMemory scratch(per * sample, false);
+    std::lock_guard<std::mutex> lock(ctx.m_stage_mutex);
+    const auto scratch = ctx.layoutScratch(per * sample);
     for(int n = 0; n < dv.dims[0]; n += per) {
         SagaTensorView a = hv, b = dv;
         a.dims[0] = b.dims[0] = std::min(per, dv.dims[0] - n);
-        a.ptr = scratch.m_ptr;
+        a.ptr = scratch->m_ptr;
         b.ptr = (char *)dv.ptr + n * dv.strides[0] * (int64_t)es;
         chkHip(hipMemcpy(a.ptr, (const char *)src + n * sample, a.dims[0] * sample, hipMemcpyHostToDevice));
         chkSaga(saga_hip_copy(&a, &b, (saga_stream_t)st));
@@ -546,18 +547,19 @@ void HipTensor::readHost(void *dst)
         memcpy(dst, hv.ptr, bytes);
         return;
     }
-    ctx.sync();
     if(rowMajor()) {
+        ctx.sync();
         chkHip(hipMemcpy(dst, dv.ptr, bytes, hipMemcpyDeviceToHost));
         return;
     }
     const size_t sample = bytes / dv.dims[0];
     const int per = (int)std::max<size_t>(1, std::min<size_t>(dv.dims[0], (16 << 20) / sample));
-    HipMemory scratch(per * sample, false);
+    std::lock_guard<std::mutex> lock(ctx.m_stage_mutex);
+    const auto scratch = ctx.layoutScratch(per * sample);
     for(int n = 0; n < dv.dims[0]; n += per) {
         SagaTensorView a = hv, b = dv;
         a.dims[0] = b.dims[0] = std::min(per, dv.dims[0] - n);
-        a.ptr = scratch.m_ptr;
+        a.ptr = scratch->m_ptr;
         b.ptr = (char *)dv.ptr + n * dv.strides[0] * (int64_t)es;
         chkSaga(saga_hip_copy(&b, &a, (saga_stream_t)st));
         chkHip(hipStreamSynchronize(st));
