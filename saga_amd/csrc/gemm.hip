@@ -4,7 +4,8 @@
 //    wave), operands staged through LDS with the reduction index contiguous; an operand
 //    stored with the other index contiguous is transposed on its way into LDS; gemm_split_f16,
 //    32x32 tiles whose reduction is split over a block, for grids that leave compute units idle.
-//  * fp32: stream_f32_gemm (stream_f32.hip); gemm_mfma_f32, 64x64x16 LDS tiles on v_mfma_f32_32x32x2_f32, for reductions
+//  * fp32: gemm_split_f32, 16x16 or 32x32 tiles whose reduction is split over a block, for small grids; stream_f32_gemm
+//    (stream_f32.hip) for large ones; gemm_mfma_f32, 64x64x16 LDS tiles on v_mfma_f32_32x32x2_f32, for reductions
 //    of up to 16 and operands beyond 2 GB.
 #include "stream_f32.hpp"
 
@@ -332,6 +333,133 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
 
 } // namespace
 
+// fp32, the same plan: T x T tiles (v_mfma_f32_16x16x4 / 32x32x2), W wavefronts that split the reduction in slices of 32
+// steps (a cache line per row), DEPTH slices of each wavefront in flight.  Small grids are bound by the few compute units
+// that work, and the streaming kernel there by the address unit besides, since its lanes load from a row each: fc 64x3136 ->
+// 1024 ran in 64 blocks, 21 us; in 256 of 16x16 tiles it takes 11, fc 64x1024 -> 10 8 instead of 11 (4 if the weights' rows
+// run along the reduction).
+template <int T, int W, bool tA, bool tB, bool VEC>
+__global__ void __launch_bounds__(64 * W)
+    gemm_split_f32(int M, int N, int K, float alpha, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
+                   float beta, float *__restrict__ C, int ldc, ColumnBias cb)
+{
+    constexpr int KS = 32, LD = KS + 4, NL = T / 8, DEPTH = 2, NV = T * T / 64;
+    typedef float acc_t __attribute__((ext_vector_type(NV)));
+    __shared__ __attribute__((aligned(16))) float st[W][2][T][LD];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int m0 = blockIdx.y * T, n0 = blockIdx.x * T;
+    acc_t acc;
+#pragma unroll
+    for(int v = 0; v < NV; v++)
+        acc[v] = 0.0f;
+    constexpr int RL = T / 4, KL = 64 / RL; // lanes along the rows and steps per load, where the rows are contiguous
+    auto fetch = [&](float4_t(&d)[NL], const float *__restrict__ base, int ld, bool kcontig, int row0, int rows, int k0) {
+#pragma unroll
+        for(int j = 0; j < NL; j++) {
+            const int r = row0 + (kcontig ? (lane >> 3) + 8 * j : (lane % RL) * 4), k = k0 + (kcontig ? (lane & 7) * 4 : lane / RL + KL * j);
+            if constexpr(VEC) { // runs are either whole or outside: no branch around the load
+                const bool ok = r < rows && k < K;
+                d[j] = *(const float4_t *)(base + (ok ? kcontig ? (int64_t)r * ld + k : (int64_t)k * ld + r : 0));
+            } else {
+#pragma unroll
+                for(int e = 0; e < 4; e++) {
+                    const int re = kcontig ? r : r + e, ke = kcontig ? k + e : k;
+                    const bool ok = re < rows && ke < K;
+                    const float v = base[ok ? kcontig ? (int64_t)re * ld + ke : (int64_t)ke * ld + re : 0];
+                    d[j][e] = ok ? v : 0.0f;
+                }
+            }
+        }
+    };
+    // (steps beyond the reduction become zeros here, not where they are loaded: that would wait for the load)
+    auto put = [&](float(*d)[LD], float4_t(&v)[NL], bool kcontig, int k0) {
+#pragma unroll
+        for(int j = 0; j < NL; j++) {
+            if(k0 + (kcontig ? (lane & 7) * 4 : lane / RL + KL * j) >= K)
+                v[j] = float4_t{0, 0, 0, 0};
+            if(kcontig) {
+                *(float4_t *)&d[(lane >> 3) + 8 * j][(lane & 7) * 4] = v[j];
+            } else {
+#pragma unroll
+                for(int e = 0; e < 4; e++)
+                    d[(lane % RL) * 4 + e][lane / RL + KL * j] = v[j][e];
+            }
+        }
+    };
+    const int slices = (K + KS - 1) / KS;
+    const int fr = lane % T, fk = lane / T;
+    float4_t va[DEPTH][NL], vb[DEPTH][NL];
+    auto load = [&](int u, int s) {
+        if(s >= slices)
+            return;
+        fetch(va[u], A, lda, !tA, m0, M, s * KS);
+        fetch(vb[u], B, ldb, tB, n0, N, s * KS);
+    };
+#pragma unroll
+    for(int u = 0; u < DEPTH; u++)
+        load(u, wave + W * u);
+    for(int s0 = wave; s0 < slices; s0 += W * DEPTH) {
+#pragma unroll
+        for(int u = 0; u < DEPTH; u++) {
+            const int s = s0 + W * u;
+            if(s >= slices)
+                break;
+            put(st[wave][0], va[u], !tA, s * KS);
+            put(st[wave][1], vb[u], tB, s * KS);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            load(u, s + W * DEPTH);
+            constexpr int STEP = 4 * (64 / T); // steps that one 16-byte read per lane covers
+#pragma unroll
+            for(int kk = 0; kk < KS; kk += STEP) {
+                const float4_t fa = *(const float4_t *)&st[wave][0][fr][kk + 4 * fk];
+                const float4_t fb = *(const float4_t *)&st[wave][1][fr][kk + 4 * fk];
+#pragma unroll
+                for(int e = 0; e < 4; e++) {
+                    if constexpr(T == 32)
+                        acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fa[e], fb[e], acc, 0, 0, 0);
+                    else
+                        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(fa[e], fb[e], acc, 0, 0, 0);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+    __syncthreads();
+    float(*red)[T][T + 1] = (float(*)[T][T + 1]) & st[0][0][0][0];
+    static_assert(sizeof(st) >= W * T * (T + 1) * sizeof(float), "the tiles of the sum fit the staging area");
+#pragma unroll
+    for(int v = 0; v < NV; v++) // column lane % T; rows: eights of fours (32x32), fours (16x16)
+        red[wave][T == 32 ? (v >> 2) * 8 + fk * 4 + (v & 3) : fk * 4 + v][fr] = acc[v];
+    __syncthreads();
+    for(int e = tid; e < T * T; e += 64 * W) {
+        const int ml = e / T, nl = e % T, m = m0 + ml, n = n0 + nl;
+        float r = 0;
+#pragma unroll
+        for(int w = 0; w < W; w++)
+            r += red[w][ml][nl];
+        if(m < M && n < N) {
+            float *o = C + (int64_t)m * ldc + n;
+            r *= alpha;
+            *o = cb.apply(beta != 0.0f ? r + beta * *o : r, n);
+        }
+    }
+}
+
+template <int T, int W>
+static void launch_split_f32(bool tA, bool tB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
+                             float *C, int ldc, const ColumnBias &cb, hipStream_t st)
+{
+    // (a run of 4 that is only partly in range goes element by element)
+    const bool vec = lda % 4 == 0 && ldb % 4 == 0 && aligned16(A) && aligned16(B) && (tA ? M : K) % 4 == 0 && (tB ? K : N) % 4 == 0;
+    auto kern = tA ? tB ? vec ? gemm_split_f32<T, W, true, true, true> : gemm_split_f32<T, W, true, true, false>
+                        : vec ? gemm_split_f32<T, W, true, false, true> : gemm_split_f32<T, W, true, false, false>
+                   : tB ? vec ? gemm_split_f32<T, W, false, true, true> : gemm_split_f32<T, W, false, true, false>
+                        : vec ? gemm_split_f32<T, W, false, false, true> : gemm_split_f32<T, W, false, false, false>;
+    kern<<<dim3((N + T - 1) / T, (M + T - 1) / T), 64 * W, 0, st>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, cb);
+}
+
 static int gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B, int ldb,
                 float beta, void *C, int ldc, int dtype, const ColumnBias &cb, saga_stream_t stream)
 {
@@ -362,7 +490,20 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
         gemm_mfma_f16<<<grid, 256, 0, st>>>(transA, transB, M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
                                             ldb, beta, (half_t *)C, ldc, a_vec, b_vec, cb);
     } else if(dtype == SAGA_FLOAT) {
-        // (one slice of the LDS tiles holds such a reduction: 3.5 against 5.8 us on 31x17x9)
+        // (one slice of the LDS tiles holds such a reduction)
+        // Up to one 32x32 tile per compute unit the reduction is split over a block (us, stream / 16x16 tiles on 16 and on 4
+        // wavefronts / 32x32 on 8: 64x1024x3136 21 / 11 / 13 / 23, 64x10x1024 11 / 8 / 10 / 18, 64x3136x1024 13 / 12 / 10 / 9,
+        // 128x1000x2048 16 / 18 / 15 / 17, 512x512x512 8.1 / 9.4 / 7.4 / 6.6, 300x300x32 4.7 / 3.6 / 2.7 / 3.4; beyond it
+        // 512x1024x3136 43 / 69 / 57 / 46, 1024x1024x256 11 / 22 / 13 / 14).
+        const int64_t t32 = ((int64_t)(M + 31) / 32) * ((N + 31) / 32), t16 = ((int64_t)(M + 15) / 16) * ((N + 15) / 16);
+        if(t32 <= 256) {
+            auto go = t16 <= 256 && K > 128   ? launch_split_f32<16, 16>
+                      : t32 >= 192 && K > 64 ? launch_split_f32<32, 8>
+                                             : launch_split_f32<16, 4>;
+            go(transA, transB, M, N, K, alpha, (const float *)A, lda, (const float *)B, ldb, beta, (float *)C, ldc, cb, st);
+            SAGA_CHECK_LAUNCH();
+            return 0;
+        }
         if(K > 16) {
             const int r = stream_f32_gemm(transA, transB, M, N, K, alpha, (const float *)A, lda, (const float *)B, ldb, beta,
                                           (float *)C, ldc, cb.f, cb.relu, st);

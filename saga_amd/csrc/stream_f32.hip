@@ -13,8 +13,7 @@
 // Small problems fill the chip by splitting the reduction over the KS wavefronts of a block, which add up through LDS
 // at the end: one launch, no partial results in memory, a fixed order of additions.
 //
-// Measured against the LDS-tiled kernels that did all of this before (us; graph replays, launch included): fc 64x3136 ->
-// 1024 306 -> 21, its backward data 95 -> 14; 4096^3 2433 -> 1038 (132 TFLOP/s); 3x3 512->512 at 8x7x7 499 -> 28 with a
+// Measured against the LDS-tiled kernels that did all of this before (us; graph replays, launch included): 4096^3 2433 -> 1038 (132 TFLOP/s); 3x3 512->512 at 8x7x7 499 -> 28 with a
 // packed filter, 256->256 at 8x14x14 249 -> 27, at 32x14x14 250 -> 79 (94 TFLOP/s); stride-2 backward data of 3x3 128->128
 // at 8x56x56 292 -> 45.  A fp32 ResNet-50 batch of 8 7.5 -> 1.5 ms.  What bounds the small ones now is the launch, the first
 // trip to memory, and the last round of tiles.
@@ -465,7 +464,6 @@ struct Config {
 // Filters and matrices read in place or through a table: large tiles reuse what they load.
 //   1x1 1024->256, 8x14x14   1,1,4,1  18     2,1,4,1  20     1,1,1,4  33
 //   1x1 64->256,   8x56x56   2,1,1,4  22     1,1,1,4  23     1,1,4,1  37
-//   fc 64x3136 -> 1024       1,1,8,1  21     1,1,4,1  26     2,1,4,1  44     2,2,1,4 244
 Config choose(bool packed, long long pixels, int N, long long steps)
 {
     auto tiles = [&](int tm, int tn) { return ((pixels + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };

@@ -33,6 +33,20 @@ def test_gemm_split(M, N, Kd, tA, tB):
     assert_close(host(Cd), 0.5 * (A.astype(np.float64) @ B) + 1, HALF, "gemm", tol=1e-3)
 
 
+@pytest.mark.parametrize("tA", [0, 1])
+@pytest.mark.parametrize("tB", [0, 1])
+@pytest.mark.parametrize("M,N,Kd", [(1, 1, 1), (5, 3, 2), (16, 16, 32), (17, 33, 129), (64, 1024, 3136), (260, 250, 128), (250, 260, 131),
+                                    (500, 512, 65), (512, 512, 512), (31, 1030, 64)])
+def test_gemm_split_fp32(M, N, Kd, tA, tB):
+    rng = np.random.default_rng(M + Kd)
+    A, B = rnd(rng, M, Kd), rnd(rng, Kd, N)
+    Ad, Bd = dev(A.T if tA else A), dev(B.T if tB else B)
+    Cd = dev(np.ones((M, N), np.float32))
+    K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 0.5, K.ptr(Ad), Ad.shape[1], K.ptr(Bd), Bd.shape[1], 1.0, K.ptr(Cd), N,
+                                  K.FLOAT, S()))
+    assert_close(host(Cd), 0.5 * (A.astype(np.float64) @ B) + 1, F32, "gemm", tol=1e-5)
+
+
 @pytest.mark.parametrize("layout,padc,dtype", [("nhwc", 0, HALF), ("nhwc", 8, HALF), ("nchw", 0, F32), ("nhwc", 0, F32)])
 @pytest.mark.parametrize("k,pad,stride,H", [(4, 0, 4, 9), (7, 0, 7, 7), (8, 3, 2, 12), (15, 0, 1, 15), (16, 0, 1, 17), (31, 2, 3, 33),
                                             (90, 0, 1, 90)])
