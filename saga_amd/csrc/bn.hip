@@ -145,21 +145,174 @@ __device__ __forceinline__ RowRun row_run(int64_t rows, int rb, int ty, int cvb)
     return rr;
 }
 
+// Small tensors: the streaming pass finalizes the statistics itself.  A launch that does nothing but add partial sums costs
+// 3 - 5 us and the pause in front of the next; here every block adds the partials of its slab of up to 64 channels again,
+// while its first rows are on their way (us of finalizing and normalizing, before -> after: 64 channels of 128x8x8 from 32
+// partial rows 6.8 -> 4.7, 1024 of 23x13x13 from 16 11.0 -> 7.0).  The blocks of row 0 write what outlives the launch.  Where there are
+// thousands of partials or blocks, reading them again costs more than the launch (see self_finalizing).
+struct StatsFin {
+    const float *partial;
+    int prows;
+    const float *s, *b;
+    float *run_m, *run_v, *save_mean, *save_invstd;
+    double M;
+    float eps, expavg;
+};
+struct BwdFin {
+    const float *partial;
+    int prows;
+    const float *s, *save_invstd;
+    float *ds, *db;
+    double M;
+    float beta_p;
+};
+
+// totals of a slab of CS channels from cb on: valid for threads below CS
+__device__ __forceinline__ void slab_sums(const float *__restrict__ partial, int prows, int C, int cb, int CS, double &s0, double &s1)
+{
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    __shared__ double red[2][256];
+    const int tid = threadIdx.x, c = tid % CS, l = tid / CS, lanes = 256 / CS;
+    const float2_t *p = (const float2_t *)partial + (cb + c < C ? cb + c : 0);
+    double a0 = 0, a1 = 0;
+    for(int g = l; g < prows; g += 8 * lanes) {
+        float2_t v[8];
+#pragma unroll
+        for(int u = 0; u < 8; u++)
+            v[u] = p[(int64_t)(g + u * lanes < prows ? g + u * lanes : 0) * C];
+#pragma unroll
+        for(int u = 0; u < 8; u++)
+            if(g + u * lanes < prows) {
+                a0 += v[u][0];
+                a1 += v[u][1];
+            }
+    }
+    red[0][tid] = a0;
+    red[1][tid] = a1;
+    __syncthreads();
+    s0 = s1 = 0;
+    if(tid < CS)
+        for(int k = 0; k < lanes; k++) {
+            s0 += red[0][k * CS + tid];
+            s1 += red[1][k * CS + tid];
+        }
+}
+
+// mean, biased variance, 1/std and what follows from them, as bn_stats_finalize has it
+__device__ __forceinline__ void finish_stats(double s0, double s1, double k, double M, float eps, float expavg, float sv, float bv,
+                                             float rm_old, float rv_old, bool write, float *run_m, float *run_v, float *save_mean,
+                                             float *save_invstd, int c, float &scale, float &shift)
+{
+    const double dm = s0 / M;
+    double var = s1 / M - dm * dm;
+    if(var < 0)
+        var = 0;
+    const double mean = k + dm;
+    const float inv = (float)(1.0 / sqrt(var + (double)eps));
+    if(write) {
+        if(save_mean)
+            save_mean[c] = (float)mean;
+        if(save_invstd)
+            save_invstd[c] = inv;
+        if(run_m)
+            run_m[c] = (float)((1.0 - expavg) * rm_old + expavg * mean);
+        if(run_v) {
+            const double unb = M > 1 ? var * M / (M - 1.0) : var;
+            run_v[c] = (float)((1.0 - expavg) * rv_old + expavg * unb);
+        }
+    }
+    scale = sv * inv;
+    shift = __builtin_fmaf(-(float)mean, scale, bv); // same expression as the backward mask recompute
+}
+
+__device__ __forceinline__ void stats_slab(const StatsFin &f, int C, int cb, int CS, float (&tab)[2][64])
+{
+    const int tid = threadIdx.x, c = cb + tid;
+    const bool own = tid < CS && c < C, write = blockIdx.x == 0;
+    float sv = 0, bv = 0, rm = 0, rv = 0;
+    if(own) {
+        sv = f.s[c];
+        bv = f.b[c];
+        if(write && f.run_m)
+            rm = f.run_m[c];
+        if(write && f.run_v)
+            rv = f.run_v[c];
+    }
+    double s0, s1;
+    slab_sums(f.partial, f.prows, C, cb, CS, s0, s1);
+    if(own)
+        finish_stats(s0, s1, 0.0, f.M, f.eps, f.expavg, sv, bv, rm, rv, write, f.run_m, f.run_v, f.save_mean, f.save_invstd, c,
+                     tab[0][tid], tab[1][tid]);
+    __syncthreads();
+}
+
+__device__ __forceinline__ void bwd_slab(const BwdFin &f, int C, int cb, int CS, float (&tab)[3][64])
+{
+    const int tid = threadIdx.x, c = cb + tid;
+    const bool own = tid < CS && c < C, write = blockIdx.x == 0;
+    float sv = 0, inv = 0, ds_old = 0, db_old = 0;
+    if(own) {
+        sv = f.s[c];
+        inv = f.save_invstd[c];
+        if(write && f.beta_p != 0.0f) {
+            ds_old = f.ds[c];
+            db_old = f.db[c];
+        }
+    }
+    double s0, s1;
+    slab_sums(f.partial, f.prows, C, cb, CS, s0, s1);
+    if(own) {
+        const double dsv = s1 * inv;
+        if(write) {
+            f.ds[c] = (float)(f.beta_p != 0.0f ? dsv + (double)f.beta_p * ds_old : dsv);
+            f.db[c] = (float)(f.beta_p != 0.0f ? s0 + (double)f.beta_p * db_old : s0);
+        }
+        tab[0][tid] = (float)(sv * (double)inv);
+        tab[1][tid] = (float)(s0 / f.M);
+        tab[2][tid] = (float)(dsv * inv / f.M);
+    }
+    __syncthreads();
+}
+
+// Grid of a self-finalizing pass (blocks of four row groups, about a thousand at most), or false.  A thread adds at most 32
+// partials forward (128 rows of 64 channels, 512 of 16) and 16 backward, where its registers leave fewer wavefronts to hide
+// that (us, separate / own finalizing: forward 512 channels of 23x25x25 11.1 / 9.5;
+// linked backward of 1024 of 23x13x13 10.3 / 8.0, 512 of 23x25x25 13 / 15, 16 of 128x32x32 from 512
+// rows 7.0 / 8.5).
+static bool self_finalizing(int64_t rows, int C, int prows, bool backward, Shape *sh)
+{
+    const int cvec = C / 8;
+    int cvb = 1;
+    while(cvb < cvec && cvb < 8)
+        cvb <<= 1;
+    const int rb = 256 / cvb, lanes = 256 / (cvb * 8);
+    if(C % 8 || prows > (backward ? 16 : 32) * lanes)
+        return false;
+    sh->cvb = cvb;
+    sh->rb = rb;
+    sh->gy = (cvec + cvb - 1) / cvb;
+    const int64_t groups = (rows + rb - 1) / rb;
+    if(groups * sh->gy > (backward ? 2400 : 4096))
+        return false;
+    sh->gx = sh->gxa = (int)((groups + 3) / 4);
+    return true;
+}
+
 // y = x*scale[c] + shift[c] (+ z) (relu).  MODE 0: scale/shift from s,b,m,v (inference);
-// MODE 1: scale/shift precomputed in ss[0..C), ss[C..2C) (training, second pass).
+// MODE 1: scale/shift precomputed in ss[0..C), ss[C..2C) (training, second pass); MODE 2: from partial sums (StatsFin).
 template <typename T, int VN, int MODE>
 __global__ void __launch_bounds__(256)
     bn_apply_cl(const T *__restrict__ x, int64_t px, const T *__restrict__ z, int64_t pz, T *__restrict__ y, int64_t py,
                 const float *__restrict__ s, const float *__restrict__ b, const float *__restrict__ m,
                 const float *__restrict__ v, const float *__restrict__ ss, float eps, int64_t rows, int C, int cvb_,
-                int flags, uint8_t *__restrict__ mask = nullptr)
+                int flags, uint8_t *__restrict__ mask = nullptr, StatsFin fin = StatsFin())
 {
     // mask (VN == 8 only): one byte per row and 8-channel vector, bit j set where the stored y is > 0;
     // the backward pass of a fused add + relu layer reads it instead of y
     const int cvb = cvb_ < 0 ? -cvb_ : cvb_;
     const int tx = threadIdx.x % cvb, ty = threadIdx.x / cvb, rb = 256 / cvb;
     const int c0 = (blockIdx.y * cvb + tx) * VN;
-    if(c0 >= C)
+    if(MODE != 2 && c0 >= C)
         return;
     float sc[VN], sh[VN];
 #pragma unroll
@@ -167,7 +320,7 @@ __global__ void __launch_bounds__(256)
         if(MODE == 0) {
             sc[j] = s[c0 + j] * rsqrtf(v[c0 + j] + eps);
             sh[j] = b[c0 + j] - m[c0 + j] * sc[j];
-        } else {
+        } else if(MODE == 1) {
             sc[j] = ss[c0 + j];
             sh[j] = ss[C + c0 + j];
         }
@@ -175,12 +328,12 @@ __global__ void __launch_bounds__(256)
     const bool relu = flags & SAGA_BN_RELU, add = flags & SAGA_BN_ADD;
     typedef Ld<T, VN> L;
     typedef typename L::V V;
-    // MODE 1 runs right after the statistics pass over the same rows: walking them in the
+    // MODE 1 and 2 run right after the statistics pass over the same rows: walking them in the
     // opposite direction meets the rows that pass touched last, which are the ones most
     // likely to be still cached
     const RowRun rr = row_run(rows, rb, ty, cvb_);
     const int64_t stride = rr.stride;
-    auto row = [&](int64_t r) { return MODE == 1 ? rows - 1 - r : r; };
+    auto row = [&](int64_t r) { return MODE >= 1 ? rows - 1 - r : r; };
     auto finish = [&](const V &xr, const V &zr, int64_t r) {
         float o[VN];
 #pragma unroll
@@ -205,16 +358,39 @@ __global__ void __launch_bounds__(256)
     };
     int64_t r = rr.r0;
     const int64_t rend = rr.rend;
-    for(; r + 3 * stride < rend; r += 4 * stride) {
-        V xr[4], zr[4];
+    V xr[4], zr[4];
+    auto load4 = [&]() {
 #pragma unroll
         for(int u = 0; u < 4; u++) {
             xr[u] = L::raw(x + row(r + u * stride) * px + c0);
             zr[u] = add ? L::raw(z + row(r + u * stride) * pz + c0) : xr[u];
         }
+    };
+    auto finish4 = [&]() {
 #pragma unroll
         for(int u = 0; u < 4; u++)
             finish(xr[u], zr[u], row(r + u * stride));
+        r += 4 * stride;
+    };
+    if constexpr(MODE == 2) {
+        __shared__ float tab[2][64];
+        const bool ahead = c0 < C && r + 3 * stride < rend;
+        if(ahead)
+            load4();
+        stats_slab(fin, C, blockIdx.y * cvb * VN, cvb * VN, tab);
+        if(c0 >= C)
+            return;
+#pragma unroll
+        for(int j = 0; j < VN; j++) {
+            sc[j] = tab[0][tx * VN + j];
+            sh[j] = tab[1][tx * VN + j];
+        }
+        if(ahead)
+            finish4();
+    }
+    while(r + 3 * stride < rend) {
+        load4();
+        finish4();
     }
     for(; r < rend; r += stride) {
         const V xr = L::raw(x + row(r) * px + c0);
@@ -223,12 +399,71 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// The sums of a block's 256 / cvb row lanes, for its cvb channel vectors, into its row of partials.  All threads take part,
+// in a fixed order (one row of threads that walked the others' values took 4 us of the 10 that the backward statistics of
+// 16 channels need).  red: (256 + cvb) * 2 * VN floats; the pitch keeps the walks off each other's banks.
+template <int VN>
+__device__ __forceinline__ void block_partials(const float (&a0)[VN], const float (&a1)[VN], float *red, int tx, int cvb,
+                                               float *__restrict__ partial, int C)
+{
+    const int tid = threadIdx.x, pitch = 256 + cvb, rb = 256 / cvb, sums = cvb * 2 * VN;
+#pragma unroll
+    for(int j = 0; j < VN; j++) {
+        red[j * pitch + tid] = a0[j];
+        red[(VN + j) * pitch + tid] = a1[j];
+    }
+    __syncthreads();
+    const int parts = sums < 256 ? 256 / sums : 1; // threads per sum
+    const int len = (rb + parts - 1) / parts;
+    float *o = partial + ((int64_t)blockIdx.x * C + blockIdx.y * cvb * VN) * 2;
+    auto store = [&](int q, float v) {
+        const int k = q / cvb, c = (q % cvb) * VN + k % VN; // k: the value's number in its thread
+        if((int)blockIdx.y * cvb * VN + c < C)
+            o[c * 2 + k / VN] = v;
+    };
+    if(parts == 1) { // few rows: one of them adds the others
+        const int c0 = (blockIdx.y * cvb + tx) * VN;
+        if(tid >= cvb || c0 >= C)
+            return;
+        float t0[VN], t1[VN];
+#pragma unroll
+        for(int j = 0; j < VN; j++) {
+            t0[j] = a0[j];
+            t1[j] = a1[j];
+        }
+        for(int t = 1; t < rb; t++)
+#pragma unroll
+            for(int j = 0; j < VN; j++) {
+                t0[j] += red[j * pitch + t * cvb + tx];
+                t1[j] += red[(VN + j) * pitch + t * cvb + tx];
+            }
+#pragma unroll
+        for(int j = 0; j < VN; j++) {
+            o[(tx * VN + j) * 2] = t0[j];
+            o[(tx * VN + j) * 2 + 1] = t1[j];
+        }
+        return;
+    }
+    const int q = tid % sums, p = tid / sums;
+    float v = 0;
+    for(int t = p * len; t < (p + 1) * len && t < rb; t++)
+        v += red[(q / cvb) * pitch + t * cvb + q % cvb];
+    __syncthreads();
+    red[tid] = v;
+    __syncthreads();
+    if(tid < sums) {
+        for(int k = 1; k < parts; k++)
+            v += red[k * sums + tid];
+        store(tid, v);
+    }
+}
+
 // Pass 1 of training forward: per-block partial sums of (x-K) and (x-K)^2, K = x[row 0].
 template <typename T, int VN>
 __global__ void __launch_bounds__(256)
     bn_stats_cl(const T *__restrict__ x, int64_t px, float *__restrict__ partial, int64_t rows, int C, int cvb_)
 {
-    __shared__ float red[256 * VN * 2];
+    __shared__ float red[320 * VN * 2];
     const int cvb = cvb_ < 0 ? -cvb_ : cvb_;
     const int tx = threadIdx.x % cvb, ty = threadIdx.x / cvb, rb = 256 / cvb;
     const int c0 = (blockIdx.y * cvb + tx) * VN;
@@ -264,27 +499,7 @@ __global__ void __launch_bounds__(256)
         for(; r < rend; r += stride)
             add(L::raw(x + r * px + c0));
     }
-#pragma unroll
-    for(int j = 0; j < VN; j++) {
-        red[(ty * cvb + tx) * VN * 2 + j] = a0[j];
-        red[(ty * cvb + tx) * VN * 2 + VN + j] = a1[j];
-    }
-    __syncthreads();
-    if(ty == 0 && c0 < C) {
-        for(int t = 1; t < rb; t++) {
-#pragma unroll
-            for(int j = 0; j < VN; j++) {
-                a0[j] += red[(t * cvb + tx) * VN * 2 + j];
-                a1[j] += red[(t * cvb + tx) * VN * 2 + VN + j];
-            }
-        }
-        float *o = partial + ((int64_t)blockIdx.x * C + c0) * 2;
-#pragma unroll
-        for(int j = 0; j < VN; j++) {
-            o[j * 2] = a0[j];
-            o[j * 2 + 1] = a1[j];
-        }
-    }
+    block_partials<VN>(a0, a1, red, tx, cvb, partial, C);
 }
 
 __device__ __forceinline__ double wave_sum_f64(double v)
@@ -363,25 +578,7 @@ __global__ void __launch_bounds__(256)
     sum_partials(partial, gx, C, c, s0, s1);
     if(threadIdx.x != 0)
         return;
-    const double dm = s0 / M;
-    double var = s1 / M - dm * dm;
-    if(var < 0)
-        var = 0;
-    const double mean = k + dm;
-    const float inv = (float)(1.0 / sqrt(var + (double)eps));
-    if(save_mean)
-        save_mean[c] = (float)mean;
-    if(save_invstd)
-        save_invstd[c] = inv;
-    if(run_m)
-        run_m[c] = (float)((1.0 - expavg) * rm_old + expavg * mean);
-    if(run_v) {
-        const double unb = M > 1 ? var * M / (M - 1.0) : var;
-        run_v[c] = (float)((1.0 - expavg) * rv_old + expavg * unb);
-    }
-    const float sc = sv * inv;
-    ss[c] = sc;
-    ss[C + c] = __builtin_fmaf(-(float)mean, sc, bv); // same expression as the backward mask recompute
+    finish_stats(s0, s1, k, M, eps, expavg, sv, bv, rm_old, rv_old, true, run_m, run_v, save_mean, save_invstd, c, ss[c], ss[C + c]);
 }
 
 // Pass 1 of backward: partial sums of dy' and dy'*(x-mean); dy' = dy masked by y>0 when fused relu.
@@ -398,7 +595,7 @@ __global__ void __launch_bounds__(256)
     // gradient anyway), and the second pass reads it instead of y and dy
     // rs/rb_/rinv (scale, bias, saved 1/std) set: the relu mask is recomputed from x as
     // half(fma(x, sc, sh)) > 0, exactly what the forward stored, and y is not read
-    __shared__ float red[256 * VN * 2];
+    __shared__ float red[320 * VN * 2];
     const int cvb = cvb_ < 0 ? -cvb_ : cvb_;
     const int tx = threadIdx.x % cvb, ty = threadIdx.x / cvb, rb = 256 / cvb;
     const int c0 = (blockIdx.y * cvb + tx) * VN;
@@ -458,27 +655,7 @@ __global__ void __launch_bounds__(256)
             add(xr, gr, relu && !recompute && !mask ? L::raw(y + r * py + c0) : gr, mask ? mask[r * mp + mc] : 0u, r);
         }
     }
-#pragma unroll
-    for(int j = 0; j < VN; j++) {
-        red[(ty * cvb + tx) * VN * 2 + j] = a0[j];
-        red[(ty * cvb + tx) * VN * 2 + VN + j] = a1[j];
-    }
-    __syncthreads();
-    if(ty == 0 && c0 < C) {
-        for(int t = 1; t < rb; t++) {
-#pragma unroll
-            for(int j = 0; j < VN; j++) {
-                a0[j] += red[(t * cvb + tx) * VN * 2 + j];
-                a1[j] += red[(t * cvb + tx) * VN * 2 + VN + j];
-            }
-        }
-        float *o = partial + ((int64_t)blockIdx.x * C + c0) * 2;
-#pragma unroll
-        for(int j = 0; j < VN; j++) {
-            o[j * 2] = a0[j];
-            o[j * 2 + 1] = a1[j];
-        }
-    }
+    block_partials<VN>(a0, a1, red, tx, cvb, partial, C);
 }
 
 // coef[0..C) = s*invstd ; coef[C..2C) = db/M ; coef[2C..3C) = ds*invstd/M ; writes ds, db.
@@ -505,28 +682,32 @@ __global__ void __launch_bounds__(256)
 }
 
 // Pass 2 of backward: dx = s*invstd*(dy' - db/M - (x-mean)*invstd*ds/M) ; dz = dy'.
-template <typename T, int VN, bool RC>
+template <typename T, int VN, bool RC, bool FIN = false>
 __global__ void __launch_bounds__(256)
     bn_bwd_apply_cl(const T *__restrict__ x, int64_t px, const T *__restrict__ y, int64_t py, const T *__restrict__ dy,
                     int64_t pdy, T *__restrict__ dx, int64_t pdx, T *__restrict__ dz, int64_t pdz,
                     const float *__restrict__ save_mean, const float *__restrict__ coef, int64_t rows, int C, int cvb_,
-                    int flags, float beta_dx, float beta_dz, const float *__restrict__ rb_)
+                    int flags, float beta_dx, float beta_dz, const float *__restrict__ rb_, BwdFin fin = BwdFin())
 {
     const int cvb = cvb_ < 0 ? -cvb_ : cvb_;
     const int tx = threadIdx.x % cvb, ty = threadIdx.x / cvb, rb = 256 / cvb;
     const int c0 = (blockIdx.y * cvb + tx) * VN;
-    if(c0 >= C)
+    if(!FIN && c0 >= C)
         return;
     const bool relu = flags & SAGA_BN_RELU;
     constexpr bool recompute = RC;
     float mean[VN], a[VN], k0[VN], k1[VN], sh[VN];
 #pragma unroll
     for(int j = 0; j < VN; j++) {
-        mean[j] = save_mean[c0 + j];
-        a[j] = coef[c0 + j]; // s * invstd: also the forward's scale
-        k0[j] = coef[C + c0 + j];
-        k1[j] = coef[2 * C + c0 + j];
-        sh[j] = recompute ? __builtin_fmaf(-mean[j], a[j], rb_[c0 + j]) : 0.0f;
+        const int c = FIN && c0 >= C ? 0 : c0 + j;
+        mean[j] = save_mean[c];
+        sh[j] = recompute ? rb_[c] : 0.0f;
+        if constexpr(!FIN) {
+            a[j] = coef[c]; // s * invstd: also the forward's scale
+            k0[j] = coef[C + c];
+            k1[j] = coef[2 * C + c];
+            sh[j] = recompute ? __builtin_fmaf(-mean[j], a[j], sh[j]) : 0.0f;
+        }
     }
     typedef Ld<T, VN> L;
     typedef typename L::V V;
@@ -563,8 +744,8 @@ __global__ void __launch_bounds__(256)
         }
     };
     int64_t r = rr.r0;
-    for(; r + 3 * stride < rend; r += 4 * stride) {
-        V xr[4], gr[4], yr[4];
+    V xr[4], gr[4], yr[4];
+    auto load4 = [&]() {
 #pragma unroll
         for(int u = 0; u < 4; u++) {
             const int64_t q = row(r + u * stride);
@@ -572,9 +753,35 @@ __global__ void __launch_bounds__(256)
             gr[u] = L::raw(dy + q * pdy + c0);
             yr[u] = relu && !recompute ? L::raw(y + q * py + c0) : gr[u];
         }
+    };
+    auto finish4 = [&]() {
 #pragma unroll
         for(int u = 0; u < 4; u++)
             finish(xr[u], gr[u], yr[u], row(r + u * stride));
+        r += 4 * stride;
+    };
+    if constexpr(FIN) {
+        __shared__ float tab[3][64];
+        const bool ahead = c0 < C && r + 3 * stride < rend;
+        if(ahead)
+            load4();
+        bwd_slab(fin, C, blockIdx.y * cvb * VN, cvb * VN, tab);
+        if(c0 >= C)
+            return;
+#pragma unroll
+        for(int j = 0; j < VN; j++) {
+            a[j] = tab[0][tx * VN + j];
+            k0[j] = tab[1][tx * VN + j];
+            k1[j] = tab[2][tx * VN + j];
+            if(recompute)
+                sh[j] = __builtin_fmaf(-mean[j], a[j], sh[j]);
+        }
+        if(ahead)
+            finish4();
+    }
+    while(r + 3 * stride < rend) {
+        load4();
+        finish4();
     }
     for(; r < rend; r += stride) {
         const int64_t q = row(r);
@@ -957,8 +1164,16 @@ int saga_hip_bn_train_fwd_partials(const SagaTensorView *x, const SagaTensorView
     // the mask has one byte per 8 fp16 channels: only the 8-wide fp16 kernel with relu writes it
     if(relu_mask && !(x->dtype == SAGA_HALF && vn == 8 && (flags & SAGA_BN_RELU)))
         return SAGA_HIP_EUNSUPPORTED;
-    Shape sh = plan(lx.rows, C / vn);
-    dim3 grid(sh.gx, sh.gy);
+    Shape sh;
+    if(x->dtype == SAGA_HALF && vn == 8 && self_finalizing(lx.rows, C, partial_rows, false, &sh)) {
+        const StatsFin fin = {partial, partial_rows, s, b, run_m, run_v, save_mean, save_invstd, (double)lx.rows, eps, expavg};
+        bn_apply_cl<half_t, 8, 2><<<dim3(sh.gx, sh.gy), 256, 0, st>>>(
+            (const half_t *)x->ptr, lx.pitch, add ? (const half_t *)z->ptr : nullptr, lz.pitch, (half_t *)y->ptr, ly.pitch, nullptr,
+            nullptr, nullptr, nullptr, nullptr, eps, lx.rows, C, sh.cvb, flags, relu_mask, fin);
+        SAGA_CHECK_LAUNCH();
+        return 0;
+    }
+    sh = plan(lx.rows, C / vn);
 #define GO(T, VN)                                                                                                   \
     do {                                                                                                            \
         bn_stats_finalize<T><<<C, 256, 0, st>>>(partial, partial_rows, (const T *)nullptr, 1, s, b, run_m, \
@@ -1047,6 +1262,24 @@ int saga_hip_bn_bwd_ex(const SagaTensorView *x, const SagaTensorView *y, const S
                                                      lx.rows, C, WALK_CVB(4), flags, recompute ? s : nullptr,             \
                                                      recompute ? b : nullptr, recompute ? save_invstd : nullptr,     \
                                                      early_dz ? (T *)dz->ptr : nullptr, ldz.pitch, mk);              \
+        if constexpr(sizeof(T) == 2 && VN == 8) {                                                                    \
+            Shape sf;                                                                                                \
+            if(self_finalizing(lx.rows, C, sh.gx, true, &sf)) {                                                            \
+                const BwdFin fin = {partial, sh.gx, s, save_invstd, ds, db, (double)lx.rows, beta_p};                \
+                if(early_dz)                                                                                         \
+                    bn_bwd_apply_cl<T, VN, false, true><<<dim3(sf.gx, sf.gy), 256, 0, st>>>(                         \
+                        (const T *)x->ptr, lx.pitch, nullptr, 0, (const T *)dz->ptr, ldz.pitch, (T *)dx->ptr,        \
+                        ldx.pitch, nullptr, 0, save_mean, coef, lx.rows, C, sf.cvb, flags & ~SAGA_BN_RELU, beta_dx,  \
+                        0.0f, nullptr, fin);                                                                         \
+                else                                                                                                 \
+                    bn_bwd_apply_cl<T, VN, RC, true><<<dim3(sf.gx, sf.gy), 256, 0, st>>>(                            \
+                        (const T *)x->ptr, lx.pitch, relu ? (const T *)y->ptr : nullptr, ly.pitch,                   \
+                        (const T *)dy->ptr, ldy.pitch, (T *)dx->ptr, ldx.pitch, dz ? (T *)dz->ptr : nullptr,         \
+                        ldz.pitch, save_mean, coef, lx.rows, C, sf.cvb, flags, beta_dx, beta_dz,                     \
+                        recompute ? b : nullptr, fin);                                                               \
+                break;                                                                                               \
+            }                                                                                                        \
+        }                                                                                                            \
         bn_bwd_finalize<<<C, 256, 0, st>>>(partial, sh.gx, s, save_invstd, ds, db, coef,                \
                                                          (double)lx.rows, C, beta_p);                                \
         if(early_dz)                                                                                                 \
@@ -1106,8 +1339,16 @@ int saga_hip_bn_bwd_linked(const SagaTensorView *x, const SagaTensorView *g, con
     hipStream_t st = as_stream(stream);
     float *coef = (float *)workspace;
     const int vn = vec_width(dt, C, {x, g, dx}, {lx.pitch, lg.pitch, ldx.pitch});
+    Shape sf;
+    if(dt == SAGA_HALF && vn == 8 && self_finalizing(lx.rows, C, partial_rows, true, &sf)) {
+        const BwdFin fin = {partial, partial_rows, s, save_invstd, ds, db, (double)lx.rows, beta_p};
+        bn_bwd_apply_cl<half_t, 8, false, true><<<dim3(sf.gx, sf.gy), 256, 0, st>>>(
+            (const half_t *)x->ptr, lx.pitch, nullptr, 0, (const half_t *)g->ptr, lg.pitch, (half_t *)dx->ptr, ldx.pitch, nullptr, 0,
+            save_mean, coef, lx.rows, C, sf.cvb, 0, beta_dx, 0.0f, nullptr, fin);
+        SAGA_CHECK_LAUNCH();
+        return 0;
+    }
     const Shape sh = plan(lx.rows, C / vn, true);
-    const dim3 grid(sh.gx, sh.gy);
     bn_bwd_finalize<<<C, 256, 0, st>>>(partial, partial_rows, s, save_invstd, ds, db, coef, (double)lx.rows, C, beta_p);
 #define GO(T, VN)                                                                                                     \
     bn_bwd_apply_cl<T, VN, false><<<WALK_GRID(8), 256, 0, st>>>((const T *)x->ptr, lx.pitch, nullptr, 0, (const T *)g->ptr,    \
