@@ -1521,16 +1521,16 @@ __global__ void __launch_bounds__(256) transpose_filter_batched(const SagaFilter
     }
 }
 
-// w (K, C, R, S logical; stored K,R,S,C) -> wT stored C,R,S,K
-__global__ void __launch_bounds__(256) transpose_filter(const half_t *__restrict__ w, half_t *__restrict__ wt, int K, int C, int RS)
+// w (K, C, R, S logical; stored K,R,S,C) -> wT stored C,R,S,Kp, Kp >= K, zero filled
+__global__ void __launch_bounds__(256) transpose_filter(const half_t *__restrict__ w, half_t *__restrict__ wt, int K, int Kp, int C, int RS)
 {
-    const int64_t total = (int64_t)K * C * RS;
+    const int64_t total = (int64_t)Kp * C * RS;
     for(int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
         // i enumerates the destination: (c, tap, k) with k fastest
-        const int k = (int)(i % K);
-        const int tap = (int)((i / K) % RS);
-        const int c = (int)(i / ((int64_t)K * RS));
-        wt[i] = w[((int64_t)k * RS + tap) * C + c];
+        const int k = (int)(i % Kp);
+        const int tap = (int)((i / Kp) % RS);
+        const int c = (int)(i / ((int64_t)Kp * RS));
+        wt[i] = k < K ? w[((int64_t)k * RS + tap) * C + c] : (half_t)0;
     }
 }
 
@@ -1980,13 +1980,14 @@ __global__ void __launch_bounds__(64 * NW) conv_bwd_filter_dma(FilterArgs g, uns
     }
 }
 
-// dw[row, c] = alpha * sum_p partial[p][row, c] + beta * dw; rows = K*R*S, the partial rows are Cp wide (a multiple of
-// 8, more than C where the input channels were padded; n = elements of a partial).  16 lanes cover 64 consecutive
+// dw[row, c] = alpha * sum_p partial[p][row, c] + beta * dw; the partial rows are Cp wide (a multiple of 8, more than C
+// where the input channels were padded), n = rows of dw * Cp elements, the partials `pitch` apart (more than n where the
+// output channels were padded).  16 lanes cover 64 consecutive
 // elements with float4 loads, the 16 lane groups of a block take every 16th partial, and LDS combines the groups in a
 // fixed order (deterministic).  (One lane per element over all of the partials, as padded rows had it: 131 us for the whole
 // gradient of 3x3 3->16 at 128x32x32, 23 now.)
 __global__ void __launch_bounds__(256)
-    filter_reduce_v4(const float *__restrict__ partial, half_t *__restrict__ dw, int64_t n, int C, int Cp, int splits, float alpha,
+    filter_reduce_v4(const float *__restrict__ partial, half_t *__restrict__ dw, int64_t n, int64_t pitch, int C, int Cp, int splits, float alpha,
                      float beta)
 {
     __shared__ float4_t red[16][16];
@@ -1995,23 +1996,33 @@ __global__ void __launch_bounds__(256)
     float4_t s = {0, 0, 0, 0};
     if(e < n)
         for(int p = sl; p < splits; p += 16)
-            s += *(const float4_t *)(partial + (int64_t)p * n + e);
+            s += *(const float4_t *)(partial + (int64_t)p * pitch + e);
     red[sl][ev] = s;
     __syncthreads();
     if(sl == 0 && e < n) {
 #pragma unroll
         for(int q = 1; q < 16; q++)
             s += red[q][ev];
-        int64_t o = e;
-        int c = 0;
-        if(C != Cp) {
-            const int64_t row = e / Cp;
-            c = (int)(e - row * Cp);
-            o = row * C + c;
+        if(C == Cp) { // one store
+            typedef half_t half4u_t __attribute__((ext_vector_type(4), aligned(2)));
+            half4u_t *o = (half4u_t *)(dw + e);
+            half4u_t r;
+            const half4u_t old = beta != 0.0f ? *o : half4u_t{0, 0, 0, 0};
+#pragma unroll
+            for(int j = 0; j < 4; j++) {
+                float v = alpha * s[j];
+                if(beta != 0.0f)
+                    v += beta * (float)old[j];
+                r[j] = (half_t)v;
+            }
+            *o = r;
+            return;
         }
+        const int64_t row = e / Cp, o = row * C + (e - row * Cp);
+        const int c = (int)(e - row * Cp);
 #pragma unroll
         for(int j = 0; j < 4; j++) {
-            if(C != Cp && c + j >= C)
+            if(c + j >= C)
                 break;
             float v = alpha * s[j];
             if(beta != 0.0f)
@@ -2032,9 +2043,14 @@ __global__ void __launch_bounds__(256)
         const int64_t r = i / groups;
         const int c0 = (int)(i - r * groups) * 8;
         half8_t v;
+        if(c0 + 8 <= C) { // (rows start at any even address)
+            typedef half_t half8u_t __attribute__((ext_vector_type(8), aligned(2)));
+            v = *(const half8u_t *)(src + r * sp + c0);
+        } else {
 #pragma unroll
-        for(int e = 0; e < 8; e++)
-            v[e] = (c0 + e < C) ? src[r * sp + c0 + e] : (half_t)0;
+            for(int e = 0; e < 8; e++)
+                v[e] = (c0 + e < C) ? src[r * sp + c0 + e] : (half_t)0;
+        }
         *(half8_t *)(dst + r * Cp + c0) = v;
     }
 }
@@ -2200,11 +2216,10 @@ __global__ void __launch_bounds__(256)
 // 16 outputs per block, 16 threads per output that each add every 16th split (four loads in flight),
 // then a fixed-order sum of the 16: hundreds of splits would otherwise be one long dependent chain.
 __global__ void __launch_bounds__(256)
-    thin_filter_reduce(const float *__restrict__ partial, half_t *__restrict__ dw, int64_t n, int C, int S, int splits,
+    thin_filter_reduce(const float *__restrict__ partial, half_t *__restrict__ dw, int64_t n, int64_t np, int C, int S, int splits,
                        float alpha, float beta)
 {
     __shared__ float part[16][17];
-    const int64_t np = n / (S * C) * 32;
     const int o = threadIdx.x & 15, q = threadIdx.x >> 4;
     const int64_t i = (int64_t)blockIdx.x * 16 + o;
     float acc = 0;
@@ -3675,16 +3690,17 @@ static int tile_override()
 }
 
 // How many blocks share the reduction of a tile (1: none), by the number of tiles and slices of 32.  Fitted to measured
-// times: a slice takes a block 0.36 us, a shared launch and its second kernel cost 9 us more than a plain one, and writing
+// times: a slice takes a block 0.36 us (0.24 with 64 channels), a shared launch and its second kernel cost 9 us more than a plain one, and writing
 // and reading the sums of a 256x128 tile 33 ns; more blocks than CUs only add sums.  (us, alone -> shared by k:
 // 3x3 1024->1024 at 21x21 90 -> 28 k=10; 3x3 1024->512 at 42x42 96 -> 35 k=8; 3x3 512->512 at 64x7x7 50 -> 34 k=4;
 // at 128x7x7 52 -> 47 k=2; 1x1 2048->512 at 23x7x7 23 -> 18 k=3; 3x3 256->256 at 64x14x14 31 -> 35 k=2, not taken.)
 static int split_rule(int64_t tiles, int bn, int slices)
 {
-    double best = 0.93 * (4 + 0.36 * slices);
+    const double slice = bn == 64 ? 0.24 : 0.36;
+    double best = 0.93 * (4 + slice * slices);
     int k = 1;
     for(int c = 2; c <= 16 && tiles * c <= 256 && c * 4 <= slices; c++) {
-        const double t = 13 + 0.36 * ((slices + c - 1) / c) + 0.033 * bn / 128 * (double)(tiles * c);
+        const double t = 13 + slice * ((slices + c - 1) / c) + 0.033 * bn / 128 * (double)(tiles * c);
         if(t < best) {
             best = t;
             k = c;
@@ -3993,6 +4009,38 @@ static size_t split_bytes(bool bwd, const ConvGeom &g)
     return k > 1 ? (size_t)(tiles * k * 256 * bn * 4) : 0;
 }
 
+// The backward passes read dy in vectors of 8 channels too; other channel counts and pitches go through a padded copy in
+// front of the workspace.  (The direct kernels, which took them before, need 100 - 4000 times as long as the copy: backward
+// filter of 1x1 353->39 at 155x55x55 152 ms -> 241 us, of 3x3 314->202 at 44x44 2.1 ms -> 26 us; backward data of 5x5 370->12
+// at 34x91x91 stride 2 3.2 ms -> 307 us.)
+static bool pads_dy(const ConvGeom &g, const CLInfo &ldy) { return g.K % 8 || ldy.pitch % 8; }
+static size_t padded_bytes(int64_t rows, int K) { return ((size_t)rows * round8(K) * sizeof(half_t) + 255) & ~(size_t)255; }
+
+// dy padded to whole vectors at the start of ws, which then begins behind it; its view and the geometry that goes with it
+static int pad_dy(const SagaTensorView *dy, const CLInfo &ldy, ConvGeom &g, SagaTensorView &v, void *&ws, size_t &ws_bytes, hipStream_t st)
+{
+    const int K = g.K, Kp = round8(K);
+    const size_t bytes = padded_bytes(ldy.rows, K);
+    if(!ws || ws_bytes < bytes || !aligned16(ws))
+        return SAGA_HIP_EWORKSPACE;
+    if((int64_t)ldy.rows * Kp >= (int64_t)1 << 31)
+        return SAGA_HIP_EUNSUPPORTED;
+    pad_channels<<<grid_for(ldy.rows * (Kp / 8), 256, 256 * 16), 256, 0, st>>>((const half_t *)dy->ptr, ldy.pitch, K, (half_t *)ws, Kp,
+                                                                              ldy.rows);
+    SAGA_CHECK_LAUNCH();
+    g.K = Kp;
+    v = *dy;
+    v.ptr = ws;
+    v.dims[1] = Kp;
+    v.strides[1] = 1;
+    v.strides[3] = Kp;
+    v.strides[2] = (int64_t)Kp * v.dims[3];
+    v.strides[0] = v.strides[2] * v.dims[2];
+    ws = (char *)ws + bytes;
+    ws_bytes -= bytes;
+    return 0;
+}
+
 size_t conv_mfma_workspace(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                            const ConvGeom &g)
 {
@@ -4007,22 +4055,28 @@ size_t conv_mfma_workspace(int kind, const SagaTensorView *x, const SagaTensorVi
     const bool thin = thin_ok(g, &tg);
     if(kind == SAGA_CONV_FWD)
         return std::max(xpad + wpad, thin ? tg.x4_bytes + tg.wv_bytes : 0) + 512 + split_bytes(false, g);
+    ConvGeom gp = g; // what the kernels see of dy
+    size_t ypad = 0;
+    CLInfo ly;
+    if(as_channels_last(y, &ly) && pads_dy(g, ly)) {
+        gp.K = round8(g.K);
+        ypad = padded_bytes(ly.rows, gp.K);
+    }
     if(kind == SAGA_CONV_BWD_DATA)
-        return (size_t)g.K * g.C * g.R * g.S * sizeof(half_t) + 512 + split_bytes(true, g);
+        return ypad + (size_t)gp.K * g.C * g.R * g.S * sizeof(half_t) + 512 + split_bytes(true, gp);
     if(kind == SAGA_CONV_BWD_FILTER) {
-        ConvGeom gp = g;
         gp.C = (int)Cp;
         // the launcher falls back to the small tiles for tensors beyond the buffer-load range
         const FilterPlan p = plan_filter(gp), ps = plan_filter(gp, false);
-        size_t need = xpad + (size_t)std::max(p.splits, ps.splits) * g.K * g.R * g.S * Cp * sizeof(float);
+        size_t need = xpad + (size_t)std::max(p.splits, ps.splits) * gp.K * g.R * g.S * Cp * sizeof(float);
         if(thin) {
-            ConvGeom gv = g;
+            ConvGeom gv = gp;
             gv.C = 32;
             gv.S = 1;
             const FilterPlan pv = plan_filter(gv, true, true);
-            need = std::max(need, tg.x4_bytes + (size_t)pv.splits * g.K * g.R * 32 * sizeof(float));
+            need = std::max(need, tg.x4_bytes + (size_t)pv.splits * gp.K * g.R * 32 * sizeof(float));
         }
-        return need + 256;
+        return ypad + need + 256;
     }
     return 0;
 }
@@ -4215,9 +4269,10 @@ bool conv_mfma_bnbwd_link_ok(const SagaTensorView *dy, const SagaTensorView *w, 
 
 // wt_ready: the filter already transposed to C,R,S,K (by transpose_filter or the batched kernel below);
 // otherwise it is transposed into the workspace first
-int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx,
-                       const ConvGeom &g, float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st,
-                       const void *wt_ready, const ConvBnBwdLink *link, const void *bias, bool *bias_done)
+// g.K: channels of dy (a multiple of 8); krows: filters of w, fewer where dy was padded
+static int bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g, int krows,
+                    float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const void *wt_ready,
+                    const ConvBnBwdLink *link, const void *bias, bool *bias_done)
 {
     CLInfo ldy, ldx, lbx;
     if(!common_ok(dy, w, dx, g, &ldy, &ldx))
@@ -4239,7 +4294,7 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
     const half_t *wt = (const half_t *)wt_ready;
     // nobody has transposed the filter: the row-resident 3x3 kernel reads it as it is
     bool krsc = false;
-    if(!wt && !link && dma_stages() >= 2 && aligned16(w->ptr)) {
+    if(!wt && !link && krows == g.K && dma_stages() >= 2 && aligned16(w->ptr)) {
         wt = (const half_t *)w->ptr;
         krsc = true;
     }
@@ -4248,7 +4303,7 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
         if(!ws || ws_bytes < need || !aligned16(ws))
             return SAGA_HIP_EWORKSPACE;
         const int64_t total = (int64_t)g.K * g.C * g.R * g.S;
-        transpose_filter<<<grid_for(total, 256, 256 * 16), 256, 0, st>>>((const half_t *)w->ptr, (half_t *)ws, g.K, g.C,
+        transpose_filter<<<grid_for(total, 256, 256 * 16), 256, 0, st>>>((const half_t *)w->ptr, (half_t *)ws, krows, g.K, g.C,
                                                                         g.R * g.S);
         wt = (const half_t *)ws;
     } else if(!aligned16(wt)) {
@@ -4293,7 +4348,7 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
         if(!ws || ws_bytes < need || !aligned16(ws))
             return SAGA_HIP_EWORKSPACE;
         const int64_t total = (int64_t)g.K * g.C * g.R * g.S;
-        transpose_filter<<<grid_for(total, 256, 256 * 16), 256, 0, st>>>((const half_t *)w->ptr, (half_t *)ws, g.K, g.C,
+        transpose_filter<<<grid_for(total, 256, 256 * 16), 256, 0, st>>>((const half_t *)w->ptr, (half_t *)ws, g.K, g.K, g.C,
                                                                         g.R * g.S);
         a.b = (const half_t *)ws;
         a.b_krsc = 0;
@@ -4315,8 +4370,9 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
     return rc;
 }
 
-int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw,
-                         const ConvGeom &g, float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st)
+// g.K: channels of dy (a multiple of 8); krows: filters of dw, fewer where dy was padded
+static int bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g, int krows,
+                      float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st)
 {
     CLInfo lx, ldy;
     bool pad = false;
@@ -4324,7 +4380,7 @@ int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, cons
         return SAGA_HIP_EUNSUPPORTED;
     if(g.K % 8 || ldy.pitch % 8 || !aligned16(dy->ptr))
         return SAGA_HIP_EUNSUPPORTED;
-    const int64_t n = (int64_t)g.K * g.R * g.S * g.C;
+    const int64_t n = (int64_t)g.K * g.R * g.S * g.C, rows = (int64_t)krows * g.R * g.S;
     ThinGeom tg;
     if(dma_stages() >= 2 && thin_ok(g, &tg)) {
         ConvGeom gv = g;
@@ -4361,8 +4417,8 @@ int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, cons
         else
             conv_bwd_filter_dma<64, 128, ST, 4><<<blocks, 256, ST * BK * 384, st>>>(a, (unsigned)(px * 8), (unsigned)yb);
         SAGA_CHECK_LAUNCH();
-        thin_filter_reduce<<<(int)((n + 15) / 16), 256, 0, st>>>(a.partial, (half_t *)dw->ptr, n, g.C, g.S, p.splits,
-                                                                    alpha, beta);
+        thin_filter_reduce<<<(int)((rows * g.C + 15) / 16), 256, 0, st>>>(a.partial, (half_t *)dw->ptr, rows * g.C,
+                                                                         (int64_t)g.K * g.R * 32, g.C, g.S, p.splits, alpha, beta);
         SAGA_CHECK_LAUNCH();
         return 0;
     }
@@ -4423,8 +4479,8 @@ int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, cons
             }
             kern<<<blocks, 256, lds, st>>>(t);
             SAGA_CHECK_LAUNCH();
-            filter_reduce_v4<<<(unsigned)((n / 4 + 15) / 16), 256, 0, st>>>(t.partial, (half_t *)dw->ptr, n, g.C, g.C, blocks, alpha,
-                                                                            beta);
+            filter_reduce_v4<<<(unsigned)((rows * g.C / 4 + 15) / 16), 256, 0, st>>>(t.partial, (half_t *)dw->ptr, rows * g.C, n, g.C, g.C, blocks,
+                                                                                   alpha, beta);
             SAGA_CHECK_LAUNCH();
             return 0;
         }
@@ -4486,8 +4542,46 @@ int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, cons
     }
     SAGA_CHECK_LAUNCH();
     const int64_t np = n / g.C * Cp;
-    filter_reduce_v4<<<(unsigned)((np / 4 + 15) / 16), 256, 0, st>>>(a.partial, (half_t *)dw->ptr, np, g.C, Cp, p.splits, alpha,
-                                                                   beta);
+    filter_reduce_v4<<<(unsigned)((rows * Cp / 4 + 15) / 16), 256, 0, st>>>(a.partial, (half_t *)dw->ptr, rows * Cp, np, g.C, Cp,
+                                                                          p.splits, alpha, beta);
     SAGA_CHECK_LAUNCH();
     return 0;
+}
+
+static bool refuses_dy(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *d, const ConvGeom &g, CLInfo *ldy)
+{
+    CLInfo ld;
+    return dy->dtype != SAGA_HALF || g.group != 1 || !as_channels_last(dy, ldy) || !as_channels_last(d, &ld) || !krsc_dense(w);
+}
+
+int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g, float alpha,
+                         float beta, void *ws, size_t ws_bytes, hipStream_t st)
+{
+    CLInfo ldy;
+    if(refuses_dy(dy, dw, x, g, &ldy))
+        return SAGA_HIP_EUNSUPPORTED;
+    // (a million multiplications are over before the copy is: 1x1 10->137 at 15x5x5 7 us directly, 15 this way)
+    if(pads_dy(g, ldy) && ldy.rows * g.K * g.C * g.R * g.S <= 1 << 20)
+        return SAGA_HIP_EUNSUPPORTED;
+    if(!pads_dy(g, ldy))
+        return bwd_filter(x, dy, dw, g, g.K, alpha, beta, ws, ws_bytes, st);
+    ConvGeom gp = g;
+    SagaTensorView dyp;
+    const int r = pad_dy(dy, ldy, gp, dyp, ws, ws_bytes, st);
+    return r ? r : bwd_filter(x, &dyp, dw, gp, g.K, alpha, beta, ws, ws_bytes, st);
+}
+
+int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g, float alpha,
+                       float beta, void *ws, size_t ws_bytes, hipStream_t st, const void *wt_ready, const ConvBnBwdLink *link,
+                       const void *bias, bool *bias_done)
+{
+    CLInfo ldy;
+    if(refuses_dy(dy, w, dx, g, &ldy) || ilog2_exact(g.stride) < 0)
+        return SAGA_HIP_EUNSUPPORTED;
+    if(wt_ready || link || !pads_dy(g, ldy))
+        return bwd_data(dy, w, dx, g, g.K, alpha, beta, ws, ws_bytes, st, wt_ready, link, bias, bias_done);
+    ConvGeom gp = g;
+    SagaTensorView dyp;
+    const int r = pad_dy(dy, ldy, gp, dyp, ws, ws_bytes, st);
+    return r ? r : bwd_data(&dyp, w, dx, gp, g.K, alpha, beta, ws, ws_bytes, st, nullptr, nullptr, bias, bias_done);
 }

@@ -379,7 +379,7 @@ struct Config {
 //   4x14x14 1x1 256->1024          3136         8  2,2,2,2  7.2                                6.9
 // Beyond these the sums of a tile are better shared by several blocks of the tiled kernel (42x42 3x3 1024->512: 35 against
 // 48 us here and 96 alone).
-Config choose(long long tiles, long long steps)
+Config choose(long long tiles, long long steps, int N)
 {
     if(tiles > 3600 || (steps >= 200 && tiles >= 1500) || (steps >= 128 && tiles > 3300))
         return {0, 0, 0, 0};
@@ -395,9 +395,11 @@ Config choose(long long tiles, long long steps)
             return {4, 2, 8, 1};
         return {2, 2, steps >= 64 && tiles <= 900 ? 8 : 4, 1};
     }
+    // (wide tiles only for channels that fill them: 5x5 160->32 at 57x17x17 25 against 51 us, the tiled kernel 27.  Its tiles of
+    // 64 channels are enough blocks for narrow layers: 5x5 64->16 at 49x30x30 24 against 29, 48->40 at 7x50x50 26 against 30)
     if(steps >= 64)
-        return {4, 4, 4, 1};
-    return steps >= 16 ? Config{2, 2, 2, 2} : Config{0, 0, 0, 0};
+        return N > 32 ? Config{4, 4, 4, 1} : Config{4, 2, 4, 1};
+    return steps >= 16 && N > (steps >= 32 ? 64 : 16) ? Config{2, 2, 2, 2} : Config{0, 0, 0, 0};
 }
 
 Config config_of(const StreamF16 &g)
@@ -405,7 +407,7 @@ Config config_of(const StreamF16 &g)
     const int s = g.bwd ? g.stride : 1;
     const long long pixels = (long long)g.batch * ((g.OH + s - 1) / s) * ((g.OW + s - 1) / s) * s * s;
     const long long taps = ((g.R + s - 1) / s) * ((g.S + s - 1) / s);
-    return choose((pixels + 15) / 16 * ((g.N + 15) / 16), taps * ((g.C + 31) / 32));
+    return choose((pixels + 15) / 16 * ((g.N + 15) / 16), taps * ((g.C + 31) / 32), g.N);
 }
 
 int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }

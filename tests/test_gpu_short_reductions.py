@@ -96,3 +96,21 @@ def test_sum_of_filter_partials(N, Cc, H, Kk, dtype, layout):
     dw = dev(np.ones(want.shape, np.float32), dtype, layout)
     K.conv2d(K.CONV_BWD_FILTER, dev(x, dtype, layout), dev(dy, dtype, layout), dw, 1, 1, beta=1.0)
     assert_close(host(dw), want + 1, dtype, "bwd filter", tol=2e-3 if dtype == HALF else 1e-5)
+
+
+@pytest.mark.parametrize("N,Cc,H,W,Kk,R,stride,pad", [(2, 16, 9, 7, 1, 1, 1, 0), (3, 24, 13, 11, 7, 3, 1, 1), (2, 3, 40, 33, 20, 7, 2, 3),
+                                                      (2, 13, 21, 19, 39, 5, 2, 2), (4, 64, 56, 56, 60, 3, 1, 1), (1, 70, 30, 31, 202, 3, 4, 1)])
+def test_fp16_gradients_of_other_channel_counts(N, Cc, H, W, Kk, R, stride, pad):
+    """Output channels in other numbers than eights: dy goes through a padded copy."""
+    rng = np.random.default_rng(Kk)
+    x = rnd(rng, N, Cc, H, W, dtype=HALF)
+    w = rnd(rng, Kk, Cc, R, R, dtype=HALF, scale=(2.0 / (Cc * R * R)) ** 0.5)
+    P, Q = 1 + (H + 2 * pad - R) // stride, 1 + (W + 2 * pad - R) // stride
+    dy = rnd(rng, N, Kk, P, Q, dtype=HALF)
+    for padc in (0, 3):  # dense, and a slice of a wider tensor
+        xd, wd, dyd = dev(x, HALF, "nhwc"), dev(w, HALF, "nhwc"), dev(dy, HALF, "nhwc", padc)
+        dw, dx = dev(np.ones(w.shape, np.float32), HALF, "nhwc"), dev(np.ones(x.shape, np.float32), HALF, "nhwc")
+        K.conv2d(K.CONV_BWD_FILTER, xd, dyd, dw, pad, stride, beta=1.0)
+        assert_close(host(dw), ref.conv2d_bwd_filter(x, dy, w.shape, pad, stride) + 1, HALF, "dw", tol=2e-3)
+        K.conv2d(K.CONV_BWD_DATA, dyd, wd, dx, pad, stride, beta=1.0)
+        assert_close(host(dx), ref.conv2d_bwd_data(dy, w, x.shape, pad, stride) + 1, HALF, "dx", tol=2e-3)
