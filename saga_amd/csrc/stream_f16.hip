@@ -22,6 +22,22 @@ namespace {
 constexpr int MAX_CLASSES = 16;
 constexpr unsigned OOB = 0x7fffff00u; // beyond every buffer: the load returns zero
 
+// n / d for 0 <= n < 2^31 without a division
+struct Div {
+    unsigned mul, shift;
+};
+
+Div div_by(unsigned d)
+{
+    Div v = {1, 0};
+    while((1u << v.shift) < d)
+        v.shift++;
+    v.mul = (unsigned)((((unsigned long long)((1u << v.shift) - d)) << 32) / d) + 1;
+    return v;
+}
+
+__device__ __forceinline__ int divide(int n, Div d) { return (int)((__umulhi((unsigned)n, d.mul) + (unsigned)n) >> d.shift); }
+
 // Output pixels whose taps sit at the same distances.  Forward: all of them.  Backward data at stride s: pixels (y, x) with
 // the same y mod s and x mod s; inside a class consecutive taps are a fixed distance apart.
 struct Class {
@@ -33,12 +49,16 @@ struct Class {
     int M;        // class pixels over all images
     int block0;   // first block
     int row0;     // first row of sums
+    int nm;       // blocks along the pixels
+    Div by_OH, by_OW, by_Ts, by_nm;
 };
 
 template <int CLASSES> struct ArgsOf {
     StreamF16 g;
     int istep, ostep, tstep, rstep;
-    int nclasses, nblk_q, blocks, KS;
+    int nclasses, nblk_q, blocks;
+    int ks_log2, WM, S32; // wavefronts along the reduction and the pixels; steps of 32 channels per tap
+    Div by_q, by_S32;
     int q_outer; // blocks that are neighbours share their channels (else their pixels)
     Class cls[CLASSES];
 };
@@ -69,62 +89,107 @@ __device__ __forceinline__ int xcd_order(int b, int n)
     return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + slot;
 }
 
+// LDS of a wavefront: the ring, then its sums in the same place
+template <int TM, int TN, int DEPTH> constexpr int wave_lds()
+{
+    return std::max(DEPTH * (TM + TN) * 1024, TM * 16 * (TN * 16 + 4) * 4);
+}
+
+typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void *p, unsigned bytes)
+{
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, p ? (int)bytes : 0, 0x00020000);
+}
+
+// Four channels of a tensor from byte offset `at` (OOB: none), in one access or - rows of any pitch - one by one, `n` of
+// them inside the row.
+__device__ __forceinline__ half4_t load4(__amdgpu_buffer_rsrc_t r, unsigned at, bool vec, int n)
+{
+    if(vec)
+        return __builtin_bit_cast(half4_t, (uint2_t)__builtin_amdgcn_raw_buffer_load_b64(r, at, 0, 0));
+    half4_t v;
+#pragma unroll
+    for(int q = 0; q < 4; q++)
+        v[q] = __builtin_bit_cast(half_t, (unsigned short)__builtin_amdgcn_raw_buffer_load_b16(r, q < n ? at + 2 * q : OOB, 0, 0));
+    return v;
+}
+__device__ __forceinline__ void store4(__amdgpu_buffer_rsrc_t r, unsigned at, bool vec, int n, half4_t v)
+{
+    if(vec) {
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(uint2_t, v), r, at, 0, 0);
+        return;
+    }
+#pragma unroll
+    for(int q = 0; q < 4; q++) {
+        const half_t one = v[q]; // (the cast of a vector's element takes the first)
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, one), r, q < n ? at + 2 * q : OOB, 0, 0);
+    }
+}
+
+// A launch takes a few microseconds, and most of them are trips to memory in a row: the arguments, the code (every 64 bytes
+// are a miss the first time a CU meets them), the operands, what the epilogue reads.  So the lines of the arguments are all
+// touched first; the epilogue's operands are requested in front of the reduction, through buffer loads that need no branch
+// (behind a branch the compiler waits for each before the next); divisions are multiplications; tap bits are kept by row and
+// column; a step is the same code for all taps, its loop inside the loop over the taps.
+// One image of 14x14 pixels, us in the kernel, against the same tiles with the ring unrolled (11 KB of code): 1x1 256->1024
+// 4.8 -> 3.0 (now 0.6 setup, 0.8 filling the ring, 0.7 the rest of the reduction, 0.2 the sum of the wavefronts, 0.5
+// epilogue), 1x1 1024->256 4.7 -> 3.3, 3x3 256->256 7.1 -> 4.6; from the end of a launch to the next it is 1.4.
 // SUMS: with the per-channel sums (StreamF16::sums)
 template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__ void __launch_bounds__(64 * MAXW) stream_f16_k(A k)
 {
     extern __shared__ __attribute__((aligned(16))) float smem[];
+    constexpr bool ONE = sizeof(A) == sizeof(Args1); // one class: class pixels are output pixels
     const StreamF16 &g = k.g;
+    {
+        const __attribute__((address_space(4))) int *line = (const __attribute__((address_space(4))) int *)__builtin_amdgcn_kernarg_segment_ptr();
+        static_assert(sizeof(Args1) > 5 * 64, "arguments");
+        asm volatile("" ::"s"(line[0]), "s"(line[16]), "s"(line[32]), "s"(line[48]), "s"(line[64]), "s"(line[80]));
+    }
     // as the matrix unit wants its operands, and as the loads fetch them: row lrow, 16-byte piece lkq of its 64.  Rows 4
     // apart fall into the same banks, so they keep their pieces in another order.
     const int tid = threadIdx.x, lane = tid & 63, row = lane & 15, kq = lane >> 4, lrow = lane >> 2;
     const int lkq = (lane & 3) ^ ((lrow >> 2) & 3);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int KS = k.KS, WM = (int)(blockDim.x >> 6) / KS;
-    const int wm = wave / KS, ks = wave - wm * KS;
+    const int KS = 1 << k.ks_log2, wm = wave >> k.ks_log2, ks = wave & (KS - 1);
     int b = xcd_order(blockIdx.x, k.blocks), ci = 0;
-    while(sizeof(A) > sizeof(Args1) && ci + 1 < k.nclasses && b >= k.cls[ci + 1].block0)
+    while(!ONE && ci + 1 < k.nclasses && b >= k.cls[ci + 1].block0)
         ci++;
     const Class &c = k.cls[ci];
     b -= c.block0;
-    int bm, bq;
-    if(k.q_outer) {
-        const int nm = (c.M + 16 * TM * WM - 1) / (16 * TM * WM);
-        bq = b / nm;
-        bm = b - bq * nm;
-    } else {
-        bm = b / k.nblk_q;
-        bq = b - bm * k.nblk_q;
-    }
-    const int m0 = (bm * WM + wm) * (16 * TM), n0 = bq * (16 * TN);
-    const __amdgpu_buffer_rsrc_t ra = __builtin_amdgcn_make_buffer_rsrc((void *)g.a, 0, (int)g.a_bytes, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void *)g.b, 0, (int)g.b_bytes, 0x00020000);
+    const int outer = divide(b, k.q_outer ? c.by_nm : k.by_q), inner = b - outer * (k.q_outer ? c.nm : k.nblk_q);
+    const int bm = k.q_outer ? inner : outer, bq = k.q_outer ? outer : inner;
+    const int m0 = (bm * k.WM + wm) * (16 * TM), n0 = bq * (16 * TN);
+    const __amdgpu_buffer_rsrc_t ra = buffer(g.a, g.a_bytes), rb = buffer(g.b, g.b_bytes);
 
     // byte offset of this lane's 16 bytes of the first tap and first 32 channels (negative outside the image: only valid
-    // taps are read), and one bit per tap that falls inside
-    int base[TM];
-    unsigned long long mask[TM];
+    // taps are read), and one bit per row and column of taps that falls inside
+    int base[TM], iy[TM], ix[TM];
+    unsigned rows[TM], cols[TM];
 #pragma unroll
     for(int i = 0; i < TM; i++) {
         const int m = m0 + 16 * i + lrow;
         const bool ok = m < c.M;
         const int mm = ok ? m : 0;
-        const int ox = mm % c.OW, t = mm / c.OW;
-        const int oy = t % c.OH, n = t / c.OH;
-        const int iy = oy * k.istep + c.iy0, ix = ox * k.istep + c.ix0;
-        base[i] = ((n * g.IH + iy) * g.IW + ix) * g.lda * 2 + lkq * 16;
-        mask[i] = 0;
-        if(ok)
-            for(int a = 0; a < c.Tr; a++) {
-                const int yy = iy + a * k.tstep;
-                if(yy < 0 || yy >= g.IH)
-                    continue;
-                for(int e = 0; e < c.Ts; e++) {
-                    const int xx = ix + e * k.tstep;
-                    if(xx >= 0 && xx < g.IW)
-                        mask[i] |= 1ull << (a * c.Ts + e);
-                }
-            }
+        const int t = divide(mm, c.by_OW), ox = mm - t * c.OW;
+        const int n = divide(t, c.by_OH), oy = t - n * c.OH;
+        iy[i] = oy * k.istep + c.iy0;
+        ix[i] = ox * k.istep + c.ix0;
+        base[i] = ((n * g.IH + iy[i]) * g.IW + ix[i]) * g.lda * 2 + lkq * 16;
+        rows[i] = cols[i] = 0;
+        iy[i] = ok ? iy[i] : 0x40000000; // (no row of the image)
     }
+#pragma unroll 1
+    for(int a = 0; a < c.Tr; a++)
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+            rows[i] |= (unsigned)(iy[i] + a * k.tstep) < (unsigned)g.IH ? 1u << a : 0u;
+#pragma unroll 1
+    for(int a = 0; a < c.Ts; a++)
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+            cols[i] |= (unsigned)(ix[i] + a * k.tstep) < (unsigned)g.IW ? 1u << a : 0u;
     int qoff[TN];
 #pragma unroll
     for(int t = 0; t < TN; t++) {
@@ -134,70 +199,51 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
 
     // the four channels this lane will finish, and what their epilogue needs: requested now, used after the loop
     const int c4 = lane % (TN * 4), nown = n0 + 4 * c4;
-    float es[4], eb[4], em[4], ev[4]; // scale, bias, mean, variance of a norm to fold; or scale, bias, mean, 1/std of a linked one
-#pragma unroll
-    for(int e = 0; e < 4; e++) {
-        const int n = nown + e < g.N ? nown + e : 0;
-        es[e] = eb[e] = em[e] = ev[e] = 0.0f;
-        if(g.bn_s) {
-            es[e] = g.bn_s[n];
-            eb[e] = g.bn_b[n];
-            em[e] = g.bn_m[n];
-            ev[e] = g.bn_v[n];
-        } else if(SUMS && g.bq_x) {
-            em[e] = g.bq_mean[n];
-            if(g.bq_relu) {
-                es[e] = g.bq_s[n];
-                eb[e] = g.bq_b[n];
-                ev[e] = g.bq_invstd[n];
-            }
-        }
-    }
-
-    const int S32 = (g.C + 31) / 32, T = c.Tr * c.Ts, total = S32 * T;
-    const bool ragged = g.C % 32 != 0;
-    const int s_begin = (int)((long long)ks * total / KS), s_end = (int)((long long)(ks + 1) * total / KS);
-    int s_next = s_begin, tap = total ? s_begin / S32 : 0, c32 = s_begin - tap * S32;
-    int ta = c.Ts ? tap / c.Ts : 0, te = tap - ta * c.Ts;
-    unsigned pv[TM], qv[TN];
-    auto tap_setup = [&]() {
-        const int d = (ta * g.IW + te) * k.tstep * g.lda * 2;
-        const int f = ((c.r0 + ta * k.rstep) * g.S + c.s0 + te * k.rstep) * g.C * 2;
-#pragma unroll
-        for(int i = 0; i < TM; i++)
-            pv[i] = (mask[i] >> tap) & 1 ? (unsigned)(base[i] + d) : OOB;
-#pragma unroll
-        for(int t = 0; t < TN; t++)
-            qv[t] = qoff[t] >= 0 ? (unsigned)(qoff[t] + f) : OOB;
+    auto channels = [&](const float *p) {
+        return __builtin_bit_cast(float4_t, (uint4_t)__builtin_amdgcn_raw_buffer_load_b128(buffer(p, 4u * g.N), 4 * nown, 0, 0));
     };
-    tap_setup();
+    // scale, bias, mean, variance of a norm to fold; or scale, bias, mean, 1/std of a linked one
+    const bool linked = SUMS && g.bq_x;
+    const float4_t es = channels(linked ? g.bq_s : g.bn_s), em = channels(linked ? g.bq_mean : g.bn_m);
+    const float4_t ev = channels(linked ? g.bq_invstd : g.bn_v), eb = channels(linked ? g.bq_b : g.bn_b);
+    half4_t bias = {0, 0, 0, 0};
+    if(g.bias)
+        bias = load4(buffer(g.bias, 2u * g.N), 2 * nown, false, g.N - nown);
+    // and of the first (mostly the only) pixel: what it adds to (beta), its residual, the norm's input
+    const bool vec = ((g.N | g.ldo) & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
+    const bool zvec = vec && (g.ldz & 3) == 0 && ((uintptr_t)g.z & 7) == 0;
+    const bool with_z = g.bn_flags & SAGA_BN_ADD;
+    const __amdgpu_buffer_rsrc_t ro = buffer(g.out, g.out_bytes), rz = buffer(with_z ? g.z : nullptr, g.z_bytes);
+    const __amdgpu_buffer_rsrc_t rwas = buffer(g.beta != 0.0f ? g.out : nullptr, g.out_bytes);
+    half4_t old, zz, xx;
+    auto pixel = [&](int e) { // -1: none
+        const int m = m0 + e / (TN * 4);
+        if(ONE)
+            return e < TM * TN * 64 && m < c.M && nown < g.N ? m : -1;
+        const int t = divide(m, c.by_OW), ox = m - t * c.OW;
+        const int im = divide(t, c.by_OH), oy = t - im * c.OH;
+        return e < TM * TN * 64 && m < c.M && nown < g.N ? (im * g.OH + oy * k.ostep + c.oy) * g.OW + ox * k.ostep + c.ox : -1;
+    };
+    auto request = [&](int pix) {
+        old = load4(rwas, pix >= 0 ? (unsigned)(pix * g.ldo + nown) * 2 : OOB, vec, g.N - nown);
+        zz = load4(rz, pix >= 0 ? (unsigned)(pix * g.ldz + nown) * 2 : OOB, zvec, g.N - nown);
+        if(SUMS) // (its callers have made sure of the alignment)
+            xx = load4(buffer(g.bq_x, g.bq_bytes), pix >= 0 ? (unsigned)(pix * g.bq_ldx + nown) * 2 : OOB, true, 4);
+    };
+    int e = ks * 64 + lane, pix = pixel(e);
+    request(pix);
+
+    const int S32 = k.S32, total = S32 * c.Tr * c.Ts;
+    const bool last_ok = (S32 - 1) * 32 + lkq * 8 < g.C;
+    const int cut = g.C % 32 ? (S32 - 1) * 64 : -1; // where only some of the 32 channels are there
+    const int s_begin = (ks * total) >> k.ks_log2, steps = ((ks * total + total) >> k.ks_log2) - s_begin;
+    int tap = divide(s_begin, k.by_S32), c32 = s_begin - tap * S32;
+    int ta = divide(tap, c.by_Ts), te = tap - ta * c.Ts;
     constexpr int NL = TM + TN; // load instructions, kilobytes of LDS and operands per step
-    char *ring = (char *)smem + wave * (DEPTH * NL * 1024);
-    auto load_step = [&](int u) {
-        const bool live = s_next < s_end && (!ragged || c32 * 32 + lkq * 8 < g.C);
-        char *dst = ring + u * (NL * 1024);
-        const int so = c32 * 64;
-#pragma unroll
-        for(int i = 0; i < TM; i++) {
-            const unsigned v = live ? pv[i] : OOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(dst + i * 1024), 16, v, so, 0, 0);
-        }
-#pragma unroll
-        for(int t = 0; t < TN; t++) {
-            const unsigned v = live ? qv[t] : OOB;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rb, (lds_ptr_t)(dst + (TM + t) * 1024), 16, v, so, 0, 0);
-        }
-        if(++c32 == S32) {
-            c32 = 0;
-            tap++;
-            if(++te == c.Ts) {
-                te = 0;
-                ta++;
-            }
-            if(s_next + 1 < s_end)
-                tap_setup();
-        }
-        s_next++;
+    char *ring = (char *)smem + wave * wave_lds<TM, TN, DEPTH>();
+    const unsigned at = (unsigned)(uintptr_t)(lds_ptr_t)ring + row * 64 + (kq ^ ((row >> 2) & 3)) * 16;
+    auto load_to_lds = [](__amdgpu_buffer_rsrc_t r, char *dst, unsigned v, int at) {
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, v, at, 0, 0);
     };
     float4_t acc[TM][TN];
 #pragma unroll
@@ -205,131 +251,148 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
 #pragma unroll
         for(int t = 0; t < TN; t++)
             acc[i][t] = float4_t{0, 0, 0, 0};
-    if(g.bias && ks == 0) // one of the wavefronts that share the reduction starts from it
+    int fill = 0, drain = 0;
+    auto consume = [&]() {
+        half8_t f[NL];
+        const unsigned from = at + drain;
+        if constexpr(NL > 0) f[0] = lds_read<0 * 1024>(from);
+        if constexpr(NL > 1) f[1] = lds_read<1 * 1024>(from);
+        if constexpr(NL > 2) f[2] = lds_read<2 * 1024>(from);
+        if constexpr(NL > 3) f[3] = lds_read<3 * 1024>(from);
+        if constexpr(NL > 4) f[4] = lds_read<4 * 1024>(from);
+        if constexpr(NL > 5) f[5] = lds_read<5 * 1024>(from);
+        if constexpr(NL > 6) f[6] = lds_read<6 * 1024>(from);
+        if constexpr(NL > 7) f[7] = lds_read<7 * 1024>(from);
+        static_assert(NL <= 8, "operands");
+        drain = drain == (DEPTH - 1) * NL * 1024 ? 0 : drain + NL * 1024;
+        lds_wait(f); // before the next step loads into this slot
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+#pragma unroll
+            for(int t = 0; t < TN; t++)
+                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[TM + t], f[i], acc[i][t], 0, 0, 0);
+    };
+    int s = 0; // steps requested
+#pragma unroll 1
+    while(s < steps) {
+        const int d = (ta * g.IW + te) * k.tstep * g.lda * 2;
+        const int f = ((c.r0 + ta * k.rstep) * g.S + c.s0 + te * k.rstep) * g.C * 2;
+        unsigned pv[TM], qv[TN];
+#pragma unroll
+        for(int i = 0; i < TM; i++)
+            pv[i] = (rows[i] >> ta) & (cols[i] >> te) & 1 ? (unsigned)(base[i] + d) : OOB;
 #pragma unroll
         for(int t = 0; t < TN; t++)
-#pragma unroll
-            for(int v = 0; v < 4; v++) {
-                const int n = n0 + 16 * t + 4 * kq + v;
-                const float b = n < g.N ? (float)g.bias[n] : 0.0f;
+            qv[t] = qoff[t] >= 0 ? (unsigned)(qoff[t] + f) : OOB;
+        const int until = std::min(s + S32 - c32, steps);
+        int so = c32 * 64;
+#pragma unroll 1
+        do {
+            if(so == cut) { // (the tap's last step)
 #pragma unroll
                 for(int i = 0; i < TM; i++)
-                    acc[i][t][v] = b;
-            }
-#pragma unroll
-    for(int u = 0; u < DEPTH - 1; u++)
-        load_step(u);
-    const unsigned at = (unsigned)(uintptr_t)(lds_ptr_t)ring + row * 64 + (kq ^ ((row >> 2) & 3)) * 16;
-    auto read_step = [&](auto u, half8_t(&f)[NL]) {
-        constexpr int U = decltype(u)::value;
-        if constexpr(NL > 0) f[0] = lds_read<(U * NL + 0) * 1024>(at);
-        if constexpr(NL > 1) f[1] = lds_read<(U * NL + 1) * 1024>(at);
-        if constexpr(NL > 2) f[2] = lds_read<(U * NL + 2) * 1024>(at);
-        if constexpr(NL > 3) f[3] = lds_read<(U * NL + 3) * 1024>(at);
-        if constexpr(NL > 4) f[4] = lds_read<(U * NL + 4) * 1024>(at);
-        if constexpr(NL > 5) f[5] = lds_read<(U * NL + 5) * 1024>(at);
-        if constexpr(NL > 6) f[6] = lds_read<(U * NL + 6) * 1024>(at);
-        if constexpr(NL > 7) f[7] = lds_read<(U * NL + 7) * 1024>(at);
-        static_assert(NL <= 8, "operands");
-    };
-    auto step = [&](auto u, int s) {
-        constexpr int U = decltype(u)::value;
-        load_step((U + DEPTH - 1) % DEPTH); // into the slot that step s - 1 was read from
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * NL) : "memory");
-        half8_t f[NL];
-        read_step(u, f);
-        lds_wait(f);
-        if(s < s_end) {
-#pragma unroll
-            for(int i = 0; i < TM; i++)
+                    pv[i] = last_ok ? pv[i] : OOB;
 #pragma unroll
                 for(int t = 0; t < TN; t++)
-                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[TM + t], f[i], acc[i][t], 0, 0, 0);
+                    qv[t] = last_ok ? qv[t] : OOB;
+            }
+#pragma unroll
+            for(int i = 0; i < TM; i++)
+                load_to_lds(ra, ring + fill + i * 1024, pv[i], so);
+#pragma unroll
+            for(int t = 0; t < TN; t++)
+                load_to_lds(rb, ring + fill + (TM + t) * 1024, qv[t], so);
+            fill = fill == (DEPTH - 1) * NL * 1024 ? 0 : fill + NL * 1024;
+            so += 64;
+            if(s >= DEPTH - 1) {
+                asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * NL) : "memory");
+                consume();
+            }
+        } while(++s < until);
+        c32 = 0;
+        if(++te == c.Ts) {
+            te = 0;
+            ta++;
         }
-    };
-    for(int s = s_begin; s < s_end; s += DEPTH) {
-        step(std::integral_constant<int, 0>(), s);
-        if constexpr(DEPTH > 1) step(std::integral_constant<int, 1 % DEPTH>(), s + 1);
-        if constexpr(DEPTH > 2) step(std::integral_constant<int, 2 % DEPTH>(), s + 2);
-        if constexpr(DEPTH > 3) step(std::integral_constant<int, 3 % DEPTH>(), s + 3);
-        if constexpr(DEPTH > 4) step(std::integral_constant<int, 4 % DEPTH>(), s + 4);
-        if constexpr(DEPTH > 5) step(std::integral_constant<int, 5 % DEPTH>(), s + 5);
-        if constexpr(DEPTH > 6) step(std::integral_constant<int, 6 % DEPTH>(), s + 6);
-        if constexpr(DEPTH > 7) step(std::integral_constant<int, 7 % DEPTH>(), s + 7);
-        static_assert(DEPTH <= 8, "steps");
     }
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // the ring's memory is reused, or the block ends
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll 1
+    for(int u = std::min(steps, DEPTH - 1); u > 0; u--)
+        consume();
 
     // acc[i][t][v]: pixel 16*i + lane%16, channel 16*t + 4*(lane/16) + v
-    __syncthreads();
-    constexpr int PITCH = TN * 16 + 4, TILE = TM * 16 * PITCH; // floats; rows of a tile fall into different banks
+    constexpr int PITCH = TN * 16 + 4, WAVE = wave_lds<TM, TN, DEPTH>() / 4; // floats; rows of a tile fall into different banks
 #pragma unroll
     for(int i = 0; i < TM; i++)
 #pragma unroll
         for(int t = 0; t < TN; t++)
-            *(float4_t *)&smem[wave * TILE + (16 * i + row) * PITCH + 16 * t + 4 * kq] = acc[i][t];
-    __syncthreads();
-    float sc[4], sh[4];
+            *(float4_t *)&smem[wave * WAVE + (16 * i + row) * PITCH + 16 * t + 4 * kq] = acc[i][t];
+    float4_t sc, sh;
 #pragma unroll
-    for(int e = 0; e < 4; e++) {
-        sc[e] = es[e] * (SUMS && g.bq_x ? ev[e] : rsqrtf(ev[e] + g.bn_eps));
-        sh[e] = SUMS && g.bq_x ? __builtin_fmaf(-em[e], sc[e], eb[e]) : eb[e] - em[e] * sc[e]; // (the forward's own expressions)
+    for(int q = 0; q < 4; q++) {
+        sc[q] = es[q] * (linked ? ev[q] : rsqrtf(ev[q] + g.bn_eps));
+        sh[q] = linked ? __builtin_fmaf(-em[q], sc[q], eb[q]) : eb[q] - em[q] * sc[q]; // (the forward's own expressions)
     }
+    __syncthreads();
     float s1[4] = {0, 0, 0, 0}, s2[4] = {0, 0, 0, 0}; // of this lane's channels: statistics, or sums of a norm's backward
-    const bool vec = nown + 4 <= g.N && g.ldo % 4 == 0 && ((uintptr_t)g.out & 7) == 0;
-    const bool zvec = vec && g.ldz % 4 == 0 && ((uintptr_t)g.z & 7) == 0;
-    for(int e = ks * 64 + lane; e < TM * TN * 64; e += KS * 64) {
-        const int px = e / (TN * 4), m = m0 + px;
-        const float *s = smem + wm * KS * TILE + px * PITCH + 4 * c4;
-        float4_t v = *(const float4_t *)s;
-        for(int w = 1; w < KS; w++)
-            v += *(const float4_t *)(s + w * TILE);
-        if(m >= c.M || nown >= g.N)
-            continue;
-        const int ox = m % c.OW, t = m / c.OW;
-        const int oy = t % c.OH, im = t / c.OH;
-        const long long pix = ((long long)im * g.OH + oy * k.ostep + c.oy) * g.OW + ox * k.ostep + c.ox;
-        half_t *o = g.out + pix * g.ldo + nown;
-        const half_t *z = g.bn_flags & SAGA_BN_ADD ? g.z + pix * g.ldz + nown : nullptr;
-        half4_t old = {0, 0, 0, 0}, zz = {0, 0, 0, 0}, xx = {0, 0, 0, 0}, r = {0, 0, 0, 0};
-        if(g.beta != 0.0f && vec)
-            old = *(const half4_t *)o;
-        if(z && zvec)
-            zz = *(const half4_t *)z;
-        if(SUMS && g.bq_x) // (its callers have made sure of the alignment)
-            xx = *(const half4_t *)(g.bq_x + pix * g.bq_ldx + nown);
+#pragma unroll 1
+    for(; e < TM * TN * 64;) {
+        const float *part = smem + wm * KS * WAVE + e / (TN * 4) * PITCH + 4 * c4;
+        float4_t v = *(const float4_t *)part;
+        if(KS >= 2)
+            v += *(const float4_t *)(part + WAVE);
+        if(KS >= 4) {
+            const float4_t v2 = *(const float4_t *)(part + 2 * WAVE), v3 = *(const float4_t *)(part + 3 * WAVE);
+            v = v + v2 + v3;
+        }
+        if(KS >= 8) {
+            const float4_t v4 = *(const float4_t *)(part + 4 * WAVE), v5 = *(const float4_t *)(part + 5 * WAVE);
+            const float4_t v6 = *(const float4_t *)(part + 6 * WAVE), v7 = *(const float4_t *)(part + 7 * WAVE);
+            v = v + v4 + v5 + v6 + v7;
+        }
+        const half4_t was = old, res = zz, in = xx;
+        const int here = pix;
+        e += KS * 64;
+        if constexpr(TM * TN > 1) {
+            pix = pixel(e);
+            request(pix);
+        }
+        v *= g.alpha;
+        if(g.bias)
+            v += __builtin_convertvector(bias, float4_t);
+        if(g.beta != 0.0f)
+            v += g.beta * __builtin_convertvector(was, float4_t);
+        if(g.bn_s) {
 #pragma unroll
-        for(int q = 0; q < 4; q++) {
-            if(nown + q >= g.N)
-                break;
-            float f = g.alpha * v[q];
-            if(g.beta != 0.0f)
-                f += g.beta * (float)(vec ? old[q] : o[q]);
-            if(g.bn_s) {
-                f = __builtin_fmaf(f, sc[q], sh[q]);
-                if(z)
-                    f += (float)(zvec ? zz[q] : z[q]);
-                if(g.bn_flags & SAGA_BN_RELU)
-                    f = f != f ? f : fmaxf(f, 0.0f);
-            }
-            r[q] = (half_t)f;
-            if(SUMS && g.bq_x) {
-                const float xf = (float)xx[q];
-                if(g.bq_relu && !((float)(half_t)__builtin_fmaf(xf, sc[q], sh[q]) > 0.0f))
-                    r[q] = (half_t)0;
-                s1[q] += (float)r[q];
-                s2[q] += (float)r[q] * (xf - em[q]);
-            } else if(SUMS) {
-                s1[q] += (float)r[q];
-                s2[q] += (float)r[q] * (float)r[q];
+            for(int q = 0; q < 4; q++)
+                v[q] = __builtin_fmaf(v[q], sc[q], sh[q]);
+            if(with_z)
+                v += __builtin_convertvector(res, float4_t);
+            if(g.bn_flags & SAGA_BN_RELU)
+#pragma unroll
+                for(int q = 0; q < 4; q++)
+                    v[q] = v[q] != v[q] ? v[q] : fmaxf(v[q], 0.0f);
+        }
+        half4_t r = __builtin_convertvector(v, half4_t);
+        if(SUMS && here >= 0) {
+            if(linked) {
+#pragma unroll
+                for(int q = 0; q < 4; q++) {
+                    const float xf = (float)in[q];
+                    if(g.bq_relu && !((float)(half_t)__builtin_fmaf(xf, sc[q], sh[q]) > 0.0f))
+                        r[q] = (half_t)0;
+                    s1[q] += (float)r[q];
+                    s2[q] += (float)r[q] * (xf - em[q]);
+                }
+            } else {
+#pragma unroll
+                for(int q = 0; q < 4; q++) {
+                    s1[q] += (float)r[q];
+                    s2[q] += (float)r[q] * (float)r[q];
+                }
             }
         }
-        if(vec) {
-            *(half4_t *)o = r;
-        } else {
-            for(int q = 0; q < 4 && nown + q < g.N; q++)
-                o[q] = r[q];
-        }
+        store4(ro, here >= 0 ? (unsigned)(here * g.ldo + nown) * 2 : OOB, vec, g.N - nown, r);
     }
     if constexpr(!SUMS)
         return;
@@ -351,7 +414,7 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
     __syncthreads();
     if(tid < TN * 32 && n0 + tid / 2 < g.N) {
         float s = 0.0f;
-        for(int w = 0; w < KS * WM; w++)
+        for(int w = 0; w < KS * k.WM; w++)
             s += smem[w * TN * 32 + tid];
         g.sums[((long long)(c.row0 + bm) * g.N + n0) * 2 + tid] = s;
     }
@@ -445,8 +508,11 @@ bool classes(Args &a)
         axis(c.ox, g.S, c.s0, c.Ts, c.ix0);
         if(!c.Tr || !c.Ts)
             c.Tr = c.Ts = 0;
-        if(c.Tr * c.Ts > 64)
+        if(c.Tr > 31 || c.Ts > 31)
             return false;
+        c.by_OH = div_by(c.OH > 0 ? c.OH : 1);
+        c.by_OW = div_by(c.OW > 0 ? c.OW : 1);
+        c.by_Ts = div_by(c.Ts ? c.Ts : 1);
         c.M = g.batch * c.OH * c.OW;
     }
     return true;
@@ -458,12 +524,12 @@ template <bool SUMS, typename A> int launch_as(const A &k, const Config &cf, hip
 #define GO(TM, TN, DEPTH, MAXW)                                                                                             \
     do {                                                                                                                    \
         auto kern = stream_f16_k<TM, TN, DEPTH, MAXW, SUMS, A>;                                                                  \
-        constexpr size_t wave_lds = std::max(DEPTH * (TM + TN) * 1024, TM * 16 * (TN * 16 + 4) * 4);                         \
+        constexpr size_t lds = wave_lds<TM, TN, DEPTH>();                                                                    \
         static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,   \
-                                                           MAXW * wave_lds);                                                \
+                                                           MAXW * lds);                                                     \
         if(attr != hipSuccess)                                                                                              \
             return (int)attr;                                                                                               \
-        kern<<<k.blocks, threads, wave_lds *(threads / 64), st>>>(k);                                                       \
+        kern<<<k.blocks, threads, lds *(threads / 64), st>>>(k);                                                       \
     } while(0)
     if(cf.tm == 4 && cf.tn == 4)
         GO(4, 4, 3, 4);
@@ -494,13 +560,25 @@ int stream_f16_launch(const StreamF16 &g, hipStream_t st, int *sum_rows)
 {
     Args k = {};
     k.g = g;
+    const long long out_rows = (long long)g.batch * g.OH * g.OW;
+    const long long widest = out_rows * std::max({g.ldo, g.bn_flags & SAGA_BN_ADD ? g.ldz : 0, g.bq_x ? g.bq_ldx : 0}) * 2;
+    if(widest >= OOB)
+        return SAGA_HIP_EUNSUPPORTED;
+    k.g.out_bytes = (unsigned)(out_rows * g.ldo * 2);
+    k.g.z_bytes = g.bn_flags & SAGA_BN_ADD ? (unsigned)(out_rows * g.ldz * 2) : 0;
+    k.g.bq_bytes = g.bq_x ? (unsigned)(out_rows * g.bq_ldx * 2) : 0;
     if(g.C % 8 || g.lda % 8 || !g.a_bytes || !g.b_bytes || !classes(k))
         return SAGA_HIP_EUNSUPPORTED;
     const Config cf = config_of(g);
     if(!cf.tm)
         return SAGA_HIP_EUNSUPPORTED;
-    k.KS = cf.ks;
+    while((1 << k.ks_log2) < cf.ks)
+        k.ks_log2++;
+    k.WM = cf.wm;
+    k.S32 = (g.C + 31) / 32;
+    k.by_S32 = div_by(k.S32);
     k.nblk_q = (g.N + 16 * cf.tn - 1) / (16 * cf.tn);
+    k.by_q = div_by(k.nblk_q);
     // the larger operand is the one that each die should fetch once
     k.q_outer = (long long)g.N * g.R * g.S > (long long)g.batch * g.IH * g.IW;
     long long blocks = 0;
@@ -508,7 +586,9 @@ int stream_f16_launch(const StreamF16 &g, hipStream_t st, int *sum_rows)
     for(int i = 0; i < k.nclasses; i++) {
         k.cls[i].block0 = (int)blocks;
         k.cls[i].row0 = rows;
-        rows += (k.cls[i].M + 16 * cf.tm * cf.wm - 1) / (16 * cf.tm * cf.wm);
+        k.cls[i].nm = (k.cls[i].M + 16 * cf.tm * cf.wm - 1) / (16 * cf.tm * cf.wm);
+        k.cls[i].by_nm = div_by(k.cls[i].nm > 0 ? k.cls[i].nm : 1);
+        rows += k.cls[i].nm;
         blocks = (long long)rows * k.nblk_q;
     }
     if(sum_rows)

@@ -26,6 +26,7 @@ struct StreamF16 {
     const half_t *bq_x;
     int bq_ldx, bq_relu;
     const float *bq_mean, *bq_s, *bq_invstd, *bq_b;
+    unsigned out_bytes, z_bytes, bq_bytes; // (set by the launch)
 };
 
 // Whether this kernel is the faster one for the problem.
