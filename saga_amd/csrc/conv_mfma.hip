@@ -3689,12 +3689,14 @@ static int tile_override()
     return v;
 }
 
+} // namespace
+
 // How many blocks share the reduction of a tile (1: none), by the number of tiles and slices of 32.  Fitted to measured
 // times: a slice takes a block 0.36 us (0.24 with 64 channels), a shared launch and its second kernel cost 9 us more than a plain one, and writing
 // and reading the sums of a 256x128 tile 33 ns; more blocks than CUs only add sums.  (us, alone -> shared by k:
 // 3x3 1024->1024 at 21x21 90 -> 28 k=10; 3x3 1024->512 at 42x42 96 -> 35 k=8; 3x3 512->512 at 64x7x7 50 -> 34 k=4;
 // at 128x7x7 52 -> 47 k=2; 1x1 2048->512 at 23x7x7 23 -> 18 k=3; 3x3 256->256 at 64x14x14 31 -> 35 k=2, not taken.)
-static int split_rule(int64_t tiles, int bn, int slices)
+int conv_tile_split(int64_t tiles, int bn, int slices)
 {
     const double slice = bn == 64 ? 0.24 : 0.36;
     double best = 0.93 * (4 + slice * slices);
@@ -3709,6 +3711,8 @@ static int split_rule(int64_t tiles, int bn, int slices)
     return k;
 }
 
+namespace {
+
 template <bool BWD> static int split_of(const GatherArgs &g, int64_t tiles, int active)
 {
     const bool vec_ok = (g.ldo & 7) == 0 && (g.Ngemm & 7) == 0 && ((uintptr_t)g.out & 15) == 0;
@@ -3716,7 +3720,7 @@ template <bool BWD> static int split_of(const GatherArgs &g, int64_t tiles, int 
         return 1;
     const int sdiv = BWD ? g.stride : 1;
     const int slices = ((g.R + sdiv - 1) / sdiv) * ((g.S + sdiv - 1) / sdiv) * ((g.Cred + 31) / 32);
-    const int bn = g.Ngemm <= 64 ? 64 : 128, k = split_rule(tiles, bn, slices);
+    const int bn = g.Ngemm <= 64 ? 64 : 128, k = conv_tile_split(tiles, bn, slices);
     const int64_t tile_bytes = 256ll * bn * 4;
     return k > 1 && (int64_t)g.part_bytes >= tiles * k * tile_bytes ? k : 1;
 }
@@ -4005,7 +4009,7 @@ static size_t split_bytes(bool bwd, const ConvGeom &g)
     const int bn = n <= 64 ? 64 : 128;
     const int64_t tiles = ((Mc + 255) / 256) * ((n + bn - 1) / bn) * s * s;
     const int slices = ((g.R + s - 1) / s) * ((g.S + s - 1) / s) * ((red + 31) / 32);
-    const int k = split_rule(tiles, bn, slices);
+    const int k = conv_tile_split(tiles, bn, slices);
     return k > 1 ? (size_t)(tiles * k * 256 * bn * 4) : 0;
 }
 

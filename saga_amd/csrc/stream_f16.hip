@@ -424,53 +424,72 @@ struct Config {
     int tm, tn, ks, wm;
 };
 
-// Tile (16*tm pixels x 16*tn channels per wavefront) and wavefronts along the reduction (ks) and the pixels (wm) for a
-// problem of `tiles` 16x16 tiles and `steps` reduction steps of 32; tm = 0: a matter for the tiled kernels.  Small tiles
-// fill the chip, larger ones fetch less per multiplication, and a wavefront should walk more steps than its ring holds.
-// Measured (us; tm,tn,ks,wm; the tiled kernel last; launch included):
-//   1x14x14 3x3 256->256    tiles  208 steps  72   1,1,4,1  7.4  1,1,8,1  7.6  2,2,8,1  9.2   28
-//   1x7x7   3x3 512->512            128       144  1,1,8,1  8.5  1,1,4,1  9.1  2,2,8,1 11.2   47
-//   1x28x28 1x1 512->128            392        16  1,1,2,2  4.8  2,2,4,1  5.1  1,1,4,1  5.6    8.9
-//   1x14x14 1x1 256->1024           832         8  1,1,1,4  4.9  2,2,4,1  5.3                  6.7
-//   1x56x56 3x3 64->64              784        18  2,2,4,1  7.1  2,2,8,1  7.4  1,1,1,4  7.7   11
-//   4x14x14 3x3 256->256            784        72  2,2,8,1  9.8  2,2,4,1 10.1  4,2,8,1 11.5   28
-//   4x28x28 3x3 128->128           1568        36  2,2,4,1 10.1  4,2,8,1 10.4  2,2,2,2 10.7   18
-//   16x7x7  3x3 512->512           1568       144  4,2,8,1 18.1  2,2,4,1 21.5  2,2,2,2 22.9   48
-//   16x14x14 1x1 1024->256         3136        32  2,2,2,2 11.0  4,4,4,1 11.7  4,2,4,1 11.9   14
-//   16x14x14 3x3 256->256          3136        72  4,4,4,1 18.1  2,2,2,2 18.4  4,2,4,1 20.0   28
-//   32x14x14 3x3 256->256          6272        72  4,4,2,2 27.9                               28.5
-//   4x14x14 1x1 256->1024          3136         8  2,2,2,2  7.2                                6.9
-// Beyond these the sums of a tile are better shared by several blocks of the tiled kernel (42x42 3x3 1024->512: 35 against
-// 48 us here and 96 alone).
-Config choose(long long tiles, long long steps, int N)
+// Tile (16*tm pixels x 16*tn channels per wavefront) and wavefronts along the reduction (ks) and the pixels (wm) by what
+// they cost: start + steps of a wavefront * (step + more * rounds) + round * rounds, where a round is a block on every CU.
+// The numbers are fitted to 420 problems (1 to 90 images of 7x7 to 150x150 pixels, 8 to 2048 channels either way, filters
+// of 1 to 5) at each of the tiles, launched one behind the other with filters that are not in the cache: 8 % off on
+// average, and the choice 4 % slower than the best of everything at each problem (lines drawn by tiles and steps, which
+// stood here before: 16 %).  us, before -> now, of which the tiled kernels where they took it:
+//   1x56x56 3x3 64->64 and below  as before              23x13x13 3x3 256->256   27.1 -> 15.3 (tiled before)
+//   2x28x28 1x1 128->512     6.0 -> 5.0 (tiled before)  16x28x28 3x3 128->128   18.8 -> 14.1 (tiled before)
+//   1x28x28 1x1 128->512     5.8 -> 4.1 (tiled before)  512x8x8  3x3 64->64     18.6 -> 10.7 (tiled before)
+//   4x14x14 3x3 512->512 /2 12.7 -> 9.9                 49x30x30 5x5 64->16     23.1 -> 15.3 (tiled before)
+struct Cost {
+    Config c;
+    float start, step, more, round;
+};
+constexpr Cost COSTS[] = {
+    {{1, 1, 1, 4}, 3.48f, 0.053f, 0.046f, 0.31f},
+    {{1, 1, 4, 1}, 3.33f, 0.028f, 0.079f, 0.29f},
+    {{1, 1, 8, 1}, 1.97f, 0.046f, 0.174f, 1.70f},
+    {{2, 2, 2, 2}, 3.63f, 0.048f, 0.141f, 0.66f},
+    {{2, 2, 4, 1}, 3.31f, 0.054f, 0.167f, 0.48f},
+    {{4, 2, 2, 2}, 4.85f, -0.057f, 0.345f, 0.46f},
+    {{4, 2, 8, 1}, 1.58f, 0.051f, 0.572f, 2.63f},
+    {{4, 4, 2, 2}, 2.09f, -0.083f, 0.463f, 5.29f},
+    {{4, 4, 4, 1}, 1.49f, -0.008f, 0.439f, 4.34f},
+};
+
+int split_over(long long a, long long b) { return (int)((a + b - 1) / b); }
+
+// the tiled kernels: 256 pixels x 64 or 128 channels per block, the reduction of a tile split over k blocks where that pays
+float tiled_us(long long pixels, int steps, int N)
 {
-    if(tiles > 3600 || (steps >= 200 && tiles >= 1500) || (steps >= 128 && tiles > 3300))
-        return {0, 0, 0, 0};
-    if(tiles <= 640) {
-        if(steps < 8)
-            return {0, 0, 0, 0};
-        return steps >= 100 ? Config{1, 1, 8, 1} : steps >= 24 ? Config{1, 1, 4, 1} : steps >= 12 ? Config{1, 1, 2, 2} : Config{1, 1, 1, 4};
+    const int bn = N <= 64 ? 64 : 128;
+    const long long tiles = (pixels + 255) / 256 * split_over(N, bn);
+    const int k = N % 8 == 0 ? conv_tile_split(tiles, bn, steps) : 1, L = split_over(steps, k), rounds = split_over(tiles, 256);
+    if(k > 1)
+        return 13.3f + 0.47f * L + (bn == 64 ? 1.0f : 8.0f) * (tiles * k) / 256.0f;
+    if(bn == 64)
+        return 4.1f + L * (0.376f + 0.306f * (rounds - 1)) + 0.8f * tiles / 256.0f;
+    return 4.7f + L * (0.367f + 0.485f * (rounds - 1)) + 2.4f * tiles / 256.0f;
+}
+
+// tm = 0: a matter for the tiled kernels
+Config choose(long long pixels, int steps, int N)
+{
+    Config best = {0, 0, 0, 0};
+    float least = tiled_us(pixels, steps, N);
+    for(const Cost &o : COSTS) {
+        const long long blocks = split_over(pixels, 16 * o.c.tm * o.c.wm) * (long long)split_over(N, 16 * o.c.tn);
+        if(blocks > 640 || steps < o.c.ks) // (beyond what the numbers were fitted to)
+            continue;
+        const int rounds = split_over(blocks, 256);
+        const float us = o.start + split_over(steps, o.c.ks) * (o.step + o.more * rounds) + o.round * rounds;
+        if(us < least) {
+            least = us;
+            best = o.c;
+        }
     }
-    if(tiles <= 2048) {
-        if(steps < 12)
-            return steps >= 8 && tiles <= 900 ? Config{1, 1, 1, 4} : Config{0, 0, 0, 0};
-        if(steps >= 100 && tiles > 1200)
-            return {4, 2, 8, 1};
-        return {2, 2, steps >= 64 && tiles <= 900 ? 8 : 4, 1};
-    }
-    // (wide tiles only for channels that fill them: 5x5 160->32 at 57x17x17 25 against 51 us, the tiled kernel 27.  Its tiles of
-    // 64 channels are enough blocks for narrow layers: 5x5 64->16 at 49x30x30 24 against 29, 48->40 at 7x50x50 26 against 30)
-    if(steps >= 64)
-        return N > 32 ? Config{4, 4, 4, 1} : Config{4, 2, 4, 1};
-    return steps >= 16 && N > (steps >= 32 ? 64 : 16) ? Config{2, 2, 2, 2} : Config{0, 0, 0, 0};
+    return best;
 }
 
 Config config_of(const StreamF16 &g)
 {
     const int s = g.bwd ? g.stride : 1;
     const long long pixels = (long long)g.batch * ((g.OH + s - 1) / s) * ((g.OW + s - 1) / s) * s * s;
-    const long long taps = ((g.R + s - 1) / s) * ((g.S + s - 1) / s);
-    return choose((pixels + 15) / 16 * ((g.N + 15) / 16), taps * ((g.C + 31) / 32), g.N);
+    const int taps = ((g.R + s - 1) / s) * ((g.S + s - 1) / s);
+    return choose(pixels, taps * ((g.C + 31) / 32), g.N);
 }
 
 int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }

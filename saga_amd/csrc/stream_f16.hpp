@@ -29,6 +29,8 @@ struct StreamF16 {
     unsigned out_bytes, z_bytes, bq_bytes; // (set by the launch)
 };
 
+// Blocks that share the reduction of each of `tiles` tiles of the tiled kernels (256 pixels x bn channels); conv_mfma.hip.
+int conv_tile_split(int64_t tiles, int bn, int slices);
 // Whether this kernel is the faster one for the problem.
 bool stream_f16_wanted(const StreamF16 &g);
 // Rows of sums a launch writes at most (by batch, N, C, OH, OW, R, S, stride and bwd); 0 if it is not wanted.
