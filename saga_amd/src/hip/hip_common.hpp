@@ -404,11 +404,12 @@ public:
     void dropGraphs();
     void runOpsGraphed();
 
-    // ---- the side stream.  Per operation: where it runs, the first operation on the program's own stream that needs its
-    // results (or overwrites what it reads), and the events between the two streams (see planSide)
+    // ---- the side stream.  Per operation: where it runs, the last operation on the program's own stream that it has to run
+    // behind (-1: it may run from the start of the step), the first one there that needs its results (or overwrites what it
+    // reads), and the events between the two streams (see planSide)
     struct Side {
         bool on = false;
-        int join = 0;
+        int after = -1, join = 0;
         hipEvent_t fork = nullptr;      // the side stream waits for this one before the operation
         hipEvent_t done = nullptr;      // recorded behind it, if an operation of the main stream waits
         hipEvent_t reached = nullptr;   // main stream: recorded behind the operation, for forks

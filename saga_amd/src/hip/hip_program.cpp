@@ -270,13 +270,15 @@ void HipContext::planMemory()
             touch(ops[i]->getInputs(), true);
             touch(ops[i]->getOutputs(), false);
         }
-        // what an operation on the side stream touches stays in use until the main stream has waited for it
+        // An operation on the side stream runs at any time between the operation of the main stream that it waits for and the
+        // one that waits for it: what it touches is in use all that while.
         const auto &side = m_programs[pi]->m_side;
         for(size_t i = 0; i < side.size(); i++)
             if(side[i].on)
                 for(const auto &list : {ops[i]->getInputs(), ops[i]->getOutputs()})
                     for(const auto &a : list) {
                         Range &r = seen[a.second->m_storage.get()];
+                        r.first = std::min(r.first, side[i].after + 1);
                         r.last = std::max(r.last, std::min(side[i].join, (int)ops.size() - 1));
                     }
         for(const auto &kv : seen) {
@@ -887,8 +889,8 @@ void HipProgram::runOpsGraphed()
 //
 // An event orders each such operation behind the last one of the main stream that writes what it reads, and the first
 // operation of the main stream that reads its results, or overwrites what it reads, behind it.  One with nothing left to run
-// beside it stays on the main stream: an edge between the streams costs more than a launch.  Storages that it touches keep
-// their memory until the edge back (planMemory); a program whose operations would hold more than an eighth of the GPU's
+// beside it stays on the main stream: an edge between the streams costs more than a launch.  Storages that it touches have
+// their memory to themselves from the one edge to the other (planMemory); a program whose operations would hold more than an eighth of the GPU's
 // memory that way stays on one stream.
 void HipProgram::planSide()
 {
@@ -959,6 +961,7 @@ void HipProgram::planSide()
         int w = i - 1;
         while(w >= 0 && (side[w].on || !ordered(w, i)))
             w--;
+        side[i].after = w;
         side[i].fork = event(w >= 0 ? side[w].reached : m_side_start);
         last[side[i].join] = i;
     }

@@ -1,0 +1,68 @@
+"""What the engine plans for a program, looked at without a GPU: which memory the operations share, and in which order the two
+streams run those that do."""
+import numpy as np
+import pytest
+
+from saga_amd import api as S
+from saga_amd import networks as N
+from tests import stub_gpu
+from tests.stub_gpu import on_stub
+
+
+def behind_resize(net, image):
+    """The training graph of `net` behind a byte image that is converted and resized to the network's input."""
+    g = S.Graph()
+    pixels = S.Tensor.placeholder(S.U8, [net.batch, 3, image, image], "pixels")
+    c = g.add_node("convert", {"x": pixels}, {"scale": 1 / 255.0, "datatype": net.dtype})
+    c = g.add_node("spatialtransform", {"x": c.y()}, {"height": net.in_shape[1], "width": net.in_shape[2]})
+    t = {net.input: c.y()}
+    for name, a in net.params.items():
+        norm = name.endswith(("-s", "-m", "-v")) or name[:-2] + "-s" in net.params
+        t[name] = S.Tensor.from_numpy(a.astype(N.np_dtype(S.FLOAT if norm else net.dtype)), name=name)
+    for n in net.nodes:
+        t[n["out"]] = g.add_node(n["type"], {k: t[v] for k, v in n["in"].items()}, n["attrs"], n["name"]).y()
+    g.add_node("catclassifier", {"x": t[net.output]})
+    return g
+
+
+TRAINED = {
+    "resnet20": lambda: N.resnet20(64),
+    "resnet20 f32": lambda: N.resnet20(64, dtype=S.FLOAT),
+    "resnet50": lambda: N.resnet50(16, image=128),
+    "lenet": lambda: N.lenet(64),
+    "unet": lambda: N.unet(2, image=64),
+}
+
+
+@pytest.mark.parametrize("name", TRAINED)
+@on_stub
+def test_operations_that_share_memory_are_ordered(name):
+    net = TRAINED[name]()
+    if name == "unet":  # a scalar loss
+        b = N.Builder(net, 99)
+        b.shape[net.output] = (net.classes, 64, 64)
+        net.output = b.fc(b.pool("avgpool", net.output, global_=True), "cls", net.classes)
+    ctx = S.Context()
+    g, _ = N.build_graph(net, np.zeros((net.batch,) + tuple(net.in_shape), np.float32))
+    p = ctx.create_program(g, net.batch, training=True)
+    p.finalize()
+    ops = stub_gpu.plan(p)
+    assert any(op["side"] for op in ops)
+    bad = stub_gpu.unordered(ops)
+    assert not bad, bad[:8]
+
+
+@pytest.mark.parametrize("name,image", [("resnet20", 512), ("resnet50", 1024)])
+@on_stub
+def test_operations_in_front_of_the_first_convolution_are_ordered(name, image):
+    """Their tensors are large and done with early: what the side stream writes from the start of the step must stay out of
+    that memory."""
+    net = TRAINED[name]()
+    ctx = S.Context()
+    p = ctx.create_program(behind_resize(net, image), net.batch, training=True)
+    p.finalize()
+    ops = stub_gpu.plan(p)
+    kinds = [op["kind"] for op in ops]
+    assert kinds[:2] == ["convert", "spatialtransform"] and "filtertranspose" in [op["kind"] for op in ops if op["side"]]
+    bad = stub_gpu.unordered(ops)
+    assert not bad, bad[:8]
