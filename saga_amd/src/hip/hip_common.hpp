@@ -222,7 +222,8 @@ struct HipProgram;
 void link_bn_backward(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 // hip_ops.cpp: a strided 1x1 backward data that writes a fan-in gradient first is moved behind the last writer
 void reorder_sparse_first_writers(std::vector<std::shared_ptr<HipOperation>> &ops);
-void drop_small_packs(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
+// hip_ops.cpp: takes back copies of filters that would be made too early, or that do not pay
+void drop_filter_copies(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 void fuse_bn_pooling(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 
 struct HipProgramUnit {

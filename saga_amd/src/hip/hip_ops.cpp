@@ -101,14 +101,16 @@ struct FilterCopies : public HipOperation {
     {
         for(size_t i = 0; i < items_.size(); i++)
             if(items_[i].copy->m_storage == s) {
-                items_.erase(items_.begin() + i);
-                dropped(i);
-                dirty_ = true;
+                drop(i);
                 return true;
             }
         return false;
     }
-    virtual void dropped(size_t) {}
+    virtual void drop(size_t i)
+    {
+        items_.erase(items_.begin() + i);
+        dirty_ = true;
+    }
     // the table upload synchronises, and whether there is a launch is decided per step: not for recorded graphs
     bool graphSafe() const override { return false; }
     double bytes() const override
@@ -161,7 +163,11 @@ struct FilterPackBatch : public FilterCopies {
     };
     std::vector<Shape> shapes_;
     FilterPackBatch() : FilterCopies("filterpack") {}
-    void dropped(size_t i) override { shapes_.erase(shapes_.begin() + i); }
+    void drop(size_t i) override
+    {
+        FilterCopies::drop(i);
+        shapes_.erase(shapes_.begin() + i);
+    }
     // (the first layers of a forward pass are soon waiting for theirs)
     bool sideSafe() const override { return shapes_.size() && shapes_[0].kind == SAGA_CONV_BWD_DATA; }
     std::vector<char> table() override
@@ -350,21 +356,41 @@ struct ConvFwd : public HipOperation {
 
 } // namespace
 
-// In training every step packs: a launch for fewer than four filters costs more than the convolutions' own copies in
+// Copies of filters that a program does without: its convolutions then read the filter itself, when they run.
+//
+// A filter that an operation of the program computes, or a batched one, is not what it will be when the copies are made, in
+// front of the first convolution (the optimizers, which run last, are not in `ops` yet).
+//
+// And in training every step packs: a launch for fewer than four filters costs more than the convolutions' own copies in
 // front of their products (LeNet, one filter each way: 379 against 389 us per step).
-void drop_small_packs(HipProgram &p, HipOps &ops)
+void drop_filter_copies(HipProgram &p, HipOps &ops)
 {
-    if(p.m_pt != ProgramType::TRAINING)
-        return;
-    for(auto &batch : p.m_pack_batch) {
-        auto *b = static_cast<FilterPackBatch *>(batch.get());
-        if(!b || b->items_.size() >= 4)
+    std::set<HipStorage *> written;
+    for(const auto &op : ops)
+        for(const auto &o : op->listOutputs())
+            written.insert(o.second->m_storage.get());
+    for(auto batch : {&p.m_transpose_batch, &p.m_pack_batch[0], &p.m_pack_batch[1]}) {
+        auto *b = static_cast<FilterCopies *>(batch->get());
+        if(!b)
             continue;
-        for(auto &op : ops)
-            for(const auto &it : b->items_)
-                op->forget(it.copy);
-        ops.erase(std::find(ops.begin(), ops.end(), batch));
-        batch.reset();
+        const bool small = batch != &p.m_transpose_batch && p.m_pt == ProgramType::TRAINING;
+        auto drop = [&](size_t i) {
+            for(auto &op : ops)
+                op->forget(b->items_[i].copy);
+            b->drop(i);
+        };
+        for(size_t i = b->items_.size(); i-- > 0;) {
+            const auto &st = b->items_[i].w->m_storage;
+            if(written.count(st.get()) || st->doubleBuffered())
+                drop(i);
+        }
+        if(small && b->items_.size() < 4)
+            while(!b->items_.empty())
+                drop(b->items_.size() - 1);
+        if(b->items_.empty()) {
+            ops.erase(std::find(ops.begin(), ops.end(), *batch));
+            batch->reset();
+        }
     }
 }
 

@@ -66,3 +66,51 @@ def test_operations_in_front_of_the_first_convolution_are_ordered(name, image):
     assert kinds[:2] == ["convert", "spatialtransform"] and "filtertranspose" in [op["kind"] for op in ops if op["side"]]
     bad = stub_gpu.unordered(ops)
     assert not bad, bad[:8]
+
+
+def computed_filters(dtype, other, transpose):
+    """conv(x, w1), w2 = convert(w2h), conv(y, w2): a filter that the program computes between two convolutions."""
+    rng = np.random.default_rng(1)
+    g = S.Graph()
+    half = lambda shape: rng.standard_normal(shape).astype(np.float16)
+    x = S.Tensor.from_numpy(half((2, 16, 12, 12)).astype(N.np_dtype(dtype)))
+    w1 = S.Tensor.from_numpy(half((16, 16, 3, 3)).astype(N.np_dtype(dtype)), name="w1")
+    w2h = S.Tensor.from_numpy(half((16, 16, 3, 3)).astype(N.np_dtype(other)), name="w2h")
+    attrs = {"size": 3, "activations": 16, "pad": 1, "transpose": transpose}
+    y = g.add_node("conv", {"x": x, "w": w1}, attrs).y()
+    w2 = g.add_node("convert", {"x": w2h}, {"datatype": dtype}).y()
+    return g, w2h, g.add_node("conv", {"x": y, "w": w2}, attrs).y()
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("dtype,other", [(S.FLOAT, S.HALF), (S.HALF, S.FLOAT)], ids=["f32", "f16"])
+@on_stub
+def test_computed_filters_are_not_copied_beforehand(dtype, other, transpose):
+    g, _, out = computed_filters(dtype, other, transpose)
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False)
+    ctx.resolve(out)
+    p.finalize()
+    ops = stub_gpu.plan(p)
+    convert, = [i for i, op in enumerate(ops) if op["kind"] == "convert"]
+    (filter2, *_), = ops[convert]["writes"]
+    early = [op["kind"] for op in ops[:convert] for s, *_ in op["reads"] if s == filter2]
+    assert not early, early
+    # the filter that nothing computes still has its copy, where its kernel reads one
+    copies = [op for op in ops if op["kind"] in ("filterpack", "filtertranspose")]
+    assert len(copies) == (0 if dtype == S.HALF and not transpose else 1)
+    assert all(len(op["reads"]) == 1 for op in copies)
+
+
+@on_stub
+def test_batched_filters_are_not_copied():
+    """A batched tensor's contents and address change under the operations."""
+    g = S.Graph()
+    x = S.Tensor.from_numpy(np.zeros((2, 16, 12, 12), np.float32))
+    w = S.Tensor.from_numpy(np.zeros((16, 16, 3, 3), np.float32), name="w")
+    out = g.add_node("conv", {"x": x, "w": w}, {"size": 3, "activations": 16, "pad": 1}).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False, batched={w: S.PRE})
+    ctx.resolve(out)
+    p.finalize()
+    assert [op["kind"] for op in stub_gpu.plan(p)] == ["convfwd"]

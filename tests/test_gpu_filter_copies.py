@@ -5,6 +5,7 @@ import copy
 import numpy as np
 import pytest
 
+from oracle import ref
 from saga_amd import api as S
 from saga_amd import networks as N
 
@@ -67,3 +68,61 @@ def test_training_steps():
         got = out.read().copy()
         np.testing.assert_array_equal(got, logits(net, x, {k: v.read().copy() for k, v in weights.items()}))
         train.run(1)
+
+
+@pytest.mark.parametrize("transpose", [False, True])
+@pytest.mark.parametrize("dtype,other", [(S.FLOAT, S.HALF), (S.HALF, S.FLOAT)], ids=["f32", "f16"])
+def test_computed_filter(dtype, other, transpose):
+    """A filter that the program itself computes, between two convolutions, is used as this step computed it."""
+    rng = np.random.default_rng(3)
+    draw = lambda *shape: (rng.standard_normal(shape) / 12).astype(np.float16).astype(N.np_dtype(dtype))
+    x, w1 = draw(2, 16, 12, 12), draw(16, 16, 3, 3)
+    attrs = {"size": 3, "activations": 16, "pad": 1, "transpose": transpose}
+
+    def conv(g, x, w):
+        return g.add_node("conv", {"x": x, "w": w}, attrs).y()
+
+    def program(w2):
+        """w2: a front-end tensor's function of the graph."""
+        g, ctx = S.Graph(), S.Context()
+        y = conv(g, S.Tensor.from_numpy(x), S.Tensor.from_numpy(w1, name="w1"))
+        second = w2(g)
+        out = conv(g, y, second)
+        p = ctx.create_program(g, 2, training=False)
+        out = ctx.resolve(out)
+        p.finalize()  # places the initial values
+        return ctx, p, out
+
+    source = S.Tensor.from_numpy(draw(16, 16, 3, 3).astype(N.np_dtype(other)), name="source")
+    ctx, p, out = program(lambda g: g.add_node("convert", {"x": source}, {"datatype": dtype}).y())
+    dev = ctx.resolve(source)
+    for _ in range(3):
+        values = draw(16, 16, 3, 3)
+        dev.write(values.astype(N.np_dtype(other)))
+        p.run(1)
+        _, q, want = program(lambda g: S.Tensor.from_numpy(values, name="w2"))
+        q.run(1)
+        # the same products, added in another order where the constant filter is packed: fp32 rounding, and in fp16 at most the
+        # next value (2^-10 of the largest) where a sum lies between two
+        scale = np.abs(want.read()).max()
+        assert scale > 0
+        np.testing.assert_allclose(out.read() / scale, want.read() / scale, atol=1e-5 if dtype == S.FLOAT else 2e-3)
+
+
+def test_batched_filter():
+    """... and one that the host hands in with every batch."""
+    rng = np.random.default_rng(4)
+    draw = lambda *shape: rng.standard_normal(shape).astype(np.float32)
+    x = draw(2, 16, 12, 12)
+    g, ctx = S.Graph(), S.Context()
+    w = S.Tensor.from_numpy(draw(16, 16, 3, 3), name="w")
+    out = g.add_node("conv", {"x": S.Tensor.from_numpy(x), "w": w}, {"size": 3, "activations": 16, "pad": 1}).y()
+    p = ctx.create_program(g, 2, training=False, batched={w: S.PRE})
+    out, dev = ctx.resolve(out), ctx.resolve(w)
+    p.finalize()
+    for _ in range(3):
+        values = draw(16, 16, 3, 3)
+        dev.write(values)
+        p.run(1)
+        want = ref.conv2d_fwd(x, values, 1, 1)
+        np.testing.assert_allclose(out.read() / np.abs(want).max(), want / np.abs(want).max(), atol=1e-5)
