@@ -111,7 +111,8 @@ public:
     void *deviceMem() const override { return m_dev[m_index]; }
     bool doubleBuffered() const override { return true; }
     void *hostBack() const { return m_host[m_index ^ 1]; }
-    // host[back] -> device[back]; false (nothing enqueued) when the device already holds what the host does
+    // host[back] -> device[back]; false (nothing enqueued) when the device already holds what the host does, which is certain
+    // only while no host window is open: its pointers may be written through at any time
     bool uploadBack(hipStream_t st);
     void downloadFront(hipStream_t st); // device[front] -> host[front]
     void flip() { m_index ^= 1; }
@@ -119,6 +120,7 @@ public:
     void *m_host[2] = {nullptr, nullptr};
     // host[i] was handed out for writing, or filled by a download, since it last went to the device
     bool m_host_touched[2] = {false, false};
+    int m_windows = 0; // access objects that are alive
     bool m_written_by_ops = false; // the device side changes too: every upload counts
     int m_index = 0;
 };

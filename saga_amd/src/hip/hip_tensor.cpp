@@ -81,7 +81,7 @@ HipDoubleBuffer::~HipDoubleBuffer()
 bool HipDoubleBuffer::uploadBack(hipStream_t st)
 {
     const int b = m_index ^ 1;
-    if(!m_host_touched[b] && !m_written_by_ops)
+    if(!m_host_touched[b] && !m_written_by_ops && !m_windows)
         return false;
     m_host_touched[b] = false;
     chkHip(hipMemcpyAsync(m_dev[b], m_host[b], m_elements * m_element_size, hipMemcpyHostToDevice, st));
@@ -304,8 +304,13 @@ private:
 // Host window onto the back buffer of a batched tensor: no copies, the program moves the data.
 class HipBatchAccess : public TensorAccess {
 public:
-    HipBatchAccess(HipTensor &t, std::shared_ptr<HipDoubleBuffer> db) : m_t(t), m_db(db), m_back(db->m_index ^ 1) {}
-    ~HipBatchAccess() { m_db->m_host_touched[m_back] = true; } // writes may have come after an upload
+    HipBatchAccess(HipTensor &t, std::shared_ptr<HipDoubleBuffer> db) : m_t(t), m_db(db) { m_db->m_windows++; }
+    ~HipBatchAccess()
+    {
+        m_db->m_windows--;
+        for(int i = 0; i < 2; i++)
+            m_db->m_host_touched[i] |= m_given[i]; // writes may have come after the last upload
+    }
     Dims strides() override
     {
         Dims d;
@@ -329,13 +334,13 @@ public:
 private:
     void *back() // for writing
     {
-        m_back = m_db->m_index ^ 1;
-        m_db->m_host_touched[m_back] = true;
+        const int b = m_db->m_index ^ 1;
+        m_given[b] = m_db->m_host_touched[b] = true;
         return m_db->hostBack();
     }
     HipTensor &m_t;
     std::shared_ptr<HipDoubleBuffer> m_db;
-    int m_back;
+    bool m_given[2] = {false, false}; // the buffers that pointers were handed out into
 };
 
 std::unique_ptr<TensorAccess> HipTensor::access()

@@ -16,6 +16,7 @@ size_t g_total = (size_t)288 << 30, g_used = 0;
 std::map<void *, size_t> g_allocs;
 std::map<const void *, std::string> g_kernels;
 std::map<std::string, long> g_launches;
+long g_uploads = 0;
 
 hipError_t map_memory(void **p, size_t bytes)
 {
@@ -59,6 +60,8 @@ long hipstub_launches(const char *kernel) // of kernels whose name contains this
     return n;
 }
 
+long hipstub_uploads(void) { return g_uploads; } // asynchronous ones
+
 hipError_t hipMalloc(void **p, size_t bytes)
 {
     if(g_used + ((bytes + 4095) & ~(size_t)4095) > g_total)
@@ -90,7 +93,11 @@ hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
     memmove(d, s, n);
     return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t)
+{
+    g_uploads += k == hipMemcpyHostToDevice;
+    return hipMemcpy(d, s, n, k);
+}
 
 hipError_t hipGetDeviceCount(int *n)
 {

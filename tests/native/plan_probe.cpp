@@ -55,10 +55,12 @@ int probe_plan(void *box, char *buf, size_t capacity)
 void *probe_access(void *tensor_box) { return (*(std::shared_ptr<Tensor> *)tensor_box)->access().release(); }
 void *probe_access_data(void *ta) { return ((TensorAccess *)ta)->data(); }
 void probe_access_close(void *ta) { delete(TensorAccess *)ta; }
-// what the operations of the next step read
-void *probe_device(void *tensor_box)
+// the device buffer of a batched tensor that the operations of the last step read
+void *probe_last_batch(void *tensor_box)
 {
-    return dynamic_cast<HipTensor *>(((std::shared_ptr<Tensor> *)tensor_box)->get())->deviceMem();
+    auto *t = dynamic_cast<HipTensor *>(((std::shared_ptr<Tensor> *)tensor_box)->get());
+    auto *db = static_cast<HipDoubleBuffer *>(t->m_storage.get());
+    return db->m_dev[db->m_index ^ 1];
 }
 
 }  // extern "C"

@@ -10,6 +10,8 @@ import subprocess
 import sys
 import tempfile
 
+import numpy as np
+
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 NATIVE = os.path.join(ROOT, "tests", "native")
 
@@ -44,11 +46,12 @@ def _child(libs, module, name, kwargs):
 
     stub = C.CDLL(os.path.join(libs, "hip_stub.so"), mode=C.RTLD_GLOBAL)  # before anything that needs the runtime
     stub.hipstub_set_memory.argtypes = [C.c_size_t]
+    stub.hipstub_uploads.restype = C.c_long
     stub.hipstub_launches.argtypes, stub.hipstub_launches.restype = [C.c_char_p], C.c_long
     api.lib()
     probe = C.CDLL(os.path.join(libs, "plan_probe.so"))
     probe.probe_plan.argtypes = [C.c_void_p, C.c_char_p, C.c_size_t]
-    for f in (probe.probe_access, probe.probe_access_data, probe.probe_device):
+    for f in (probe.probe_access, probe.probe_access_data, probe.probe_last_batch):
         f.argtypes, f.restype = [C.c_void_p], C.c_void_p
     probe.probe_access_close.argtypes = [C.c_void_p]
     getattr(importlib.import_module("tests." + module), name).body(**json.loads(kwargs))
@@ -56,6 +59,10 @@ def _child(libs, module, name, kwargs):
 
 def launches(kernel):
     return stub.hipstub_launches(kernel.encode())
+
+
+def uploads():
+    return stub.hipstub_uploads()
 
 
 def plan(program):
@@ -98,3 +105,21 @@ def unordered(ops):
             if meet(w, rw2) or meet(rw, w2):
                 bad.append((j, ops[j]["kind"], i, ops[i]["kind"]))
     return bad
+
+
+class Window:
+    """A host window onto a batched tensor that stays open until close()."""
+
+    def __init__(self, tensor):
+        self._ta = probe.probe_access(tensor._h)
+
+    def floats(self, n):
+        return np.frombuffer((C.c_float * n).from_address(probe.probe_access_data(self._ta)), np.float32)
+
+    def close(self):
+        probe.probe_access_close(self._ta)
+
+
+def last_batch(tensor, n):
+    """The first n floats that the last step's operations read of a batched tensor."""
+    return np.frombuffer((C.c_float * n).from_address(probe.probe_last_batch(tensor._h)), np.float32).copy()

@@ -114,3 +114,47 @@ def test_batched_filters_are_not_copied():
     ctx.resolve(out)
     p.finalize()
     assert [op["kind"] for op in stub_gpu.plan(p)] == ["convfwd"]
+
+
+def batched_relu():
+    g = S.Graph()
+    x = S.Tensor.from_numpy(np.zeros((2, 8), np.float32), name="x")
+    y = g.add_node("relu", {"x": x}).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False, batched={x: S.PRE})
+    return p, ctx.resolve(x), ctx.resolve(y)
+
+
+@pytest.mark.parametrize("steps", [1, 2])
+@on_stub
+def test_a_pointer_kept_over_steps_is_uploaded(steps):
+    """The access object and the pointer are asked for once, the values are written before every run."""
+    p, x, _ = batched_relu()
+    p.finalize()
+    window = stub_gpu.Window(x)
+    data = window.floats(16)
+    for value in (1, 2, 3, 4):
+        data[:] = value
+        p.run(steps)
+        if steps == 1:  # (an even number of steps leaves the other buffer behind)
+            np.testing.assert_array_equal(stub_gpu.last_batch(x, 16), value)
+    data[:] = 5
+    window.close()  # what was written before the window was closed counts
+    p.run(1)
+    seen = [stub_gpu.last_batch(x, 16)[0]]
+    p.run(2)
+    seen.append(stub_gpu.last_batch(x, 16)[0])
+    assert 5 in seen, seen
+
+
+@on_stub
+def test_untouched_batches_are_uploaded_once():
+    p, x, _ = batched_relu()
+    p.finalize()
+    before = stub_gpu.uploads()
+    x.write(np.ones((2, 8), np.float32))
+    p.run(1)
+    assert stub_gpu.uploads() - before == 1
+    np.testing.assert_array_equal(stub_gpu.last_batch(x, 16), 1)
+    p.run(1)
+    assert stub_gpu.uploads() - before == 1
