@@ -195,6 +195,8 @@ struct HipOperation {
     virtual bool killOutput(const std::shared_ptr<HipStorage> &s) { return false; }
     // inference: write relu(output) to y instead of the output; false if the operation cannot
     virtual bool foldRelu(const std::shared_ptr<HipTensor> &y) { return false; }
+    // do only one's own work again, and write one's own output
+    virtual void unfold() {}
     // do without an optional input
     virtual void forget(const std::shared_ptr<HipTensor> &t) {}
     virtual std::string info() const { return ""; }
@@ -227,6 +229,10 @@ void reorder_sparse_first_writers(std::vector<std::shared_ptr<HipOperation>> &op
 // hip_ops.cpp: takes back copies of filters that would be made too early, or that do not pay
 void drop_filter_copies(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
 void fuse_bn_pooling(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
+// hip_ops.cpp: operations that the one in front of them does along
+void fold_into_producers(HipProgram &p, std::vector<std::shared_ptr<HipOperation>> &ops);
+// the storages whose contents a step finds there: read by an operation and not written by an earlier one
+std::set<HipStorage *> readBeforeWritten(const HipOps &ops);
 
 struct HipProgramUnit {
     Nodes m_transformed;
@@ -315,6 +321,9 @@ public:
     size_t m_arena_bytes = 0;    // size of the arena
     size_t m_planned_bytes = 0;  // sum of the sizes of the storages laid out in it
     void planMemory();
+    // somebody looks at this storage who did not when programs were finalized: operations that were folded into the one
+    // that writes it become operations again, from the next step on
+    void unfold(HipStorage *s);
 };
 
 class HipProgram : public Program {
@@ -430,6 +439,14 @@ public:
     // convolutions of the forward and of the backward pass, in one launch each (hip_ops.cpp)
     std::shared_ptr<HipOperation> m_transpose_batch, m_pack_batch[2];
     std::vector<HipStorage *> m_written; // by m_ops
+
+    // what fold_into_producers() did: `op` is done by `producer`, and nobody writes the storage between them
+    struct Fold {
+        HipOp producer, op;
+        std::shared_ptr<HipStorage> between;
+    };
+    std::vector<Fold> m_folded;
+    void unfold(HipStorage *s);
 
     SagaAux *m_aux = nullptr; // pinned host memory the optimizer kernels write their flags to
     float m_mp_scaling = 1.0f;

@@ -266,6 +266,12 @@ struct ConvFwd : public HipOperation {
         m_kind = "convfwd.bn";
         return true;
     }
+    void unfold() override
+    {
+        bn_s_ = bn_b_ = bn_m_ = bn_v_ = bn_z_ = bn_y_ = relu_y_ = nullptr;
+        bn_flags_ = 0;
+        m_kind = "convfwd";
+    }
     // (a kernel takes both only together, and only in fp32)
     bool foldRelu(const T &y) override
     {
@@ -680,30 +686,10 @@ struct ActBwd : public HipOperation {
     double bytes() const override { return (beta_ != 0 ? 4 : 3) * nbytes(dx_); }
 };
 
-bool single_consumer(const Nodes &nodes, const std::shared_ptr<Tensor> &t);
-
 void activation_setup(HipProgram &p, HipProgramUnit &pu, const Node &n, int mode, float alpha)
 {
     auto x = p.lower(pu, n.m_inputs["x"]);
     auto y = p.lowerLike(pu, n.m_outputs["y"], *x);
-    if(p.m_pt == ProgramType::INFERENCE && mode == SAGA_ACT_RELU && !p.m_pc.disable_op_fusing) {
-        // the one operation that writes x writes y instead, if nobody else looks at x
-        std::shared_ptr<HipOperation> producer;
-        int touching = 0;
-        for(const auto &op : pu.m_fwd)
-            for(const auto &list : {op->listInputs(), op->listOutputs()})
-                for(const auto &o : list)
-                    if(o.second->m_storage == x->m_storage) {
-                        touching++;
-                        producer = op;
-                    }
-        const auto &ex = p.m_ctx->m_exported;
-        const bool held = std::any_of(ex.begin(), ex.end(), [&](const auto &e) { return e == x->m_storage; });
-        const auto outs = producer ? producer->listOutputs() : HipOpArgs();
-        if(touching == 1 && !held && outs.size() == 1 && outs[0].second == x && single_consumer(pu.m_transformed, n.m_inputs["x"]) &&
-           producer->foldRelu(y))
-            return;
-    }
     pu.fwd(std::make_shared<ActFwd>(x, y, mode, alpha));
     if(p.m_pt == ProgramType::INFERENCE)
         return;
@@ -759,6 +745,7 @@ struct Gemm : public HipOperation {
         relu_c_ = y;
         return true;
     }
+    void unfold() override { relu_c_ = nullptr; }
     bool sideSafe() const override { return true; }
     HipOpArgs listInputs() const override
     {
@@ -1300,26 +1287,7 @@ void batchnorm_lower(HipProgram &p, HipProgramUnit &pu, const Node &n, std::shar
             throw std::runtime_error("batchnorm parameters must be fp32 vectors of C elements");
     const float eps = n.m_attributes.get("epsilon", 1e-5f);
 
-    // the operation that alone writes x, if it is a convolution
-    auto conv_producer = [&]() -> ConvFwd * {
-        ConvFwd *producer = nullptr;
-        int writers = 0;
-        for(const auto &op : pu.m_fwd)
-            for(const auto &o : op->listOutputs())
-                if(o.second->m_storage == x->m_storage) {
-                    writers++;
-                    producer = o.second == x ? dynamic_cast<ConvFwd *>(op.get()) : nullptr;
-                }
-        return writers == 1 ? producer : nullptr;
-    };
     if(p.m_pt == ProgramType::INFERENCE) {
-        // conv -> batch norm with nobody else looking at the convolution's output: one kernel
-        ConvFwd *producer = conv_producer();
-        const auto &ex = p.m_ctx->m_exported;
-        const bool held = std::any_of(ex.begin(), ex.end(), [&](const auto &e) { return e == x->m_storage; });
-        if(producer && !held && !p.m_pc.disable_op_fusing && single_consumer(pu.m_transformed, xh) &&
-           producer->foldBn(s, b, m, v, z, y, eps, flags))
-            return;
         pu.fwd(std::make_shared<BnInference>(x, z, s, b, m, v, y, eps, flags));
         return;
     }
@@ -1327,7 +1295,15 @@ void batchnorm_lower(HipProgram &p, HipProgramUnit &pu, const Node &n, std::shar
     auto sv = std::make_shared<HipTensor>(Tensor::DataType::FLOAT, *v, v->namePostfix("svar"));
     auto f = std::make_shared<BnTrain>(p, x, z, s, b, m, v, y, sm, sv, eps, flags);
     // if the op that wrote x last is a convolution and nothing else writes x, take the sums from it
-    if(ConvFwd *producer = conv_producer())
+    ConvFwd *producer = nullptr;
+    int writers = 0;
+    for(const auto &op : pu.m_fwd)
+        for(const auto &o : op->listOutputs())
+            if(o.second->m_storage == x->m_storage) {
+                writers++;
+                producer = o.second == x ? dynamic_cast<ConvFwd *>(op.get()) : nullptr;
+            }
+    if(writers == 1 && producer)
         f->stats_ = producer->offerStats();
     // residual + relu on fp16 channels-last tensors with whole 8-channel vectors, statistics from
     // the convolution: the forward pass also leaves the relu mask, one bit per element
@@ -1463,6 +1439,7 @@ struct PoolFwd : public HipOperation {
         relu_y_ = y;
         return true;
     }
+    void unfold() override { relu_y_ = nullptr; }
     HipOpArgs listInputs() const override { return {{"x", x_}}; }
     HipOpArgs listOutputs() const override { return {{"y", relu_y_ ? relu_y_ : y_}}; }
     std::string info() const override { return mode_ == SAGA_POOL_MAX ? "max" : "avg"; }
@@ -2048,6 +2025,62 @@ Nodes concat_transform(HipProgram &p, HipProgramUnit &pu, const Nodes &nodes)
 REGISTER_HIP_TRANSFORM(100, ProgramType::INFERENCE | ProgramType::TRAINING, concat_transform);
 
 }  // namespace
+
+// Inference programs: a batch norm behind a convolution, or a relu behind a convolution, product or pooling, becomes part of
+// the operation that writes its input, which then writes the result in place of that input.  Nobody else may see the input:
+// no other operation, not the host, no other program.  What the folded operation reads and writes is touched at the
+// producer's place in the list from then on, so nothing in between may write the one or touch the other.
+void fold_into_producers(HipProgram &p, HipOps &ops)
+{
+    if(p.m_pt != ProgramType::INFERENCE || p.m_pc.disable_op_fusing)
+        return;
+    auto touches = [](const HipOpArgs &args, const HipStorage *s) {
+        return std::count_if(args.begin(), args.end(), [&](const auto &a) { return a.second->m_storage.get() == s; });
+    };
+    std::set<HipStorage *> seen_elsewhere;
+    for(const auto &e : p.m_ctx->m_exported)
+        seen_elsewhere.insert(e.get());
+    for(const HipProgram *q : p.m_ctx->m_programs)
+        for(HipStorage *s : readBeforeWritten(q->m_ops))
+            seen_elsewhere.insert(s);
+    for(size_t j = 0; j < ops.size(); j++) {
+        const HipOp next = ops[j];
+        const auto *norm = dynamic_cast<BnInference *>(next.get());
+        const auto *act = dynamic_cast<ActFwd *>(next.get());
+        if(!norm && !(act && act->mode_ == SAGA_ACT_RELU))
+            continue;
+        const T x = norm ? norm->x_ : act->x_, y = norm ? norm->y_ : act->y_;
+        const HipStorage *xs = x->m_storage.get(), *ys = y->m_storage.get();
+        if(seen_elsewhere.count(x->m_storage.get()) || xs->doubleBuffered())
+            continue;
+        size_t i = j;
+        int count = 0;
+        bool clean = true;
+        for(size_t k = 0; k < ops.size(); k++) {
+            const HipOpArgs in = ops[k]->listInputs(), out = ops[k]->listOutputs();
+            count += touches(in, xs) + touches(out, xs);
+            if(k < j && out.size() == 1 && out[0].second == x)
+                i = k;
+            for(const auto &o : out)
+                clean &= k == j || o.second != y; // (several writers add up)
+        }
+        if(i == j || count != 2 || !clean)
+            continue;
+        const HipOpArgs reads = next->listInputs();
+        for(size_t k = i + 1; k < j; k++) {
+            const HipOpArgs in = ops[k]->listInputs(), out = ops[k]->listOutputs();
+            for(const auto &r : reads)
+                clean &= !touches(out, r.second->m_storage.get());
+            clean &= !touches(in, ys) && !touches(out, ys);
+        }
+        auto *conv = dynamic_cast<ConvFwd *>(ops[i].get());
+        if(!clean || !(norm ? conv && conv->foldBn(norm->s_, norm->b_, norm->m_, norm->v_, norm->z_, y, norm->eps_, norm->flags_)
+                            : ops[i]->foldRelu(y)))
+            continue;
+        p.m_folded.push_back({ops[i], next, x->m_storage});
+        ops.erase(ops.begin() + j--);
+    }
+}
 
 // Training programs: a max pooling (with position codes) whose input is the output of a batch norm (+ relu) that
 // nothing else touches - no other operation of the program reads or writes that storage (a skip connection, a

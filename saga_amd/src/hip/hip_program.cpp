@@ -211,6 +211,7 @@ std::shared_ptr<Tensor> HipContext::resolveTensor(std::shared_ptr<Tensor> src)
     if(it == m_tensors.end())
         return nullptr;
     m_exported.push_back(it->second->m_storage);
+    unfold(it->second->m_storage.get());
     // a tensor the host holds keeps its contents between steps: out of the shared arena
     // (reference: src/cuda/cuda_common.cpp:145-158)
     auto &st = it->second->m_storage;
@@ -541,6 +542,51 @@ void HipProgram::addBatchedTensors(const ProgramSource &ps)
 
 // ---------------------------------------------------------------- finalize
 
+std::set<HipStorage *> readBeforeWritten(const HipOps &ops)
+{
+    std::set<HipStorage *> read, written;
+    for(const auto &op : ops) {
+        for(const auto &i : op->getInputs())
+            if(!written.count(i.second->m_storage.get()))
+                read.insert(i.second->m_storage.get());
+        for(const auto &o : op->getOutputs())
+            written.insert(o.second->m_storage.get());
+    }
+    return read;
+}
+
+void HipContext::unfold(HipStorage *s)
+{
+    for(HipProgram *p : m_programs)
+        p->unfold(s);
+}
+
+// The folded operation goes back into the list right behind its producer.  The arena stays as it is: what the two read is
+// in use for one operation longer and what they write from one operation later, with nothing else in between, and the
+// storage between them gets memory of its own.
+void HipProgram::unfold(HipStorage *s)
+{
+    for(size_t f = 0; f < m_folded.size(); f++) {
+        if(m_folded[f].between.get() != s)
+            continue;
+        const Fold fold = m_folded[f];
+        m_folded.erase(m_folded.begin() + f--);
+        auto it = std::find(m_ops.begin(), m_ops.end(), fold.producer);
+        if(it == m_ops.end()) // nobody needed its result
+            continue;
+        const size_t i = it - m_ops.begin();
+        fold.producer->unfold();
+        m_ops.insert(it + 1, fold.op);
+        if(m_poison_before.size() + 1 == m_ops.size()) {
+            m_poison_before.insert(m_poison_before.begin() + i + 1, std::vector<HipStorage *>());
+            m_poison_after.insert(m_poison_after.begin() + i, std::vector<HipStorage *>());
+        }
+        m_written.push_back(s);
+        dropGraphs();
+        m_segments.clear();
+    }
+}
+
 // Backward liveness over the op list, treated as one iteration of a loop: a storage is needed
 // at the end of the step if the host can see it or if the next step reads it before writing
 // it (weights, running statistics, optimizer state).  Operations none of whose outputs are
@@ -551,16 +597,8 @@ void HipProgram::eliminateDeadOps()
     std::set<HipStorage *> live;
     for(const auto &s : m_ctx->m_exported)
         live.insert(s.get());
-    {
-        std::set<HipStorage *> written;
-        for(const auto &op : m_ops) {
-            for(const auto &i : op->getInputs())
-                if(!written.count(i.second->m_storage.get()))
-                    live.insert(i.second->m_storage.get()); // read before written: carried across steps
-            for(const auto &o : op->getOutputs())
-                written.insert(o.second->m_storage.get());
-        }
-    }
+    for(HipStorage *s : readBeforeWritten(m_ops)) // carried across steps
+        live.insert(s);
     HipOps kept;
     for(auto it = m_ops.rbegin(); it != m_ops.rend(); ++it) {
         auto &op = *it;
@@ -617,6 +655,9 @@ void HipProgram::finalize()
     // An accumulating writer reads its output, so the dead-op pass below keeps the first writer
     // whenever it keeps a later one.
     drop_filter_copies(*this, m_ops);
+    for(HipStorage *s : readBeforeWritten(m_ops)) // (another program's intermediate result, perhaps)
+        m_ctx->unfold(s);
+    fold_into_producers(*this, m_ops);
     if(m_pt == ProgramType::TRAINING)
         reorder_sparse_first_writers(m_ops);
     std::set<HipTensor *> written;

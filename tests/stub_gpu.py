@@ -73,6 +73,19 @@ def plan(program):
     return [json.loads(line) for line in buf.value.decode().splitlines()]
 
 
+def overlapping(ops):
+    """Pairs of storages at the same addresses of which one is written while the other still holds something that is read later
+    (operations in the order of the list)."""
+    life, place = {}, {}
+    for i, op in enumerate(ops):
+        for s, a, size, _ in op["reads"] + op["writes"]:
+            if a:
+                first, _ = life.get(s, (i, i))
+                life[s], place[s] = (first, i), (a, a + size)
+    return [(s, q) for s in life for q in life if s < q and place[s][0] < place[q][1] and place[q][0] < place[s][1]
+            and life[s][0] <= life[q][1] and life[q][0] <= life[s][1]]
+
+
 def unordered(ops):
     """Pairs of operations that touch the same addresses, one of them writing, and that neither the order of a stream nor an
     event puts one behind the other."""

@@ -158,3 +158,130 @@ def test_untouched_batches_are_uploaded_once():
     np.testing.assert_array_equal(stub_gpu.last_batch(x, 16), 1)
     p.run(1)
     assert stub_gpu.uploads() - before == 1
+
+
+def norm_params(rng, c):
+    return {k: S.Tensor.from_numpy(rng.uniform(0.5, 1.5, (1, c)).astype(np.float32), name="bn-" + k) for k in "sbmv"}
+
+
+def chain(dtype):
+    """conv + bias -> relu -> maxpool -> relu -> conv -> batch norm -> sigmoid, and its intermediate tensors by name."""
+    rng = np.random.default_rng(2)
+    draw = lambda *shape, by=1: S.Tensor.from_numpy((rng.standard_normal(shape) / by).astype(N.np_dtype(dtype)))
+    g, t = S.Graph(), {}
+    attrs = {"size": 3, "activations": 16, "pad": 1}
+    t["conv"] = g.add_node("conv", {"x": draw(2, 16, 12, 12), "w": draw(16, 16, 3, 3, by=12), "b": draw(1, 16)}, {**attrs, "bias": True}).y()
+    t["relu"] = g.add_node("relu", {"x": t["conv"]}).y()
+    t["pool"] = g.add_node("maxpool", {"x": t["relu"]}, {"size": 2, "stride": 2}).y()
+    t["relu2"] = g.add_node("relu", {"x": t["pool"]}).y()
+    t["conv2"] = g.add_node("conv", {"x": t["relu2"], "w": draw(16, 16, 3, 3, by=12)}, attrs).y()
+    t["norm"] = g.add_node("batchnorm", {"x": t["conv2"], **norm_params(rng, 16)}).y()
+    t["out"] = g.add_node("sigmoid", {"x": t["norm"]}).y()
+    return g, t
+
+
+FOLDED = {S.FLOAT: ["conv", "pool", "conv2"], S.HALF: ["pool", "conv2"]}
+
+
+def written(ops):
+    return [s for op in ops for s, *_ in op["writes"]]
+
+
+@pytest.mark.parametrize("dtype", [S.FLOAT, S.HALF], ids=["f32", "f16"])
+@on_stub
+def test_what_nobody_looks_at_is_folded_away(dtype):
+    g, t = chain(dtype)
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False)
+    ctx.resolve(t["out"])
+    p.finalize()
+    kinds = [op["kind"] for op in stub_gpu.plan(p) if op["kind"] != "filterpack"]
+    assert kinds == {S.FLOAT: ["convfwd", "poolfwd", "convfwd.bn", "actfwd"],
+                     S.HALF: ["convfwd", "actfwd", "poolfwd", "convfwd.bn", "actfwd"]}[dtype]
+
+
+@pytest.mark.parametrize("finalized", [False, True], ids=["behind create_program", "behind finalize"])
+@pytest.mark.parametrize("dtype", [S.FLOAT, S.HALF], ids=["f32", "f16"])
+@on_stub
+def test_resolved_intermediates_are_written(dtype, finalized):
+    """Also when they are resolved late, one after the other: each is an operation's output then, and all that was written before
+    still is, in an order that suits the readers."""
+    g, t = chain(dtype)
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False, anomaly_detect=True)
+    ctx.resolve(t["out"])
+    if finalized:
+        p.finalize()
+        before = stub_gpu.plan(p)
+        outputs = {s for op in before for s, *_ in op["writes"]}
+    for n, name in enumerate(FOLDED[dtype]):
+        assert ctx.resolve(t[name]) is not None
+        if finalized:
+            ops = stub_gpu.plan(p)
+            assert len(ops) == len(before) + n + 1
+            assert outputs < set(written(ops))
+    p.run(1)
+    ops = stub_gpu.plan(p)
+    assert [op["kind"] for op in ops if op["kind"] != "filterpack"] == ["convfwd", "actfwd", "poolfwd", "actfwd", "convfwd", "bninf", "actfwd"]
+    seen = written(ops)
+    assert len(seen) == len(set(seen))
+    for i, op in enumerate(ops):  # no operation reads what a later one writes
+        later = set(written(ops[i:]))
+        assert not [s for s, *_ in op["reads"] if s in later]
+    assert stub_gpu.unordered(ops) == [] and stub_gpu.overlapping(ops) == []
+
+
+@on_stub
+def test_a_window_onto_an_intermediate_keeps_it():
+    """Other views of the same storage read it too."""
+    rng = np.random.default_rng(2)
+    draw = lambda *shape: S.Tensor.from_numpy(rng.standard_normal(shape).astype(np.float32))
+    g = S.Graph()
+    y = g.add_node("conv", {"x": draw(2, 8, 6, 6), "w": draw(16, 8, 3, 3)}, {"size": 3, "activations": 16, "pad": 1}).y()
+    a = g.add_node("batchnorm", {"x": y, **norm_params(rng, 16)}).y()
+    b = g.add_node("sigmoid", g.add_node("window", {"x": y}, {"offset": [0, 4, 0, 0], "shape": [2, 8, 6, 6]})).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False)
+    ctx.resolve(a), ctx.resolve(b)
+    p.finalize()
+    ops = [op for op in stub_gpu.plan(p) if op["kind"] != "filterpack"]
+    assert sorted(op["kind"] for op in ops) == ["actfwd", "bninf", "convfwd"]
+
+
+@on_stub
+def test_a_residual_that_is_computed_behind_the_convolution():
+    """The addition cannot move in front of what it adds."""
+    rng = np.random.default_rng(2)
+    draw = lambda *shape: S.Tensor.from_numpy(rng.standard_normal(shape).astype(np.float32))
+    g = S.Graph()
+    x = draw(2, 16, 6, 6)
+    main = g.add_node("conv", {"x": x, "w": draw(16, 16, 3, 3)}, {"size": 3, "activations": 16, "pad": 1}).y()
+    side = g.add_node("conv", {"x": x, "w": draw(16, 16, 1, 1)}, {"size": 1, "activations": 16}).y()
+    side = g.add_node("sigmoid", {"x": side}).y()
+    norm = g.add_node("batchnorm", {"x": main, **norm_params(rng, 16)}).y()
+    out = g.add_node("relu", g.add_node("sum", {"x0": norm, "x1": side})).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False)
+    ctx.resolve(out)
+    p.finalize()
+    ops = stub_gpu.plan(p)
+    (sigmoid, *_), = [op["writes"][0] for op in ops if op["kind"] == "actfwd"]
+    place = [op["kind"] for op in ops].index("actfwd")
+    assert all(sigmoid not in [s for s, *_ in op["reads"]] for op in ops[:place])
+
+
+@on_stub
+def test_another_program_reads_an_intermediate():
+    """A program that starts from what another one computes on the way."""
+    g, t = chain(S.FLOAT)
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False)
+    ctx.resolve(t["out"])
+    p.finalize()
+    h = S.Graph()
+    other = h.add_node("tanh", {"x": t["conv2"]}).y()
+    q = ctx.create_program(h, 2, training=False)
+    ctx.resolve(other)
+    q.finalize()
+    (source, *_), = stub_gpu.plan(q)[0]["reads"]
+    assert source in written(stub_gpu.plan(p))
