@@ -4558,6 +4558,10 @@ static bool refuses_dy(const SagaTensorView *dy, const SagaTensorView *w, const 
     return dy->dtype != SAGA_HALF || g.group != 1 || !as_channels_last(dy, ldy) || !as_channels_last(d, &ld) || !krsc_dense(w);
 }
 
+// A padded dy needs room that the direct kernels do not: a caller who brings none, or too little, gets those.  (Nothing of the
+// result has been written when the room turns out to be too small.)
+static int without_workspace(int r) { return r == SAGA_HIP_EWORKSPACE ? SAGA_HIP_EUNSUPPORTED : r; }
+
 int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const SagaTensorView *dw, const ConvGeom &g, float alpha,
                          float beta, void *ws, size_t ws_bytes, hipStream_t st)
 {
@@ -4571,8 +4575,10 @@ int conv_mfma_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, cons
         return bwd_filter(x, dy, dw, g, g.K, alpha, beta, ws, ws_bytes, st);
     ConvGeom gp = g;
     SagaTensorView dyp;
-    const int r = pad_dy(dy, ldy, gp, dyp, ws, ws_bytes, st);
-    return r ? r : bwd_filter(x, &dyp, dw, gp, g.K, alpha, beta, ws, ws_bytes, st);
+    int r = pad_dy(dy, ldy, gp, dyp, ws, ws_bytes, st);
+    if(!r)
+        r = bwd_filter(x, &dyp, dw, gp, g.K, alpha, beta, ws, ws_bytes, st);
+    return without_workspace(r);
 }
 
 int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g, float alpha,
@@ -4586,6 +4592,8 @@ int conv_mfma_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const 
         return bwd_data(dy, w, dx, g, g.K, alpha, beta, ws, ws_bytes, st, wt_ready, link, bias, bias_done);
     ConvGeom gp = g;
     SagaTensorView dyp;
-    const int r = pad_dy(dy, ldy, gp, dyp, ws, ws_bytes, st);
-    return r ? r : bwd_data(&dyp, w, dx, gp, g.K, alpha, beta, ws, ws_bytes, st, nullptr, nullptr, bias, bias_done);
+    int r = pad_dy(dy, ldy, gp, dyp, ws, ws_bytes, st);
+    if(!r)
+        r = bwd_data(&dyp, w, dx, gp, g.K, alpha, beta, ws, ws_bytes, st, nullptr, nullptr, bias, bias_done);
+    return without_workspace(r);
 }
