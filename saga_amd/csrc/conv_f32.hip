@@ -849,6 +849,21 @@ static FilterSplit plan_filter_uniform(const ConvGeom &g)
     return p;
 }
 
+// The splits whose partials (`one` bytes each) fit into `bytes`, in whole slices of `step` pixels; false if not even one does.
+// The plan's own number is what the workspace query asks for, but a caller may bring less.
+static bool fit_splits(FilterSplit &p, const ConvGeom &g, int step, size_t one, size_t bytes)
+{
+    const long long M = (long long)g.N * g.P * g.Q, room = (long long)(bytes / one);
+    if(room < 1)
+        return false;
+    if(p.splits > room) {
+        const long long per = ((M + room - 1) / room + step - 1) / step * step;
+        p.m_per_split = (int)per;
+        p.splits = (int)((M + per - 1) / per);
+    }
+    return true;
+}
+
 static long long extent_bytes(const SagaTensorView *v)
 {
     long long ext = 1;
@@ -1147,8 +1162,8 @@ int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const
         return SAGA_HIP_EUNSUPPORTED;
     const int CRS = g.C * g.R * g.S;
     if(filter_uniform_ok(x, dy, g)) {
-        const FilterSplit p = plan_filter_uniform(g);
-        if(!ws || ws_bytes < (size_t)p.splits * g.K * CRS * sizeof(float) || !aligned16(ws))
+        FilterSplit p = plan_filter_uniform(g);
+        if(!ws || !aligned16(ws) || !fit_splits(p, g, UW_P, (size_t)g.K * CRS * sizeof(float), ws_bytes))
             return SAGA_HIP_EWORKSPACE;
         FilterU32 k;
         k.x = (const float *)x->ptr;
@@ -1183,9 +1198,9 @@ int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const
         SAGA_CHECK_LAUNCH();
         return 0;
     }
-    const FilterSplit p = plan_filter_f32(g);
-    const size_t need = tab_bytes(CRS) + (size_t)p.splits * g.K * CRS * sizeof(float);
-    if(!ws || ws_bytes < need || !aligned16(ws))
+    FilterSplit p = plan_filter_f32(g);
+    if(!ws || !aligned16(ws) || ws_bytes < tab_bytes(CRS) ||
+       !fit_splits(p, g, WBK, (size_t)g.K * CRS * sizeof(float), ws_bytes - tab_bytes(CRS)))
         return SAGA_HIP_EWORKSPACE;
     KTabA *tab = (KTabA *)ws;
     long long *tb = (long long *)(tab + CRS);

@@ -705,10 +705,9 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
         taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
     if(k.C % 8 == 0 && taps <= 64) {
         const size_t bytes = packed || packs(bwd, g) ? stream_f32_packed_bytes(bwd, g) : 0;
-        if(bytes) {
+        // (without room for the copy: through the table, or the kernels that need less)
+        if(bytes && (packed || (ws && ws_bytes >= bytes && aligned16(ws)))) {
             if(!packed) {
-                if(!ws || ws_bytes < bytes || !aligned16(ws))
-                    return SAGA_HIP_EWORKSPACE;
                 PackArgs pa;
                 pa.n = pack_jobs(k, w->ptr, (float *)ws, pa.job);
                 const dim3 grid(grid_for((long long)bytes / 16 / k.nclasses, 256, 4096), pa.n);
@@ -720,9 +719,9 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
             return launch<PTAP, QLANE>(k, st, pixels, steps);
         }
         // 1x1: the filter as it is, if its rows are dense
-        if(!bwd && k.q_sc == 1)
+        if(!bytes && !bwd && k.q_sc == 1)
             return launch<PTAP, QROW>(k, st, pixels, steps);
-        if(bwd && k.q_sn == 1)
+        if(!bytes && bwd && k.q_sn == 1)
             return launch<PTAP, QCOL>(k, st, pixels, steps);
     }
     if(taps <= 63 && (long long)taps * k.C <= MAX_TABLE - 8)

@@ -34,3 +34,43 @@ def test_fp16_gradients_with_an_odd_pitch(k, padc, share):
     torch.cuda.synchronize()
     assert_close(host(dx), ref.conv2d_bwd_data(dy, w, x.shape, 1, 1), dt, "dx", tol=2e-3)
     assert_close(host(dw), ref.conv2d_bwd_filter(x, dy, w.shape, 1, 1), dt, "dw", tol=2e-3)
+
+
+# (c, k, r, stride): channels in eights and not, filters that are packed and that are read in place, residue classes
+F32 = [(16, 24, 3, 1), (16, 24, 3, 2), (24, 16, 1, 1), (16, 8, 1, 2), (8, 40, 5, 1), (7, 13, 3, 1)]
+
+
+@pytest.mark.parametrize("share", [0.3, 0.6, 1])
+@pytest.mark.parametrize("c,k,r,stride", F32)
+def test_fp32_convolutions(c, k, r, stride, share):
+    rng, dt = np.random.default_rng(1), torch.float32
+    pad = r // 2
+    x, w = rnd(rng, 4, c, 30, 30), rnd(rng, k, c, r, r, scale=1 / np.sqrt(c * r * r))
+    want = ref.conv2d_fwd(x, w, pad, stride)
+    dy = rnd(rng, *want.shape)
+    L, p, st = K.lib(), K.ConvParams(pad, stride, 1, 1), K.stream_ptr()
+    xd, wd, dyd = dev(x), dev(w), dev(dy)
+    y, dx, dw = (torch.empty_like(t) for t in (dyd, xd, wd))
+    vx, vw, vdy, vy, vdx, vdw = (K.view(t) for t in (xd, wd, dyd, y, dx, dw))
+    r_ = C.byref
+
+    def call(kind, fn, a, b, out):
+        """With the least whole kilobyte from `share` of the query's answer up that is accepted."""
+        n = L.saga_hip_conv2d_workspace_size(kind, r_(vx), r_(vw), r_(vdy), r_(p))
+        room = int(share * n) & ~1023
+        while True:
+            ws = torch.empty(max(room, 16), dtype=torch.uint8, device="cuda")
+            rc = fn(r_(a), r_(b), r_(out), r_(p), 1.0, 0.0, K.ptr(ws), room, st)
+            if rc != -4 or room > n:
+                break
+            room += 1024
+        K.check(rc)
+
+    call(K.CONV_FWD, L.saga_hip_conv2d_fwd, vx, vw, vy)
+    call(K.CONV_BWD_DATA, L.saga_hip_conv2d_bwd_data, vdy, vw, vdx)
+    call(K.CONV_BWD_FILTER, L.saga_hip_conv2d_bwd_filter, vx, vdy, vdw)
+    torch.cuda.synchronize()
+    # sums of up to 3600 products in fp32: rounding of some 1e-6 of the largest
+    assert_close(host(y), want, dt, "y", tol=1e-5)
+    assert_close(host(dx), ref.conv2d_bwd_data(dy, w, x.shape, pad, stride), dt, "dx", tol=1e-5)
+    assert_close(host(dw), ref.conv2d_bwd_filter(x, dy, w.shape, pad, stride), dt, "dw", tol=1e-5)

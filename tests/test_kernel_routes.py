@@ -47,3 +47,19 @@ def test_fp16_gradients_without_room_for_a_padded_copy(kind, k, pitch):
             assert gradient(kind, x, w, y, room) == (0, True, False), room
     if not odd:  # (such tensors have always needed theirs)
         assert gradient(kind, x, w, y, 0)[0] == -4
+
+
+@pytest.mark.parametrize("c,k,r", [(16, 64, 3), (8, 64, 5), (7, 13, 3)])
+@on_stub
+def test_fp32_filter_gradients_with_fewer_partials(c, k, r):
+    """The reduction is split as often as the workspace allows, down to once."""
+    p = K.ConvParams(r // 2, 1, 1, 1)
+    x, w, y = (image(a, *d, dtype=K.FLOAT) for a, d in ((X, (8, c, 28, 28)), (W, (k, c, r, r)), (Y, (8, k, 28, 28))))
+    L = K.lib()
+    need = L.saga_hip_conv2d_workspace_size(K.CONV_BWD_FILTER, C.byref(x), C.byref(w), C.byref(y), C.byref(p))
+    once = 4 * k * c * r * r
+    table = 64 * c * r * r + 1024  # more than the general kernel's table of offsets takes
+    assert need > 4 * (once + table)
+    for room, want in ((need, 0), (need // 2, 0), (once + table, 0), (once - 4, -4), (0, -4)):
+        rc = L.saga_hip_conv2d_bwd_filter(C.byref(x), C.byref(y), C.byref(w), C.byref(p), 1.0, 0.0, ROOM if room else None, room, None)
+        assert rc == want, (room, rc)
