@@ -159,7 +159,7 @@ int saga_hip_conv2d_pack_jobs(int kind, const SagaTensorView *x, const SagaTenso
 int saga_hip_filter_pack_batched(const SagaFilterPackJob *jobs_device, int njobs, int total_blocks, saga_stream_t stream);
 
 /* y = act(norm(conv(x, w) + beta * y + bias) + z): what a network puts behind a convolution, in its epilogue where its
- * kernel has one and otherwise in passes of their own.  bias: any view of K elements; norm: as in
+ * kernel has one and otherwise in passes of their own.  bias: K elements, as in saga_hip_bias_add; norm: as in
  * saga_hip_conv2d_fwd_bn_infer, without bias and beta, and SAGA_HIP_EUNSUPPORTED as there; z only with a norm; all optional.
  * The backward-data form is the forward pass of a transposed convolution with a bias (may be null); wt as in
  * saga_hip_conv2d_bwd_data_wt (may be null), or a packed fp32 filter. */
@@ -224,7 +224,8 @@ int saga_hip_conv2d_bwd_data_bnbwd(const SagaTensorView *dy, const SagaTensorVie
                                    const SagaTensorView *dx, const SagaConvParams *p, float alpha, float beta,
                                    void *workspace, size_t ws_bytes, SagaBnBwdLink *link, saga_stream_t stream);
 
-/* y[n,c,:,:] += b[c] : cudnnAddTensor of a {1,C,1,1} bias (src/cuda/cuda_dnn.cpp:39-68). b is fp32 or y's type. */
+/* y[n,c,:,:] += b[c] : cudnnAddTensor of a {1,C,1,1} bias (src/cuda/cuda_dnn.cpp:39-68). b is fp32 or y's type: a
+ * view of C elements at any constant distance (SAGA_HIP_EUNSUPPORTED without one). */
 int saga_hip_bias_add(const SagaTensorView *y, const SagaTensorView *b, saga_stream_t stream);
 /* db[c] = beta*db + sum_{n,h,w} dy : cudnnConvolutionBackwardBias (src/cuda/cuda_dnn.cpp:378-385). */
 size_t saga_hip_bias_bwd_workspace_size(const SagaTensorView *dy);

@@ -60,6 +60,23 @@ static inline int64_t view_elements(const SagaTensorView *v)
     return (int64_t)v->dims[0] * v->dims[1] * v->dims[2] * v->dims[3];
 }
 
+// A view read as a vector of all its elements in logical order: true if they are a constant number of elements apart (*step).
+static inline bool as_vector(const SagaTensorView *v, int64_t *step)
+{
+    *step = 1;
+    int64_t count = 1;
+    for(int i = 3; i >= 0; i--) {
+        if(v->dims[i] == 1)
+            continue;
+        if(count == 1)
+            *step = v->strides[i];
+        else if(v->strides[i] != count * *step)
+            return false;
+        count *= v->dims[i];
+    }
+    return true;
+}
+
 // Channels-last with a row pitch: element (n,c,h,w) at ((n*H+h)*W+w)*pitch + c.
 // pitch > C describes a channel slice of a wider NHWC tensor.
 struct CLInfo {

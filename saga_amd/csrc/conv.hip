@@ -112,9 +112,19 @@ static int add_bias(const SagaTensorView *bias, const SagaTensorView *out, int r
     return r || !relu ? r : saga_hip_act_fwd(SAGA_ACT_RELU, 0, out, out, 0.0f, stream);
 }
 
-static bool bias_ok(const SagaTensorView *bias, const SagaTensorView *out)
+static int check_bias(const SagaTensorView *bias, const SagaTensorView *out)
 {
-    return valid_view(bias) && view_elements(bias) == out->dims[1];
+    int64_t step;
+    if(!valid_view(bias) || view_elements(bias) != out->dims[1])
+        return SAGA_HIP_ESHAPE;
+    return as_vector(bias, &step) ? 0 : SAGA_HIP_EUNSUPPORTED;
+}
+
+// whether a kernel's epilogue can read it, which takes elements of this type next to each other
+static bool fuses(const SagaTensorView *bias, int dtype)
+{
+    int64_t step;
+    return bias && bias->dtype == dtype && as_vector(bias, &step) && step == 1;
 }
 
 int saga_hip_conv2d_fwd_ex(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
@@ -135,16 +145,16 @@ int saga_hip_conv2d_fwd_ex(const SagaTensorView *x, const SagaTensorView *w, con
     if(e->z || (e->relu && !e->bias))
         return SAGA_HIP_EUNSUPPORTED;
     const SagaTensorView *bias = e->bias;
-    if(bias && !bias_ok(bias, y))
-        return SAGA_HIP_ESHAPE;
+    if(bias && (r = check_bias(bias, y)))
+        return r;
     bool done = false;
     r = SAGA_HIP_EUNSUPPORTED;
     if(!force_direct()) {
         r = conv_mfma_fwd(x, w, y, g, 1.0f, beta, workspace, ws_bytes, st, nullptr, 0, nullptr, nullptr,
-                          bias && bias->dtype == SAGA_HALF && !e->relu ? bias->ptr : nullptr, &done);
+                          fuses(bias, SAGA_HALF) && !e->relu ? bias->ptr : nullptr, &done);
         if(r == SAGA_HIP_EUNSUPPORTED) {
             StreamEpilogue se;
-            done = bias && bias->dtype == SAGA_FLOAT;
+            done = fuses(bias, SAGA_FLOAT);
             if(done) {
                 se.bias = (const float *)bias->ptr;
                 se.relu = e->relu;
@@ -192,8 +202,8 @@ int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView
     int r = geometry(dx, w, dy, p, &g);
     if(r)
         return r;
-    if(bias && !bias_ok(bias, dx))
-        return SAGA_HIP_ESHAPE;
+    if(bias && (r = check_bias(bias, dx)))
+        return r;
     if(wt && !takes_wt(dy, w, dx, g))
         return SAGA_HIP_EUNSUPPORTED;
     hipStream_t st = as_stream(stream);
@@ -201,10 +211,10 @@ int saga_hip_conv2d_bwd_data_bias(const SagaTensorView *dy, const SagaTensorView
     r = SAGA_HIP_EUNSUPPORTED;
     if(!force_direct()) {
         r = conv_mfma_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, wt, nullptr,
-                               bias && bias->dtype == SAGA_HALF ? bias->ptr : nullptr, &done);
+                               fuses(bias, SAGA_HALF) ? bias->ptr : nullptr, &done);
         if(r == SAGA_HIP_EUNSUPPORTED) {
             StreamEpilogue e;
-            done = bias && bias->dtype == SAGA_FLOAT;
+            done = fuses(bias, SAGA_FLOAT);
             if(done)
                 e.bias = (const float *)bias->ptr;
             r = conv_f32_bwd_data(dy, w, dx, g, 1.0f, beta, workspace, ws_bytes, st, e, wt);

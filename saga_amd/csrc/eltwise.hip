@@ -278,9 +278,9 @@ int launch_convert(const SagaTensorView *src, const SagaTensorView *dst, float s
     return 0;
 }
 
-// y[row, c] += b[c] on channels-last rows.
+// y[row, c] += b[c * step] on channels-last rows.
 template <typename T, typename TB>
-__global__ void __launch_bounds__(256) bias_add_cl(T *y, int64_t pitch, const TB *b, int64_t rows, int C)
+__global__ void __launch_bounds__(256) bias_add_cl(T *y, int64_t pitch, const TB *b, int64_t step, int64_t rows, int C)
 {
     const int64_t total = rows * C;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -288,12 +288,12 @@ __global__ void __launch_bounds__(256) bias_add_cl(T *y, int64_t pitch, const TB
         const int64_t r = i / C;
         const int c = (int)(i - r * C);
         T *p = y + r * pitch + c;
-        *p = (T)((float)*p + (float)b[c]);
+        *p = (T)((float)*p + (float)b[c * step]);
     }
 }
 
 template <typename T, typename TB>
-__global__ void __launch_bounds__(256) bias_add_cf(T *y, int64_t npitch, const TB *b, int N, int C, int64_t HW)
+__global__ void __launch_bounds__(256) bias_add_cf(T *y, int64_t npitch, const TB *b, int64_t step, int N, int C, int64_t HW)
 {
     const int64_t total = (int64_t)N * C * HW;
     const int64_t stride = (int64_t)gridDim.x * blockDim.x;
@@ -302,7 +302,7 @@ __global__ void __launch_bounds__(256) bias_add_cf(T *y, int64_t npitch, const T
         const int c = (int)(nc % C);
         const int64_t n = nc / C;
         T *p = y + n * npitch + (int64_t)c * HW + (i - nc * HW);
-        *p = (T)((float)*p + (float)b[c]);
+        *p = (T)((float)*p + (float)b[c * step]);
     }
 }
 
@@ -652,6 +652,9 @@ int saga_hip_bias_add(const SagaTensorView *y, const SagaTensorView *b, saga_str
         return SAGA_HIP_EINVAL;
     if(view_elements(b) != y->dims[1])
         return SAGA_HIP_ESHAPE;
+    int64_t step;
+    if(!as_vector(b, &step))
+        return SAGA_HIP_EUNSUPPORTED;
     hipStream_t st = as_stream(stream);
     const int64_t total = view_elements(y);
     CLInfo cl;
@@ -659,10 +662,10 @@ int saga_hip_bias_add(const SagaTensorView *y, const SagaTensorView *b, saga_str
 #define BIAS_ADD(T, TB)                                                                                       \
     if(as_channels_last(y, &cl))                                                                              \
         bias_add_cl<T, TB><<<grid_for(total, 256, 256 * 32), 256, 0, st>>>((T *)y->ptr, cl.pitch,               \
-                                                                           (const TB *)b->ptr, cl.rows, cl.C); \
+                                                                           (const TB *)b->ptr, step, cl.rows, cl.C); \
     else if(as_channels_first(y, &cf))                                                                        \
         bias_add_cf<T, TB><<<grid_for(total, 256, 256 * 32), 256, 0, st>>>((T *)y->ptr, cf.npitch,              \
-                                                                           (const TB *)b->ptr, cf.N, cf.C, cf.HW); \
+                                                                           (const TB *)b->ptr, step, cf.N, cf.C, cf.HW); \
     else                                                                                                      \
         return SAGA_HIP_EUNSUPPORTED;
     if(y->dtype == SAGA_HALF && b->dtype == SAGA_HALF) {

@@ -769,7 +769,8 @@ void fc_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
     const bool transW = n.m_attributes.get("transW", false);
     const int in = x->m_dims[1], out = y->m_dims[1], batch = x->m_dims[0];
 
-    const bool takes = b && (b->m_data_type == Tensor::DataType::FLOAT || b->m_data_type == x->m_data_type);
+    // (the epilogue reads a dense vector)
+    const bool takes = b && b->rowMajor() && (b->m_data_type == Tensor::DataType::FLOAT || b->m_data_type == x->m_data_type);
     const T fused_b = takes && !p.m_pc.disable_op_fusing ? b : nullptr; // the bias goes along in the epilogue
     // y[batch,out] = x[batch,in] * W ; W stored [in,out], or [out,in] when transW
     pu.fwd(std::make_shared<Gemm>(0, transW ? 1 : 0, batch, out, in, x, in, w, transW ? in : out, y, out,

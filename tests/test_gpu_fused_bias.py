@@ -7,7 +7,9 @@ import pytest
 import torch
 
 from oracle import ref
+from saga_amd import api as S
 from saga_amd import kernels as K
+from saga_amd import networks as N
 from tests.gpu_util import assert_close, dev, host, rnd
 
 pytestmark = pytest.mark.gpu
@@ -113,3 +115,62 @@ def test_pooling(mode, k, stride, pad, dtype):
     K.check(K.lib().saga_hip_pool_fwd_relu(K.POOL_MAX if mode == "max" else K.POOL_AVG, C.byref(K.view(xd)), C.byref(K.view(yd)), k, pad,
                                            stride, K.stream_ptr()))
     np.testing.assert_allclose(host(yd), want, atol=2e-3 if dtype == HALF else 1e-6)
+
+
+@pytest.mark.parametrize("step", [2, 5])
+@pytest.mark.parametrize("name", ["fp16 small grid", "fp16 rows", "fp16 relu", "fp32 stream", "fp32 table"])
+def test_bias_with_gaps(name, step):
+    """A column of a matrix: read at its stride, in a pass of its own."""
+    dtype, N, Cc, H, W, Kk, R, stride, pad, relu = CONVS[name]
+    rng = np.random.default_rng(step)
+    x, wide = rnd(rng, N, Cc, H, W, dtype=dtype), rnd(rng, Kk, step, dtype=dtype)
+    w = rnd(rng, Kk, Cc, R, R, dtype=dtype, scale=(2.0 / (Cc * R * R)) ** 0.5)
+    b = wide[:, 1]
+    want = ref.conv2d_fwd(x, w, pad, stride) + b[None, :, None, None]
+    lay = layout(dtype)
+    xd, wd, bd = dev(x, dtype, lay), dev(w, dtype, lay), dev(wide, dtype)[:, 1]
+    yd = dev(np.full(want.shape, np.nan, np.float32), dtype, lay)
+    vx, vw, vb, vy, p = K.view(xd), K.view(wd), K.view(bd), K.view(yd), K.ConvParams(pad, stride, 1, 1)
+    assert list(vb.dims) == [Kk, 1, 1, 1] and vb.strides[0] == step
+    L, st = K.lib(), K.stream_ptr()
+    ws, n = workspace(K.CONV_FWD, vx, vw, vy, p)
+    e = K.ConvExtras(bias=C.pointer(vb), relu=relu)
+    K.check(L.saga_hip_conv2d_fwd_ex(C.byref(vx), C.byref(vw), C.byref(vy), C.byref(p), 0.0, C.byref(e), K.ptr(ws), n, st))
+    assert_close(host(yd), np.maximum(want, 0) if relu else want, dtype, name, tol=2e-3 if dtype == HALF else None)
+    if stride == 1:  # backward data of the same filter, with a bias per input channel
+        wide = rnd(rng, step, Cc, dtype=dtype).T.copy()
+        bd = dev(wide, dtype)[:, 0]
+        vb = K.view(bd)
+        ws, n = workspace(K.CONV_BWD_DATA, vx, vw, vy, p)
+        dy = rnd(rng, *want.shape, dtype=dtype)
+        dyd, dx = dev(dy, dtype, lay), dev(np.full(x.shape, np.nan, np.float32), dtype, lay)
+        K.check(L.saga_hip_conv2d_bwd_data_bias(C.byref(K.view(dyd)), C.byref(vw), None, C.byref(vb), C.byref(K.view(dx)), C.byref(p),
+                                                0.0, K.ptr(ws), n, st))
+        want = ref.conv2d_bwd_data(dy, w, x.shape, pad, stride) + wide[:, 0][None, :, None, None]
+        assert_close(host(dx), want, dtype, name + " transposed", tol=2e-3 if dtype == HALF else None)
+
+
+@pytest.mark.parametrize("dtype", [S.FLOAT, S.HALF], ids=["f32", "f16"])
+def test_bias_from_a_window(dtype):
+    """The same in a program: convolution and product with a column of a matrix as their bias."""
+    rng = np.random.default_rng(7)
+    draw = lambda *shape: rng.standard_normal(shape).astype(N.np_dtype(dtype))
+    x, w, m = draw(2, 8, 6, 6), draw(16, 8, 3, 3), draw(16, 3)
+    fx, fw, fm = draw(4, 24), draw(24, 16), draw(16, 3)
+
+    def column(g, a):
+        return g.add_node("window", {"x": S.Tensor.from_numpy(a)}, {"offset": [0, 1], "shape": [16, 1]}).y()
+
+    g = S.Graph()
+    y = g.add_node("conv", {"x": S.Tensor.from_numpy(x), "w": S.Tensor.from_numpy(w), "b": column(g, m)},
+                   {"size": 3, "activations": 16, "pad": 1, "bias": True}).y()
+    f = g.add_node("fc", {"x": S.Tensor.from_numpy(fx), "w": S.Tensor.from_numpy(fw), "b": column(g, fm)},
+                   {"outputs": 16, "bias": True}).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=False)
+    y, f = ctx.resolve(y), ctx.resolve(f)
+    p.run(1)
+    tol = 2e-3 if dtype == S.HALF else 1e-5
+    wide = lambda a: a.astype(np.float32)
+    assert_close(wide(y.read()), ref.conv2d_fwd(wide(x), wide(w), 1, 1) + wide(m)[None, :, 1, None, None], None, "conv", tol=tol)
+    assert_close(wide(f.read()), wide(fx) @ wide(fw) + wide(fm)[None, :, 1], None, "fc", tol=tol)

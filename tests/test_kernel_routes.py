@@ -63,3 +63,22 @@ def test_fp32_filter_gradients_with_fewer_partials(c, k, r):
     for room, want in ((need, 0), (need // 2, 0), (once + table, 0), (once - 4, -4), (0, -4)):
         rc = L.saga_hip_conv2d_bwd_filter(C.byref(x), C.byref(y), C.byref(w), C.byref(p), 1.0, 0.0, ROOM if room else None, room, None)
         assert rc == want, (room, rc)
+
+
+@on_stub
+def test_biases_that_are_no_vector_are_refused():
+    """Elements at no constant distance; a constant one other than 1 goes to a pass of its own."""
+    x, w, y, p = image(X, 2, 16, 9, 9), image(W, 16, 16, 3, 3), image(Y, 2, 16, 9, 9), K.ConvParams(1, 1, 1, 1)
+    L = K.lib()
+    n = L.saga_hip_conv2d_workspace_size(K.CONV_FWD, C.byref(x), C.byref(w), C.byref(y), C.byref(p))
+    for dims, strides, want, passes in (([1, 16, 1, 1], [16, 1, 1, 1], 0, 0), ([16, 1, 1, 1], [1, 1, 1, 1], 0, 0),
+                                        ([4, 1, 4, 1], [4, 9, 1, 9], 0, 0), ([1, 16, 1, 1], [1, 3, 1, 1], 0, 1),
+                                        ([4, 1, 4, 1], [12, 9, 3, 9], 0, 1), ([4, 4, 1, 1], [5, 1, 1, 1], -3, 0),
+                                        ([1, 15, 1, 1], [1, 1, 1, 1], -2, 0)):
+        b = image(1 << 33, 1, 16, 1, 1)
+        b.dims[:], b.strides[:] = dims, strides
+        before = stub_gpu.launches("bias_add")
+        e = K.ConvExtras(bias=C.pointer(b))
+        rc = L.saga_hip_conv2d_fwd_ex(C.byref(x), C.byref(w), C.byref(y), C.byref(p), 0.0, C.byref(e), ROOM, n, None)
+        assert (rc, stub_gpu.launches("bias_add") - before) == (want, passes), (dims, strides)
+        assert L.saga_hip_bias_add(C.byref(y), C.byref(b), None) == want
