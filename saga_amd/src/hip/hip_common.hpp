@@ -321,6 +321,9 @@ public:
     size_t m_arena_bytes = 0;    // size of the arena
     size_t m_planned_bytes = 0;  // sum of the sizes of the storages laid out in it
     void planMemory();
+    struct ArenaPlan;
+    ArenaPlan layOutArena();
+    void leaveArena(HipStorage &s);
     // somebody looks at this storage who did not when programs were finalized: operations that were folded into the one
     // that writes it become operations again, from the next step on
     void unfold(HipStorage *s);

@@ -214,16 +214,20 @@ std::shared_ptr<Tensor> HipContext::resolveTensor(std::shared_ptr<Tensor> src)
     unfold(it->second->m_storage.get());
     // a tensor the host holds keeps its contents between steps: out of the shared arena
     // (reference: src/cuda/cuda_common.cpp:145-158)
-    auto &st = it->second->m_storage;
-    if(st->m_in_arena) {
-        // memory of its own from here on; what the arena slot holds right now moves along
-        sync();
-        auto keep = st->m_memory;
-        void *old = st->m_data;
-        st->allocOwn();
-        chkHip(hipMemcpy(st->m_data, old, st->bytes(), hipMemcpyDeviceToDevice));
-    }
+    leaveArena(*it->second->m_storage);
     return it->second;
+}
+
+// Memory of its own from here on; what the arena slot holds right now moves along.
+void HipContext::leaveArena(HipStorage &st)
+{
+    if(!st.m_in_arena)
+        return;
+    sync();
+    const auto keep = st.m_memory;
+    void *old = st.m_data;
+    st.allocOwn();
+    chkHip(hipMemcpy(st.m_data, old, st.bytes(), hipMemcpyDeviceToDevice));
 }
 
 // Storage reuse.  A storage qualifies when, in every finalized program that touches it, the
@@ -235,11 +239,7 @@ std::shared_ptr<Tensor> HipContext::resolveTensor(std::shared_ptr<Tensor> src)
 // conflict.  The reference walks one program with a best-fit free list
 // (src/cuda/cuda_analysis.cpp:472-530); planning per context instead keeps an inference and a
 // training program that share activations from overwriting each other's tensors.
-void HipContext::planMemory()
-{
-    static const bool disabled = getenv("SAGA_HIP_NO_ARENA") != nullptr;
-    if(disabled)
-        return;
+struct HipContext::ArenaPlan {
     struct Range {
         int prog, first, last;
     };
@@ -249,6 +249,17 @@ void HipContext::planMemory()
         std::vector<Range> ranges;
     };
     std::unordered_map<HipStorage *, Item> items;
+    std::vector<Item *> placed;
+    size_t total = 0, planned = 0; // size of the arena, and of what is placed in it
+    size_t own = 0;                // what is still to be allocated outside of it
+};
+
+HipContext::ArenaPlan HipContext::layOutArena()
+{
+    using Range = ArenaPlan::Range;
+    using Item = ArenaPlan::Item;
+    ArenaPlan plan;
+    auto &items = plan.items;
     std::set<HipStorage *> carried;
     for(size_t pi = 0; pi < m_programs.size(); pi++) {
         const HipOps &ops = m_programs[pi]->m_ops;
@@ -294,8 +305,11 @@ void HipContext::planMemory()
     std::vector<Item *> cand;
     for(auto &kv : items) {
         HipStorage *st = kv.first;
-        if(carried.count(st) || exported.count(st) || st->doubleBuffered())
+        if(carried.count(st) || exported.count(st) || st->doubleBuffered()) {
+            leaveArena(*st); // (a later program starts from its contents)
+            plan.own += st->allocated() || st->doubleBuffered() ? 0 : st->bytes();
             continue;
+        }
         if(st->allocated() && !st->m_in_arena)
             continue;
         kv.second.bytes = (st->bytes() + 255) & ~(size_t)255;
@@ -311,11 +325,9 @@ void HipContext::planMemory()
                     return true;
         return false;
     };
-    std::vector<Item *> placed;
-    size_t total = 0, planned = 0;
     for(Item *it : cand) {
         std::vector<std::pair<size_t, size_t>> busy; // [begin, end) of conflicting storages
-        for(Item *q : placed)
+        for(Item *q : plan.placed)
             if(conflict(*it, *q))
                 busy.emplace_back(q->offset, q->offset + q->bytes);
         std::sort(busy.begin(), busy.end());
@@ -326,14 +338,57 @@ void HipContext::planMemory()
             off = std::max(off, b.second);
         }
         it->offset = off;
-        placed.push_back(it);
-        total = std::max(total, off + it->bytes);
-        planned += it->bytes;
+        plan.placed.push_back(it);
+        plan.total = std::max(plan.total, off + it->bytes);
+        plan.planned += it->bytes;
     }
+    return plan;
+}
+
+// Where operations run on a side stream, what they touch is in use for longer and the arena is larger; they need a workspace of
+// their own, too.  That is given up, one program after the other and the newest first, where all of it takes more than three
+// quarters of the memory that is free: what fits on one stream still fits, and elsewhere a quarter is left for what comes later.
+void HipContext::planMemory()
+{
+    static const bool disabled = getenv("SAGA_HIP_NO_ARENA") != nullptr;
+    auto allocSideWorkspace = [&] {
+        if(std::any_of(m_programs.begin(), m_programs.end(), [](const HipProgram *p) { return !p->m_side.empty(); })) {
+            m_side_workspace.request(m_workspace.size());
+            m_side_workspace.alloc();
+        }
+    };
+    if(disabled)
+        return allocSideWorkspace();
+    ArenaPlan plan = layOutArena();
+    // the old arena goes first: nothing in it is kept
+    for(const auto *it : plan.placed)
+        if(it->s->m_in_arena) {
+            it->s->rehome(nullptr, nullptr);
+            it->s->m_in_arena = true;
+        }
+    m_arena.reset();
+    for(size_t pi = m_programs.size(); pi-- > 0;) {
+        HipProgram *pr = m_programs[pi];
+        if(pr->m_side.empty())
+            continue;
+        size_t free_bytes = 0, total_bytes = 0;
+        chkHip(hipMemGetInfo(&free_bytes, &total_bytes));
+        const size_t workspace = m_workspace.size() - std::min(m_workspace.size(), m_side_workspace.size());
+        if(plan.total + plan.own + workspace <= free_bytes / 4 * 3)
+            break;
+        if(getenv("SAGA_HIP_VERBOSE"))
+            fprintf(stderr, "hip: program %d stays on one stream, %.1f of %.1f MB would be in use\n", pr->m_index,
+                    (plan.total + plan.own + workspace) / 1e6, free_bytes / 1e6);
+        pr->m_side.clear();
+        plan = layOutArena();
+    }
+    allocSideWorkspace();
+    const auto &placed = plan.placed;
+    const size_t total = plan.total, planned = plan.planned;
     if(placed.empty())
         return;
     auto arena = std::make_shared<HipMemory>(total); // zero filled once; slots are not cleared on reuse
-    for(Item *it : placed) {
+    for(const auto *it : placed) {
         it->s->rehome(arena, (char *)arena->m_ptr + it->offset);
         it->s->m_in_arena = true;
     }
@@ -341,7 +396,7 @@ void HipContext::planMemory()
         HipProgram *pr = m_programs[pi];
         pr->m_poison_before.assign(pr->m_ops.size(), {});
         pr->m_poison_after.assign(pr->m_ops.size(), {});
-        for(Item *it : placed)
+        for(const auto *it : placed)
             for(const auto &r : it->ranges)
                 if(r.prog == (int)pi) {
                     pr->m_poison_before[r.first].push_back(it->s);
@@ -931,8 +986,8 @@ void HipProgram::runOpsGraphed()
 // An event orders each such operation behind the last one of the main stream that writes what it reads, and the first
 // operation of the main stream that reads its results, or overwrites what it reads, behind it.  One with nothing left to run
 // beside it stays on the main stream: an edge between the streams costs more than a launch.  Storages that it touches have
-// their memory to themselves from the one edge to the other (planMemory); a program whose operations would hold more than an eighth of the GPU's
-// memory that way stays on one stream.
+// their memory to themselves from the one edge to the other; a program whose operations would hold more than an eighth of the GPU's
+// memory that way stays on one stream, and so does one that would not fit well otherwise (planMemory).
 void HipProgram::planSide()
 {
     m_side.clear();
@@ -1016,8 +1071,6 @@ void HipProgram::planSide()
     m_side = side;
     if(!m_ctx->m_side_stream)
         chkHip(hipStreamCreateWithFlags(&m_ctx->m_side_stream, hipStreamDefault));
-    m_ctx->m_side_workspace.request(m_ctx->m_workspace.size());
-    m_ctx->m_side_workspace.alloc();
 }
 
 void HipProgram::runOps(const HipOps &ops)

@@ -12,7 +12,7 @@
 
 namespace {
 
-size_t g_total = (size_t)288 << 30, g_used = 0;
+size_t g_total = (size_t)288 << 30, g_used = 0, g_peak = 0;
 std::map<void *, size_t> g_allocs;
 std::map<const void *, std::string> g_kernels;
 std::map<std::string, long> g_launches;
@@ -51,6 +51,13 @@ template <typename H> hipError_t new_handle(H *h)
 extern "C" {
 
 void hipstub_set_memory(size_t total) { g_total = total; }
+size_t hipstub_used(void) { return g_used; }
+size_t hipstub_peak(void) // since the last question
+{
+    const size_t p = g_peak;
+    g_peak = g_used;
+    return p;
+}
 long hipstub_launches(const char *kernel) // of kernels whose name contains this
 {
     long n = 0;
@@ -67,8 +74,10 @@ hipError_t hipMalloc(void **p, size_t bytes)
     if(g_used + ((bytes + 4095) & ~(size_t)4095) > g_total)
         return hipErrorOutOfMemory;
     const hipError_t e = map_memory(p, bytes);
-    if(e == hipSuccess)
+    if(e == hipSuccess) {
         g_used += g_allocs[*p];
+        g_peak = g_used > g_peak ? g_used : g_peak;
+    }
     return e;
 }
 hipError_t hipFree(void *p) { return unmap_memory(p, true); }

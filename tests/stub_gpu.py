@@ -47,6 +47,7 @@ def _child(libs, module, name, kwargs):
     stub = C.CDLL(os.path.join(libs, "hip_stub.so"), mode=C.RTLD_GLOBAL)  # before anything that needs the runtime
     stub.hipstub_set_memory.argtypes = [C.c_size_t]
     stub.hipstub_uploads.restype = C.c_long
+    stub.hipstub_used.restype = stub.hipstub_peak.restype = C.c_size_t
     stub.hipstub_launches.argtypes, stub.hipstub_launches.restype = [C.c_char_p], C.c_long
     api.lib()
     probe = C.CDLL(os.path.join(libs, "plan_probe.so"))

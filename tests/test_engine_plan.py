@@ -285,3 +285,45 @@ def test_another_program_reads_an_intermediate():
     q.finalize()
     (source, *_), = stub_gpu.plan(q)[0]["reads"]
     assert source in written(stub_gpu.plan(p))
+
+
+@pytest.mark.parametrize("with_inference", [False, True], ids=["training alone", "training and inference"])
+@pytest.mark.parametrize("name", ["lenet", "resnet20", "resnet20 behind large images"])
+@on_stub
+def test_what_fits_on_one_stream_fits(name, with_inference):
+    """The second stream is given up where memory is short, and only there."""
+    import gc
+    import os
+
+    def train():
+        ctx = S.Context()
+        if name.endswith("images"):
+            net = N.resnet20(16)
+            g = behind_resize(net, 1536)
+        else:
+            net = TRAINED[name]()
+            g, _ = N.build_graph(net, np.zeros((net.batch,) + tuple(net.in_shape), np.float32))
+        p = ctx.create_program(g, net.batch, training=True)
+        p.run(2)
+        if with_inference:
+            q = ctx.create_program(g, net.batch, training=False)
+            q.run(1)
+            p.run(1)
+        return any(op["side"] for op in stub_gpu.plan(p))
+
+    def run(total):
+        gc.collect()
+        start = stub_gpu.stub.hipstub_used()
+        stub_gpu.stub.hipstub_set_memory(total + start)
+        stub_gpu.stub.hipstub_peak()
+        side = train()
+        return stub_gpu.stub.hipstub_peak() - start, side
+
+    train()  # (what the library keeps)
+    os.environ["SAGA_HIP_ONE_STREAM"] = "1"
+    least, side = run(1 << 38)
+    assert not side
+    del os.environ["SAGA_HIP_ONE_STREAM"]
+    assert run(1 << 38)[1]
+    sides = [run(int(least * f))[1] for f in (1, 1.02, 1.1, 1.25, 1.5, 2, 40)]  # (running out of memory ends the process)
+    assert sides == sorted(sides) and sides[-1], sides
