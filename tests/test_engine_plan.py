@@ -9,10 +9,11 @@ from tests import stub_gpu
 from tests.stub_gpu import on_stub
 
 
-def behind_resize(net, image):
-    """The training graph of `net` behind a byte image that is converted and resized to the network's input."""
+def behind_resize(net, image, pixels=None):
+    """The training graph of `net` behind byte images that are converted and resized to the network's input, and its tensors."""
     g = S.Graph()
-    pixels = S.Tensor.placeholder(S.U8, [net.batch, 3, image, image], "pixels")
+    if pixels is None:
+        pixels = S.Tensor.placeholder(S.U8, [net.batch, 3, image, image], "pixels")
     c = g.add_node("convert", {"x": pixels}, {"scale": 1 / 255.0, "datatype": net.dtype})
     c = g.add_node("spatialtransform", {"x": c.y()}, {"height": net.in_shape[1], "width": net.in_shape[2]})
     t = {net.input: c.y()}
@@ -21,8 +22,9 @@ def behind_resize(net, image):
         t[name] = S.Tensor.from_numpy(a.astype(N.np_dtype(S.FLOAT if norm else net.dtype)), name=name)
     for n in net.nodes:
         t[n["out"]] = g.add_node(n["type"], {k: t[v] for k, v in n["in"].items()}, n["attrs"], n["name"]).y()
-    g.add_node("catclassifier", {"x": t[net.output]})
-    return g
+    head = g.add_node("catclassifier", {"x": t[net.output]})
+    t["loss"], t["labels"] = head.output("loss"), head.y().grad()
+    return g, t
 
 
 TRAINED = {
@@ -59,7 +61,7 @@ def test_operations_in_front_of_the_first_convolution_are_ordered(name, image):
     that memory."""
     net = TRAINED[name]()
     ctx = S.Context()
-    p = ctx.create_program(behind_resize(net, image), net.batch, training=True)
+    p = ctx.create_program(behind_resize(net, image)[0], net.batch, training=True)
     p.finalize()
     ops = stub_gpu.plan(p)
     kinds = [op["kind"] for op in ops]
@@ -279,12 +281,18 @@ def test_another_program_reads_an_intermediate():
     ctx.resolve(t["out"])
     p.finalize()
     h = S.Graph()
-    other = h.add_node("tanh", {"x": t["conv2"]}).y()
+    outs = [h.add_node("tanh", {"x": t[k]}).y() for k in ("conv2", "relu", "norm")]
     q = ctx.create_program(h, 2, training=False)
-    ctx.resolve(other)
+    for v in outs:
+        ctx.resolve(v)
     q.finalize()
-    (source, *_), = stub_gpu.plan(q)[0]["reads"]
-    assert source in written(stub_gpu.plan(p))
+    ops = stub_gpu.plan(p)
+    sources = [op["reads"][0] for op in stub_gpu.plan(q)]
+    assert {s for s, *_ in sources} <= set(written(ops))
+    # what it starts from shares memory with nothing: p runs to its end in between
+    for s, a, size, _ in sources:
+        for other, b, n, _ in [x for op in ops + stub_gpu.plan(q) for x in op["reads"] + op["writes"]]:
+            assert other == s or not a or not b or a + size <= b or b + n <= a
 
 
 @pytest.mark.parametrize("with_inference", [False, True], ids=["training alone", "training and inference"])
@@ -299,7 +307,7 @@ def test_what_fits_on_one_stream_fits(name, with_inference):
         ctx = S.Context()
         if name.endswith("images"):
             net = N.resnet20(16)
-            g = behind_resize(net, 1536)
+            g, _ = behind_resize(net, 1536)
         else:
             net = TRAINED[name]()
             g, _ = N.build_graph(net, np.zeros((net.batch,) + tuple(net.in_shape), np.float32))
