@@ -43,7 +43,8 @@ struct ConvStatsLink {
 };
 
 // A copy of filters in another layout, all of a program's in one launch: made again when one of the filters may have
-// changed (HipStorage::m_version), so in training once per step and in inference once.  The copies have memory of their own.
+// changed (HipStorage::m_version), so in training once per step and in inference once.  The copies have memory of their own,
+// except the transposed ones of training programs, which live in the arena from the launch to their last reader.
 struct FilterCopies : public HipOperation {
     struct Item {
         T w, copy;
