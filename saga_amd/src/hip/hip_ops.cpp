@@ -1181,9 +1181,13 @@ void reorder_sparse_first_writers(HipOps &ops)
 {
     if(getenv("SAGA_HIP_NO_WRITER_REORDER"))
         return;
+    auto sparse = [](const HipOp &op) -> ConvBwdData * {
+        auto *c = dynamic_cast<ConvBwdData *>(op.get());
+        return c && c->cp_.stride >= 2 && ((int)c->w_->m_dims[2] < c->cp_.stride || (int)c->w_->m_dims[3] < c->cp_.stride) ? c : nullptr;
+    };
     for(size_t i = 0; i < ops.size(); i++) {
-        auto *conv = dynamic_cast<ConvBwdData *>(ops[i].get());
-        if(!conv || conv->cp_.stride < 2 || ((int)conv->w_->m_dims[2] >= conv->cp_.stride && (int)conv->w_->m_dims[3] >= conv->cp_.stride))
+        auto *conv = sparse(ops[i]);
+        if(!conv)
             continue;
         const T &t = conv->dx_;
         bool first = true;
@@ -1194,7 +1198,7 @@ void reorder_sparse_first_writers(HipOps &ops)
         if(!first)
             continue;
         ssize_t last = -1;
-        bool ok = true;
+        bool ok = true, dense = false;
         for(size_t k = i + 1; k < ops.size() && ok; k++) {
             bool writes = false;
             for(const auto &o : ops[k]->listOutputs())
@@ -1204,10 +1208,13 @@ void reorder_sparse_first_writers(HipOps &ops)
                         ok = false;
                     writes = true;
                 }
-            if(writes)
+            if(writes) {
                 last = (ssize_t)k;
+                dense |= !sparse(ops[k]);
+            }
         }
-        if(!ok || last < 0)
+        // (among writers that are all of this kind the first one fills the tensor, whichever it is)
+        if(!ok || !dense)
             continue;
         for(size_t k = i + 1; k <= (size_t)last && ok; k++) {
             for(const auto &in : ops[k]->listInputs())

@@ -1040,6 +1040,8 @@ void HipProgram::planSide()
     }
     size_t free_bytes = 0, total_bytes = 0;
     chkHip(hipMemGetInfo(&free_bytes, &total_bytes));
+    if(any && held > total_bytes / 8 && getenv("SAGA_HIP_VERBOSE"))
+        fprintf(stderr, "hip: program %d stays on one stream, %.1f MB would be held for the other\n", m_index, held / 1e6);
     if(!any || held > total_bytes / 8)
         return;
     auto event = [&](hipEvent_t &e) {

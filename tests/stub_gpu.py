@@ -1,11 +1,13 @@
 """Tests of the engine's host side without a GPU: the real engine and kernel library over a HIP runtime whose device memory is
 host memory and whose launches do nothing (native/hip_stub.cpp).  The stub stands in for the runtime of a whole process, so each
 test runs in a child."""
+import atexit
 import ctypes as C
 import functools
 import importlib
 import json
 import os
+import shutil
 import subprocess
 import sys
 import tempfile
@@ -19,6 +21,7 @@ NATIVE = os.path.join(ROOT, "tests", "native")
 @functools.lru_cache(maxsize=1)
 def _built():
     out = tempfile.mkdtemp(prefix="saga_stub_")
+    atexit.register(shutil.rmtree, out, ignore_errors=True)
     for name in ("hip_stub", "plan_probe"):
         subprocess.check_call(["g++", "-O1", "-std=c++17", "-march=x86-64-v3", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__",
                                "-I", os.path.join(ROOT, "saga_amd", "src"), "-I", os.path.join(ROOT, "include"),

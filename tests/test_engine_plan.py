@@ -335,3 +335,29 @@ def test_what_fits_on_one_stream_fits(name, with_inference):
     assert run(1 << 38)[1]
     sides = [run(int(least * f))[1] for f in (1, 1.02, 1.1, 1.25, 1.5, 2, 40)]  # (running out of memory ends the process)
     assert sides == sorted(sides) and sides[-1], sides
+
+
+@pytest.mark.parametrize("others", [[1, 1], [1, 1, 3], [3, 1, 1]], ids=str)
+@on_stub
+def test_several_strided_writers_of_a_gradient(others):
+    """1x1 convolutions at stride 2 write a quarter of a gradient: those go behind a dense writer, if there is one, and the order
+    among themselves is left alone."""
+    rng = np.random.default_rng(2)
+    draw = lambda *shape: S.Tensor.from_numpy(rng.standard_normal(shape).astype(np.float16), name=f"p{shape}{rng.integers(1 << 40)}")
+    g = S.Graph()
+    x = g.add_node("conv", {"x": draw(2, 16, 8, 8), "w": draw(16, 16, 3, 3)}, {"size": 3, "activations": 16, "pad": 1}).y()
+    ys = [g.add_node("conv", {"x": x, "w": draw(16, 16, r, r)}, {"size": r, "activations": 16, "pad": r // 2, "stride": 2}).y() for r in others]
+    y = ys[0]
+    for other in ys[1:]:
+        y = g.add_node("sum", {"x0": y, "x1": other}).y()
+    y = g.add_node("fc", {"x": g.add_node("avgpool", {"x": y}, {"global": True}).y(), "w": draw(16, 10)}, {"outputs": 10}).y()
+    g.add_node("catclassifier", {"x": y})
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=True)
+    p.finalize()
+    ops = stub_gpu.plan(p)
+    gradient = [op for op in ops if op["kind"].startswith("convbwddata")]
+    filters = [size for op in gradient for _, _, size, name in op["reads"] if name == "w"]
+    want = [16 * 16 * r * r * 2 for r in others]
+    assert len(filters) == len(others) and sorted(filters) == sorted(want)
+    assert filters[0] == max(want)  # the dense one, where there is one, overwrites
