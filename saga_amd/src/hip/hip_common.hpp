@@ -236,6 +236,8 @@ std::set<HipStorage *> readBeforeWritten(const HipOps &ops);
 
 struct HipProgramUnit {
     Nodes m_transformed;
+    // inputs of the window and concat nodes, which transforms have taken out of the list: the views still read them
+    std::set<std::shared_ptr<Tensor>> m_aliased;
     int m_batch_size = 1;
     HipOps m_fwd, m_bwd, m_tail;
     void fwd(const HipOp &op) { m_fwd.push_back(op); }

@@ -831,14 +831,14 @@ void convert_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
 }
 REGISTER_HIP_OP("convert", convert_setup);
 
-Nodes convert_transform(HipProgram &, HipProgramUnit &, const Nodes &input)
+Nodes convert_transform(HipProgram &, HipProgramUnit &pu, const Nodes &input)
 {
     Nodes nodes = input;
     bool again = true;
     while(again) {
         again = false;
         for(auto &n : nodes) {
-            if(n->m_type != "convert")
+            if(n->m_type != "convert" || pu.m_aliased.count(n->y()))
                 continue;
             auto it = nodes.findSingleDownStreamNode(n->y(), "convert");
             if(it == nodes.end())
@@ -1354,8 +1354,11 @@ void batchnorm_fused_setup(HipProgram &p, HipProgramUnit &pu, const Node &n)
 }
 REGISTER_HIP_OP("batchnorm.persistent", batchnorm_fused_setup);
 
-bool single_consumer(const Nodes &nodes, const std::shared_ptr<Tensor> &t)
+// whether one node reads t, and no view of it exists
+bool single_consumer(const HipProgramUnit &pu, const Nodes &nodes, const std::shared_ptr<Tensor> &t)
 {
+    if(pu.m_aliased.count(t))
+        return false;
     int uses = 0;
     for(const auto &n : nodes)
         for(const auto &in : n->m_inputs)
@@ -1385,7 +1388,7 @@ std::shared_ptr<Node> fuse_bn(std::shared_ptr<Node> bn, std::shared_ptr<Node> su
 // bn,relu / bn,sum,relu runs of ADJACENT nodes become one fused node
 // (reference: batchnorm_relu_transform, :2326-2369; that one is limited to fp16 channels-last
 // training programs, the kernels here take any type and layout and fuse in inference too).
-Nodes batchnorm_relu_transform(HipProgram &p, HipProgramUnit &, const Nodes &nodes)
+Nodes batchnorm_relu_transform(HipProgram &p, HipProgramUnit &pu, const Nodes &nodes)
 {
     if(p.m_pc.disable_op_fusing)
         return nodes;
@@ -1396,14 +1399,14 @@ Nodes batchnorm_relu_transform(HipProgram &p, HipProgramUnit &, const Nodes &nod
         if(n->m_type == "batchnorm") {
             const auto bn_y = n->m_outputs["y"];
             if(i + 1 < count && nodes[i + 1]->m_type == "relu" && nodes[i + 1]->m_inputs["x"] == bn_y &&
-               single_consumer(nodes, bn_y)) {
+               single_consumer(pu, nodes, bn_y)) {
                 n = fuse_bn(nodes[i], nullptr, nodes[i + 1]);
                 i += 1;
             } else if(i + 2 < count && nodes[i + 1]->m_type == "sum" && nodes[i + 2]->m_type == "relu" &&
                       (nodes[i + 1]->m_inputs["x0"] == bn_y || nodes[i + 1]->m_inputs["x1"] == bn_y) &&
                       nodes[i + 1]->m_inputs["x0"] != nodes[i + 1]->m_inputs["x1"] &&
-                      nodes[i + 2]->m_inputs["x"] == nodes[i + 1]->m_outputs["y"] && single_consumer(nodes, bn_y) &&
-                      single_consumer(nodes, nodes[i + 1]->m_outputs["y"])) {
+                      nodes[i + 2]->m_inputs["x"] == nodes[i + 1]->m_outputs["y"] && single_consumer(pu, nodes, bn_y) &&
+                      single_consumer(pu, nodes, nodes[i + 1]->m_outputs["y"])) {
                 n = fuse_bn(nodes[i], nodes[i + 1], nodes[i + 2]);
                 i += 2;
             }
@@ -1981,6 +1984,7 @@ Nodes window_transform(HipProgram &p, HipProgramUnit &pu, const Nodes &nodes)
             continue;
         }
         auto x = p.lower(pu, n->m_inputs["x"]);
+        pu.m_aliased.insert(n->m_inputs["x"]);
         auto yh = n->m_outputs["y"];
         const std::vector<int> off = n->m_attributes.get("offset", std::vector<int>{});
         int64_t o = x->m_offset;
@@ -2022,6 +2026,7 @@ Nodes concat_transform(HipProgram &p, HipProgramUnit &pu, const Nodes &nodes)
             auto x = alias_of(y, xd, y->m_strides, y->m_offset + along * y->m_strides[axis], xh->namePostfix("alias"));
             x->copyFromHost(*xh); // inputs that carry values (graph inputs) are placed right away
             p.m_ctx->m_tensors[xh] = x;
+            pu.m_aliased.insert(xh);
             if(dy)
                 p.m_ctx->m_tensors[xh->grad()] = alias_of(dy, xd, dy->m_strides,
                                                           dy->m_offset + along * dy->m_strides[axis],

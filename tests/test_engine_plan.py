@@ -250,6 +250,41 @@ def test_a_window_onto_an_intermediate_keeps_it():
     assert sorted(op["kind"] for op in ops) == ["actfwd", "bninf", "convfwd"]
 
 
+@pytest.mark.parametrize("training", [False, True])
+@pytest.mark.parametrize("view", ["window", "concat"])
+@on_stub
+def test_views_of_a_norms_output_keep_it(view, training):
+    """A norm and the relu behind it are one operation, unless a view looks at what is between them."""
+    rng = np.random.default_rng(2)
+    draw = lambda *shape: S.Tensor.from_numpy(rng.standard_normal(shape).astype(np.float32), name=f"p{rng.integers(1 << 40)}")
+    g = S.Graph()
+    x = draw(2, 16, 6, 6)
+    y = g.add_node("conv", {"x": x, "w": draw(16, 16, 3, 3)}, {"size": 3, "activations": 16, "pad": 1}).y()
+    n = g.add_node("batchnorm", {"x": y, **norm_params(rng, 16)}).y()
+    a = g.add_node("relu", {"x": n}).y()
+    if view == "window":
+        b = g.add_node("window", {"x": n}, {"offset": [0, 0, 0, 0], "shape": [2, 16, 6, 6]}).y()
+    else:
+        other = g.add_node("conv", {"x": x, "w": draw(8, 16, 1, 1)}, {"size": 1, "activations": 8}).y()
+        b = g.add_node("concat", {"x0": n, "x1": other}, {"axis": 1}).y()
+    b = g.add_node("conv", {"x": b, "w": draw(16, 16 if view == "window" else 24, 1, 1)}, {"size": 1, "activations": 16}).y()
+    s = g.add_node("sum", {"x0": a, "x1": b}).y()
+    out = g.add_node("fc", {"x": g.add_node("avgpool", {"x": s}, {"global": True}).y(), "w": draw(16, 10)}, {"outputs": 10}).y()
+    if training:
+        g.add_node("catclassifier", {"x": out})
+    ctx = S.Context()
+    p = ctx.create_program(g, 2, training=training)
+    ctx.resolve(out)
+    p.finalize()
+    ops = [op for op in stub_gpu.plan(p) if op["kind"] != "filterpack"]
+    kinds = [op["kind"] for op in ops]
+    norm = kinds.index("bntrain" if training else "convfwd.bn")
+    assert "actfwd" in kinds[norm:]
+    (between, *_), = [w for w in ops[norm]["writes"] if w[3] == "y"]
+    readers = [op["kind"] for op in ops[norm + 1:] for s, *_ in op["reads"] if s == between]
+    assert "actfwd" in readers and "convfwd" in readers
+
+
 @on_stub
 def test_a_residual_that_is_computed_behind_the_convolution():
     """The addition cannot move in front of what it adds."""
