@@ -16,6 +16,8 @@ size_t g_total = (size_t)288 << 30, g_used = 0, g_peak = 0;
 std::map<void *, size_t> g_allocs;
 std::map<const void *, std::string> g_kernels;
 std::map<std::string, long> g_launches;
+std::string g_log; // kernel, grid and block of every launch, a line each
+dim3 g_grid, g_block;
 long g_uploads = 0;
 
 hipError_t map_memory(void **p, size_t bytes)
@@ -67,6 +69,13 @@ long hipstub_launches(const char *kernel) // of kernels whose name contains this
     return n;
 }
 
+const char *hipstub_log(void) // since the last question
+{
+    static std::string last;
+    last.swap(g_log);
+    g_log.clear();
+    return last.c_str();
+}
 long hipstub_uploads(void) { return g_uploads; } // asynchronous ones
 
 hipError_t hipMalloc(void **p, size_t bytes)
@@ -179,16 +188,24 @@ void __hipRegisterFunction(void **, const void *host, char *, const char *name, 
     g_kernels[host] = name;
 }
 void __hipRegisterVar(void **, void *, char *, const char *, int, size_t, int, int) {}
-hipError_t __hipPushCallConfiguration(dim3, dim3, size_t, hipStream_t) { return hipSuccess; }
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t, hipStream_t)
+{
+    g_grid = grid;
+    g_block = block;
+    return hipSuccess;
+}
 hipError_t __hipPopCallConfiguration(dim3 *g, dim3 *b, size_t *lds, hipStream_t *s)
 {
-    *g = *b = dim3(1, 1, 1);
+    *g = g_grid;
+    *b = g_block;
     *lds = 0;
     *s = nullptr;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **, size_t, hipStream_t)
+hipError_t hipLaunchKernel(const void *f, dim3 grid, dim3 block, void **, size_t, hipStream_t)
 {
+    if(g_log.size() < (1 << 20))
+        g_log += g_kernels[f] + " " + std::to_string(grid.x) + " " + std::to_string(block.x) + "\n";
     g_launches[g_kernels[f]]++;
     return hipSuccess;
 }

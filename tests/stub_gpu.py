@@ -7,6 +7,7 @@ import functools
 import importlib
 import json
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -51,6 +52,7 @@ def _child(libs, module, name, kwargs):
     stub.hipstub_set_memory.argtypes = [C.c_size_t]
     stub.hipstub_uploads.restype = C.c_long
     stub.hipstub_used.restype = stub.hipstub_peak.restype = C.c_size_t
+    stub.hipstub_log.restype = C.c_char_p
     stub.hipstub_launches.argtypes, stub.hipstub_launches.restype = [C.c_char_p], C.c_long
     api.lib()
     probe = C.CDLL(os.path.join(libs, "plan_probe.so"))
@@ -63,6 +65,18 @@ def _child(libs, module, name, kwargs):
 
 def launches(kernel):
     return stub.hipstub_launches(kernel.encode())
+
+
+def launched():
+    """The launches since the last call: (kernel, its whole-number template arguments, blocks, threads)."""
+    out = []
+    for line in stub.hipstub_log().decode().splitlines():
+        name, grid, block = line.rsplit(" ", 2)
+        m = re.match(r"_ZN12_GLOBAL__N_1(\d+)", name) or re.match(r"_Z(\d+)", name)
+        base, rest = name[m.end():m.end() + int(m.group(1))], name[m.end() + int(m.group(1)):]
+        # (the arguments of the function behind the template's hold no such numbers)
+        out.append((base, tuple(int(v) for v in re.findall(r"L[ib](\d+)E", rest)), int(grid), int(block)))
+    return out
 
 
 def uploads():

@@ -14,22 +14,35 @@ from tests.gpu_util import assert_close, dev, host, rnd
 pytestmark = pytest.mark.gpu
 HALF = torch.float16
 
-# N, C, H, W, K, R, stride, pad
+# N, C, H, W, K, R, stride, pad.  The names say what the rules choose, forward and, where it is something else, backward
+# (tests/test_kernel_routes.py holds them to it): pixels x channels of a wavefront's tile and what the block's wavefronts share.
 SHAPES = {
-    "16x16, eight along the reduction": (1, 400, 5, 6, 72, 3, 1, 1),
-    "16x16, four along the reduction": (1, 256, 6, 7, 40, 3, 1, 1),
-    "16x16, two and two": (2, 512, 5, 5, 24, 1, 1, 0),
-    "16x16, four along the pixels": (3, 256, 9, 9, 64, 1, 1, 0),
-    "32x32, four along the reduction": (2, 64, 30, 31, 128, 3, 1, 1),
-    "32x32, eight along the reduction": (4, 256, 14, 13, 248, 3, 1, 1),
-    "32x32, two and two": (1, 72, 50, 53, 256, 3, 1, 1),
-    "64x32, eight along the reduction": (8, 384, 7, 13, 512, 3, 1, 1),
-    "64x64, four along the reduction": (1, 256, 50, 53, 256, 3, 1, 1),
-    "residue classes": (3, 64, 19, 17, 48, 3, 2, 1),
-    "classes no tap reaches": (2, 64, 11, 12, 64, 1, 2, 0),
-    "shared 256x128 tiles": (1, 720, 29, 28, 480, 3, 1, 1),
-    "shared 256x64 tiles": (1, 256, 120, 122, 64, 3, 1, 1),
-    "shared tiles of residue classes": (1, 512, 60, 59, 1024, 3, 2, 1),
+    "16x16, four along the pixels": (1, 80, 10, 11, 24, 1, 1, 0),
+    "16x16, four along the reduction": (1, 136, 5, 4, 152, 1, 1, 0),
+    "16x16, four along the reduction (3x3)": (1, 400, 5, 6, 72, 3, 1, 1),
+    "16x16, four along the reduction (whole slices)": (1, 256, 6, 7, 40, 3, 1, 1),
+    "16x16, four along the reduction; backward 16x16, four along the pixels": (2, 512, 5, 5, 24, 1, 1, 0),
+    "16x16, four along the reduction; backward 16x16, four along the pixels (three images)": (3, 256, 9, 9, 64, 1, 1, 0),
+    "32x32, two and two": (1, 176, 69, 70, 56, 1, 1, 0),
+    "32x32, four along the reduction": (1, 104, 27, 26, 168, 1, 1, 0),
+    "32x32, four along the reduction; backward 16x16, four along the reduction": (2, 64, 30, 31, 128, 3, 1, 1),
+    "32x32, four along the reduction (3x3)": (4, 256, 14, 13, 248, 3, 1, 1),
+    "64x32, two and two": (5, 72, 45, 44, 80, 3, 1, 1),
+    "64x32, eight along the reduction": (3, 232, 22, 24, 232, 1, 1, 0),
+    "64x32, eight along the reduction (3x3)": (8, 384, 7, 13, 512, 3, 1, 1),
+    "64x64, two and two": (5, 464, 24, 23, 488, 1, 1, 0),
+    "64x64, four along the reduction": (1, 488, 38, 40, 496, 1, 1, 0),
+    "64x64, four along the reduction (3x3)": (1, 256, 50, 53, 256, 3, 1, 1),
+    "64x64, four along the reduction; backward 32x32, four along the reduction": (1, 72, 50, 53, 256, 3, 1, 1),
+    "16x16, four along the reduction; backward classes of 32x32, four along the reduction": (3, 64, 19, 17, 48, 3, 2, 1),
+    "16x16, four along the pixels; backward classes, some that no tap reaches, of 16x16, four along the pixels": (2, 64, 11, 12, 64, 1, 2, 0),
+    "64x64, four along the reduction; backward classes of 64x64, two and two": (1, 512, 60, 59, 1024, 3, 2, 1),
+    "shared 256x128 tiles": (1, 1048, 8, 7, 1048, 5, 1, 2),
+    "shared 256x64 tiles; backward 256x128 tiles": (1, 816, 66, 65, 40, 3, 1, 1),
+    "backward shared 256x64 tiles": (5, 48, 40, 41, 760, 3, 1, 1),
+    "backward classes of shared 256x128 tiles": (1, 592, 40, 41, 1016, 3, 2, 1),
+    "64x32, eight along the reduction; backward 64x64, four along the reduction": (1, 720, 29, 28, 480, 3, 1, 1),
+    "64x64, four along the reduction; backward 256x128 tiles": (1, 256, 120, 122, 64, 3, 1, 1),
 }
 
 

@@ -28,10 +28,12 @@ def layout(dtype):
 # N, C, H, W, K, R, stride, pad, relu
 CONVS = {
     "fp16 small grid": (HALF, 2, 64, 9, 11, 40, 3, 1, 1, 0),
-    "fp16 shared tiles": (HALF, 1, 720, 29, 28, 480, 3, 1, 1, 0),
+    "fp16 larger tile of a small grid": (HALF, 1, 720, 29, 28, 480, 3, 1, 1, 0),
+    "fp16 shared tiles": (HALF, 1, 1048, 8, 7, 1048, 5, 1, 2, 0),
     "fp16 tiles of 128 channels": (HALF, 8, 32, 91, 90, 136, 3, 1, 1, 0),
     "fp16 tiles of 64 channels": (HALF, 8, 64, 97, 94, 12, 1, 1, 0, 0),
-    "fp16 rows": (HALF, 32, 64, 56, 56, 64, 3, 1, 1, 0),
+    "fp16 tiles of 64 channels (3x3)": (HALF, 32, 64, 56, 56, 64, 3, 1, 1, 0),
+    "fp16 rows": (HALF, 40, 64, 56, 56, 64, 3, 1, 1, 0),
     "fp16 thin": (HALF, 2, 3, 40, 41, 24, 7, 2, 3, 0),
     "fp16 relu": (HALF, 2, 16, 9, 9, 8, 3, 1, 1, 1),
     "fp32 stream": (F32, 2, 24, 11, 13, 40, 3, 2, 1, 1),
@@ -64,7 +66,8 @@ def test_convolution(name):
 TRANSPOSED = {
     "fp16 small grid": (HALF, 1, 64, 22, 24, 128, 2, 2, 0),
     "fp16 tiles": (HALF, 6, 64, 128, 130, 128, 2, 2, 0),
-    "fp16 shared tiles": (HALF, 1, 512, 60, 59, 1024, 3, 2, 1),
+    "fp16 larger tile of a small grid": (HALF, 1, 512, 60, 59, 1024, 3, 2, 1),
+    "fp16 shared tiles": (HALF, 1, 592, 40, 41, 1016, 3, 2, 1),
     "fp16 classes no tap reaches": (HALF, 2, 64, 90, 91, 64, 1, 2, 0),
     "fp32": (F32, 2, 24, 12, 13, 32, 2, 2, 0),
     "fp32 accumulating": (F32, 2, 8, 10, 9, 16, 3, 1, 1),

@@ -14,18 +14,26 @@ from tests.gpu_util import assert_close, dev, host, rnd
 pytestmark = pytest.mark.gpu
 F32 = torch.float32
 
-# N, C, H, W, K, R, stride, pad
+# N, C, H, W, K, R, stride, pad: what the launch rule chooses forward (tests/test_kernel_routes.py holds it to that)
 CONVS = [
+    # filters read in place or through the table
     (2, 8, 255, 257, 65, 1, 1, 0),    # 64x64 tiles, four along the pixels
-    (1, 128, 150, 161, 64, 3, 1, 1),  # 64x64 tiles, the reduction over four wavefronts
-    (1, 48, 127, 131, 30, 3, 1, 1),   # 64x32 tiles, the reduction over four
+    (1, 1032, 79, 80, 200, 1, 1, 0),  # 64x64 tiles, the reduction over four wavefronts
+    (1, 392, 90, 92, 40, 1, 1, 0),    # 64x32 tiles, the reduction over four
     (1, 16, 311, 317, 7, 1, 1, 0),    # 64x32 tiles, four along the pixels
-    (1, 512, 3, 5, 33, 3, 1, 1),      # 32x32, sixteen wavefronts along the reduction
     (3, 64, 9, 7, 31, 1, 1, 0),       # 32x32, few steps per wavefront
-    (2, 24, 11, 13, 40, 3, 2, 1),     # residue classes backward, tap-major copy
-    (2, 16, 10, 9, 24, 2, 3, 0),      # stride beyond the filter: classes no tap reaches
     (2, 13, 12, 11, 9, 5, 2, 2),      # table: channels in other numbers than eights
     (1, 3, 23, 29, 16, 7, 2, 3),
+    # packed filters
+    (1, 24, 180, 183, 72, 3, 1, 1),   # 64x64 tiles, four along the pixels
+    (1, 24, 311, 317, 24, 3, 1, 1),   # 64x32 tiles, four along the pixels
+    (1, 40, 157, 158, 64, 3, 1, 1),   # 32x32, four along the pixels
+    (1, 16, 141, 142, 64, 3, 1, 1),   # 32x32, two and two
+    (1, 128, 150, 161, 64, 3, 1, 1),  # 32x32, the reduction over four
+    (1, 48, 127, 131, 30, 3, 1, 1),
+    (1, 512, 3, 5, 33, 3, 1, 1),      # 32x32, sixteen wavefronts along the reduction
+    (2, 24, 11, 13, 40, 3, 2, 1),     # residue classes backward
+    (2, 16, 10, 9, 24, 2, 3, 0),      # stride beyond the filter: classes no tap reaches
     (2, 8, 9, 9, 8, 3, 4, 1),
 ]
 

@@ -1,5 +1,6 @@
 """Which kernels the library's entry points launch, and what they refuse, without a GPU (over the stub runtime)."""
 import ctypes as C
+import re
 
 import pytest
 
@@ -82,3 +83,109 @@ def test_biases_that_are_no_vector_are_refused():
         rc = L.saga_hip_conv2d_fwd_ex(C.byref(x), C.byref(w), C.byref(y), C.byref(p), 0.0, C.byref(e), ROOM, n, None)
         assert (rc, stub_gpu.launches("bias_add") - before) == (want, passes), (dims, strides)
         assert L.saga_hip_bias_add(C.byref(y), C.byref(b), None) == want
+
+
+def convolution(kind, shape, dtype, bias=False):
+    """The launches of a convolution of dense tensors (forward: also with a bias), and the pixels of its classes and its columns."""
+    n, c, h, w, k, r, stride, pad = shape
+    p, q = 1 + (h + 2 * pad - r) // stride, 1 + (w + 2 * pad - r) // stride
+    x, f, y = (image(a, *d, dtype=dtype) for a, d in ((X, (n, c, h, w)), (W << 2, (k, c, r, r)), (Y << 3, (n, k, p, q))))
+    if dtype == K.FLOAT:  # channels-first
+        for v in (x, f, y):
+            d = v.dims
+            v.strides[:] = [d[1] * d[2] * d[3], d[2] * d[3], d[3], 1]
+    L, cp = K.lib(), K.ConvParams(pad, stride, 1, 1)
+    room = L.saga_hip_conv2d_workspace_size(kind, C.byref(x), C.byref(f), C.byref(y), C.byref(cp))
+    b = image(1 << 35, 1, k if kind == K.CONV_FWD else c, 1, 1, dtype=dtype)
+    stub_gpu.launched()
+    if kind == K.CONV_FWD:
+        e = K.ConvExtras(bias=C.pointer(b)) if bias else K.ConvExtras()
+        rc = L.saga_hip_conv2d_fwd_ex(C.byref(x), C.byref(f), C.byref(y), C.byref(cp), 0.0, C.byref(e), 1 << 36, room, None)
+    else:
+        rc = L.saga_hip_conv2d_bwd_data_bias(C.byref(y), C.byref(f), None, C.byref(b) if bias else None, C.byref(x), C.byref(cp), 0.0,
+                                             1 << 36, room, None)
+    assert rc == 0
+    classes = [n * p * q] if kind == K.CONV_FWD else [n * -(-(h - a) // stride) * -(-(w - b) // stride) for a in range(stride) for b in range(stride)]
+    return stub_gpu.launched(), classes, k if kind == K.CONV_FWD else c
+
+
+def small_grid_tile(launches, classes, columns):
+    """What tests/test_gpu_conv_small_grids.py calls it."""
+    split = {(1, 4): "four along the pixels", (2, 2): "two and two", (4, 1): "four along the reduction", (8, 1): "eight along the reduction"}
+    for name, t, blocks, threads in launches:
+        if name == "stream_f16_k":
+            tm, tn = t[:2]
+            for (ks, wm), text in split.items():
+                if threads == 64 * ks * wm and blocks == sum(-(-m // (16 * tm * wm)) for m in classes) * -(-columns // (16 * tn)):
+                    return f"{16 * tm}x{16 * tn}, {text}"
+    shared = any(name == "split_reduce" for name, *_ in launches)
+    (tile,) = [t for name, t, *_ in launches if name == "conv_gather_gemm_dma"]
+    return f"{'shared ' if shared else ''}{tile[0]}x{tile[1]} tiles"
+
+
+@on_stub
+def test_fp16_small_grid_shapes_are_what_their_names_say():
+    from tests.test_gpu_conv_small_grids import SHAPES
+
+    seen = set()
+    for name, shape in SHAPES.items():
+        text = re.sub(r" \([^)]*\)", "", name).replace(", some that no tap reaches,", "")
+        forward, _, backward = text.partition("; backward ")
+        if forward.startswith("backward "):
+            forward, backward = None, forward[len("backward "):]
+        for kind, want in ((K.CONV_FWD, forward), (K.CONV_BWD_DATA, backward or forward)):
+            if want is None:
+                continue
+            launches, classes, columns = convolution(kind, shape, K.HALF)
+            assert want.startswith("classes of ") == (len(classes) > 1), name
+            want = want.replace("classes of ", "")
+            got = small_grid_tile(launches, classes, columns)
+            assert got == want, (name, kind, got)
+            seen.add((kind, len(classes) > 1, got))
+    small = ["16x16, four along the pixels", "16x16, four along the reduction", "32x32, two and two", "32x32, four along the reduction",
+             "64x32, two and two", "64x32, eight along the reduction", "64x64, two and two", "64x64, four along the reduction"]
+    for kind in (K.CONV_FWD, K.CONV_BWD_DATA):
+        for tile in small + ["shared 256x128 tiles", "shared 256x64 tiles"]:
+            assert (kind, False, tile) in seen, (kind, tile)
+    assert (K.CONV_BWD_DATA, True, "shared 256x128 tiles") in seen
+
+
+# tile rows and columns in 32s, wavefronts along the reduction and along the pixels
+F32_TILES = {(2, 8, 255, 257, 65, 1, 1, 0): (2, 2, 1, 4), (1, 1032, 79, 80, 200, 1, 1, 0): (2, 2, 4, 1), (1, 392, 90, 92, 40, 1, 1, 0): (2, 1, 4, 1),
+             (1, 16, 311, 317, 7, 1, 1, 0): (2, 1, 1, 4), (3, 64, 9, 7, 31, 1, 1, 0): (1, 1, 1, 4), (1, 24, 180, 183, 72, 3, 1, 1): (2, 2, 1, 4),
+             (1, 24, 311, 317, 24, 3, 1, 1): (2, 1, 1, 4), (1, 40, 157, 158, 64, 3, 1, 1): (1, 1, 1, 4), (1, 16, 141, 142, 64, 3, 1, 1): (1, 1, 2, 2),
+             (1, 128, 150, 161, 64, 3, 1, 1): (1, 1, 4, 1), (1, 512, 3, 5, 33, 3, 1, 1): (1, 1, 16, 1)}
+
+
+@on_stub
+def test_fp32_shapes_are_what_their_comments_say():
+    from tests.test_gpu_stream_f32 import CONVS
+
+    assert set(F32_TILES) <= set(CONVS)
+    for shape, (tm, tn, ks, wm) in F32_TILES.items():
+        launches, (pixels,), columns = convolution(K.CONV_FWD, shape, K.FLOAT)
+        (tile,) = [x for x in launches if x[0] == "stream_f32_k"]
+        assert tile[1][2:4] == (tm, tn) and tile[3] == 64 * ks * wm, (shape, tile)
+        assert tile[2] == -(-pixels // (32 * tm * wm)) * -(-columns // (32 * tn)), (shape, tile)
+        assert (tile[1][1] == 3) == any(x[0] == "stream_pack_call" for x in launches) == (shape[5] > 1)
+
+
+BIAS_KERNELS = {"small grid": "stream_f16_k", "larger tile of a small grid": "stream_f16_k", "shared tiles": "split_reduce",
+                "tiles": "conv_gather_gemm_dma", "rows": "conv_rows64", "thin": "conv_thin_rows", "stream": "stream_f32_k", "table": "stream_f32_k"}
+
+
+@on_stub
+def test_fused_bias_shapes_are_what_their_names_say():
+    import torch
+
+    from tests.test_gpu_fused_bias import CONVS, TRANSPOSED
+
+    for table, kind in ((CONVS, K.CONV_FWD), (TRANSPOSED, K.CONV_BWD_DATA)):
+        for name, (dtype, *shape) in table.items():
+            launches = [x[0] for x in convolution(kind, shape[:8], K.HALF if dtype == torch.float16 else K.FLOAT, bias=True)[0]]
+            what = max((k for k in BIAS_KERNELS if k in name), key=len, default=None)
+            if what == "tiles" and dtype == torch.float32:
+                assert any(x.startswith("conv_f32_gather") for x in launches), (name, launches)
+            elif what:
+                assert any(x.startswith(BIAS_KERNELS[what]) for x in launches), (name, launches)
+                assert ("split_reduce" in launches) == (what == "shared tiles"), (name, launches)
