@@ -43,6 +43,9 @@ SHAPES = {
     "backward classes of shared 256x128 tiles": (1, 592, 40, 41, 1016, 3, 2, 1),
     "64x32, eight along the reduction; backward 64x64, four along the reduction": (1, 720, 29, 28, 480, 3, 1, 1),
     "64x64, four along the reduction; backward 256x128 tiles": (1, 256, 120, 122, 64, 3, 1, 1),
+    "32x32, four along the reduction; backward classes of 64x32, eight along the reduction": (3, 168, 21, 23, 240, 1, 2, 0),
+    "256x64 tiles": (3, 48, 70, 71, 48, 1, 1, 0),
+    "256x128 tiles": (5, 112, 45, 47, 112, 1, 1, 0),
 }
 
 

@@ -71,6 +71,9 @@ TRANSPOSED = {
     "fp16 classes no tap reaches": (HALF, 2, 64, 90, 91, 64, 1, 2, 0),
     "fp32": (F32, 2, 24, 12, 13, 32, 2, 2, 0),
     "fp32 accumulating": (F32, 2, 8, 10, 9, 16, 3, 1, 1),
+    "fp32 larger filter": (F32, 2, 24, 30, 31, 16, 9, 1, 4),
+    "fp32 larger stride": (F32, 1, 72, 31, 32, 8, 5, 5, 0),
+    "fp32 tiles": (F32, 8, 72, 182, 183, 8, 1, 1, 0),
 }
 
 

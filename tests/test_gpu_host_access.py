@@ -1,9 +1,13 @@
 """Host access to device tensors: Tensor.write and Tensor.read move every element to its place and back, whatever the
 layout of the device tensor, the size (staged, whole, sample by sample) and the number of channels."""
+import ctypes
+
 import numpy as np
 import pytest
+import torch
 
 from saga_amd import api as S
+from saga_amd import kernels as K
 
 pytestmark = pytest.mark.gpu
 
@@ -65,3 +69,27 @@ def test_slices_of_a_wider_tensor(layout):
     da.write(a + 1)
     np.testing.assert_array_equal(da.read(), a + 1)
     np.testing.assert_array_equal(dy.read(), np.concatenate([a + 1, b], 1))
+
+
+# the tile of a transposition is 64 channels by up to 1024 pixels; the third layout has none of its own
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (2, 3, 33, 65), (2, 64, 8, 8), (3, 65, 1, 9), (2, 130, 5, 13)])
+@pytest.mark.parametrize("dtype", ["uint8", "int16", "int32", "int64"])
+def test_copies_of_bit_patterns(shape, dtype):
+    t = torch.from_numpy(np.random.default_rng(len(dtype)).integers(0, 256, shape).astype(dtype))
+    t = (t * 127).cuda()
+    n, c, h, w = shape
+
+    def like(order):
+        wide = torch.full((n, c, h, w) if order == "nchw" else (w, h, n, c + 1) if order == "whnc" else (n, h, w, c + (order == "slice")), 7,
+                          dtype=t.dtype, device="cuda")
+        return wide, {"nchw": lambda: wide, "nhwc": lambda: wide.permute(0, 3, 1, 2), "slice": lambda: wide[..., :c].permute(0, 3, 1, 2),
+                      "whnc": lambda: wide[..., :c].permute(2, 3, 1, 0)}[order]()
+
+    for a in ("nchw", "nhwc", "slice", "whnc"):
+        for b in ("nchw", "nhwc", "slice", "whnc"):
+            (_, src), (wide, dst) = like(a), like(b)
+            src.copy_(t)
+            K.check(K.lib().saga_hip_copy(ctypes.byref(K.view(src)), ctypes.byref(K.view(dst)), K.stream_ptr()))
+            assert torch.equal(dst, t), (a, b)
+            if b in ("slice", "whnc"):
+                assert bool((wide[..., c] == 7).all()), (a, b)

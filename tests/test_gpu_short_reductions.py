@@ -47,7 +47,7 @@ def test_gemm_split_fp32(M, N, Kd, tA, tB):
     assert_close(host(Cd), 0.5 * (A.astype(np.float64) @ B) + 1, F32, "gemm", tol=1e-5)
 
 
-@pytest.mark.parametrize("layout,padc,dtype", [("nhwc", 0, HALF), ("nhwc", 8, HALF), ("nchw", 0, F32), ("nhwc", 0, F32)])
+@pytest.mark.parametrize("layout,padc,dtype", [("nhwc", 0, HALF), ("nhwc", 8, HALF), ("nchw", 0, HALF), ("nchw", 0, F32), ("nhwc", 0, F32)])
 @pytest.mark.parametrize("k,pad,stride,H", [(4, 0, 4, 9), (7, 0, 7, 7), (8, 3, 2, 12), (15, 0, 1, 15), (16, 0, 1, 17), (31, 2, 3, 33),
                                             (90, 0, 1, 90)])
 def test_average_shared_by_lanes(k, pad, stride, H, layout, padc, dtype):
@@ -84,6 +84,23 @@ def test_bias_gradient_of_planes(shape, dtype):
     K.check(K.lib().saga_hip_bias_bwd(C.byref(K.view(dev(y, dtype))), C.byref(K.view(db.view(1, shape[1], 1, 1))), 1.0, None, 0, S()))
     scale = np.abs(y.astype(np.float64)).sum(axis=(0, 2, 3)).max()
     assert np.abs(host(db) - (ref.bias_bwd(y) + 1)).max() <= 2e-6 * scale + 1e-6
+
+
+# the gradient in the tensor's own 16-bit type: 2**-10 of it is more than its rounding (channels-last, the last two: in two passes)
+@pytest.mark.parametrize("layout,padc", [("nchw", 0), ("nhwc", 0), ("nhwc", 3)])
+@pytest.mark.parametrize("shape", [(1, 3, 1, 1), (5, 7, 13, 13), (2, 64, 129, 65), (1, 67, 127, 126)])
+def test_bias_gradient_of_16_bits(shape, layout, padc):
+    rng = np.random.default_rng(shape[0])
+    y = rnd(rng, *shape, dtype=HALF)
+    yd, db = dev(y, HALF, layout, padc), dev(np.ones(shape[1], np.float32), HALF)
+    yv = K.view(yd)
+    room = K.lib().saga_hip_bias_bwd_workspace_size(C.byref(yv))
+    assert (room > 0) == (layout == "nhwc" and y.size >= 1 << 20)
+    ws = torch.empty(max(room, 4), dtype=torch.uint8, device="cuda")
+    K.check(K.lib().saga_hip_bias_bwd(C.byref(yv), C.byref(K.view(db.view(1, shape[1], 1, 1))), 1.0, K.ptr(ws) if room else None, room, S()))
+    want = ref.bias_bwd(y) + 1
+    scale = np.abs(y.astype(np.float64)).sum(axis=(0, 2, 3)).max()
+    assert (np.abs(host(db) - want) <= 2.0**-10 * np.abs(want) + 2e-6 * scale + 1e-6).all()
 
 
 # few, some and many partials per element; channels that are padded to vectors (fp16) and tap-major columns (fp32, 32)

@@ -37,8 +37,13 @@ CONVS = [
     (2, 8, 9, 9, 8, 3, 4, 1),
 ]
 
+# beside that kernel: tiles in LDS, forward or (more than 48 input channels, few output channels) backward, and filters of more
+# taps and strides of more classes than it takes
+LDS = [(5, 13, 182, 183, 72, 1, 1, 0), (9, 8, 182, 183, 56, 3, 1, 1), (8, 72, 182, 183, 8, 1, 1, 0), (8, 56, 182, 183, 8, 3, 1, 1),
+       (2, 8, 30, 31, 72, 9, 1, 4), (1, 72, 40, 41, 20, 9, 2, 4), (2, 16, 31, 33, 24, 3, 5, 1), (1, 70, 26, 27, 9, 2, 5, 0)]
 
-@pytest.mark.parametrize("shape", CONVS)
+
+@pytest.mark.parametrize("shape", CONVS + LDS)
 @pytest.mark.parametrize("layout", ["nchw", "nhwc"])
 def test_conv(shape, layout):
     N, Cc, H, W, Kk, R, stride, pad = shape
@@ -55,11 +60,16 @@ def test_conv(shape, layout):
     assert_close(host(yd), 1.5 * y_ref, F32, "accumulated y")
     dxd = dev(np.full(x.shape, 7.0, np.float32), F32, layout)
     K.conv2d(K.CONV_BWD_DATA, dyd, wd, dxd, pad, stride)
-    assert_close(host(dxd), ref.conv2d_bwd_data(dy, w, x.shape, pad, stride), F32, "dx")
+    dx_ref = ref.conv2d_bwd_data(dy, w, x.shape, pad, stride)
+    assert_close(host(dxd), dx_ref, F32, "dx")
+    K.conv2d(K.CONV_BWD_DATA, dyd, wd, dxd, pad, stride, alpha=0.5, beta=1.0)
+    assert_close(host(dxd), 1.5 * dx_ref, F32, "accumulated dx")
 
 
 @pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
-@pytest.mark.parametrize("size", [(64, 1030, 400), (33, 31, 17), (1, 1, 24), (5, 70, 1027), (130, 300, 65), (640, 2048, 20)])
+@pytest.mark.parametrize("size", [(64, 1030, 400), (33, 31, 17), (1, 1, 24), (5, 70, 1027), (130, 300, 65), (640, 2048, 20),
+                                  # 64x64 tiles without and with a split, 64x32 tiles without and with; a reduction for the LDS tiles
+                                  (2890, 3010, 21), (1300, 1290, 1030), (1000, 3100, 20), (520, 1060, 390), (640, 1030, 9)])
 def test_gemm(tA, tB, size):
     M, N, Kd = size
     rng = np.random.default_rng(M + N + Kd)
@@ -71,10 +81,13 @@ def test_gemm(tA, tB, size):
     K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 2.0, K.ptr(Ad), Ad.shape[1], K.ptr(Bd), Bd.shape[1], 3.0, K.ptr(Cd), N,
                                   K.FLOAT, stream))
     assert_close(host(Cd), 2 * want + 3, F32, "C")
+    K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 1.0, K.ptr(Ad), Ad.shape[1], K.ptr(Bd), Bd.shape[1], 0.0, K.ptr(Cd), N,
+                                  K.FLOAT, stream))
+    assert_close(host(Cd), want, F32, "C, overwritten")
 
 
 @pytest.mark.parametrize("flags", [0, K.BN_RELU, K.BN_ADD | K.BN_RELU])
-@pytest.mark.parametrize("shape", CONVS + [(8, 8, 190, 191, 80, 1, 1, 0), (2, 3, 186, 184, 64, 3, 1, 1)])  # the last: tiles in LDS
+@pytest.mark.parametrize("shape", CONVS + LDS + [(8, 8, 190, 191, 80, 1, 1, 0), (2, 3, 186, 184, 64, 3, 1, 1)])
 def test_folded_norm(shape, flags):
     N, Cc, H, W, Kk, R, stride, pad = shape
     rng = np.random.default_rng(sum(shape) + flags)

@@ -159,7 +159,7 @@ F32_TILES = {(2, 8, 255, 257, 65, 1, 1, 0): (2, 2, 1, 4), (1, 1032, 79, 80, 200,
 
 @on_stub
 def test_fp32_shapes_are_what_their_comments_say():
-    from tests.test_gpu_stream_f32 import CONVS
+    from tests.test_gpu_stream_f32 import CONVS, LDS
 
     assert set(F32_TILES) <= set(CONVS)
     for shape, (tm, tn, ks, wm) in F32_TILES.items():
@@ -168,6 +168,30 @@ def test_fp32_shapes_are_what_their_comments_say():
         assert tile[1][2:4] == (tm, tn) and tile[3] == 64 * ks * wm, (shape, tile)
         assert tile[2] == -(-pixels // (32 * tm * wm)) * -(-columns // (32 * tn)), (shape, tile)
         assert (tile[1][1] == 3) == any(x[0] == "stream_pack_call" for x in launches) == (shape[5] > 1)
+    seen = {(kind, name, tile[:2] if "uniform" in name else ()) for shape in LDS for kind in (K.CONV_FWD, K.CONV_BWD_DATA)
+            for name, tile, *_ in convolution(kind, shape, K.FLOAT)[0]}
+    for kind in (K.CONV_FWD, K.CONV_BWD_DATA):
+        assert {(kind, "conv_f32_gather_uniform", (128, 128)), (kind, "conv_f32_gather_uniform", (128, 64)), (kind, "conv_f32_gather", ())} <= seen
+
+
+# as above; None: tiles in LDS
+GEMM_TILES = {(640, 2048, 20): (1, 1, 1, 4), (2890, 3010, 21): (2, 2, 1, 4), (1300, 1290, 1030): (2, 2, 4, 1), (1000, 3100, 20): (2, 1, 1, 4),
+              (520, 1060, 390): (2, 1, 4, 1), (640, 1030, 9): None}
+
+
+@pytest.mark.parametrize("tA,tB", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@on_stub
+def test_fp32_products_are_what_their_comments_say(tA, tB):
+    for (m, n, k), want in GEMM_TILES.items():
+        stub_gpu.launched()
+        assert K.lib().saga_hip_gemm(tA, tB, m, n, k, 1.0, X, m if tA else k, Y, k if tB else n, 0.0, ROOM, n, K.FLOAT, None) == 0
+        ((name, tile, blocks, threads),) = stub_gpu.launched()
+        if want is None:
+            assert name == "gemm_mfma_f32"
+        else:
+            tm, tn, ks, wm = want
+            got = name, tile[2:4], threads, blocks
+            assert got == ("stream_f32_k", (tm, tn), 64 * ks * wm, -(-n // (32 * tm * wm)) * -(-m // (32 * tn))), (m, n, k)
 
 
 BIAS_KERNELS = {"small grid": "stream_f16_k", "larger tile of a small grid": "stream_f16_k", "shared tiles": "split_reduce",
