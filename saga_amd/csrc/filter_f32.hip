@@ -254,7 +254,7 @@ __global__ void __launch_bounds__(256, 1) conv_f32_bwd_filter_windows(WindowFilt
     for(int tp = 0; tp < TAPS; tp++)
 #pragma unroll
         for(int v = 0; v < 16; v++) {
-            acc[tp][v] += low[tp][v];
+            acc[tp][v] = (acc[tp][v] + low[tp][v]) * SPLIT_SUM;
             bad = __builtin_fmaf(acc[tp][v], 0.0f, bad);
         }
     if(__builtin_amdgcn_ballot_w64(bad != bad)) {

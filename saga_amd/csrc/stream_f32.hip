@@ -327,7 +327,7 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
             for(int t = 0; t < TN; t++)
 #pragma unroll
                 for(int v = 0; v < 16; v++) {
-                    acc[i][t][v] += low[i][t][v];
+                    acc[i][t][v] = (acc[i][t][v] + low[i][t][v]) * SPLIT_SUM;
                     bad = __builtin_fmaf(acc[i][t][v], 0.0f, bad);
                 }
         if(__builtin_amdgcn_ballot_w64(bad != bad)) {
@@ -348,9 +348,7 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
                     for(int i = 0; i < TM; i++)
 #pragma unroll
                         for(int t = 0; t < TN; t++)
-                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(
-                                (float)part(qr[0][t][0])[j] + (float)part(qr[0][t][1])[j] + (float)part(qr[0][t][2])[j], pr[0][i][j],
-                                acc[i][t], 0, 0, 0);
+                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(qr[0][t], j), pr[0][i][j], acc[i][t], 0, 0, 0);
             }
         }
     }

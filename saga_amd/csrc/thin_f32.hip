@@ -181,7 +181,7 @@ template <int TN, int WAVES, bool EX> __global__ void __launch_bounds__(64 * WAV
             for(int t = 0; t < TN; t++)
 #pragma unroll
                 for(int v = 0; v < 16; v++) {
-                    acc[i][t][v] += low[i][t][v];
+                    acc[i][t][v] = (acc[i][t][v] + low[i][t][v]) * SPLIT_SUM;
                     bad = __builtin_fmaf(acc[i][t][v], 0.0f, bad);
                 }
         if(__builtin_amdgcn_ballot_w64(bad != bad)) { // operands without three parts: in fp32 products
@@ -197,17 +197,16 @@ template <int TN, int WAVES, bool EX> __global__ void __launch_bounds__(64 * WAV
                 pick(step, f);
 #pragma unroll
                 for(int t = 0; t < TN; t++) {
-                    bf16x8_t q[3];
+                    uint4_t q[3];
 #pragma unroll
                     for(int h = 0; h < 3; h++)
-                        q[h] = part(parts[((t * g.steps + step) * 3 + h) * 64 + lane]);
+                        q[h] = parts[((t * g.steps + step) * 3 + h) * 64 + lane];
 #pragma unroll
                     for(int j = 0; j < 8; j++) {
                         const bool in = step * 16 + 8 * fk + j < g.CRS; // (what a lane picks behind the last may be anything)
 #pragma unroll
                         for(int i = 0; i < TM; i++)
-                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)q[0][j] + (float)q[1][j] + (float)q[2][j],
-                                                                           in ? f[i][j] : 0.0f, acc[i][t], 0, 0, 0);
+                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(q, j), in ? f[i][j] : 0.0f, acc[i][t], 0, 0, 0);
                     }
                 }
             }

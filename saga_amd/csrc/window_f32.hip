@@ -269,7 +269,7 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
         for(int t = 0; t < TN; t++)
 #pragma unroll
             for(int v = 0; v < 16; v++) {
-                acc[i][t][v] += low[i][t][v];
+                acc[i][t][v] = (acc[i][t][v] + low[i][t][v]) * SPLIT_SUM;
                 bad = __builtin_fmaf(acc[i][t][v], 0.0f, bad);
             }
     if(__builtin_amdgcn_ballot_w64(bad != bad)) {
@@ -297,16 +297,15 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
                 }
 #pragma unroll
                 for(int t = 0; t < TN; t++) {
-                    bf16x8_t q[3];
+                    float4_t q[3];
 #pragma unroll
                     for(int h = 0; h < 3; h++)
-                        q[h] = part(load4(rq, qoff[t] + 1024 * h, (unsigned)(tp * S16 + st) * 3072u));
+                        q[h] = load4(rq, qoff[t] + 1024 * h, (unsigned)(tp * S16 + st) * 3072u);
 #pragma unroll
                     for(int j = 0; j < 8; j++)
 #pragma unroll
                         for(int i = 0; i < TM; i++)
-                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32((float)q[0][j] + (float)q[1][j] + (float)q[2][j], a[i][j],
-                                                                           acc[i][t], 0, 0, 0);
+                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(q, j), a[i][j], acc[i][t], 0, 0, 0);
                 }
             }
     }

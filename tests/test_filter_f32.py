@@ -105,6 +105,20 @@ def test_no_worse_than_fp32():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("scales", [(-120, 80), (80, -120), (-140, 100), (-20, -100)], ids=str)
+def test_small_numbers(scales):
+    """Operands whose low bits a bf16 cannot hold, subnormal ones among them: the same bound."""
+    n, c, h, w, k = 40, 8, 33, 21, 24
+    g = torch.Generator().manual_seed(7)  # (on the host: what makes subnormal numbers on the device is not asked here)
+    x, dy = (torch.ldexp(torch.randn(n, ch, h, w, generator=g), torch.tensor(s)).cuda() for ch, s in ((c, scales[0]), (k, scales[1])))
+    f = torch.zeros(k, c, 3, 3, device="cuda")
+    gradient(x, dy, f)
+    error, want = (f.double() - oracle(x, dy)).abs(), oracle(x, dy)
+    assert error.norm() / want.norm() < 3e-7
+    assert (want.abs() > 0).all()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("value", [float("inf"), float("nan"), 3.4e38], ids=str)
 def test_without_three_parts(value):
     """Such an operand reaches the sums that have it and no other."""

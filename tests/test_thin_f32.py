@@ -72,21 +72,52 @@ def test_against_64_bits(shape, layout):
         assert np.linalg.norm(got - want) <= bound * np.linalg.norm(want)
 
 
+def plain(shape, x, w):
+    """Of float32 operands on the host: the kernel's result."""
+    yd = dev(np.full(out_shape(shape), 7.0, np.float32), F32)
+    xd, wd = dev(x, F32), dev(w, F32)
+    call(shape, K.view(xd), K.view(wd), K.view(yd), None, K.stream_ptr())
+    return host(yd).astype(np.float64)
+
+
+def reference(shape, x, w):
+    return torch.nn.functional.conv2d(*(torch.from_numpy(a).double() for a in (x, w)), None, shape[6], shape[7], shape[8]).numpy()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("scales", [(-120, 80), (80, -120), (-140, 100), (-20, -100)], ids=str)
+@pytest.mark.parametrize("shape", SHAPES)
+def test_small_numbers(shape, scales):
+    """Operands whose low bits a bf16 cannot hold, subnormal ones among them, are multiplied with all their bits."""
+    n, c, h, wd, k, r, stride, pad, dil = shape
+    rng = np.random.default_rng(2)
+    x, w = rnd(rng, n, c, h, wd, dtype=F32), rnd(rng, k, c, r, r, dtype=F32, scale=(2.0 / (c * r * r)) ** 0.5)
+    x, w = np.ldexp(x, scales[0]), np.ldexp(w, scales[1])
+    want = reference(shape, x, w)
+    bound = 2.0 ** -23 * (6 * max(c * r * r, 16) / 16) ** 0.5  # (as above)
+    assert np.linalg.norm(plain(shape, x, w) - want) <= bound * np.linalg.norm(want)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape", SHAPES)
 def test_numbers_without_three_parts(shape):
+    """Infinities, NaNs and numbers next to the largest: where they belong, nowhere else; and what shares a wavefront with them is
+    multiplied with all bits of its weights."""
     n, c, h, wd, k, r, stride, pad, dil = shape
     rng = np.random.default_rng(1)
-    x = rnd(rng, n, c, h, wd, dtype=F32)
-    w = np.where(rng.random((k, c, r, r)) < 0.5, np.float32(-0.5), np.float32(0.5))  # (an infinity times other parts would be NaN)
+    x, w = rnd(rng, n, c, h, wd, dtype=F32), rnd(rng, k, c, r, r, dtype=F32, scale=(2.0 / (c * r * r)) ** 0.5)
     for value in (np.inf, -np.inf, np.nan, 3.4e38):
         x.reshape(-1)[rng.integers(x.size)] = value
-    want = torch.nn.functional.conv2d(torch.from_numpy(x).double(), torch.from_numpy(w).double(), None, stride, pad, dil).numpy().astype(np.float32)
-    yd = dev(np.full(out_shape(shape), 7.0, np.float32), F32)
-    xd, wd_ = dev(x, F32), dev(w, F32)
-    call(shape, K.view(xd), K.view(wd_), K.view(yd), None, K.stream_ptr())
-    got = host(yd)
-    np.testing.assert_array_equal(np.isnan(got), np.isnan(want))
-    np.testing.assert_array_equal(got[np.isinf(want)], want[np.isinf(want)])
-    ok = np.isfinite(want)
-    np.testing.assert_allclose(got[ok], want[ok], rtol=1e-4, atol=1e-4)
+    w.reshape(-1)[rng.integers(w.size)] = 1.2345678e32
+    want, spread = reference(shape, x, w), reference(shape, x.astype(np.float64) ** 2, w.astype(np.float64) ** 2)
+    with np.errstate(over="ignore"):
+        ref = want.astype(np.float32)
+    got = plain(shape, x, w)
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    np.testing.assert_array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
+    ok = np.isfinite(ref)
+    # The largest of up to 10^7 errors, each a chain of roundings of up to half a unit at random: 2**-24 / sqrt(3) of a partial sum each,
+    # which grows like the root of its length to the sum's deviation, or to the sum itself where that is larger.  (Weights without their
+    # third part: some 2e-6 of a deviation on average.)
+    size = np.sqrt(spread[ok]) + np.abs(want[ok])
+    assert (np.abs(got[ok] - want[ok]) <= 6 * (2.0 ** -24 / 3 ** 0.5 * (c * r * r / 2) ** 0.5 + 2.0 ** -24) * size).all()

@@ -29,6 +29,8 @@ SHAPES = {
     (60, 16, 28, 28, 130, 5, 1, 0): (1, 1, 25, 4),   # backward: more padding than the filter needs, pixels out of order: not here
 }
 
+CLASSES = (2, 24, 11, 13, 40, 3, 2, 1)  # backward: residue classes of pixels, straight from memory (csrc/stream_f32.hip)
+
 
 def views(shape, x, w, y):
     """Views of dense tensors at these addresses."""
@@ -124,22 +126,46 @@ def test_against_64_bits(shape):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [*SHAPES, (2, 24, 11, 13, 40, 3, 2, 1), (1, 24, 150, 161, 24, 3, 1, 1)])
-def test_numbers_without_three_parts(shape):
-    """Infinities, NaNs and numbers next to the largest in either operand: where they belong, nowhere else."""
+@pytest.mark.parametrize("scales", [(-120, 80), (80, -120), (-140, 100), (-20, -100)], ids=str)
+@pytest.mark.parametrize("shape", [*SHAPES, CLASSES], ids=str)
+def test_small_numbers(shape, scales):
+    """Operands whose low bits a bf16 cannot hold, subnormal ones among them, are multiplied with all their bits."""
     n, c, h, wd, k, r, stride, pad = shape
     x, w, dy = operands(shape)
-    w = np.where(w < 0, np.float32(-0.5), np.float32(0.5))  # (one part is all of it: an infinity times the others would be NaN)
+    x, dy = (np.ldexp(a, scales[0]) for a in (x, dy))
+    w = np.ldexp(w, scales[1])
+    want = reference(shape, x, w, dy)
+    for kind, got, _ in both(shape, x, w, dy):
+        ref, red = want[kind], c if kind == K.CONV_FWD else k
+        bound = 2.0 ** -24 * (6 * max(red, 16) * r ** 2 / 16) ** 0.5 + 2.0 ** -24  # (as above)
+        assert np.linalg.norm(got.astype(np.float64) - ref) <= 2 * bound * np.linalg.norm(ref)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", [*SHAPES, CLASSES, (1, 24, 150, 161, 24, 3, 1, 1)])
+def test_numbers_without_three_parts(shape):
+    """Infinities, NaNs and numbers next to the largest in either operand: where they belong, nowhere else; and what shares a
+    wavefront with them is multiplied with all bits of its weights."""
+    n, c, h, wd, k, r, stride, pad = shape
+    x, w, dy = operands(shape)
     rng = np.random.default_rng(1)
     for value in (np.inf, -np.inf, np.nan, 3.4e38):
         for a in (x, dy):
             a.reshape(-1)[rng.integers(a.size)] = value
+    w.reshape(-1)[rng.integers(w.size)] = 1.2345678e32
     if r == 1:  # (the zeros around an image times an infinity are NaN, here and in every kernel that multiplies them)
         w[rng.integers(k), rng.integers(c)] = np.inf
     want = reference(shape, x, w, dy)
+    spread = reference(shape, *(a.astype(np.float64) ** 2 for a in (x, w, dy)))
     for kind, got, _ in both(shape, x, w, dy):
-        ref = want[kind].astype(np.float32)
+        with np.errstate(over="ignore"):
+            ref = want[kind].astype(np.float32)
         np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
         np.testing.assert_array_equal(got[np.isinf(ref)], ref[np.isinf(ref)])
         ok = np.isfinite(ref)
-        np.testing.assert_allclose(got[ok], ref[ok], rtol=1e-4, atol=1e-4)
+        # The largest of some 10^6 errors, each a chain of `red` roundings of up to half a unit at random: 2**-24 / sqrt(3) of a partial
+        # sum each, which grows like the root of its length to the sum's deviation, or to the sum itself where that is larger.
+        # (Weights without their third part: some 2e-6 of a deviation on average.)
+        red = (c if kind == K.CONV_FWD else k) * r * r
+        size = np.sqrt(spread[kind][ok]) + np.abs(want[kind][ok])
+        assert (np.abs(got[ok] - want[kind][ok]) <= 6 * (2.0 ** -24 / 3 ** 0.5 * (red / 2) ** 0.5 + 2.0 ** -24) * size).all()
