@@ -15,8 +15,8 @@
 // hit 64 banks, and as the width of a tile is known here, every read is an immediate offset from five addresses.
 //
 // Tiles overlap at the right and the lower border of an image that they do not divide; pixels seen before have zeros
-// for dy.  (Pixels that are not there would do as well but for infinities in x, which must not meet such zeros under taps that
-// have no other product with them.)
+// for dy.  An infinity of x there makes a NaN of a sum that should be infinite: a block that ends with a NaN looks for
+// one, and if there is one takes its share again, with zeros for x as well.
 #include "filter_strips.hpp"
 
 #include <algorithm>
@@ -25,7 +25,7 @@
 namespace {
 
 typedef short short4_t __attribute__((ext_vector_type(4)));
-typedef short short8_t __attribute__((ext_vector_type(8)));
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
 struct StripArgs {
@@ -63,6 +63,7 @@ template <int I, int N, class F> __device__ __forceinline__ void each(F &&f)
 // The order of a tile's work: instruction 18 * j + m multiplies, in step j, x operand m % 6 / 2 (the tap's column) of the top (m < 6),
 // middle and bottom taps with half m % 2 of dy.  Operands are read in the order of their first use, AHEAD instructions early.
 constexpr int AHEAD = 8;
+constexpr unsigned OOB = 0x7fffff00u; // behind every buffer: loads return zero, stores do nothing
 constexpr int first_uses(int t, int nst)
 {
     const int j = t / 18, m = t % 18;
@@ -85,6 +86,95 @@ template <int TW, int NST> struct StripTile {
     static constexpr int LDS = std::max(2 * (XB + YB), 4 * 36 * 1024); // (the groups' sums: half of a wavefront's accumulators)
     static_assert(TR * TW * 8 % 256 == 0 && LDS <= 160 * 1024 && NLX + NLY < 32, "tile");
 };
+
+// whether an infinity of x, in the block's channels from c0 on, is seen by pixels of its tiles that another tile has too (or by those next to them)
+template <int TW, int TR> __device__ __forceinline__ bool infinity_under_overlap(const StripArgs &t, int split, int c0)
+{
+    bool found = false;
+#pragma unroll 1
+    for(int tile = split; tile < t.ntiles; tile += t.splits) {
+        const int n = tile / t.tpi, in = tile - n * t.tpi, ty = in / t.nx, tx = in - ty * t.nx;
+        const int ox = std::min(tx * TW, t.W - TW), oy = std::min(ty * TR, t.H - TR);
+        if(ox == tx * TW && oy == ty * TR)
+            continue;
+        const half_t *const img = t.x + (int64_t)n * t.H * t.W * t.ldx + c0;
+#pragma unroll 4
+        for(int i = threadIdx.x; i < (TR + 2) * (TW + 2) * 8; i += 256) {
+            const int pos = i >> 3, ch = (i & 7) * 8, y = oy + pos / (TW + 2) - 1, x = ox + pos % (TW + 2) - 1;
+            if(ch < t.C - c0 && (unsigned)y < (unsigned)t.H && (unsigned)x < (unsigned)t.W) {
+                const uint4_t v = *(const uint4_t *)(img + ((int64_t)y * t.W + x) * t.ldx + ch);
+#pragma unroll
+                for(int j = 0; j < 4; j++)
+                    found |= (v[j] & 0x7fffu) == 0x7c00u || (v[j] & 0x7fff0000u) == 0x7c000000u;
+            }
+        }
+    }
+    return found;
+}
+
+// A block's share once more, straight from memory: a wavefront's 32 output channels from k0 on, this lane's input channel c.
+// (us, second pass included, 192->192 at 15x23x19 / 512->512 at 9x17x33: finite 31 / 67, one NaN 41 / 99, one infinity
+// under an overlap 83 / 262.)
+template <int TW, int TR> __device__ __forceinline__ void strips_again(const StripArgs &t, int split, int k0, int c, __amdgpu_buffer_rsrc_t ro)
+{
+    const int lane = threadIdx.x & 63, hi = lane >> 5, k = k0 + (lane & 31);
+    const int64_t ximg = (int64_t)t.H * t.W * t.ldx, yimg = (int64_t)t.H * t.W * t.ldy;
+    float16_t acc[9];
+#pragma unroll
+    for(int tp = 0; tp < 9; tp++)
+#pragma unroll
+        for(int v = 0; v < 16; v++)
+            acc[tp][v] = 0.0f;
+#pragma unroll 1
+    for(int tile = split; tile < t.ntiles; tile += t.splits) {
+        const int n = tile / t.tpi, in = tile - n * t.tpi, ty = in / t.nx, tx = in - ty * t.nx;
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(t.x + n * ximg), 0, (unsigned)(ximg * 2), 0x00020000);
+        const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)(t.dy + n * yimg), 0, (unsigned)(yimg * 2), 0x00020000);
+        const int ox = std::min(tx * TW, t.W - TW), oy = std::min(ty * TR, t.H - TR);
+#pragma unroll 1
+        for(int step = 0; step < TR / 2 * (TW / 8); step++) { // eight columns of two rows
+            const int y = oy + step / (TW / 8) * 2 + hi, x0 = ox + step % (TW / 8) * 8;
+            uint4_t keep; // pixels that no tile before had
+#pragma unroll
+            for(int i = 0; i < 4; i++) {
+                const unsigned pair = (x0 + 2 * i >= tx * TW ? 0xffffu : 0u) | (x0 + 2 * i + 1 >= tx * TW ? 0xffff0000u : 0u);
+                keep[i] = y >= ty * TR ? pair : 0u;
+            }
+            auto load = [&](__amdgpu_buffer_rsrc_t r, int yy, int xx, int ld, int ch, int channels) {
+                const bool there = ch < channels && (unsigned)yy < (unsigned)t.H && (unsigned)xx < (unsigned)t.W;
+                return (unsigned)__builtin_amdgcn_raw_buffer_load_b16(r, there ? (unsigned)(((yy * t.W + xx) * ld + ch) * 2) : OOB, 0, 0);
+            };
+            auto eight = [&](const unsigned *w) {
+                uint4_t v;
+#pragma unroll
+                for(int i = 0; i < 4; i++)
+                    v[i] = (w[2 * i] | w[2 * i + 1] << 16) & keep[i];
+                return __builtin_bit_cast(half8_t, v);
+            };
+            unsigned g[8], p[3][10];
+#pragma unroll
+            for(int e = 0; e < 8; e++)
+                g[e] = load(ry, y, x0 + e, t.ldy, k, t.K);
+#pragma unroll
+            for(int r = 0; r < 3; r++)
+#pragma unroll
+                for(int e = 0; e < 10; e++)
+                    p[r][e] = load(rx, y + r - 1, x0 + e - 1, t.ldx, c, t.C);
+#pragma unroll
+            for(int tp = 0; tp < 9; tp++)
+                acc[tp] = __builtin_amdgcn_mfma_f32_32x32x16_f16(eight(g), eight(p[tp / 3] + tp % 3), acc[tp], 0, 0, 0);
+        }
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // (the stores before)
+#pragma unroll
+    for(int tp = 0; tp < 9; tp++)
+#pragma unroll
+        for(int v = 0; v < 16; v++) {
+            const float sum = acc[tp][v];
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), ro,
+                                                  c < t.C ? (unsigned)((((k0 + 8 * (v / 4) + 4 * hi + v % 4) * 9 + tp) * t.C + c) * 4) : OOB, 0, 0);
+        }
+}
 
 template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_filter_strips(StripArgs t)
 {
@@ -243,6 +333,11 @@ template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_fi
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
     asm volatile("s_waitcnt vmcnt(0)\n\ts_barrier" ::: "memory");
 
+    // (a share's partial result is one buffer: rows and columns beyond the filter are outside)
+    const unsigned sbytes = (unsigned)t.K * 9u * (unsigned)t.C * 4u;
+    const __amdgpu_buffer_rsrc_t ro =
+        __builtin_amdgcn_make_buffer_rsrc((void *)((char *)t.partial + (int64_t)split * sbytes), 0, sbytes, 0x00020000);
+    const int c = c0 + nt * 32 + (lane & 31);
     // group g finishes half g of the output channels; the other half goes to the other group
     float4_t *const red = (float4_t *)smem;
     auto leave = [&](auto H) {
@@ -253,11 +348,7 @@ template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_fi
                 red[(wave * 36 + tp * 4 + v) * 64 + lane] = float4_t{acc[tp][H.value][4 * v], acc[tp][H.value][4 * v + 1],
                                                                      acc[tp][H.value][4 * v + 2], acc[tp][H.value][4 * v + 3]};
     };
-    // (a share's partial result is one buffer: rows and columns beyond the filter are outside)
-    const unsigned sbytes = (unsigned)t.K * 9u * (unsigned)t.C * 4u;
-    const __amdgpu_buffer_rsrc_t ro =
-        __builtin_amdgcn_make_buffer_rsrc((void *)((char *)t.partial + (int64_t)split * sbytes), 0, sbytes, 0x00020000);
-    const int c = c0 + nt * 32 + (lane & 31);
+    bool nan = false;
     auto finish = [&](auto H) {
         const int k = k0 + H.value * 32 + 4 * hi;
 #pragma unroll
@@ -266,9 +357,12 @@ template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_fi
             for(int v = 0; v < 4; v++) {
                 const float4_t o = red[((wave ^ 2) * 36 + tp * 4 + v) * 64 + lane];
 #pragma unroll
-                for(int e = 0; e < 4; e++)
-                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, acc[tp][H.value][4 * v + e] + o[e]), ro,
-                                                          c < t.C ? (unsigned)((((k + 8 * v + e) * 9 + tp) * t.C + c) * 4) : 0x7fffff00u, 0, 0);
+                for(int e = 0; e < 4; e++) {
+                    const float sum = acc[tp][H.value][4 * v + e] + o[e];
+                    nan |= sum != sum;
+                    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), ro,
+                                                          c < t.C ? (unsigned)((((k + 8 * v + e) * 9 + tp) * t.C + c) * 4) : OOB, 0, 0);
+                }
             }
     };
     if(grp == 0)
@@ -280,6 +374,17 @@ template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_fi
         finish(std::integral_constant<int, 0>());
     else
         finish(std::integral_constant<int, 1>());
+    if(!(dup_cols | dup_rows))
+        return;
+    volatile int *const found = (volatile int *)smem;
+    auto any = [&](bool here) {
+        __syncthreads();
+        found[wave] = __builtin_amdgcn_ballot_w64(here) != 0;
+        __syncthreads();
+        return (found[0] | found[1] | found[2] | found[3]) != 0;
+    };
+    if(any(nan) && any(infinity_under_overlap<TW, TR>(t, split, c0)))
+        strips_again<TW, TR>(t, split, k0 + grp * 32, c, ro); // (over what this wavefront has stored)
 }
 
 template <int TW, int NST> int launch(const StripArgs &t, int blocks, hipStream_t st)

@@ -93,3 +93,22 @@ def test_infinities(shape):
     assert torch.equal(torch.isfinite(f), torch.isfinite(want)) and not torch.isfinite(want).all()
     ok = torch.isfinite(want)
     assert torch.equal(f[ok], want[ok].half())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", SHAPES, ids=str)
+def test_infinities_where_tiles_overlap(shape):
+    """They meet the zeros of pixels seen before under no tap: sums that should be infinite are, all others are as they should be."""
+    n, c, h, w, k = shape
+    g = torch.Generator("cuda").manual_seed(2)
+    half = lambda *d: torch.randint(1, 3, d, device="cuda", generator=g).half().contiguous(memory_format=torch.channels_last)
+    x, dy = half(n, c, h, w), half(n, k, h, w)
+    x[0, 3, h // 2, w // 2], x[1, c - 1, h - 15, w - 7] = float("inf"), float("-inf")
+    x[2, 5, h - 14, :], x[3, 40, :, w - 8] = float("inf"), float("inf")
+    x[4, 17, h // 2, w // 2] = float("nan")
+    f = torch.zeros(k, c, 3, 3, device="cuda", dtype=torch.float16).contiguous(memory_format=torch.channels_last)
+    want = oracle(x, dy).half()
+    gradient(x, dy, f, 0.0)
+    assert torch.equal(torch.isnan(f), torch.isnan(want)) and torch.isinf(want).any()
+    ok = ~torch.isnan(want)
+    assert torch.equal(f[ok], want[ok])
