@@ -1466,7 +1466,13 @@ static int num_cus();
 static FilterStrips filter_strips(const ConvGeom &g)
 {
     static const bool on = !(getenv("SAGA_HIP_FILTER_ROWS64") && atoi(getenv("SAGA_HIP_FILTER_ROWS64")) == 0);
-    return on ? plan_filter_strips(g, num_cus()) : FilterStrips{0, 0, 0, 0};
+    if(!on)
+        return FilterStrips{0, 0, 0, 0};
+    // what conv_bwd_filter_dma takes instead, in ns: what does not depend on the size, and its tiles' area times the pixels
+    // (fitted to 53 shapes of 16 to 512 channels; of the two the slower one is taken in one of them, by 5 %)
+    const FilterPlan p = plan_filter(g);
+    const double rate = p.bm == 64 ? (p.bn == 128 ? 3.7e-6 : 2.7e-6) : p.bm == 128 ? (p.bn == 128 ? 2.4e-6 : 2.2e-6) : 2.7e-6;
+    return plan_filter_strips(g, num_cus(), 15500 + rate * g.N * g.P * g.Q * p.tiles_k * p.bm * p.tiles_c * p.bn);
 }
 
 static bool krsc_dense(const SagaTensorView *w)

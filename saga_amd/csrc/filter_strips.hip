@@ -176,7 +176,8 @@ template <int TW, int TR> __device__ __forceinline__ void strips_again(const Str
         }
 }
 
-template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_filter_strips(StripArgs t)
+// OVERLAP: tiles do not divide the image
+template <int TW, int NST, bool OVERLAP> __global__ void __launch_bounds__(256, 1) conv_bwd_filter_strips(StripArgs t)
 {
     using T = StripTile<TW, NST>;
     constexpr int TR = T::TR, SR = T::SR, NLX = T::NLX, NLY = T::NLY, XB = T::XB, YB = T::YB;
@@ -359,7 +360,8 @@ template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_fi
 #pragma unroll
                 for(int e = 0; e < 4; e++) {
                     const float sum = acc[tp][H.value][4 * v + e] + o[e];
-                    nan |= sum != sum;
+                    if constexpr(OVERLAP)
+                        nan |= sum != sum;
                     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), ro,
                                                           c < t.C ? (unsigned)((((k + 8 * v + e) * 9 + tp) * t.C + c) * 4) : OOB, 0, 0);
                 }
@@ -374,50 +376,54 @@ template <int TW, int NST> __global__ void __launch_bounds__(256, 1) conv_bwd_fi
         finish(std::integral_constant<int, 0>());
     else
         finish(std::integral_constant<int, 1>());
-    if(!(dup_cols | dup_rows))
+    if constexpr(!OVERLAP)
         return;
     volatile int *const found = (volatile int *)smem;
-    auto any = [&](bool here) {
-        __syncthreads();
+    auto any = [&](bool here) { // (barriers that do not wait for the stores)
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         found[wave] = __builtin_amdgcn_ballot_w64(here) != 0;
-        __syncthreads();
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
         return (found[0] | found[1] | found[2] | found[3]) != 0;
     };
     if(any(nan) && any(infinity_under_overlap<TW, TR>(t, split, c0)))
         strips_again<TW, TR>(t, split, k0 + grp * 32, c, ro); // (over what this wavefront has stored)
 }
 
-template <int TW, int NST> int launch(const StripArgs &t, int blocks, hipStream_t st)
+template <int TW, int NST, bool OVERLAP> int launch_as(const StripArgs &t, int blocks, hipStream_t st)
 {
     constexpr int lds = StripTile<TW, NST>::LDS;
-    static bool once = false;
-    if(!once) {
-        const hipError_t e =
-            hipFuncSetAttribute((const void *)conv_bwd_filter_strips<TW, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-        if(e != hipSuccess)
-            return (int)e;
-        once = true;
-    }
-    conv_bwd_filter_strips<TW, NST><<<blocks, 256, lds, st>>>(t);
+    const auto kern = conv_bwd_filter_strips<TW, NST, OVERLAP>;
+    static const hipError_t allowed = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if(allowed != hipSuccess)
+        return (int)allowed;
+    kern<<<blocks, 256, lds, st>>>(t);
     SAGA_CHECK_LAUNCH();
     return 0;
+}
+
+template <int TW, int NST> int launch(const StripArgs &t, int blocks, hipStream_t st)
+{
+    return t.W % TW || t.H % StripTile<TW, NST>::TR ? launch_as<TW, NST, true>(t, blocks, st) : launch_as<TW, NST, false>(t, blocks, st);
 }
 
 int tile_rows(int tw, int nst) { return (tw == 16 ? 2 : 4) * nst; }
 
 } // namespace
 
-// Where a block walks three tiles or more.  What does not depend on their number - both launches, the first tile's way to LDS,
-// and a partial result per block, 38 MB of them to write and read - is 20 us, which fewer do not make up for, while padding to
-// blocks of 64 channels is cheaper than it looks: the operands are read either way.  us, tiles of a GEMM (conv_bwd_filter_dma) /
-// strips (before, whole rows in LDS for 64->64 with one operand per tap: 96 at 256x56x56):
-//   64->64   256x56x56   136 /  65    64->64    64x56x56  44 / 34    64->64    32x56x56 (2 tiles) 31.4 / 30.7
+// Where a block walks three tiles or more, and where that takes less than tiles of a GEMM (conv_bwd_filter_dma).  Both launches, the
+// first tile's way to LDS and the sum over partial results are 14 us, the partial results themselves (38 MB from 256 blocks of 64 x 64) up
+// to 8, a tile of 16x16 3, the look for NaNs where tiles overlap 1.  What tiles have twice or channels that a block of 64 lacks cost as much as what counts, and more of
+// it than the GEMM's tiles have.  us, GEMM / strips (before, whole rows in LDS for 64->64 with one operand per tap: 96 at 256x56x56):
+//   64->64   256x56x56   121 /  67    64->64    64x56x56  45 / 34    64->64    32x56x56 (2 tiles) 31.4 / 30.7
 //   64->64   16x256x256  170 /  82    16->16   256x56x56  66 / 48    64->64    16x56x56 (1 tile)  26.5 / 27.2
 //   128->64  16x256x256  274 / 139    32->32    64x56x56  33 / 29    32->32   128x16x16 (1)       15.0 / 22.3
 //   128->128 16x128x128  111 /  77    24->24  64x112x112  64 / 48    128->128  23x25x25 (2)       28.2 / 29.6
 //   512->512 16x32x32    102 /  81    80->160   64x56x56 121 / 72    96->96     8x56x56 (2)       24.2 / 26.9
+// and left to the GEMM for what tiles have twice or channels lack:
+//   512->512 16x17x17     50 /  74    512->512   9x17x33  55 / 67    40->40   100x34x18           20 / 28
+//   40->312  31x20x20     22 /  28    72->72    70x28x9   19 / 24    16->368   11x67x67           25 / 32
 // (139 us for 155 GFLOP: 1240 TFLOP/s behind the fixed part, what a large matrix product reaches on this card.)
-FilterStrips plan_filter_strips(const ConvGeom &g, int cus)
+FilterStrips plan_filter_strips(const ConvGeom &g, int cus, double other_ns)
 {
     FilterStrips best = {0, 0, 0, 0};
     if(g.R != 3 || g.S != 3 || g.stride != 1 || g.pad != 1 || g.dil != 1 || g.group != 1 || g.P != g.H || g.Q != g.W)
@@ -437,7 +443,8 @@ FilterStrips plan_filter_strips(const ConvGeom &g, int cus)
             const int64_t each = (tiles + splits - 1) / splits, cost = each * (18 * nst + 16); // instructions, and a tile's own time
             if(tiles < 0x7fffffff && (!least || cost < least)) {
                 least = cost;
-                best = {tw, each >= 3 ? nst : 0, (int)pairs, splits};
+                const double ns = 14000 + (g.W % tw || g.H % tr ? 1300 : 0) + 19.0 * cost + 0.8e-3 * splits * g.K * 9.0 * g.C;
+                best = {tw, each >= 3 && ns < other_ns ? nst : 0, (int)pairs, splits};
             }
         }
     return best;

@@ -7,8 +7,8 @@ struct FilterStrips {
     int pairs;      // blocks of 64 output channels times blocks of 64 input channels
     int splits;     // partial results: shares of the tiles
 };
-// g.C, g.K: as the kernel sees them (multiples of 8)
-FilterStrips plan_filter_strips(const ConvGeom &g, int cus);
+// g.C, g.K: as the kernel sees them (multiples of 8); other_ns: what the other kernel takes
+FilterStrips plan_filter_strips(const ConvGeom &g, int cus, double other_ns);
 static inline size_t filter_strips_bytes(const FilterStrips &p, const ConvGeom &g)
 {
     return p.nst ? (size_t)p.splits * g.K * 9 * g.C * sizeof(float) : 0;
