@@ -152,7 +152,7 @@ typedef struct SagaFilterPackJob {
     int64_t w_sn, w_sc, w_sr, w_ss;
     int32_t N, C, T, Ts, r0, s0, rstep;
     int32_t first_block, blocks;
-    int32_t dtype; /* SAGA_HALF; anything else is SAGA_FLOAT */
+    int32_t dtype; /* SAGA_HALF; SAGA_I32: fp32, copied; anything else: fp32, in the parts that some kernels read */
 } SagaFilterPackJob;
 size_t saga_hip_conv2d_pack_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                                   const SagaConvParams *p);

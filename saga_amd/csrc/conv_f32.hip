@@ -943,7 +943,8 @@ size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorVie
 {
     if(!f32_ok(x, w, y, g))
         return 0;
-    const size_t stream = kind == SAGA_CONV_BWD_FILTER ? 0 : stream_f32_conv_workspace(kind == SAGA_CONV_BWD_DATA, g) + 256;
+    const bool bwd = kind == SAGA_CONV_BWD_DATA;
+    const size_t stream = kind == SAGA_CONV_BWD_FILTER ? 0 : stream_f32_conv_workspace(bwd, bwd ? y : x, bwd ? x : y, g) + 256;
     if(kind == SAGA_CONV_FWD) {
         const size_t a = tab_bytes(g.C * g.R * g.S), b = plan_uniform(g.C * g.R * g.S, g.K).bytes;
         return std::max(stream, (a > b ? a : b) + 256);
@@ -961,11 +962,12 @@ size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorVie
 // convolution: 521 against 562 us on 3x3 64->64 at 256x56x56 (windows: 289; 1x1 64->256 at 8x56x56, one round: equal).  Reduction channels
 // in other numbers than eights go through a table in both kernels, and the stream kernel's is read by every lane: 42
 // against 53 us on 7x7 3->64 at 8x224x224.
-static bool tiles_in_lds(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g)
+static bool tiles_in_lds(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room)
 {
     const int cols = out->dims[1], bn = cols > 64 ? 128 : 64;
     const long long tiles = ((long long)out->dims[0] * out->dims[2] * out->dims[3] + FBM - 1) / FBM * ((cols + bn - 1) / bn);
-    return tiles >= ((bwd ? g.K : g.C) % 8 ? 512 : 2048) && cols > 48 && uniform_ok(bwd, a, g) && !stream_f32_windows(bwd, a, out, g);
+    return tiles >= ((bwd ? g.K : g.C) % 8 ? 512 : 2048) && cols > 48 && uniform_ok(bwd, a, g) &&
+           !stream_f32_windows(bwd, a, out, g, packed, room);
 }
 
 static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out,
@@ -975,7 +977,7 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
     // forward: a = x (N,C,H,W), out = y (N,K,P,Q); backward data: a = dy (N,K,P,Q), out = dx (N,C,H,W)
     const int red_ch = bwd ? g.K : g.C;
     const int Kred = red_ch * g.R * g.S;
-    if(!tiles_in_lds(bwd, a, out, g)) {
+    if(!tiles_in_lds(bwd, a, out, g, packed != nullptr, ws && aligned16(ws) ? ws_bytes : 0)) {
         const int r = stream_f32_conv(bwd, a, w, out, g, alpha, beta, e, packed, ws, ws_bytes, st);
         if(r != SAGA_HIP_EUNSUPPORTED)
             return r;
@@ -1138,7 +1140,7 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
 size_t conv_f32_packed_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g)
 {
     const bool bwd = kind == SAGA_CONV_BWD_DATA;
-    return f32_ok(x, w, y, g) && !tiles_in_lds(bwd, bwd ? y : x, bwd ? x : y, g) ? stream_f32_packed_bytes(bwd, g) : 0;
+    return f32_ok(x, w, y, g) && !tiles_in_lds(bwd, bwd ? y : x, bwd ? x : y, g, true, 0) ? stream_f32_packed_bytes(bwd, g) : 0;
 }
 
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,

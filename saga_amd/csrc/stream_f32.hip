@@ -1,5 +1,5 @@
-// fp32 matrix products straight from global memory: on v_mfma_f32_32x32x2_f32, or, from a packed filter, on the bf16 matrix
-// unit (split_f32.hpp).  (Packed filters of one class of pixels over dense planes: window_f32.hip.)
+// fp32 matrix products straight from global memory: on v_mfma_f32_32x32x2_f32, or, from a filter packed for windows
+// (window_f32.hip) that are not the faster one after all, on the bf16 matrix unit (split_f32.hpp).
 //
 // An fp32 matrix instruction keeps the matrix unit busy for 64 cycles with 256 bytes of each operand, so a wavefront
 // that loads its own operands from the caches into registers needs 8 - 16 bytes per cycle and SIMD's share of the L1:
@@ -28,10 +28,13 @@ namespace {
 
 // The lanes-side operand P: PTAP: addressed by tap and channel, the channel count a multiple of eight (also a matrix
 // with the lanes' index contiguous); PTAB: by a table of all reduction indices; PROW: reduction index contiguous.
-// The other operand Q: QROW: reduction index contiguous; QCOL: row index contiguous; QTAB: by the same table; QSPLIT: packed
-// in three parts, 3 KB per step of sixteen of 32 rows in the order of the lanes (stream_pack).
+// The other operand Q: QLANE: packed, 1 KB per step of 32 rows in the order of the lanes (stream_pack); QROW: reduction
+// index contiguous; QCOL: row index contiguous; QTAB: by the same table; QSPLIT: packed in three parts, 3 KB per step of sixteen.
+// (Without windows the parts gain nothing: every tap's operands are split again.  us, QLANE / QSPLIT: 3x3 8->416 at 78x12x12 24 / 37,
+// 5x5 8->288 at 243x32x32, stride 2 102 / 161, 7x7 456->40 at 2x15x15 113 / 130, 16->120 at 16x34x34 60 / 52; over 180 such
+// layers QSPLIT is 1 to 2 % slower at the median.)
 enum { PTAP, PTAB, PROW };
-enum { QROW, QCOL, QTAB, QSPLIT };
+enum { QROW, QCOL, QTAB, QLANE, QSPLIT };
 
 constexpr int MAX_CLASSES = 16;
 constexpr int MAX_TABLE = 4096; // reduction indices of a table
@@ -148,7 +151,8 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
     for(int t = 0; t < TN; t++) {
         const int n = n0 + 32 * t + fr;
         nok[t] = n < g.N;
-        const long long o = QM == QSPLIT ? c.q0 + (long long)(n0 / 32 + t) * T * ((g.C + 15) / 16) * 3072 + lane * 16
+        const long long o = QM == QLANE  ? c.q0 + (long long)(n0 / 32 + t) * (kred / 8) * 1024 + lane * 16
+                            : QM == QSPLIT ? c.q0 + (long long)(n0 / 32 + t) * T * ((g.C + 15) / 16) * 3072 + lane * 16
                             : QM == QROW ? ((long long)n * g.q_sn + 4 * fk) * 4
                             : QM == QCOL ? (n + 4 * fk * g.q_sc) * 4
                                          : n * g.q_sn * 4;
@@ -227,8 +231,8 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
 #pragma unroll
                     for(int h = 0; h < 3; h++)
                         qr[u][t][h] = load4(rq, v + 1024 * h, (unsigned)(live ? s_next : 0) * 3072u);
-                } else if constexpr(QM == QROW) {
-                    qr[u][t][0] = load4(rq, v, (unsigned)(s_next * 32));
+                } else if constexpr(QM == QLANE || QM == QROW) {
+                    qr[u][t][0] = load4(rq, v, (unsigned)(s_next * (QM == QLANE ? 1024 : 32)));
                 } else {
 #pragma unroll
                     for(int j = 0; j < 4; j++)
@@ -452,16 +456,25 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
     }
 }
 
-// The filter in the order that the kernel's lanes load it, in three parts: [class][32 rows][step of sixteen][part][lane][8].  A
-// 16-byte load whose neighbouring lanes are rows of the filter apart takes the address unit four times as long as one of
-// consecutive addresses (73 and 16 cycles for a kilobyte).
+// The filter in the order that the kernels' lanes load it: [class][32 rows][step of eight][lane][4], or in three parts [class]
+// [32 rows][step of sixteen][part][lane][8].  A 16-byte load whose neighbouring lanes are rows of the filter apart takes the
+// address unit four times as long as one of consecutive addresses (73 and 16 cycles for a kilobyte), and that unit, not the
+// matrix unit, bounded 32x32 tiles: 3x3 256->256 at 8x14x14 44 -> 34 us, 512->512 at 8x7x7 51 -> 40, this copy included.
+constexpr int AS_IT_IS = SAGA_I32; // SagaFilterPackJob::dtype of an fp32 filter that is not split
+
+__device__ __host__ inline long long pack_chunks(const SagaFilterPackJob &g) // of a lane's elements
+{
+    return (long long)g.T * (g.dtype == AS_IT_IS ? g.C / 8 : (g.C + 15) / 16) * 64 * ((g.N + 31) / 32);
+}
+
 __device__ __forceinline__ void pack_chunk(const SagaFilterPackJob &g, long long i)
 {
-    const int S16 = (g.C + 15) / 16, steps = g.T * S16;
+    const int each = g.dtype == AS_IT_IS ? 4 : 8; // elements of a lane
+    const int S = (g.C + 2 * each - 1) / (2 * each), steps = g.T * S;
     const int lane = (int)(i & 63);
     const long long q = i >> 6;
     const int tile = (int)(q / steps), step = (int)(q - (long long)tile * steps);
-    const int n = tile * 32 + (lane & 31), tap = step / S16, ch = (step - tap * S16) * 16 + 8 * (lane >> 5);
+    const int n = tile * 32 + (lane & 31), tap = step / S, ch = (step - tap * S) * 2 * each + each * (lane >> 5);
     const int a = tap / g.Ts, s = tap - a * g.Ts;
     if(g.dtype == SAGA_HALF) { // (window_f16.hip; channels are contiguous)
         half8_t v = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -475,7 +488,12 @@ __device__ __forceinline__ void pack_chunk(const SagaFilterPackJob &g, long long
     if(n < g.N && ch < g.C) { // channels come in eights
 #pragma unroll
         for(int j = 0; j < 8; j++)
-            v[j] = src[j * g.w_sc];
+            if(j < each)
+                v[j] = src[j * g.w_sc];
+    }
+    if(g.dtype == AS_IT_IS) {
+        *((float4_t *)g.packed + i) = float4_t{v[0], v[1], v[2], v[3]};
+        return;
     }
     Parts p;
     split3_any(v, p);
@@ -485,7 +503,7 @@ __device__ __forceinline__ void pack_chunk(const SagaFilterPackJob &g, long long
         out[64 * h] = __builtin_bit_cast(float4_t, p.v[h]);
 }
 
-constexpr int PACK_CHUNKS = 1024; // of eight elements, per block
+constexpr int PACK_CHUNKS = 1024; // per block
 
 __global__ void __launch_bounds__(256) stream_pack(const SagaFilterPackJob *__restrict__ jobs, int njobs)
 {
@@ -498,7 +516,7 @@ __global__ void __launch_bounds__(256) stream_pack(const SagaFilterPackJob *__re
             hi = mid - 1;
     }
     const SagaFilterPackJob g = jobs[lo];
-    const long long total = (long long)g.T * ((g.C + 15) / 16) * 64 * ((g.N + 31) / 32);
+    const long long total = pack_chunks(g);
 #pragma unroll
     for(int k = 0; k < PACK_CHUNKS / 256; k++) {
         const long long i = (long long)((int)blockIdx.x - g.first_block) * PACK_CHUNKS + k * 256 + threadIdx.x;
@@ -515,7 +533,7 @@ struct PackArgs {
 __global__ void __launch_bounds__(256) stream_pack_call(PackArgs a)
 {
     const SagaFilterPackJob &g = a.job[blockIdx.y];
-    const long long total = (long long)g.T * ((g.C + 15) / 16) * 64 * ((g.N + 31) / 32);
+    const long long total = pack_chunks(g);
     for(long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < total; i += (long long)gridDim.x * 256)
         pack_chunk(g, i);
 }
@@ -527,13 +545,15 @@ struct Config {
 // Tile (32*tm x 32*tn per wavefront), wavefronts of a block along the reduction (ks) and along the pixels (wm) for
 // `pixels` x N results with `steps` reduction steps of eight.  Splits fill 1024 SIMDs; the limits are where the measured
 // times cross (us, tm,tn,ks,wm; launches included).
-// Packed filters (those that windows do not take): the smallest tile balances best, four wavefronts to one tile (blocks of one
-// tile spread more evenly than blocks of four), unless the reduction is so short that writing the result dominates:
-//   3x3   64->64,  8x56x56   1,1,4,1  23.6   1,1,1,4  24.6   1,1,2,2  24.7   2,1,1,4  26.7
-//   3x3  256->256, 8x14x14   1,1,8,1  27.1   1,1,4,1  29.1   2,1,4,1  31.9
-//   3x3  512->512, 8x7x7     1,1,16,1 31.0   1,1,8,1  31.3   1,1,4,1  35.3
-//   1x1  256->64,  8x56x56   1,1,1,4  14.2   1,1,2,2  15.3   1,1,4,1  16.7   2,1,1,4  15.7
-//   1x1  256->512, 8x56x56 at stride 2  2,2,1,4  26.2   1,1,2,2  32.5   1,1,1,4  34.7
+// Packed filters: the address unit has room, so the smallest tile balances best, four wavefronts to one tile (blocks of
+// one tile spread more evenly than blocks of four), unless the reduction is so short that writing the result dominates:
+//   3x3   64->64,  8x56x56   1,1,4,1  27.5   1,1,1,4  27.8   2,1,4,1  30.7   1,1,2,2  28.7
+//   3x3  256->256, 32x14x14  1,1,4,1  79.1   2,2,4,1  84.3   1,1,2,2  87.9
+//   3x3  256->256, 8x14x14   1,1,8,1  26.8   1,1,4,1  28.5   2,1,4,1  32.3
+//   3x3  512->512, 8x7x7     1,1,8,1  28.1   1,1,16,1 28.3   1,1,4,1  34.9
+//   1x1  256->64,  8x56x56   1,1,1,4  15.6   1,1,2,2  17.1   1,1,4,1  17.9   2,1,1,4  17.6
+//   1x1   64->256, 8x56x56   2,2,1,4  18.2   1,1,1,4  20.3
+//   3x3   64->64,  32x56x56  1,1,1,4  80.0   2,2,1,4  82.8
 // Filters and matrices read in place or through a table: large tiles reuse what they load.
 //   1x1 1024->256, 8x14x14   1,1,4,1  18     2,1,4,1  20     1,1,1,4  33
 //   1x1 64->256,   8x56x56   2,1,1,4  22     1,1,1,4  23     1,1,4,1  37
@@ -589,7 +609,7 @@ template <int PM, int QM, bool EX, typename A> int launch_as(const A &k, const C
 
 template <int PM, int QM> int launch(Args &g, hipStream_t st, long long pixels, long long steps)
 {
-    const Config cf = choose(QM == QSPLIT, pixels, g.N, steps);
+    const Config cf = choose(QM == QLANE || QM == QSPLIT, pixels, g.N, steps);
     g.KS = cf.ks;
     g.nblk_q = (g.N + 32 * cf.tn - 1) / (32 * cf.tn);
     long long blocks = 0;
@@ -630,13 +650,14 @@ long long extent(const SagaTensorView *v)
 int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }
 
 // packed size of a class with that many taps
-long long packed_class(bool bwd, const ConvGeom &g, int taps)
+long long packed_class(bool bwd, const ConvGeom &g, int taps, bool parts)
 {
-    return (long long)taps * (((bwd ? g.K : g.C) + 15) / 16) * (((bwd ? g.C : g.K) + 31) / 32) * 3072;
+    const int red = bwd ? g.K : g.C, tiles = ((bwd ? g.C : g.K) + 31) / 32;
+    return parts ? (long long)taps * ((red + 15) / 16) * tiles * 3072 : (long long)taps * red * tiles * 128;
 }
 
 // the classes of a convolution and how its taps step; false if there are too many
-bool classes(bool bwd, const ConvGeom &g, Args &a)
+bool classes(bool bwd, const ConvGeom &g, Args &a, bool parts = false)
 {
     const int s = bwd ? g.stride : 1;
     if(s * s > MAX_CLASSES)
@@ -675,7 +696,7 @@ bool classes(bool bwd, const ConvGeom &g, Args &a)
             return false;
         c.M = (int)M;
         c.q0 = at;
-        at += packed_class(bwd, g, c.Tr * c.Ts);
+        at += packed_class(bwd, g, c.Tr * c.Ts, parts);
     }
     return true;
 }
@@ -686,14 +707,33 @@ WindowConv window_of(const Args &k)
     return {c.Tr, c.Ts, c.iy0, c.ix0, k.istep, k.tstep, k.p_bytes};
 }
 
-// The filter is packed: it cannot be read in place, or there is so much to multiply that the copy does not count (its launch takes
-// about 3 us).
-bool packs(bool bwd, const ConvGeom &g)
+// The filter can be read in place (given dense rows, or columns).
+bool in_place(bool bwd, const ConvGeom &g) { return g.R == 1 && g.S == 1 && (!bwd || g.stride == 1); }
+
+// What a filter that is packed beforehand is packed for, windows (in three parts) or QLANE.  It is read by calls on images of
+// any number and any strides, so that neither counts here.
+bool for_windows(bool bwd, const ConvGeom &g, const Args &k)
 {
-    if((bwd ? g.K : g.C) % 8)
-        return false;
+    return k.nclasses == 1 && window_f32_may(window_of(k), bwd ? g.K : g.C, bwd ? g.P : g.H, bwd ? g.Q : g.W, bwd ? g.H : g.P, bwd ? g.W : g.Q);
+}
+
+size_t packed_size(bool bwd, const ConvGeom &g, const Args &k, bool parts)
+{
+    long long n = 0;
+    int taps = 0;
+    for(int i = 0; i < k.nclasses; i++) {
+        n += packed_class(bwd, g, k.cls[i].Tr * k.cls[i].Ts, parts);
+        taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
+    }
+    return taps <= 64 && n <= 0x7ffffe00ll ? (size_t)n : 0;
+}
+
+// Windows of a filter that can be read in place: there has to be so much to multiply that the copy does not count (its launch takes
+// about 3 us).
+bool pays(bool bwd, const ConvGeom &g)
+{
     const long long pixels = bwd ? (long long)g.N * g.H * g.W : (long long)g.N * g.P * g.Q;
-    return g.R > 1 || g.S > 1 || (bwd && g.stride > 1) || pixels * (bwd ? g.C : g.K) >= 1ll << 24;
+    return !in_place(bwd, g) || pixels * (bwd ? g.C : g.K) >= 1ll << 24;
 }
 
 void describe(bool bwd, const SagaTensorView *w, Args &k)
@@ -706,7 +746,7 @@ void describe(bool bwd, const SagaTensorView *w, Args &k)
 
 static_assert(sizeof(SagaFilterPackJob) == 88, "as it was before it had a dtype");
 
-int pack_jobs(const Args &k, const void *w, char *packed, SagaFilterPackJob *jobs)
+int pack_jobs(const Args &k, const void *w, char *packed, bool parts, SagaFilterPackJob *jobs)
 {
     int n = 0;
     for(int i = 0; i < k.nclasses; i++) {
@@ -724,7 +764,7 @@ int pack_jobs(const Args &k, const void *w, char *packed, SagaFilterPackJob *job
         j.r0 = c.r0;
         j.s0 = c.s0;
         j.rstep = k.rstep;
-        j.dtype = SAGA_FLOAT;
+        j.dtype = parts ? SAGA_FLOAT : AS_IT_IS;
         j.first_block = 0;
         j.blocks = stream_pack_blocks(j);
     }
@@ -733,23 +773,14 @@ int pack_jobs(const Args &k, const void *w, char *packed, SagaFilterPackJob *job
 
 } // namespace
 
-int stream_pack_blocks(const SagaFilterPackJob &j)
-{
-    return (int)(((long long)j.T * ((j.C + 15) / 16) * 64 * ((j.N + 31) / 32) + PACK_CHUNKS - 1) / PACK_CHUNKS);
-}
+int stream_pack_blocks(const SagaFilterPackJob &j) { return (int)((pack_chunks(j) + PACK_CHUNKS - 1) / PACK_CHUNKS); }
 
 size_t stream_f32_packed_bytes(bool bwd, const ConvGeom &g)
 {
     Args k = {};
     if((bwd ? g.K : g.C) % 8 || g.group != 1 || !classes(bwd, g, k))
         return 0;
-    long long n = 0;
-    int taps = 0;
-    for(int i = 0; i < k.nclasses; i++) {
-        n += packed_class(bwd, g, k.cls[i].Tr * k.cls[i].Ts);
-        taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
-    }
-    return taps <= 64 && n <= 0x7ffffe00ll ? (size_t)n : 0;
+    return packed_size(bwd, g, k, for_windows(bwd, g, k));
 }
 
 int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob *jobs)
@@ -757,10 +788,12 @@ int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, v
     Args k = {};
     if(!classes(bwd, g, k))
         return 0;
+    const bool parts = for_windows(bwd, g, k);
+    classes(bwd, g, k, parts);
     k.N = bwd ? g.C : g.K;
     k.C = bwd ? g.K : g.C;
     describe(bwd, w, k);
-    return pack_jobs(k, w->ptr, (char *)packed, jobs);
+    return pack_jobs(k, w->ptr, (char *)packed, parts, jobs);
 }
 
 int stream_f32_pack(const SagaFilterPackJob *jobs, int njobs, int blocks, hipStream_t st)
@@ -770,17 +803,26 @@ int stream_f32_pack(const SagaFilterPackJob *jobs, int njobs, int blocks, hipStr
     return 0;
 }
 
-bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g)
+bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room)
 {
     Args k = {};
     const long long bytes = extent(a);
-    if(g.group != 1 || bytes < 0 || bytes > 0x7ffffe00ll || !classes(bwd, g, k) || k.nclasses > 1)
+    if(g.group != 1 || (bwd ? g.K : g.C) % 8 || bytes < 0 || bytes > 0x7ffffe00ll || !classes(bwd, g, k) || k.nclasses > 1)
         return false;
     k.p_bytes = (unsigned)bytes;
-    return window_f32_takes(window_of(k), a, out);
+    const size_t need = packed_size(bwd, g, k, true);
+    return need && (packed ? for_windows(bwd, g, k) : pays(bwd, g) && room >= need) && window_f32_takes(window_of(k), a, out);
 }
 
-size_t stream_f32_conv_workspace(bool bwd, const ConvGeom &g) { return packs(bwd, g) ? stream_f32_packed_bytes(bwd, g) : 0; }
+size_t stream_f32_conv_workspace(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g)
+{
+    Args k = {};
+    if((bwd ? g.K : g.C) % 8 || g.group != 1 || !classes(bwd, g, k))
+        return 0;
+    if(stream_f32_windows(bwd, a, out, g, false, ~(size_t)0))
+        return packed_size(bwd, g, k, true);
+    return in_place(bwd, g) ? 0 : packed_size(bwd, g, k, false);
+}
 
 int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g,
                     float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st)
@@ -812,29 +854,44 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
     for(int i = 0; i < k.nclasses; i++)
         taps = std::max(taps, k.cls[i].Tr * k.cls[i].Ts);
     if(k.C % 8 == 0 && taps <= 64) {
-        const size_t bytes = packed || packs(bwd, g) ? stream_f32_packed_bytes(bwd, g) : 0;
-        // (without room for the copy: through the table, or the kernels that need less)
-        if(bytes && (packed || (ws && ws_bytes >= bytes && aligned16(ws)))) {
+        const size_t room = ws && aligned16(ws) ? ws_bytes : 0;
+        // in three parts for windows, or as it is; packed beforehand as for_windows() has it
+        auto from = [&](bool parts) {
+            const size_t bytes = packed_size(bwd, g, k, parts);
+            classes(bwd, g, k, parts);
             if(!packed) {
                 PackArgs pa;
-                pa.n = pack_jobs(k, w->ptr, (char *)ws, pa.job);
-                const dim3 grid(grid_for((long long)bytes / 48 / k.nclasses, 256, 4096), pa.n);
+                pa.n = pack_jobs(k, w->ptr, (char *)ws, parts, pa.job);
+                const dim3 grid(grid_for((long long)bytes / (parts ? 48 : 16) / k.nclasses, 256, 4096), pa.n);
                 stream_pack_call<<<grid, 256, 0, st>>>(pa);
-                packed = ws;
             }
-            k.q = (const float *)packed;
+            k.q = (const float *)(packed ? packed : ws);
             k.q_bytes = (unsigned)bytes;
-            if(k.nclasses == 1) {
-                const int r = window_f32_conv(window_of(k), a, out, alpha, beta, e, packed, bytes, st);
-                if(r != SAGA_HIP_EUNSUPPORTED)
-                    return r;
-            }
-            return launch<PTAP, QSPLIT>(k, st, pixels, steps);
+            return bytes;
+        };
+        if(stream_f32_windows(bwd, a, out, g, packed != nullptr, room)) {
+            const Args before = k;
+            const size_t bytes = from(true);
+            const int r = window_f32_conv(window_of(k), a, out, alpha, beta, e, k.q, bytes, st);
+            if(r != SAGA_HIP_EUNSUPPORTED || packed)
+                return r == SAGA_HIP_EUNSUPPORTED ? launch<PTAP, QSPLIT>(k, st, pixels, steps) : r;
+            k = before; // (an output out of its reach)
+        }
+        if(packed && packed_size(bwd, g, k, for_windows(bwd, g, k))) {
+            const bool parts = for_windows(bwd, g, k);
+            from(parts);
+            return parts ? launch<PTAP, QSPLIT>(k, st, pixels, steps) : launch<PTAP, QLANE>(k, st, pixels, steps);
+        }
+        const size_t plain = packed_size(bwd, g, k, false);
+        // (without room for the copy: through the table, or the kernels that need less)
+        if(!in_place(bwd, g) && plain && room >= plain) {
+            from(false);
+            return launch<PTAP, QLANE>(k, st, pixels, steps);
         }
         // 1x1: the filter as it is, if its rows are dense
-        if(!bytes && !bwd && k.q_sc == 1)
+        if(in_place(bwd, g) && !bwd && k.q_sc == 1)
             return launch<PTAP, QROW>(k, st, pixels, steps);
-        if(!bytes && bwd && k.q_sn == 1)
+        if(in_place(bwd, g) && bwd && k.q_sn == 1)
             return launch<PTAP, QCOL>(k, st, pixels, steps);
     }
     if(taps <= 63 && (long long)taps * k.C <= MAX_TABLE - 8)

@@ -426,7 +426,7 @@ Plan fit(const WinArgs &g, int Tr, int kg, const Config &cf)
 // A wavefront under nine taps has enough to do on 64 pixels as soon as there is one per SIMD or nearly; under one tap, which waits
 // for memory, two are better.  Fewer than those: the reduction is split.  Then blocks as large as leave one for three CUs of
 // four: those of a group read the same window, and through the L1 the same filter.
-Plan choose(const WinArgs &g, int Tr, int kg)
+Plan tiles_for(const WinArgs &g, int Tr, int kg)
 {
     const int taps = g.T, slices = (g.C + 8 * kg - 1) / (8 * kg), columns = (g.o.N + 31) / 32;
     auto tiles = [&](int tm) { return (long long)((g.M + 32 * tm - 1) / (32 * tm)) * columns; };
@@ -473,10 +473,50 @@ Plan choose(const WinArgs &g, int Tr, int kg)
     return {};
 }
 
+// Where operands straight from memory (stream_f32.hip) are faster after all (us, those / windows):
+//   1x1 over many pixels, with a slice of 64 channels or a tile of 64 results that is not full: 16->56 70x111x111 61 / 162, 88->16
+//   247x66x66 96 / 210, 24->456 45x68x68 156 / 184, 64->352 109x24x24 48 / 55 (128->256 123x49x49 228 / 193);
+//   blocks of two wavefronts that take a CU's LDS, or under 25 taps: 3x3 at stride 2, 40->64 103x13x13 13 / 21, 472->16 41x13x13
+//   30 / 41, 3x3 336->16 1x107x107 36 / 59, 5x5 32->16 5x86x86 31 / 56, 40->136 3x24x24 19 / 24;
+//   few slices over four or eight groups, half of which has one to do less: 3x3 72->152 17x16x16 20 / 30, 72->16 29x37x37 25 / 39;
+//   few slices for each of four groups, or one tile, and a last round of blocks that is nearly empty: 3x3 72->128 3x54x54 26 / 32,
+//   160->64 2x53x53 22 / 28; of one tile and a large window, over half of the CUs: 104->24 1x70x70 12.5 / 14;
+//   one step of channels at stride 2, where a window is four times what its pixels see, and two over many pixels: 3x3 16->296
+//   141x48x48 98 / 135, 24->392 61x55x55 122 / 154.
+// Of 553 layers under 9 and 25 taps these rules leave 483 to windows, 14 of them (58 before) slower by more than 4 %.
+bool worth(const WinArgs &g, const Plan &p)
+{
+    const Config &c = p.cf;
+    if(g.T == 1)
+        return (long long)g.M * g.o.N < 1ll << 24 || (g.C > 64 && g.o.N > 64);
+    const int waves = c.wm * c.wn * c.ks, slices = (g.C + 15) / 16;
+    const long long blocks = (long long)((g.M + 32 * c.tm * c.wm - 1) / (32 * c.tm * c.wm)) * ((g.o.N + 32 * c.wn - 1) / (32 * c.wn));
+    if(g.T == 9 && g.istep > 1 && g.C <= (blocks > 2048 ? 32 : 16))
+        return false;
+    if(g.T == 9 && (slices + c.ks - 1) / c.ks * c.ks * 2 > slices * 3)
+        return false;
+    if((160 * 1024) / (p.lds + 2560) > 1)
+        return waves > 2 || g.T == 9;
+    if(waves <= 2)
+        return false;
+    if(g.T != 9 || c.ks < 4)
+        return true;
+    const long long rounds = (blocks + 255) / 256;
+    if(rounds > 1 && rounds * 256 * 5 > blocks * 6 && (waves == 4 || slices <= 2 * c.ks))
+        return false;
+    return !(waves == 4 && g.istep == 1 && p.quads > 30 && blocks > 128);
+}
+
+Plan choose(const WinArgs &g, int Tr, int kg)
+{
+    const Plan p = tiles_for(g, Tr, kg);
+    return p.quads && worth(g, p) ? p : Plan{};
+}
+
 bool describe(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, WinArgs &g)
 {
     const int taps = c.Tr * c.Ts, IH = a->dims[2], IW = a->dims[3];
-    if((taps != 1 && taps != 9 && taps != 25) || a->dims[1] % 8 || a->dims[1] < 16 ||
+    if(!window_f32_may(c, a->dims[1], IH, IW, out->dims[2], out->dims[3]) ||
        (IW > 1 && a->strides[3] != 1) || (IH > 1 && a->strides[2] != IW))
         return false;
     const long long pixels = (long long)out->dims[0] * out->dims[2] * out->dims[3];
@@ -539,6 +579,28 @@ template <int KG, int TAPS, int DEPTH, bool APART, bool EX> int launch_as(const 
 }
 
 } // namespace
+
+bool window_f32_may(const WindowConv &c, int channels, int IH, int IW, int OH, int OW)
+{
+    WinArgs g = {};
+    g.T = c.Tr * c.Ts;
+    if((g.T != 1 && g.T != 9 && g.T != 25) || channels % 8 || channels < 16 || (long long)IH * IW >= 1ll << 30)
+        return false;
+    g.Ts = c.Ts;
+    g.IH = IH;
+    g.IW = IW;
+    g.iy0 = c.iy0;
+    g.ix0 = c.ix0;
+    g.istep = c.istep;
+    g.tstep = c.tstep;
+    g.plane4 = (int)(((long long)IH * IW + 3) / 4 * 4);
+    g.ow = fast_div(OW);
+    g.oh = fast_div(OH);
+    for(int wn = 1; wn <= 8; wn *= 2) // (the smallest tile; with more wavefronts to load its window)
+        if(fit(g, c.Tr, slice_groups(g.T), {1, 1, 1, wn, 1}).quads || fit(g, c.Tr, slice_groups(g.T), {1, 1, wn, 1, 1}).quads)
+            return true;
+    return false;
+}
 
 bool window_f32_takes(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out)
 {

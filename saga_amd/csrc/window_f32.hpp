@@ -8,6 +8,8 @@ struct WindowConv {
     unsigned a_bytes; // of the tensor read
 };
 
+// whether any such convolution of so many channels, input and output pixels could, whatever the number and the strides of its images
+bool window_f32_may(const WindowConv &c, int channels, int IH, int IW, int OH, int OW);
 // whether such a convolution goes through the kernel (with operands of the usual extent)
 bool window_f32_takes(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out);
 // packed: the filter as stream_f32_pack leaves it.  SAGA_HIP_EUNSUPPORTED (nothing enqueued) outside what the kernel covers.

@@ -85,8 +85,9 @@ def test_biases_that_are_no_vector_are_refused():
         assert L.saga_hip_bias_add(C.byref(y), C.byref(b), None) == want
 
 
-def convolution(kind, shape, dtype, bias=False):
-    """The launches of a convolution of dense tensors (forward: also with a bias), and the pixels of its classes and its columns."""
+def convolution(kind, shape, dtype, bias=False, room=1.0):
+    """The launches of a convolution of dense tensors (forward: also with a bias), and the pixels of its classes and its columns.
+    room: bytes of workspace, or (a float) a share of what the query asks for."""
     n, c, h, w, k, r, stride, pad = shape
     p, q = 1 + (h + 2 * pad - r) // stride, 1 + (w + 2 * pad - r) // stride
     x, f, y = (image(a, *d, dtype=dtype) for a, d in ((X, (n, c, h, w)), (W << 2, (k, c, r, r)), (Y << 3, (n, k, p, q))))
@@ -95,7 +96,8 @@ def convolution(kind, shape, dtype, bias=False):
             d = v.dims
             v.strides[:] = [d[1] * d[2] * d[3], d[2] * d[3], d[3], 1]
     L, cp = K.lib(), K.ConvParams(pad, stride, 1, 1)
-    room = L.saga_hip_conv2d_workspace_size(kind, C.byref(x), C.byref(f), C.byref(y), C.byref(cp))
+    if isinstance(room, float):
+        room = int(room * L.saga_hip_conv2d_workspace_size(kind, C.byref(x), C.byref(f), C.byref(y), C.byref(cp)))
     b = image(1 << 35, 1, k if kind == K.CONV_FWD else c, 1, 1, dtype=dtype)
     stub_gpu.launched()
     if kind == K.CONV_FWD:
@@ -213,3 +215,44 @@ def test_fused_bias_shapes_are_what_their_names_say():
             elif what:
                 assert any(x.startswith(BIAS_KERNELS[what]) for x in launches), (name, launches)
                 assert ("split_reduce" in launches) == (what == "shared tiles"), (name, launches)
+
+
+# a forward pass or backward data, a workspace in bytes or a share of what is asked for: the kernel, how it reads the filter (fp32 from
+# memory: 0 and 1 in place, 2 through a table, 3 packed)
+F32_ROUTES = [
+    # 1x1 over many pixels: windows where there is room to pack the filter, and otherwise in place as ever
+    ((4, 256, 128, 128, 256, 1, 1, 0), K.CONV_FWD, 1.0, "stream_f32_k_window", None),
+    ((4, 256, 128, 128, 256, 1, 1, 0), K.CONV_FWD, 0, "stream_f32_k", 0),
+    ((4, 256, 128, 128, 256, 1, 1, 0), K.CONV_BWD_DATA, 0, "stream_f32_k", 1),
+    ((4, 4104, 128, 128, 256, 1, 1, 0), K.CONV_FWD, 0, "stream_f32_k", 0),
+    ((32, 64, 112, 112, 48, 1, 1, 0), K.CONV_FWD, 0, "stream_f32_k", 0),
+    # ... and where a slice of channels or a tile of results would not be full, in place or in tiles, with room too
+    ((217, 16, 62, 62, 40, 1, 1, 0), K.CONV_FWD, 1.0, "stream_f32_k", 0),
+    ((205, 56, 59, 59, 48, 1, 1, 0), K.CONV_FWD, 1.0, "stream_f32_k", 0),
+    ((84, 64, 56, 56, 56, 1, 1, 0), K.CONV_FWD, 1.0, "conv_f32_gather_uniform", None),
+    ((109, 64, 62, 62, 352, 1, 1, 0), K.CONV_FWD, 1.0, "conv_f32_gather_uniform", None),
+    # no room for three parts, but for the filter as it is; not for that either
+    ((8, 512, 14, 14, 512, 3, 1, 1), K.CONV_FWD, 1.0, "stream_f32_k_window", None),
+    ((8, 512, 14, 14, 512, 3, 1, 1), K.CONV_FWD, 4 * 9 * 512 * 512, "stream_f32_k", 3),
+    ((8, 512, 14, 14, 512, 3, 1, 1), K.CONV_BWD_DATA, 4 * 9 * 512 * 512, "stream_f32_k", 3),
+    ((8, 64, 28, 28, 64, 3, 1, 1), K.CONV_FWD, 64, "stream_f32_k", 2),
+    ((256, 64, 56, 56, 64, 3, 1, 1), K.CONV_FWD, 1.0, "stream_f32_k_window", None),
+    ((256, 64, 56, 56, 64, 3, 1, 1), K.CONV_FWD, 6 * 9 * 64 * 64 - 16, "conv_f32_gather_uniform", None),
+    # windows that would leave the chip half empty
+    ((103, 40, 13, 13, 64, 3, 2, 1), K.CONV_FWD, 1.0, "stream_f32_k", 3),
+    ((1, 16, 107, 107, 336, 3, 1, 1), K.CONV_BWD_DATA, 1.0, "stream_f32_k", 3),
+    ((29, 72, 37, 37, 16, 3, 1, 1), K.CONV_FWD, 1.0, "stream_f32_k", 3),
+    ((3, 128, 54, 54, 72, 3, 1, 1), K.CONV_BWD_DATA, 1.0, "stream_f32_k", 3),
+    ((141, 16, 48, 48, 296, 3, 2, 1), K.CONV_FWD, 1.0, "stream_f32_k", 3),
+    # what windows do not take at all
+    ((243, 8, 32, 32, 288, 5, 2, 2), K.CONV_FWD, 1.0, "stream_f32_k", 3),
+    ((2, 456, 15, 15, 40, 7, 1, 3), K.CONV_FWD, 1.0, "stream_f32_k", 3),
+]
+
+
+@on_stub
+def test_fp32_routes():
+    for shape, kind, room, kernel, reads in F32_ROUTES:
+        launches = convolution(kind, shape, K.FLOAT, room=room)[0]
+        (ran,) = [x for x in launches if "pack" not in x[0] and "build" not in x[0]]
+        assert ran[0] == kernel and reads in (None, ran[1][1]), (shape, kind, room, ran)

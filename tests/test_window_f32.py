@@ -20,16 +20,18 @@ SHAPES = {
     (9, 136, 27, 30, 72, 1, 2, 0): (1, 4, 1, 2),     # pixels apart
     (40, 64, 43, 64, 170, 1, 3, 0): (1, 1, 1, 8),
     (90, 40, 33, 32, 96, 1, 2, 1): (1, 1, 1, 4),     # some of them outside the image
-    (9, 72, 7, 7, 40, 3, 1, 1): (1, 1, 9, 4),        # windows over several images; half a step of channels
+    (9, 104, 7, 7, 40, 3, 1, 1): (1, 1, 9, 4),       # windows over several images; half a step of channels
     (8, 64, 28, 30, 128, 3, 1, 1): (2, 1, 9, 8),     # the reduction over four
     (5, 40, 70, 66, 64, 3, 1, 1): (2, 1, 9, 4),      # 128 pixels to a window
     (7, 24, 20, 126, 17, 3, 1, 1): (1, 2, 9, 4),     # two rounds of loads
-    (6, 16, 21, 23, 24, 3, 2, 1): (1, 2, 9, 1),      # stride 2 (backward: classes, not here)
-    (4, 32, 14, 14, 64, 5, 1, 2): (1, 1, 25, 2),
+    (60, 24, 21, 23, 40, 3, 2, 1): (1, 1, 9, 4),     # stride 2 (backward: classes, not here)
+    (4, 64, 14, 14, 64, 5, 1, 2): (1, 1, 25, 4),     # the reduction over four
     (60, 16, 28, 28, 130, 5, 1, 0): (1, 1, 25, 4),   # backward: more padding than the filter needs, pixels out of order: not here
 }
 
-CLASSES = (2, 24, 11, 13, 40, 3, 2, 1)  # backward: residue classes of pixels, straight from memory (csrc/stream_f32.hip)
+# straight from memory (csrc/stream_f32.hip): backward residue classes of pixels, of filters as they are; and, too few pixels for a
+# window, filters in three parts
+CLASSES, FEW = (2, 24, 11, 13, 40, 3, 2, 1), (1, 24, 9, 11, 40, 3, 1, 1)
 
 
 def views(shape, x, w, y):
@@ -61,6 +63,15 @@ def test_shapes_are_what_they_are_said_to_be():
         run(K.CONV_FWD, shape, 1 << 20, 1 << 33, 1 << 34, 1 << 35)
         ((name, tile, blocks, threads),) = stub_gpu.launched()
         assert name == "stream_f32_k_window" and (tile[0], tile[4], tile[5], threads) == (tm, rounds, taps, 64 * waves), (shape, tile, threads)
+
+
+@on_stub
+def test_packed_filters_without_windows():
+    for shape, kind, q in ((CLASSES, K.CONV_FWD, 4), (CLASSES, K.CONV_BWD_DATA, 3), (FEW, K.CONV_FWD, 4), (FEW, K.CONV_BWD_DATA, 4)):
+        stub_gpu.launched()
+        run(kind, shape, 1 << 20, 1 << 33, 1 << 34, 1 << 35)
+        ((name, tile, blocks, threads),) = stub_gpu.launched()
+        assert (name, tile[1]) == ("stream_f32_k", q), (shape, kind, tile)
 
 
 def reference(shape, x, w, dy):
@@ -127,7 +138,7 @@ def test_against_64_bits(shape):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("scales", [(-120, 80), (80, -120), (-140, 100), (-20, -100)], ids=str)
-@pytest.mark.parametrize("shape", [*SHAPES, CLASSES], ids=str)
+@pytest.mark.parametrize("shape", [*SHAPES, CLASSES, FEW], ids=str)
 def test_small_numbers(shape, scales):
     """Operands whose low bits a bf16 cannot hold, subnormal ones among them, are multiplied with all their bits."""
     n, c, h, wd, k, r, stride, pad = shape
@@ -142,7 +153,7 @@ def test_small_numbers(shape, scales):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("shape", [*SHAPES, CLASSES, (1, 24, 150, 161, 24, 3, 1, 1)])
+@pytest.mark.parametrize("shape", [*SHAPES, CLASSES, FEW, (1, 24, 150, 161, 24, 3, 1, 1)])
 def test_numbers_without_three_parts(shape):
     """Infinities, NaNs and numbers next to the largest in either operand: where they belong, nowhere else; and what shares a
     wavefront with them is multiplied with all bits of its weights."""
