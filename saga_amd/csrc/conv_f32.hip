@@ -866,6 +866,32 @@ static bool fit_splits(FilterSplit &p, const ConvGeom &g, int step, size_t one, 
     return true;
 }
 
+static size_t tab_bytes(int n) { return (((size_t)n * (sizeof(KTabA) + sizeof(long long))) + 255) & ~(size_t)255; }
+
+// The kernel for windows (filter_f32.hip) with `bytes` of workspace for partial results, or none where the others take less
+// time: both launches, the tiles' area times the pixels, a block's slices one after the other, partial results (fitted to 221 layers of
+// 8 to 512 channels, 15 % off at most).
+static FilterWindows filter_windows(const ConvGeom &g, size_t bytes)
+{
+    const size_t one = (size_t)g.K * g.C * g.R * g.S * sizeof(float);
+    FilterWindows w = plan_filter_windows(g);
+    w.splits = (int)std::min<size_t>(w.splits, bytes / one);
+    if(!w.splits)
+        return w;
+    const bool uniform = g.C % 32 == 0;
+    FilterSplit p = uniform ? plan_filter_uniform(g) : plan_filter_f32(g);
+    const size_t table = uniform ? 0 : tab_bytes(g.C * g.R * g.S);
+    if(bytes < table || !fit_splits(p, g, uniform ? UW_P : WBK, one, bytes - table))
+        return w; // (the others have no room at all)
+    const double area = (double)p.tiles_k * p.tiles_c * (uniform ? UW_K * UW_C : WBM * WBN) * g.N * g.P * g.Q;
+    const double partials = (double)p.splits * g.K * g.C * g.R * g.S;
+    const double other = uniform ? 7400 + 12.5e-6 * area + 30 * p.m_per_split + 2.6e-3 * partials
+                                 : 9100 + 29.6e-6 * area + 21 * p.m_per_split + 1.9e-3 * partials;
+    if(filter_windows_ns(w, g) >= other)
+        w.splits = 0;
+    return w;
+}
+
 static long long extent_bytes(const SagaTensorView *v)
 {
     long long ext = 1;
@@ -896,7 +922,6 @@ static bool f32_ok(const SagaTensorView *a, const SagaTensorView *b, const SagaT
            (long long)g.C * g.R * g.S < big;
 }
 
-static size_t tab_bytes(int n) { return (((size_t)n * (sizeof(KTabA) + sizeof(long long))) + 255) & ~(size_t)255; }
 
 // the wave-uniform gather kernel: padded table + transposed, padded filter
 struct UniPlan {
@@ -954,7 +979,7 @@ size_t conv_f32_workspace(int kind, const SagaTensorView *x, const SagaTensorVie
         return std::max(stream, (a > b ? a : b) + 256);
     }
     const FilterSplit p = plan_filter_f32(g), pu = plan_filter_uniform(g);
-    const int splits = std::max(std::max(p.splits, pu.splits), plan_filter_windows(g).splits);
+    const int splits = std::max(std::max(p.splits, pu.splits), filter_windows(g, ~(size_t)0).splits);
     return tab_bytes(g.C * g.R * g.S) + (size_t)splits * g.K * g.C * g.R * g.S * sizeof(float) + 256;
 }
 
@@ -1168,8 +1193,7 @@ int conv_f32_bwd_filter(const SagaTensorView *x, const SagaTensorView *dy, const
     if(!f32_ok(x, dy, dw, g))
         return SAGA_HIP_EUNSUPPORTED;
     const int CRS = g.C * g.R * g.S;
-    FilterWindows fw = plan_filter_windows(g);
-    fw.splits = (int)std::min<size_t>(fw.splits, ws && aligned16(ws) ? ws_bytes / ((size_t)g.K * CRS * sizeof(float)) : 0);
+    const FilterWindows fw = filter_windows(g, ws && aligned16(ws) ? ws_bytes : 0);
     if(fw.splits) {
         const int r = launch_filter_windows(fw, x, dy, (float *)ws, g, st);
         if(r != SAGA_HIP_EUNSUPPORTED) {

@@ -314,11 +314,14 @@ unsigned image_bytes(const SagaTensorView *v)
 
 } // namespace
 
-// Where a block walks three tiles or more.  us, the kernel for fp32 matrix instructions (conv_f32_bwd_filter_uniform, where channels come
+// Where a block walks three tiles or more, and where that takes less time than the kernels for fp32 matrix instructions, which have
+// fewer pixels outside small images and fewer channels that are not there.  us, the kernel for fp32 matrix instructions (conv_f32_bwd_filter_uniform, where channels come
 // in 32s) / this one, both with the second pass:
 //   64->64   256x56x56  581 / 312   128->128 64x28x28  169 / 114   512->512  8x28x28  355 / 207   96->160 32x40x40    189 / 124
 //   64->64    64x56x56  178 /  95   256->256 128x14x14 311 / 192   32->32  128x16x16   46 /  37   16->16  128x32x32    67 /  51
 //   64->64    16x56x56   59 /  45   256->256  32x14x14  96 /  64   72->136   9x29x17   41 /  35   8->24    64x32x32    31 /  31
+// and left to them: 16->128 225x9x9 31 / 48, 32->104 130x11x11 27 / 39, 8->416 78x12x12 38 / 53, 64->120 76x11x11 32 / 41.  Of the 221
+// layers the slower kernel is taken in two, by 5 and 8 %.
 // 312 us are 190 TFLOP/s of fp32 work, 1140 of bf16: what bounds it is the matrix unit, and the reading of operands for the first step of
 // a tile, which nothing hides.  Relative error against 64 bits, the same shapes: 4.3e-7 to 9.8e-7 before, 1.2e-7 to 2.5e-7.
 FilterWindows plan_filter_windows(const ConvGeom &g)
@@ -332,6 +335,14 @@ FilterWindows plan_filter_windows(const ConvGeom &g)
     if(pairs > 1024 || tiles >= 0x7fffffff || tiles < 2 * share + 1)
         return {0, 0};
     return {(int)pairs, share};
+}
+
+// Both launches and the first tile, tiles of a block one after the other, and partial results to write and add up (fitted to 221 layers of 8
+// to 512 channels, 16 % off at most).
+double filter_windows_ns(const FilterWindows &p, const ConvGeom &g)
+{
+    const int64_t tiles = (int64_t)((g.W + TILE - 1) / TILE) * ((g.H + TILE - 1) / TILE) * g.N;
+    return 9500 + 4430.0 * ((tiles + p.splits - 1) / p.splits) + 2.24e-3 * p.splits * g.K * g.C * TAPS;
 }
 
 int launch_filter_windows(const FilterWindows &p, const SagaTensorView *x, const SagaTensorView *dy, float *partial, const ConvGeom &g,

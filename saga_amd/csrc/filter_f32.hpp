@@ -7,6 +7,7 @@ struct FilterWindows {
     int splits; // partial results: shares of the tiles
 };
 FilterWindows plan_filter_windows(const ConvGeom &g);
+double filter_windows_ns(const FilterWindows &p, const ConvGeom &g); // what it takes
 // partial[splits][K][9][C]; splits may be fewer than planned.  SAGA_HIP_EUNSUPPORTED: nothing was launched.
 int launch_filter_windows(const FilterWindows &p, const SagaTensorView *x, const SagaTensorView *dy, float *partial, const ConvGeom &g,
                           hipStream_t st);
