@@ -45,8 +45,8 @@ def test_routes():
             stub_gpu.launched()
             rc = L.saga_hip_conv2d_bwd_filter(C.byref(x), C.byref(y), C.byref(f), p, 1.0, 0.0, 1 << 33, room, None)
             ran = [(name, blocks) for name, _, blocks, _ in stub_gpu.launched() if name == "conv_f32_bwd_filter_windows"]
-            if not taken:
-                assert ran == [], (n, c, h, w, k)
+            if not taken:  # (with room for one partial result and no table, whatever can run does)
+                assert ran == [] or room == one, (n, c, h, w, k)
             elif room < one:
                 assert rc != 0 and ran == []
             else:
