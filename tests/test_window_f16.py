@@ -57,9 +57,12 @@ def test_forms():
 
     for shape, form in SHAPES.items():
         assert forward(*shape) == [form], shape
-        # training: a large one, or a short reduction (there all of it in any case)
+        # training: from 2**17 values of a channel on, or with one slice of channels (half and wide forms: of 32, the others: of 16)
         n, c, h, w, k = shape
-        assert forward(*shape, stats=True) == ([form] if n * h * w * c >= 12800000 or c <= 32 else []), shape
+        slice = 32 if form[:3] in ((4, 2, 2), (2, 2, 4)) else 16
+        assert forward(*shape, stats=True) == ([form] if n * h * w >= 1 << 17 or c <= slice else []), shape
+    for n, h, taken in ((167, 28, 0), (168, 28, 1), (255, 28, 1), (256, 28, 1), (31, 65, 0), (32, 65, 1)):  # 130928, 131712 ... values
+        assert len(forward(n, 128, h, h, 128, stats=True)) == taken, (n, h)
     assert forward(262, 72, 14, 14, 256, room=0) == []  # no room for the packed filter, and nobody has it
     assert forward(6, 24, 95, 98, 256, room=0) == [(4, 2, 2, 10, 0)]
     assert forward(4, 72, 14, 14, 256) == []  # a small grid
