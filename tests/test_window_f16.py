@@ -66,6 +66,7 @@ def test_forms():
     assert forward(262, 72, 14, 14, 256, room=0) == []  # no room for the packed filter, and nobody has it
     assert forward(6, 24, 95, 98, 256, room=0) == [(4, 2, 2, 10, 0)]
     assert forward(4, 72, 14, 14, 256) == []  # a small grid
+    assert forward(106, 128, 17, 17, 16) == [] and len(forward(174, 392, 14, 14, 16)) == 1  # few results of a filter to pack
     assert forward(200, 16, 3, 330, 40) == []  # a row too long for a window, patches of which the image fills little
 
 
