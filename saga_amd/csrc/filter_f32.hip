@@ -14,7 +14,7 @@
 // columns, 32 channels) over all banks, the lower bits by fours, which do the same for a write (sixteen columns, one chunk).
 //
 // Tiles overlap where they do not divide an image, with zeros for the gradients of pixels seen before.  A sum that is not
-// finite had an operand without three parts: its wavefront takes its share again in fp32.
+// finite had an operand without three parts: its block takes its share again in fp32 products.
 #include "split_f32.hpp"
 #include "filter_f32.hpp"
 
@@ -60,6 +60,97 @@ template <int I, int N, class F> __device__ __forceinline__ void each(F &&f)
         f(std::integral_constant<int, I>());
         each<I + 1, N>(f);
     }
+}
+
+__device__ __forceinline__ void store_sums(const WindowFilterArgs &t, int split, int k, int c, const float16_t (&acc)[TAPS]) // (below)
+{
+    // (a share's partial result is one buffer: rows and columns beyond the filter are outside)
+    const unsigned bytes = (unsigned)t.K * (TAPS * 4u) * (unsigned)t.C, krow = TAPS * 4u * (unsigned)t.C;
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void *)((char *)t.partial + (int64_t)split * bytes), 0, bytes, 0x00020000);
+    const unsigned first = c < t.C ? (unsigned)k * krow + (unsigned)c * 4u : OOB;
+#pragma unroll
+    for(int tp = 0; tp < TAPS; tp++)
+#pragma unroll
+        for(int v = 0; v < 16; v++) {
+            const float sum = acc[tp][v]; // (the cast takes a vector's element for its first)
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), ro, first + (8 * (v / 4) + v % 4) * krow,
+                                                  tp * t.C * 4, 0);
+        }
+}
+
+// A block's share in fp32 products: a tile's pixels of x, with a border of one, and of dy go to LDS as they are, a matrix
+// instruction takes two neighbouring pixels, the next tile's loads are on their way meanwhile.  us, second pass included, finite / one
+// NaN (a wavefront's share pixel by pixel, as it was): 64->64 at 256x56x56 311 / 1110 (3320), 512->512 at 9x8x8 50 / 102 (222); the
+// kernel for fp32 matrix instructions 580 and 68.
+__device__ __forceinline__ void windows_again(const WindowFilterArgs &t, int split, int k0, int c0, int mt, int nt, char *smem)
+{
+    constexpr int XPITCH = SR * SR + 1, YPITCH = TILE * TILE + 1; // of a channel; odd, for the banks
+    float *const xs = (float *)smem, *const ys = xs + 64 * XPITCH;
+    const int tid = threadIdx.x, lane = tid & 63, hi = lane >> 5;
+    float16_t acc[TAPS];
+#pragma unroll
+    for(int tp = 0; tp < TAPS; tp++)
+#pragma unroll
+        for(int v = 0; v < 16; v++)
+            acc[tp][v] = 0.0f;
+    constexpr int XN = 64 * SR * SR / 256, YN = 64 * TILE * TILE / 256;
+    static_assert(XN * 256 == 64 * SR * SR && YN * 256 == 64 * TILE * TILE, "whole rounds");
+    const unsigned xrange = t.x_bytes - (unsigned)(c0 * t.x_sc * 4), yrange = t.y_bytes - (unsigned)(k0 * t.y_sc * 4);
+    struct Tile {
+        int n, ox, oy, dup_cols, dup_rows;
+    };
+    auto place = [&](int tile) {
+        const int n = tile / t.tpi, in = tile - n * t.tpi, ty = in / t.nx, tx = in - ty * t.nx;
+        const int ox = std::min(tx * TILE, t.W - TILE), oy = std::min(ty * TILE, t.H - TILE);
+        return Tile{n, ox, oy, tx * TILE - ox, ty * TILE - oy};
+    };
+    float xr[XN], yr[YN]; // the next tile's
+    auto load = [&](const Tile &p) {
+        const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void *)(t.x + p.n * t.x_sn + c0 * t.x_sc), 0, xrange, 0x00020000);
+        const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc((void *)(t.dy + p.n * t.y_sn + k0 * t.y_sc), 0, yrange, 0x00020000);
+#pragma unroll
+        for(int u = 0; u < XN; u++) {
+            const int i = u * 256 + tid, ch = i / (SR * SR), pos = i - ch * SR * SR, iy = p.oy + pos / SR - 1, ix = p.ox + pos % SR - 1;
+            const bool there = c0 + ch < t.C && (unsigned)iy < (unsigned)t.H && (unsigned)ix < (unsigned)t.W;
+            xr[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                  rx, there ? (unsigned)((ch * t.x_sc + iy * t.x_sh + ix * t.x_sw) * 4) : OOB, 0, 0));
+        }
+#pragma unroll
+        for(int u = 0; u < YN; u++) {
+            const int i = u * 256 + tid, ch = i / (TILE * TILE), pos = i % (TILE * TILE), iy = p.oy + pos / TILE, ix = p.ox + pos % TILE;
+            yr[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                  ry, k0 + ch < t.K ? (unsigned)((ch * t.y_sc + iy * t.y_sh + ix * t.y_sw) * 4) : OOB, 0, 0));
+        }
+    };
+    Tile p = place(split);
+    load(p);
+#pragma unroll 1
+    for(int tile = split; tile < t.ntiles; tile += t.splits) {
+        __syncthreads();
+#pragma unroll
+        for(int u = 0; u < XN; u++)
+            xs[(u * 256 + tid) / (SR * SR) * XPITCH + (u * 256 + tid) % (SR * SR)] = xr[u];
+#pragma unroll
+        for(int u = 0; u < YN; u++)
+            ys[(u * 256 + tid) / (TILE * TILE) * YPITCH + (u * 256 + tid) % (TILE * TILE)] = yr[u];
+        __syncthreads();
+        const int dup_cols = p.dup_cols, dup_rows = p.dup_rows; // that a tile before had: both operands zero
+        p = place(tile + t.splits < t.ntiles ? tile + t.splits : tile);
+        load(p);
+        const float *const xc = xs + (nt * 32 + (lane & 31)) * XPITCH, *const yc = ys + (mt * 32 + (lane & 31)) * YPITCH;
+#pragma unroll 1
+        for(int row = dup_rows; row < TILE; row++)
+#pragma unroll
+            for(int two = 0; two < TILE; two += 2) {
+                const int col = two + hi;
+                const bool own = col >= dup_cols;
+                const float g = own ? yc[row * TILE + col] : 0.0f;
+#pragma unroll
+                for(int tp = 0; tp < TAPS; tp++)
+                    acc[tp] = __builtin_amdgcn_mfma_f32_32x32x2f32(g, own ? xc[(row + tp / 3) * SR + col + tp % 3] : 0.0f, acc[tp], 0, 0, 0);
+            }
+    }
+    store_sums(t, split, k0 + mt * 32 + 4 * hi, c0 + nt * 32 + (lane & 31), acc);
 }
 
 __global__ void __launch_bounds__(256, 1) conv_f32_bwd_filter_windows(WindowFilterArgs t)
@@ -248,7 +339,6 @@ __global__ void __launch_bounds__(256, 1) conv_f32_bwd_filter_windows(WindowFilt
     // (the products of the last instructions are on their way, and the compiler knows only of its own)
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
 
-    const int c = c0 + nt * 32 + (lane & 31), kl = k0 + mt * 32 + 4 * hi; // this lane's elements: channel c, kl + 8 * (v / 4) + v % 4
     float bad = 0.0f;
 #pragma unroll
     for(int tp = 0; tp < TAPS; tp++)
@@ -257,47 +347,15 @@ __global__ void __launch_bounds__(256, 1) conv_f32_bwd_filter_windows(WindowFilt
             acc[tp][v] = (acc[tp][v] + low[tp][v]) * SPLIT_SUM;
             bad = __builtin_fmaf(acc[tp][v], 0.0f, bad);
         }
-    if(__builtin_amdgcn_ballot_w64(bad != bad)) {
-#pragma unroll
-        for(int tp = 0; tp < TAPS; tp++)
-#pragma unroll
-            for(int v = 0; v < 16; v++)
-                acc[tp][v] = 0.0f;
-        for(tile = split; tile < t.ntiles; tile += t.splits) {
-            const int n = tile / t.tpi, in = tile - n * t.tpi, ty = in / t.nx, tx = in - ty * t.nx;
-            const int ox = std::min(tx * TILE, t.W - TILE), oy = std::min(ty * TILE, t.H - TILE);
-            for(int y = ty * TILE; y < oy + TILE; y++)
-                for(int xx = tx * TILE; xx < ox + TILE; xx++) {
-                    float g[16];
-#pragma unroll
-                    for(int v = 0; v < 16; v++) {
-                        const int k = kl + 8 * (v / 4) + v % 4;
-                        g[v] = k < t.K ? t.dy[n * t.y_sn + k * t.y_sc + y * t.y_sh + xx * t.y_sw] : 0.0f;
-                    }
-#pragma unroll
-                    for(int tp = 0; tp < TAPS; tp++) {
-                        const int iy = y + tp / 3 - 1, ix = xx + tp % 3 - 1;
-                        const bool in_image = (unsigned)iy < (unsigned)t.H && (unsigned)ix < (unsigned)t.W && c < t.C;
-                        const float p = in_image ? t.x[n * t.x_sn + c * t.x_sc + iy * t.x_sh + ix * t.x_sw] : 0.0f;
-#pragma unroll
-                        for(int v = 0; v < 16; v++)
-                            acc[tp][v] = __builtin_fmaf(g[v], p, acc[tp][v]);
-                    }
-                }
-        }
-    }
-    // (a share's partial result is one buffer: rows and columns beyond the filter are outside)
-    const unsigned bytes = (unsigned)t.K * (TAPS * 4u) * (unsigned)t.C, krow = TAPS * 4u * (unsigned)t.C;
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc((void *)((char *)t.partial + (int64_t)split * bytes), 0, bytes, 0x00020000);
-    const unsigned first = c < t.C ? (unsigned)kl * krow + (unsigned)c * 4u : OOB;
-#pragma unroll
-    for(int tp = 0; tp < TAPS; tp++)
-#pragma unroll
-        for(int v = 0; v < 16; v++) {
-            const float sum = acc[tp][v]; // (the cast takes a vector's element for its first)
-            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, sum), ro, first + (8 * (v / 4) + v % 4) * krow,
-                                                  tp * t.C * 4, 0);
-        }
+    // (everybody's writes of a tile behind the last are done)
+    volatile int *const found = (volatile int *)smem;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    found[wave] = __builtin_amdgcn_ballot_w64(bad != bad) != 0;
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if(found[0] | found[1] | found[2] | found[3])
+        windows_again(t, split, k0, c0, mt, nt, smem);
+    else
+        store_sums(t, split, k0 + mt * 32 + 4 * hi, c0 + nt * 32 + (lane & 31), acc); // acc[tap][v]: output channel 8 * (v / 4) + v % 4 of a half's
 }
 
 // bytes of one image, or 0
