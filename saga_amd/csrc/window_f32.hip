@@ -17,6 +17,8 @@
 // 3x3 256->256 at 8x14x14 28 -> 17, of which the matrix instructions take 5: the launch 3, finding the window and the first
 // slice 2, the filter from the L2 (4 KB per 16 channels and 32 pixels x 32 channels) most of the rest.  1x1 256->1024 at 8x14x14 16.5 ->
 // 10.6: trips to memory, four slices one behind the other.
+// Operands without three parts cost the wavefronts that meet them their share again in fp32 products, loaded without staging: 3x3 64->64 at
+// 256x56x56 in 360 us, 320 with one NaN in x and 1030 with nothing else (the kernel for fp32 products 520).
 #include "split_f32.hpp"
 #include "out_f32.hpp"
 #include "window_f32.hpp"
@@ -433,10 +435,11 @@ Plan tiles_for(const WinArgs &g, int Tr, int kg)
     // (images of longer rows on small grids: the windows are several times the pixels)
     if(taps > 1 && g.IW > 128 && tiles(2) < 3000)
         return {};
-    // 25 taps: four wavefronts next to each other along the pixels share what they load (us, the rules below / this: 32->64 64x14x14
-    // 14.7 / 12.9, 200x14x14 31.9 / 29.2, 512x14x14 60.0 / 60.6, 64->64 32x28x28 32.7 / 32.1, 56->136 45x35x35 149 / 132; with one column
-    // of tiles, 16->32 16x56x56, 14.2 / 15.4)
-    if(taps == 25 && g.istep == 1 && columns > 1 && tiles(1) >= 750) {
+    // 25 taps: four wavefronts next to each other along the pixels share what they load, from 140 blocks of them on; fewer do better
+    // with the reduction split (us, the rules below / this: 32->64 at 14x14, 32 images (392 tiles) 10.3 / 12.0, 40 (490) 11.2 / 12.0, 48
+    // (588) 13.4 / 12.1, 64 (784) 14.7 / 12.5, 128 (1568) 20.5 / 20.4; 128->192 3x30x30 (510) 23 / 32, 64->96 5x35x35 (576) 19.6 / 18.2,
+    // 160->88 20x19x19 (678) 40 / 36, 144->88 174x7x7 (801) 76 / 36; with one column of tiles, 16->32 16x56x56, 14.2 / 15.4)
+    if(taps == 25 && g.istep == 1 && columns > 1 && tiles(1) >= 560) {
         const Plan p = fit(g, Tr, kg, {1, 1, 4, 1, 1});
         if(p.quads)
             return p;

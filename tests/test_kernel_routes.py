@@ -256,3 +256,11 @@ def test_fp32_routes():
         launches = convolution(kind, shape, K.FLOAT, room=room)[0]
         (ran,) = [x for x in launches if "pack" not in x[0] and "build" not in x[0]]
         assert ran[0] == kernel and reads in (None, ran[1][1]), (shape, kind, room, ran)
+
+
+@on_stub
+def test_fp32_windows_of_25_taps():
+    """Blocks of four wavefronts along the pixels from 560 tiles on; fewer share the reduction."""
+    for images, four in ((32, False), (45, False), (46, True), (64, True)):
+        _, (name, _, blocks, _) = convolution(K.CONV_FWD, (images, 32, 14, 14, 64, 5, 1, 2), K.FLOAT)[0]
+        assert name == "stream_f32_k_window" and (blocks == -(-images * 196 // 128) * 2) == four, (images, blocks)
