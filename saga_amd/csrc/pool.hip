@@ -108,15 +108,15 @@ __device__ __forceinline__ void decode(int64_t i, int C, int H, int W, int &n, i
 __device__ __forceinline__ bool better(float v, float best) { return !(v <= best) && best == best; }
 __device__ __forceinline__ bool same(float a, float b) { return a == b || (a != a && b != b); }
 
-template <typename T, int VN, int MODE>
+template <typename T, int VN, int MODE, typename I>
 __global__ void __launch_bounds__(256)
-    pool_fwd_k(DView x, DView y, DView idx, int has_idx, int k, int pad, int stride, int relu, int64_t total)
+    pool_fwd_k(DView x, DView y, DView idx, int has_idx, int k, int pad, int stride, int relu, I total)
 {
     const int C = y.d[1], P = y.d[2], Q = y.d[3], H = x.d[2], W = x.d[3];
     const float inv = 1.0f / (float)(k * k);
-    for(int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
+    for(I i = (I)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (I)gridDim.x * blockDim.x) {
         int n, c, p, q;
-        decode<VN>(i, C, P, Q, n, c, p, q);
+        decode_as<VN>(i, C, P, Q, n, c, p, q);
         float acc[VN];
         int best[VN];
         bool first = true; // the first in-bounds position seeds the maximum for every channel
@@ -1188,6 +1188,9 @@ static int pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y, 
             pool_max_k<T, VN, 2><<<g, 256, 0, st>>>(dvx, dvy, dvi, idx != nullptr, pad, stride, relu, (int)total); \
         else if(mode == SAGA_POOL_MAX && size == 3 && small)                                             \
             pool_max_k<T, VN, 3><<<g, 256, 0, st>>>(dvx, dvy, dvi, idx != nullptr, pad, stride, relu, (int)total); \
+        else if(mode == SAGA_POOL_MAX && small)                                                          \
+            pool_fwd_k<T, VN, SAGA_POOL_MAX><<<g, 256, 0, st>>>(dvx, dvy, dvi, idx != nullptr, size, pad, \
+                                                                stride, relu, (unsigned)total);          \
         else if(mode == SAGA_POOL_MAX)                                                                   \
             pool_fwd_k<T, VN, SAGA_POOL_MAX><<<g, 256, 0, st>>>(dvx, dvy, dvi, idx != nullptr, size, pad, \
                                                                 stride, relu, total);                    \
@@ -1196,6 +1199,8 @@ static int pool_fwd(int mode, const SagaTensorView *x, const SagaTensorView *y, 
         else if(lanes)                                                                                   \
             avgpool_fwd_split_k<T, VN, 256><<<(int)((total * lanes + 255) / 256), 256, 0, st>>>(dvx, dvy, size, pad, stride, \
                                                                                                 lanes, total); \
+        else if(small)                                                                                   \
+            pool_fwd_k<T, VN, SAGA_POOL_AVG><<<g, 256, 0, st>>>(dvx, dvy, dvi, 0, size, pad, stride, relu, (unsigned)total); \
         else                                                                                             \
             pool_fwd_k<T, VN, SAGA_POOL_AVG><<<g, 256, 0, st>>>(dvx, dvy, dvi, 0, size, pad, stride, relu, total); \
     } while(0)
