@@ -188,7 +188,7 @@ __global__ void __launch_bounds__(256, 1) conv_f32_bwd_filter_windows(WindowFilt
             cols |= col < dup_cols ? 1u << u : 0u;
             rows |= r < dup_rows ? 1u << u : 0u;
         }
-        // (lanes of x without a position write where another part will be: behind the last, that is, nowhere)
+        // (lanes of x without a position write nothing)
         slot[u] = g < 8 ? (unsigned)((is_x ? 0 : 3 * XPART) + pos * 128 + ((g ^ chunk_swizzle(col)) << 4)) : 0xffffffffu;
     }
     struct Tile {

@@ -1,7 +1,7 @@
 // fp32 convolutions on the bf16 matrix unit (split_f32.hpp), each image position read and split once per slice of channels and
 // not once per tap.
 //
-// A block owns 32*TM*WM output pixels, consecutive in (sample, row, column), and 32*TN*WN output channels; KS groups of WM x WN
+// A block owns 32*TM*WM output pixels, consecutive in (sample, row, column), and 32*WN output channels; KS groups of WM x WN
 // wavefronts share the reduction.  What the pixels see of the input under any tap is consecutive in (sample, position) too:
 // the window.  For every slice of 8*KG channels a group loads its window in fours of positions, splits it into three parts,
 // eight channels to 16 bytes, and leaves it in LDS, where every tap is an offset; the filter comes packed, in the order of the
@@ -53,8 +53,8 @@ __host__ __device__ constexpr int window_pitch(int quads) { return quads + ((4 -
 constexpr int window_bytes(int quads, int kg) { return 3 * kg * 4 * window_pitch(quads) * 16; }
 
 // APART: one tap at a stride; the window is the positions of the block's pixels and nothing between them, loaded one by one.
-template <int TM, int TN, int DEPTH, int KG, int NR, int TAPS, bool APART, bool EX>
-__global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinArgs g)
+template <int TM, int DEPTH, int KG, int NR, int TAPS, bool APART, bool EX>
+__global__ void __launch_bounds__(512) stream_f32_k_window(WinArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ __attribute__((aligned(16))) float chan[2][EX ? 256 : 1]; // scale and shift of the block's channels
@@ -74,7 +74,7 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
     const int nb = g.blocks, per = nb >> 3, rem = nb & 7, xcd = blockIdx.x & 7;
     const int b = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (blockIdx.x >> 3);
     const int bm = g.blk.div(b), bq = b - bm * g.nblk_q;
-    const int m0 = bm * (32 * TM * WM), n0 = bq * (32 * TN * WN), nw = n0 + 32 * TN * wn;
+    const int m0 = bm * (32 * TM * WM), n0 = bq * (32 * WN), nw = n0 + 32 * wn;
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)g.p, 0, (int)g.p_bytes, 0x00020000);
     const __amdgpu_buffer_rsrc_t rq = __builtin_amdgcn_make_buffer_rsrc((void *)g.q, 0, (int)g.q_bytes, 0x00020000);
 
@@ -82,19 +82,14 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
     const int S16 = (g.C + 15) / 16, total = (S16 + KG / 2 - 1) / (KG / 2), rounds = (total + KS - 1) / KS, s0 = ks * rounds;
     constexpr int STEPS = TAPS * (KG / 2);
     static_assert(STEPS % DEPTH == 0, "the ring goes round in every slice");
-    float4_t qr[DEPTH][TN][3];
-    unsigned qoff[TN];
-#pragma unroll
-    for(int t = 0; t < TN; t++)
-        qoff[t] = nw + 32 * t < g.o.N ? (unsigned)(nw / 32 + t) * (unsigned)(g.T * S16 * 3072) + lane * 16 : OOB;
+    float4_t qr[DEPTH][3];
+    const unsigned qoff = nw < g.o.N ? (unsigned)(nw / 32) * (unsigned)(g.T * S16 * 3072) + lane * 16 : OOB;
     auto load_q = [&](int slice, int k) {
         const int st = slice * (KG / 2) + k % (KG / 2);
         const unsigned off = (unsigned)(k % STEPS / (KG / 2) * S16 + (st < S16 ? st : S16 - 1)) * 3072u; // (the window holds zeros there)
 #pragma unroll
-        for(int t = 0; t < TN; t++)
-#pragma unroll
-            for(int h = 0; h < 3; h++)
-                qr[k % DEPTH][t][h] = load4(rq, qoff[t] + 1024 * h, off);
+        for(int h = 0; h < 3; h++)
+            qr[k % DEPTH][h] = load4(rq, qoff + 1024 * h, off);
     };
 #pragma unroll
     for(int k = 0; k < DEPTH; k++)
@@ -180,7 +175,7 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
         load_x(r, s0);
 
     EpilogueF32::Raw raw;
-    if(EX && g.o.e.affine() && tid < 32 * TN * WN)
+    if(EX && g.o.e.affine() && tid < 32 * WN)
         raw = g.o.e.fetch(n0 + tid < g.o.N ? n0 + tid : g.o.N - 1);
 
     // this lane's pixels: where they are in the window under the first tap, and one bit per tap that falls inside the image
@@ -204,14 +199,12 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
     for(int k = lane + 64 * wg; k < 6 * KG; k += 64 * GW)
         *(float4_t *)(win + (k * 4 * pitch + zero) * 16) = float4_t{0, 0, 0, 0};
 
-    float16_t acc[TM][TN], low[TM][TN]; // the products of the leading parts, and all others (split_f32.hpp)
+    float16_t acc[TM], low[TM]; // the products of the leading parts, and all others (split_f32.hpp)
 #pragma unroll
     for(int i = 0; i < TM; i++)
 #pragma unroll
-        for(int t = 0; t < TN; t++)
-#pragma unroll
-            for(int v = 0; v < 16; v++)
-                acc[i][t][v] = low[i][t][v] = 0.0f;
+        for(int v = 0; v < 16; v++)
+            acc[i][v] = low[i][v] = 0.0f;
 
     auto meet = [&]() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
 #pragma unroll
@@ -249,9 +242,7 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
             for(int j = 0; j < SPLIT_PRODUCTS; j++)
 #pragma unroll
                 for(int i = 0; i < TM; i++)
-#pragma unroll
-                    for(int t = 0; t < TN; t++)
-                        mfma_split(j, pp[k & 1][i], qr[k % DEPTH][t], acc[i][t], low[i][t]);
+                    mfma_split(j, pp[k & 1][i], qr[k % DEPTH], acc[i], low[i]);
             load_q(k + DEPTH < STEPS ? slice : slice + 1, k + DEPTH);
 #pragma unroll
             for(int u = k * EACH * NR / STEPS; u < (k + 1) * EACH * NR / STEPS; u++) {
@@ -268,22 +259,18 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
 #pragma unroll
     for(int i = 0; i < TM; i++)
 #pragma unroll
-        for(int t = 0; t < TN; t++)
-#pragma unroll
-            for(int v = 0; v < 16; v++) {
-                acc[i][t][v] = (acc[i][t][v] + low[i][t][v]) * SPLIT_SUM;
-                bad = __builtin_fmaf(acc[i][t][v], 0.0f, bad);
-            }
+        for(int v = 0; v < 16; v++) {
+            acc[i][v] = (acc[i][v] + low[i][v]) * SPLIT_SUM;
+            bad = __builtin_fmaf(acc[i][v], 0.0f, bad);
+        }
     if(__builtin_amdgcn_ballot_w64(bad != bad)) {
         // An infinity, a NaN or a number next to the largest among the operands has no three parts: this wavefront's share
         // once more, in fp32 products.
 #pragma unroll
         for(int i = 0; i < TM; i++)
 #pragma unroll
-            for(int t = 0; t < TN; t++)
-#pragma unroll
-                for(int v = 0; v < 16; v++)
-                    acc[i][t][v] = 0.0f;
+            for(int v = 0; v < 16; v++)
+                acc[i][v] = 0.0f;
         const int first = s0 * (KG / 2), behind = first + rounds * (KG / 2) < S16 ? first + rounds * (KG / 2) : S16;
         for(int st = first; st < behind; st++)
             for(int tp = 0; tp < TAPS; tp++) {
@@ -297,22 +284,19 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
                     for(int j = 0; j < 8; j++)
                         a[i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rp, v, (unsigned)(st * 16 + j) * psc4, 0));
                 }
+                float4_t q[3];
 #pragma unroll
-                for(int t = 0; t < TN; t++) {
-                    float4_t q[3];
+                for(int h = 0; h < 3; h++)
+                    q[h] = load4(rq, qoff + 1024 * h, (unsigned)(tp * S16 + st) * 3072u);
 #pragma unroll
-                    for(int h = 0; h < 3; h++)
-                        q[h] = load4(rq, qoff[t] + 1024 * h, (unsigned)(tp * S16 + st) * 3072u);
+                for(int j = 0; j < 8; j++)
 #pragma unroll
-                    for(int j = 0; j < 8; j++)
-#pragma unroll
-                        for(int i = 0; i < TM; i++)
-                            acc[i][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(q, j), a[i][j], acc[i][t], 0, 0, 0);
-                }
+                    for(int i = 0; i < TM; i++)
+                        acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(joined(q, j), a[i][j], acc[i], 0, 0, 0);
             }
     }
 
-    // acc[i][t][v]: this lane's pixel i, channel nw + 32*t + 8*(v/4) + 4*(lane/32) + v%4
+    // acc[i][v]: this lane's pixel i, channel nw + 8*(v/4) + 4*(lane/32) + v%4
     const FourOut<EX> out(g.o, fk);
     unsigned opos[TM], zpos[TM];
 #pragma unroll
@@ -320,30 +304,28 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
         opos[i] = out.out_at(ok[i], pn[i], py[i], px[i]);
         zpos[i] = out.z_at(ok[i], pn[i], py[i], px[i]);
     }
-    if(EX && g.o.e.affine() && tid < 32 * TN * WN)
+    if(EX && g.o.e.affine() && tid < 32 * WN)
         g.o.e.leave(raw, chan[0][tid], chan[1][tid]);
-    auto channel = [&](int t, int v) { return nw + 32 * t + 8 * v; };
+    auto channel = [&](int v) { return nw + 8 * v; };
     auto store = [&](unsigned pos, int n, const Four &val, const Four &was, const Four &res) {
         out.store(pos, n, val, was, res, &chan[0][EX ? n - n0 + 4 * fk : 0], &chan[1][EX ? n - n0 + 4 * fk : 0]);
     };
-    constexpr int NV = TM * TN * 16;
+    constexpr int NV = TM * 16;
     if(KS == 1) {
         if(EX && g.o.e.affine())
             __syncthreads();
 #pragma unroll
-        for(int i = 0; i < TM; i++)
+        for(int i = 0; i < TM; i++) {
+            Four before[4], res[4];
 #pragma unroll
-            for(int t = 0; t < TN; t++) {
-                Four before[4], res[4];
-#pragma unroll
-                for(int v = 0; v < 4; v++) {
-                    before[v] = out.before(opos[i], channel(t, v));
-                    res[v] = out.residual(zpos[i], channel(t, v));
-                }
-#pragma unroll
-                for(int v = 0; v < 4; v++)
-                    store(opos[i], channel(t, v), {acc[i][t][4 * v], acc[i][t][4 * v + 1], acc[i][t][4 * v + 2], acc[i][t][4 * v + 3]}, before[v], res[v]);
+            for(int v = 0; v < 4; v++) {
+                before[v] = out.before(opos[i], channel(v));
+                res[v] = out.residual(zpos[i], channel(v));
             }
+#pragma unroll
+            for(int v = 0; v < 4; v++)
+                store(opos[i], channel(v), {acc[i][4 * v], acc[i][4 * v + 1], acc[i][4 * v + 2], acc[i][4 * v + 3]}, before[v], res[v]);
+        }
         return;
     }
     // the groups' sums meet in LDS; each wavefront finishes its share of the fours
@@ -351,28 +333,25 @@ __global__ void __launch_bounds__(TN == 2 ? 256 : 512) stream_f32_k_window(WinAr
 #pragma unroll
     for(int i = 0; i < TM; i++)
 #pragma unroll
-        for(int t = 0; t < TN; t++)
-#pragma unroll
-            for(int v = 0; v < 4; v++)
-                red[(wave * (NV / 4) + (i * TN + t) * 4 + v) * 64 + lane] =
-                    float4_t{acc[i][t][4 * v], acc[i][t][4 * v + 1], acc[i][t][4 * v + 2], acc[i][t][4 * v + 3]};
+        for(int v = 0; v < 4; v++)
+            red[(wave * (NV / 4) + i * 4 + v) * 64 + lane] = float4_t{acc[i][4 * v], acc[i][4 * v + 1], acc[i][4 * v + 2], acc[i][4 * v + 3]};
     __syncthreads();
 #pragma unroll
     for(int f = 0; f < NV / 4; f++) {
         if((f & (KS - 1)) != ks)
             continue;
-        const int i = f / (4 * TN), t = f / 4 % TN, v = f % 4;
-        const Four before = out.before(opos[i], channel(t, v)), res = out.residual(zpos[i], channel(t, v));
+        const int i = f / 4, v = f % 4;
+        const Four before = out.before(opos[i], channel(v)), res = out.residual(zpos[i], channel(v));
         float4_t sum = {0, 0, 0, 0};
         for(int k = 0; k < KS; k++)
             sum += red[((k * GW + wg) * (NV / 4) + f) * 64 + lane];
-        store(opos[i], channel(t, v), {sum[0], sum[1], sum[2], sum[3]}, before, res);
+        store(opos[i], channel(v), {sum[0], sum[1], sum[2], sum[3]}, before, res);
     }
 }
 
-// Tile of a wavefront in 32s, wavefronts of a group along the pixels and the channels, groups along the reduction.
+// Pixels of a wavefront in 32s (of channels it has 32), wavefronts of a group along the pixels and the channels, groups along the reduction.
 struct Config {
-    int tm, tn, wm, wn, ks;
+    int tm, wm, wn, ks;
 };
 
 constexpr int MAX_LDS = 160 * 1024 - 2048 - 512;
@@ -411,13 +390,13 @@ Plan fit(const WinArgs &g, int Tr, int kg, const Config &cf)
     Plan p = {cf, window_quads(g, Tr, 32 * cf.tm * cf.wm), 0, 0};
     const bool apart = g.T == 1 && g.istep > 1;
     p.nr = ((apart ? 32 * cf.tm * cf.wm : p.quads - 1) + at_once - 1) / at_once;
-    p.lds = std::max((size_t)cf.ks * 2 * window_bytes(p.quads, kg), cf.ks > 1 ? (size_t)cf.ks * waves * cf.tm * cf.tn * 4096 : 0);
+    p.lds = std::max((size_t)cf.ks * 2 * window_bytes(p.quads, kg), cf.ks > 1 ? (size_t)cf.ks * waves * cf.tm * 4096 : 0);
     if(p.nr > (apart ? 4 : 2) || p.lds > MAX_LDS)
         p.quads = 0;
     return p;
 }
 
-// What was measured on small grids (us; tm, wm, wn, ks; tn 1; launch included, packing not):
+// What was measured on small grids (us; tm, wm, wn, ks; launch included, packing not):
 //   3x3  64->64   8x56x56  2,2,2,1 15.2  2,2,2,2 15.5  1,2,2,1 16.1  2,1,2,1 16.7   1x1  64->64   8x56x56  1,1,2,1  6.7  2,2,2,1  7.4
 //   3x3 128->128  8x28x28  2,1,2,4 15.4  1,1,2,2 16.3  2,1,2,2 16.4  2,1,1,4 20.4   1x1  64->256  8x56x56  2,1,8,1 15.1  2,1,4,1 15.5
 //   3x3 256->256  8x14x14  1,1,2,4 17.0  2,1,1,4 17.5  1,1,1,4 17.7  2,1,2,4 23.2   1x1 256->64   8x56x56  1,1,2,1 11.6  2,2,2,1 12.4
@@ -440,7 +419,7 @@ Plan tiles_for(const WinArgs &g, int Tr, int kg)
     // (588) 13.4 / 12.1, 64 (784) 14.7 / 12.5, 128 (1568) 20.5 / 20.4; 128->192 3x30x30 (510) 23 / 32, 64->96 5x35x35 (576) 19.6 / 18.2,
     // 160->88 20x19x19 (678) 40 / 36, 144->88 174x7x7 (801) 76 / 36; with one column of tiles, 16->32 16x56x56, 14.2 / 15.4)
     if(taps == 25 && g.istep == 1 && columns > 1 && tiles(1) >= 560) {
-        const Plan p = fit(g, Tr, kg, {1, 1, 4, 1, 1});
+        const Plan p = fit(g, Tr, kg, {1, 4, 1, 1});
         if(p.quads)
             return p;
     }
@@ -468,7 +447,7 @@ Plan tiles_for(const WinArgs &g, int Tr, int kg)
             while(taps > 1 && 2 * wm * wn * k <= most && bm * ((columns + wn - 1) / wn) >= 2 * wm * 190)
                 wm *= 2;
             for(; wm; wm /= 2) {
-                const Plan p = fit(g, Tr, kg, {tm, 1, wm, wn, k});
+                const Plan p = fit(g, Tr, kg, {tm, wm, wn, k});
                 if(p.quads)
                     return p;
             }
@@ -551,9 +530,9 @@ int slice_groups(int taps) { return taps == 1 ? 8 : 2; } // eights of channels; 
 
 template <int KG, int TAPS, int DEPTH, bool APART, bool EX> int launch_as(const WinArgs &g, const Plan &p, hipStream_t st)
 {
-#define GO(TM, TN, NR)                                                                                                     \
+#define GO(TM, NR)                                                                                                         \
     do {                                                                                                               \
-        auto kern = stream_f32_k_window<TM, TN, DEPTH, KG, NR, TAPS, APART, EX>;                                              \
+        auto kern = stream_f32_k_window<TM, DEPTH, KG, NR, TAPS, APART, EX>;                                                  \
         static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS); \
         if(attr != hipSuccess)                                                                                         \
             return (int)attr;                                                                                          \
@@ -562,20 +541,20 @@ template <int KG, int TAPS, int DEPTH, bool APART, bool EX> int launch_as(const 
     if constexpr(APART)
         if(p.nr > 2) { // (a block of one or two wavefronts)
             if(p.cf.tm == 1)
-                GO(1, 1, 4);
+                GO(1, 4);
             else
-                GO(2, 1, 4);
+                GO(2, 4);
             SAGA_CHECK_LAUNCH();
             return 0;
         }
     if(p.cf.tm == 1 && p.nr == 1)
-        GO(1, 1, 1);
+        GO(1, 1);
     else if(p.cf.tm == 1)
-        GO(1, 1, 2);
+        GO(1, 2);
     else if(p.nr == 1)
-        GO(2, 1, 1);
+        GO(2, 1);
     else
-        GO(2, 1, 2);
+        GO(2, 2);
 #undef GO
     SAGA_CHECK_LAUNCH();
     return 0;
@@ -600,7 +579,7 @@ bool window_f32_may(const WindowConv &c, int channels, int IH, int IW, int OH, i
     g.ow = fast_div(OW);
     g.oh = fast_div(OH);
     for(int wn = 1; wn <= 8; wn *= 2) // (the smallest tile; with more wavefronts to load its window)
-        if(fit(g, c.Tr, slice_groups(g.T), {1, 1, 1, wn, 1}).quads || fit(g, c.Tr, slice_groups(g.T), {1, 1, wn, 1, 1}).quads)
+        if(fit(g, c.Tr, slice_groups(g.T), {1, 1, wn, 1}).quads || fit(g, c.Tr, slice_groups(g.T), {1, wn, 1, 1}).quads)
             return true;
     return false;
 }
@@ -627,7 +606,7 @@ int window_f32_conv(const WindowConv &c, const SagaTensorView *a, const SagaTens
     g.WM = p.cf.wm;
     g.WN = p.cf.wn;
     g.KS = p.cf.ks;
-    g.nblk_q = (g.o.N + 32 * p.cf.tn * p.cf.wn - 1) / (32 * p.cf.tn * p.cf.wn);
+    g.nblk_q = (g.o.N + 32 * p.cf.wn - 1) / (32 * p.cf.wn);
     g.blk = fast_div(g.nblk_q);
     const long long blocks = (g.M + tile - 1) / tile * g.nblk_q;
     if(blocks >= 1ll << 31)

@@ -62,7 +62,7 @@ def test_shapes_are_what_they_are_said_to_be():
         stub_gpu.launched()
         run(K.CONV_FWD, shape, 1 << 20, 1 << 33, 1 << 34, 1 << 35)
         ((name, tile, blocks, threads),) = stub_gpu.launched()
-        assert name == "stream_f32_k_window" and (tile[0], tile[4], tile[5], threads) == (tm, rounds, taps, 64 * waves), (shape, tile, threads)
+        assert name == "stream_f32_k_window" and (tile[0], tile[3], tile[4], threads) == (tm, rounds, taps, 64 * waves), (shape, tile, threads)
 
 
 @on_stub
