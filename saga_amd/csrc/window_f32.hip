@@ -423,11 +423,13 @@ Plan tiles_for(const WinArgs &g, int Tr, int kg)
         if(p.quads)
             return p;
     }
+    // (25 taps on 64 pixels take more registers than there are; us, 64 / 32: 16->72 82x18x18 backward 60 / 26, 344->16 3x91x91 155 / 81,
+    // 96->16 16x96x96 210 / 150, 16->16 75x98x98 179 / 203)
     const long long one = taps == 1 ? 1500 : 750;
     int tm = 1, ks = 1;
-    if(tiles(2) >= one && (g.istep == 1 || taps == 1))
+    if(taps != 25 && tiles(2) >= one && (g.istep == 1 || taps == 1))
         tm = 2;
-    else if(taps > 1 && tiles(2) >= one / 2 && g.istep == 1)
+    else if(taps > 1 && taps != 25 && tiles(2) >= one / 2 && g.istep == 1)
         tm = 2, ks = 4;
     else
         while(ks < 8 && tiles(1) * ks < (taps == 1 ? 1500 : 800))
@@ -459,13 +461,13 @@ Plan tiles_for(const WinArgs &g, int Tr, int kg)
 //   1x1 over many pixels, with a slice of 64 channels or a tile of 64 results that is not full: 16->56 70x111x111 61 / 162, 88->16
 //   247x66x66 96 / 210, 24->456 45x68x68 156 / 184, 64->352 109x24x24 48 / 55 (128->256 123x49x49 228 / 193);
 //   blocks of two wavefronts that take a CU's LDS, or under 25 taps: 3x3 at stride 2, 40->64 103x13x13 13 / 21, 472->16 41x13x13
-//   30 / 41, 3x3 336->16 1x107x107 36 / 59, 5x5 32->16 5x86x86 31 / 56, 40->136 3x24x24 19 / 24;
+//   30 / 41, 3x3 336->16 1x107x107 36 / 59, 5x5 40->136 3x24x24 19 / 24;
 //   few slices over four or eight groups, half of which has one to do less: 3x3 72->152 17x16x16 20 / 30, 72->16 29x37x37 25 / 39;
 //   few slices for each of four groups, or one tile, and a last round of blocks that is nearly empty: 3x3 72->128 3x54x54 26 / 32,
 //   160->64 2x53x53 22 / 28; of one tile and a large window, over half of the CUs: 104->24 1x70x70 12.5 / 14;
 //   one step of channels at stride 2, where a window is four times what its pixels see, and two over many pixels: 3x3 16->296
 //   141x48x48 98 / 135, 24->392 61x55x55 122 / 154.
-// Of 553 layers under 9 and 25 taps these rules leave 483 to windows, 14 of them (58 before) slower by more than 4 %.
+// Of 553 layers under 9 and 25 taps these rules leave 486 to windows, 8 of them (58 without the rules) slower by more than 4 %, one by more than 8.
 bool worth(const WinArgs &g, const Plan &p)
 {
     const Config &c = p.cf;
@@ -547,7 +549,12 @@ template <int KG, int TAPS, int DEPTH, bool APART, bool EX> int launch_as(const 
             SAGA_CHECK_LAUNCH();
             return 0;
         }
-    if(p.cf.tm == 1 && p.nr == 1)
+    if constexpr(TAPS == 25) {
+        if(p.nr == 1)
+            GO(1, 1);
+        else
+            GO(1, 2);
+    } else if(p.cf.tm == 1 && p.nr == 1)
         GO(1, 1);
     else if(p.cf.tm == 1)
         GO(1, 2);
