@@ -1165,7 +1165,8 @@ static int gather_launch(bool bwd, const SagaTensorView *a, const SagaTensorView
 size_t conv_f32_packed_bytes(int kind, const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g)
 {
     const bool bwd = kind == SAGA_CONV_BWD_DATA;
-    return f32_ok(x, w, y, g) && !tiles_in_lds(bwd, bwd ? y : x, bwd ? x : y, g, true, 0) ? stream_f32_packed_bytes(bwd, g) : 0;
+    const SagaTensorView *a = bwd ? y : x, *out = bwd ? x : y;
+    return f32_ok(x, w, y, g) && !tiles_in_lds(bwd, a, out, g, true, 0) ? stream_f32_packed_bytes(bwd, a, w, out, g) : 0;
 }
 
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,

@@ -775,12 +775,18 @@ int pack_jobs(const Args &k, const void *w, char *packed, bool parts, SagaFilter
 
 int stream_pack_blocks(const SagaFilterPackJob &j) { return (int)((pack_chunks(j) + PACK_CHUNKS - 1) / PACK_CHUNKS); }
 
-size_t stream_f32_packed_bytes(bool bwd, const ConvGeom &g)
+size_t stream_f32_packed_bytes(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g)
 {
     Args k = {};
     if((bwd ? g.K : g.C) % 8 || g.group != 1 || !classes(bwd, g, k))
         return 0;
-    return packed_size(bwd, g, k, for_windows(bwd, g, k));
+    const bool parts = for_windows(bwd, g, k);
+    // Windows are not the faster one here, and the filter as it is serves many pixels as well as a packed one (us, that / three parts:
+    // 64->352 109x24x24 44 / 58, 48->120 100x40x40 33 / 46; of few pixels, 2048->512 4x7x7, 19.8 / 16.5)
+    const long long pixels = (long long)out->dims[0] * out->dims[2] * out->dims[3];
+    if(parts && in_place(bwd, g) && w->strides[1] == 1 && pixels >= 4096 && !stream_f32_windows(bwd, a, out, g, true, 0))
+        return 0;
+    return packed_size(bwd, g, k, parts);
 }
 
 int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob *jobs)

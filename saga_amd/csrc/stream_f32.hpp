@@ -58,7 +58,7 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
 // whether a convolution is done in windows (window_f32.hip), of a filter packed beforehand or with that much workspace to pack it
 bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room);
 // the filter in the order that the kernel loads it: bytes (0: not for this convolution), jobs (at most 16), launch
-size_t stream_f32_packed_bytes(bool bwd, const ConvGeom &g);
+size_t stream_f32_packed_bytes(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g);
 int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob *jobs);
 int stream_pack_blocks(const SagaFilterPackJob &j); // of stream_f32_pack
 int stream_f32_pack(const SagaFilterPackJob *jobs, int njobs, int blocks, hipStream_t st);

@@ -458,8 +458,9 @@ Plan tiles_for(const WinArgs &g, int Tr, int kg)
 }
 
 // Where operands straight from memory (stream_f32.hip) are faster after all (us, those / windows):
-//   1x1 over many pixels, with a slice of 64 channels or a tile of 64 results that is not full: 16->56 70x111x111 61 / 162, 88->16
-//   247x66x66 96 / 210, 24->456 45x68x68 156 / 184, 64->352 109x24x24 48 / 55 (128->256 123x49x49 228 / 193);
+//   1x1 over many pixels and few results, 88->16 247x66x66 95 / 201, 96->24 12x40x40 6.4 / 9.3 (4x40x40 6.2 / 5.3), 256->64 96x56x56
+//   111 / 120 (64x56x56 79 / 73), sooner with one slice of channels, 64->64 32x56x56 18 / 22 (24x56x56 17.3 / 16.8); and with a slice
+//   of 64 that is not nearly full (window_f32_may), 16->40 217x62x62 48 / 128, 24->144 12x40x40 8.7 / 13.3, 32->192 12x28x28 7.1 / 10.5;
 //   blocks of two wavefronts that take a CU's LDS, or under 25 taps: 3x3 at stride 2, 40->64 103x13x13 13 / 21, 472->16 41x13x13
 //   30 / 41, 3x3 336->16 1x107x107 36 / 59, 5x5 40->136 3x24x24 19 / 24;
 //   few slices over four or eight groups, half of which has one to do less: 3x3 72->152 17x16x16 20 / 30, 72->16 29x37x37 25 / 39;
@@ -472,7 +473,7 @@ bool worth(const WinArgs &g, const Plan &p)
 {
     const Config &c = p.cf;
     if(g.T == 1)
-        return (long long)g.M * g.o.N < 1ll << 24 || (g.C > 64 && g.o.N > 64);
+        return g.o.N > 64 || (g.o.N <= 32 ? g.M < 10000 : (long long)g.M * g.o.N < (g.C <= 64 ? 3ll << 21 : 1ll << 24));
     const int waves = c.wm * c.wn * c.ks, slices = (g.C + 15) / 16;
     const long long blocks = (long long)((g.M + 32 * c.tm * c.wm - 1) / (32 * c.tm * c.wm)) * ((g.o.N + 32 * c.wn - 1) / (32 * c.wn));
     if(g.T == 9 && g.istep > 1 && g.C <= (blocks > 2048 ? 32 : 16))
@@ -573,7 +574,7 @@ bool window_f32_may(const WindowConv &c, int channels, int IH, int IW, int OH, i
 {
     WinArgs g = {};
     g.T = c.Tr * c.Ts;
-    if((g.T != 1 && g.T != 9 && g.T != 25) || channels % 8 || channels < 16 || (long long)IH * IW >= 1ll << 30)
+    if((g.T != 1 && g.T != 9 && g.T != 25) || channels % 8 || channels < (g.T == 1 ? 48 : 16) || (long long)IH * IW >= 1ll << 30)
         return false;
     g.Ts = c.Ts;
     g.IH = IH;

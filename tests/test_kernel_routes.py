@@ -230,7 +230,8 @@ F32_ROUTES = [
     ((217, 16, 62, 62, 40, 1, 1, 0), K.CONV_FWD, 1.0, "stream_f32_k", 0),
     ((205, 56, 59, 59, 48, 1, 1, 0), K.CONV_FWD, 1.0, "stream_f32_k", 0),
     ((84, 64, 56, 56, 56, 1, 1, 0), K.CONV_FWD, 1.0, "conv_f32_gather_uniform", None),
-    ((109, 64, 62, 62, 352, 1, 1, 0), K.CONV_FWD, 1.0, "conv_f32_gather_uniform", None),
+    ((60, 40, 60, 60, 200, 1, 1, 0), K.CONV_FWD, 1.0, "conv_f32_gather_uniform", None),
+    ((109, 64, 62, 62, 352, 1, 1, 0), K.CONV_FWD, 1.0, "stream_f32_k_window", None),
     # no room for three parts, but for the filter as it is; not for that either
     ((8, 512, 14, 14, 512, 3, 1, 1), K.CONV_FWD, 1.0, "stream_f32_k_window", None),
     ((8, 512, 14, 14, 512, 3, 1, 1), K.CONV_FWD, 4 * 9 * 512 * 512, "stream_f32_k", 3),
@@ -264,3 +265,18 @@ def test_fp32_windows_of_25_taps():
     for images, four in ((32, False), (45, False), (46, True), (64, True)):
         _, (name, _, blocks, _) = convolution(K.CONV_FWD, (images, 32, 14, 14, 64, 5, 1, 2), K.FLOAT)[0]
         assert name == "stream_f32_k_window" and (blocks == -(-images * 196 // 128) * 2) == four, (images, blocks)
+
+
+@on_stub
+def test_fp32_1x1_filters_that_a_program_packs():
+    """Size of the copy: in three parts for windows, as it is where they cannot be, none where the filter in place is as good."""
+    for shape, floats in (((24, 64, 56, 56, 64, 1, 1, 0), 6 / 4 * 64 * 64), ((32, 64, 56, 56, 64, 1, 1, 0), 0), ((12, 96, 40, 40, 24, 1, 1, 0), 0),
+                          ((4, 96, 40, 40, 24, 1, 1, 0), 6 / 4 * 32 * 96), ((12, 24, 40, 40, 144, 1, 1, 0), 160 * 24), ((4, 2048, 7, 7, 512, 1, 1, 0), 6 / 4 * 512 * 2048),
+                          ((96, 64, 56, 56, 64, 1, 1, 0), 0), ((8, 256, 56, 56, 512, 1, 2, 0), 6 / 4 * 512 * 256)):
+        n, c, h, w, k, r, stride, pad = shape
+        views = []
+        for a, d in ((X, (n, c, h, w)), (W, (k, c, r, r)), (Y, (n, k, (h - 1) // stride + 1, (w - 1) // stride + 1))):
+            v = image(a, *d, dtype=K.FLOAT)
+            v.strides[:] = [d[1] * d[2] * d[3], d[2] * d[3], d[3], 1]
+            views.append(C.byref(v))
+        assert K.lib().saga_hip_conv2d_pack_bytes(K.CONV_FWD, *views, C.byref(K.ConvParams(pad, stride, 1, 1))) == 4 * floats, shape

@@ -15,11 +15,11 @@ F32 = torch.float32
 
 # N, C, H, W, K, R, stride, pad: forward launch's tile rows in 32s, rounds of loads, taps, wavefronts
 SHAPES = {
-    (3, 16, 17, 11, 33, 1, 1, 0): (1, 2, 1, 1),      # images of no whole fours, a ragged last tile of both kinds
+    (3, 48, 17, 11, 33, 1, 1, 0): (1, 2, 1, 1),      # images of no whole fours, a ragged last tile of both kinds
     (70, 200, 16, 16, 170, 1, 1, 0): (2, 1, 1, 8),   # three whole slices and one of eight channels
     (9, 136, 27, 30, 72, 1, 2, 0): (1, 4, 1, 2),     # pixels apart
     (40, 64, 43, 64, 170, 1, 3, 0): (1, 1, 1, 8),
-    (90, 40, 33, 32, 96, 1, 2, 1): (1, 1, 1, 4),     # some of them outside the image
+    (90, 56, 33, 32, 96, 1, 2, 1): (1, 1, 1, 4),     # some of them outside the image
     (9, 104, 7, 7, 40, 3, 1, 1): (1, 1, 9, 4),       # windows over several images; half a step of channels
     (8, 64, 28, 30, 128, 3, 1, 1): (2, 1, 9, 8),     # the reduction over four
     (5, 40, 70, 66, 64, 3, 1, 1): (2, 1, 9, 4),      # 128 pixels to a window
