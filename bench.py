@@ -47,10 +47,10 @@ FAMILIES = {
 # lines, the per-kernel table and the commit the counters were taken at are in
 # profiles/resnet50_b256_fp16_hbm_counters.txt; they go stale when kernels change, hence the label.
 MEASURED_HBM_BYTES_PER_LAUNCH = {
-    "conv": 268600613,
-    "batchnorm": 413289930,
+    "conv": 266865687,
+    "batchnorm": 413286931,
 }
-TRAFFIC_SOURCE = "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE snapshot at commit 5cfc1f8 (profiles/resnet50_b256_fp16_hbm_counters.txt)"
+TRAFFIC_SOURCE = "rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE snapshot at commit 75bde84 (profiles/resnet50_b256_fp16_hbm_counters.txt)"
 
 
 def by_kind(rows):

@@ -47,8 +47,9 @@ __device__ __forceinline__ float4_t load4(__amdgpu_buffer_rsrc_t r, unsigned v, 
     return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
 }
 
-// Position v of a window is slot (v % 4) * pitch + v / 4 of 16 bytes: with a pitch of 4 mod 8 both writes, four positions apart, and
-// reads, one apart, fall into different banks.  One of the fours is never written by positions: zeros, for taps outside.
+// Position v of a window is slot (v % 4) * pitch + v / 4 of 16 bytes: with a pitch of 4 mod 8 writes, four positions apart, and
+// reads, one apart from a multiple of four on, fall into different banks (a tap beside begins between two: 35 % of the LDS unit's cycles
+// are bank conflicts under nine taps by its counter, 1 % under one).  One of the fours is never written by positions: zeros, for taps outside.
 __host__ __device__ constexpr int window_pitch(int quads) { return quads + ((4 - quads) & 7); }
 constexpr int window_bytes(int quads, int kg) { return 3 * kg * 4 * window_pitch(quads) * 16; }
 

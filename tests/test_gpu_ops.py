@@ -54,8 +54,8 @@ CONV_CASES = [
     # per image; a partial last tile, a row length that is no multiple of anything and 56 output channels
     (37, 64, 56, 56, 64, 3, 1, 1, 1),
     (130, 64, 30, 27, 56, 3, 1, 1, 1),
-    # ... and for the backward filter that does the same (tiles of a whole number of 16-pixel steps): 48 output
-    # channels and a last tile of two rows; eight rows of 32 pixels per tile
+    # ... 48 output channels and a last tile of two rows; eight rows of 32 pixels per tile (the backward filter of these two
+    # goes to the tiles of the GEMM: strips would take no less)
     (64, 64, 30, 56, 48, 3, 1, 1, 1),
     (128, 64, 32, 32, 64, 3, 1, 1, 1),
     # 1x1 from 64 to 256 channels: enough pixels for the streaming kernel (a partial last strip of 64), and a small
