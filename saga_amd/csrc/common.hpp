@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <type_traits>
 
 #include "saga_hip.h"
 
@@ -21,6 +22,25 @@ typedef float float16_t __attribute__((ext_vector_type(16)));
         if(e__ != hipSuccess)                \
             return (int)e__;                 \
     } while(0)
+
+__device__ __forceinline__ int xcd_remap(int b, int nblocks)
+{
+    // hardware hands consecutive workgroup ids to the 8 XCDs round-robin; give each XCD a
+    // contiguous range of tiles instead
+    const int per = nblocks >> 3, rem = nblocks & 7;
+    const int xcd = b & 7, slot = b >> 3;
+    const int base = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
+    return base + slot;
+}
+
+// f(integral_constant I), f(I + 1), .. f(N - 1)
+template <int I, int N, class F> __device__ __forceinline__ void each(F &&f)
+{
+    if constexpr(I < N) {
+        f(std::integral_constant<int, I>());
+        each<I + 1, N>(f);
+    }
+}
 
 static inline hipStream_t as_stream(saga_stream_t s) { return (hipStream_t)s; }
 

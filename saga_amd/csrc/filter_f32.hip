@@ -54,14 +54,6 @@ template <int OFF> __device__ __forceinline__ bf16x8_t read_pixels(unsigned lo, 
     return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
 }
 
-template <int I, int N, class F> __device__ __forceinline__ void each(F &&f)
-{
-    if constexpr(I < N) {
-        f(std::integral_constant<int, I>());
-        each<I + 1, N>(f);
-    }
-}
-
 __device__ __forceinline__ void store_sums(const WindowFilterArgs &t, int split, int k, int c, const float16_t (&acc)[TAPS]) // (below)
 {
     // (a share's partial result is one buffer: rows and columns beyond the filter are outside)
@@ -159,8 +151,7 @@ __global__ void __launch_bounds__(256, 1) conv_f32_bwd_filter_windows(WindowFilt
     const int tid = threadIdx.x, lane = tid & 63, hi = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int mt = wave >> 1, nt = wave & 1;
-    const int nb = gridDim.x, per = nb >> 3, rem = nb & 7, xcd = blockIdx.x & 7;
-    const int b0 = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (blockIdx.x >> 3);
+    const int b0 = xcd_remap(blockIdx.x, gridDim.x);
     const int split = __builtin_amdgcn_readfirstlane(b0 / t.pairs), pair = b0 - split * t.pairs;
     const int kb = __builtin_amdgcn_readfirstlane(pair / t.pairs_c), k0 = kb * 64, c0 = (pair - kb * t.pairs_c) * 64;
 

@@ -36,12 +36,6 @@ struct StripArgs {
     int pairs, pairs_c, splits;
 };
 
-__device__ __forceinline__ int xcd_order(int b, int n)
-{
-    const int per = n >> 3, rem = n & 7, xcd = b & 7;
-    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (b >> 3);
-}
-
 // 8 pixels of one channel: instructions that the compiler does not know to read LDS (it would wait for every load into LDS that is
 // on its way, the next tile's too).  The caller waits.
 template <int LO> __device__ __forceinline__ half8_t read_pixels(unsigned addr)
@@ -50,14 +44,6 @@ template <int LO> __device__ __forceinline__ half8_t read_pixels(unsigned addr)
     asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(a) : "v"(addr), "n"(LO) : "memory");
     asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(b) : "v"(addr), "n"(LO + 512) : "memory");
     return __builtin_bit_cast(half8_t, __builtin_shufflevector(a, b, 0, 1, 2, 3, 4, 5, 6, 7));
-}
-
-template <int I, int N, class F> __device__ __forceinline__ void each(F &&f)
-{
-    if constexpr(I < N) {
-        f(std::integral_constant<int, I>());
-        each<I + 1, N>(f);
-    }
 }
 
 // The order of a tile's work: instruction 18 * j + m multiplies, in step j, x operand m % 6 / 2 (the tap's column) of the top (m < 6),
@@ -185,7 +171,7 @@ template <int TW, int NST, bool OVERLAP> __global__ void __launch_bounds__(256, 
     const int tid = threadIdx.x, lane = tid & 63, hi = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int grp = wave >> 1, nt = wave & 1;
-    const int b0 = xcd_order(blockIdx.x, gridDim.x); // blocks of one share of the tiles are neighbours: they read the same pixels
+    const int b0 = xcd_remap(blockIdx.x, gridDim.x); // blocks of one share of the tiles are neighbours: they read the same pixels
     const int split = __builtin_amdgcn_readfirstlane(b0 / t.pairs), pair = b0 - split * t.pairs;
     const int kb = __builtin_amdgcn_readfirstlane(pair / t.pairs_c), k0 = kb * 64, c0 = (pair - kb * t.pairs_c) * 64;
 

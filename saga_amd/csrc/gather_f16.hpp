@@ -67,16 +67,6 @@ namespace {
 
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 
-__device__ __forceinline__ int xcd_remap(int b, int nblocks)
-{
-    // hardware hands consecutive workgroup ids to the 8 XCDs round-robin; give each XCD a
-    // contiguous range of tiles instead
-    const int per = nblocks >> 3, rem = nblocks & 7;
-    const int xcd = b & 7, slot = b >> 3;
-    const int base = xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per;
-    return base + slot;
-}
-
 // The MFMA takes the filter tile as its first operand, so a lane ends up with 4 consecutive
 // output CHANNELS of one pixel per accumulator group; v_permlane32_swap pairs the two halves
 // of the wave and every lane stores (and, for beta != 0, loads) 16 contiguous bytes.

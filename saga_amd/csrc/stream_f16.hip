@@ -83,12 +83,6 @@ template <int N> __device__ __forceinline__ void lds_wait(half8_t (&v)[N])
         asm volatile("" : "+v"(v[i])); // (results of the reads above, not to be used before the wait)
 }
 
-__device__ __forceinline__ int xcd_order(int b, int n)
-{
-    const int per = n >> 3, rem = n & 7, xcd = b & 7, slot = b >> 3;
-    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + slot;
-}
-
 // LDS of a wavefront: the ring, then its sums in the same place
 template <int TM, int TN, int DEPTH> constexpr int wave_lds()
 {
@@ -153,7 +147,7 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
     const int lkq = (lane & 3) ^ ((lrow >> 2) & 3);
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KS = 1 << k.ks_log2, wm = wave >> k.ks_log2, ks = wave & (KS - 1);
-    int b = xcd_order(blockIdx.x, k.blocks), ci = 0;
+    int b = xcd_remap(blockIdx.x, k.blocks), ci = 0;
     while(!ONE && ci + 1 < k.nclasses && b >= k.cls[ci + 1].block0)
         ci++;
     const Class &c = k.cls[ci];

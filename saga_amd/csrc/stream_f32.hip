@@ -83,12 +83,6 @@ __device__ __forceinline__ float4_t load4(__amdgpu_buffer_rsrc_t r, unsigned v, 
     return __builtin_bit_cast(float4_t, __builtin_amdgcn_raw_buffer_load_b128(r, v, s, 0));
 }
 
-__device__ __forceinline__ int xcd_order(int b, int n)
-{
-    const int per = n >> 3, rem = n & 7, xcd = b & 7, slot = b >> 3;
-    return (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + slot;
-}
-
 template <int PM, int QM, int TM, int TN, int DEPTH, int MAXW, bool EX, typename A>
 __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
 {
@@ -100,7 +94,7 @@ __global__ void __launch_bounds__(64 * MAXW) stream_f32_k(A g)
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KS = g.KS, WM = (int)(blockDim.x >> 6) / KS;
     const int wm = wave / KS, ks = wave - wm * KS;
-    int b = xcd_order(blockIdx.x, g.blocks), ci = 0;
+    int b = xcd_remap(blockIdx.x, g.blocks), ci = 0;
     while(sizeof(A) > sizeof(Args1) && ci + 1 < g.nclasses && b >= g.cls[ci + 1].block0)
         ci++;
     const Class &c = g.cls[ci];

@@ -23,7 +23,6 @@
 #include "out_f32.hpp"
 #include "window_f32.hpp"
 
-#include <stdlib.h>
 #include <algorithm>
 
 namespace {
@@ -72,8 +71,7 @@ __global__ void __launch_bounds__(512) stream_f32_k_window(WinArgs g)
         wn -= WN;
         wm++;
     }
-    const int nb = g.blocks, per = nb >> 3, rem = nb & 7, xcd = blockIdx.x & 7;
-    const int b = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + (blockIdx.x >> 3);
+    const int b = xcd_remap(blockIdx.x, g.blocks);
     const int bm = g.blk.div(b), bq = b - bm * g.nblk_q;
     const int m0 = bm * (32 * TM * WM), n0 = bq * (32 * WN), nw = n0 + 32 * wn;
     const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc((void *)g.p, 0, (int)g.p_bytes, 0x00020000);
