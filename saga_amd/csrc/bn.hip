@@ -14,6 +14,8 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
+
 namespace {
 
 template <typename T, int VN> struct VecT;
@@ -791,14 +793,66 @@ __global__ void __launch_bounds__(256)
 }
 
 // ---------------------------------------------------------------- channels-first kernels
-// One block per channel; HW runs are contiguous, lanes stride along them.
+// A channel is one plane of HW values per sample.  A block owns a contiguous run of a channel's vectors over all samples, so
+// that a channel is spread over as many blocks as the tensor is worth, not one; sums leave a block as one pair, and the pass
+// that follows adds a channel's pairs itself.  A thread's vectors are 256 apart; it has the loads of four on their way at once.
+// us, training forward and backward with relu (one block per channel, one value at a time, which this replaces / this), fp32:
+//   16 channels of 128x32x32  66 /  9, 253 / 10     64 of 128x8x8  24 /  8,  73 / 10     512 of 16x7x7  9 /  8, 12 / 10
+//   16 channels of 512x32x32 534 / 16, 2370 / 39   256 of 32x56x56 175 / 53, 696 / 114   64 of 512x7x7 80 / 12, 586 / 15
+// (256 of 32x56x56: forward 308 MB, backward 719 MB, 5.8 and 6.3 TB/s); two launches each are what bounds the small ones.
 
-template <typename T> __device__ __forceinline__ void block_sum2(float &a, float &b)
+constexpr int CF_MAX_SPLITS = 256; // blocks whose sums one block adds, a pair to a thread
+
+struct Planes {
+    int64_t hwv, vectors, per; // vectors of a plane, of a channel over all samples, of a block
+    int64_t HW, dn;            // values of a plane; how far 256 vectors are, in samples ...
+    int dhw;                   // ... and vectors
+    int splits, partials;      // blocks of a channel, and sums of it
+};
+
+// the vectors of a thread, one after the other
+struct PlaneWalk {
+    int64_t n, hw, i, end;
+    __device__ __forceinline__ PlaneWalk(const Planes &g, int split)
+    {
+        i = split * g.per + threadIdx.x;
+        end = (split + 1) * g.per < g.vectors ? (split + 1) * g.per : g.vectors;
+        n = g.vectors < 1ll << 31 ? (int64_t)((unsigned)i / (unsigned)g.hwv) : i / g.hwv;
+        hw = i - n * g.hwv;
+    }
+    __device__ __forceinline__ void next(const Planes &g)
+    {
+        i += 256;
+        n += g.dn;
+        hw += g.dhw;
+        if(hw >= g.hwv) {
+            hw -= g.hwv;
+            n++;
+        }
+    }
+};
+
+template <int N> struct PlaneBatch { // a thread's next four vectors: where they are, and whether they are
+    int64_t n[N], at[N];
+    bool ok[N];
+    __device__ __forceinline__ void take(PlaneWalk &w, const Planes &g, int64_t c, int VN)
+    {
+#pragma unroll
+        for(int u = 0; u < N; u++) {
+            ok[u] = w.i < w.end;
+            n[u] = ok[u] ? w.n : 0;
+            at[u] = c * g.HW + (ok[u] ? w.hw * VN : 0);
+            w.next(g);
+        }
+    }
+};
+
+// sums of a block's threads, for all of them
+__device__ __forceinline__ void block_sum2(float &a, float &b)
 {
     __shared__ float red[2][4];
     a = wave_sum(a);
     b = wave_sum(b);
-    __syncthreads();
     if((threadIdx.x & 63) == 0) {
         red[0][threadIdx.x >> 6] = a;
         red[1][threadIdx.x >> 6] = b;
@@ -808,121 +862,230 @@ template <typename T> __device__ __forceinline__ void block_sum2(float &a, float
     b = red[1][0] + red[1][1] + red[1][2] + red[1][3];
 }
 
-template <typename T>
-__global__ void __launch_bounds__(256)
-    bn_stats_cf(const T *__restrict__ x, int64_t npitch, int N, int C, int64_t HW, const float *__restrict__ s,
-                const float *__restrict__ b, float *run_m, float *run_v, float *save_mean, float *save_invstd,
-                float *ss, float eps, float expavg)
+// sums of a channel's pairs, for all threads of a block
+__device__ __forceinline__ void channel_sums(const float *__restrict__ partial, int64_t c, int count, double &s0, double &s1)
 {
-    const int c = blockIdx.x;
-    const float k = (float)x[(int64_t)c * HW];
-    float a0 = 0, a1 = 0;
-    for(int n = 0; n < N; n++) {
-        const T *p = x + n * npitch + (int64_t)c * HW;
-        for(int64_t i = threadIdx.x; i < HW; i += 256) {
-            const float d = (float)p[i] - k;
-            a0 += d;
-            a1 += d * d;
-        }
+    typedef float float2_t __attribute__((ext_vector_type(2)));
+    __shared__ double red[2][4];
+    const int tid = threadIdx.x;
+    const float2_t v = tid < count ? ((const float2_t *)partial)[c * count + tid] : float2_t{0, 0};
+    const double a0 = wave_sum_f64(v[0]), a1 = wave_sum_f64(v[1]);
+    if((tid & 63) == 0) {
+        red[0][tid >> 6] = a0;
+        red[1][tid >> 6] = a1;
     }
-    block_sum2<T>(a0, a1);
+    __syncthreads();
+    s0 = red[0][0] + red[0][1] + red[0][2] + red[0][3];
+    s1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+}
+
+// Pass 1 of training forward: sums of (x-K) and (x-K)^2, K the channel's first value (kept: the second pass may write over it).
+template <typename T, int VN>
+__global__ void __launch_bounds__(256)
+    bn_stats_cf(const T *__restrict__ x, int64_t npx, float *__restrict__ partial, float *__restrict__ first, Planes g)
+{
+    typedef Ld<T, VN, false> L;
+    const int64_t c = blockIdx.x / g.splits;
+    const int split = blockIdx.x - (int)c * g.splits;
+    const float k = (float)x[c * g.HW];
+    float a0 = 0, a1 = 0;
+    PlaneWalk w(g, split);
+    while(w.i < w.end) {
+        PlaneBatch<4> p;
+        p.take(w, g, c, VN);
+        typename L::V xr[4];
+#pragma unroll
+        for(int u = 0; u < 4; u++)
+            xr[u] = L::raw(x + p.n[u] * npx + p.at[u]);
+#pragma unroll
+        for(int u = 0; u < 4; u++)
+            if(p.ok[u])
+#pragma unroll
+                for(int j = 0; j < VN; j++) {
+                    const float d = L::at(xr[u], j) - k;
+                    a0 += d;
+                    a1 += d * d;
+                }
+    }
+    block_sum2(a0, a1);
     if(threadIdx.x == 0) {
-        const double M = (double)N * HW;
-        const double dm = a0 / M;
-        double var = a1 / M - dm * dm;
-        if(var < 0)
-            var = 0;
-        const double mean = k + dm;
-        const float inv = (float)(1.0 / sqrt(var + (double)eps));
-        if(save_mean)
-            save_mean[c] = (float)mean;
-        if(save_invstd)
-            save_invstd[c] = inv;
-        if(run_m)
-            run_m[c] = (float)((1.0 - expavg) * run_m[c] + expavg * mean);
-        if(run_v) {
-            const double unb = M > 1 ? var * M / (M - 1.0) : var;
-            run_v[c] = (float)((1.0 - expavg) * run_v[c] + expavg * unb);
-        }
-        const float sc = s[c] * inv;
-        ss[c] = sc;
-        ss[C + c] = b[c] - (float)mean * sc;
+        partial[2 * (int64_t)blockIdx.x] = a0;
+        partial[2 * (int64_t)blockIdx.x + 1] = a1;
+        if(split == 0)
+            first[c] = k;
     }
 }
 
-template <typename T, int MODE>
+// y = x*scale[c] + shift[c] (+ z) (relu).  TRAIN: from the sums that bn_stats_cf left; the first block of a channel writes what
+// outlives the launch.  Otherwise run_m and run_v are the mean and the variance to normalise with.
+template <typename T, int VN, bool TRAIN>
 __global__ void __launch_bounds__(256)
-    bn_apply_cf(const T *__restrict__ x, int64_t npx, const T *__restrict__ z, int64_t npz, T *__restrict__ y,
-                int64_t npy, const float *__restrict__ s, const float *__restrict__ b, const float *__restrict__ m,
-                const float *__restrict__ v, const float *__restrict__ ss, float eps, int N, int C, int64_t HW,
-                int flags)
+    bn_apply_cf(const T *x, int64_t npx, const T *z, int64_t npz, T *y, int64_t npy, const float *__restrict__ partial,
+                const float *__restrict__ kept, const float *__restrict__ s, const float *__restrict__ b, float *run_m, float *run_v, float *save_mean, float *save_invstd, double M, float eps, float expavg, int flags, Planes g)
 {
-    const int64_t total = (int64_t)N * C * HW;
-    const bool relu = flags & SAGA_BN_RELU, add = flags & SAGA_BN_ADD;
-    for(int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t nc = i / HW, hw = i - nc * HW;
-        const int c = (int)(nc % C);
-        const int64_t n = nc / C;
-        float sc, sh;
-        if(MODE == 0) {
-            sc = s[c] * rsqrtf(v[c] + eps);
-            sh = b[c] - m[c] * sc;
-        } else {
-            sc = ss[c];
-            sh = ss[C + c];
+    typedef Ld<T, VN, false> L;
+    const int64_t c = blockIdx.x / g.splits;
+    const int split = blockIdx.x - (int)c * g.splits;
+    const bool relu = flags & SAGA_BN_RELU, add = flags & SAGA_BN_ADD, first = split == 0 && threadIdx.x == 0;
+    PlaneWalk w(g, split);
+    PlaneBatch<4> p;
+    typename L::V xr[4], zr[4];
+    auto load = [&]() {
+        p.take(w, g, c, VN);
+#pragma unroll
+        for(int u = 0; u < 4; u++) {
+            xr[u] = L::raw(x + p.n[u] * npx + p.at[u]);
+            zr[u] = add ? L::raw(z + p.n[u] * npz + p.at[u]) : xr[u];
         }
-        float o = (float)x[n * npx + (int64_t)c * HW + hw] * sc + sh;
-        if(add)
-            o += (float)z[n * npz + (int64_t)c * HW + hw];
-        if(relu)
-            o = (o != o) ? o : fmaxf(o, 0.0f);
-        y[n * npy + (int64_t)c * HW + hw] = (T)o;
+    };
+    // (a thread without a vector requests the channel's first: all have to meet below)
+    bool more = w.i < w.end;
+    load();
+    float sc, sh;
+    if constexpr(TRAIN) {
+        const float k = kept[c], sv = s[c], bv = b[c];
+        const float rm = first && run_m ? run_m[c] : 0.0f, rv = first && run_v ? run_v[c] : 0.0f;
+        double s0, s1;
+        channel_sums(partial, c, g.partials, s0, s1);
+        finish_stats(s0, s1, k, M, eps, expavg, sv, bv, rm, rv, first, run_m, run_v, save_mean, save_invstd, (int)c, sc, sh);
+    } else {
+        sc = s[c] * rsqrtf(run_v[c] + eps);
+        sh = b[c] - run_m[c] * sc;
+    }
+    while(more) {
+#pragma unroll
+        for(int u = 0; u < 4; u++) {
+            if(!p.ok[u])
+                continue;
+            float o[VN];
+#pragma unroll
+            for(int j = 0; j < VN; j++) {
+                float t = __builtin_fmaf(L::at(xr[u], j), sc, sh);
+                if(add)
+                    t += L::at(zr[u], j);
+                if(relu)
+                    t = (t != t) ? t : fmaxf(t, 0.0f);
+                o[j] = t;
+            }
+            L::store(y + p.n[u] * npy + p.at[u], o);
+        }
+        more = w.i < w.end;
+        if(more)
+            load();
     }
 }
 
-template <typename T>
+// Pass 1 of backward: sums of dy' and dy'*(x-mean); dy' = dy, zero where the relu's y is.  dz set: dy' goes there on the way,
+// and the second pass reads it in place of y and dy.
+template <typename T, int VN>
 __global__ void __launch_bounds__(256)
-    bn_bwd_cf(const T *__restrict__ x, int64_t npx, const T *__restrict__ y, int64_t npy, const T *__restrict__ dy,
-              int64_t npdy, T *__restrict__ dx, int64_t npdx, T *__restrict__ dz, int64_t npdz,
-              const float *__restrict__ s, const float *__restrict__ save_mean, const float *__restrict__ save_invstd,
-              float *ds, float *db, int N, int C, int64_t HW, int flags, float beta_dx, float beta_dz, float beta_p)
+    bn_bwd_stats_cf(const T *__restrict__ x, int64_t npx, const T *__restrict__ y, int64_t npy, const T *__restrict__ dy, int64_t npdy,
+                    T *__restrict__ dz, int64_t npdz, const float *__restrict__ save_mean, float *__restrict__ partial, Planes g)
 {
-    const int c = blockIdx.x;
-    const bool relu = flags & SAGA_BN_RELU;
-    const float mean = save_mean[c], inv = save_invstd[c];
+    typedef Ld<T, VN, false> L;
+    const int64_t c = blockIdx.x / g.splits;
+    const int split = blockIdx.x - (int)c * g.splits;
+    const float mean = save_mean[c];
     float a0 = 0, a1 = 0;
-    for(int n = 0; n < N; n++) {
-        const int64_t o = (int64_t)c * HW;
-        for(int64_t i = threadIdx.x; i < HW; i += 256) {
-            float g = (float)dy[n * npdy + o + i];
-            if(relu && !((float)y[n * npy + o + i] > 0.0f))
-                g = 0.0f;
-            a0 += g;
-            a1 += g * ((float)x[n * npx + o + i] - mean);
+    PlaneWalk w(g, split);
+    while(w.i < w.end) {
+        PlaneBatch<4> p;
+        p.take(w, g, c, VN);
+        typename L::V xr[4], gr[4], yr[4];
+#pragma unroll
+        for(int u = 0; u < 4; u++) {
+            xr[u] = L::raw(x + p.n[u] * npx + p.at[u]);
+            gr[u] = L::raw(dy + p.n[u] * npdy + p.at[u]);
+            yr[u] = y ? L::raw(y + p.n[u] * npy + p.at[u]) : gr[u];
+        }
+#pragma unroll
+        for(int u = 0; u < 4; u++) {
+            if(!p.ok[u])
+                continue;
+            float gm[VN];
+#pragma unroll
+            for(int j = 0; j < VN; j++) {
+                gm[j] = y && !(L::at(yr[u], j) > 0.0f) ? 0.0f : L::at(gr[u], j);
+                a0 += gm[j];
+                a1 += gm[j] * (L::at(xr[u], j) - mean);
+            }
+            if(dz)
+                L::store(dz + p.n[u] * npdz + p.at[u], gm);
         }
     }
-    block_sum2<T>(a0, a1);
-    const double M = (double)N * HW;
-    const float dsv = a1 * inv;
-    const float a = s[c] * inv, k0 = (float)(a0 / M), k1 = (float)(dsv * inv / M);
-    for(int n = 0; n < N; n++) {
-        const int64_t o = (int64_t)c * HW;
-        for(int64_t i = threadIdx.x; i < HW; i += 256) {
-            float g = (float)dy[n * npdy + o + i];
-            if(relu && !((float)y[n * npy + o + i] > 0.0f))
-                g = 0.0f;
-            const float v = a * (g - k0 - ((float)x[n * npx + o + i] - mean) * k1);
-            T *pd = dx + n * npdx + o + i;
-            *pd = (T)(beta_dx != 0.0f ? v + beta_dx * (float)*pd : v);
+    block_sum2(a0, a1);
+    if(threadIdx.x == 0) {
+        partial[2 * (int64_t)blockIdx.x] = a0;
+        partial[2 * (int64_t)blockIdx.x + 1] = a1;
+    }
+}
+
+// Pass 2 of backward: dx = s*invstd*(dy' - db/M - (x-mean)*invstd*ds/M) ; dz = dy'.
+template <typename T, int VN>
+__global__ void __launch_bounds__(256)
+    bn_bwd_apply_cf(const T *x, int64_t npx, const T *y, int64_t npy, const T *dy, int64_t npdy, T *dx, int64_t npdx, T *dz,
+                    int64_t npdz, const float *__restrict__ partial, const float *__restrict__ s,
+                    const float *__restrict__ save_mean, const float *__restrict__ save_invstd, float *ds, float *db, double M,
+                    float beta_dx, float beta_dz, float beta_p, Planes g)
+{
+    typedef Ld<T, VN, false> L;
+    const int64_t c = blockIdx.x / g.splits;
+    const int split = blockIdx.x - (int)c * g.splits;
+    const bool first = split == 0 && threadIdx.x == 0;
+    PlaneWalk w(g, split);
+    PlaneBatch<4> p;
+    typename L::V xr[4], gr[4], yr[4];
+    auto load = [&]() {
+        p.take(w, g, c, VN);
+#pragma unroll
+        for(int u = 0; u < 4; u++) {
+            xr[u] = L::raw(x + p.n[u] * npx + p.at[u]);
+            gr[u] = L::raw(dy + p.n[u] * npdy + p.at[u]);
+            yr[u] = y ? L::raw(y + p.n[u] * npy + p.at[u]) : gr[u];
+        }
+    };
+    bool more = w.i < w.end;
+    load();
+    const float mean = save_mean[c], inv = save_invstd[c], sv = s[c];
+    const float ds_old = first && beta_p != 0.0f ? ds[c] : 0.0f, db_old = first && beta_p != 0.0f ? db[c] : 0.0f;
+    double s0, s1;
+    channel_sums(partial, c, g.partials, s0, s1);
+    const double dsv = s1 * inv;
+    if(first) {
+        ds[c] = (float)(beta_p != 0.0f ? dsv + (double)beta_p * ds_old : dsv);
+        db[c] = (float)(beta_p != 0.0f ? s0 + (double)beta_p * db_old : s0);
+    }
+    const float a = (float)(sv * (double)inv), k0 = (float)(s0 / M), k1 = (float)(dsv * inv / M);
+    while(more) {
+#pragma unroll
+        for(int u = 0; u < 4; u++) {
+            if(!p.ok[u])
+                continue;
+            float gv[VN], ov[VN], res[VN];
+            T *const pd = dx + p.n[u] * npdx + p.at[u];
+            if(beta_dx != 0.0f)
+                L::load(pd, ov);
+#pragma unroll
+            for(int j = 0; j < VN; j++) {
+                gv[j] = y && !(L::at(yr[u], j) > 0.0f) ? 0.0f : L::at(gr[u], j);
+                const float v = a * (gv[j] - k0 - (L::at(xr[u], j) - mean) * k1);
+                res[j] = beta_dx != 0.0f ? v + beta_dx * ov[j] : v;
+            }
+            L::store(pd, res);
             if(dz) {
-                T *pz = dz + n * npdz + o + i;
-                *pz = (T)(beta_dz != 0.0f ? g + beta_dz * (float)*pz : g);
+                T *const pz = dz + p.n[u] * npdz + p.at[u];
+                if(beta_dz != 0.0f) {
+                    L::load(pz, ov);
+#pragma unroll
+                    for(int j = 0; j < VN; j++)
+                        gv[j] += beta_dz * ov[j];
+                }
+                L::store(pz, gv);
             }
         }
-    }
-    if(threadIdx.x == 0) {
-        ds[c] = beta_p != 0.0f ? dsv + beta_p * ds[c] : dsv;
-        db[c] = beta_p != 0.0f ? a0 + beta_p * db[c] : a0;
+        more = w.i < w.end;
+        if(more)
+            load();
     }
 }
 
@@ -949,6 +1112,18 @@ static int vec_width(int dtype, int C, std::initializer_list<const SagaTensorVie
     return vn;
 }
 
+// the same for planes
+static int cf_vec_width(int dtype, const CFInfo &f, std::initializer_list<std::pair<const SagaTensorView *, int64_t>> vs)
+{
+    const int vn = dtype == SAGA_HALF ? 8 : 4;
+    if(f.HW % vn)
+        return 1;
+    for(const auto &v : vs)
+        if(v.first && (!aligned16(v.first->ptr) || v.second % vn))
+            return 1;
+    return vn;
+}
+
 // SAGA_HIP_BN_GRIDSTRIDE: bits select the kernels that walk their rows grid-strided (row_run)
 // (1 forward apply, 2 forward statistics, 4 backward statistics, 8 backward apply); default: the two apply passes
 static int gridstride_mask()
@@ -968,6 +1143,24 @@ static bool force_y_mask()
     }
     return v == 1;
 }
+
+// Vectors of a plane of several samples, and blocks with about four of them per thread (at most some 8192, and at most `most` of a channel).
+static Planes plan_planes(const CFInfo &f, int vn, int64_t most)
+{
+    Planes g;
+    g.HW = f.HW;
+    g.hwv = f.HW / vn;
+    g.vectors = g.hwv * f.N;
+    g.dn = 256 / g.hwv;
+    g.dhw = (int)(256 - g.dn * g.hwv);
+    int64_t splits = std::min((g.vectors + 1023) / 1024, std::min(most, std::max<int64_t>(1, 8192 / f.C)));
+    g.per = ((g.vectors + splits - 1) / splits + 255) / 256 * 256;
+    g.splits = g.partials = (int)((g.vectors + g.per - 1) / g.per);
+    return g;
+}
+
+// The blocks of a channel whose sums the workspace has room for: it is sized by the plans for channels-last tensors.
+static int64_t cf_room(const CFInfo &f) { return std::min<int64_t>(CF_MAX_SPLITS, plan((int64_t)f.N * f.HW, f.C).gx); }
 
 static size_t ws_floats(int64_t rows, int C, int dtype)
 {
@@ -1034,18 +1227,18 @@ int saga_hip_bn_infer(const SagaTensorView *x, const SagaTensorView *z, const Sa
         }
 #undef GO
     } else if(as_channels_first(x, &fx) && as_channels_first(y, &fy) && (!add || as_channels_first(z, &fz))) {
-        const int64_t total = (int64_t)fx.N * fx.C * fx.HW;
-        const int g = grid_for(total, 256, 256 * 32);
-        if(x->dtype == SAGA_HALF)
-            bn_apply_cf<half_t, 0><<<g, 256, 0, st>>>((const half_t *)x->ptr, fx.npitch,
-                                                      add ? (const half_t *)z->ptr : nullptr, fz.npitch,
-                                                      (half_t *)y->ptr, fy.npitch, s, b, m, v, nullptr, eps, fx.N,
-                                                      fx.C, fx.HW, flags);
-        else
-            bn_apply_cf<float, 0><<<g, 256, 0, st>>>((const float *)x->ptr, fx.npitch,
-                                                     add ? (const float *)z->ptr : nullptr, fz.npitch,
-                                                     (float *)y->ptr, fy.npitch, s, b, m, v, nullptr, eps, fx.N, fx.C,
-                                                     fx.HW, flags);
+        const int vn = cf_vec_width(x->dtype, fx, {{x, fx.npitch}, {y, fy.npitch}, {add ? z : nullptr, fz.npitch}});
+        const Planes g = plan_planes(fx, vn, 1 << 16);
+#define GO(T, VN)                                                                                                                 \
+    bn_apply_cf<T, VN, false><<<(unsigned)(g.splits * (int64_t)fx.C), 256, 0, st>>>(                                              \
+        (const T *)x->ptr, fx.npitch, add ? (const T *)z->ptr : nullptr, fz.npitch, (T *)y->ptr, fy.npitch, nullptr, nullptr, s, b, \
+        (float *)m, (float *)v, nullptr, nullptr, 0.0, eps, 0.0f, flags, g)
+        if(x->dtype == SAGA_HALF) {
+            if(vn == 8) GO(half_t, 8); else GO(half_t, 1);
+        } else {
+            if(vn == 4) GO(float, 4); else GO(float, 1);
+        }
+#undef GO
     } else {
         return SAGA_HIP_EUNSUPPORTED;
     }
@@ -1096,19 +1289,24 @@ int saga_hip_bn_train_fwd(const SagaTensorView *x, const SagaTensorView *z, cons
         }
 #undef GO
     } else if(as_channels_first(x, &fx) && as_channels_first(y, &fy) && (!add || as_channels_first(z, &fz))) {
-        const int C = fx.C;
-        float *ss = ws;
-        const int64_t total = (int64_t)fx.N * C * fx.HW;
-        const int g = grid_for(total, 256, 256 * 32);
-#define GO(T)                                                                                                      \
-    do {                                                                                                           \
-        bn_stats_cf<T><<<C, 256, 0, st>>>((const T *)x->ptr, fx.npitch, fx.N, C, fx.HW, s, b, run_m, run_v,          \
-                                          save_mean, save_invstd, ss, eps, expavg);                                \
-        bn_apply_cf<T, 1><<<g, 256, 0, st>>>((const T *)x->ptr, fx.npitch, add ? (const T *)z->ptr : nullptr,        \
-                                             fz.npitch, (T *)y->ptr, fy.npitch, nullptr, nullptr, nullptr, nullptr, \
-                                             ss, eps, fx.N, C, fx.HW, flags);                                      \
+        const int vn = cf_vec_width(x->dtype, fx, {{x, fx.npitch}, {y, fy.npitch}, {add ? z : nullptr, fz.npitch}});
+        const Planes g1 = plan_planes(fx, vn, cf_room(fx));
+        Planes g2 = plan_planes(fx, vn, 1 << 16);
+        g2.partials = g1.partials;
+        float *const kept = ws + 2 * (int64_t)fx.C * g1.splits;
+        const double M = (double)fx.N * fx.HW;
+#define GO(T, VN)                                                                                                                 \
+    do {                                                                                                                          \
+        bn_stats_cf<T, VN><<<(unsigned)(g1.splits * (int64_t)fx.C), 256, 0, st>>>((const T *)x->ptr, fx.npitch, ws, kept, g1);    \
+        bn_apply_cf<T, VN, true><<<(unsigned)(g2.splits * (int64_t)fx.C), 256, 0, st>>>(                                          \
+            (const T *)x->ptr, fx.npitch, add ? (const T *)z->ptr : nullptr, fz.npitch, (T *)y->ptr, fy.npitch, ws, kept, s, b,   \
+            run_m, run_v, save_mean, save_invstd, M, eps, expavg, flags, g2);                                                     \
     } while(0)
-        if(x->dtype == SAGA_HALF) GO(half_t); else GO(float);
+        if(x->dtype == SAGA_HALF) {
+            if(vn == 8) GO(half_t, 8); else GO(half_t, 1);
+        } else {
+            if(vn == 4) GO(float, 4); else GO(float, 1);
+        }
 #undef GO
     } else {
         return SAGA_HIP_EUNSUPPORTED;
@@ -1303,12 +1501,30 @@ int saga_hip_bn_bwd_ex(const SagaTensorView *x, const SagaTensorView *y, const S
 #undef GO2
     } else if(!recompute && as_channels_first(x, &fx) && as_channels_first(dy, &fdy) && as_channels_first(dx, &fdx) &&
               (!relu || as_channels_first(y, &fy)) && (!dz || as_channels_first(dz, &fdz))) {
-#define GO(T)                                                                                                         \
-    bn_bwd_cf<T><<<fx.C, 256, 0, st>>>((const T *)x->ptr, fx.npitch, relu ? (const T *)y->ptr : nullptr, fy.npitch,     \
-                                       (const T *)dy->ptr, fdy.npitch, (T *)dx->ptr, fdx.npitch,                      \
-                                       dz ? (T *)dz->ptr : nullptr, fdz.npitch, s, save_mean, save_invstd, ds, db,    \
-                                       fx.N, fx.C, fx.HW, flags, beta_dx, beta_dz, beta_p)
-        if(dt == SAGA_HALF) GO(half_t); else GO(float);
+        const int vn = cf_vec_width(dt, fx, {{x, fx.npitch}, {dy, fdy.npitch}, {dx, fdx.npitch}, {relu ? y : nullptr, fy.npitch}, {dz, fdz.npitch}});
+        const Planes g1 = plan_planes(fx, vn, cf_room(fx));
+        Planes g2 = plan_planes(fx, vn, 1 << 16);
+        g2.partials = g1.partials;
+        const double M = (double)fx.N * fx.HW;
+        // (as above: the first pass leaves dy' in dz)
+        const bool early_dz = dz && beta_dz == 0.0f && relu && dz->ptr != dy->ptr && dz->ptr != x->ptr && dz->ptr != y->ptr;
+#define GO(T, VN)                                                                                                                 \
+    do {                                                                                                                          \
+        T *const zp = dz ? (T *)dz->ptr : nullptr;                                                                                \
+        const T *const yp = relu ? (const T *)y->ptr : nullptr;                                                                   \
+        bn_bwd_stats_cf<T, VN><<<(unsigned)(g1.splits * (int64_t)fx.C), 256, 0, st>>>(                                            \
+            (const T *)x->ptr, fx.npitch, yp, fy.npitch, (const T *)dy->ptr, fdy.npitch, early_dz ? zp : nullptr, fdz.npitch,     \
+            save_mean, ws, g1);                                                                                                   \
+        bn_bwd_apply_cf<T, VN><<<(unsigned)(g2.splits * (int64_t)fx.C), 256, 0, st>>>(                                            \
+            (const T *)x->ptr, fx.npitch, early_dz ? nullptr : yp, fy.npitch, early_dz ? zp : (const T *)dy->ptr,                 \
+            early_dz ? fdz.npitch : fdy.npitch, (T *)dx->ptr, fdx.npitch, early_dz ? nullptr : zp, fdz.npitch, ws, s, save_mean,  \
+            save_invstd, ds, db, M, beta_dx, beta_dz, beta_p, g2);                                                                \
+    } while(0)
+        if(dt == SAGA_HALF) {
+            if(vn == 8) GO(half_t, 8); else GO(half_t, 1);
+        } else {
+            if(vn == 4) GO(float, 4); else GO(float, 1);
+        }
 #undef GO
     } else {
         return SAGA_HIP_EUNSUPPORTED;
