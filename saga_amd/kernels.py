@@ -5,6 +5,7 @@ PyTorch fallback for any entry point.
 """
 import ctypes as C
 import os
+import struct
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "lib", "libsaga_hip.so")
@@ -18,6 +19,10 @@ BN_RELU, BN_ADD = 1, 2
 
 class TensorView(C.Structure):
     _fields_ = [("ptr", C.c_void_p), ("dims", C.c_int32 * 4), ("strides", C.c_int64 * 4), ("dtype", C.c_int32)]
+
+
+_VIEW = struct.Struct("=Q4i4qi4x")  # TensorView's layout
+assert _VIEW.size == C.sizeof(TensorView)
 
 
 class ConvParams(C.Structure):
@@ -160,16 +165,12 @@ def view(t):
     """SagaTensorView of a torch tensor of rank <= 4 (logical N,C,H,W; strides as they are)."""
     if t is None:
         return None
-    dims = list(t.shape) + [1] * (4 - t.dim())
-    strides = list(t.stride())
-    while len(strides) < 4:
-        strides.append(1)
-    v = TensorView()
-    v.ptr = t.data_ptr()
-    v.dims = (C.c_int32 * 4)(*dims)
-    v.strides = (C.c_int64 * 4)(*strides)
-    v.dtype = _dtype_code(t)
-    return v
+    dims, strides = t.shape, t.stride()
+    if len(dims) < 4:
+        ones = (1,) * (4 - len(dims))
+        dims, strides = (*dims, *ones), (*strides, *ones)
+    # (the fields packed at once: 0.6 us, where setting them one by one takes 1.5 of the 17 that a small convolution takes here)
+    return TensorView.from_buffer_copy(_VIEW.pack(t.data_ptr(), *dims, *strides, _dtype_code(t)))
 
 
 def _ref(v):
@@ -179,6 +180,10 @@ def _ref(v):
 def stream_ptr():
     import torch
 
+    # the handle by itself takes 0.1 us, by way of a Stream object 2.9
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None:
+        return C.c_void_p(raw(torch.cuda.current_device()))
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
