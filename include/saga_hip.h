@@ -197,6 +197,16 @@ int saga_hip_conv2d_fwd_bn_infer(const SagaTensorView *x, const SagaTensorView *
                                  const float *m, const float *v, float eps, int flags, void *workspace,
                                  size_t ws_bytes, saga_stream_t stream);
 
+/* ---- the same with a relu and a max pooling behind it (y: the pooled tensor), which is the stem of an image network: what is between
+ *      them does not reach memory.  Returns SAGA_HIP_EUNSUPPORTED, with nothing written, where there is no such kernel: it is
+ *      for 7x7 convolutions of three channels at stride 2 and pooling of 3x3 at stride 2, fp16 channels-last.  _ok: whether there
+ *      is, for tensors like these at addresses that are multiples of 16. */
+int saga_hip_conv2d_fwd_bn_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
+                                      const SagaConvParams *p, int pool_size, int pool_pad, int pool_stride);
+int saga_hip_conv2d_fwd_bn_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
+                                   const SagaConvParams *p, const float *s, const float *b, const float *m, const float *v,
+                                   float eps, int pool_size, int pool_pad, int pool_stride, saga_stream_t stream);
+
 /* ---- backward data of the convolution that consumes a batch norm's (+ relu) output, with the first pass
  *      of that norm's backward done in the epilogue.  The reference runs cudnnConvolutionBackwardData
  *      (src/cuda/cuda_dnn.cpp:467-476) and then cudnnBatchNormalizationBackwardEx (:2138-2163), whose first

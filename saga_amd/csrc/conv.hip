@@ -273,6 +273,40 @@ int saga_hip_conv2d_fwd_bn_infer(const SagaTensorView *x, const SagaTensorView *
     return fwd_norm(x, w, y, g, e, workspace, ws_bytes, as_stream(stream));
 }
 
+// geometry() of a convolution whose output there is no view of
+static int pooled_geometry(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p, ConvGeom *g)
+{
+    if(!valid_view(x) || !valid_view(w) || !valid_view(y) || !p || p->stride < 1 || p->pad < 0 || p->dilation < 1)
+        return SAGA_HIP_EINVAL;
+    SagaTensorView between = *y;
+    between.dims[1] = w->dims[0];
+    between.dims[2] = conv_dim(x->dims[2], w->dims[2], p->pad, p->stride, p->dilation);
+    between.dims[3] = conv_dim(x->dims[3], w->dims[3], p->pad, p->stride, p->dilation);
+    return between.dims[2] < 1 || between.dims[3] < 1 ? SAGA_HIP_ESHAPE : geometry(x, w, &between, p, g);
+}
+
+int saga_hip_conv2d_fwd_bn_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
+                                      int pool_size, int pool_pad, int pool_stride)
+{
+    ConvGeom g;
+    return !force_direct() && !pooled_geometry(x, w, y, p, &g) && conv_bn_maxpool_ok(x, w, y, g, pool_size, pool_pad, pool_stride);
+}
+
+int saga_hip_conv2d_fwd_bn_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
+                                   const float *s, const float *b, const float *m, const float *v, float eps, int pool_size,
+                                   int pool_pad, int pool_stride, saga_stream_t stream)
+{
+    ConvGeom g;
+    const int r = pooled_geometry(x, w, y, p, &g);
+    if(r)
+        return r;
+    if(!s || !b || !m || !v)
+        return SAGA_HIP_EINVAL;
+    if(force_direct())
+        return SAGA_HIP_EUNSUPPORTED;
+    return conv_bn_maxpool(x, w, y, g, s, b, m, v, eps, pool_size, pool_pad, pool_stride, as_stream(stream));
+}
+
 int saga_hip_conv2d_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx,
                              const SagaConvParams *p, float alpha, float beta, void *workspace, size_t ws_bytes,
                              saga_stream_t stream)

@@ -36,6 +36,12 @@ int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
                   float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, float *stats = nullptr,
                   size_t stats_floats = 0, int *stats_rows = nullptr, const ConvBnFold *bn = nullptr, const void *bias = nullptr,
                   bool *bias_done = nullptr, const void *packed = nullptr);
+// The same with a norm, relu and max pooling behind it, in one launch (stem_f16.hip); y: the pooled tensor.  ok: whether there is one
+// for tensors like these (at addresses of whole vectors).
+bool conv_bn_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, int size,
+                        int pool_pad, int pool_stride);
+int conv_bn_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, const float *s,
+                    const float *b, const float *m, const float *v, float eps, int size, int pool_pad, int pool_stride, hipStream_t st);
 // bytes of the packed filter that a forward launch on these tensors reads (window_f16.hip); 0: none
 size_t conv_mfma_packed_bytes(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g);
 void conv_mfma_pack_job(const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob &job);

@@ -195,7 +195,7 @@ struct HipOperation {
     virtual bool killOutput(const std::shared_ptr<HipStorage> &s) { return false; }
     // inference: write relu(output) to y instead of the output; false if the operation cannot
     virtual bool foldRelu(const std::shared_ptr<HipTensor> &y) { return false; }
-    // do only one's own work again, and write one's own output
+    // do without what was folded in last, and write what was the output before
     virtual void unfold() {}
     // do without an optional input
     virtual void forget(const std::shared_ptr<HipTensor> &t) {}

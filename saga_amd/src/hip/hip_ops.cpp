@@ -233,6 +233,9 @@ struct ConvFwd : public HipOperation {
     const T b_;
     T relu_y_;
     T packed_; // the filter as the kernel loads it
+    // inference: the max pooling behind a folded norm and relu, which is then this operation's output
+    T pool_y_;
+    int pool_size_ = 0, pool_pad_ = 0, pool_stride_ = 0;
     ConvFwd(HipProgram &p, HipProgramUnit &pu, T x, T w, T y, SagaConvParams cp, T b = nullptr)
       : HipOperation("convfwd")
       , x_(x)
@@ -271,8 +274,27 @@ struct ConvFwd : public HipOperation {
         m_kind = "convfwd.bn";
         return true;
     }
+    bool foldPool(int mode, const T &y, int size, int pad, int stride)
+    {
+        if(!bn_y_ || pool_y_ || bn_flags_ != SAGA_BN_RELU || mode != SAGA_POOL_MAX)
+            return false;
+        const SagaTensorView vx = x_->shapeView(), vw = w_->shapeView(), vy = y->shapeView();
+        if(!saga_hip_conv2d_fwd_bn_maxpool_ok(&vx, &vw, &vy, &cp_, size, pad, stride))
+            return false;
+        pool_y_ = y;
+        pool_size_ = size;
+        pool_pad_ = pad;
+        pool_stride_ = stride;
+        m_kind = "convfwd.bn.pool";
+        return true;
+    }
     void unfold() override
     {
+        if(pool_y_) {
+            pool_y_ = nullptr;
+            m_kind = "convfwd.bn";
+            return;
+        }
         bn_s_ = bn_b_ = bn_m_ = bn_v_ = bn_z_ = bn_y_ = relu_y_ = nullptr;
         bn_flags_ = 0;
         m_kind = "convfwd";
@@ -306,8 +328,25 @@ struct ConvFwd : public HipOperation {
                                     p.workspace().size(), S(p)));
         chkSaga(saga_hip_bn_infer(&vy, bn_z_ ? &vz : nullptr, &vo, s, b, m, v, bn_eps_, bn_flags_, S(p)));
     }
+    void execPooled(HipProgram &p)
+    {
+        const SagaTensorView vx = x_->view(), vw = w_->view(), vy = pool_y_->view();
+        const int r = saga_hip_conv2d_fwd_bn_maxpool(&vx, &vw, &vy, &cp_, (const float *)bn_s_->deviceMem(),
+                                                     (const float *)bn_b_->deviceMem(), (const float *)bn_m_->deviceMem(),
+                                                     (const float *)bn_v_->deviceMem(), bn_eps_, pool_size_, pool_pad_,
+                                                     pool_stride_, S(p));
+        if(r == 0)
+            return;
+        if(r != SAGA_HIP_EUNSUPPORTED)
+            chkSaga(r);
+        execFolded(p);
+        const SagaTensorView vb = bn_y_->view();
+        chkSaga(saga_hip_pool_fwd(SAGA_POOL_MAX, &vb, &vy, nullptr, pool_size_, pool_pad_, pool_stride_, S(p)));
+    }
     void exec(HipProgram &p) override
     {
+        if(pool_y_)
+            return execPooled(p);
         if(bn_y_)
             return execFolded(p);
         const SagaTensorView vx = x_->view(), vw = w_->view(), vy = relu_y_ ? relu_y_->view() : y_->view();
@@ -356,12 +395,12 @@ struct ConvFwd : public HipOperation {
         if(packed_ == t)
             packed_ = nullptr;
     }
-    HipOpArgs listOutputs() const override { return {{"y", bn_y_ ? bn_y_ : relu_y_ ? relu_y_ : y_}}; }
+    HipOpArgs listOutputs() const override { return {{"y", pool_y_ ? pool_y_ : bn_y_ ? bn_y_ : relu_y_ ? relu_y_ : y_}}; }
     float *getBeta(const T &t) override { return !bn_y_ && !relu_y_ && t == y_ ? &beta_ : nullptr; }
     double flops() const override { return conv_flops(x_, w_, y_, cp_.group); }
     double bytes() const override
     {
-        return nbytes(x_) + nbytes(w_) + nbytes(y_) * (beta_ != 0 ? 2 : 1) + (bn_z_ ? nbytes(bn_z_) : 0);
+        return nbytes(x_) + nbytes(w_) + (pool_y_ ? nbytes(pool_y_) : nbytes(y_) * (beta_ != 0 ? 2 : 1)) + (bn_z_ ? nbytes(bn_z_) : 0);
     }
 };
 
@@ -2044,8 +2083,8 @@ REGISTER_HIP_TRANSFORM(100, ProgramType::INFERENCE | ProgramType::TRAINING, conc
 
 }  // namespace
 
-// Inference programs: a batch norm behind a convolution, or a relu behind a convolution, product or pooling, becomes part of
-// the operation that writes its input, which then writes the result in place of that input.  Nobody else may see the input:
+// Inference programs: a batch norm behind a convolution, a relu behind a convolution, product or pooling, or a max pooling behind
+// the two in a network's stem becomes part of the operation that writes its input, which then writes the result in place of that input.  Nobody else may see the input:
 // no other operation, not the host, no other program.  What the folded operation reads and writes is touched at the
 // producer's place in the list from then on, so nothing in between may write the one or touch the other.
 void fold_into_producers(HipProgram &p, HipOps &ops)
@@ -2065,9 +2104,10 @@ void fold_into_producers(HipProgram &p, HipOps &ops)
         const HipOp next = ops[j];
         const auto *norm = dynamic_cast<BnInference *>(next.get());
         const auto *act = dynamic_cast<ActFwd *>(next.get());
-        if(!norm && !(act && act->mode_ == SAGA_ACT_RELU))
+        const auto *pool = dynamic_cast<PoolFwd *>(next.get());
+        if(!norm && !pool && !(act && act->mode_ == SAGA_ACT_RELU))
             continue;
-        const T x = norm ? norm->x_ : act->x_, y = norm ? norm->y_ : act->y_;
+        const T x = norm ? norm->x_ : pool ? pool->x_ : act->x_, y = norm ? norm->y_ : pool ? pool->y_ : act->y_;
         const HipStorage *xs = x->m_storage.get(), *ys = y->m_storage.get();
         if(seen_elsewhere.count(x->m_storage.get()) || xs->doubleBuffered())
             continue;
@@ -2092,8 +2132,9 @@ void fold_into_producers(HipProgram &p, HipOps &ops)
             clean &= !touches(in, ys) && !touches(out, ys);
         }
         auto *conv = dynamic_cast<ConvFwd *>(ops[i].get());
-        if(!clean || !(norm ? conv && conv->foldBn(norm->s_, norm->b_, norm->m_, norm->v_, norm->z_, y, norm->eps_, norm->flags_)
-                            : ops[i]->foldRelu(y)))
+        if(!clean || !(norm   ? conv && conv->foldBn(norm->s_, norm->b_, norm->m_, norm->v_, norm->z_, y, norm->eps_, norm->flags_)
+                       : pool ? conv && conv->foldPool(pool->mode_, y, pool->size_, pool->pad_, pool->stride_)
+                              : ops[i]->foldRelu(y)))
             continue;
         p.m_folded.push_back({ops[i], next, x->m_storage});
         ops.erase(ops.begin() + j--);

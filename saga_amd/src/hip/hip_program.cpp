@@ -616,29 +616,35 @@ void HipContext::unfold(HipStorage *s)
         p->unfold(s);
 }
 
-// The folded operation goes back into the list right behind its producer.  The arena stays as it is: what the two read is
-// in use for one operation longer and what they write from one operation later, with nothing else in between, and the
-// storage between them gets memory of its own.
+// The folded operation goes back into the list right behind its producer, after those that were folded into that one later:
+// what they wrote is behind what it writes.  The arena stays as it is: what they read is in use for an operation longer and what
+// they write from an operation later, with nothing else in between, and the storages between them get memory of their own.
 void HipProgram::unfold(HipStorage *s)
 {
     for(size_t f = 0; f < m_folded.size(); f++) {
         if(m_folded[f].between.get() != s)
             continue;
-        const Fold fold = m_folded[f];
-        m_folded.erase(m_folded.begin() + f--);
-        auto it = std::find(m_ops.begin(), m_ops.end(), fold.producer);
-        if(it == m_ops.end()) // nobody needed its result
-            continue;
-        const size_t i = it - m_ops.begin();
-        fold.producer->unfold();
-        m_ops.insert(it + 1, fold.op);
-        if(m_poison_before.size() + 1 == m_ops.size()) {
-            m_poison_before.insert(m_poison_before.begin() + i + 1, std::vector<HipStorage *>());
-            m_poison_after.insert(m_poison_after.begin() + i, std::vector<HipStorage *>());
+        const HipOp producer = m_folded[f].producer;
+        for(size_t k = m_folded.size(); k-- > f;) {
+            if(m_folded[k].producer != producer)
+                continue;
+            const Fold fold = m_folded[k];
+            m_folded.erase(m_folded.begin() + k);
+            auto it = std::find(m_ops.begin(), m_ops.end(), producer);
+            if(it == m_ops.end()) // nobody needed its result
+                continue;
+            const size_t i = it - m_ops.begin();
+            producer->unfold();
+            m_ops.insert(it + 1, fold.op);
+            if(m_poison_before.size() + 1 == m_ops.size()) {
+                m_poison_before.insert(m_poison_before.begin() + i + 1, std::vector<HipStorage *>());
+                m_poison_after.insert(m_poison_after.begin() + i, std::vector<HipStorage *>());
+            }
+            m_written.push_back(fold.between.get());
+            dropGraphs();
+            m_segments.clear();
         }
-        m_written.push_back(s);
-        dropGraphs();
-        m_segments.clear();
+        f--;
     }
 }
 
