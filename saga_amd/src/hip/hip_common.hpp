@@ -427,12 +427,13 @@ public:
     struct Side {
         bool on = false;
         int after = -1, join = 0;
-        hipEvent_t fork = nullptr;      // the side stream waits for this one before the operation
+        hipEvent_t fork = nullptr;      // the side stream waits for this one before the operation (null: it has waited)
         hipEvent_t done = nullptr;      // recorded behind it, if an operation of the main stream waits
         hipEvent_t reached = nullptr;   // main stream: recorded behind the operation, for forks
         hipEvent_t needs = nullptr;     // main stream: waited for in front of the operation
     };
     std::vector<Side> m_side; // indexed like m_ops; empty: all on the program's stream
+    HipOps m_one_stream_ops;  // m_ops before some moved behind others to share an edge
     hipEvent_t m_side_start = nullptr, m_side_end = nullptr; // fork from the step's start, join behind its last operation
     std::vector<hipEvent_t> m_side_events;
     bool m_on_side = false;

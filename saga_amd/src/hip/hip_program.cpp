@@ -380,6 +380,7 @@ void HipContext::planMemory()
             fprintf(stderr, "hip: program %d stays on one stream, %.1f of %.1f MB would be in use\n", pr->m_index,
                     (plan.total + plan.own + workspace) / 1e6, free_bytes / 1e6);
         pr->m_side.clear();
+        pr->m_ops = pr->m_one_stream_ops;
         plan = layOutArena();
     }
     allocSideWorkspace();
@@ -981,6 +982,13 @@ void HipProgram::runOpsGraphed()
     }
 }
 
+// An edge between the streams costs the host 13 us (hipStreamWaitEvent 12 of them), and the main stream 2: a step of ResNet-20 waited
+// for the host, not the GPU, with an edge for every convolution.  So much work of the side stream shares one (us of a step, an edge for each / 20 us / 40
+// / 70: batch 16 1057 / 813 / 844 / 864, 48 1070 / 892 / 909 / 939, 128 1099 / 1064 / 1108 / 1154, 256 1371 / 1343 / 1354 / 1360; more has less to run
+// beside).  How long an operation takes, roughly: launches, and operations and bytes at half of what large ones reach.
+static const double EDGE_US = 20;
+static double estimated_us(const HipOperation &op) { return 8 + std::max(op.flops() / 0.5e9, op.bytes() / 3e6); }
+
 // Which operations run on the context's side stream.
 //
 // Weight and bias gradients are read by the optimizer alone, and the transposed filters by the backward pass: beside the
@@ -993,7 +1001,8 @@ void HipProgram::runOpsGraphed()
 // operation of the main stream that reads its results, or overwrites what it reads, behind it.  One with nothing left to run
 // beside it stays on the main stream: an edge between the streams costs more than a launch.  Storages that it touches have
 // their memory to themselves from the one edge to the other; a program whose operations would hold more than an eighth of the GPU's
-// memory that way stays on one stream, and so does one that would not fit well otherwise (planMemory).
+// memory that way stays on one stream, and so does one that would not fit well otherwise (planMemory); in the order that holds
+// its tensors least long.
 void HipProgram::planSide()
 {
     m_side.clear();
@@ -1031,6 +1040,41 @@ void HipProgram::planSide()
             beside |= !side[j].on;
         side[i].on = beside;
     }
+    // Those that are done before an edge has paid for itself share one: they move behind the operations that follow, as far as
+    // nothing there needs them, until enough of them wait.
+    {
+        std::vector<int> order, waiting;
+        double us = 0, left = 0; // of what waits; of the main stream from here on
+        for(int i = 0; i < n; i++)
+            left += side[i].on ? 0 : estimated_us(*m_ops[i]);
+        for(int i = 0; i < n; i++) {
+            if(side[i].on) {
+                waiting.push_back(i);
+                us += estimated_us(*m_ops[i]);
+            }
+            const bool enough = us >= EDGE_US || left < 2 * EDGE_US;
+            if(enough || std::any_of(waiting.begin(), waiting.end(), [&](int k) { return k != i && ordered(k, i); })) {
+                order.insert(order.end(), waiting.begin(), waiting.end());
+                waiting.clear();
+                us = 0;
+            }
+            if(!side[i].on) {
+                order.push_back(i);
+                left -= estimated_us(*m_ops[i]);
+            }
+        }
+        order.insert(order.end(), waiting.begin(), waiting.end());
+        m_one_stream_ops = m_ops;
+        auto reordered = [&](auto &v) {
+            auto old = v;
+            for(int i = 0; i < n; i++)
+                v[i] = old[order[i]];
+        };
+        reordered(m_ops);
+        reordered(reads);
+        reordered(writes);
+        reordered(side);
+    }
     size_t held = 0;
     std::set<HipStorage *> counted;
     bool any = false;
@@ -1048,8 +1092,10 @@ void HipProgram::planSide()
     chkHip(hipMemGetInfo(&free_bytes, &total_bytes));
     if(any && held > total_bytes / 8 && getenv("SAGA_HIP_VERBOSE"))
         fprintf(stderr, "hip: program %d stays on one stream, %.1f MB would be held for the other\n", m_index, held / 1e6);
-    if(!any || held > total_bytes / 8)
+    if(!any || held > total_bytes / 8) {
+        m_ops = m_one_stream_ops;
         return;
+    }
     auto event = [&](hipEvent_t &e) {
         if(!e) {
             // (both streams are this GPU's: a fence towards the host took 57 of ResNet-20's 1318 us)
@@ -1059,14 +1105,21 @@ void HipProgram::planSide()
         return e;
     };
     std::vector<int> last(n + 1, -1); // the last operation of the side stream that the main stream waits for at each place
+    // the last operation of the main stream that one of a run on the side stream waits for, once for all of them
+    int forked = -2;
     for(int i = 0; i < n; i++) {
         if(!side[i].on)
             continue;
-        int w = i - 1;
-        while(w >= 0 && (side[w].on || !ordered(w, i)))
-            w--;
-        side[i].after = w;
-        side[i].fork = event(w >= 0 ? side[w].reached : m_side_start);
+        int w = -1;
+        for(int k = i; k < n && (k == i || side[k].on); k++)
+            for(int v = i - 1; v > w; v--)
+                if(!side[v].on && ordered(v, k))
+                    w = v;
+        w = std::max(w, forked); // (what it waited for before)
+        side[i].after = std::max(w, -1);
+        if(w > forked || forked == -2)
+            side[i].fork = event(w >= 0 ? side[w].reached : m_side_start);
+        forked = std::max(w, -1);
         last[side[i].join] = i;
     }
     int waited = -1; // the side stream runs in order: what was waited for once covers what came before it
@@ -1121,7 +1174,8 @@ void HipProgram::runOps(const HipOps &ops)
         if(side && side->needs)
             chkHip(hipStreamWaitEvent(m_ctx->m_stream, side->needs, 0));
         if(side && side->on) {
-            chkHip(hipStreamWaitEvent(m_ctx->m_side_stream, side->fork, 0));
+            if(side->fork)
+                chkHip(hipStreamWaitEvent(m_ctx->m_side_stream, side->fork, 0));
             m_on_side = true;
         }
         try {

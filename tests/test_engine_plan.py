@@ -396,3 +396,24 @@ def test_several_strided_writers_of_a_gradient(others):
     want = [16 * 16 * r * r * 2 for r in others]
     assert len(filters) == len(others) and sorted(filters) == sorted(want)
     assert filters[0] == max(want)  # the dense one, where there is one, overwrites
+
+
+@on_stub
+def test_small_operations_share_an_edge():
+    """An edge between the streams costs the host as much as several launches: weight gradients that are done sooner share one, large
+    ones have their own."""
+
+    def edges(net):
+        ctx = S.Context()
+        g, _ = N.build_graph(net, np.zeros((net.batch,) + tuple(net.in_shape), np.float32))
+        p = ctx.create_program(g, net.batch, training=True)
+        p.finalize()
+        ops = stub_gpu.plan(p)
+        assert not stub_gpu.unordered(ops)
+        filters = [op for op in ops if op["side"] and op["kind"] == "convbwdfilter"]
+        return len({op["fork"] for op in filters} - {-1}), len(filters)
+
+    few, count = edges(N.resnet20(16))
+    assert 6 <= few <= 0.7 * count
+    all_, count = edges(N.resnet20(8192))
+    assert all_ >= 0.9 * count
