@@ -229,7 +229,7 @@ __global__ void __launch_bounds__(256) conv_gather_gemm(GatherArgs g)
 // pixels are numbered over the grid OHc x OWc = ceil(OH/stride) x ceil(OW/stride).
 //
 template <int BM, int BN, int WGM, int WGN, int STAGES, int BKT, bool BWD, int PROD = 0, bool BQ = false, bool SPLIT = false>
-__global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ && WGM * WGN + PROD == 8) ? 4 : PROD ? (WGM * WGN + PROD + 3) / 4 : 1)
+__global__ void __launch_bounds__(64 * (WGM * WGN + PROD), (BQ || PROD) && WGM * WGN + PROD == 8 ? 4 : PROD ? (WGM * WGN + PROD + 3) / 4 : 1)
     conv_gather_gemm_dma(GatherArgs g)
 {
     constexpr int NW = WGM * WGN;                      // wavefronts per block

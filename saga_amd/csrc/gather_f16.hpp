@@ -80,12 +80,47 @@ __device__ __forceinline__ unsigned pack2(float a, float b)
     return __builtin_bit_cast(unsigned, v);
 }
 
+// Eight halves at any address of a half; `count` of them are inside the row (the rest reads as zero, and is not written).  Rows of a
+// pitch or at an address that is no multiple of 16 bytes take the same accesses of 16 bytes as others (the hardware splits
+// them where they cross a line), and smaller ones for the vector in which a row ends.
+typedef unsigned any4_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef unsigned any1_t __attribute__((aligned(2)));
+typedef unsigned vec4_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ vec4_t load_any(const half_t *p, int count)
+{
+    vec4_t o = {0, 0, 0, 0};
+    if(count >= 8)
+        o = *(const any4_t *)p;
+    else
+#pragma unroll
+        for(int k = 0; k < 4; k++) {
+            if(count >= 2 * k + 2)
+                o[k] = *(const any1_t *)(p + 2 * k);
+            else if(count == 2 * k + 1)
+                o[k] = *(const unsigned short *)(p + 2 * k);
+        }
+    return o;
+}
+__device__ __forceinline__ void store_any(half_t *p, vec4_t o, int count)
+{
+    if(count >= 8)
+        *(any4_t *)p = o;
+    else
+#pragma unroll
+        for(int k = 0; k < 4; k++) {
+            if(count >= 2 * k + 2)
+                *(any1_t *)(p + 2 * k) = o[k];
+            else if(count == 2 * k + 1)
+                *(unsigned short *)(p + 2 * k) = (unsigned short)o[k];
+        }
+}
+
 // Reads the 32 channels nb .. nb+31 of this lane's pixel row the way the epilogue stores them
 // (16 contiguous bytes per lane: the lower half-wave channels 16q .. 16q+7, the upper one
 // 16q+8 .. 16q+15) and hands every lane the values of ITS accumulator elements: the same
 // half-wave swap as on the way out undoes the regrouping.  All lanes must call it.
-// f[v] belongs to channel nb + 8*(v/4) + 4*hi + v%4.
-__device__ __forceinline__ void load_row32(const half_t *row, bool ok, int nb, int ncols, int hi, float (&f)[16])
+// f[v] belongs to channel nb + 8*(v/4) + 4*hi + v%4.  ANY: rows at any address, of any number of channels.
+template <bool ANY = false> __device__ __forceinline__ void load_row32(const half_t *row, bool ok, int nb, int ncols, int hi, float (&f)[16])
 {
     typedef unsigned u4 __attribute__((ext_vector_type(4)));
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
@@ -93,8 +128,12 @@ __device__ __forceinline__ void load_row32(const half_t *row, bool ok, int nb, i
     for(int q = 0; q < 2; q++) {
         const int n = nb + 16 * q + 8 * hi;
         u4 o = {0, 0, 0, 0};
-        if(ok && n < ncols)
-            o = *(const u4 *)(row + n);
+        if(ok && n < ncols) {
+            if constexpr(ANY)
+                o = load_any(row + n, ncols - n);
+            else
+                o = *(const u4 *)(row + n);
+        }
         const auto s0 = __builtin_amdgcn_permlane32_swap(o[0], o[2], false, false);
         const auto s1 = __builtin_amdgcn_permlane32_swap(o[1], o[3], false, false);
         const unsigned w[4] = {s0[0], s1[0], s0[1], s1[1]}; // elements 8q .. 8q+7, two per word
@@ -251,8 +290,7 @@ __device__ __forceinline__ void stats_block_write(const GatherArgs &g, char *red
 
 template <int TM, int TN, int BN, bool BWD> __device__ __forceinline__ bool stores_staged(const GatherArgs &g)
 {
-    const bool vec_ok = (g.ldo & 7) == 0 && (g.Ngemm & 7) == 0 && ((uintptr_t)g.out & 15) == 0;
-    return TM % 2 == 0 && TN == 2 && BN >= 128 && vec_ok && !(BWD && g.classes > 1) && !g.no_stage;
+    return TM % 2 == 0 && TN == 2 && BN >= 128 && !(BWD && g.classes > 1) && !g.no_stage;
 }
 
 // Inference with a folded batch norm: scale = s/sqrt(v+eps) and shift = b - m*scale of the block's BN channels
@@ -299,17 +337,20 @@ __device__ __forceinline__ void gather_epilogue(const GatherArgs &g, float16_t (
     char *stg = smem + wave * (TM * 32 * TN * 64);
     if(staged && !(!BWD && g.bn_s)) // (the fold's barriers have already seen to it)
         __syncthreads();           // every wavefront is done reading the last slice, which the tiles overwrite
+    // ANY: rows off the grid of 16 bytes, or ending inside it.  us, one channel at a time, which stood here before / this: 48->398
+    // channels, 1x1, 37x25x25 38.9 / @1, 16->180, 3x3, 118x29x29 59.0 / @2 (400 and 184 channels: 8.8, 23.0).
+    auto store = [&](auto any) {
+        constexpr bool ANY = decltype(any)::value;
 #pragma unroll
-    for(int i = 0; i < TM; i++) {
-        bool ok;
-        int64_t pix;
-        rowpix(wm + i * 32 + (lane & 31), ok, pix);
-        okr[i] = ok;
-        half_t *orow = g.out + pix * g.ldo;
+        for(int i = 0; i < TM; i++) {
+            bool ok;
+            int64_t pix;
+            rowpix(wm + i * 32 + (lane & 31), ok, pix);
+            okr[i] = ok;
+            half_t *orow = g.out + pix * g.ldo;
 #pragma unroll
-        for(int j = 0; j < TN; j++) {
-            const int nb = n0 + wn + j * 32;
-            if(vec_ok) {
+            for(int j = 0; j < TN; j++) {
+                const int nb = n0 + wn + j * 32;
                 float f[16];
 #pragma unroll
                 for(int v = 0; v < 16; v++)
@@ -317,7 +358,7 @@ __device__ __forceinline__ void gather_epilogue(const GatherArgs &g, float16_t (
                 typedef _Float16 half4_t __attribute__((ext_vector_type(4)));
                 if(g.beta != 0.0f) {
                     float old[16];
-                    load_row32(orow, ok, nb, g.Ngemm, hi, old);
+                    load_row32<ANY>(orow, ok, nb, g.Ngemm, hi, old);
 #pragma unroll
                     for(int v = 0; v < 16; v++)
                         f[v] += g.beta * old[v];
@@ -326,7 +367,7 @@ __device__ __forceinline__ void gather_epilogue(const GatherArgs &g, float16_t (
                     if(g.bn_s) {
                         float zz[16];
                         if(g.bn_flags & SAGA_BN_ADD)
-                            load_row32(g.z + pix * g.ldz, ok, nb, g.Ngemm, hi, zz);
+                            load_row32<ANY>(g.z + pix * g.ldz, ok, nb, g.Ngemm, hi, zz);
 #pragma unroll
                         for(int q = 0; q < 4; q++) {
                             // scale and shift of the block's channels were put into LDS after the main loop
@@ -346,6 +387,8 @@ __device__ __forceinline__ void gather_epilogue(const GatherArgs &g, float16_t (
                 }
                 // after the swaps: lower half-wave holds channels 0..7 (then 16..23) of the tile,
                 // upper half-wave 8..15 (24..31): one store covers 32 contiguous bytes per pixel
+                if constexpr(ANY)
+                    __builtin_amdgcn_sched_barrier(0); // (one after the other: the registers are the other branch's)
 #pragma unroll
                 for(int q = 0; q < 2; q++) {
                     const unsigned x0 = pack2(f[8 * q + 0], f[8 * q + 1]), x1 = pack2(f[8 * q + 2], f[8 * q + 3]);
@@ -363,63 +406,57 @@ __device__ __forceinline__ void gather_epilogue(const GatherArgs &g, float16_t (
                         const int row = i * 32 + (lane & 31), chunk = 4 * j + 2 * q + hi;
                         *(u4 *)(stg + row * (TN * 64) + ((chunk ^ (row & 7)) << 4)) = o;
                     } else if(ok && n < g.Ngemm) {
-                        *(u4 *)(orow + n) = o;
+                        if constexpr(ANY)
+                            store_any(orow + n, o, g.Ngemm - n);
+                        else
+                            *(u4 *)(orow + n) = o;
                     }
                 }
-            } else if(ok) {
+            }
+        }
+        if constexpr(CAN_STAGE) {
+            if(staged) {
+                // LDS operations of one wavefront complete in order: its reads below see its writes above
+                typedef unsigned u4 __attribute__((ext_vector_type(4)));
+                constexpr int CH = TN * 4, RPI_ = 64 / CH; // 16-byte chunks per row, rows per store instruction
+                const int chunk = lane % CH;
+                const int n = n0 + wn + chunk * 8;
+                // (no residue classes here: the pixel number is the row number, and rows * pitch fits 31 bits)
+                bool ok0;
+                int64_t pix0;
+                rowpix(wm + lane / CH, ok0, pix0);
+                const int p0 = (int)pix0;
+                const int sw = (chunk ^ ((lane / CH) & 7)) << 4; // RPI_ is a multiple of 8: the same for every row of the lane
+                static_assert(RPI_ % 8 == 0, "swizzle period");
 #pragma unroll
-                for(int v = 0; v < 16; v++) {
-                    const int n = nb + (v >> 2) * 8 + hi * 4 + (v & 3);
-                    if(n >= g.Ngemm)
-                        continue;
-                    float val = g.alpha * acc[i][j][v];
-                    if(g.beta != 0.0f)
-                        val += g.beta * (float)orow[n];
-                    if constexpr(!BWD) {
-                        if(g.bn_s) {
-                            const float sc = g.bn_s[n] * rsqrtf(g.bn_v[n] + g.bn_eps);
-                            val = __builtin_fmaf(val, sc, g.bn_b[n] - g.bn_m[n] * sc);
-                            if(g.bn_flags & SAGA_BN_ADD)
-                                val += (float)g.z[pix * g.ldz + n];
-                            if(g.bn_flags & SAGA_BN_RELU)
-                                val = (val != val) ? val : fmaxf(val, 0.0f);
+                for(int it = 0; it < TM * 32 / RPI_; it++) {
+                    const int row = it * RPI_ + lane / CH;
+                    const int p = p0 + it * RPI_;
+                    const u4 o = *(const u4 *)(stg + row * (TN * 64) + sw);
+                    if constexpr(ROWS) {
+                        bool ok;
+                        int64_t pix;
+                        rowpix(wm + row, ok, pix);
+                        if(ok && n < g.Ngemm) {
+                            if constexpr(ANY)
+                                store_any(g.out + (pix * g.ldo + n), o, g.Ngemm - n);
+                            else
+                                *(u4 *)(g.out + (pix * g.ldo + n)) = o;
                         }
+                    } else if(p < g.M && n < g.Ngemm) {
+                        if constexpr(ANY)
+                            store_any(g.out + ((int64_t)p * g.ldo + n), o, g.Ngemm - n);
+                        else
+                            *(u4 *)(g.out + (p * g.ldo + n)) = o;
                     }
-                    orow[n] = (half_t)val;
                 }
             }
         }
-    }
-    if constexpr(CAN_STAGE) {
-        if(staged) {
-            // LDS operations of one wavefront complete in order: its reads below see its writes above
-            typedef unsigned u4 __attribute__((ext_vector_type(4)));
-            constexpr int CH = TN * 4, RPI_ = 64 / CH; // 16-byte chunks per row, rows per store instruction
-            const int chunk = lane % CH;
-            const int n = n0 + wn + chunk * 8;
-            // (no residue classes here: the pixel number is the row number, and rows * pitch fits 31 bits)
-            bool ok0;
-            int64_t pix0;
-            rowpix(wm + lane / CH, ok0, pix0);
-            const int p0 = (int)pix0;
-            const int sw = (chunk ^ ((lane / CH) & 7)) << 4; // RPI_ is a multiple of 8: the same for every row of the lane
-            static_assert(RPI_ % 8 == 0, "swizzle period");
-#pragma unroll
-            for(int it = 0; it < TM * 32 / RPI_; it++) {
-                const int row = it * RPI_ + lane / CH;
-                const int p = p0 + it * RPI_;
-                const u4 o = *(const u4 *)(stg + row * (TN * 64) + sw);
-                if constexpr(ROWS) {
-                    bool ok;
-                    int64_t pix;
-                    rowpix(wm + row, ok, pix);
-                    if(ok && n < g.Ngemm)
-                        *(u4 *)(g.out + (pix * g.ldo + n)) = o;
-                } else if(p < g.M && n < g.Ngemm)
-                    *(u4 *)(g.out + (p * g.ldo + n)) = o;
-            }
-        }
-    }
+    };
+    if(BUFST || vec_ok) // (BUFST's callers have made sure)
+        store(std::false_type());
+    else
+        store(std::true_type());
     // Optional: per-channel sum and sum of squares of this block's outputs, for a batch normalisation that follows
     // (stats_lane_totals, stats_block_write).
     if constexpr(!BWD) {

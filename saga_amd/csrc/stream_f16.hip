@@ -97,8 +97,8 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer(const void *p, unsigned
     return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, p ? (int)bytes : 0, 0x00020000);
 }
 
-// Four channels of a tensor from byte offset `at` (OOB: none), in one access or - rows of any pitch - one by one, `n` of
-// them inside the row.
+// Four channels of a tensor from byte offset `at` (OOB: none), in one access - at any address of a half, the hardware splits what crosses
+// a line - or, where a block's channels end inside four, one by one, `n` of them inside the row.
 __device__ __forceinline__ half4_t load4(__amdgpu_buffer_rsrc_t r, unsigned at, bool vec, int n)
 {
     if(vec)
@@ -204,8 +204,7 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
     if(g.bias)
         bias = load4(buffer(g.bias, 2u * g.N), 2 * nown, false, g.N - nown);
     // and of the first (mostly the only) pixel: what it adds to (beta), its residual, the norm's input
-    const bool vec = ((g.N | g.ldo) & 3) == 0 && ((uintptr_t)g.out & 7) == 0;
-    const bool zvec = vec && (g.ldz & 3) == 0 && ((uintptr_t)g.z & 7) == 0;
+    const bool vec = (g.N & 3) == 0 || n0 + 16 * TN <= g.N;
     const bool with_z = g.bn_flags & SAGA_BN_ADD;
     const __amdgpu_buffer_rsrc_t ro = buffer(g.out, g.out_bytes), rz = buffer(with_z ? g.z : nullptr, g.z_bytes);
     const __amdgpu_buffer_rsrc_t rwas = buffer(g.beta != 0.0f ? g.out : nullptr, g.out_bytes);
@@ -220,7 +219,7 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
     };
     auto request = [&](int pix) {
         old = load4(rwas, pix >= 0 ? (unsigned)(pix * g.ldo + nown) * 2 : OOB, vec, g.N - nown);
-        zz = load4(rz, pix >= 0 ? (unsigned)(pix * g.ldz + nown) * 2 : OOB, zvec, g.N - nown);
+        zz = load4(rz, pix >= 0 ? (unsigned)(pix * g.ldz + nown) * 2 : OOB, vec, g.N - nown);
         if(SUMS) // (its callers have made sure of the alignment)
             xx = load4(buffer(g.bq_x, g.bq_bytes), pix >= 0 ? (unsigned)(pix * g.bq_ldx + nown) * 2 : OOB, true, 4);
     };
