@@ -338,7 +338,7 @@ __device__ __forceinline__ void gather_epilogue(const GatherArgs &g, float16_t (
     if(staged && !(!BWD && g.bn_s)) // (the fold's barriers have already seen to it)
         __syncthreads();           // every wavefront is done reading the last slice, which the tiles overwrite
     // ANY: rows off the grid of 16 bytes, or ending inside it.  us, one channel at a time, which stood here before / this: 48->398
-    // channels, 1x1, 37x25x25 38.9 / @1, 16->180, 3x3, 118x29x29 59.0 / @2 (400 and 184 channels: 8.8, 23.0).
+    // channels, 1x1, 37x25x25 38.9 / 9.6, 16->180, 3x3, 118x29x29 59.0 / 23.7 (400 and 184 channels: 8.8, 23.0).
     auto store = [&](auto any) {
         constexpr bool ANY = decltype(any)::value;
 #pragma unroll
