@@ -3,8 +3,11 @@
 #include "conv.hpp"
 
 struct FilterWindows {
-    int pairs;  // blocks of 64 output channels times blocks of 64 input channels; 0: not this kernel's
-    int splits; // partial results: shares of the tiles
+    int pairs = 0;  // blocks of output channels times blocks of input channels; 0: not this kernel's
+    int splits = 0; // partial results: shares of the tiles
+    int kb, cb;     // output and input channels of a block
+    int rows;       // of a tile, of 8 columns
+    int tiles;      // of all images
 };
 FilterWindows plan_filter_windows(const ConvGeom &g);
 double filter_windows_ns(const FilterWindows &p, const ConvGeom &g); // what it takes

@@ -138,3 +138,54 @@ def test_without_three_parts(value):
     big = want.abs() > 1e30
     assert torch.equal(f[ok & ~big].double(), want[ok & ~big])
     assert torch.allclose(f[ok & big].double(), want[ok & big], rtol=1e-6)
+
+
+# N, C, H, W, K of layers with 32 channels or fewer of a kind, whose wavefronts share a tile's rows: one block and a part of one, the lowest
+# images, tiles that overlap by most of a tile, blocks with unequal numbers of tiles; and what stays with the others
+FEW = {
+    (130, 16, 16, 8, 16): None,     # too little work
+    (420, 16, 17, 9, 8): 256,       # 16 channels of 32 are loaded
+    (48, 16, 32, 32, 16): 128,
+    (90, 32, 33, 17, 24): 256,
+    (130, 24, 16, 31, 32): 173,
+    (500, 32, 8, 9, 32): 256,       # images lower than 16 rows: blocks of 64 input channels
+    (60, 72, 31, 30, 24): 256,      # 32 output channels to a block, two blocks of input channels
+    (60, 24, 15, 40, 200): 256,     # the other way round
+}
+
+
+def _few_routes():
+    L, p = K.lib(), C.byref(P)
+    for (n, c, h, w, k), blocks in FEW.items():
+        x, y, f = (view(torch.empty(d, device="meta"), a) for d, a in (((n, c, h, w), 1 << 20), ((n, k, h, w), 1 << 31), ((k, c, 3, 3), 1 << 32)))
+        need = L.saga_hip_conv2d_workspace_size(K.CONV_BWD_FILTER, C.byref(x), C.byref(f), C.byref(y), p)
+        stub_gpu.launched()
+        assert L.saga_hip_conv2d_bwd_filter(C.byref(x), C.byref(y), C.byref(f), p, 1.0, 0.0, 1 << 33, need, None) == 0
+        yield [b for name, _, b, _ in stub_gpu.launched() if name == "conv_f32_bwd_filter_windows"], blocks
+
+
+@on_stub
+def test_routes_of_few_channels():
+    for ran, blocks in _few_routes():
+        print(ran, blocks)
+        assert ran == ([] if blocks is None else [blocks])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("value", [None, float("inf"), float("nan")], ids=str)
+@pytest.mark.parametrize("shape", [s for s, blocks in FEW.items() if blocks], ids=str)
+def test_few_channels(shape, value):
+    """Exact on whole numbers, as above; an operand without three parts reaches the sums that have it and no other."""
+    n, c, h, w, k = shape
+    g = torch.Generator("cuda").manual_seed(c + h)
+    x = torch.randint(-1023, 1024, (n, c, h, w), device="cuda", generator=g).float()
+    dy = torch.randint(-2, 3, (n, k + 3, h + 2, w + 5), device="cuda", generator=g).float()[:, 2:2 + k, 1:1 + h, 3:3 + w]
+    dy *= torch.rand(dy.shape, device="cuda", generator=g) < 0.25
+    f = torch.randint(-9, 10, (k, c, 3, 3), device="cuda", generator=g).float()
+    if value is not None:
+        x[0, c - 1, h - 1, w - 1] = x[n // 2, 3, 5, 0] = value
+    want = 2 * oracle(x, dy) + f.double()
+    gradient(x, dy, f, 2.0, 1.0)
+    ok = torch.isfinite(want)
+    assert torch.equal(torch.isfinite(f), ok) and want[ok].abs().max() < 2 ** 23
+    assert torch.equal(f[ok].double(), want[ok])
