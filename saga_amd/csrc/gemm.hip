@@ -227,6 +227,35 @@ __global__ void __launch_bounds__(256)
     }
 }
 
+// A lane of the kernels below loads N consecutive elements, at any address.  Where the operand ends before the run does, the run is moved
+// to end there: every load is whole, whatever the sizes, without a branch, and the elements are put where they belong afterwards (rows
+// that two lanes have got are written twice).  Nothing beyond the operand is read.  Loaded element by element where a dimension was no multiple of
+// the run or an address not its own, all of them had to be there before the next could go out; us, before -> now, fp32 / fp16: 64x10x1024
+// 7.9 -> 4.7 / 14 -> 4.7, 33x257x999 9.1 -> 5.0 / 19 -> 5.4, 23x1000x2041 15 -> 6.5 / 21 -> 7.3; the launch is 4.7.
+typedef unsigned run_t __attribute__((ext_vector_type(4)));
+typedef half_t any8_t __attribute__((ext_vector_type(8), aligned(2)));
+typedef float any4_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ int run_of_rows(int n, int row, int rows) { return row < rows - n ? row : rows - n; }
+__device__ __forceinline__ int64_t run_at(bool kcontig, int n, int ld, int row, int rows, int k, int K)
+{
+    return kcontig ? (int64_t)(row < rows ? row : rows - 1) * ld + run_of_rows(n, k, K)
+                   : (int64_t)(k < K ? k : K - 1) * ld + run_of_rows(n, row, rows);
+}
+// steps k to k + N - 1, of which those beyond the reduction are zeros, from the run that was loaded for them
+template <int N, typename V> __device__ __forceinline__ V run_of_steps(V v, int k, int K)
+{
+    run_t w = __builtin_bit_cast(run_t, v);
+    const int by = k - run_of_rows(N, k, K);
+    if(K % N) { // (or it is a whole run, or none)
+        const unsigned far = N == 8 ? by & 4 : by & 2, near = N == 8 ? by & 2 : by & 1;
+        w = far ? run_t{w[2], w[3], 0, 0} : w;
+        w = near ? run_t{w[1], w[2], w[3], 0} : w;
+        if(N == 8)
+            w = by & 1 ? run_t{w[0] >> 16 | w[1] << 16, w[1] >> 16 | w[2] << 16, w[2] >> 16 | w[3] << 16, w[3] >> 16} : w;
+    }
+    return __builtin_bit_cast(V, by < N ? w : run_t{0, 0, 0, 0});
+}
+
 // The same for grids that leave compute units idle (few rows, or few outputs): a 32x32 tile per block of 8 wavefronts that
 // split the reduction, every eighth slice of 64 steps each, and add their tiles through LDS in a fixed order.  What bounds
 // such a product is the chain of trips to memory of one block: with 64x64 tiles fc 2048 -> 1000 ran in 16 blocks of 16
@@ -236,7 +265,7 @@ __global__ void __launch_bounds__(256)
 // the loop holds no barrier.
 constexpr int GS_K = 64, GS_LD = GS_K + 8, GS_WAVES = 8;
 
-template <bool tA, bool tB, bool VEC>
+template <bool tA, bool tB, bool RUNS>
 __global__ void __launch_bounds__(64 * GS_WAVES)
     gemm_split_f16(int M, int N, int K, float alpha, const half_t *__restrict__ A, int lda,
                    const half_t *__restrict__ B, int ldb, float beta, half_t *__restrict__ C, int ldc, ColumnBias cb)
@@ -253,9 +282,8 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
 #pragma unroll
         for(int j = 0; j < 4; j++) {
             const int r = row0 + (kcontig ? (lane >> 3) + 8 * j : (lane & 3) * 8), k = k0 + (kcontig ? (lane & 7) * 8 : (lane >> 2) + 16 * j);
-            if constexpr(VEC) { // runs are either whole or outside: no branch around the load
-                const bool ok = r < rows && k < K;
-                d[j] = *(const half8_t *)(base + (ok ? kcontig ? (int64_t)r * ld + k : (int64_t)k * ld + r : 0));
+            if constexpr(RUNS) {
+                d[j] = *(const any8_t *)(base + run_at(kcontig, 8, ld, r, rows, k, K));
             } else {
 #pragma unroll
                 for(int e = 0; e < 8; e++) {
@@ -269,17 +297,22 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
     };
     // (steps beyond the reduction become zeros here, not where they are loaded: that would wait for the load; rows beyond
     // the operand feed outputs that are not stored)
-    auto put = [&](half_t(*d)[GS_LD], half8_t(&v)[4], bool kcontig, int k0) {
+    auto put = [&](half_t(*d)[GS_LD], half8_t(&v)[4], bool kcontig, int row0, int rows, int k0) {
 #pragma unroll
         for(int j = 0; j < 4; j++) {
-            if(k0 + (kcontig ? (lane & 7) * 8 : (lane >> 2) + 16 * j) >= K)
-                v[j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+            const int k = k0 + (kcontig ? (lane & 7) * 8 : (lane >> 2) + 16 * j);
             if(kcontig) {
+                if(RUNS && k0 + GS_K > K)
+                    v[j] = run_of_steps<8>(v[j], k, K);
                 *(half8_t *)&d[(lane >> 3) + 8 * j][(lane & 7) * 8] = v[j];
             } else {
+                if(k >= K)
+                    v[j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+                const int r = RUNS ? run_of_rows(8, row0 + (lane & 3) * 8, rows) - row0 : (lane & 3) * 8;
 #pragma unroll
                 for(int e = 0; e < 8; e++)
-                    d[(lane & 3) * 8 + e][(lane >> 2) + 16 * j] = v[j][e];
+                    if(!RUNS || r + e >= 0)
+                        d[r + e][(lane >> 2) + 16 * j] = v[j][e];
             }
         }
     };
@@ -293,8 +326,8 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
     if(wave < slices)
         load(wave);
     for(int s = wave; s < slices; s += GS_WAVES) {
-        put(st[wave][0], va, !tA, s * GS_K);
-        put(st[wave][1], vb, tB, s * GS_K);
+        put(st[wave][0], va, !tA, m0, M, s * GS_K);
+        put(st[wave][1], vb, tB, n0, N, s * GS_K);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
         if(s + GS_WAVES < slices)
@@ -336,9 +369,8 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
 // fp32, the same plan: T x T tiles (v_mfma_f32_16x16x4 / 32x32x2), W wavefronts that split the reduction in slices of 32
 // steps (a cache line per row), DEPTH slices of each wavefront in flight.  Small grids are bound by the few compute units
 // that work, and the streaming kernel there by the address unit besides, since its lanes load from a row each: fc 64x3136 ->
-// 1024 ran in 64 blocks, 21 us; in 256 of 16x16 tiles it takes 11, fc 64x1024 -> 10 8 instead of 11 (4 if the weights' rows
-// run along the reduction).
-template <int T, int W, bool tA, bool tB, bool VEC>
+// 1024 ran in 64 blocks, 21 us; in 256 of 16x16 tiles it takes 10.
+template <int T, int W, bool tA, bool tB, bool RUNS>
 __global__ void __launch_bounds__(64 * W)
     gemm_split_f32(int M, int N, int K, float alpha, const float *__restrict__ A, int lda, const float *__restrict__ B, int ldb,
                    float beta, float *__restrict__ C, int ldc, ColumnBias cb)
@@ -357,9 +389,8 @@ __global__ void __launch_bounds__(64 * W)
 #pragma unroll
         for(int j = 0; j < NL; j++) {
             const int r = row0 + (kcontig ? (lane >> 3) + 8 * j : (lane % RL) * 4), k = k0 + (kcontig ? (lane & 7) * 4 : lane / RL + KL * j);
-            if constexpr(VEC) { // runs are either whole or outside: no branch around the load
-                const bool ok = r < rows && k < K;
-                d[j] = *(const float4_t *)(base + (ok ? kcontig ? (int64_t)r * ld + k : (int64_t)k * ld + r : 0));
+            if constexpr(RUNS) {
+                d[j] = *(const any4_t *)(base + run_at(kcontig, 4, ld, r, rows, k, K));
             } else {
 #pragma unroll
                 for(int e = 0; e < 4; e++) {
@@ -372,17 +403,22 @@ __global__ void __launch_bounds__(64 * W)
         }
     };
     // (steps beyond the reduction become zeros here, not where they are loaded: that would wait for the load)
-    auto put = [&](float(*d)[LD], float4_t(&v)[NL], bool kcontig, int k0) {
+    auto put = [&](float(*d)[LD], float4_t(&v)[NL], bool kcontig, int row0, int rows, int k0) {
 #pragma unroll
         for(int j = 0; j < NL; j++) {
-            if(k0 + (kcontig ? (lane & 7) * 4 : lane / RL + KL * j) >= K)
-                v[j] = float4_t{0, 0, 0, 0};
+            const int k = k0 + (kcontig ? (lane & 7) * 4 : lane / RL + KL * j);
             if(kcontig) {
+                if(RUNS && k0 + KS > K)
+                    v[j] = run_of_steps<4>(v[j], k, K);
                 *(float4_t *)&d[(lane >> 3) + 8 * j][(lane & 7) * 4] = v[j];
             } else {
+                if(k >= K)
+                    v[j] = float4_t{0, 0, 0, 0};
+                const int r = RUNS ? run_of_rows(4, row0 + (lane % RL) * 4, rows) - row0 : (lane % RL) * 4;
 #pragma unroll
                 for(int e = 0; e < 4; e++)
-                    d[(lane % RL) * 4 + e][lane / RL + KL * j] = v[j][e];
+                    if(!RUNS || r + e >= 0)
+                        d[r + e][lane / RL + KL * j] = v[j][e];
             }
         }
     };
@@ -404,8 +440,8 @@ __global__ void __launch_bounds__(64 * W)
             const int s = s0 + W * u;
             if(s >= slices)
                 break;
-            put(st[wave][0], va[u], !tA, s * KS);
-            put(st[wave][1], vb[u], tB, s * KS);
+            put(st[wave][0], va[u], !tA, m0, M, s * KS);
+            put(st[wave][1], vb[u], tB, n0, N, s * KS);
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
             __builtin_amdgcn_wave_barrier();
             load(u, s + W * DEPTH);
@@ -451,12 +487,12 @@ template <int T, int W>
 static void launch_split_f32(bool tA, bool tB, int M, int N, int K, float alpha, const float *A, int lda, const float *B, int ldb, float beta,
                              float *C, int ldc, const ColumnBias &cb, hipStream_t st)
 {
-    // (a run of 4 that is only partly in range goes element by element)
-    const bool vec = lda % 4 == 0 && ldb % 4 == 0 && aligned16(A) && aligned16(B) && (tA ? M : K) % 4 == 0 && (tB ? K : N) % 4 == 0;
-    auto kern = tA ? tB ? vec ? gemm_split_f32<T, W, true, true, true> : gemm_split_f32<T, W, true, true, false>
-                        : vec ? gemm_split_f32<T, W, true, false, true> : gemm_split_f32<T, W, true, false, false>
-                   : tB ? vec ? gemm_split_f32<T, W, false, true, true> : gemm_split_f32<T, W, false, true, false>
-                        : vec ? gemm_split_f32<T, W, false, false, true> : gemm_split_f32<T, W, false, false, false>;
+    // (what is shorter than a run goes element by element)
+    const bool runs = (tA ? M : K) >= 4 && (tB ? K : N) >= 4;
+    auto kern = tA ? tB ? runs ? gemm_split_f32<T, W, true, true, true> : gemm_split_f32<T, W, true, true, false>
+                        : runs ? gemm_split_f32<T, W, true, false, true> : gemm_split_f32<T, W, true, false, false>
+                   : tB ? runs ? gemm_split_f32<T, W, false, true, true> : gemm_split_f32<T, W, false, true, false>
+                        : runs ? gemm_split_f32<T, W, false, false, true> : gemm_split_f32<T, W, false, false, false>;
     kern<<<dim3((N + T - 1) / T, (M + T - 1) / T), 64 * W, 0, st>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, cb);
 }
 
@@ -473,15 +509,16 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
         const int a_vec = lda % 8 == 0 && ((uintptr_t)A & 15) == 0, b_vec = ldb % 8 == 0 && ((uintptr_t)B & 15) == 0;
         // Below one 64x64 tile per compute unit the reduction is split, unless it is shorter than there are tiles: then a tile's
         // chain is short beside the work of the others (1024x1024: K = 1024 19 -> 14 us, 256 equal, 64 5.0 -> 5.4 us;
-        // 1000x2048, 512 tiles, K = 256: 12 -> 14 us).  A reduction of up to 16 is one slice in both.
+        // 1000x2048, 512 tiles, K = 256: 12 -> 14 us).  A reduction of up to 16 is one slice in both, and loaded in runs here
+        // (64x1024, K = 10 6.3 -> 4.8 us, 600x300, K = 12 6.6 -> 4.8; 1000x512, K = 16 equal).
         const int64_t tiles = (int64_t)grid.x * grid.y;
-        if(tiles <= 256 && K > 16 && (tiles <= 64 || K > tiles)) {
-            // (a run of 8 that is only partly in range goes element by element)
-            const bool vec = a_vec && (transA ? M : K) % 8 == 0 && b_vec && (transB ? K : N) % 8 == 0;
-            auto kern = transA ? transB ? vec ? gemm_split_f16<true, true, true> : gemm_split_f16<true, true, false>
-                                        : vec ? gemm_split_f16<true, false, true> : gemm_split_f16<true, false, false>
-                               : transB ? vec ? gemm_split_f16<false, true, true> : gemm_split_f16<false, true, false>
-                                        : vec ? gemm_split_f16<false, false, true> : gemm_split_f16<false, false, false>;
+        if(tiles <= 256 && (tiles <= 64 || K > tiles)) {
+            // (what is shorter than a run goes element by element)
+            const bool runs = (transA ? M : K) >= 8 && (transB ? K : N) >= 8;
+            auto kern = transA ? transB ? runs ? gemm_split_f16<true, true, true> : gemm_split_f16<true, true, false>
+                                        : runs ? gemm_split_f16<true, false, true> : gemm_split_f16<true, false, false>
+                               : transB ? runs ? gemm_split_f16<false, true, true> : gemm_split_f16<false, true, false>
+                                        : runs ? gemm_split_f16<false, false, true> : gemm_split_f16<false, false, false>;
             kern<<<dim3((N + 31) / 32, (M + 31) / 32), 64 * GS_WAVES, 0, st>>>(M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
                                                                              ldb, beta, (half_t *)C, ldc, cb);
             SAGA_CHECK_LAUNCH();
@@ -492,7 +529,7 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
     } else if(dtype == SAGA_FLOAT) {
         // (one slice of the LDS tiles holds such a reduction)
         // Up to one 32x32 tile per compute unit the reduction is split over a block (us, stream / 16x16 tiles on 16 and on 4
-        // wavefronts / 32x32 on 8: 64x1024x3136 21 / 11 / 13 / 23, 64x10x1024 11 / 8 / 10 / 18, 64x3136x1024 13 / 12 / 10 / 9,
+        // wavefronts / 32x32 on 8: 64x1024x3136 21 / 11 / 13 / 23, 64x10x1024, by elements, 11 / 8 / 10 / 18, 64x3136x1024 13 / 12 / 10 / 9,
         // 128x1000x2048 16 / 18 / 15 / 17, 512x512x512 8.1 / 9.4 / 7.4 / 6.6, 300x300x32 4.7 / 3.6 / 2.7 / 3.4; beyond it
         // 512x1024x3136 43 / 69 / 57 / 46, 1024x1024x256 11 / 22 / 13 / 14).
         const int64_t t32 = ((int64_t)(M + 31) / 32) * ((N + 31) / 32), t16 = ((int64_t)(M + 15) / 16) * ((N + 15) / 16);

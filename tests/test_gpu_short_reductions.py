@@ -131,3 +131,25 @@ def test_fp16_gradients_of_other_channel_counts(N, Cc, H, W, Kk, R, stride, pad)
         assert_close(host(dw), ref.conv2d_bwd_filter(x, dy, w.shape, pad, stride) + 1, HALF, "dw", tol=2e-3)
         K.conv2d(K.CONV_BWD_DATA, dyd, wd, dx, pad, stride, beta=1.0)
         assert_close(host(dx), ref.conv2d_bwd_data(dy, w, x.shape, pad, stride) + 1, HALF, "dx", tol=2e-3)
+
+
+@pytest.mark.parametrize("dtype", [HALF, F32])
+@pytest.mark.parametrize("tA", [0, 1])
+@pytest.mark.parametrize("tB", [0, 1])
+@pytest.mark.parametrize("M,N,Kd", [(8, 8, 8), (9, 10, 15), (39, 10, 64), (64, 10, 1024), (35, 17, 9), (17, 35, 70), (4, 5, 131), (33, 66, 7)])
+def test_gemm_runs(M, N, Kd, tA, tB, dtype):
+    """Runs that end where an operand's row does, at any address: operands inside larger ones full of NaN."""
+    rng = np.random.default_rng(M + N + Kd)
+    A, B = rnd(rng, M, Kd, dtype=dtype), rnd(rng, Kd, N, dtype=dtype)
+
+    def inside(a):
+        t = torch.full((a.shape[0] + 2, a.shape[1] + 3), float("nan"), device="cuda", dtype=dtype)
+        t[1:-1, 1:-2] = dev(a, dtype)
+        return t, t.data_ptr() + (t.shape[1] + 1) * t.element_size()
+
+    Ad, pa = inside(A.T if tA else A)
+    Bd, pb = inside(B.T if tB else B)
+    Cd = dev(np.ones((M, N), np.float32), dtype)
+    K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 0.5, pa, Ad.shape[1], pb, Bd.shape[1], 1.0, K.ptr(Cd), N,
+                                  K.HALF if dtype == HALF else K.FLOAT, S()))
+    assert_close(host(Cd), 0.5 * (A.astype(np.float64) @ B) + 1, dtype, "gemm", tol=1e-3 if dtype == HALF else 1e-5)
