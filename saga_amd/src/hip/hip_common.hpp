@@ -328,7 +328,7 @@ public:
     void leaveArena(HipStorage &s);
     // somebody looks at this storage who did not when programs were finalized: operations that were folded into the one
     // that writes it become operations again, from the next step on
-    void unfold(HipStorage *s);
+    bool unfold(HipStorage *s);
 };
 
 class HipProgram : public Program {
@@ -452,7 +452,7 @@ public:
         std::shared_ptr<HipStorage> between;
     };
     std::vector<Fold> m_folded;
-    void unfold(HipStorage *s);
+    bool unfold(HipStorage *s);
 
     SagaAux *m_aux = nullptr; // pinned host memory the optimizer kernels write their flags to
     float m_mp_scaling = 1.0f;

@@ -211,7 +211,8 @@ std::shared_ptr<Tensor> HipContext::resolveTensor(std::shared_ptr<Tensor> src)
     if(it == m_tensors.end())
         return nullptr;
     m_exported.push_back(it->second->m_storage);
-    unfold(it->second->m_storage.get());
+    if(unfold(it->second->m_storage.get()) && !it->second->m_storage->allocated())
+        it->second->m_storage->allocOwn(); // (not by the operation that writes it: its next launch may be one that is recorded)
     // a tensor the host holds keeps its contents between steps: out of the shared arena
     // (reference: src/cuda/cuda_common.cpp:145-158)
     leaveArena(*it->second->m_storage);
@@ -611,17 +612,20 @@ std::set<HipStorage *> readBeforeWritten(const HipOps &ops)
     return read;
 }
 
-void HipContext::unfold(HipStorage *s)
+bool HipContext::unfold(HipStorage *s)
 {
+    bool any = false;
     for(HipProgram *p : m_programs)
-        p->unfold(s);
+        any |= p->unfold(s);
+    return any;
 }
 
 // The folded operation goes back into the list right behind its producer, after those that were folded into that one later:
 // what they wrote is behind what it writes.  The arena stays as it is: what they read is in use for an operation longer and what
 // they write from an operation later, with nothing else in between, and the storages between them get memory of their own.
-void HipProgram::unfold(HipStorage *s)
+bool HipProgram::unfold(HipStorage *s)
 {
+    bool any = false;
     for(size_t f = 0; f < m_folded.size(); f++) {
         if(m_folded[f].between.get() != s)
             continue;
@@ -644,9 +648,11 @@ void HipProgram::unfold(HipStorage *s)
             m_written.push_back(fold.between.get());
             dropGraphs();
             m_segments.clear();
+            any = true;
         }
         f--;
     }
+    return any;
 }
 
 // Backward liveness over the op list, treated as one iteration of a loop: a storage is needed

@@ -90,3 +90,21 @@ def test_residual_behind_the_convolution_and_a_window():
 
     for got, want in zip(run(), run(disable_op_fusing=True)):
         close(got, want, S.FLOAT)
+
+
+def test_late_resolve_inside_a_recorded_run(monkeypatch):
+    """What a folded operation wrote gets its memory when somebody asks for it, not between the launches that are recorded."""
+    monkeypatch.setenv("SAGA_HIP_GRAPH", "1")
+    net = N.resnet20(4, dtype=S.FLOAT)
+    x = np.random.default_rng(3).standard_normal((4,) + tuple(net.in_shape)).astype(np.float32)
+    g, t = N.build_graph(net, x, with_classifier=False)
+    ctx = S.Context()
+    p = ctx.create_program(g, 4, training=False)
+    out = ctx.resolve(t[net.output])
+    p.run(4)
+    first = out.read().copy()
+    conv = ctx.resolve(t[[n for n in net.nodes if n["type"] == "conv"][9]["out"]])
+    for _ in range(3):
+        p.run(2)
+        np.testing.assert_allclose(out.read(), first, rtol=0, atol=1e-5 * np.abs(first).max())
+        assert np.abs(conv.read()).max() > 0
