@@ -269,6 +269,11 @@ int saga_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, cons
 int saga_hip_gemm_bias(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B,
                        int ldb, float beta, void *C, int ldc, int dtype, const void *bias, int bias_dtype, int relu,
                        saga_stream_t stream);
+/* C = op(A)*op(B) * alpha where y is positive, else zero: the gradient of the input of a relu whose output is y (C's type and ldc).
+ * Products whose reduction is split (_ok); SAGA_HIP_EUNSUPPORTED (nothing enqueued) otherwise. */
+int saga_hip_gemm_relu_bwd_ok(int M, int N, int K, int dtype);
+int saga_hip_gemm_relu_bwd(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B, int ldb,
+                           void *C, int ldc, int dtype, const void *y, saga_stream_t stream);
 
 /* ---- batch normalisation (spatial, per channel; s,b,m,v and saved statistics are fp32 [C]).
  *      infer: cudnnBatchNormalizationForwardInference (src/cuda/cuda_dnn.cpp:1641-1651);
@@ -342,6 +347,12 @@ int saga_hip_pool_fwd_relu(int mode, const SagaTensorView *x, const SagaTensorVi
                            saga_stream_t stream);
 int saga_hip_pool_bwd(int mode, const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *dy,
                       const SagaTensorView *dx, int size, int pad, int stride, float beta, saga_stream_t stream);
+/* The backward of a max pooling and of the relu whose output x it pools: dx is the gradient of the relu's input.  Windows that tile
+ * rows of consecutive elements (2x2 and 3x3); SAGA_HIP_EUNSUPPORTED (nothing enqueued) otherwise. */
+int saga_hip_maxpool_bwd_relu_ok(const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *dy, const SagaTensorView *dx,
+                                 int size, int pad, int stride);
+int saga_hip_maxpool_bwd_relu(const SagaTensorView *x, const SagaTensorView *y, const SagaTensorView *dy, const SagaTensorView *dx,
+                              int size, int pad, int stride, saga_stream_t stream);
 /* Max pooling for training that remembers where each maximum came from.  No single counterpart in the
  * reference: cudnnPoolingBackward re-derives the maximum from x and y (src/cuda/cuda_dnn.cpp:873-899); here
  * the forward pass leaves one byte per output element (window position r*size + s of the first maximum,

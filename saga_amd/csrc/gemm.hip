@@ -73,11 +73,18 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// what follows a product: a bias per column, in the product's type or fp32, and a relu
+// what follows a product: a bias per column, in the product's type or fp32, and a relu; or the backward of a relu, whose output
+// (of the product's type, its rows as far apart) is positive where the gradient passes.  Only the split reductions have the latter:
+// of fc 64x10 -> 1024 it takes nothing (4.9 us with the launch), a launch of its own 4.6.
 struct ColumnBias {
     const half_t *h;
     const float *f;
     int relu;
+    const void *gate;
+    template <typename T> __device__ __forceinline__ float pass(float v, int64_t at) const
+    {
+        return gate ? v * ((float)((const T *)gate)[at] > 0.0f ? 1.0f : 0.0f) : v;
+    }
     __device__ __forceinline__ float apply(float v, int n) const
     {
         if(h)
@@ -359,7 +366,7 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
         if(m < M && n < N) {
             half_t *o = C + (int64_t)m * ldc + n;
             r *= alpha;
-            *o = (half_t)cb.apply(beta != 0.0f ? r + beta * (float)*o : r, n);
+            *o = (half_t)cb.pass<half_t>(cb.apply(beta != 0.0f ? r + beta * (float)*o : r, n), (int64_t)m * ldc + n);
         }
     }
 }
@@ -478,7 +485,7 @@ __global__ void __launch_bounds__(64 * W)
         if(m < M && n < N) {
             float *o = C + (int64_t)m * ldc + n;
             r *= alpha;
-            *o = cb.apply(beta != 0.0f ? r + beta * *o : r, n);
+            *o = cb.pass<float>(cb.apply(beta != 0.0f ? r + beta * *o : r, n), (int64_t)m * ldc + n);
         }
     }
 }
@@ -496,6 +503,17 @@ static void launch_split_f32(bool tA, bool tB, int M, int N, int K, float alpha,
     kern<<<dim3((N + T - 1) / T, (M + T - 1) / T), 64 * W, 0, st>>>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, cb);
 }
 
+// Below one 64x64 tile per compute unit the reduction of a product in fp16 is split, unless it is shorter than there are tiles: then a tile's
+// chain is short beside the work of the others (1024x1024: K = 1024 19 -> 14 us, 256 equal, 64 5.0 -> 5.4 us;
+// 1000x2048, 512 tiles, K = 256: 12 -> 14 us).  A reduction of up to 16 is one slice in both, and loaded in runs there
+// (64x1024, K = 10 6.3 -> 4.8 us, 600x300, K = 12 6.6 -> 4.8; 1000x512, K = 16 equal).
+// In fp32 it is split up to one 32x32 tile per compute unit.
+static bool splits(int M, int N, int K, int dtype)
+{
+    const int64_t t64 = ((int64_t)(M + 63) / 64) * ((N + 63) / 64), t32 = ((int64_t)(M + 31) / 32) * ((N + 31) / 32);
+    return dtype == SAGA_HALF ? t64 <= 256 && (t64 <= 64 || K > t64) : t32 <= 256;
+}
+
 static int gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B, int ldb,
                 float beta, void *C, int ldc, int dtype, const ColumnBias &cb, saga_stream_t stream)
 {
@@ -507,12 +525,7 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
     hipStream_t st = as_stream(stream);
     if(dtype == SAGA_HALF) {
         const int a_vec = lda % 8 == 0 && ((uintptr_t)A & 15) == 0, b_vec = ldb % 8 == 0 && ((uintptr_t)B & 15) == 0;
-        // Below one 64x64 tile per compute unit the reduction is split, unless it is shorter than there are tiles: then a tile's
-        // chain is short beside the work of the others (1024x1024: K = 1024 19 -> 14 us, 256 equal, 64 5.0 -> 5.4 us;
-        // 1000x2048, 512 tiles, K = 256: 12 -> 14 us).  A reduction of up to 16 is one slice in both, and loaded in runs here
-        // (64x1024, K = 10 6.3 -> 4.8 us, 600x300, K = 12 6.6 -> 4.8; 1000x512, K = 16 equal).
-        const int64_t tiles = (int64_t)grid.x * grid.y;
-        if(tiles <= 256 && (tiles <= 64 || K > tiles)) {
+        if(splits(M, N, K, dtype)) {
             // (what is shorter than a run goes element by element)
             const bool runs = (transA ? M : K) >= 8 && (transB ? K : N) >= 8;
             auto kern = transA ? transB ? runs ? gemm_split_f16<true, true, true> : gemm_split_f16<true, true, false>
@@ -524,16 +537,18 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
             SAGA_CHECK_LAUNCH();
             return 0;
         }
+        if(cb.gate)
+            return SAGA_HIP_EUNSUPPORTED;
         gemm_mfma_f16<<<grid, 256, 0, st>>>(transA, transB, M, N, K, alpha, (const half_t *)A, lda, (const half_t *)B,
                                             ldb, beta, (half_t *)C, ldc, a_vec, b_vec, cb);
     } else if(dtype == SAGA_FLOAT) {
         // (one slice of the LDS tiles holds such a reduction)
-        // Up to one 32x32 tile per compute unit the reduction is split over a block (us, stream / 16x16 tiles on 16 and on 4
+        // us, stream / 16x16 tiles on 16 and on 4
         // wavefronts / 32x32 on 8: 64x1024x3136 21 / 11 / 13 / 23, 64x10x1024, by elements, 11 / 8 / 10 / 18, 64x3136x1024 13 / 12 / 10 / 9,
         // 128x1000x2048 16 / 18 / 15 / 17, 512x512x512 8.1 / 9.4 / 7.4 / 6.6, 300x300x32 4.7 / 3.6 / 2.7 / 3.4; beyond it
         // 512x1024x3136 43 / 69 / 57 / 46, 1024x1024x256 11 / 22 / 13 / 14).
         const int64_t t32 = ((int64_t)(M + 31) / 32) * ((N + 31) / 32), t16 = ((int64_t)(M + 15) / 16) * ((N + 15) / 16);
-        if(t32 <= 256) {
+        if(splits(M, N, K, dtype)) {
             auto go = t16 <= 256 && K > 128   ? launch_split_f32<16, 16>
                       : t32 >= 192 && K > 64 ? launch_split_f32<32, 8>
                                              : launch_split_f32<16, 4>;
@@ -541,6 +556,8 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
             SAGA_CHECK_LAUNCH();
             return 0;
         }
+        if(cb.gate)
+            return SAGA_HIP_EUNSUPPORTED;
         if(K > 16) {
             const int r = stream_f32_gemm(transA, transB, M, N, K, alpha, (const float *)A, lda, (const float *)B, ldb, beta,
                                           (float *)C, ldc, cb.f, cb.relu, st);
@@ -558,7 +575,7 @@ static int gemm(int transA, int transB, int M, int N, int K, float alpha, const 
 extern "C" int saga_hip_gemm(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda,
                              const void *B, int ldb, float beta, void *C, int ldc, int dtype, saga_stream_t stream)
 {
-    return gemm(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, dtype, ColumnBias{nullptr, nullptr, 0}, stream);
+    return gemm(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, dtype, ColumnBias{nullptr, nullptr, 0, nullptr}, stream);
 }
 
 extern "C" int saga_hip_gemm_bias(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda,
@@ -568,6 +585,19 @@ extern "C" int saga_hip_gemm_bias(int transA, int transB, int M, int N, int K, f
     if(bias && bias_dtype != SAGA_FLOAT && !(bias_dtype == SAGA_HALF && dtype == SAGA_HALF))
         return SAGA_HIP_EUNSUPPORTED;
     const ColumnBias cb = {bias_dtype == SAGA_HALF ? (const half_t *)bias : nullptr, bias_dtype == SAGA_FLOAT ? (const float *)bias : nullptr,
-                           relu};
+                           relu, nullptr};
     return gemm(transA, transB, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, dtype, cb, stream);
+}
+
+extern "C" int saga_hip_gemm_relu_bwd_ok(int M, int N, int K, int dtype)
+{
+    return M > 0 && N > 0 && K > 0 && (dtype == SAGA_HALF || dtype == SAGA_FLOAT) && splits(M, N, K, dtype);
+}
+
+extern "C" int saga_hip_gemm_relu_bwd(int transA, int transB, int M, int N, int K, float alpha, const void *A, int lda, const void *B,
+                                      int ldb, void *C, int ldc, int dtype, const void *y, saga_stream_t stream)
+{
+    if(!y)
+        return SAGA_HIP_EINVAL;
+    return gemm(transA, transB, M, N, K, alpha, A, lda, B, ldb, 0.0f, C, ldc, dtype, ColumnBias{nullptr, nullptr, 0, y}, stream);
 }

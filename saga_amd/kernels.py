@@ -106,6 +106,10 @@ SIGNATURES = {
     "saga_hip_pool_fwd": (_I, [_I, _TV, _TV, _TV, _I, _I, _I, _VP]),
     "saga_hip_pool_fwd_relu": (_I, [_I, _TV, _TV, _I, _I, _I, _VP]),
     "saga_hip_pool_bwd": (_I, [_I, _TV, _TV, _TV, _TV, _I, _I, _I, _F, _VP]),
+    "saga_hip_gemm_relu_bwd_ok": (_I, [_I, _I, _I, _I]),
+    "saga_hip_gemm_relu_bwd": (_I, [_I, _I, _I, _I, _I, _F, _VP, _I, _VP, _I, _VP, _I, _I, _VP, _VP]),
+    "saga_hip_maxpool_bwd_relu_ok": (_I, [_TV, _TV, _TV, _TV, _I, _I, _I]),
+    "saga_hip_maxpool_bwd_relu": (_I, [_TV, _TV, _TV, _TV, _I, _I, _I, _VP]),
     "saga_hip_add": (_I, [_TV, _TV, _TV, _VP]),
     "saga_hip_axpby": (_I, [_TV, _TV, _F, _F, _VP]),
     "saga_hip_convert": (_I, [_TV, _TV, _F, _VP]),

@@ -193,7 +193,7 @@ struct HipOperation {
     virtual float *getBeta(const std::shared_ptr<HipTensor> &t) { return nullptr; }
     // drop an output nobody reads; false if the op cannot do without it
     virtual bool killOutput(const std::shared_ptr<HipStorage> &s) { return false; }
-    // inference: write relu(output) to y instead of the output; false if the operation cannot
+    // write relu(output) to y instead of the output; false if the operation cannot
     virtual bool foldRelu(const std::shared_ptr<HipTensor> &y) { return false; }
     // do without what was folded in last, and write what was the output before
     virtual void unfold() {}
@@ -213,12 +213,17 @@ struct HipOperation {
 
     // inputs plus the outputs that are accumulated into
     HipOpArgs getInputs();
-    HipOpArgs getOutputs() const { return listOutputs(); }
+    HipOpArgs getOutputs() const;
+    // exec() and what was folded into it once and is not any more
+    void run(HipProgram &p);
     std::string str();
     void dump(FILE *out, bool full);
     const std::string &name() const { return m_kind; }
 
     std::string m_kind;
+    // training: operations that this one did along until somebody looked at what is between them, in their order.  They stay at its
+    // place in the list, whose indices the plan of the two streams holds.
+    HipOps m_behind;
 };
 
 struct HipProgram;

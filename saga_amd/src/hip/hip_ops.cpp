@@ -229,7 +229,7 @@ struct ConvFwd : public HipOperation {
     T bn_s_, bn_b_, bn_m_, bn_v_, bn_z_, bn_y_;
     float bn_eps_ = 0;
     int bn_flags_ = 0;
-    // the layer's bias, and (inference) the tensor of a relu behind it
+    // the layer's bias, and the tensor of a relu behind it
     const T b_;
     T relu_y_;
     T packed_; // the filter as the kernel loads it
@@ -721,10 +721,14 @@ struct ActBwd : public HipOperation {
     }
     void exec(HipProgram &p) override
     {
-        const SagaTensorView vx = x_->view(), vy = y_->view(), vdy = dy_->view(), vdx = dx_->view();
+        // (a relu's output is positive where its input is, and then nobody but the relu has to read that)
+        const SagaTensorView vy = y_->view(), vx = mode_ == SAGA_ACT_RELU ? vy : x_->view(), vdy = dy_->view(), vdx = dx_->view();
         chkSaga(saga_hip_act_bwd(mode_, alpha_, &vx, &vy, &vdy, &vdx, beta_, S(p)));
     }
-    HipOpArgs listInputs() const override { return {{"x", x_}, {"y", y_}, {"dy", dy_}}; }
+    HipOpArgs listInputs() const override
+    {
+        return mode_ == SAGA_ACT_RELU ? HipOpArgs{{"y", y_}, {"dy", dy_}} : HipOpArgs{{"x", x_}, {"y", y_}, {"dy", dy_}};
+    }
     HipOpArgs listOutputs() const override { return {{"dx", dx_}}; }
     float *getBeta(const T &t) override { return t == dx_ ? &beta_ : nullptr; }
     double bytes() const override { return (beta_ != 0 ? 4 : 3) * nbytes(dx_); }
@@ -765,7 +769,8 @@ struct Gemm : public HipOperation {
     const T a_, b_, c_;
     const int lda_, ldb_, ldc_;
     const T bias_; // per column
-    T relu_c_;     // inference: the tensor of a relu behind it
+    T relu_c_;     // the tensor of a relu behind it, or the gradient of the input of one
+    T gate_;       // in the latter case: the relu's output
     float beta_ = 0;
     Gemm(int ta, int tb, int m, int n, int k, T a, int lda, T b, int ldb, T c, int ldc, const char *name, T bias = nullptr)
       : HipOperation(name), ta_(ta), tb_(tb), m_(m), n_(n), k_(k), a_(a), b_(b), c_(c), lda_(lda), ldb_(ldb), ldc_(ldc), bias_(bias)
@@ -777,6 +782,11 @@ struct Gemm : public HipOperation {
     }
     void exec(HipProgram &p) override
     {
+        if(gate_) {
+            chkSaga(saga_hip_gemm_relu_bwd(ta_, tb_, m_, n_, k_, 1.0f, a_->deviceMem(), lda_, b_->deviceMem(), ldb_, relu_c_->deviceMem(),
+                                           ldc_, (int)a_->m_data_type, gate_->deviceMem(), S(p)));
+            return;
+        }
         chkSaga(saga_hip_gemm_bias(ta_, tb_, m_, n_, k_, 1.0f, a_->deviceMem(), lda_, b_->deviceMem(), ldb_, beta_,
                                    (relu_c_ ? relu_c_ : c_)->deviceMem(), ldc_, (int)a_->m_data_type,
                                    bias_ ? bias_->deviceMem() : nullptr, bias_ ? (int)bias_->m_data_type : SAGA_FLOAT,
@@ -789,13 +799,25 @@ struct Gemm : public HipOperation {
         relu_c_ = y;
         return true;
     }
-    void unfold() override { relu_c_ = nullptr; }
+    // the gradient of the input of a relu whose output y is
+    bool foldReluBwd(const T &y, const T &dx)
+    {
+        if(relu_c_ || bias_ || !y->rowMajor() || !dx->rowMajor() || y->m_data_type != a_->m_data_type || dx->m_data_type != a_->m_data_type ||
+           !saga_hip_gemm_relu_bwd_ok(m_, n_, k_, (int)a_->m_data_type))
+            return false;
+        gate_ = y;
+        relu_c_ = dx;
+        return true;
+    }
+    void unfold() override { relu_c_ = gate_ = nullptr; }
     bool sideSafe() const override { return true; }
     HipOpArgs listInputs() const override
     {
         HipOpArgs r{{"a", a_}, {"b", b_}};
         if(bias_)
             r.push_back({"bias", bias_});
+        if(gate_)
+            r.push_back({"y", gate_});
         return r;
     }
     HipOpArgs listOutputs() const override { return {{"c", relu_c_ ? relu_c_ : c_}}; }
@@ -1486,7 +1508,7 @@ struct PoolFwd : public HipOperation {
         chkSaga(saga_hip_pool_fwd(mode_, &vx, &vr, nullptr, size_, pad_, stride_, S(p)));
         chkSaga(saga_hip_act_fwd(SAGA_ACT_RELU, 0, &vr, &vr, 0.0f, S(p)));
     }
-    T relu_y_; // inference: the tensor of a relu behind it
+    T relu_y_; // the tensor of a relu behind it
     bool foldRelu(const T &y) override
     {
         if(relu_y_)
@@ -1511,12 +1533,37 @@ struct PoolBwd : public HipOperation {
     }
     void exec(HipProgram &p) override
     {
-        const SagaTensorView vx = x_->view(), vy = y_->view(), vdy = dy_->view(), vdx = dx_->view();
+        const SagaTensorView vx = x_->view(), vy = y_->view(), vdy = dy_->view();
+        if(relu_dx_) {
+            const SagaTensorView vr = relu_dx_->view();
+            const int r = saga_hip_maxpool_bwd_relu(&vx, &vy, &vdy, &vr, size_, pad_, stride_, S(p));
+            if(r == 0)
+                return;
+            if(r != SAGA_HIP_EUNSUPPORTED)
+                chkSaga(r);
+        }
+        const SagaTensorView vdx = dx_->view();
         chkSaga(saga_hip_pool_bwd(mode_, &vx, &vy, &vdy, &vdx, size_, pad_, stride_, beta_, S(p)));
+        if(relu_dx_) {
+            const SagaTensorView vr = relu_dx_->view();
+            chkSaga(saga_hip_act_bwd(SAGA_ACT_RELU, 0, &vx, &vx, &vdx, &vr, 0.0f, S(p)));
+        }
     }
+    T relu_dx_; // the gradient of the input of a relu whose output x is
+    bool foldReluBwd(const T &y, const T &dx)
+    {
+        if(relu_dx_ || mode_ != SAGA_POOL_MAX || y != x_)
+            return false;
+        const SagaTensorView vx = x_->shapeView(), vy = y_->shapeView(), vdy = dy_->shapeView(), vdx = dx->shapeView();
+        if(!saga_hip_maxpool_bwd_relu_ok(&vx, &vy, &vdy, &vdx, size_, pad_, stride_))
+            return false;
+        relu_dx_ = dx;
+        return true;
+    }
+    void unfold() override { relu_dx_ = nullptr; }
     HipOpArgs listInputs() const override { return {{"x", x_}, {"y", y_}, {"dy", dy_}}; }
-    HipOpArgs listOutputs() const override { return {{"dx", dx_}}; }
-    float *getBeta(const T &t) override { return t == dx_ ? &beta_ : nullptr; }
+    HipOpArgs listOutputs() const override { return {{"dx", relu_dx_ ? relu_dx_ : dx_}}; }
+    float *getBeta(const T &t) override { return !relu_dx_ && t == dx_ ? &beta_ : nullptr; }
     double bytes() const override
     {
         return nbytes(dx_) + nbytes(dy_) + (mode_ == SAGA_POOL_MAX ? nbytes(x_) + nbytes(y_) : 0);
@@ -2087,9 +2134,14 @@ REGISTER_HIP_TRANSFORM(100, ProgramType::INFERENCE | ProgramType::TRAINING, conc
 // the two in a network's stem becomes part of the operation that writes its input, which then writes the result in place of that input.  Nobody else may see the input:
 // no other operation, not the host, no other program.  What the folded operation reads and writes is touched at the
 // producer's place in the list from then on, so nothing in between may write the one or touch the other.
+//
+// In training programs that goes for relus, whose backward reads their output, and for a relu's backward behind that of a max
+// pooling or a product which read its output: launches that move a tensor twice to change its signs (64 samples of 32x28x28 fp32: 5 us each way).
+// (The anomaly checks look at every tensor.)
 void fold_into_producers(HipProgram &p, HipOps &ops)
 {
-    if(p.m_pt != ProgramType::INFERENCE || p.m_pc.disable_op_fusing)
+    const bool training = p.m_pt == ProgramType::TRAINING;
+    if(p.m_pc.disable_op_fusing || (training && p.m_pc.anomaly_detect))
         return;
     auto touches = [](const HipOpArgs &args, const HipStorage *s) {
         return std::count_if(args.begin(), args.end(), [&](const auto &a) { return a.second->m_storage.get() == s; });
@@ -2105,9 +2157,10 @@ void fold_into_producers(HipProgram &p, HipOps &ops)
         const auto *norm = dynamic_cast<BnInference *>(next.get());
         const auto *act = dynamic_cast<ActFwd *>(next.get());
         const auto *pool = dynamic_cast<PoolFwd *>(next.get());
-        if(!norm && !pool && !(act && act->mode_ == SAGA_ACT_RELU))
+        const auto *back = dynamic_cast<ActBwd *>(next.get());
+        if(!(norm && !training) && !(pool && !training) && !(act && act->mode_ == SAGA_ACT_RELU) && !(back && back->mode_ == SAGA_ACT_RELU))
             continue;
-        const T x = norm ? norm->x_ : pool ? pool->x_ : act->x_, y = norm ? norm->y_ : pool ? pool->y_ : act->y_;
+        const T x = norm ? norm->x_ : pool ? pool->x_ : act ? act->x_ : back->dy_, y = norm ? norm->y_ : pool ? pool->y_ : act ? act->y_ : back->dx_;
         const HipStorage *xs = x->m_storage.get(), *ys = y->m_storage.get();
         if(seen_elsewhere.count(x->m_storage.get()) || xs->doubleBuffered())
             continue;
@@ -2132,8 +2185,11 @@ void fold_into_producers(HipProgram &p, HipOps &ops)
             clean &= !touches(in, ys) && !touches(out, ys);
         }
         auto *conv = dynamic_cast<ConvFwd *>(ops[i].get());
+        auto *pool_bwd = dynamic_cast<PoolBwd *>(ops[i].get());
+        auto *product = dynamic_cast<Gemm *>(ops[i].get());
         if(!clean || !(norm   ? conv && conv->foldBn(norm->s_, norm->b_, norm->m_, norm->v_, norm->z_, y, norm->eps_, norm->flags_)
                        : pool ? conv && conv->foldPool(pool->mode_, y, pool->size_, pool->pad_, pool->stride_)
+                       : back ? (pool_bwd && pool_bwd->foldReluBwd(back->y_, y)) || (product && product->foldReluBwd(back->y_, y))
                               : ops[i]->foldRelu(y)))
             continue;
         p.m_folded.push_back({ops[i], next, x->m_storage});

@@ -73,7 +73,33 @@ HipOpArgs HipOperation::getInputs()
         if(beta && *beta != 0.0f)
             r.push_back(o);
     }
+    std::set<HipStorage *> own;
+    for(const auto &o : listOutputs())
+        own.insert(o.second->m_storage.get());
+    for(const auto &op : m_behind) {
+        for(const auto &i : op->getInputs())
+            if(!own.count(i.second->m_storage.get()))
+                r.push_back(i);
+        for(const auto &o : op->listOutputs())
+            own.insert(o.second->m_storage.get());
+    }
     return r;
+}
+
+HipOpArgs HipOperation::getOutputs() const
+{
+    HipOpArgs r = listOutputs();
+    for(const auto &op : m_behind)
+        for(const auto &o : op->listOutputs())
+            r.push_back(o);
+    return r;
+}
+
+void HipOperation::run(HipProgram &p)
+{
+    exec(p);
+    for(const auto &op : m_behind)
+        op->exec(p);
 }
 
 std::string HipOperation::str()
@@ -640,10 +666,14 @@ bool HipProgram::unfold(HipStorage *s)
                 continue;
             const size_t i = it - m_ops.begin();
             producer->unfold();
-            m_ops.insert(it + 1, fold.op);
-            if(m_poison_before.size() + 1 == m_ops.size()) {
-                m_poison_before.insert(m_poison_before.begin() + i + 1, std::vector<HipStorage *>());
-                m_poison_after.insert(m_poison_after.begin() + i, std::vector<HipStorage *>());
+            if(m_pt == ProgramType::TRAINING) {
+                producer->m_behind.insert(producer->m_behind.begin(), fold.op);
+            } else {
+                m_ops.insert(it + 1, fold.op);
+                if(m_poison_before.size() + 1 == m_ops.size()) {
+                    m_poison_before.insert(m_poison_before.begin() + i + 1, std::vector<HipStorage *>());
+                    m_poison_after.insert(m_poison_after.begin() + i, std::vector<HipStorage *>());
+                }
             }
             m_written.push_back(fold.between.get());
             dropGraphs();
@@ -924,7 +954,7 @@ void HipProgram::runOpsGraphed()
         }
         std::set<HipStorage *> seen;
         for(auto &op : m_ops)
-            for(const auto &list : {op->listInputs(), op->listOutputs()})
+            for(const auto &list : {op->getInputs(), op->getOutputs()})
                 for(const auto &t : list) {
                     HipStorage *st = t.second->m_storage.get();
                     if(st->doubleBuffered() && seen.insert(st).second)
@@ -934,7 +964,7 @@ void HipProgram::runOpsGraphed()
     if(m_graph_dbufs.size() > 16) { // one recording per combination of front buffers: keep that bounded
         for(auto &op : m_ops) {
             try {
-                op->exec(*this);
+                op->run(*this);
             } catch(const std::exception &ex) {
                 throw std::runtime_error(fmt("Op %s failed -- %s", op->name().c_str(), ex.what()));
             }
@@ -953,7 +983,7 @@ void HipProgram::runOpsGraphed()
     auto exec_range = [&](size_t b, size_t e) {
         for(size_t i = b; i < e; i++) {
             try {
-                m_ops[i]->exec(*this);
+                m_ops[i]->run(*this);
             } catch(const std::exception &ex) {
                 throw std::runtime_error(fmt("Op %s failed -- %s", m_ops[i]->name().c_str(), ex.what()));
             }
@@ -1185,7 +1215,7 @@ void HipProgram::runOps(const HipOps &ops)
             m_on_side = true;
         }
         try {
-            op->exec(*this);
+            op->run(*this);
         } catch(const std::exception &e) {
             m_on_side = false;
             if(two_streams)
