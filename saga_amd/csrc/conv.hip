@@ -307,6 +307,46 @@ int saga_hip_conv2d_fwd_bn_maxpool(const SagaTensorView *x, const SagaTensorView
     return conv_bn_maxpool(x, w, y, g, s, b, m, v, eps, pool_size, pool_pad, pool_stride, as_stream(stream));
 }
 
+// what follows the convolution, for a kernel that does a max pooling behind it; false: not that
+static bool pooled_epilogue(const SagaTensorView *y, const SagaConvExtras *e, StreamEpilogue *se)
+{
+    if(!e || e->z || (e->s && (!e->b || !e->m || !e->v || e->bias)) || (e->bias && (check_bias(e->bias, y) || !fuses(e->bias, SAGA_FLOAT))))
+        return false;
+    se->bias = e->bias ? (const float *)e->bias->ptr : nullptr;
+    se->bn_s = e->s, se->bn_b = e->b, se->bn_m = e->m, se->bn_v = e->v;
+    se->bn_eps = e->eps;
+    se->relu = e->relu;
+    return true;
+}
+
+static bool pools_twos(const SagaTensorView *y, const ConvGeom &g, int size, int pad, int stride)
+{
+    return size == 2 && pad == 0 && stride == 2 && y->dims[0] == g.N && y->dims[1] == g.K && y->dims[2] == g.P / 2 && y->dims[3] == g.Q / 2;
+}
+
+int saga_hip_conv2d_fwd_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
+                                   const SagaConvExtras *e, int pool_size, int pool_pad, int pool_stride)
+{
+    ConvGeom g;
+    StreamEpilogue se;
+    return !force_direct() && !pooled_geometry(x, w, y, p, &g) && pools_twos(y, g, pool_size, pool_pad, pool_stride) &&
+           pooled_epilogue(y, e, &se) && conv_f32_maxpool_ok(x, w, y, g, e->packed != nullptr);
+}
+
+int saga_hip_conv2d_fwd_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
+                                const SagaConvExtras *e, int pool_size, int pool_pad, int pool_stride, void *workspace, size_t ws_bytes,
+                                saga_stream_t stream)
+{
+    ConvGeom g;
+    StreamEpilogue se;
+    const int r = pooled_geometry(x, w, y, p, &g);
+    if(r)
+        return r;
+    if(force_direct() || !pools_twos(y, g, pool_size, pool_pad, pool_stride) || !pooled_epilogue(y, e, &se))
+        return SAGA_HIP_EUNSUPPORTED;
+    return conv_f32_maxpool(x, w, y, g, workspace, ws_bytes, se, e->packed, as_stream(stream));
+}
+
 int saga_hip_conv2d_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx,
                              const SagaConvParams *p, float alpha, float beta, void *workspace, size_t ws_bytes,
                              saga_stream_t stream)

@@ -83,6 +83,10 @@ struct StreamEpilogue {
 int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, float alpha,
                  float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue(),
                  const void *packed = nullptr);
+// and a max pooling of 2x2 windows, whose output y is, in the same launch; packed: there is a packed filter
+bool conv_f32_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, bool packed);
+int conv_f32_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, void *ws, size_t ws_bytes,
+                     const StreamEpilogue &e, const void *packed, hipStream_t st);
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
                       float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e = StreamEpilogue(),
                       const void *packed = nullptr);

@@ -1180,6 +1180,20 @@ int conv_f32_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTen
     return gather_launch(false, x, w, y, g, alpha, beta, e, packed, ws, ws_bytes, st);
 }
 
+bool conv_f32_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, bool packed)
+{
+    return f32_ok(x, w, y, g) && (thin_f32_maxpool_ok(x, w, y, g) || stream_f32_windows(false, x, y, g, packed, ~(size_t)0, true));
+}
+
+int conv_f32_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, void *ws, size_t ws_bytes,
+                     const StreamEpilogue &e, const void *packed, hipStream_t st)
+{
+    if(!f32_ok(x, w, y, g))
+        return SAGA_HIP_EUNSUPPORTED;
+    const int r = thin_f32_conv(x, w, y, g, 1.0f, 0.0f, e, st, true);
+    return r != SAGA_HIP_EUNSUPPORTED ? r : stream_f32_conv(false, x, w, y, g, 1.0f, 0.0f, e, packed, ws, ws_bytes, st, true);
+}
+
 int conv_f32_bwd_data(const SagaTensorView *dy, const SagaTensorView *w, const SagaTensorView *dx, const ConvGeom &g,
                       float alpha, float beta, void *ws, size_t ws_bytes, hipStream_t st, const StreamEpilogue &e, const void *packed)
 {

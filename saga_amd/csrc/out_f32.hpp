@@ -63,9 +63,24 @@ struct Four {
     float v[4];
 };
 
+// Pixel m of a convolution's output: rows one after the other, or, POOL, the 2x2 windows of a max pooling (ow and oh count those), four
+// neighbouring lanes each in the order in which they are compared.
+template <bool POOL> __device__ __forceinline__ void place_pixel(const FastDiv &ow, const FastDiv &oh, int m, int &n, int &oy, int &ox)
+{
+    const int at = POOL ? m >> 2 : m, t = ow.div(at);
+    ox = at - t * (int)ow.d;
+    n = oh.div(t);
+    oy = t - n * (int)oh.d;
+    if(POOL) {
+        ox = 2 * ox + (m & 1);
+        oy = 2 * oy + ((m >> 1) & 1);
+    }
+}
+
 // Everything per lane is in the vector offset, everything per value in the scalar one; a pixel or a channel that is not
-// there gets an offset behind the buffer.  EX: there is something to add to the values or to apply to them.
-template <bool EX> struct FourOut {
+// there gets an offset behind the buffer.  EX: there is something to add to the values or to apply to them.  POOL: the largest of a window's
+// four goes out, in the place of its four pixels; the lanes of a window exchange them and store one channel each.
+template <bool EX, bool POOL = false> struct FourOut {
     const OutArgs &g;
     __amdgpu_buffer_rsrc_t ro, rz;
     unsigned osc4, zsc4;
@@ -80,7 +95,23 @@ template <bool EX> struct FourOut {
     }
     __device__ __forceinline__ unsigned out_at(bool ok, int n, int y, int x) const
     {
+        if constexpr(POOL)
+            return ok ? (unsigned)((n * g.o_sn + (y >> 1) * g.o_sh + (x >> 1) * g.o_sw + (4 * fk + (threadIdx.x & 3)) * g.o_sc) * 4) : OUT_NOWHERE;
         return ok ? (unsigned)((n * g.o_sn + y * g.o_sh + x * g.o_sw + 4 * fk * g.o_sc) * 4) : OUT_NOWHERE;
+    }
+    // of the window of four lanes, which run along it (the rule of the pooling kernels: what is not at most the largest so far, and a
+    // NaN stays)
+    __device__ __forceinline__ static float largest(float x)
+    {
+        const int i = __builtin_bit_cast(int, x);
+        float most = __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, 0x00, 0xf, 0xf, true));
+        const float others[3] = {__builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, 0x55, 0xf, 0xf, true)),
+                                 __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, 0xaa, 0xf, 0xf, true)),
+                                 __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, i, 0xff, 0xf, 0xf, true))};
+#pragma unroll
+        for(int k = 0; k < 3; k++)
+            most = !(others[k] <= most) && most == most ? others[k] : most;
+        return most;
     }
     __device__ __forceinline__ unsigned z_at(bool ok, int n, int y, int x) const
     {
@@ -106,6 +137,18 @@ template <bool EX> struct FourOut {
         if(EX && g.e.affine()) {
             scale = *(const float4_t *)chan_scale;
             shift = *(const float4_t *)chan_shift;
+        }
+        if constexpr(POOL) {
+            const int e = threadIdx.x & 3;
+            float own = 0.0f;
+#pragma unroll
+            for(int j = 0; j < 4; j++) {
+                const float most = largest(g.e.apply(val.v[j] * g.alpha, scale[j], shift[j], 0.0f));
+                own = e == j ? most : own;
+            }
+            __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, own), ro, n + 4 * fk + e < g.N ? pos : OUT_NOWHERE,
+                                                  n < g.N ? n * osc4 : 0, 0);
+            return;
         }
 #pragma unroll
         for(int j = 0; j < 4; j++) {

@@ -803,7 +803,7 @@ int stream_f32_pack(const SagaFilterPackJob *jobs, int njobs, int blocks, hipStr
     return 0;
 }
 
-bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room)
+bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room, bool pool)
 {
     Args k = {};
     const long long bytes = extent(a);
@@ -811,7 +811,7 @@ bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView 
         return false;
     k.p_bytes = (unsigned)bytes;
     const size_t need = packed_size(bwd, g, k, true);
-    return need && (packed ? for_windows(bwd, g, k) : pays(bwd, g) && room >= need) && window_f32_takes(window_of(k), a, out);
+    return need && (packed ? for_windows(bwd, g, k) : pays(bwd, g) && room >= need) && window_f32_takes(window_of(k), a, out, pool);
 }
 
 size_t stream_f32_conv_workspace(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g)
@@ -825,7 +825,7 @@ size_t stream_f32_conv_workspace(bool bwd, const SagaTensorView *a, const SagaTe
 }
 
 int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g,
-                    float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st)
+                    float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st, bool pool)
 {
     Args k = {};
     const long long pe = extent(a), qe = extent(w);
@@ -869,14 +869,18 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
             k.q_bytes = (unsigned)bytes;
             return bytes;
         };
-        if(stream_f32_windows(bwd, a, out, g, packed != nullptr, room)) {
+        if(stream_f32_windows(bwd, a, out, g, packed != nullptr, room, pool)) {
             const Args before = k;
             const size_t bytes = from(true);
-            const int r = window_f32_conv(window_of(k), a, out, alpha, beta, e, k.q, bytes, st);
+            const int r = window_f32_conv(window_of(k), a, out, alpha, beta, e, k.q, bytes, pool, st);
+            if(pool)
+                return r;
             if(r != SAGA_HIP_EUNSUPPORTED || packed)
                 return r == SAGA_HIP_EUNSUPPORTED ? launch<PTAP, QSPLIT>(k, st, pixels, steps) : r;
             k = before; // (an output out of its reach)
         }
+        if(pool)
+            return SAGA_HIP_EUNSUPPORTED;
         if(packed && packed_size(bwd, g, k, for_windows(bwd, g, k))) {
             const bool parts = for_windows(bwd, g, k);
             from(parts);
@@ -894,7 +898,7 @@ int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, 
         if(in_place(bwd, g) && bwd && k.q_sn == 1)
             return launch<PTAP, QCOL>(k, st, pixels, steps);
     }
-    if(taps <= 63 && (long long)taps * k.C <= MAX_TABLE - 8)
+    if(!pool && taps <= 63 && (long long)taps * k.C <= MAX_TABLE - 8)
         return launch<PTAB, QTAB>(k, st, pixels, steps);
     return SAGA_HIP_EUNSUPPORTED;
 }

@@ -54,9 +54,11 @@ inline EpilogueF32 epilogue_f32(const StreamEpilogue &e)
 size_t stream_f32_conv_workspace(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g);
 // a: x or dy, out: y or dx; packed (may be null): what stream_f32_pack left, otherwise packed into ws where needed.  SAGA_HIP_EUNSUPPORTED (nothing enqueued) outside what the kernel covers.
 int stream_f32_conv(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g,
-                    float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st);
+                    float alpha, float beta, const StreamEpilogue &e, const void *packed, void *ws, size_t ws_bytes, hipStream_t st,
+                    bool pool = false); // pool: and a max pooling of 2x2 windows, whose output `out` is, where windows (below) do that
 // whether a convolution is done in windows (window_f32.hip), of a filter packed beforehand or with that much workspace to pack it
-bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room);
+bool stream_f32_windows(bool bwd, const SagaTensorView *a, const SagaTensorView *out, const ConvGeom &g, bool packed, size_t room,
+                        bool pool = false);
 // the filter in the order that the kernel loads it: bytes (0: not for this convolution), jobs (at most 16), launch
 size_t stream_f32_packed_bytes(bool bwd, const SagaTensorView *a, const SagaTensorView *w, const SagaTensorView *out, const ConvGeom &g);
 int stream_f32_pack_jobs(bool bwd, const SagaTensorView *w, const ConvGeom &g, void *packed, SagaFilterPackJob *jobs);

@@ -33,7 +33,9 @@ struct ThinArgs {
     OutArgs o;
 };
 
-template <int TN, int WAVES, bool EX> __global__ void __launch_bounds__(64 * WAVES, 2) stream_f32_k_thin(ThinArgs g)
+// POOL: a max pooling of 2x2 windows behind it (out_f32.hpp): a quarter of the results to store, and none to read again.  us, both launches / this:
+// 5x5 1->32 at 64x28x28 15.1 / 8.7, at 512x28x28 43 / 25; 3x3 3->64 at 8x224x224 86 / 54.
+template <int TN, int WAVES, bool EX, bool POOL> __global__ void __launch_bounds__(64 * WAVES, 2) stream_f32_k_thin(ThinArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
     __shared__ __attribute__((aligned(16))) int at_tap[MOST], w_at[MOST]; // of a reduction index: in the window; in the filter (bytes)
@@ -56,12 +58,7 @@ template <int TN, int WAVES, bool EX> __global__ void __launch_bounds__(64 * WAV
         at_tap[tid] = in ? c * g.window + r * g.dil * g.pitch + s * g.dil : 0; // (behind the last the filter is zero)
         w_at[tid] = in ? (int)((c * g.w_sc + r * g.w_sr + s * g.w_ss) * 4) : -1;
     }
-    auto place = [&](int m, int &n, int &oy, int &ox) {
-        const int t = g.ow.div(m);
-        ox = m - t * (int)g.ow.d;
-        n = g.oh.div(t);
-        oy = t - n * (int)g.oh.d;
-    };
+    auto place = [&](int m, int &n, int &oy, int &ox) { place_pixel<POOL>(g.ow, g.oh, m, n, oy, ox); };
     auto virt = [&](int n, int oy, int ox) { return n * g.plane + oy * g.stride * g.pitch + ox * g.stride; };
     auto load_window = [&](int tile) {
         int n, oy, ox;
@@ -211,7 +208,7 @@ template <int TN, int WAVES, bool EX> __global__ void __launch_bounds__(64 * WAV
                 }
             }
         }
-        const FourOut<EX> out(g.o, fk);
+        const FourOut<EX, POOL> out(g.o, fk);
         int first = n0;
         asm volatile("" : "+s"(first)); // (or every value's scalar offset is kept from one tile to the next)
 #pragma unroll
@@ -234,9 +231,9 @@ template <int TN, int WAVES, bool EX> __global__ void __launch_bounds__(64 * WAV
     }
 }
 
-template <int TN, int WAVES, bool EX> int launch(const ThinArgs &g, size_t bytes, hipStream_t st)
+template <int TN, int WAVES, bool EX, bool POOL = false> int launch(const ThinArgs &g, size_t bytes, hipStream_t st)
 {
-    auto kern = stream_f32_k_thin<TN, WAVES, EX>;
+    auto kern = stream_f32_k_thin<TN, WAVES, EX, POOL>;
     static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS_ROOM);
     if(attr != hipSuccess)
         return (int)attr;
@@ -247,15 +244,23 @@ template <int TN, int WAVES, bool EX> int launch(const ThinArgs &g, size_t bytes
 
 } // namespace
 
-int thin_f32_conv(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &c, float alpha,
-                  float beta, const StreamEpilogue &e, hipStream_t st)
+// what there is to launch: wavefronts of a block, channels of a block in 32s, its LDS
+struct Launch {
+    int waves, tn;
+    long long bytes;
+};
+
+static int describe(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &c, float alpha, float beta,
+                    const StreamEpilogue &e, bool pool, ThinArgs &g, Launch &l)
 {
-    ThinArgs g = {};
     const long long xb = extent_of(x), wb = extent_of(w);
     if(c.C > 4 || c.group != 1 || (long long)c.C * c.R * c.S > MOST || xb < 0 || wb < 0 || xb > OUT_NOWHERE || wb > OUT_NOWHERE ||
        !describe_out(y, alpha, beta, e, g.o))
         return SAGA_HIP_EUNSUPPORTED;
-    const long long pixels = (long long)c.N * c.P * c.Q, pitch = c.W + 2ll * c.pad, plane = pitch * (c.H + 2ll * c.pad);
+    if(pool && (beta != 0.0f || e.z || c.P < 2 || c.Q < 2))
+        return SAGA_HIP_EUNSUPPORTED;
+    const int P = pool ? c.P / 2 : c.P, Q = pool ? c.Q / 2 : c.Q; // (of windows)
+    const long long pixels = ((long long)c.N * P * Q) << (2 * pool), pitch = c.W + 2ll * c.pad, plane = pitch * (c.H + 2ll * c.pad);
     if(pixels >= 1ll << 30 || (c.N + 1) * plane >= 1ll << 30)
         return SAGA_HIP_EUNSUPPORTED;
     g.x = (const float *)x->ptr;
@@ -275,9 +280,15 @@ int thin_f32_conv(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
     // positions from the first pixel's first tap to the last one's last: rows skip what is right of the last pixel and stride - 1
     // rows, images what is below
     auto window_of = [&](long long count) {
+        const long long taps = (c.R - 1ll) * c.dil * pitch + (c.S - 1ll) * c.dil + 1;
+        if(pool) { // the same of windows of two rows and columns, the last one's last pixel a row below and a column beside its first
+            const long long n = count / 4 - 1, rows = (n + Q - 1) / Q, images = (n + (long long)P * Q - 1) / ((long long)P * Q);
+            return 2 * n * c.stride + rows * 2 * c.stride * (pitch - Q) + images * std::max(0ll, plane - 2ll * P * c.stride * pitch) +
+                   c.stride * (pitch + 1) + taps;
+        }
         const long long n = count - 1, rows = (n + c.Q - 1) / c.Q, images = (n + (long long)c.P * c.Q - 1) / ((long long)c.P * c.Q);
         const long long row = c.stride * (pitch - c.Q), image = plane - (long long)c.P * c.stride * pitch;
-        return n * c.stride + rows * std::max(0ll, row) + images * std::max(0ll, image) + (c.R - 1ll) * c.dil * pitch + (c.S - 1ll) * c.dil + 1;
+        return n * c.stride + rows * std::max(0ll, row) + images * std::max(0ll, image) + taps;
     };
     const int tn = g.o.N > 32 ? 2 : 1;
     auto bytes_of = [&](int waves) { return tn * g.steps * 3072ll + window_of(64 * waves) * c.C * 4; };
@@ -292,12 +303,38 @@ int thin_f32_conv(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
     g.tiles = (int)((pixels + 64 * waves - 1) / (64 * waves));
     g.nblk_n = (g.o.N + 32 * tn - 1) / (32 * tn);
     g.walkers = std::min(g.tiles, std::max(1, (bytes <= 75 * 1024 ? 512 : 256) / g.nblk_n));
-    g.ow = fast_div(c.Q);
-    g.oh = fast_div(c.P);
+    g.ow = fast_div(Q);
+    g.oh = fast_div(P);
     g.by_pitch = fast_div(g.pitch);
     g.by_plane = fast_div(g.plane);
     g.x_sn = x->strides[0]; g.x_sc = x->strides[1]; g.x_sh = x->strides[2]; g.x_sw = x->strides[3];
     g.w_sn = w->strides[0]; g.w_sc = w->strides[1]; g.w_sr = w->strides[2]; g.w_ss = w->strides[3];
+    l = {waves, tn, bytes};
+    return 0;
+}
+
+bool thin_f32_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &c)
+{
+    ThinArgs g = {};
+    Launch l;
+    return describe(x, w, y, c, 1.0f, 0.0f, StreamEpilogue(), true, g, l) == 0;
+}
+
+int thin_f32_conv(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &c, float alpha,
+                  float beta, const StreamEpilogue &e, hipStream_t st, bool pool)
+{
+    ThinArgs g = {};
+    Launch l;
+    const int r = describe(x, w, y, c, alpha, beta, e, pool, g, l);
+    if(r)
+        return r;
+    const int waves = l.waves, tn = l.tn;
+    const long long bytes = l.bytes;
+    if(pool) {
+        if(waves == 4)
+            return tn == 1 ? launch<1, 4, true, true>(g, (size_t)bytes, st) : launch<2, 4, true, true>(g, (size_t)bytes, st);
+        return tn == 1 ? launch<1, 8, true, true>(g, (size_t)bytes, st) : launch<2, 8, true, true>(g, (size_t)bytes, st);
+    }
     const bool ex = beta != 0.0f || e.bias || e.bn_s || e.z || e.relu;
     if(waves == 4) {
         if(tn == 1)

@@ -34,6 +34,7 @@ struct WinArgs {
     int M, C, T, Ts; // pixels, reduction channels, taps, taps of a row
     int IH, IW, iy0, ix0, istep, tstep;
     int plane4, quads, WM, WN, KS, nblk_q, blocks;
+    int pool; // 1: M counts the pixels of 2x2 windows, ow and oh the windows
     FastDiv ow, oh, blk;
     long long p_sn, p_sc;
     OutArgs o;
@@ -53,7 +54,8 @@ __host__ __device__ constexpr int window_pitch(int quads) { return quads + ((4 -
 constexpr int window_bytes(int quads, int kg) { return 3 * kg * 4 * window_pitch(quads) * 16; }
 
 // APART: one tap at a stride; the window is the positions of the block's pixels and nothing between them, loaded one by one.
-template <int TM, int DEPTH, int KG, int NR, int TAPS, bool APART, bool EX>
+// POOL: a max pooling of 2x2 windows behind it (one group; out_f32.hpp).
+template <int TM, int DEPTH, int KG, int NR, int TAPS, bool APART, bool EX, bool POOL>
 __global__ void __launch_bounds__(512) stream_f32_k_window(WinArgs g)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[];
@@ -99,12 +101,7 @@ __global__ void __launch_bounds__(512) stream_f32_k_window(WinArgs g)
     char *const win = lds + ks * 2 * half;
     const int last = m0 + 32 * TM * WM < g.M ? m0 + 32 * TM * WM - 1 : g.M - 1;
     const int dh = g.tstep * g.IW, dw = g.tstep;
-    auto place = [&](int m, int &n, int &oy, int &ox) {
-        const int t = g.ow.div(m);
-        ox = m - t * (int)g.ow.d;
-        n = g.oh.div(t);
-        oy = t - n * (int)g.oh.d;
-    };
+    auto place = [&](int m, int &n, int &oy, int &ox) { place_pixel<POOL>(g.ow, g.oh, m, n, oy, ox); };
     auto virt = [&](int n, int oy, int ox) { return n * g.plane4 + (oy * g.istep + g.iy0) * g.IW + ox * g.istep + g.ix0; };
     int n_a, y_a, x_a, n_z, y_z, x_z;
     place(m0, n_a, y_a, x_a);
@@ -296,7 +293,7 @@ __global__ void __launch_bounds__(512) stream_f32_k_window(WinArgs g)
     }
 
     // acc[i][v]: this lane's pixel i, channel nw + 8*(v/4) + 4*(lane/32) + v%4
-    const FourOut<EX> out(g.o, fk);
+    const FourOut<EX, POOL> out(g.o, fk);
     unsigned opos[TM], zpos[TM];
 #pragma unroll
     for(int i = 0; i < TM; i++) {
@@ -310,7 +307,7 @@ __global__ void __launch_bounds__(512) stream_f32_k_window(WinArgs g)
         out.store(pos, n, val, was, res, &chan[0][EX ? n - n0 + 4 * fk : 0], &chan[1][EX ? n - n0 + 4 * fk : 0]);
     };
     constexpr int NV = TM * 16;
-    if(KS == 1) {
+    if(POOL || KS == 1) {
         if(EX && g.o.e.affine())
             __syncthreads();
 #pragma unroll
@@ -361,18 +358,24 @@ int window_quads(const WinArgs &g, int Tr, int pixels)
 {
     if(g.T == 1 && g.istep > 1)
         return (pixels + 3) / 4 + 1;
-    const int OW = (int)g.ow.d, OH = (int)g.oh.d;
+    const int OW = (int)g.ow.d << g.pool, OH = (int)g.oh.d << g.pool;
     auto sees = [&](int count, int first, int n, int size) {
         const int reach = (n - 1) * g.tstep;
         return (count - 1) * g.istep + first + std::min(reach, 0) < size && first + std::max(reach, 0) >= 0;
     };
     if(!sees(OH, g.iy0, Tr, g.IH) || !sees(OW, g.ix0, g.Ts, g.IW))
         return 0;
+    const long long reach = (long long)(Tr - 1) * g.tstep * g.IW + (long long)(g.Ts - 1) * g.tstep;
+    if(g.pool) { // windows of two rows and columns; the last one's last pixel is a row below and a column beside its first
+        const long long n = pixels / 4 - 1, per = OW / 2, rows = (n + per - 1) / per, images = (n + per * (OH / 2) - 1) / (per * (OH / 2));
+        const long long most = 2 * n + rows * std::max(0ll, 2ll * g.IW - OW) + images * std::max(0ll, g.plane4 - (long long)OH * g.IW) + g.IW + 1 +
+                               std::llabs(reach) + 1;
+        return most <= 1024 ? (int)((most + 3) / 4 + 2) : 0;
+    }
     const long long px = pixels - 1, rows = (px + OW - 1) / OW, images = (px + (long long)OW * OH - 1) / ((long long)OW * OH);
     const long long row = (long long)g.istep * (g.IW - OW), image = g.plane4 - (long long)OH * g.istep * g.IW;
     const long long skip = (long long)(g.istep - 1) * g.IW; // rows between those of two rows of pixels
-    const long long taps = (long long)(Tr - 1) * g.tstep * g.IW + (long long)(g.Ts - 1) * g.tstep;
-    const long long most = px * g.istep + rows * (std::max(0ll, row) + skip) + images * std::max(0ll, image) + std::llabs(taps) + 1;
+    const long long most = px * g.istep + rows * (std::max(0ll, row) + skip) + images * std::max(0ll, image) + std::llabs(reach) + 1;
     return most <= 1024 ? (int)((most + 3) / 4 + 2) : 0;
 }
 
@@ -494,16 +497,21 @@ bool worth(const WinArgs &g, const Plan &p)
 Plan choose(const WinArgs &g, int Tr, int kg)
 {
     const Plan p = tiles_for(g, Tr, kg);
-    return p.quads && worth(g, p) ? p : Plan{};
+    return p.quads && worth(g, p) && !(g.pool && p.cf.ks > 1) ? p : Plan{};
 }
 
-bool describe(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, WinArgs &g)
+bool describe(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, bool pool, WinArgs &g)
 {
     const int taps = c.Tr * c.Ts, IH = a->dims[2], IW = a->dims[3];
-    if(!window_f32_may(c, a->dims[1], IH, IW, out->dims[2], out->dims[3]) ||
+    // A max pooling behind it: windows of two rows see more of the input, the more the longer its rows.  us, packing, convolution and pooling /
+    // packing and this: 5x5 32->64 at 64x14x14 22 / 17, at 512x14x14 80 / 67; 3x3 16->32 64x32x32 22 / 14, 64->64 32x56x56 63 / 54, 128->128
+    // 16x56x56 98 / 89, 256->256 8x28x28 56 / 52, 512->512 64x14x14 306 / 304; 128->128 3x90x90 56 / 58, 8x112x112 173 / 200.
+    if(pool && (taps == 1 || c.istep != 1 || IW > 64))
+        return false;
+    if(!window_f32_may(c, a->dims[1], IH, IW, out->dims[2] << pool, out->dims[3] << pool) ||
        (IW > 1 && a->strides[3] != 1) || (IH > 1 && a->strides[2] != IW))
         return false;
-    const long long pixels = (long long)out->dims[0] * out->dims[2] * out->dims[3];
+    const long long pixels = ((long long)out->dims[0] * out->dims[2] * out->dims[3]) << (2 * pool);
     const long long plane4 = ((long long)IH * IW + 3) / 4 * 4;
     if(pixels < 256 || pixels >= 1ll << 30 || (out->dims[0] + 1ll) * plane4 >= 1ll << 30)
         return false;
@@ -519,6 +527,7 @@ bool describe(const WindowConv &c, const SagaTensorView *a, const SagaTensorView
     g.ix0 = c.ix0;
     g.istep = c.istep;
     g.tstep = c.tstep;
+    g.pool = pool;
     g.M = (int)pixels;
     g.plane4 = (int)plane4;
     g.ow = fast_div(out->dims[3]);
@@ -530,11 +539,11 @@ bool describe(const WindowConv &c, const SagaTensorView *a, const SagaTensorView
 
 int slice_groups(int taps) { return taps == 1 ? 8 : 2; } // eights of channels; under one tap a slice of sixteen waits for memory longer than it works
 
-template <int KG, int TAPS, int DEPTH, bool APART, bool EX> int launch_as(const WinArgs &g, const Plan &p, hipStream_t st)
+template <int KG, int TAPS, int DEPTH, bool APART, bool EX, bool POOL = false> int launch_as(const WinArgs &g, const Plan &p, hipStream_t st)
 {
 #define GO(TM, NR)                                                                                                         \
     do {                                                                                                               \
-        auto kern = stream_f32_k_window<TM, DEPTH, KG, NR, TAPS, APART, EX>;                                                  \
+        auto kern = stream_f32_k_window<TM, DEPTH, KG, NR, TAPS, APART, EX, POOL>;                                                  \
         static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS); \
         if(attr != hipSuccess)                                                                                         \
             return (int)attr;                                                                                          \
@@ -591,17 +600,17 @@ bool window_f32_may(const WindowConv &c, int channels, int IH, int IW, int OH, i
     return false;
 }
 
-bool window_f32_takes(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out)
+bool window_f32_takes(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, bool pool)
 {
     WinArgs g = {};
-    return describe(c, a, out, g) && choose(g, c.Tr, slice_groups(g.T)).quads;
+    return describe(c, a, out, pool, g) && choose(g, c.Tr, slice_groups(g.T)).quads;
 }
 
 int window_f32_conv(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, float alpha, float beta,
-                    const StreamEpilogue &e, const void *packed, size_t packed_bytes, hipStream_t st)
+                    const StreamEpilogue &e, const void *packed, size_t packed_bytes, bool pool, hipStream_t st)
 {
     WinArgs g = {};
-    if(!describe(c, a, out, g) || !describe_out(out, alpha, beta, e, g.o))
+    if((pool && (beta != 0.0f || e.z)) || !describe(c, a, out, pool, g) || !describe_out(out, alpha, beta, e, g.o))
         return SAGA_HIP_EUNSUPPORTED;
     const Plan p = choose(g, c.Tr, slice_groups(g.T));
     if(!p.quads)
@@ -625,6 +634,8 @@ int window_f32_conv(const WindowConv &c, const SagaTensorView *a, const SagaTens
             return ex ? launch_as<8, 1, 4, true, true>(g, p, st) : launch_as<8, 1, 4, true, false>(g, p, st);
         return ex ? launch_as<8, 1, 4, false, true>(g, p, st) : launch_as<8, 1, 4, false, false>(g, p, st);
     }
+    if(pool)
+        return g.T == 9 ? launch_as<2, 9, 3, false, true, true>(g, p, st) : launch_as<2, 25, 5, false, true, true>(g, p, st);
     if(g.T == 9)
         return ex ? launch_as<2, 9, 3, false, true>(g, p, st) : launch_as<2, 9, 3, false, false>(g, p, st);
     return ex ? launch_as<2, 25, 5, false, true>(g, p, st) : launch_as<2, 25, 5, false, false>(g, p, st);

@@ -65,6 +65,8 @@ SIGNATURES = {
     "saga_hip_init": (_I, [_I, C.POINTER(C.c_int)]),
     "saga_hip_conv2d_workspace_size": (_SZ, [_I, _TV, _TV, _TV, C.POINTER(ConvParams)]),
     "saga_hip_conv2d_fwd": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), _F, _F, _VP, _SZ, _VP]),
+    "saga_hip_conv2d_fwd_maxpool_ok": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), C.POINTER(ConvExtras), _I, _I, _I]),
+    "saga_hip_conv2d_fwd_maxpool": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), C.POINTER(ConvExtras), _I, _I, _I, _VP, _SZ, _VP]),
     "saga_hip_conv2d_fwd_ex": (_I, [_TV, _TV, _TV, C.POINTER(ConvParams), _F, C.POINTER(ConvExtras), _VP, _SZ, _VP]),
     "saga_hip_conv2d_pack_bytes": (_SZ, [_I, _TV, _TV, _TV, C.POINTER(ConvParams)]),
     "saga_hip_conv2d_pack_jobs": (_I, [_I, _TV, _TV, _TV, C.POINTER(ConvParams), _VP, C.POINTER(FilterPackJob)]),

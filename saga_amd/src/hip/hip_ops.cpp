@@ -276,23 +276,35 @@ struct ConvFwd : public HipOperation {
     }
     bool foldPool(int mode, const T &y, int size, int pad, int stride)
     {
-        if(!bn_y_ || pool_y_ || bn_flags_ != SAGA_BN_RELU || mode != SAGA_POOL_MAX)
+        if(pool_y_ || mode != SAGA_POOL_MAX || y->m_data_type != x_->m_data_type)
             return false;
         const SagaTensorView vx = x_->shapeView(), vw = w_->shapeView(), vy = y->shapeView();
-        if(!saga_hip_conv2d_fwd_bn_maxpool_ok(&vx, &vw, &vy, &cp_, size, pad, stride))
+        if(x_->m_data_type == Tensor::DataType::FLOAT) {
+            const float *there = (const float *)256; // (nothing is allocated, and nothing read, to answer the question)
+            SagaConvExtras e = {};
+            SagaTensorView vb;
+            e.packed = packed_ ? there : nullptr;
+            if(bn_y_)
+                e.s = e.b = e.m = e.v = there;
+            else if(b_)
+                vb = b_->shapeView(), e.bias = &vb;
+            if(bn_z_ || !saga_hip_conv2d_fwd_maxpool_ok(&vx, &vw, &vy, &cp_, &e, size, pad, stride))
+                return false;
+        } else if(!bn_y_ || bn_flags_ != SAGA_BN_RELU || !saga_hip_conv2d_fwd_bn_maxpool_ok(&vx, &vw, &vy, &cp_, size, pad, stride)) {
             return false;
+        }
         pool_y_ = y;
         pool_size_ = size;
         pool_pad_ = pad;
         pool_stride_ = stride;
-        m_kind = "convfwd.bn.pool";
+        m_kind += ".pool";
         return true;
     }
     void unfold() override
     {
         if(pool_y_) {
             pool_y_ = nullptr;
-            m_kind = "convfwd.bn";
+            m_kind = bn_y_ ? "convfwd.bn" : "convfwd";
             return;
         }
         bn_s_ = bn_b_ = bn_m_ = bn_v_ = bn_z_ = bn_y_ = relu_y_ = nullptr;
@@ -307,16 +319,34 @@ struct ConvFwd : public HipOperation {
         relu_y_ = y;
         return true;
     }
+    // what goes into the launch (the views behind the pointers live where the caller says)
+    SagaConvExtras extras(SagaTensorView *bias, SagaTensorView *residual) const
+    {
+        SagaConvExtras e = {};
+        e.packed = packed_ ? packed_->deviceMem() : nullptr;
+        if(bn_y_) {
+            e.s = (const float *)bn_s_->deviceMem(), e.b = (const float *)bn_b_->deviceMem();
+            e.m = (const float *)bn_m_->deviceMem(), e.v = (const float *)bn_v_->deviceMem();
+            e.eps = bn_eps_;
+            e.relu = bn_flags_ & SAGA_BN_RELU ? 1 : 0;
+            if(bn_flags_ & SAGA_BN_ADD) {
+                *residual = bn_z_->view();
+                e.z = residual;
+            }
+        } else {
+            if(b_) {
+                *bias = b_->view();
+                e.bias = bias;
+            }
+            e.relu = relu_y_ ? 1 : 0;
+        }
+        return e;
+    }
     void execFolded(HipProgram &p)
     {
         const SagaTensorView vx = x_->view(), vw = w_->view(), vo = bn_y_->view();
-        SagaTensorView vz;
-        if(bn_z_)
-            vz = bn_z_->view();
-        const float *s = (const float *)bn_s_->deviceMem(), *b = (const float *)bn_b_->deviceMem();
-        const float *m = (const float *)bn_m_->deviceMem(), *v = (const float *)bn_v_->deviceMem();
-        const SagaConvExtras e = {packed_ ? packed_->deviceMem() : nullptr, nullptr, s, b, m, v, bn_eps_,
-                                  bn_flags_ & SAGA_BN_ADD ? &vz : nullptr, bn_flags_ & SAGA_BN_RELU ? 1 : 0};
+        SagaTensorView vb, vz;
+        const SagaConvExtras e = extras(&vb, &vz);
         const int r = saga_hip_conv2d_fwd_ex(&vx, &vw, &vo, &cp_, 0.0f, &e, p.workspace().ptr(), p.workspace().size(), S(p));
         if(r == 0)
             return;
@@ -326,11 +356,30 @@ struct ConvFwd : public HipOperation {
         const SagaTensorView vy = y_->view();
         chkSaga(saga_hip_conv2d_fwd(&vx, &vw, &vy, &cp_, 1.0f, 0.0f, p.workspace().ptr(),
                                     p.workspace().size(), S(p)));
-        chkSaga(saga_hip_bn_infer(&vy, bn_z_ ? &vz : nullptr, &vo, s, b, m, v, bn_eps_, bn_flags_, S(p)));
+        if(bn_z_)
+            vz = bn_z_->view();
+        chkSaga(saga_hip_bn_infer(&vy, bn_z_ ? &vz : nullptr, &vo, e.s, e.b, e.m, e.v, bn_eps_, bn_flags_, S(p)));
     }
     void execPooled(HipProgram &p)
     {
         const SagaTensorView vx = x_->view(), vw = w_->view(), vy = pool_y_->view();
+        if(x_->m_data_type == Tensor::DataType::FLOAT) {
+            SagaTensorView vb;
+            const SagaConvExtras e = extras(&vb, nullptr); // (no residual)
+            const int r = saga_hip_conv2d_fwd_maxpool(&vx, &vw, &vy, &cp_, &e, pool_size_, pool_pad_, pool_stride_, p.workspace().ptr(),
+                                                      p.workspace().size(), S(p));
+            if(r == 0)
+                return;
+            if(r != SAGA_HIP_EUNSUPPORTED)
+                chkSaga(r);
+            const T out = pool_y_;
+            pool_y_ = nullptr;
+            exec(p);
+            pool_y_ = out;
+            const SagaTensorView between = (bn_y_ ? bn_y_ : relu_y_ ? relu_y_ : y_)->view();
+            chkSaga(saga_hip_pool_fwd(SAGA_POOL_MAX, &between, &vy, nullptr, pool_size_, pool_pad_, pool_stride_, S(p)));
+            return;
+        }
         const int r = saga_hip_conv2d_fwd_bn_maxpool(&vx, &vw, &vy, &cp_, (const float *)bn_s_->deviceMem(),
                                                      (const float *)bn_b_->deviceMem(), (const float *)bn_m_->deviceMem(),
                                                      (const float *)bn_v_->deviceMem(), bn_eps_, pool_size_, pool_pad_,
@@ -352,10 +401,7 @@ struct ConvFwd : public HipOperation {
         const SagaTensorView vx = x_->view(), vw = w_->view(), vy = relu_y_ ? relu_y_->view() : y_->view();
         if(b_ || packed_) {
             SagaTensorView vb;
-            if(b_)
-                vb = b_->view();
-            const SagaConvExtras e = {packed_ ? packed_->deviceMem() : nullptr, b_ ? &vb : nullptr, nullptr, nullptr, nullptr,
-                                      nullptr, 0.0f, nullptr, relu_y_ ? 1 : 0};
+            const SagaConvExtras e = extras(&vb, nullptr);
             chkSaga(saga_hip_conv2d_fwd_ex(&vx, &vw, &vy, &cp_, beta_, &e, p.workspace().ptr(), p.workspace().size(), S(p)));
             return;
         }
@@ -2131,7 +2177,7 @@ REGISTER_HIP_TRANSFORM(100, ProgramType::INFERENCE | ProgramType::TRAINING, conc
 }  // namespace
 
 // Inference programs: a batch norm behind a convolution, a relu behind a convolution, product or pooling, or a max pooling behind
-// the two in a network's stem becomes part of the operation that writes its input, which then writes the result in place of that input.  Nobody else may see the input:
+// a convolution with these becomes part of the operation that writes its input, which then writes the result in place of that input.  Nobody else may see the input:
 // no other operation, not the host, no other program.  What the folded operation reads and writes is touched at the
 // producer's place in the list from then on, so nothing in between may write the one or touch the other.
 //
@@ -2163,6 +2209,12 @@ void fold_into_producers(HipProgram &p, HipOps &ops)
         const T x = norm ? norm->x_ : pool ? pool->x_ : act ? act->x_ : back->dy_, y = norm ? norm->y_ : pool ? pool->y_ : act ? act->y_ : back->dx_;
         const HipStorage *xs = x->m_storage.get(), *ys = y->m_storage.get();
         if(seen_elsewhere.count(x->m_storage.get()) || xs->doubleBuffered())
+            continue;
+        // (a relu behind a pooling is the pooling's: a convolution has one of its own)
+        if(pool && x->m_data_type == Tensor::DataType::FLOAT && std::any_of(ops.begin() + j, ops.end(), [&](const HipOp &op) {
+               const auto *behind = dynamic_cast<ActFwd *>(op.get());
+               return behind && behind->mode_ == SAGA_ACT_RELU && behind->x_ == y;
+           }))
             continue;
         size_t i = j;
         int count = 0;
