@@ -994,15 +994,14 @@ __global__ void __launch_bounds__(256)
 // (recomputed from the norm's input x as half(fma(x, sc, sh)) > 0, the forward's own expression), and goes
 // straight into the norm's backward: MODE 0 leaves per block and channel the sums of g and g * (x - mean),
 // MODE 1 writes dx = a * (g - k0 - (x - mean) * k1) (+ beta * dx).  The norm's output gradient never exists.
-// A block walks AG consecutive patch rows, so that there are few partial rows.
+// A block walks AG consecutive patch rows, so that there are few partial rows (bn_pool_rows_per_block).
 // blockIdx.z = sample, blockIdx.y = group of patch rows, threadIdx.x = channel vector, threadIdx.y (+ blockIdx.x) = b
-constexpr int BNPOOL_AG = 16; // patch rows per block (measured on the 112x112 stem: 1 row 579 us, 8 rows 450 us, 16 or 64 rows 430 us)
-template <typename T, int VN, int MODE, int AG>
+template <typename T, int VN, int MODE>
 __global__ void __launch_bounds__(256)
     bn_pool_bwd_3x3s2_k(const uint8_t *__restrict__ codes, DView dp, DView x, DView dx, int pad, int na,
                         const float *__restrict__ mean_, const float *__restrict__ s_, const float *__restrict__ invstd_,
                         const float *__restrict__ b_, int relu, const float *__restrict__ coef, float *__restrict__ partial,
-                        float beta)
+                        float beta, int AG)
 {
     __shared__ float red[MODE == 0 ? 256 * VN * 2 : 1];
     const int C = x.d[1], H = x.d[2], W = x.d[3], P = dp.d[2], Q = dp.d[3];
@@ -1554,8 +1553,8 @@ int saga_hip_maxpool_bwd_codes(const uint8_t *codes, const SagaTensorView *dy, c
 
 } // extern "C"
 
-// Shape of the fused launch: patches along rows in groups of BNPOOL_AG; returns the number of partial rows.
-static int64_t bn_pool_launch_shape(const SagaTensorView *x, int pad, dim3 &grid, dim3 &block, int *na_out, int ag = BNPOOL_AG)
+// Shape of the fused launch: patches along rows in groups of `ag`; returns the number of partial rows.
+static int64_t bn_pool_launch_shape(const SagaTensorView *x, int pad, dim3 &grid, dim3 &block, int *na_out, int ag)
 {
     const int vn = x->dtype == SAGA_HALF ? 8 : 4;
     const int na = (x->dims[2] + pad) / 2 + 1, nb = (x->dims[3] + pad) / 2 + 1;
@@ -1563,6 +1562,19 @@ static int64_t bn_pool_launch_shape(const SagaTensorView *x, int pad, dim3 &grid
     if(na_out)
         *na_out = na;
     return (int64_t)grid.x * grid.y * grid.z;
+}
+
+// Patch rows that a block walks, one trip to memory after the other: as many as leave two blocks per compute unit, sums not fewer than 4
+// (us, both passes and what is between them, 16 rows each / these: 8x64x64 100 / 32, 23x97x97 96 / 52, 16x128x128 96 / 66, 64x80x80 110 / 81;
+// 256x112x112, 16 rows anyway, 402, and 431 with 2 rows in the second pass, 486 in the first).
+static int bn_pool_rows_per_block(const SagaTensorView *x, int pad, bool apply)
+{
+    const int least = apply ? 1 : 4;
+    int ag = 16;
+    for(dim3 grid, block; ag > least; ag /= 2)
+        if(bn_pool_launch_shape(x, pad, grid, block, nullptr, ag) >= 512)
+            break;
+    return ag;
 }
 
 static bool bn_pool_ok(const SagaTensorView *x, const SagaTensorView *dp, const SagaTensorView *dx, int size, int pad, int stride)
@@ -1584,7 +1596,7 @@ size_t saga_hip_bn_bwd_pooled_workspace_size(const SagaTensorView *x, const Saga
     if(!x || !dp || !bn_pool_ok(x, dp, nullptr, size, pad, stride))
         return 0;
     dim3 grid, block;
-    const int64_t rows = bn_pool_launch_shape(x, pad, grid, block, nullptr);
+    const int64_t rows = bn_pool_launch_shape(x, pad, grid, block, nullptr, bn_pool_rows_per_block(x, pad, false));
     return ((size_t)rows * x->dims[1] * 2 + 3 * (size_t)x->dims[1] + 64) * sizeof(float);
 }
 
@@ -1605,9 +1617,11 @@ int saga_hip_bn_bwd_pooled(const SagaTensorView *x, const SagaTensorView *dp, co
     const size_t need = saga_hip_bn_bwd_pooled_workspace_size(x, dp, size, pad, stride);
     if(!workspace || ws_bytes < need)
         return SAGA_HIP_EWORKSPACE;
-    dim3 grid, block;
+    dim3 grid, grid1, block;
     int na = 0;
-    const int64_t rows = bn_pool_launch_shape(x, pad, grid, block, &na);
+    const int ag = bn_pool_rows_per_block(x, pad, false), ag1 = bn_pool_rows_per_block(x, pad, true);
+    const int64_t rows = bn_pool_launch_shape(x, pad, grid, block, &na, ag);
+    bn_pool_launch_shape(x, pad, grid1, block, &na, ag1);
     if(rows >= (1ll << 31))
         return SAGA_HIP_EUNSUPPORTED;
 
@@ -1618,13 +1632,13 @@ int saga_hip_bn_bwd_pooled(const SagaTensorView *x, const SagaTensorView *dp, co
     const double M = (double)x->dims[0] * x->dims[2] * x->dims[3];
 #define GO(T, VN)                                                                                                       \
     do {                                                                                                                \
-        bn_pool_bwd_3x3s2_k<T, VN, 0, BNPOOL_AG><<<grid, block, 0, st>>>(codes, dvp, dvx, dvdx, pad, na, save_mean, s,     \
-                                                                        save_invstd, b, relu, nullptr, partial, 0.0f); \
+        bn_pool_bwd_3x3s2_k<T, VN, 0><<<grid, block, 0, st>>>(codes, dvp, dvx, dvdx, pad, na, save_mean, s, save_invstd, b, relu,  \
+                                                             nullptr, partial, 0.0f, ag);                                 \
         const int rc = bn_launch_bwd_finalize(partial, (int)rows, s, save_invstd, ds, db, coef, M, C, beta_p, st);       \
         if(rc)                                                                                                          \
             return rc;                                                                                                  \
-        bn_pool_bwd_3x3s2_k<T, VN, 1, BNPOOL_AG><<<grid, block, 0, st>>>(codes, dvp, dvx, dvdx, pad, na, save_mean, s,           \
-                                                                  save_invstd, b, relu, coef, nullptr, beta_dx);        \
+        bn_pool_bwd_3x3s2_k<T, VN, 1><<<grid1, block, 0, st>>>(codes, dvp, dvx, dvdx, pad, na, save_mean, s, save_invstd, b, relu, \
+                                                              coef, nullptr, beta_dx, ag1);                                \
     } while(0)
     if(x->dtype == SAGA_HALF)
         GO(half_t, 8);

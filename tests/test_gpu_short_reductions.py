@@ -9,6 +9,7 @@ import torch
 
 from oracle import ref
 from saga_amd import kernels as K
+from tests import test_gpu_ops as test_ops
 from tests.gpu_util import assert_close, dev, host, rnd
 
 pytestmark = pytest.mark.gpu
@@ -153,3 +154,10 @@ def test_gemm_runs(M, N, Kd, tA, tB, dtype):
     K.check(K.lib().saga_hip_gemm(tA, tB, M, N, Kd, 0.5, pa, Ad.shape[1], pb, Bd.shape[1], 1.0, K.ptr(Cd), N,
                                   K.HALF if dtype == HALF else K.FLOAT, S()))
     assert_close(host(Cd), 0.5 * (A.astype(np.float64) @ B) + 1, dtype, "gemm", tol=1e-3 if dtype == HALF else 1e-5)
+
+
+@pytest.mark.parametrize("dtype", [HALF, F32])
+@pytest.mark.parametrize("H", [700, 1401, 2800, 5450])
+def test_blocks_of_several_patch_rows(H, dtype):
+    """Tall images, whose blocks walk 2 to 16 rows of patches, the last one fewer, in the passes of the norm's backward."""
+    test_ops.test_batch_norm_backward_through_a_max_pooling(1, H, 9, True, 0.0, dtype)
