@@ -169,26 +169,41 @@ struct BwdFin {
     float beta_p;
 };
 
-// totals of a slab of CS channels from cb on: valid for threads below CS
-__device__ __forceinline__ void slab_sums(const float *__restrict__ partial, int prows, int C, int cb, int CS, double &s0, double &s1)
+// Every `lanes`-th of the partials from row l on, up to N of them, which are all on their way at once.
+template <int N> __device__ __forceinline__ void lane_sums(const float *__restrict__ partial, int prows, int C, int c, int l, int lanes, double &a0, double &a1)
 {
     typedef float float2_t __attribute__((ext_vector_type(2)));
+    const float2_t *p = (const float2_t *)partial + c;
+    float2_t v[N];
+#pragma unroll
+    for(int u = 0; u < N; u++)
+        v[u] = p[(int64_t)(l + u * lanes < prows ? l + u * lanes : 0) * C];
+#pragma unroll
+    for(int u = 0; u < N; u++)
+        if(l + u * lanes < prows) {
+            a0 += v[u][0];
+            a1 += v[u][1];
+        }
+}
+
+// totals of a slab of CS channels from cb on: valid for threads below CS.  A thread's partials (32 at most, MOST backward) are one trip to
+// memory: in batches of eight, one after the other, normalizing 16 channels of 128x32x32 from 512 rows took 9.6 us and now takes 7.7,
+// the backward of 32 of 128x16x16 7.8 and 7.2; and no more loads than needed, 1024 of 23x13x13 from 61 rows 7.2 with 8, 9.1 with 32.
+template <int MOST>
+__device__ __forceinline__ void slab_sums(const float *__restrict__ partial, int prows, int C, int cb, int CS, double &s0, double &s1)
+{
     __shared__ double red[2][256];
-    const int tid = threadIdx.x, c = tid % CS, l = tid / CS, lanes = 256 / CS;
-    const float2_t *p = (const float2_t *)partial + (cb + c < C ? cb + c : 0);
+    const int tid = threadIdx.x, c = cb + tid % CS < C ? cb + tid % CS : 0, l = tid / CS, lanes = 256 / CS;
     double a0 = 0, a1 = 0;
-    for(int g = l; g < prows; g += 8 * lanes) {
-        float2_t v[8];
-#pragma unroll
-        for(int u = 0; u < 8; u++)
-            v[u] = p[(int64_t)(g + u * lanes < prows ? g + u * lanes : 0) * C];
-#pragma unroll
-        for(int u = 0; u < 8; u++)
-            if(g + u * lanes < prows) {
-                a0 += v[u][0];
-                a1 += v[u][1];
-            }
-    }
+    int g = l;
+    if(MOST > 16 && prows > 16 * lanes)
+        for(; g < prows; g += MOST * lanes)
+            lane_sums<MOST>(partial, prows, C, c, g, lanes, a0, a1);
+    else if(prows > 8 * lanes)
+        for(; g < prows; g += 16 * lanes)
+            lane_sums<16>(partial, prows, C, c, g, lanes, a0, a1);
+    else
+        lane_sums<8>(partial, prows, C, c, g, lanes, a0, a1);
     red[0][tid] = a0;
     red[1][tid] = a1;
     __syncthreads();
@@ -241,7 +256,7 @@ __device__ __forceinline__ void stats_slab(const StatsFin &f, int C, int cb, int
             rv = f.run_v[c];
     }
     double s0, s1;
-    slab_sums(f.partial, f.prows, C, cb, CS, s0, s1);
+    slab_sums<32>(f.partial, f.prows, C, cb, CS, s0, s1);
     if(own)
         finish_stats(s0, s1, 0.0, f.M, f.eps, f.expavg, sv, bv, rm, rv, write, f.run_m, f.run_v, f.save_mean, f.save_invstd, c,
                      tab[0][tid], tab[1][tid]);
@@ -262,7 +277,7 @@ __device__ __forceinline__ void bwd_slab(const BwdFin &f, int C, int cb, int CS,
         }
     }
     double s0, s1;
-    slab_sums(f.partial, f.prows, C, cb, CS, s0, s1);
+    slab_sums<16>(f.partial, f.prows, C, cb, CS, s0, s1);
     if(own) {
         const double dsv = s1 * inv;
         if(write) {
