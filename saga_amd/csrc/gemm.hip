@@ -83,7 +83,8 @@ struct ColumnBias {
     const void *gate;
     template <typename T> __device__ __forceinline__ float pass(float v, int64_t at) const
     {
-        return gate ? v * ((float)((const T *)gate)[at] > 0.0f ? 1.0f : 0.0f) : v;
+        // (the gradient in its own type first: one that overflows is infinite, and not a number where nothing passes)
+        return gate ? (float)(T)v * ((float)((const T *)gate)[at] > 0.0f ? 1.0f : 0.0f) : v;
     }
     __device__ __forceinline__ float apply(float v, int n) const
     {
