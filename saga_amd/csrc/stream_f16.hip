@@ -3,11 +3,11 @@
 // The tiled kernels of conv_mfma.hip give a block 256 output pixels x 64 or 128 channels and the whole reduction: a single
 // image of ResNet-50's last stages is one block row, two to eight blocks on 256 CUs, each walking up to 144 reduction
 // slices one barrier at a time (47 us for a 0.23 GFLOP layer whose filter is 4.7 MB).  Here the tile is as small as 16
-// pixels x 16 channels and the wavefronts of a block share the reduction: each walks its own part of it, 32 elements a step
-// (v_mfma_f32_16x16x32_f16), through a ring of DEPTH steps of LDS that no other wavefront touches - filled by loads to
+// pixels x 16 channels and the wavefronts of a block share the reduction: each walks its own part of it, 32 or 64 elements a
+// step (v_mfma_f32_16x16x32_f16), through a ring of DEPTH steps of LDS that no other wavefront touches - filled by loads to
 // LDS DEPTH - 1 steps ahead, read back in the matrix unit's order, no barrier until the sums of the wavefronts meet at the
 // end and leave through the folded batch norm.  The trip through LDS is what makes the loads fast: a load instruction
-// fetches 64 bytes of 16 rows with four neighbouring lanes per row, where the operand order would put neighbouring lanes
+// fetches 64 bytes of 16 rows with four neighbouring lanes per row, or 128 of 8 with eight, where the operand order would put neighbouring lanes
 // on different rows (measured: 73 cycles per kilobyte that way, 34 GB/s and CU).
 // Every byte is fetched by every block that needs it, which the caches take while the problem is small; large grids belong
 // to the tiled kernels.
@@ -57,8 +57,8 @@ template <int CLASSES> struct ArgsOf {
     StreamF16 g;
     int istep, ostep, tstep, rstep;
     int nclasses, nblk_q, blocks;
-    int ks_log2, WM, S32; // wavefronts along the reduction and the pixels; steps of 32 channels per tap
-    Div by_q, by_S32;
+    int ks_log2, WM, S; // wavefronts along the reduction and the pixels; steps per tap
+    Div by_q, by_S;
     int q_outer; // blocks that are neighbours share their channels (else their pixels)
     Class cls[CLASSES];
 };
@@ -75,18 +75,29 @@ template <int OFFSET> __device__ __forceinline__ half8_t lds_read(unsigned addr)
     asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFFSET));
     return v;
 }
-template <int N> __device__ __forceinline__ void lds_wait(half8_t (&v)[N])
+// tiles I to N - 1 of SIZE bytes each
+template <int SIZE, int I = 0, int N> __device__ __forceinline__ void lds_read_tiles(half8_t (&v)[N], unsigned addr)
+{
+    if constexpr(I < N) {
+        v[I] = lds_read<I * SIZE>(addr);
+        lds_read_tiles<SIZE, I + 1>(v, addr);
+    }
+}
+template <int U, int N> __device__ __forceinline__ void lds_wait(half8_t (&v)[U][N])
 {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-    for(int i = 0; i < N; i++)
-        asm volatile("" : "+v"(v[i])); // (results of the reads above, not to be used before the wait)
+    for(int u = 0; u < U; u++)
+#pragma unroll
+        for(int i = 0; i < N; i++)
+            asm volatile("" : "+v"(v[u][i])); // (results of the reads above, not to be used before the wait)
 }
 
-// LDS of a wavefront: the ring, then its sums in the same place
-template <int TM, int TN, int DEPTH> constexpr int wave_lds()
+// LDS of a wavefront: the ring of DEPTH steps, or for DEPTH = 0 of RING tiles, then its sums in the same place
+constexpr int RING = 9;
+template <int TM, int TN, int U, int DEPTH> constexpr int wave_lds()
 {
-    return std::max(DEPTH * (TM + TN) * 1024, TM * 16 * (TN * 16 + 4) * 4);
+    return std::max((DEPTH ? DEPTH * (TM + TN) : RING) * U * 1024, TM * 16 * (TN * 16 + 4) * 4);
 }
 
 typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
@@ -131,7 +142,14 @@ __device__ __forceinline__ void store4(__amdgpu_buffer_rsrc_t r, unsigned at, bo
 // 4.8 -> 3.0 (now 0.6 setup, 0.8 filling the ring, 0.7 the rest of the reduction, 0.2 the sum of the wavefronts, 0.5
 // epilogue), 1x1 1024->256 4.7 -> 3.3, 3x3 256->256 7.1 -> 4.6; from the end of a launch to the next it is 1.4.
 // SUMS: with the per-channel sums (StreamF16::sums)
-template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__ void __launch_bounds__(64 * MAXW) stream_f16_k(A k)
+// U: a step takes 32 * U channels.  With 32, two steps share the cache lines of their rows, and what the other wavefronts load
+// between them is more than a CU's cache holds: every line came from L2 twice, and that is what bounds the larger problems (1x21x21
+// 3x3 1024->1024: 5.6 M lines read for 5.9 M pieces of 64 bytes).  With 64 an instruction takes whole lines.  us, 32 / 64, the best tile of
+// each: 1x21x21 3x3 1024->1024 30.0 / 21.1, 1x42x42 3x3 512->512 25.2 / 17.8, 23x13x13 3x3 256->256 15.5 / 12.5, 1x7x7 3x3 512->512
+// 7.0 / 6.4, 4x14x14 3x3 512->512 at stride 2 10.2 / 9.2; with few steps to a wavefront (1x28x28 3x3 128->128) equal.
+// DEPTH = 0: eight wavefronts with tiles of 64 pixels x 32 channels have no room for two steps of 64 channels, but for one and a half.
+// Their ring holds single operands of 16 rows, each of which leaves room for the one nine later as soon as it is in registers.
+template <int TM, int TN, int U, int DEPTH, int MAXW, bool SUMS, typename A> __global__ void __launch_bounds__(64 * MAXW) stream_f16_k(A k)
 {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     constexpr bool ONE = sizeof(A) == sizeof(Args1); // one class: class pixels are output pixels
@@ -141,10 +159,13 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
         static_assert(sizeof(Args1) > 5 * 64, "arguments");
         asm volatile("" ::"s"(line[0]), "s"(line[16]), "s"(line[32]), "s"(line[48]), "s"(line[64]), "s"(line[80]));
     }
-    // as the matrix unit wants its operands, and as the loads fetch them: row lrow, 16-byte piece lkq of its 64.  Rows 4
-    // apart fall into the same banks, so they keep their pieces in another order.
-    const int tid = threadIdx.x, lane = tid & 63, row = lane & 15, kq = lane >> 4, lrow = lane >> 2;
-    const int lkq = (lane & 3) ^ ((lrow >> 2) & 3);
+    // as the matrix unit wants its operands (row, kq), and as the loads fetch them: 16 / U rows by an instruction, each lane the
+    // 16-byte piece lkq of the 64 * U bytes of a row.  Rows 4 / U apart fall into the same banks, so they keep their pieces
+    // in another order; that of the second half of 16 rows is the first's with bit 2 flipped.
+    const int tid = threadIdx.x, lane = tid & 63, row = lane & 15, kq = lane >> 4;
+    auto lrow = [&](int i) { return 16 / U * i + lane / (4 * U); };
+    auto lkq = [&](int i) { return U == 1 ? (lane & 3) ^ (lane >> 4) : (lane & 7) ^ (lane >> 4) ^ 4 * (i & 1); };
+    auto spot = [&](int u) { return row * (64 * U) + ((4 * u + kq) ^ (row * U >> 2)) * 16; };
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int KS = 1 << k.ks_log2, wm = wave >> k.ks_log2, ks = wave & (KS - 1);
     int b = xcd_remap(blockIdx.x, k.blocks), ci = 0;
@@ -159,36 +180,37 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
 
     // byte offset of this lane's 16 bytes of the first tap and first 32 channels (negative outside the image: only valid
     // taps are read), and one bit per row and column of taps that falls inside
-    int base[TM], iy[TM], ix[TM];
-    unsigned rows[TM], cols[TM];
+    constexpr int LM = TM * U, LN = TN * U; // load instructions of a step
+    int base[LM], iy[LM], ix[LM];
+    unsigned rows[LM], cols[LM];
 #pragma unroll
-    for(int i = 0; i < TM; i++) {
-        const int m = m0 + 16 * i + lrow;
+    for(int i = 0; i < LM; i++) {
+        const int m = m0 + lrow(i);
         const bool ok = m < c.M;
         const int mm = ok ? m : 0;
         const int t = divide(mm, c.by_OW), ox = mm - t * c.OW;
         const int n = divide(t, c.by_OH), oy = t - n * c.OH;
         iy[i] = oy * k.istep + c.iy0;
         ix[i] = ox * k.istep + c.ix0;
-        base[i] = ((n * g.IH + iy[i]) * g.IW + ix[i]) * g.lda * 2 + lkq * 16;
+        base[i] = ((n * g.IH + iy[i]) * g.IW + ix[i]) * g.lda * 2 + lkq(i) * 16;
         rows[i] = cols[i] = 0;
         iy[i] = ok ? iy[i] : 0x40000000; // (no row of the image)
     }
 #pragma unroll 1
     for(int a = 0; a < c.Tr; a++)
 #pragma unroll
-        for(int i = 0; i < TM; i++)
+        for(int i = 0; i < LM; i++)
             rows[i] |= (unsigned)(iy[i] + a * k.tstep) < (unsigned)g.IH ? 1u << a : 0u;
 #pragma unroll 1
     for(int a = 0; a < c.Ts; a++)
 #pragma unroll
-        for(int i = 0; i < TM; i++)
+        for(int i = 0; i < LM; i++)
             cols[i] |= (unsigned)(ix[i] + a * k.tstep) < (unsigned)g.IW ? 1u << a : 0u;
-    int qoff[TN];
+    int qoff[LN];
 #pragma unroll
-    for(int t = 0; t < TN; t++) {
-        const int n = n0 + 16 * t + lrow;
-        qoff[t] = n < g.N ? n * (g.R * g.S * g.C) * 2 + lkq * 16 : -1;
+    for(int t = 0; t < LN; t++) {
+        const int n = n0 + lrow(t);
+        qoff[t] = n < g.N ? n * (g.R * g.S * g.C) * 2 + lkq(t) * 16 : -1;
     }
 
     // the four channels this lane will finish, and what their epilogue needs: requested now, used after the loop
@@ -226,15 +248,15 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
     int e = ks * 64 + lane, pix = pixel(e);
     request(pix);
 
-    const int S32 = k.S32, total = S32 * c.Tr * c.Ts;
-    const bool last_ok = (S32 - 1) * 32 + lkq * 8 < g.C;
-    const int cut = g.C % 32 ? (S32 - 1) * 64 : -1; // where only some of the 32 channels are there
+    const int S = k.S, total = S * c.Tr * c.Ts;
+    const bool last_ok = (S - 1) * 32 + lkq(0) * 8 < g.C;
+    const int cut = U == 1 && g.C % 32 ? (S - 1) * 64 : -1; // where only some of the 32 channels are there
     const int s_begin = (ks * total) >> k.ks_log2, steps = ((ks * total + total) >> k.ks_log2) - s_begin;
-    int tap = divide(s_begin, k.by_S32), c32 = s_begin - tap * S32;
+    int tap = divide(s_begin, k.by_S), c0 = s_begin - tap * S;
     int ta = divide(tap, c.by_Ts), te = tap - ta * c.Ts;
-    constexpr int NL = TM + TN; // load instructions, kilobytes of LDS and operands per step
-    char *ring = (char *)smem + wave * wave_lds<TM, TN, DEPTH>();
-    const unsigned at = (unsigned)(uintptr_t)(lds_ptr_t)ring + row * 64 + (kq ^ ((row >> 2) & 3)) * 16;
+    constexpr int NL = LM + LN; // load instructions, kilobytes of LDS and operands per step
+    char *ring = (char *)smem + wave * wave_lds<TM, TN, U, DEPTH>();
+    const unsigned at = (unsigned)(uintptr_t)(lds_ptr_t)ring;
     auto load_to_lds = [](__amdgpu_buffer_rsrc_t r, char *dst, unsigned v, int at) {
         __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)dst, 16, v, at, 0, 0);
     };
@@ -246,75 +268,116 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
             acc[i][t] = float4_t{0, 0, 0, 0};
     int fill = 0, drain = 0;
     auto consume = [&]() {
-        half8_t f[NL];
-        const unsigned from = at + drain;
-        if constexpr(NL > 0) f[0] = lds_read<0 * 1024>(from);
-        if constexpr(NL > 1) f[1] = lds_read<1 * 1024>(from);
-        if constexpr(NL > 2) f[2] = lds_read<2 * 1024>(from);
-        if constexpr(NL > 3) f[3] = lds_read<3 * 1024>(from);
-        if constexpr(NL > 4) f[4] = lds_read<4 * 1024>(from);
-        if constexpr(NL > 5) f[5] = lds_read<5 * 1024>(from);
-        if constexpr(NL > 6) f[6] = lds_read<6 * 1024>(from);
-        if constexpr(NL > 7) f[7] = lds_read<7 * 1024>(from);
-        static_assert(NL <= 8, "operands");
+        half8_t f[U][TM + TN];
+#pragma unroll
+        for(int u = 0; u < U; u++)
+            lds_read_tiles<U * 1024>(f[u], at + drain + spot(u));
         drain = drain == (DEPTH - 1) * NL * 1024 ? 0 : drain + NL * 1024;
         lds_wait(f); // before the next step loads into this slot
 #pragma unroll
-        for(int i = 0; i < TM; i++)
+        for(int u = 0; u < U; u++)
+#pragma unroll
+            for(int i = 0; i < TM; i++)
+#pragma unroll
+                for(int t = 0; t < TN; t++)
+                    acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[u][TM + t], f[u][i], acc[i][t], 0, 0, 0);
+    };
+    // operand v of a step: of the channels, then of the pixels
+    half8_t fn[TN][U];
+    auto take = [&](int v) {
+        half8_t f[U][1];
+#pragma unroll
+        for(int u = 0; u < U; u++)
+            f[u][0] = lds_read<0>(at + drain + spot(u));
+        drain = drain == (RING - 1) * U * 1024 ? 0 : drain + U * 1024;
+        lds_wait(f); // before its place is loaded again
+#pragma unroll
+        for(int u = 0; u < U; u++)
 #pragma unroll
             for(int t = 0; t < TN; t++)
-                acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(f[TM + t], f[i], acc[i][t], 0, 0, 0);
+                if(v == t)
+                    fn[t][u] = f[u][0];
+                else if(v >= TN)
+                    acc[v - TN][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(fn[t][u], f[u][0], acc[v - TN][t], 0, 0, 0);
     };
     int s = 0; // steps requested
 #pragma unroll 1
     while(s < steps) {
         const int d = (ta * g.IW + te) * k.tstep * g.lda * 2;
         const int f = ((c.r0 + ta * k.rstep) * g.S + c.s0 + te * k.rstep) * g.C * 2;
-        unsigned pv[TM], qv[TN];
+        unsigned pv[LM], qv[LN];
 #pragma unroll
-        for(int i = 0; i < TM; i++)
+        for(int i = 0; i < LM; i++)
             pv[i] = (rows[i] >> ta) & (cols[i] >> te) & 1 ? (unsigned)(base[i] + d) : OOB;
 #pragma unroll
-        for(int t = 0; t < TN; t++)
+        for(int t = 0; t < LN; t++)
             qv[t] = qoff[t] >= 0 ? (unsigned)(qoff[t] + f) : OOB;
-        const int until = std::min(s + S32 - c32, steps);
-        int so = c32 * 64;
+        const int until = std::min(s + S - c0, steps);
+        int so = c0 * (64 * U);
 #pragma unroll 1
         do {
             if(so == cut) { // (the tap's last step)
 #pragma unroll
-                for(int i = 0; i < TM; i++)
+                for(int i = 0; i < LM; i++)
                     pv[i] = last_ok ? pv[i] : OOB;
 #pragma unroll
-                for(int t = 0; t < TN; t++)
+                for(int t = 0; t < LN; t++)
                     qv[t] = last_ok ? qv[t] : OOB;
             }
+            if constexpr(DEPTH == 0) {
 #pragma unroll
-            for(int i = 0; i < TM; i++)
+                for(int v = 0; v < TM + TN; v++) {
+#pragma unroll
+                    for(int u = 0; u < U; u++)
+                        load_to_lds(v < TN ? rb : ra, ring + fill + u * 1024, v < TN ? qv[v * U + u] : pv[(v - TN) * U + u], so);
+                    fill = fill == (RING - 1) * U * 1024 ? 0 : fill + U * 1024;
+                    constexpr int BEHIND = RING - 1, PER = TM + TN; // operands requested behind the one to take
+                    if(s * PER + v >= BEHIND) {
+                        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(BEHIND * U) : "memory");
+                        take((v + 2 * PER - BEHIND) % PER);
+                    }
+                }
+                so += 64 * U;
+                continue;
+            }
+#pragma unroll
+            for(int i = 0; i < LM; i++)
                 load_to_lds(ra, ring + fill + i * 1024, pv[i], so);
 #pragma unroll
-            for(int t = 0; t < TN; t++)
-                load_to_lds(rb, ring + fill + (TM + t) * 1024, qv[t], so);
+            for(int t = 0; t < LN; t++)
+                load_to_lds(rb, ring + fill + (LM + t) * 1024, qv[t], so);
             fill = fill == (DEPTH - 1) * NL * 1024 ? 0 : fill + NL * 1024;
-            so += 64;
+            so += 64 * U;
             if(s >= DEPTH - 1) {
                 asm volatile("s_waitcnt vmcnt(%0)" ::"n"((DEPTH - 1) * NL) : "memory");
                 consume();
             }
         } while(++s < until);
-        c32 = 0;
+        c0 = 0;
         if(++te == c.Ts) {
             te = 0;
             ta++;
         }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr(DEPTH == 0) {
+        static_assert(DEPTH || (RING > TM + TN && RING - 1 <= 2 * (TM + TN)), "the last operands of a step and all of the next");
+#pragma unroll
+        for(int v = 2 * (TM + TN) - (RING - 1); v < TM + TN; v++)
+            if(steps > 1)
+                take(v);
+#pragma unroll
+        for(int v = 0; v < TM + TN; v++)
+            if(steps > 0)
+                take(v);
+    } else {
 #pragma unroll 1
-    for(int u = std::min(steps, DEPTH - 1); u > 0; u--)
-        consume();
+        for(int u = std::min(steps, DEPTH - 1); u > 0; u--)
+            consume();
+    }
 
     // acc[i][t][v]: pixel 16*i + lane%16, channel 16*t + 4*(lane/16) + v
-    constexpr int PITCH = TN * 16 + 4, WAVE = wave_lds<TM, TN, DEPTH>() / 4; // floats; rows of a tile fall into different banks
+    constexpr int PITCH = TN * 16 + 4, WAVE = wave_lds<TM, TN, U, DEPTH>() / 4; // floats; rows of a tile fall into different banks
 #pragma unroll
     for(int i = 0; i < TM; i++)
 #pragma unroll
@@ -414,15 +477,17 @@ template <int TM, int TN, int DEPTH, int MAXW, bool SUMS, typename A> __global__
 }
 
 struct Config {
-    int tm, tn, ks, wm;
+    int tm, tn, u, ks, wm;
 };
 
-// Tile (16*tm pixels x 16*tn channels per wavefront) and wavefronts along the reduction (ks) and the pixels (wm) by what
-// they cost: start + steps of a wavefront * (step + more * rounds) + round * rounds, where a round is a block on every CU.
+// Tile (16*tm pixels x 16*tn channels per wavefront), 32*u channels to a step (64 only where they divide C) and wavefronts along the
+// reduction (ks) and the pixels (wm) by what they cost: start + steps of a wavefront * (step + more * rounds) + round * rounds, where a round is a block on every CU.
 // The numbers are fitted to 420 problems (1 to 90 images of 7x7 to 150x150 pixels, 8 to 2048 channels either way, filters
-// of 1 to 5) at each of the tiles, launched one behind the other with filters that are not in the cache: 8 % off on
-// average, and the choice 4 % slower than the best of everything at each problem (lines drawn by tiles and steps, which
-// stood here before: 16 %).  us, before -> now, of which the tiled kernels where they took it:
+// of 1 to 5; those of u = 2 to 180 of 64 to 2048 channels) at each of the tiles, launched one behind the other with filters that are not
+// in the cache: 8 % off on average, and the choice 4 % (2 % with u = 2 in it) slower than the best of everything at each problem
+// (lines drawn by tiles and steps, which stood here before: 16 %).  Left out, as no choice got better with them: u = 2 at 1x1 tiles
+// without a split or of 8, 2x2 of 2x2 and of 8, 4x2 of 2x2.  us, drawn lines -> fitted costs of u = 1, of which the tiled kernels
+// where they took it:
 //   1x56x56 3x3 64->64 and below  as before              23x13x13 3x3 256->256   27.1 -> 15.3 (tiled before)
 //   2x28x28 1x1 128->512     6.0 -> 5.0 (tiled before)  16x28x28 3x3 128->128   18.8 -> 14.1 (tiled before)
 //   1x28x28 1x1 128->512     5.8 -> 4.1 (tiled before)  512x8x8  3x3 64->64     18.6 -> 10.7 (tiled before)
@@ -432,15 +497,20 @@ struct Cost {
     float start, step, more, round;
 };
 constexpr Cost COSTS[] = {
-    {{1, 1, 1, 4}, 3.48f, 0.053f, 0.046f, 0.31f},
-    {{1, 1, 4, 1}, 3.33f, 0.028f, 0.079f, 0.29f},
-    {{1, 1, 8, 1}, 1.97f, 0.046f, 0.174f, 1.70f},
-    {{2, 2, 2, 2}, 3.63f, 0.048f, 0.141f, 0.66f},
-    {{2, 2, 4, 1}, 3.31f, 0.054f, 0.167f, 0.48f},
-    {{4, 2, 2, 2}, 4.85f, -0.057f, 0.345f, 0.46f},
-    {{4, 2, 8, 1}, 1.58f, 0.051f, 0.572f, 2.63f},
-    {{4, 4, 2, 2}, 2.09f, -0.083f, 0.463f, 5.29f},
-    {{4, 4, 4, 1}, 1.49f, -0.008f, 0.439f, 4.34f},
+    {{1, 1, 1, 1, 4}, 3.48f, 0.053f, 0.046f, 0.31f},
+    {{1, 1, 1, 4, 1}, 3.33f, 0.028f, 0.079f, 0.29f},
+    {{1, 1, 1, 8, 1}, 1.97f, 0.046f, 0.174f, 1.70f},
+    {{2, 2, 1, 2, 2}, 3.63f, 0.048f, 0.141f, 0.66f},
+    {{2, 2, 1, 4, 1}, 3.31f, 0.054f, 0.167f, 0.48f},
+    {{4, 2, 1, 2, 2}, 4.85f, -0.057f, 0.345f, 0.46f},
+    {{4, 2, 1, 8, 1}, 1.58f, 0.051f, 0.572f, 2.63f},
+    {{4, 4, 1, 2, 2}, 2.09f, -0.083f, 0.463f, 5.29f},
+    {{4, 4, 1, 4, 1}, 1.49f, -0.008f, 0.439f, 4.34f},
+    {{1, 1, 2, 4, 1}, 2.96f, 0.016f, 0.134f, 0.45f},
+    {{2, 2, 2, 4, 1}, 3.32f, 0.044f, 0.256f, 0.62f},
+    {{4, 2, 2, 8, 1}, 1.41f, 0.000f, 0.878f, 3.89f},
+    {{4, 4, 2, 2, 2}, 3.48f, 0.000f, 0.554f, 5.20f},
+    {{4, 4, 2, 4, 1}, 4.45f, 0.000f, 0.594f, 2.50f},
 };
 
 int split_over(long long a, long long b) { return (int)((a + b - 1) / b); }
@@ -459,13 +529,18 @@ float tiled_us(long long pixels, int steps, int N)
 }
 
 // tm = 0: a matter for the tiled kernels
-Config choose(long long pixels, int steps, int N)
+Config choose(long long pixels, int taps, int C, int N)
 {
-    Config best = {0, 0, 0, 0};
-    float least = tiled_us(pixels, steps, N);
+    Config best = {0, 0, 0, 0, 0};
+    float least = tiled_us(pixels, taps * split_over(C, 32), N);
     for(const Cost &o : COSTS) {
         const long long blocks = split_over(pixels, 16 * o.c.tm * o.c.wm) * (long long)split_over(N, 16 * o.c.tn);
+        const int steps = taps * split_over(C, 32 * o.c.u);
         if(blocks > 640 || steps < o.c.ks) // (beyond what the numbers were fitted to)
+            continue;
+        // Those of u = 2 to up to 2e10 operations.  Beyond, their blocks of a whole CU's LDS lose beside another stream's kernels what they
+        // win alone: training a U-Net at 16x256x256, 3x3 1024->512 over 16x16x16 took 120 us in them, tiled 96 and 9 for its shares.
+        if(o.c.u == 2 && (C % 64 || (double)pixels * N * taps * C > 1e10))
             continue;
         const int rounds = split_over(blocks, 256);
         const float us = o.start + split_over(steps, o.c.ks) * (o.step + o.more * rounds) + o.round * rounds;
@@ -482,7 +557,7 @@ Config config_of(const StreamF16 &g)
     const int s = g.bwd ? g.stride : 1;
     const long long pixels = (long long)g.batch * ((g.OH + s - 1) / s) * ((g.OW + s - 1) / s) * s * s;
     const int taps = ((g.R + s - 1) / s) * ((g.S + s - 1) / s);
-    return choose(pixels, taps * ((g.C + 31) / 32), g.N);
+    return choose(pixels, taps, g.C, g.N);
 }
 
 int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }
@@ -533,24 +608,32 @@ bool classes(Args &a)
 template <bool SUMS, typename A> int launch_as(const A &k, const Config &cf, hipStream_t st)
 {
     const int threads = 64 * cf.ks * cf.wm;
-#define GO(TM, TN, DEPTH, MAXW)                                                                                             \
+#define GO(TM, TN, U, DEPTH, MAXW)                                                                                          \
     do {                                                                                                                    \
-        auto kern = stream_f16_k<TM, TN, DEPTH, MAXW, SUMS, A>;                                                                  \
-        constexpr size_t lds = wave_lds<TM, TN, DEPTH>();                                                                    \
+        auto kern = stream_f16_k<TM, TN, U, DEPTH, MAXW, SUMS, A>;                                                                  \
+        constexpr size_t lds = wave_lds<TM, TN, U, DEPTH>();                                                                    \
         static const hipError_t attr = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize,   \
                                                            MAXW * lds);                                                     \
         if(attr != hipSuccess)                                                                                              \
             return (int)attr;                                                                                               \
         kern<<<k.blocks, threads, lds *(threads / 64), st>>>(k);                                                       \
     } while(0)
-    if(cf.tm == 4 && cf.tn == 4)
-        GO(4, 4, 3, 4);
+    if(cf.tm == 4 && cf.tn == 4 && cf.u == 2)
+        GO(4, 4, 2, 2, 4);
+    else if(cf.tm == 4 && cf.tn == 4)
+        GO(4, 4, 1, 3, 4);
+    else if(cf.tm == 4 && cf.u == 2)
+        GO(4, 2, 2, 0, 8);
     else if(cf.tm == 4)
-        GO(4, 2, 3, 8);
+        GO(4, 2, 1, 3, 8);
+    else if(cf.tm == 2 && cf.u == 2)
+        GO(2, 2, 2, 2, 8);
     else if(cf.tm == 2)
-        GO(2, 2, 4, 8);
+        GO(2, 2, 1, 4, 8);
+    else if(cf.u == 2)
+        GO(1, 1, 2, 4, 8);
     else
-        GO(1, 1, 8, 8);
+        GO(1, 1, 1, 8, 8);
 #undef GO
     SAGA_CHECK_LAUNCH();
     return 0;
@@ -587,8 +670,8 @@ int stream_f16_launch(const StreamF16 &g, hipStream_t st, int *sum_rows)
     while((1 << k.ks_log2) < cf.ks)
         k.ks_log2++;
     k.WM = cf.wm;
-    k.S32 = (g.C + 31) / 32;
-    k.by_S32 = div_by(k.S32);
+    k.S = (g.C + 32 * cf.u - 1) / (32 * cf.u);
+    k.by_S = div_by(k.S);
     k.nblk_q = (g.N + 16 * cf.tn - 1) / (16 * cf.tn);
     k.by_q = div_by(k.nblk_q);
     // the larger operand is the one that each die should fetch once
