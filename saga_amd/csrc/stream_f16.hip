@@ -529,7 +529,7 @@ float tiled_us(long long pixels, int steps, int N)
 }
 
 // tm = 0: a matter for the tiled kernels
-Config choose(long long pixels, int taps, int C, int N)
+Config choose(long long pixels, int taps, int C, int N, bool training)
 {
     Config best = {0, 0, 0, 0, 0};
     float least = tiled_us(pixels, taps * split_over(C, 32), N);
@@ -540,7 +540,10 @@ Config choose(long long pixels, int taps, int C, int N)
             continue;
         // Those of u = 2 to up to 2e10 operations.  Beyond, their blocks of a whole CU's LDS lose beside another stream's kernels what they
         // win alone: training a U-Net at 16x256x256, 3x3 1024->512 over 16x16x16 took 120 us in them, tiled 96 and 9 for its shares.
-        if(o.c.u == 2 && (C % 64 || (double)pixels * N * taps * C > 1e10))
+        // Passes of a training step (with sums for norms, or backward) keep the order of sums of u = 1: a step of Adam and norms of few values
+        // pass a difference in rounding on.  The loss of a ResNet-50's third step, u = 2 against 1: both ways 5.6 % apart at 19x160x160, 2.8 at
+        // 90x144x144, backward alone 5.7 and 2.6; a step at 23x193x193 takes 4060 us, 4080 backward alone, 4100 without.
+        if(o.c.u == 2 && (training || C % 64 || (double)pixels * N * taps * C > 1e10))
             continue;
         const int rounds = split_over(blocks, 256);
         const float us = o.start + split_over(steps, o.c.ks) * (o.step + o.more * rounds) + o.round * rounds;
@@ -552,12 +555,12 @@ Config choose(long long pixels, int taps, int C, int N)
     return best;
 }
 
-Config config_of(const StreamF16 &g)
+Config config_of(const StreamF16 &g, bool sums)
 {
     const int s = g.bwd ? g.stride : 1;
     const long long pixels = (long long)g.batch * ((g.OH + s - 1) / s) * ((g.OW + s - 1) / s) * s * s;
     const int taps = ((g.R + s - 1) / s) * ((g.S + s - 1) / s);
-    return choose(pixels, taps, g.C, g.N);
+    return choose(pixels, taps, g.C, g.N, sums || g.bwd);
 }
 
 int gcd(int a, int b) { return b ? gcd(b, a % b) : a; }
@@ -618,20 +621,26 @@ template <bool SUMS, typename A> int launch_as(const A &k, const Config &cf, hip
             return (int)attr;                                                                                               \
         kern<<<k.blocks, threads, lds *(threads / 64), st>>>(k);                                                       \
     } while(0)
-    if(cf.tm == 4 && cf.tn == 4 && cf.u == 2)
-        GO(4, 4, 2, 2, 4);
-    else if(cf.tm == 4 && cf.tn == 4)
+    if constexpr(!SUMS && sizeof(A) == sizeof(Args1)) { // (forward, without sums)
+        if(cf.u == 2) {
+            if(cf.tm == 4 && cf.tn == 4)
+                GO(4, 4, 2, 2, 4);
+            else if(cf.tm == 4)
+                GO(4, 2, 2, 0, 8);
+            else if(cf.tm == 2)
+                GO(2, 2, 2, 2, 8);
+            else
+                GO(1, 1, 2, 4, 8);
+            SAGA_CHECK_LAUNCH();
+            return 0;
+        }
+    }
+    if(cf.tm == 4 && cf.tn == 4)
         GO(4, 4, 1, 3, 4);
-    else if(cf.tm == 4 && cf.u == 2)
-        GO(4, 2, 2, 0, 8);
     else if(cf.tm == 4)
         GO(4, 2, 1, 3, 8);
-    else if(cf.tm == 2 && cf.u == 2)
-        GO(2, 2, 2, 2, 8);
     else if(cf.tm == 2)
         GO(2, 2, 1, 4, 8);
-    else if(cf.u == 2)
-        GO(1, 1, 2, 4, 8);
     else
         GO(1, 1, 1, 8, 8);
 #undef GO
@@ -641,11 +650,11 @@ template <bool SUMS, typename A> int launch_as(const A &k, const Config &cf, hip
 
 } // namespace
 
-bool stream_f16_wanted(const StreamF16 &g) { return config_of(g).tm > 0; }
+bool stream_f16_wanted(const StreamF16 &g) { return config_of(g, g.sums).tm > 0; }
 
 int stream_f16_sum_rows(const StreamF16 &g)
 {
-    const Config cf = config_of(g);
+    const Config cf = config_of(g, true);
     const int s = g.bwd ? g.stride : 1;
     const long long M = (long long)g.batch * ((g.OH + s - 1) / s) * ((g.OW + s - 1) / s);
     return cf.tm ? (int)((M + 16 * cf.tm * cf.wm - 1) / (16 * cf.tm * cf.wm)) * s * s : 0;
@@ -664,7 +673,7 @@ int stream_f16_launch(const StreamF16 &g, hipStream_t st, int *sum_rows)
     k.g.bq_bytes = g.bq_x ? (unsigned)(out_rows * g.bq_ldx * 2) : 0;
     if(g.C % 8 || g.lda % 8 || !g.a_bytes || !g.b_bytes || !classes(k))
         return SAGA_HIP_EUNSUPPORTED;
-    const Config cf = config_of(g);
+    const Config cf = config_of(g, g.sums);
     if(!cf.tm)
         return SAGA_HIP_EUNSUPPORTED;
     while((1 << k.ks_log2) < cf.ks)
