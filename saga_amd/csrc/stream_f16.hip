@@ -542,7 +542,7 @@ Config choose(long long pixels, int taps, int C, int N, bool training)
         // win alone: training a U-Net at 16x256x256, 3x3 1024->512 over 16x16x16 took 120 us in them, tiled 96 and 9 for its shares.
         // Passes of a training step (with sums for norms, or backward) keep the order of sums of u = 1: a step of Adam and norms of few values
         // pass a difference in rounding on.  The loss of a ResNet-50's third step, u = 2 against 1: both ways 5.6 % apart at 19x160x160, 2.8 at
-        // 90x144x144, backward alone 5.7 and 2.6; a step at 23x193x193 takes 4060 us, 4080 backward alone, 4100 without.
+        // 90x144x144, backward alone 5.7 and 2.6; a step at 23x193x193 takes 4060 to 4080 us with and without.
         if(o.c.u == 2 && (training || C % 64 || (double)pixels * N * taps * C > 1e10))
             continue;
         const int rounds = split_over(blocks, 256);
