@@ -266,7 +266,7 @@ struct ConvFwd : public HipOperation {
     }
     bool foldBn(T s, T b, T m, T v, T z, T y, float eps, int flags)
     {
-        if(stats_ || bn_y_ || b_)
+        if(stats_ || bn_y_ || b_ || pool_y_) // (a norm behind the pooling is not one in front of it)
             return false;
         bn_s_ = s; bn_b_ = b; bn_m_ = m; bn_v_ = v; bn_z_ = z; bn_y_ = y;
         bn_eps_ = eps;
@@ -314,7 +314,7 @@ struct ConvFwd : public HipOperation {
     // (a kernel takes both only together, and only in fp32)
     bool foldRelu(const T &y) override
     {
-        if(!b_ || relu_y_ || x_->m_data_type != Tensor::DataType::FLOAT)
+        if(!b_ || relu_y_ || pool_y_ || x_->m_data_type != Tensor::DataType::FLOAT)
             return false;
         relu_y_ = y;
         return true;

@@ -87,6 +87,45 @@ def test_the_digits_classifier():
     assert kinds == ["convfwd", "actfwd", "poolfwd"] * 2 + ["fc.fwd.n", "actfwd", "fc.fwd.n"]
 
 
+def pooled_then_normalised(behind, **config):
+    """conv -> max pooling -> batch norm or relu, and the result."""
+    rng = np.random.default_rng(5)
+    tensor = lambda a: S.Tensor.from_numpy(a.astype(np.float32))
+    g = S.Graph()
+    x, w = tensor(rng.standard_normal((64, 1, 28, 28))), tensor(rng.standard_normal((32, 1, 5, 5)) / 5)
+    y = g.add_node("conv", {"x": x, "w": w}, {"size": 5, "activations": 32, "pad": 2}).y()
+    y = g.add_node("maxpool", {"x": y}, {"size": 2, "stride": 2}).y()
+    if behind == "norm":  # (scales of either sign: a norm and a pooling do not change places)
+        params = {k: tensor(rng.standard_normal((1, 32)) if k != "v" else rng.uniform(0.5, 1.5, (1, 32))) for k in "sbmv"}
+        y = g.add_node("batchnorm", {"x": y, **params}).y()
+    else:
+        y = g.add_node(behind, {"x": y}).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 64, training=False, **config)
+    return p, ctx.resolve(y)
+
+
+@on_stub
+def test_a_norm_behind_the_pooling_stays_there():
+    for behind, want in (("norm", ["convfwd.pool", "bninf"]), ("relu", ["convfwd", "poolfwd"])):
+        p, _ = pooled_then_normalised(behind)
+        p.finalize()
+        ops = [op for op in stub_gpu.plan(p) if op["kind"] != "filterpack"]
+        assert [op["kind"] for op in ops] == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("behind", ["norm", "relu"])
+def test_what_is_behind_the_pooling(behind):
+    got = []
+    for fused in (True, False):
+        p, out = pooled_then_normalised(behind, disable_op_fusing=not fused)
+        p.run(1)
+        got.append(out.read().copy())
+    assert np.abs(got[1]).max() > 0
+    np.testing.assert_allclose(*got, rtol=0, atol=1e-5 * np.abs(got[1]).max())
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("what", ["bias", "norm", "nothing", "not finite"])
 @pytest.mark.parametrize("shape", [s for s, k in SHAPES.items() if k], ids=str)
