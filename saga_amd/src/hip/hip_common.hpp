@@ -332,8 +332,9 @@ public:
     ArenaPlan layOutArena();
     void leaveArena(HipStorage &s);
     // somebody looks at this storage who did not when programs were finalized: operations that were folded into the one
-    // that writes it become operations again, from the next step on
-    bool unfold(HipStorage *s);
+    // that writes it become operations again, from the next step on.  The storages that are written again, which may have no memory
+    // yet: it is given to them before the step, whose launches may be recorded
+    std::vector<std::shared_ptr<HipStorage>> unfold(HipStorage *s);
 };
 
 class HipProgram : public Program {
@@ -457,7 +458,7 @@ public:
         std::shared_ptr<HipStorage> between;
     };
     std::vector<Fold> m_folded;
-    bool unfold(HipStorage *s);
+    std::vector<std::shared_ptr<HipStorage>> unfold(HipStorage *s);
 
     SagaAux *m_aux = nullptr; // pinned host memory the optimizer kernels write their flags to
     float m_mp_scaling = 1.0f;

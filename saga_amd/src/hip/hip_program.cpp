@@ -237,8 +237,9 @@ std::shared_ptr<Tensor> HipContext::resolveTensor(std::shared_ptr<Tensor> src)
     if(it == m_tensors.end())
         return nullptr;
     m_exported.push_back(it->second->m_storage);
-    if(unfold(it->second->m_storage.get()) && !it->second->m_storage->allocated())
-        it->second->m_storage->allocOwn(); // (not by the operation that writes it: its next launch may be one that is recorded)
+    for(const auto &st : unfold(it->second->m_storage.get()))
+        if(!st->allocated())
+            st->allocOwn();
     // a tensor the host holds keeps its contents between steps: out of the shared arena
     // (reference: src/cuda/cuda_common.cpp:145-158)
     leaveArena(*it->second->m_storage);
@@ -638,20 +639,21 @@ std::set<HipStorage *> readBeforeWritten(const HipOps &ops)
     return read;
 }
 
-bool HipContext::unfold(HipStorage *s)
+std::vector<std::shared_ptr<HipStorage>> HipContext::unfold(HipStorage *s)
 {
-    bool any = false;
+    std::vector<std::shared_ptr<HipStorage>> again;
     for(HipProgram *p : m_programs)
-        any |= p->unfold(s);
-    return any;
+        for(const auto &st : p->unfold(s))
+            again.push_back(st);
+    return again;
 }
 
 // The folded operation goes back into the list right behind its producer, after those that were folded into that one later:
 // what they wrote is behind what it writes.  The arena stays as it is: what they read is in use for an operation longer and what
 // they write from an operation later, with nothing else in between, and the storages between them get memory of their own.
-bool HipProgram::unfold(HipStorage *s)
+std::vector<std::shared_ptr<HipStorage>> HipProgram::unfold(HipStorage *s)
 {
-    bool any = false;
+    std::vector<std::shared_ptr<HipStorage>> again;
     for(size_t f = 0; f < m_folded.size(); f++) {
         if(m_folded[f].between.get() != s)
             continue;
@@ -678,11 +680,11 @@ bool HipProgram::unfold(HipStorage *s)
             m_written.push_back(fold.between.get());
             dropGraphs();
             m_segments.clear();
-            any = true;
+            again.push_back(fold.between);
         }
         f--;
     }
-    return any;
+    return again;
 }
 
 // Backward liveness over the op list, treated as one iteration of a loop: a storage is needed
@@ -753,8 +755,10 @@ void HipProgram::finalize()
     // An accumulating writer reads its output, so the dead-op pass below keeps the first writer
     // whenever it keeps a later one.
     drop_filter_copies(*this, m_ops);
+    std::vector<std::shared_ptr<HipStorage>> again;
     for(HipStorage *s : readBeforeWritten(m_ops)) // (another program's intermediate result, perhaps)
-        m_ctx->unfold(s);
+        for(const auto &st : m_ctx->unfold(s))
+            again.push_back(st);
     fold_into_producers(*this, m_ops);
     if(m_pt == ProgramType::TRAINING)
         reorder_sparse_first_writers(m_ops);
@@ -794,6 +798,9 @@ void HipProgram::finalize()
     planSide();
     m_ctx->m_programs.push_back(this);
     m_ctx->planMemory();
+    for(const auto &st : again)
+        if(!st->allocated())
+            st->allocOwn();
 }
 
 // ---------------------------------------------------------------- run loop

@@ -233,6 +233,49 @@ def test_resolved_intermediates_are_written(dtype, finalized):
     assert stub_gpu.unordered(ops) == [] and stub_gpu.overlapping(ops) == []
 
 
+def nothing_without_memory(p):
+    """(memory that nobody has asked for yet would be allocated by a launch, which may be one that is recorded)"""
+    return all(address for op in stub_gpu.plan(p) for _, address, *_ in op["reads"] + op["writes"])
+
+
+@pytest.mark.parametrize("name", ["lenet", "resnet50"])
+@on_stub
+def test_what_is_written_again_has_memory(name):
+    """Of several operations that are folded into one, all come back with the first: also the tensors between the others."""
+    net = N.lenet(64) if name == "lenet" else N.resnet50(1, dtype=S.HALF)
+    g, t = N.build_graph(net, np.zeros((net.batch,) + tuple(net.in_shape), np.float32), with_classifier=False)
+    ctx = S.Context()
+    p = ctx.create_program(g, net.batch, training=False)
+    ctx.resolve(t[net.output])
+    p.run(3)
+    assert nothing_without_memory(p)
+    count = len(stub_gpu.plan(p))
+    ctx.resolve(t[net.nodes[0]["out"]])
+    assert len(stub_gpu.plan(p)) == count + 2 and nothing_without_memory(p)
+
+
+@pytest.mark.parametrize("arena", [True, False])
+@on_stub
+def test_what_another_program_brings_back_has_memory(arena):
+    import os
+
+    if not arena:
+        os.environ["SAGA_HIP_NO_ARENA"] = "1"
+    net = N.lenet(64)
+    g, t = N.build_graph(net, np.zeros((64,) + tuple(net.in_shape), np.float32), with_classifier=False)
+    ctx = S.Context()
+    p = ctx.create_program(g, 64, training=False)
+    ctx.resolve(t[net.output])
+    p.run(3)
+    count = len(stub_gpu.plan(p))
+    h = S.Graph()
+    ctx_out = h.add_node("tanh", {"x": t[net.nodes[0]["out"]]}).y()
+    q = ctx.create_program(h, 64, training=False)
+    ctx.resolve(ctx_out)
+    q.finalize()
+    assert len(stub_gpu.plan(p)) == count + 2 and nothing_without_memory(p)
+
+
 @on_stub
 def test_a_window_onto_an_intermediate_keeps_it():
     """Other views of the same storage read it too."""

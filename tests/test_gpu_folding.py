@@ -68,6 +68,27 @@ def test_late_resolve_under_graphs(fused, monkeypatch):
         assert np.abs(conv.read()).max() > 0
 
 
+def test_late_resolve_of_several_folds_under_graphs(monkeypatch):
+    """The stem's convolution has its norm and its pooling: both come back, and what is between them has memory before it is recorded."""
+    net = N.resnet50(2, dtype=S.HALF, image=64)
+    x = np.random.default_rng(3).standard_normal((2,) + tuple(net.in_shape)).astype(np.float16)
+    seen = []
+    for graphs in ("0", "1"):
+        monkeypatch.setenv("SAGA_HIP_GRAPH", graphs)
+        g, t = N.build_graph(net, x, with_classifier=False)
+        ctx = S.Context()
+        p = ctx.create_program(g, 2, training=False)
+        out = ctx.resolve(t[net.output])
+        p.run(4)
+        seen.append([out.read().copy()])
+        conv = ctx.resolve(t[net.nodes[0]["out"]])
+        for _ in range(3):
+            p.run(2)
+            seen[-1] += [out.read().copy(), conv.read().copy()]
+    for a, b in zip(*seen):
+        assert np.abs(a).max() > 0 and np.array_equal(a, b)
+
+
 def test_residual_behind_the_convolution_and_a_window():
     rng = np.random.default_rng(2)
     draw = lambda *shape: S.Tensor.from_numpy(rng.standard_normal(shape).astype(np.float32))
