@@ -409,6 +409,8 @@ void HipContext::planMemory()
                     (plan.total + plan.own + workspace) / 1e6, free_bytes / 1e6);
         pr->m_side.clear();
         pr->m_ops = pr->m_one_stream_ops;
+        pr->dropGraphs();
+        pr->m_segments.clear(); // (of the other order)
         plan = layOutArena();
     }
     allocSideWorkspace();

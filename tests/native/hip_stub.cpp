@@ -19,6 +19,7 @@ std::map<std::string, long> g_launches;
 std::string g_log; // kernel, grid and block of every launch, a line each
 dim3 g_grid, g_block;
 long g_uploads = 0;
+bool g_capturing = false; // launches are being recorded into a graph: nothing may be allocated or waited for
 
 hipError_t map_memory(void **p, size_t bytes)
 {
@@ -80,6 +81,8 @@ long hipstub_uploads(void) { return g_uploads; } // asynchronous ones
 
 hipError_t hipMalloc(void **p, size_t bytes)
 {
+    if(g_capturing)
+        return hipErrorStreamCaptureUnsupported;
     if(g_used + ((bytes + 4095) & ~(size_t)4095) > g_total)
         return hipErrorOutOfMemory;
     const hipError_t e = map_memory(p, bytes);
@@ -108,6 +111,8 @@ hipError_t hipMemset(void *p, int v, size_t bytes)
 }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
 {
+    if(g_capturing)
+        return hipErrorStreamCaptureUnsupported;
     memmove(d, s, n);
     return hipSuccess;
 }
@@ -153,7 +158,7 @@ hipError_t hipGetSymbolAddress(void **p, const void *)
 
 hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned) { return new_handle(s); }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) { return g_capturing ? hipErrorStreamCaptureUnsupported : hipSuccess; }
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned) { return hipSuccess; }
 hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d)
 {
@@ -162,9 +167,23 @@ hipError_t hipStreamGetDevice(hipStream_t, hipDevice_t *d)
 }
 hipError_t hipStreamIsCapturing(hipStream_t, hipStreamCaptureStatus *s)
 {
-    *s = hipStreamCaptureStatusNone;
+    *s = g_capturing ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
     return hipSuccess;
 }
+hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode)
+{
+    g_capturing = true;
+    return hipSuccess;
+}
+hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g)
+{
+    g_capturing = false;
+    return new_handle(g);
+}
+hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) { return new_handle(e); }
+hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
 hipError_t hipEventCreate(hipEvent_t *e) { return new_handle(e); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return new_handle(e); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }

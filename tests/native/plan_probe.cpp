@@ -27,7 +27,8 @@ static std::string touched(const HipOpArgs &args)
 extern "C" {
 
 // One line of JSON per operation.  fork: the operation of the main stream that one on the side stream waits for, -1 for the
-// start of the step; needs: the operation of the side stream that one of the main stream waits for.
+// start of the step; needs: the operation of the side stream that one of the main stream waits for.  recorded: whether its launches
+// go into a graph; safe: whether they may.
 int probe_plan(void *box, char *buf, size_t capacity)
 {
     HipProgram *p = program(box);
@@ -42,8 +43,12 @@ int probe_plan(void *box, char *buf, size_t capacity)
                 if(side[i].needs && side[i].needs == side[j].done)
                     needs = (int)j;
             }
-        out += fmt("{\"kind\":\"%s\",\"side\":%d,\"fork\":%d,\"needs\":%d,\"reads\":[%s],\"writes\":[%s]}\n", p->m_ops[i]->name().c_str(),
-                   i < side.size() && side[i].on ? 1 : 0, fork, needs, touched(p->m_ops[i]->getInputs()).c_str(),
+        bool recorded = false;
+        for(const auto &sg : p->m_segments)
+            recorded |= sg.graph && sg.begin <= i && i < sg.end;
+        out += fmt("{\"kind\":\"%s\",\"side\":%d,\"fork\":%d,\"needs\":%d,\"recorded\":%d,\"safe\":%d,\"reads\":[%s],\"writes\":[%s]}\n",
+                   p->m_ops[i]->name().c_str(), i < side.size() && side[i].on ? 1 : 0, fork, needs, recorded ? 1 : 0,
+                   p->m_ops[i]->graphSafe() ? 1 : 0, touched(p->m_ops[i]->getInputs()).c_str(),
                    touched(p->m_ops[i]->getOutputs()).c_str());
     }
     if(buf && capacity > out.size())

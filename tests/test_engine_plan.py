@@ -415,6 +415,32 @@ def test_what_fits_on_one_stream_fits(name, with_inference):
     assert sides == sorted(sides) and sides[-1], sides
 
 
+@on_stub
+def test_what_is_recorded_after_the_second_stream_is_given_up():
+    """The operations are in another order then: which of their launches may go into a graph is asked again."""
+    import os
+
+    os.environ["SAGA_HIP_GRAPH"] = "1"
+    net = TRAINED["resnet20"]()
+    g, _ = N.build_graph(net, np.zeros((net.batch,) + tuple(net.in_shape), np.float32))
+    ctx = S.Context()
+    p = ctx.create_program(g, net.batch, training=True)
+    p.run(4)
+    before = stub_gpu.plan(p)
+    assert any(op["side"] for op in before) and any(op["recorded"] for op in before)
+    stub_gpu.stub.hipstub_set_memory(stub_gpu.stub.hipstub_used())
+    q = ctx.create_program(g, net.batch, training=False)
+    stub_gpu.stub.hipstub_set_memory(stub_gpu.stub.hipstub_used() + (1 << 20))
+    q.finalize()
+    ops = stub_gpu.plan(p)
+    assert not any(op["side"] for op in ops) and [op["kind"] for op in ops] != [op["kind"] for op in before]
+    stub_gpu.stub.hipstub_set_memory(1 << 38)
+    for _ in range(2):
+        assert all(op["safe"] for op in stub_gpu.plan(p) if op["recorded"])
+        p.run(1)
+    assert any(op["recorded"] for op in stub_gpu.plan(p))
+
+
 @pytest.mark.parametrize("others", [[1, 1], [1, 1, 3], [3, 1, 1]], ids=str)
 @on_stub
 def test_several_strided_writers_of_a_gradient(others):
