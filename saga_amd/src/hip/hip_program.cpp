@@ -961,6 +961,7 @@ void HipProgram::runOpsGraphed()
             m_segments.push_back(sg);
             i = sg.end;
         }
+        m_graph_dbufs.clear();
         std::set<HipStorage *> seen;
         for(auto &op : m_ops)
             for(const auto &list : {op->getInputs(), op->getOutputs()})

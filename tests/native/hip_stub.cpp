@@ -18,7 +18,7 @@ std::map<const void *, std::string> g_kernels;
 std::map<std::string, long> g_launches;
 std::string g_log; // kernel, grid and block of every launch, a line each
 dim3 g_grid, g_block;
-long g_uploads = 0;
+long g_uploads = 0, g_replays = 0;
 bool g_capturing = false; // launches are being recorded into a graph: nothing may be allocated or waited for
 
 hipError_t map_memory(void **p, size_t bytes)
@@ -77,6 +77,7 @@ const char *hipstub_log(void) // since the last question
     g_log.clear();
     return last.c_str();
 }
+long hipstub_replays(void) { return g_replays; } // launches of graphs
 long hipstub_uploads(void) { return g_uploads; } // asynchronous ones
 
 hipError_t hipMalloc(void **p, size_t bytes)
@@ -183,7 +184,11 @@ hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g)
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) { return new_handle(e); }
 hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
 hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
-hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t) { return hipSuccess; }
+hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t)
+{
+    g_replays++;
+    return hipSuccess;
+}
 hipError_t hipEventCreate(hipEvent_t *e) { return new_handle(e); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return new_handle(e); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }

@@ -50,7 +50,7 @@ def _child(libs, module, name, kwargs):
 
     stub = C.CDLL(os.path.join(libs, "hip_stub.so"), mode=C.RTLD_GLOBAL)  # before anything that needs the runtime
     stub.hipstub_set_memory.argtypes = [C.c_size_t]
-    stub.hipstub_uploads.restype = C.c_long
+    stub.hipstub_uploads.restype = stub.hipstub_replays.restype = C.c_long
     stub.hipstub_used.restype = stub.hipstub_peak.restype = C.c_size_t
     stub.hipstub_log.restype = C.c_char_p
     stub.hipstub_launches.argtypes, stub.hipstub_launches.restype = [C.c_char_p], C.c_long
@@ -81,6 +81,10 @@ def launched():
 
 def uploads():
     return stub.hipstub_uploads()
+
+
+def replays():
+    return stub.hipstub_replays()
 
 
 def plan(program):

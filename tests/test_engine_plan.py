@@ -441,6 +441,29 @@ def test_what_is_recorded_after_the_second_stream_is_given_up():
     assert any(op["recorded"] for op in stub_gpu.plan(p))
 
 
+@on_stub
+def test_late_looks_do_not_end_the_recording():
+    """Each has the operations cut into segments anew; their batched tensors are as many as before."""
+    import os
+
+    os.environ["SAGA_HIP_GRAPH"] = "1"
+    net = N.resnet20(4, dtype=S.FLOAT)
+    g, t = N.build_graph(net, np.zeros((4,) + tuple(net.in_shape), np.float32), with_classifier=False)
+    ctx = S.Context()
+    p = ctx.create_program(g, 4, training=False, batched={t[net.input]: S.PRE, t[net.output]: S.POST})
+    p.run(3)
+    looks = 0
+    for n in net.nodes:
+        before = len(stub_gpu.plan(p))
+        ctx.resolve(t[n["out"]])
+        looks += len(stub_gpu.plan(p)) > before
+        p.run(1)
+    assert looks > 8
+    before = stub_gpu.replays()
+    p.run(1)
+    assert stub_gpu.replays() > before
+
+
 @pytest.mark.parametrize("others", [[1, 1], [1, 1, 3], [3, 1, 1]], ids=str)
 @on_stub
 def test_several_strided_writers_of_a_gradient(others):
