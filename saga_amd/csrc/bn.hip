@@ -812,10 +812,13 @@ __global__ void __launch_bounds__(256)
 // that a channel is spread over as many blocks as the tensor is worth, not one; sums leave a block as one pair, and the pass
 // that follows adds a channel's pairs itself.  A thread's vectors are 256 apart; it has the loads of four on their way at once.
 // us, training forward and backward with relu (one block per channel, one value at a time, which this replaces / this), fp32:
-//   16 channels of 128x32x32  66 /  9, 253 / 10     64 of 128x8x8  24 /  8,  73 / 10     512 of 16x7x7  9 /  8, 12 / 10
-//   16 channels of 512x32x32 534 / 16, 2370 / 39   256 of 32x56x56 175 / 53, 696 / 114   64 of 512x7x7 80 / 12, 586 / 15
-// (256 of 32x56x56: forward 308 MB, backward 719 MB, 5.8 and 6.3 TB/s); two launches each are what bounds the small ones.
+//   16 channels of 128x32x32  66 /  9, 253 / 10     64 of 128x8x8  23 /  7,  74 /  8     512 of 16x7x7  8 /  4, 12 /  4
+//   16 channels of 512x32x32 534 / 16, 2370 / 39   256 of 32x56x56 175 / 53, 696 / 112   64 of 512x7x7 84 / 13, 546 / 15
+// (256 of 32x56x56: forward 308 MB, backward 719 MB, 5.8 and 6.4 TB/s); two launches each are what bounds the small ones.  Channels of up to
+// four vectors to a thread take one launch, in which a block holds its channel between the sums and what follows from them (us, in two launches /
+// in one, forward and backward: 512 of 1x7x7 6.9 / 3.6, 7.3 / 3.7, 2048 of 8x7x7 12.2 / 6.9, 14.0 / 7.2, 64 of 1x56x56 7.0 / 4.1, 8.1 / 4.4).
 
+constexpr int CF_HELD = 1024;      // vectors of a channel that its block holds: four to a thread
 constexpr int CF_MAX_SPLITS = 256; // blocks whose sums one block adds, a pair to a thread
 
 struct Planes {
@@ -828,11 +831,12 @@ struct Planes {
 // the vectors of a thread, one after the other
 struct PlaneWalk {
     int64_t n, hw, i, end;
-    __device__ __forceinline__ PlaneWalk(const Planes &g, int split)
+    // (held: the block has all of a channel, of CF_HELD vectors at most)
+    __device__ __forceinline__ PlaneWalk(const Planes &g, int split, bool held = false)
     {
-        i = split * g.per + threadIdx.x;
-        end = (split + 1) * g.per < g.vectors ? (split + 1) * g.per : g.vectors;
-        n = g.vectors < 1ll << 31 ? (int64_t)((unsigned)i / (unsigned)g.hwv) : i / g.hwv;
+        i = held ? (int64_t)threadIdx.x : split * g.per + threadIdx.x;
+        end = held || (split + 1) * g.per > g.vectors ? g.vectors : (split + 1) * g.per;
+        n = held || g.vectors < 1ll << 31 ? (int64_t)((unsigned)i / (unsigned)g.hwv) : i / g.hwv;
         hw = i - n * g.hwv;
     }
     __device__ __forceinline__ void next(const Planes &g)
@@ -931,18 +935,19 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// y = x*scale[c] + shift[c] (+ z) (relu).  TRAIN: from the sums that bn_stats_cf left; the first block of a channel writes what
-// outlives the launch.  Otherwise run_m and run_v are the mean and the variance to normalise with.
-template <typename T, int VN, bool TRAIN>
+// y = x*scale[c] + shift[c] (+ z) (relu).  FROM_PAIRS: from the sums that bn_stats_cf left; FROM_HELD: from the block's own; the first block of
+// a channel writes what outlives the launch.  FROM_RUNNING: run_m and run_v are the mean and the variance to normalise with.
+enum { FROM_RUNNING, FROM_PAIRS, FROM_HELD };
+template <typename T, int VN, int FROM>
 __global__ void __launch_bounds__(256)
     bn_apply_cf(const T *x, int64_t npx, const T *z, int64_t npz, T *y, int64_t npy, const float *__restrict__ partial,
                 const float *__restrict__ kept, const float *__restrict__ s, const float *__restrict__ b, float *run_m, float *run_v, float *save_mean, float *save_invstd, double M, float eps, float expavg, int flags, Planes g)
 {
     typedef Ld<T, VN, false> L;
-    const int64_t c = blockIdx.x / g.splits;
-    const int split = blockIdx.x - (int)c * g.splits;
+    const int64_t c = FROM == FROM_HELD ? blockIdx.x : blockIdx.x / g.splits;
+    const int split = FROM == FROM_HELD ? 0 : blockIdx.x - (int)c * g.splits;
     const bool relu = flags & SAGA_BN_RELU, add = flags & SAGA_BN_ADD, first = split == 0 && threadIdx.x == 0;
-    PlaneWalk w(g, split);
+    PlaneWalk w(g, split, FROM == FROM_HELD);
     PlaneBatch<4> p;
     typename L::V xr[4], zr[4];
     auto load = [&]() {
@@ -957,11 +962,28 @@ __global__ void __launch_bounds__(256)
     bool more = w.i < w.end;
     load();
     float sc, sh;
-    if constexpr(TRAIN) {
-        const float k = kept[c], sv = s[c], bv = b[c];
+    if constexpr(FROM != FROM_RUNNING) {
+        // (y may be x: nobody writes before the sums have met)
+        const float k = FROM == FROM_HELD ? (float)x[c * g.HW] : kept[c], sv = s[c], bv = b[c];
         const float rm = first && run_m ? run_m[c] : 0.0f, rv = first && run_v ? run_v[c] : 0.0f;
         double s0, s1;
-        channel_sums(partial, c, g.partials, s0, s1);
+        if constexpr(FROM == FROM_HELD) {
+            float a0 = 0, a1 = 0;
+#pragma unroll
+            for(int u = 0; u < 4; u++)
+                if(p.ok[u])
+#pragma unroll
+                    for(int j = 0; j < VN; j++) {
+                        const float d = L::at(xr[u], j) - k;
+                        a0 += d;
+                        a1 += d * d;
+                    }
+            block_sum2(a0, a1);
+            s0 = a0;
+            s1 = a1;
+        } else {
+            channel_sums(partial, c, g.partials, s0, s1);
+        }
         finish_stats(s0, s1, k, M, eps, expavg, sv, bv, rm, rv, first, run_m, run_v, save_mean, save_invstd, (int)c, sc, sh);
     } else {
         sc = s[c] * rsqrtf(run_v[c] + eps);
@@ -984,9 +1006,37 @@ __global__ void __launch_bounds__(256)
             }
             L::store(y + p.n[u] * npy + p.at[u], o);
         }
-        more = w.i < w.end;
+        more = FROM != FROM_HELD && w.i < w.end;
         if(more)
             load();
+    }
+}
+
+// Inference, vectors in the order of memory, whatever their channel is (infer_in_order).
+template <typename T, int VN>
+__global__ void __launch_bounds__(256)
+    bn_infer_cf(const T *x, int64_t npx, const T *z, int64_t npz, T *y, int64_t npy, const float *__restrict__ s, const float *__restrict__ b,
+                const float *__restrict__ m, const float *__restrict__ v, float eps, int flags, int C, unsigned hwv, unsigned total)
+{
+    typedef Ld<T, VN, false> L;
+    const bool relu = flags & SAGA_BN_RELU, add = flags & SAGA_BN_ADD;
+    for(unsigned i = blockIdx.x * 256 + threadIdx.x; i < total; i += gridDim.x * 256) {
+        const unsigned nc = i / hwv, n = nc / (unsigned)C, c = nc - n * (unsigned)C;
+        const int64_t at = ((int64_t)c * hwv + (i - nc * hwv)) * VN;
+        const auto xr = L::raw(x + n * npx + at);
+        const auto zr = add ? L::raw(z + n * npz + at) : xr;
+        const float sc = s[c] * rsqrtf(v[c] + eps), sh = b[c] - m[c] * sc;
+        float o[VN];
+#pragma unroll
+        for(int j = 0; j < VN; j++) {
+            float t = __builtin_fmaf(L::at(xr, j), sc, sh);
+            if(add)
+                t += L::at(zr, j);
+            if(relu)
+                t = (t != t) ? t : fmaxf(t, 0.0f);
+            o[j] = t;
+        }
+        L::store(y + n * npy + at, o);
     }
 }
 
@@ -1035,8 +1085,8 @@ __global__ void __launch_bounds__(256)
     }
 }
 
-// Pass 2 of backward: dx = s*invstd*(dy' - db/M - (x-mean)*invstd*ds/M) ; dz = dy'.
-template <typename T, int VN>
+// Pass 2 of backward: dx = s*invstd*(dy' - db/M - (x-mean)*invstd*ds/M) ; dz = dy'.  HELD: and pass 1, of what the block holds.
+template <typename T, int VN, bool HELD>
 __global__ void __launch_bounds__(256)
     bn_bwd_apply_cf(const T *x, int64_t npx, const T *y, int64_t npy, const T *dy, int64_t npdy, T *dx, int64_t npdx, T *dz,
                     int64_t npdz, const float *__restrict__ partial, const float *__restrict__ s,
@@ -1044,10 +1094,10 @@ __global__ void __launch_bounds__(256)
                     float beta_dx, float beta_dz, float beta_p, Planes g)
 {
     typedef Ld<T, VN, false> L;
-    const int64_t c = blockIdx.x / g.splits;
-    const int split = blockIdx.x - (int)c * g.splits;
+    const int64_t c = HELD ? blockIdx.x : blockIdx.x / g.splits;
+    const int split = HELD ? 0 : blockIdx.x - (int)c * g.splits;
     const bool first = split == 0 && threadIdx.x == 0;
-    PlaneWalk w(g, split);
+    PlaneWalk w(g, split, HELD);
     PlaneBatch<4> p;
     typename L::V xr[4], gr[4], yr[4];
     auto load = [&]() {
@@ -1064,7 +1114,23 @@ __global__ void __launch_bounds__(256)
     const float mean = save_mean[c], inv = save_invstd[c], sv = s[c];
     const float ds_old = first && beta_p != 0.0f ? ds[c] : 0.0f, db_old = first && beta_p != 0.0f ? db[c] : 0.0f;
     double s0, s1;
-    channel_sums(partial, c, g.partials, s0, s1);
+    if constexpr(HELD) { // (dx and dz may be what was read: nobody writes before the sums have met)
+        float a0 = 0, a1 = 0;
+#pragma unroll
+        for(int u = 0; u < 4; u++)
+            if(p.ok[u])
+#pragma unroll
+                for(int j = 0; j < VN; j++) {
+                    const float gm = y && !(L::at(yr[u], j) > 0.0f) ? 0.0f : L::at(gr[u], j);
+                    a0 += gm;
+                    a1 += gm * (L::at(xr[u], j) - mean);
+                }
+        block_sum2(a0, a1);
+        s0 = a0;
+        s1 = a1;
+    } else {
+        channel_sums(partial, c, g.partials, s0, s1);
+    }
     const double dsv = s1 * inv;
     if(first) {
         ds[c] = (float)(beta_p != 0.0f ? dsv + (double)beta_p * ds_old : dsv);
@@ -1098,7 +1164,7 @@ __global__ void __launch_bounds__(256)
                 L::store(pz, gv);
             }
         }
-        more = w.i < w.end;
+        more = !HELD && w.i < w.end;
         if(more)
             load();
     }
@@ -1174,6 +1240,16 @@ static Planes plan_planes(const CFInfo &f, int vn, int64_t most)
     return g;
 }
 
+// Whether inference takes the vectors in the order of memory (bn_infer_cf).  In the order of the channels neighbouring lanes are planes apart
+// where planes are small, and a block waits for its channel's numbers before it has four vectors' work to do.  us, by channel / in order:
+// fp32 512x64x2x2 4.4 / 2.5, 512x512x3x3 13.1 / 7.9, 1x64x56x56 3.5 / 2.5, 64x256x14x14 6.6 / 5.2, 1024x512x4x4 17.7 / 12.4, 64x1024x13x13 24 / 24.  Single
+// values of two bytes are the exception once there are many: 512x512x7x7 23 / 27, 2x16x300x301 7.2 / 8.1, 64x256x14x14 8.2 / 8.9; 512x512x6x6 22 / 20.
+static bool infer_in_order(const Planes &g, int C, int vn, int dtype)
+{
+    const int64_t total = g.vectors * C;
+    return total < 1ll << 31 && !(vn == 1 && dtype == SAGA_HALF && g.HW >= 49 && total >= 1 << 21);
+}
+
 // The blocks of a channel whose sums the workspace has room for: it is sized by the plans for channels-last tensors.
 static int64_t cf_room(const CFInfo &f) { return std::min<int64_t>(CF_MAX_SPLITS, plan((int64_t)f.N * f.HW, f.C).gx); }
 
@@ -1244,8 +1320,23 @@ int saga_hip_bn_infer(const SagaTensorView *x, const SagaTensorView *z, const Sa
     } else if(as_channels_first(x, &fx) && as_channels_first(y, &fy) && (!add || as_channels_first(z, &fz))) {
         const int vn = cf_vec_width(x->dtype, fx, {{x, fx.npitch}, {y, fy.npitch}, {add ? z : nullptr, fz.npitch}});
         const Planes g = plan_planes(fx, vn, 1 << 16);
+        const int64_t total = g.vectors * fx.C;
+        if(infer_in_order(g, fx.C, vn, x->dtype)) {
 #define GO(T, VN)                                                                                                                 \
-    bn_apply_cf<T, VN, false><<<(unsigned)(g.splits * (int64_t)fx.C), 256, 0, st>>>(                                              \
+    bn_infer_cf<T, VN><<<grid_for(total, 256, 256 * 32), 256, 0, st>>>((const T *)x->ptr, fx.npitch, add ? (const T *)z->ptr : nullptr, fz.npitch, \
+                                                                       (T *)y->ptr, fy.npitch, s, b, m, v, eps, flags, fx.C, (unsigned)g.hwv,      \
+                                                                       (unsigned)total)
+            if(x->dtype == SAGA_HALF) {
+                if(vn == 8) GO(half_t, 8); else GO(half_t, 1);
+            } else {
+                if(vn == 4) GO(float, 4); else GO(float, 1);
+            }
+#undef GO
+            SAGA_CHECK_LAUNCH();
+            return 0;
+        }
+#define GO(T, VN)                                                                                                                 \
+    bn_apply_cf<T, VN, FROM_RUNNING><<<(unsigned)(g.splits * (int64_t)fx.C), 256, 0, st>>>(                                              \
         (const T *)x->ptr, fx.npitch, add ? (const T *)z->ptr : nullptr, fz.npitch, (T *)y->ptr, fy.npitch, nullptr, nullptr, s, b, \
         (float *)m, (float *)v, nullptr, nullptr, 0.0, eps, 0.0f, flags, g)
         if(x->dtype == SAGA_HALF) {
@@ -1310,10 +1401,13 @@ int saga_hip_bn_train_fwd(const SagaTensorView *x, const SagaTensorView *z, cons
         g2.partials = g1.partials;
         float *const kept = ws + 2 * (int64_t)fx.C * g1.splits;
         const double M = (double)fx.N * fx.HW;
+        const bool held = g2.vectors <= CF_HELD;
 #define GO(T, VN)                                                                                                                 \
     do {                                                                                                                          \
-        bn_stats_cf<T, VN><<<(unsigned)(g1.splits * (int64_t)fx.C), 256, 0, st>>>((const T *)x->ptr, fx.npitch, ws, kept, g1);    \
-        bn_apply_cf<T, VN, true><<<(unsigned)(g2.splits * (int64_t)fx.C), 256, 0, st>>>(                                          \
+        if(!held)                                                                                                                 \
+            bn_stats_cf<T, VN><<<(unsigned)(g1.splits * (int64_t)fx.C), 256, 0, st>>>((const T *)x->ptr, fx.npitch, ws, kept, g1); \
+        auto kern = held ? bn_apply_cf<T, VN, FROM_HELD> : bn_apply_cf<T, VN, FROM_PAIRS>;                                        \
+        kern<<<(unsigned)(g2.splits * (int64_t)fx.C), 256, 0, st>>>(                                                              \
             (const T *)x->ptr, fx.npitch, add ? (const T *)z->ptr : nullptr, fz.npitch, (T *)y->ptr, fy.npitch, ws, kept, s, b,   \
             run_m, run_v, save_mean, save_invstd, M, eps, expavg, flags, g2);                                                     \
     } while(0)
@@ -1521,16 +1615,19 @@ int saga_hip_bn_bwd_ex(const SagaTensorView *x, const SagaTensorView *y, const S
         Planes g2 = plan_planes(fx, vn, 1 << 16);
         g2.partials = g1.partials;
         const double M = (double)fx.N * fx.HW;
+        const bool held = g2.vectors <= CF_HELD;
         // (as above: the first pass leaves dy' in dz)
-        const bool early_dz = dz && beta_dz == 0.0f && relu && dz->ptr != dy->ptr && dz->ptr != x->ptr && dz->ptr != y->ptr;
+        const bool early_dz = !held && dz && beta_dz == 0.0f && relu && dz->ptr != dy->ptr && dz->ptr != x->ptr && dz->ptr != y->ptr;
 #define GO(T, VN)                                                                                                                 \
     do {                                                                                                                          \
         T *const zp = dz ? (T *)dz->ptr : nullptr;                                                                                \
         const T *const yp = relu ? (const T *)y->ptr : nullptr;                                                                   \
-        bn_bwd_stats_cf<T, VN><<<(unsigned)(g1.splits * (int64_t)fx.C), 256, 0, st>>>(                                            \
-            (const T *)x->ptr, fx.npitch, yp, fy.npitch, (const T *)dy->ptr, fdy.npitch, early_dz ? zp : nullptr, fdz.npitch,     \
-            save_mean, ws, g1);                                                                                                   \
-        bn_bwd_apply_cf<T, VN><<<(unsigned)(g2.splits * (int64_t)fx.C), 256, 0, st>>>(                                            \
+        if(!held)                                                                                                                 \
+            bn_bwd_stats_cf<T, VN><<<(unsigned)(g1.splits * (int64_t)fx.C), 256, 0, st>>>(                                        \
+                (const T *)x->ptr, fx.npitch, yp, fy.npitch, (const T *)dy->ptr, fdy.npitch, early_dz ? zp : nullptr, fdz.npitch, \
+                save_mean, ws, g1);                                                                                               \
+        auto kern = held ? bn_bwd_apply_cf<T, VN, true> : bn_bwd_apply_cf<T, VN, false>;                                          \
+        kern<<<(unsigned)(g2.splits * (int64_t)fx.C), 256, 0, st>>>(                                                              \
             (const T *)x->ptr, fx.npitch, early_dz ? nullptr : yp, fy.npitch, early_dz ? zp : (const T *)dy->ptr,                 \
             early_dz ? fdz.npitch : fdy.npitch, (T *)dx->ptr, fdx.npitch, early_dz ? nullptr : zp, fdz.npitch, ws, s, save_mean,  \
             save_invstd, ds, db, M, beta_dx, beta_dz, beta_p, g2);                                                                \

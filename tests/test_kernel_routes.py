@@ -66,6 +66,37 @@ def test_fp32_filter_gradients_with_fewer_partials(c, k, r):
         assert rc == want, (room, rc)
 
 
+@pytest.mark.parametrize("dtype", [K.HALF, K.FLOAT])
+@on_stub
+def test_norms_of_planes(dtype):
+    """Channels that a block holds take one launch, others two; inference goes through the values in their order in memory."""
+    L = K.lib()
+    channel = [ROOM + (i << 20) for i in range(8)]
+    vector = 8 if dtype == K.HALF else 4
+
+    def ran(n, c, h, w):
+        t = [image(a, n, c, h, w, dtype=dtype) for a in (X, Y, W)]
+        for v in t:
+            v.strides[:] = [c * h * w, h * w, w, 1]
+        x, y, dy = (C.byref(v) for v in t)
+        stub_gpu.launched()
+        s, b, m, v, mean, std, ds, db = channel
+        ws = 64 * ROOM, 1 << 30
+        assert L.saga_hip_bn_train_fwd(x, None, y, s, b, m, v, mean, std, 1e-5, 0.1, K.BN_RELU, *ws, None) == 0
+        assert L.saga_hip_bn_bwd(x, y, dy, dy, None, s, mean, std, ds, db, 0.0, 0.0, 0.0, K.BN_RELU, *ws, None) == 0
+        train = [name for name, *_ in stub_gpu.launched()]
+        assert L.saga_hip_bn_infer(x, None, y, s, b, m, v, 1e-5, K.BN_RELU, None) == 0
+        return train, [name for name, *_ in stub_gpu.launched()]
+
+    one, two = ["bn_apply_cf", "bn_bwd_apply_cf"], ["bn_stats_cf", "bn_apply_cf", "bn_bwd_stats_cf", "bn_bwd_apply_cf"]
+    assert ran(1, 512, 7, 7) == (one, ["bn_infer_cf"])
+    assert ran(8, 2048, 7, 7) == (one, ["bn_infer_cf"])
+    assert ran(512, 64, 2, 2) == (one if dtype == K.FLOAT else two, ["bn_infer_cf"])
+    assert ran(1024 // 64, 4, 8, 8 * vector) == (one, ["bn_infer_cf"])
+    assert ran(1024 // 64 + 1, 4, 8, 8 * vector) == (two, ["bn_infer_cf"])
+    assert ran(512, 512, 7, 7) == (two, ["bn_apply_cf" if dtype == K.HALF else "bn_infer_cf"])
+
+
 @on_stub
 def test_biases_that_are_no_vector_are_refused():
     """Elements at no constant distance; a constant one other than 1 goes to a pass of its own."""
