@@ -316,11 +316,19 @@ __global__ void __launch_bounds__(64 * GS_WAVES)
             } else {
                 if(k >= K)
                     v[j] = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-                const int r = RUNS ? run_of_rows(8, row0 + (lane & 3) * 8, rows) - row0 : (lane & 3) * 8;
+                half_t(*const to)[GS_LD] = d + (lane & 3) * 8;
+                const int col = (lane >> 2) + 16 * j;
+                if(!RUNS || row0 + 32 <= rows || rows % 8 == 0) { // (no run was moved, or only whole ones behind the last row)
 #pragma unroll
-                for(int e = 0; e < 8; e++)
-                    if(!RUNS || r + e >= 0)
-                        d[r + e][(lane >> 2) + 16 * j] = v[j][e];
+                    for(int e = 0; e < 8; e++)
+                        to[e][col] = v[j][e];
+                } else {
+                    const int r = run_of_rows(8, row0 + (lane & 3) * 8, rows) - row0;
+#pragma unroll
+                    for(int e = 0; e < 8; e++)
+                        if(r + e >= 0)
+                            d[r + e][col] = v[j][e];
+                }
             }
         }
     };
@@ -422,11 +430,19 @@ __global__ void __launch_bounds__(64 * W)
             } else {
                 if(k >= K)
                     v[j] = float4_t{0, 0, 0, 0};
-                const int r = RUNS ? run_of_rows(4, row0 + (lane % RL) * 4, rows) - row0 : (lane % RL) * 4;
+                float(*const to)[LD] = d + (lane % RL) * 4;
+                const int col = lane / RL + KL * j;
+                if(!RUNS || row0 + T <= rows || rows % 4 == 0) { // (no run was moved, or only whole ones behind the last row)
 #pragma unroll
-                for(int e = 0; e < 4; e++)
-                    if(!RUNS || r + e >= 0)
-                        d[r + e][lane / RL + KL * j] = v[j][e];
+                    for(int e = 0; e < 4; e++)
+                        to[e][col] = v[j][e];
+                } else {
+                    const int r = run_of_rows(4, row0 + (lane % RL) * 4, rows) - row0;
+#pragma unroll
+                    for(int e = 0; e < 4; e++)
+                        if(r + e >= 0)
+                            d[r + e][col] = v[j][e];
+                }
             }
         }
     };
