@@ -1396,13 +1396,12 @@ struct PadJob {
     int C, Cp;
     int blocks;
 };
-constexpr int PAD_VECTORS = 4;
 
-// One or two copies, the blocks of the first in front.  A block copies runs of 1024 vectors; a thread has four loads on their way and
+// One or two copies, the blocks of the first in front.  A block copies runs of 256 * PAD_VECTORS vectors; a thread has its loads on their way at once and
 // one division for all of them.
-// us of a call with both copies of its operands, one after the other and a vector to a thread / this: forward 15->427, 1x1, 166x17x17 19.8 /
-// 17.5, 19->10, 3x3 at stride 2, 56x60x60 21.6 / 18.9, filter gradient of the two 34.2 / 31.1, 27.2 / 23.8.
-__global__ void __launch_bounds__(256) pad_channels(PadJob a, PadJob b)
+// us of a call, copies one after the other, a vector to a thread / this: with both operands copied forward 19->10, 3x3 at stride 2, 56x60x60 21.9 /
+// 17.9, filter gradient of it 26.9 / 23.6, of 15->427, 1x1, 166x17x17 34.9 / 31.3; with one, small, backward data of 10->122, 1x1, 3x7x7 7.4 / 7.4.
+template <int PAD_VECTORS> __global__ void __launch_bounds__(256) pad_channels(PadJob a, PadJob b)
 {
     const bool second = (int)blockIdx.x >= a.blocks;
     const PadJob j = second ? b : a;
@@ -1413,10 +1412,19 @@ __global__ void __launch_bounds__(256) pad_channels(PadJob a, PadJob b)
         int64_t r = total < 1ll << 31 ? (int64_t)((unsigned)i / (unsigned)groups) : i / groups;
         int g = (int)(i - r * groups);
         vec4_t v[PAD_VECTORS];
+        int by[PAD_VECTORS];
 #pragma unroll
         for(int u = 0; u < PAD_VECTORS; u++) {
             // (rows start at any even address; behind the last vector nothing is read)
-            v[u] = load_any(j.src + r * j.sp + g * 8, i + 256 * u < total ? j.C - g * 8 : 0);
+            const bool there = i + 256 * u < total;
+            if(j.C >= 8) { // the row's last vector is loaded where it is whole, and moved: no lane waits for another's small loads
+                const int c0 = there ? g * 8 : 0, from = c0 < j.C - 8 ? c0 : j.C - 8;
+                v[u] = *(const any4_t *)(j.src + (there ? r : 0) * j.sp + from);
+                by[u] = c0 - from;
+            } else {
+                v[u] = load_any(j.src + (there ? r : 0) * j.sp, j.C);
+                by[u] = 0;
+            }
             r += dr;
             g += dg;
             if(g >= groups) {
@@ -1425,18 +1433,32 @@ __global__ void __launch_bounds__(256) pad_channels(PadJob a, PadJob b)
             }
         }
 #pragma unroll
-        for(int u = 0; u < PAD_VECTORS; u++)
+        for(int u = 0; u < PAD_VECTORS; u++) {
+            vec4_t w = v[u];
+            w = by[u] & 4 ? vec4_t{w[2], w[3], 0, 0} : w;
+            w = by[u] & 2 ? vec4_t{w[1], w[2], w[3], 0} : w;
+            w = by[u] & 1 ? vec4_t{w[0] >> 16 | w[1] << 16, w[1] >> 16 | w[2] << 16, w[2] >> 16 | w[3] << 16, w[3] >> 16} : w;
             if(i + 256 * u < total)
-                *(vec4_t *)(j.dst + (i + 256 * u) * 8) = v[u];
+                *(vec4_t *)(j.dst + (i + 256 * u) * 8) = w;
+        }
     }
 }
 
-static PadJob pad_job(const half_t *src, int64_t sp, int C, half_t *dst, int Cp, int64_t rows)
-{
-    return {src, dst, sp, rows, C, Cp, grid_for(rows * (Cp / 8), 256 * PAD_VECTORS, 256 * 16)};
-}
+static PadJob pad_job(const half_t *src, int64_t sp, int C, half_t *dst, int Cp, int64_t rows) { return {src, dst, sp, rows, C, Cp, 0}; }
 
-static void launch_pad_channels(const PadJob &a, const PadJob &b, hipStream_t st) { pad_channels<<<a.blocks + b.blocks, 256, 0, st>>>(a, b); }
+// Four vectors to a thread where there are more than eight blocks to a compute unit without: fewer leave threads idle, and the others in a chain
+// (backward data of 5->116, 1x1, 68x12x12 8.6 us with one, 9.1 with four, 24->371, 5x5 at stride 2, 5x51x51 21.8 and 22.5).
+static void launch_pad_channels(PadJob a, PadJob b, hipStream_t st)
+{
+    auto blocks = [](const PadJob &j, int vectors) { return j.rows ? grid_for(j.rows * (j.Cp / 8), 256 * vectors, 256 * 16) : 0; };
+    const bool few = blocks(a, 1) + blocks(b, 1) <= 2048;
+    a.blocks = blocks(a, few ? 1 : 4);
+    b.blocks = blocks(b, few ? 1 : 4);
+    if(few)
+        pad_channels<1><<<a.blocks + b.blocks, 256, 0, st>>>(a, b);
+    else
+        pad_channels<4><<<a.blocks + b.blocks, 256, 0, st>>>(a, b);
+}
 
 struct FilterPlan {
     int bm, bn, tiles_k, tiles_c, splits, m_per_split;

@@ -50,6 +50,18 @@ def test_fp16_gradients_without_room_for_a_padded_copy(kind, k, pitch):
         assert gradient(kind, x, w, y, 0)[0] == -4
 
 
+@on_stub
+def test_padded_copies_by_their_size():
+    """A vector to a thread in small ones, both operands' in one launch."""
+    L, p = K.lib(), K.ConvParams(0, 1, 1, 1)
+    for n, c, k, image_size, want in ((5, 64, 122, 13, [1, 53]), (5, 65, 122, 13, [1, 83]), (64, 64, 122, 60, [4, 3600])):
+        x, w, y = image(X, n, c, image_size, image_size), image(W, k, c, 1, 1), image(Y, n, k, image_size, image_size)
+        stub_gpu.launched()
+        assert L.saga_hip_conv2d_bwd_filter(C.byref(x), C.byref(y), C.byref(w), C.byref(p), 1.0, 0.0, ROOM, 1 << 30, None) == 0
+        pads = [(args, blocks) for name, args, blocks, _ in stub_gpu.launched() if name == "pad_channels"]
+        assert len(pads) == 1 and pads[0][0] == tuple(want[:1]) and pads[0][1] == want[1]
+
+
 @pytest.mark.parametrize("c,k,r", [(16, 64, 3), (8, 64, 5), (7, 13, 3)])
 @on_stub
 def test_fp32_filter_gradients_with_fewer_partials(c, k, r):
