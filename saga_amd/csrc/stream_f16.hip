@@ -529,7 +529,7 @@ float tiled_us(long long pixels, int steps, int N)
 }
 
 // tm = 0: a matter for the tiled kernels
-Config choose(long long pixels, int taps, int C, int N, bool training)
+Config choose(long long pixels, int taps, int C, int N, bool sums_or_bwd)
 {
     Config best = {0, 0, 0, 0, 0};
     float least = tiled_us(pixels, taps * split_over(C, 32), N);
@@ -538,16 +538,19 @@ Config choose(long long pixels, int taps, int C, int N, bool training)
         const int steps = taps * split_over(C, 32 * o.c.u);
         if(blocks > 640 || steps < o.c.ks) // (beyond what the numbers were fitted to)
             continue;
-        // Those of u = 2 to up to 2e10 operations.  Beyond, their blocks of a whole CU's LDS lose beside another stream's kernels what they
-        // win alone: training a U-Net at 16x256x256, 3x3 1024->512 over 16x16x16 took 120 us in them, tiled 96 and 9 for its shares.
-        // Passes of a training step (with sums for norms, or backward) keep the order of sums of u = 1: a step of Adam and norms of few values
+        // Those of u = 2 to up to 2e10 operations, which their numbers were fitted to.  Of 120 problems of 1.6e10 to 1e11 ten would take
+        // them beyond: nine 2 to 39 % faster (52x16x16 5x5 512->64 54 -> 37 us), one 11 % slower (20x25x25 5x5 384->160 74 -> 82).
+        // Passes with sums for norms and backward passes keep the order of sums of u = 1: a step of Adam and norms of few values
         // pass a difference in rounding on.  The loss of a ResNet-50's third step, u = 2 against 1: both ways 5.6 % apart at 19x160x160, 2.8 at
-        // 90x144x144, backward alone 5.7 and 2.6; a step at 23x193x193 takes 4060 to 4080 us with and without.
-        if(o.c.u == 2 && (training || C % 64 || (double)pixels * N * taps * C > 1e10))
+        // 90x144x144, backward alone 5.7 and 2.6; a step at 23x193x193 takes 4060 to 4080 us with and without.  (A forward convolution
+        // without a norm behind it takes u = 2 in a training step as well: a call does not know what it is part of.)
+        if(o.c.u == 2 && (sums_or_bwd || C % 64 || (double)pixels * N * taps * C > 1e10))
             continue;
         const int rounds = split_over(blocks, 256);
         const float us = o.start + split_over(steps, o.c.ks) * (o.step + o.more * rounds) + o.round * rounds;
-        if(us < least) {
+        // u = 2 has to be cheaper by more than the numbers are off.  Of 1200 problems of 64 to 2048 channels 24 were 4 to 15 % slower than what
+        // u = 2 takes the place of without these lines, 6 with them (the worst 1x49x49 3x3 1536->272 42 -> 48 us); 538 and 501 4 % and more faster.
+        if(us < least * (o.c.u == 2 && best.u != 2 ? best.tm ? 0.92f : 0.86f : 1.0f)) {
             least = us;
             best = o.c;
         }
