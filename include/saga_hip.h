@@ -199,8 +199,8 @@ int saga_hip_conv2d_fwd_bn_infer(const SagaTensorView *x, const SagaTensorView *
 
 /* ---- the same with a relu and a max pooling behind it (y: the pooled tensor), which is the stem of an image network: what is between
  *      them does not reach memory.  Returns SAGA_HIP_EUNSUPPORTED, with nothing written, where there is no such kernel: it is
- *      for 7x7 convolutions of three channels at stride 2 and pooling of 3x3 at stride 2, fp16 channels-last.  _ok: whether there
- *      is, for tensors like these at addresses that are multiples of 16. */
+ *      for 7x7 convolutions of three channels at stride 2 and pooling of 3x3 at stride 2, fp16 channels-last, with w and y at
+ *      multiples of 16.  _ok: whether there is, for tensors like these at addresses as well aligned as these. */
 int saga_hip_conv2d_fwd_bn_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,
                                       const SagaConvParams *p, int pool_size, int pool_pad, int pool_stride);
 int saga_hip_conv2d_fwd_bn_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y,

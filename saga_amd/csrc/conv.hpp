@@ -37,7 +37,7 @@ int conv_mfma_fwd(const SagaTensorView *x, const SagaTensorView *w, const SagaTe
                   size_t stats_floats = 0, int *stats_rows = nullptr, const ConvBnFold *bn = nullptr, const void *bias = nullptr,
                   bool *bias_done = nullptr, const void *packed = nullptr);
 // The same with a norm, relu and max pooling behind it, in one launch (stem_f16.hip); y: the pooled tensor.  ok: whether there is one
-// for tensors like these (at addresses of whole vectors).
+// for tensors like these.
 bool conv_bn_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, int size,
                         int pool_pad, int pool_stride);
 int conv_bn_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, const float *s,

@@ -316,15 +316,15 @@ StemArgs plan(const SagaTensorView *x, const SagaTensorView *w, const SagaTensor
 bool conv_bn_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, int size,
                         int pool_pad, int pool_stride)
 {
-    return plan(x, w, y, g, size, pool_pad, pool_stride).ntiles > 0;
+    return aligned16(w->ptr) && aligned16(y->ptr) && plan(x, w, y, g, size, pool_pad, pool_stride).ntiles > 0;
 }
 
 int conv_bn_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const ConvGeom &g, const float *s,
                     const float *b, const float *m, const float *v, float eps, int size, int pool_pad, int pool_stride, hipStream_t st)
 {
-    StemArgs t = plan(x, w, y, g, size, pool_pad, pool_stride);
-    if(!t.ntiles || !aligned16(w->ptr) || !aligned16(y->ptr))
+    if(!conv_bn_maxpool_ok(x, w, y, g, size, pool_pad, pool_stride))
         return SAGA_HIP_EUNSUPPORTED;
+    StemArgs t = plan(x, w, y, g, size, pool_pad, pool_stride);
     t.x = (const half_t *)x->ptr;
     t.w = (const half_t *)w->ptr;
     t.y = (half_t *)y->ptr;

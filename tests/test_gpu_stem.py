@@ -9,6 +9,8 @@ import torch
 
 from saga_amd import api as S
 from saga_amd import kernels as K
+from tests import stub_gpu
+from tests.stub_gpu import on_stub
 from tests.test_engine_plan import norm_params
 
 HALF = torch.float16
@@ -111,6 +113,28 @@ def test_what_it_does_not_take():
     assert not ok(v(2, 4, 64, 64), v(64, 4, 7, 7), v(2, 64, 16, 16))
     assert not ok(v(2, 3, 64, 64), v(64, 3, 5, 5), v(2, 64, 16, 16), pad=2)
     assert not ok(v(2, 3, 32, 1100), v(64, 3, 7, 7), v(2, 64, 8, 275))  # rows of which no strip fits
+
+
+@pytest.mark.parametrize("front", [4, 8])
+@on_stub
+def test_a_part_of_a_wider_tensor(front):
+    """Channels behind 4 others lie at no address of whole vectors: the launches are apart, and what is between them has memory."""
+    rng = np.random.default_rng(4)
+    tensor = lambda *d: S.Tensor.from_numpy(rng.standard_normal(d).astype(np.float16))
+    g = S.Graph()
+    y = g.add_node("conv", {"x": tensor(3, 3, 38, 42), "w": tensor(16, 3, 7, 7)}, {"size": 7, "activations": 16, "pad": 3, "stride": 2}).y()
+    y = g.add_node("batchnorm", {"x": y, **norm_params(rng, 16)}).y()
+    y = g.add_node("maxpool", {"x": g.add_node("relu", y).y()}, {"size": 3, "pad": 1, "stride": 2}).y()
+    y = g.add_node("concat", {"x0": tensor(3, front, 10, 11), "x1": y, "x2": tensor(3, front, 10, 11)}, {"axis": 1}).y()
+    ctx = S.Context()
+    p = ctx.create_program(g, 3, training=False)
+    ctx.resolve(y)
+    p.finalize()
+    used = stub_gpu.stub.hipstub_used()
+    p.run(2)
+    kinds = [op["kind"] for op in stub_gpu.plan(p)]
+    assert any(kind.endswith(".pool") for kind in kinds) == (front == 8), kinds
+    assert stub_gpu.stub.hipstub_used() == used  # no launch had to ask for any
 
 
 @pytest.mark.gpu
