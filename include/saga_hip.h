@@ -210,7 +210,7 @@ int saga_hip_conv2d_fwd_bn_maxpool(const SagaTensorView *x, const SagaTensorView
 /* ---- a forward with extras and a max pooling behind it (y: the pooled tensor): windows of 2x2 at stride 2, fp32, without a residual; for
  *      convolutions of up to four input channels, and 3x3 and 5x5 at stride 1 on grids that need no split reduction.
  *      SAGA_HIP_EUNSUPPORTED, with nothing written, otherwise.  _ok: whether there is such a kernel for tensors like these, at addresses that are
- *      multiples of 16, with the workspace that the convolution asks for. */
+ *      multiples of 16, with the workspace that the convolution asks for (an output over 2 GiB: none). */
 int saga_hip_conv2d_fwd_maxpool_ok(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,
                                    const SagaConvExtras *e, int pool_size, int pool_pad, int pool_stride);
 int saga_hip_conv2d_fwd_maxpool(const SagaTensorView *x, const SagaTensorView *w, const SagaTensorView *y, const SagaConvParams *p,

@@ -603,7 +603,8 @@ bool window_f32_may(const WindowConv &c, int channels, int IH, int IW, int OH, i
 bool window_f32_takes(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, bool pool)
 {
     WinArgs g = {};
-    return describe(c, a, out, pool, g) && choose(g, c.Tr, slice_groups(g.T)).quads;
+    // (a convolution alone has other kernels for an output out of reach; who asks for a pooling leaves the launches apart then)
+    return describe(c, a, out, pool, g) && (!pool || describe_out(out, 1.0f, 0.0f, StreamEpilogue(), g.o)) && choose(g, c.Tr, slice_groups(g.T)).quads;
 }
 
 int window_f32_conv(const WindowConv &c, const SagaTensorView *a, const SagaTensorView *out, float alpha, float beta,

@@ -126,6 +126,22 @@ def test_what_is_behind_the_pooling(behind):
     np.testing.assert_allclose(*got, rtol=0, atol=1e-5 * np.abs(got[1]).max())
 
 
+@pytest.mark.parametrize("shape", [s for s, k in SHAPES.items() if k and s[0] > 1], ids=str)
+@on_stub
+def test_an_output_out_of_reach(shape):
+    """Pooled results that are part of a tensor of more than 2 GiB: no such launch, and asked beforehand there is none either."""
+    L = K.lib()
+    xs, ws, _, ys, p = dims(shape)
+    x, w, y = (K.TensorView() for _ in range(3))
+    for v, d, at in ((x, xs, 20), (w, ws, 30), (y, ys, 31)):
+        v.ptr, v.dtype, v.dims[:] = 1 << at, K.FLOAT, d
+        v.strides[:] = torch.empty(d, device="meta").stride()
+    y.strides[0] = (1 << 29) // (ys[0] - 1)
+    X, W, Y, P, e = (C.byref(a) for a in (x, w, y, p, extras(relu=1)))
+    assert L.saga_hip_conv2d_fwd_maxpool(X, W, Y, P, e, 2, 0, 2, 1 << 33, 1 << 30, None) == -3
+    assert not L.saga_hip_conv2d_fwd_maxpool_ok(X, W, Y, P, e, 2, 0, 2)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("what", ["bias", "norm", "nothing", "not finite"])
 @pytest.mark.parametrize("shape", [s for s, k in SHAPES.items() if k], ids=str)
