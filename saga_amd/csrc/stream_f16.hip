@@ -550,6 +550,7 @@ Config choose(long long pixels, int taps, int C, int N, bool sums_or_bwd)
         const float us = o.start + split_over(steps, o.c.ks) * (o.step + o.more * rounds) + o.round * rounds;
         // u = 2 has to be cheaper by more than the numbers are off.  Of 1200 problems of 64 to 2048 channels 24 were 4 to 15 % slower than what
         // u = 2 takes the place of without these lines, 4 with them (the worst 1x49x49 3x3 1536->272 41 -> 47 us); 538 and 515 4 % and more faster.
+        // (Layers of a few us lose what little they gained: one image through ResNet-50 328 us without, 333 with them.)
         if(us < least * (o.c.u == 2 && best.u != 2 ? best.tm ? 0.95f : 0.86f : 1.0f)) {
             least = us;
             best = o.c;

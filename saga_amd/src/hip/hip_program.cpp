@@ -1031,7 +1031,8 @@ void HipProgram::runOpsGraphed()
 // An edge between the streams costs the host 13 us (hipStreamWaitEvent 12 of them), and the main stream 2: a step of ResNet-20 waited
 // for the host, not the GPU, with an edge for every convolution.  So much work of the side stream shares one (us of a step, an edge for each / 20 us / 40
 // / 70: batch 16 1057 / 813 / 844 / 864, 48 1070 / 892 / 909 / 939, 128 1099 / 1064 / 1108 / 1154, 256 1371 / 1343 / 1354 / 1360; more has less to run
-// beside).  How long an operation takes, roughly: launches, and operations and bytes at half of what large ones reach.
+// beside).  Fitted there; steps of ResNet-50 at 256 and of the U-Net at 16 x 256^2 take as long as when each had one (21.1 and 7.4 ms).  How long an
+// operation takes, roughly: launches, and operations and bytes at half of what large ones reach.
 static const double EDGE_US = 20;
 static double estimated_us(const HipOperation &op) { return 8 + std::max(op.flops() / 0.5e9, op.bytes() / 3e6); }
 
