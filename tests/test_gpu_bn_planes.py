@@ -1,5 +1,5 @@
 """Batch norm on channels-first tensors, whose channels are shared by several blocks: planes of whole vectors and of odd sizes, one
-block to a channel, that holds it between the sums and what follows or does not quite, and as many as one adds up, runs that end inside a plane, slices of wider tensors, addresses off the vectors'
+block to a channel and as many as one adds up, runs that end inside a plane, slices of wider tensors, addresses off the vectors'
 alignment, results over the input."""
 import ctypes as C
 
@@ -16,7 +16,7 @@ HALF, F32 = torch.float16, torch.float32
 
 # N, C, H, W, channels on either side in the tensor it is a slice of, elements before it
 SHAPES = [(1, 2, 1, 2, 0, 0), (3, 5, 1, 4, 0, 0), (2, 3, 7, 9, 0, 0), (33, 16, 8, 8, 0, 0), (33, 16, 8, 8, 0, 1), (5, 70, 13, 12, 2, 0),
-          (4, 6, 32, 32, 0, 0), (41, 3, 10, 10, 0, 0), (16, 5, 8, 8, 0, 1), (1, 4, 64, 64, 0, 0), (5, 3, 31, 33, 1, 0), (300, 2, 64, 64, 0, 0), (1025, 4, 3, 3, 0, 0), (2, 600, 4, 8, 0, 0)]
+          (4, 6, 32, 32, 0, 0), (1, 4, 64, 64, 0, 0), (5, 3, 31, 33, 1, 0), (300, 2, 64, 64, 0, 0), (1025, 4, 3, 3, 0, 0), (2, 600, 4, 8, 0, 0)]
 
 
 def placed(a, dtype, side, shift):
@@ -78,3 +78,11 @@ def test_planes(shape, dtype):
             assert_close(host(dxd), dx * (1 + beta_dz) + beta, dtype, "dx")
             if add:
                 np.testing.assert_array_equal(host(dzd), (g * (1 + beta_dz)).astype(np.float16).astype(np.float32) if dtype == HALF else g * (1 + beta_dz))
+
+
+# a channel that its block does not quite hold between the sums and what follows (1025 vectors; fp16: 4100 values), and one that it
+# just does (1024 values off the vectors' alignment)
+@pytest.mark.parametrize("dtype", [F32, HALF], ids=["f32", "f16"])
+@pytest.mark.parametrize("shape", [(41, 3, 10, 10, 0, 0), (16, 5, 8, 8, 0, 1)], ids=str)
+def test_planes_at_what_a_block_holds(shape, dtype):
+    test_planes(shape, dtype)
